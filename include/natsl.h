@@ -43,7 +43,8 @@ enum natsl_flags {
   NATSL_DECAY_NON_LINEAR = 1, /* decay_for_non_gdn_blocks / decay_for_non_mamba_blocks */
   NATSL_QK_L2NORM = 2,        /* lattn_use_qk_l2norm_in_kernel */
   NATSL_INTRA_CHUNK = 4,      /* the linear op also scores its own incomplete block ('all', 'gated_delta_net', 'mamba') */
-  NATSL_QUERY_ONLY = 8        /* recurrent entries: outputs from the decayed block-start state, nothing updated ('attn') */
+  NATSL_QUERY_ONLY = 8,       /* recurrent entries: outputs from the decayed block-start state, nothing updated ('attn') */
+  NATSL_FRESH_BLOCK_START = 16 /* recurrent entries: h_block_start is written only; the block starts from h0 (zeros if NULL) */
 };
 
 /* One row per packed sequence (cu_seqlens / cu_seqlens_nats of the reference, plus prefix
@@ -349,6 +350,18 @@ int natsl_kv_compact(const void* src_k, const void* src_v, long long src_tokens,
                      int HN, int K, int V, int dtype, int block, int NB, int n_complete, int tail_dst, int tail_tokens,
                      natsl_stream_t stream);
 
+/* Decode: both operators of a step in one call and two launches -- what natsl_attn_masked_fwd and natsl_gdn_recurrent_fwd
+ * (is_delta) or natsl_mamba_recurrent_fwd give on the same arguments, bf16, without the query-only form.  The attention runs
+ * next to the recurrence and splits its keys over more workgroups; workspace of natsl_decode_workspace_bytes().
+ * Replaces the pair of calls at src/nats/ops/mixed_ops/mixed_attn_gdn.py:475-503. */
+size_t natsl_decode_workspace_bytes(int B, int T, int TK, int HQ, int VA);
+int natsl_decode_fwd(int is_delta, const void* q_attn, const void* k_attn, const void* v_attn, const uint8_t* mask, void* o_attn,
+                     int B, int T, int TK, int HQ, int HKV, int HM, int KA, int VA, float scale_attn, int64_t k_batch_stride,
+                     int64_t v_batch_stride, void* workspace, size_t workspace_bytes, const void* q, const void* k,
+                     const void* v, const float* g, const float* g_cumsum, const void* beta, const float* h0,
+                     float* h_block_start, void* o, float* ht, const void* types, int types_dtype,
+                     const int32_t* n_tokens_in_block, int n_tokens_in_block_scalar, int H, int HN, int K, int V, int block,
+                     float scale, int flags, natsl_stream_t stream);
 
 #ifdef __cplusplus
 }

@@ -15,7 +15,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "csrc", "libnatsl.so")
 
 F32, BF16 = 0, 1
-DECAY_NON_LINEAR, QK_L2NORM, INTRA_CHUNK, QUERY_ONLY = 1, 2, 4, 8
+DECAY_NON_LINEAR, QK_L2NORM, INTRA_CHUNK, QUERY_ONLY, FRESH_BLOCK_START = 1, 2, 4, 8, 16
 
 _lib = None
 
@@ -71,6 +71,9 @@ _SIGNATURES = {
     "natsl_attn_masked_static_scratch_bytes": (c_size_t, []),
     "natsl_attn_masked_fwd_static": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                                              c_int, c_int, c_float, c_int, c_void_p]),
+    "natsl_decode_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
+    "natsl_decode_fwd": (c_int, [c_int] + [c_void_p] * 5 + [c_int] * 8 + [c_float, c_int64, c_int64, c_void_p, c_size_t] + [c_void_p] * 11 +
+                                [c_int, c_void_p] + [c_int] * 6 + [c_float, c_int, c_void_p]),
     "natsl_kv_compact": (c_int, [c_void_p, c_void_p, c_longlong, c_int, c_void_p, c_void_p, c_longlong, c_void_p, c_int, c_void_p,
                                  c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
 }
@@ -120,8 +123,10 @@ def dtype_code(t: torch.dtype) -> int:
 
 
 def ptr(t):
-    return None if t is None else c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def stream_ptr(device=None):
-    return c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """The current stream's handle as a number (the raw query: no Stream object is made)."""
+    index = device.index if isinstance(device, torch.device) else device
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)

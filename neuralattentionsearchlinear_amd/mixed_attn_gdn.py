@@ -161,6 +161,71 @@ def fused_recurrent_gated_delta_rule_nats_fwd(q, k, v, g, g_cumsum, beta, nats_b
     return o, ht, initial_state_in_current_block
 
 
+def _cache_view(t):
+    """(tensor, batch stride) of keys / values: the front part [:, :TK] of a cache buffer [B, capacity, H, D] is read in place (only
+    its batch stride differs from a dense tensor's); anything else is made contiguous."""
+    if t.is_contiguous():
+        return t, 0
+    _, TK, HKV, D = t.shape
+    s0, s1, s2, s3 = t.stride()
+    if s3 == 1 and s2 == D and s1 == HKV * D and s0 >= TK * HKV * D and s0 % 8 == 0:
+        return t, s0
+    return t.contiguous(), 0
+
+
+def decode_pair(delta: bool, q_attn, k_attn, v_attn, attn_msk, scale_attn, q, k, v, g, g_cumsum, beta, types, n_in, block, scale, state, start,
+                flags):
+    """Both operators of a decode step in one call (natsl_decode_fwd) -> (o_linear, o_attn, final state, block-start state), or None
+    for what it is not built for (fp32 tensors, head dims without a kernel, no cached key)."""
+    from . import _capi
+    bf16, f32 = torch.bfloat16, torch.float32
+    B, T, H, K = q.shape
+    HQ, KA = q_attn.shape[2:]
+    TK, HKV, VA = k_attn.shape[1], k_attn.shape[2], v_attn.shape[3]
+    V = v.shape[3]
+    if not (q.dtype == k.dtype == v.dtype == q_attn.dtype == k_attn.dtype == v_attn.dtype == bf16 and (not delta or beta.dtype == bf16)):
+        return None
+    if TK == 0 or q_attn.shape[1] != T or KA not in (64, 128) or VA not in (64, 128) or K not in (64, 128, 192) or types.shape[1] != 1:
+        return None
+    if attn_msk.dim() != 4 or attn_msk.shape[0] != B or attn_msk.shape[2] != T or attn_msk.shape[3] != TK:
+        raise ValueError(f"attn_msk must be [B, heads, {T}, {TK}], got {tuple(attn_msk.shape)}")
+    if start is not None and (start.dtype != f32 or not start.is_contiguous()):
+        raise ValueError("initial_state_in_current_block must be a contiguous fp32 tensor (it is updated in place)")
+    dev = q.device
+    (k_attn, k_bs), (v_attn, v_bs) = _cache_view(k_attn), _cache_view(v_attn)
+    q_attn, q, k, v = q_attn.contiguous(), q.contiguous(), k.contiguous(), v.contiguous()
+    if delta:
+        beta = beta.contiguous()
+    g = g.to(f32).contiguous()
+    if types.dtype not in (f32, bf16):
+        types = types.float()
+    types = types.contiguous()
+    mask = attn_msk.to(torch.bool).contiguous()
+    if state is not None:
+        state = state.to(f32).contiguous()
+    if start is None:
+        start = torch.empty(B, H, K, V, dtype=f32, device=dev)
+        flags |= _capi.FRESH_BLOCK_START
+    if g_cumsum is not None:
+        g_cumsum = g_cumsum.to(f32).reshape(B, H).contiguous()
+    if torch.is_tensor(n_in):
+        n_ptr, n_scalar = n_in.to(device=dev, dtype=torch.int32).contiguous(), 0
+    else:
+        n_ptr, n_scalar = None, int(n_in)
+    o_attn = torch.empty(B, T, HQ, VA, dtype=bf16, device=dev)
+    o = torch.empty(B, T, H, V, dtype=bf16, device=dev)
+    ht = torch.empty(B, H, K, V, dtype=f32, device=dev)
+    L, P = _capi.lib(), _capi.ptr
+    ws_bytes = L.natsl_decode_workspace_bytes(B, T, TK, HQ, VA)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+    rc = L.natsl_decode_fwd(
+        int(delta), P(q_attn), P(k_attn), P(v_attn), P(mask), P(o_attn), B, T, TK, HQ, HKV, mask.shape[1], KA, VA, scale_attn, k_bs, v_bs,
+        P(ws), ws_bytes, P(q), P(k), P(v), P(g), P(g_cumsum), P(beta), P(state), P(start), P(o), P(ht), P(types),
+        _capi.dtype_code(types.dtype), P(n_ptr), n_scalar, H, types.shape[2], K, V, block, scale, flags, _capi.stream_ptr(dev))
+    _capi.check(rc, "natsl_decode_fwd")
+    return o, o_attn, ht, start
+
+
 def masked_attention(q, k, v, attn_msk, scale):
     """Softmax attention of a few queries over cached keys under a boolean mask [B, HM, TQ, TK] (HM divides the
     number of query heads); replaces repeat_masks + scaled_dot_product_attention at
@@ -173,15 +238,7 @@ def masked_attention(q, k, v, attn_msk, scale):
     if TK == 0:
         return q.new_zeros(B, TQ, HQ, V)          # no cached key yet: every query sees nothing
     q = q.contiguous()
-
-    def cache_view(t):
-        # the front part [:, :TK] of a cache buffer [B, capacity, H, D] is read in place (only its batch stride differs
-        # from a dense tensor's); anything else is made contiguous
-        D = t.shape[-1]
-        if t.stride(3) == 1 and t.stride(2) == D and t.stride(1) == HKV * D and t.stride(0) >= TK * HKV * D and t.stride(0) % 8 == 0:
-            return t, t.stride(0)
-        return t.contiguous(), 0
-    (k, k_bs), (v, v_bs) = cache_view(k), cache_view(v)
+    (k, k_bs), (v, v_bs) = _cache_view(k), _cache_view(v)
     if not (q.dtype == k.dtype == v.dtype):
         raise ValueError("q, k, v must share a dtype")
     mask = attn_msk.to(torch.bool).contiguous().view(torch.uint8)
@@ -248,6 +305,14 @@ def nats_mixed_attn_gdn_recurrent(
         from . import _capi
         raise _capi.NatslError("the NAtS-L mixed operator runs on the GPU only (no CPU fallback)")
     with torch.no_grad():
+        if strategy.gated_delta_net:
+            from . import _capi
+            flags = (_capi.DECAY_NON_LINEAR if decay_for_non_gdn_blocks else 0) | (_capi.QK_L2NORM if lattn_use_qk_l2norm_in_kernel else 0)
+            pair = decode_pair(True, q_attn, k_attn, v_attn, attn_msk, scale_attn, q_lattn, k_lattn, v_lattn, g, g_cumsum, beta,
+                               nats_block_types, n_tokens_in_current_block, nats_block_size, scale_lattn, initial_state_gated_delta,
+                               initial_state_gated_delta_chunk_start, flags)
+            if pair is not None:
+                return pair
         o_attn = masked_attention(q_attn, k_attn, v_attn, attn_msk, scale_attn)
         if strategy.gated_delta_net:
             o_gdn, final_state, start = fused_recurrent_gated_delta_rule_nats_fwd(

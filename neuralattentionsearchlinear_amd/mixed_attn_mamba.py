@@ -175,7 +175,7 @@ def nats_mixed_attn_mamba_recurrent(
     defaults to K**-0.5 here.  'all' / 'mamba': the linear operator also runs on the incomplete block.  'attn' (:516-591): the
     new tokens read the (decayed) state that entered the block, and the state advances when the block is complete, by the
     token recurrence over the block's cached k, v, g; built for nats_block_size = 64 and steps that stay inside the block."""
-    from .mixed_attn_gdn import masked_attention
+    from .mixed_attn_gdn import decode_pair, masked_attention
     if scale_attn is None:
         scale_attn = k_attn.shape[-1] ** -0.5
     if scale_lattn is None:
@@ -197,6 +197,13 @@ def nats_mixed_attn_mamba_recurrent(
         from . import _capi
         raise _capi.NatslError("the NAtS-L mixed operator runs on the GPU only (no CPU fallback)")
     with torch.no_grad():
+        if strategy.mamba:
+            from . import _capi
+            pair = decode_pair(False, q_attn, k_attn, v_attn, attn_msk, scale_attn, q_lattn, k_lattn, v_lattn, g, g_cumsum, None,
+                               nats_block_types, n_tokens_in_current_block, nats_block_size, scale_lattn, initial_state_mamba,
+                               initial_state_mamba_chunk_start, _capi.DECAY_NON_LINEAR if decay_for_non_mamba_blocks else 0)
+            if pair is not None:
+                return pair
         o_attn = masked_attention(q_attn, k_attn, v_attn, attn_msk, scale_attn)
         if strategy.mamba:
             o_mamba, final_state, start = fused_recurrent_mamba_nats_fwd(

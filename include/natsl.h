@@ -363,6 +363,47 @@ int natsl_decode_fwd(int is_delta, const void* q_attn, const void* k_attn, const
                      const int32_t* n_tokens_in_block, int n_tokens_in_block_scalar, int H, int HN, int K, int V, int block,
                      float scale, int flags, natsl_stream_t stream);
 
+/* A generation step of a whole hybrid layer (bf16): T new tokens for each of B cached sequences, all inside the current
+ * selector block, from the hidden states to the layer's output.  Replaces the decode path of the layers' forward
+ * (src/nats/layers/natsl_attn_gdn.py:387-666, src/nats/layers/natsl_attn_mamba2.py:328-599) together with what their cache
+ * does with the new tokens (src/nats/models/utils.py:178-457) when no block is compacted.
+ * Weights are the layers' own (row-major [out, in], bf16; convolutions [channels, conv_width]); H linear heads of K / V, HQ
+ * attention heads that divide them evenly, HN selector heads; B*T <= 64.  The cache rows of the new tokens are written in
+ * place: cache_k / cache_v [B, cache_tokens, HQ, *] at token n_kept*block + n_in, cache_valid (a byte per (sequence, block,
+ * selector head)) for the incomplete block, block_k / block_v / block_g / block_beta / block_hidden [B, block, ...] at n_in
+ * (block_hidden may be NULL).  States and convolution states are read from one tensor and written to another. */
+enum natsl_step_flags {
+  NATSL_STEP_DECAY = 1,          /* decay_for_non_*_blocks */
+  NATSL_STEP_SILU = 2,           /* the convolutions' activation */
+  NATSL_STEP_ATTN_FROM_CONV = 4, /* the attention view takes the convolved q, k, v (else the projections) */
+  NATSL_STEP_ATTN_NORM = 8,      /* RMSNorm of the attention view's q and k rows */
+  NATSL_STEP_L2_ROWS = 16,       /* the linear view's q and k rows are L2-normalised (and rounded) first (Mamba layer) */
+  NATSL_STEP_ATTN_OWN_BLOCK = 32,/* the softmax operator runs on the incomplete block */
+  NATSL_STEP_NEG_EIGVAL = 64,    /* beta doubled */
+  NATSL_STEP_FRESH_START = 128   /* block_start is written only: the block starts from `state` */
+};
+typedef struct natsl_layer_step {
+  int32_t B, T, D, H, K, V, HQ, HN, block, conv_width, is_delta, flags;
+  int32_t n_in, n_kept, cache_tokens, types_dtype, norm_dtype, gate_dtype, out_norm_dtype, reserved;
+  float scale_attn, scale_linear, norm_eps, l2_eps, out_norm_eps, reserved_f;
+  const void *wq, *wk, *wv, *wg, *wa, *wb, *w_mix, *wo;
+  const void *conv_wq, *conv_wk, *conv_wv, *conv_bq, *conv_bk, *conv_bv;
+  const void *norm_q, *norm_k, *a_log, *dt_bias, *out_norm1, *out_norm2;
+  const void *x, *types;
+  const void *conv_state_q, *conv_state_k, *conv_state_v;
+  void *conv_out_q, *conv_out_k, *conv_out_v;
+  const float *state, *g_cumsum;
+  float *block_start, *state_out, *g_cumsum_out;
+  void *cache_k, *cache_v;
+  uint8_t* cache_valid;
+  void *block_k, *block_v;
+  float* block_g;
+  void *block_beta, *block_hidden;
+  void* out;
+} natsl_layer_step;
+size_t natsl_layer_step_workspace_bytes(const natsl_layer_step* step);
+int natsl_layer_step_fwd(const natsl_layer_step* step, void* workspace, size_t workspace_bytes, natsl_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

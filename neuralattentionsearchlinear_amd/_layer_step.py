@@ -1,0 +1,203 @@
+"""The layers' generation step as one native call (natsl_layer_step_fwd): a few new tokens of cached sequences, from the hidden
+states to the layer's output, with the cache's new rows written in place.
+
+A step of a layer is a few microseconds of memory traffic per kernel, so what it costs is launches and host time: the same step
+as separate torch operations and operator calls is forty launches and ~0.57 ms of host time (340M geometry), this is five
+launches behind one ctypes call.  `layer_step` declines (returns None) whatever the call is not built for -- other dtypes,
+tensors that want gradients, replaced or hooked submodules, the 'attn' mode, more than 64 new tokens in all -- and the layers'
+general path runs.
+"""
+from __future__ import annotations
+
+import ctypes
+
+import torch
+import torch.nn as nn
+
+from . import _capi
+from .modules import FusedMultiInputRMSNormGated, RMSNorm, ShortConvolution
+
+MAX_ROWS = 64
+
+_INTS = ("B", "T", "D", "H", "K", "V", "HQ", "HN", "block", "conv_width", "is_delta", "flags", "n_in", "n_kept", "cache_tokens", "types_dtype",
+         "norm_dtype", "gate_dtype", "out_norm_dtype", "reserved")
+_FLOATS = ("scale_attn", "scale_linear", "norm_eps", "l2_eps", "out_norm_eps", "reserved_f")
+_WEIGHTS = ("wq", "wk", "wv", "wg", "wa", "wb", "w_mix", "wo", "conv_wq", "conv_wk", "conv_wv", "conv_bq", "conv_bk", "conv_bv", "norm_q", "norm_k",
+            "a_log", "dt_bias", "out_norm1", "out_norm2")
+_TENSORS = ("x", "types", "conv_state_q", "conv_state_k", "conv_state_v", "conv_out_q", "conv_out_k", "conv_out_v", "state", "g_cumsum",
+            "block_start", "state_out", "g_cumsum_out", "cache_k", "cache_v", "cache_valid", "block_k", "block_v", "block_g", "block_beta",
+            "block_hidden", "out")
+
+
+class LayerStep(ctypes.Structure):
+    """natsl_layer_step of include/natsl.h."""
+    _fields_ = ([(n, ctypes.c_int32) for n in _INTS] + [(n, ctypes.c_float) for n in _FLOATS] +
+                [(n, ctypes.c_void_p) for n in _WEIGHTS + _TENSORS])
+
+
+DECAY, SILU, ATTN_FROM_CONV, ATTN_NORM, L2_ROWS, ATTN_OWN_BLOCK, NEG_EIGVAL, FRESH_START = (1 << i for i in range(8))
+
+# where the weights are: (field, submodule or None, parameter, exact submodule type or None)
+_PARAMS = (("wq", "q_proj", "weight", nn.Linear), ("wk", "k_proj", "weight", nn.Linear), ("wv", "v_proj", "weight", nn.Linear),
+           ("wg", "g_proj", "weight", nn.Linear), ("wa", "a_proj", "weight", nn.Linear), ("wb", "b_proj", "weight", nn.Linear),
+           ("w_mix", "nats_out_weights_layer", "weight", nn.Linear), ("wo", "o_proj", "weight", nn.Linear),
+           ("conv_wq", "q_conv1d", "weight", ShortConvolution), ("conv_wk", "k_conv1d", "weight", ShortConvolution),
+           ("conv_wv", "v_conv1d", "weight", ShortConvolution), ("conv_bq", "q_conv1d", "bias", None), ("conv_bk", "k_conv1d", "bias", None),
+           ("conv_bv", "v_conv1d", "bias", None), ("norm_q", "q_norm", "weight", RMSNorm), ("norm_k", "k_norm", "weight", RMSNorm),
+           ("a_log", None, "A_log", None), ("dt_bias", None, "dt_bias", None), ("out_norm1", "o_norm", "weight1", FusedMultiInputRMSNormGated),
+           ("out_norm2", "o_norm", "weight2", FusedMultiInputRMSNormGated))
+_OPTIONAL = {"wb", "norm_q", "norm_k", "conv_bq", "conv_bk", "conv_bv"}
+_EITHER_DTYPE = {"norm_q", "norm_k", "a_log", "dt_bias", "out_norm1", "out_norm2"}       # the others are bf16
+
+
+def _parameters(layer):
+    """The current weight tensors by field (None where the layer has none), or None when a submodule is not the plain one."""
+    mods, own = layer._modules, layer._parameters
+    out = []
+    for _, mod, name, kind in _PARAMS:
+        if mod is None:
+            out.append(own.get(name))
+            continue
+        m = mods.get(mod)
+        if m is None:
+            out.append(None)
+            continue
+        if kind is not None and (type(m) is not kind or m._forward_hooks or m._forward_pre_hooks or 'forward' in m.__dict__):
+            return None
+        out.append(m._parameters.get(name))
+    return out
+
+
+class _Plan:
+    """What stays the same from step to step: the weights' addresses, the geometry and the mode."""
+
+    def __init__(self, layer, kind, key, params):
+        self.key = key
+        self.built = False
+        s = self.fixed = LayerStep()
+        by = dict(zip((p[0] for p in _PARAMS), params))
+        delta = kind == 'gdn'
+        K, V, H, HQ = layer.head_k_dim, layer.head_v_dim, layer.num_heads, layer.num_attn_heads
+        for n, t in by.items():
+            if t is None:
+                if n not in _OPTIONAL or (n == "wb" and delta) or (n in ("norm_q", "norm_k") and layer.attn_qk_norm):
+                    return
+                continue
+            if not (t.is_cuda and t.is_contiguous() and t.device == params[0].device and
+                    (t.dtype == torch.bfloat16 or (n in _EITHER_DTYPE and t.dtype == torch.float32))):
+                return
+            setattr(s, n, t.data_ptr())
+        same = lambda a, b: by[a] is None or by[a].dtype == by[b].dtype
+        if not (same("norm_q", "norm_k") and same("a_log", "dt_bias") and same("out_norm1", "out_norm2")):
+            return
+        if not layer.use_short_conv or layer.num_v_heads != H or layer.ops_for_incomplete_chunks == 'attn':
+            return
+        convs = [layer.q_conv1d, layer.k_conv1d, layer.v_conv1d]
+        W, act = convs[0].kernel_size[0], convs[0].activation
+        if any(c.kernel_size[0] != W or (c.activation is None) != (act is None) for c in convs) or W not in (2, 3, 4):
+            return
+        if any(layer._modules[m].bias is not None for m in ("q_proj", "k_proj", "v_proj", "g_proj", "a_proj", "nats_out_weights_layer", "o_proj")):
+            return
+        D, KA, VA = layer.hidden_size, layer.head_attn_k_dim, layer.head_attn_v_dim
+        if K not in (64, 128, 192) or KA not in (64, 128) or VA not in (64, 128) or K % KA or HQ % H or HQ % layer.num_nats_head or \
+                H % layer.num_nats_head or V % 16 or D % 32 or (H * V) % 32 or layer.nats_block_size % 64:
+            return
+        code = lambda n: _capi.dtype_code(by[n].dtype) if by[n] is not None else _capi.BF16
+        s.D, s.H, s.K, s.V, s.HQ, s.HN, s.block, s.conv_width, s.is_delta = D, H, K, V, HQ, layer.num_nats_head, layer.nats_block_size, W, int(delta)
+        s.norm_dtype, s.gate_dtype, s.out_norm_dtype = code("norm_q"), code("a_log"), code("out_norm1")
+        if by["norm_q"] is not None:
+            if layer.q_norm.eps != layer.k_norm.eps:
+                return
+            s.norm_eps = layer.q_norm.eps
+        s.scale_attn, s.out_norm_eps = KA ** -0.5, layer.o_norm.eps
+        flags = (SILU if act is not None else 0) | (ATTN_FROM_CONV if layer.attn_with_short_conv else 0) | \
+                (ATTN_NORM if layer.attn_qk_norm else 0) | (ATTN_OWN_BLOCK if layer.ops_for_incomplete_chunks == 'all' else 0)
+        if delta:
+            flags |= (DECAY if layer.decay_for_non_gdn_blocks else 0) | (NEG_EIGVAL if layer.allow_neg_eigval else 0)
+            s.scale_linear = K ** -0.5
+        else:
+            flags |= (DECAY if layer.decay_for_non_mamba_blocks else 0) | L2_ROWS
+            s.scale_linear = 1.0
+            if layer.q_norm2.eps != layer.k_norm2.eps:
+                return
+            s.l2_eps = layer.q_norm2.eps
+        s.flags = flags
+        self.device = params[0].device
+        self.conv_shapes = ((H * K, W), (H * K, W), (H * V, W))
+        self.built = True
+
+
+def layer_step(layer, kind, x, cache):
+    """The layer's output [B,T,D] for new tokens x on `cache` (NAtSLayerCache), which is brought up to date; None when the general
+    path has to run.  Called with the cache as it is before the step and only for steps that stay inside the block."""
+    B, T, D = x.shape
+    if B * T > MAX_ROWS or T < 1 or x.dtype != torch.bfloat16 or torch.is_grad_enabled() and _wants_grad(layer, x) or torch.is_autocast_enabled():
+        return None
+    params = _parameters(layer)
+    if params is None:
+        return None
+    key = tuple([None if t is None else (t.data_ptr(), t.dtype) for t in params])
+    plan = layer.__dict__.get('_step_plan')
+    if plan is None or plan.key != key:
+        plan = layer.__dict__['_step_plan'] = _Plan(layer, kind, key, params)
+    if not plan.built:
+        return None
+    bs, n_in, n_kept = cache.nats_block_size, cache._n_tokens_in_nats_block, cache.n_attn_blocks_max
+    conv, state, start = cache.conv_state, cache.recurrent_state, cache.recurrent_state_block_start
+    f = plan.fixed
+    if (cache.attn_k is None or cache.l_attn_k is None or cache.block_type_state is None or state is None or conv is None or
+            conv[0] is None or cache.valid_attn_tokens is None or bs != f.block or n_in + T > bs or x.device != plan.device or
+            cache.n_attn_blocks is None or (cache._linear_only == bool(f.flags & ATTN_OWN_BLOCK)) or cache.attn_k.dtype != torch.bfloat16 or
+            state.dtype != torch.float32 or cache.op_for_incomplete_chunk == 'attn'):
+        return None
+    for c, (ch, W) in zip(conv, plan.conv_shapes):
+        if c.dtype != torch.bfloat16 or c.shape != (B, ch, W) or not c.is_contiguous():
+            return None
+    if cache.attn_k.shape[0] != B or state.shape[0] != B or not state.is_contiguous():
+        return None
+    types = None
+    if n_in + T == bs:
+        types, _, _ = layer.select_ops(cache.update_attn_types(input_hidden_states=x), None, force_last_block=False)
+        types = types.contiguous()
+    cache._grow(cache.n_attn_tokens_max + T)
+    x = x.contiguous()
+    dev = x.device
+    s = LayerStep.from_buffer_copy(f)
+    s.B, s.T, s.n_in, s.n_kept, s.cache_tokens = B, T, n_in, n_kept, cache.attn_k.shape[1]
+    new_conv = tuple([torch.empty_like(c) for c in conv])
+    state_out = torch.empty_like(state)
+    if start is None:
+        start = torch.empty_like(state)
+        s.flags |= FRESH_START
+    g_sum = cache.g_cumsum
+    if g_sum is not None and (g_sum.dtype != torch.float32 or not g_sum.is_contiguous()):
+        g_sum = g_sum.float().contiguous()
+    g_out = torch.empty((B, 1, f.H), dtype=torch.float32, device=dev)
+    out = torch.empty((B, T, D), dtype=torch.bfloat16, device=dev)
+    s.x, s.out, s.state, s.state_out, s.block_start = x.data_ptr(), out.data_ptr(), state.data_ptr(), state_out.data_ptr(), start.data_ptr()
+    s.conv_state_q, s.conv_state_k, s.conv_state_v = conv[0].data_ptr(), conv[1].data_ptr(), conv[2].data_ptr()
+    s.conv_out_q, s.conv_out_k, s.conv_out_v = new_conv[0].data_ptr(), new_conv[1].data_ptr(), new_conv[2].data_ptr()
+    s.g_cumsum, s.g_cumsum_out = None if g_sum is None else g_sum.data_ptr(), g_out.data_ptr()
+    s.cache_k, s.cache_v, s.cache_valid = cache.attn_k.data_ptr(), cache.attn_v.data_ptr(), cache.valid_attn_tokens.data_ptr()
+    s.block_k, s.block_v, s.block_g = cache.l_attn_k.data_ptr(), cache.l_attn_v.data_ptr(), cache.lattn_g.data_ptr()
+    if cache.lattn_beta is not None:
+        s.block_beta = cache.lattn_beta.data_ptr()
+    if types is None:
+        s.block_hidden = cache.block_type_state.data_ptr()
+    else:
+        s.types, s.types_dtype = types.data_ptr(), _capi.dtype_code(types.dtype)
+    L = _capi.lib()
+    ref = ctypes.byref(s)
+    ws = torch.empty(L.natsl_layer_step_workspace_bytes(ref), dtype=torch.uint8, device=dev)
+    _capi.check(L.natsl_layer_step_fwd(ref, ws.data_ptr(), ws.numel(), _capi.stream_ptr(dev)), "natsl_layer_step_fwd")
+    if types is None:
+        cache.note_step(state_out, start, new_conv, g_out, T)
+    else:
+        cache.update(recurrent_state=state_out, recurrent_state_block_start=start, attn_state=(cache.attn_k, cache.attn_v), conv_state=new_conv,
+                     nats_block_types=types, g=cache.lattn_g, n_new_tokens=T)
+    layer.last_recurrent_state, layer.last_block_start_state = state_out, start
+    return out
+
+
+def _wants_grad(layer, x):
+    return x.requires_grad or any(p.requires_grad for p in layer.parameters())

@@ -247,6 +247,16 @@ class NAtSLayerCache:
         if tail_tokens:
             self.valid_attn_tokens[:, new_max] = True
 
+    def note_step(self, recurrent_state, recurrent_state_block_start, conv_state, g_cumsum, n_new_tokens: int):
+        """What update() does for tokens that stay inside the incomplete block, where the step itself has written the cache's
+        rows, the block's validity flags and the sum of g (natsl_layer_step_fwd)."""
+        self.recurrent_state, self.recurrent_state_block_start = recurrent_state, recurrent_state_block_start
+        self.conv_state, self.g_cumsum = conv_state, g_cumsum
+        self._n_tokens_in_nats_block += n_new_tokens
+        self.n_attn_tokens_max += n_new_tokens
+        self.n_observed_tokens += n_new_tokens
+        self.seen_tokens += n_new_tokens
+
     def update(self, recurrent_state=None, recurrent_state_block_start=None, attn_state=None, conv_state=None,
                nats_block_types: Optional[torch.Tensor] = None, ffn_state=None, g: Optional[torch.Tensor] = None,
                n_new_tokens: int = 0, cache_kwargs: Optional[Dict[str, Any]] = None, l_attn_state=None):

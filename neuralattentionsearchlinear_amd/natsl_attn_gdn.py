@@ -21,6 +21,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import nats_util
+from ._layer_step import layer_step
 from .cache import NAtSCache, NAtSLayerCache
 from .mixed_attn_gdn import nats_mixed_attn_gdn, nats_mixed_attn_gdn_chunk_inference, nats_mixed_attn_gdn_recurrent
 from .modules import FusedMultiInputRMSNormGated, RMSNorm, ShortConvolution
@@ -162,6 +163,10 @@ class NeuralAttentionSearchLinearAttnGDN(nn.Module):
                 o1 = self.forward(hidden_states[:, :first], attention_mask, **kw)[0]
                 o2 = self.forward(hidden_states[:, first:], attention_mask, **kw)[0]
                 return torch.cat([o1, o2], 1), None, past_key_values
+        if cache is not None and mode != 'chunk' and use_cache:
+            o = layer_step(self, 'gdn', hidden_states, cache)
+            if o is not None:
+                return o, None, past_key_values
         # selector: on a cache, over the tokens of the incomplete block + the new ones, once they complete a block
         if cache is not None:
             selector_input = cache.update_attn_types(input_hidden_states=hidden_states)

@@ -14,6 +14,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import nats_util
+from ._layer_step import layer_step
 from .cache import NAtSLayerCache
 from .mixed_attn_mamba import (nats_mixed_attn_mamba, nats_mixed_attn_mamba_chunk_inference,
                                nats_mixed_attn_mamba_recurrent)
@@ -135,6 +136,10 @@ class NeuralAttentionSearchLinearAttnMamba(nn.Module):
                 kw = dict(cache_params=cache_params, use_cache=use_cache, output_attentions=output_attentions, **kwargs)
                 return torch.cat([self.forward(hidden_states[:, :first], attention_mask, **kw),
                                   self.forward(hidden_states[:, first:], attention_mask, **kw)], 1)
+        if cache is not None and mode != 'chunk':
+            o = layer_step(self, 'mamba', hidden_states, cache)
+            if o is not None:
+                return o
         selector_input = cache.update_attn_types(input_hidden_states=hidden_states) if cache is not None else hidden_states
         if selector_input is not None:
             raw_types, _, _ = self.select_ops(selector_input, cu_seqlens, force_last_block=False)

@@ -1,0 +1,102 @@
+"""The layers' generation step as one native call (natsl_layer_step_fwd) against the layers' general decode path (separate torch
+operations and operator calls), which the other tests pin to the oracle."""
+import pytest
+import torch
+
+from tests._util import rel_l2
+from tests.test_gpu_layers import PUBLISHED
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda:0'
+
+
+def _layer(kind, geometry, ops, **more):
+    from neuralattentionsearchlinear_amd.natsl_attn_gdn import NeuralAttentionSearchLinearAttnGDN as G
+    from neuralattentionsearchlinear_amd.natsl_attn_mamba2 import NeuralAttentionSearchLinearAttnMamba as M
+    torch.manual_seed(3)
+    if kind == 'gdn':
+        cfg = dict(hidden_size=256, expand_v=2, head_dim=128, num_heads=2, num_attn_heads=4, ops_for_incomplete_chunks=ops, layer_idx=0)
+        cfg.update(PUBLISHED[geometry] if geometry else {})
+        layer = G(**dict(cfg, **more))
+    else:
+        layer = M(**dict(dict(hidden_size=256, expand_v=0.5, head_dim=128, num_heads=4, num_attn_heads=4, ops_for_incomplete_chunks=ops,
+                              layer_idx=0), **more))
+    return layer.to(DEV).to(torch.bfloat16).eval()
+
+
+def _generate(layer, kind, x, T0, sizes):
+    from neuralattentionsearchlinear_amd.cache import NAtSCache, NAtSMamba2Cache
+    holder = NAtSCache() if kind == 'gdn' else NAtSMamba2Cache()
+    kw = dict(past_key_values=holder, use_cache=True) if kind == 'gdn' else dict(cache_params=holder, use_cache=True)
+    outs, t = [], 0
+    with torch.no_grad():
+        for n in [T0] + list(sizes):
+            o = layer(x[:, t:t + n], **kw)
+            outs.append(o[0] if isinstance(o, tuple) else o)
+            t += n
+    return outs, (holder[0] if kind == 'gdn' else holder.nats_cache[0])
+
+
+@pytest.mark.parametrize("kind,geometry,ops,B,T0,sizes,more", [
+    ('gdn', None, 'all', 1, 100, (1, 1, 5, 1), {}),                       # one row; several tokens at once
+    ('gdn', '340M', 'all', 3, 321, (1, 20, 1), {}),                       # 20 x 3 rows: four row tiles
+    ('gdn', '760M', 'all', 2, 130, (1, 2), dict(allow_neg_eigval=True, conv_bias=True)),
+    ('gdn', None, 'all', 17, 70, (1, 3, 1), {}),                          # two row tiles, one of them with one row
+    ('gdn', None, 'all', 64, 65, (1,), {}),                               # the most rows it takes
+    ('gdn', None, 'all', 1, 128, (1, 63, 1), {}),                         # a block's first token, and a step that completes it (64 rows at most)
+    ('gdn', None, 'gated_delta_net', 2, 100, (1, 3), {}),                 # the softmax operator skips the incomplete block
+    ('gdn', None, 'all', 2, 200, (1, 1), dict(attn_with_short_conv=False, attn_qk_norm=False, conv_size=3, conv_activation=None)),
+    ('mamba', None, 'all', 2, 257, (1, 4), {}),
+    ('mamba', None, 'mamba', 5, 190, (1, 1, 1), dict(attn_qk_norm=True, conv_size=2)),
+])
+def test_layer_step_matches_the_general_path(kind, geometry, ops, B, T0, sizes, more, monkeypatch):
+    import neuralattentionsearchlinear_amd._layer_step as LS
+    from neuralattentionsearchlinear_amd import natsl_attn_gdn, natsl_attn_mamba2
+    layer = _layer(kind, geometry, ops, **more)
+    torch.manual_seed(T0)
+    x = torch.randn(B, T0 + sum(sizes), layer.hidden_size, device=DEV).bfloat16()
+    taken = []
+    for mod in (natsl_attn_gdn, natsl_attn_mamba2):
+        monkeypatch.setattr(mod, 'layer_step', lambda *a: taken.append(LS.layer_step(*a)) or taken[-1])
+    fast, cf = _generate(layer, kind, x, T0, sizes)
+    assert len(taken) == len(sizes) and all(t is not None for t in taken), "the native step declined"
+    for mod in (natsl_attn_gdn, natsl_attn_mamba2):
+        monkeypatch.setattr(mod, 'layer_step', lambda *a: None)
+    slow, cs = _generate(layer, kind, x, T0, sizes)
+    # both round to bf16 at the same places; a value that falls on a rounding edge moves by one ulp (2^-8) there, and such
+    # differences pass through two more products: 5e-3 in the norm, the bound the operators are held to
+    for i, (a, b) in enumerate(zip(fast, slow)):
+        assert a.shape == b.shape and a.dtype == b.dtype
+        assert rel_l2(a.float(), b.float()) <= 5e-3, f"step {i}: rel-L2 {rel_l2(a.float(), b.float()):.3e}"
+    assert (cf._n_tokens_in_nats_block, cf.n_attn_blocks_max, cf.n_attn_tokens_max, cf.n_observed_tokens) == \
+        (cs._n_tokens_in_nats_block, cs.n_attn_blocks_max, cs.n_attn_tokens_max, cs.n_observed_tokens)
+    assert torch.equal(cf.n_attn_blocks, cs.n_attn_blocks) and torch.equal(cf.valid_attn_tokens, cs.valid_attn_tokens)
+    n_in, start = cf._n_tokens_in_nats_block, cf.n_attn_blocks_max * cf.nats_block_size
+    pairs = [(cf.attn_k[:, start:start + n_in], cs.attn_k[:, start:start + n_in]), (cf.attn_v[:, start:start + n_in], cs.attn_v[:, start:start + n_in]),
+             (cf.recurrent_state, cs.recurrent_state), (cf.g_cumsum, cs.g_cumsum), (cf.l_attn_v[:, :n_in], cs.l_attn_v[:, :n_in]),
+             (cf.l_attn_k[:, :n_in], cs.l_attn_k[:, :n_in]), (cf.lattn_g[:, :n_in], cs.lattn_g[:, :n_in]),
+             (cf.block_type_state[:, :n_in], cs.block_type_state[:, :n_in])] + list(zip(cf.conv_state, cs.conv_state))
+    if kind == 'gdn':
+        pairs.append((cf.lattn_beta[:, :n_in], cs.lattn_beta[:, :n_in]))
+    if cs.recurrent_state_block_start is not None:
+        pairs.append((cf.recurrent_state_block_start, cs.recurrent_state_block_start))
+    for i, (a, b) in enumerate(pairs):
+        assert a.shape == b.shape and rel_l2(a.float(), b.float()) <= 5e-3, f"cache tensor {i}: rel-L2 {rel_l2(a.float(), b.float()):.3e}"
+
+
+def test_layer_step_follows_replaced_weights_and_declines_hooks():
+    """The step reads the layer's current parameters, and a hooked submodule sends the layer down the general path."""
+    import neuralattentionsearchlinear_amd._layer_step as LS
+    layer = _layer('gdn', None, 'all')
+    torch.manual_seed(1)
+    x = torch.randn(2, 102, 256, device=DEV).bfloat16()
+    _, cache = _generate(layer, 'gdn', x[:, :100], 100, ())
+    calls = []
+    with torch.no_grad():
+        handle = layer.v_proj.register_forward_hook(lambda *a: calls.append(1))
+        assert LS.layer_step(layer, 'gdn', x[:, 100:101], cache) is None
+        handle.remove()
+        assert LS.layer_step(layer, 'gdn', x[:, 100:101], cache) is not None
+        layer.o_proj.weight = torch.nn.Parameter(torch.zeros_like(layer.o_proj.weight))
+        out = LS.layer_step(layer, 'gdn', x[:, 101:102], cache)
+    assert float(out.abs().max()) == 0.0

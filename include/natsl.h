@@ -350,6 +350,40 @@ int natsl_kv_compact(const void* src_k, const void* src_v, long long src_tokens,
                      int HN, int K, int V, int dtype, int block, int NB, int n_complete, int tail_dst, int tail_tokens,
                      natsl_stream_t stream);
 
+/* The mixed operator's forward (src/nats/ops/mixed_ops/mixed_attn_gdn.py:47-191, src/nats/ops/mixed_ops/mixed_attn_mamba.py:51-192)
+ * in one call: natsl_route, natsl_softmax_sparse_fwd and natsl_gdn_chunk_fwd (is_delta) or natsl_mamba_chunk_fwd with the
+ * arguments those take, in bf16, and in front of and behind them the conversions of fp32 tensors (cast_in: fp32 -> bf16,
+ * cast_out: bf16 -> fp32; tensors on 16 bytes).  `phases` says which steps to enqueue, so that a caller can time them one by
+ * one.  attn_stream carries routing and the softmax branch: the same stream, or another one, which is then made to wait for
+ * `stream` before (at ROUTE) and waited for after (at JOIN).  The attention view may hold other lengths (a prefix of cached
+ * keys): T_attn tokens in TN_attn blocks. */
+#define NATSL_MIXED_CASTS 8
+enum natsl_mixed_phases { NATSL_MIXED_CONVERT = 1, NATSL_MIXED_ROUTE = 2, NATSL_MIXED_SOFTMAX = 4, NATSL_MIXED_LINEAR = 8, NATSL_MIXED_JOIN = 16 };
+typedef struct natsl_cast { const void* src; void* dst; int64_t n; } natsl_cast;
+typedef struct natsl_mixed {
+  int32_t is_delta, B, T, H, HN, K, V, TN, block, flags;
+  int32_t T_attn, TN_attn, HQ, HKV, KA, VA, same_block_visible, types_dtype;
+  int32_t n_seqs, total_chunks, total_qtiles, n_cast_in, n_cast_out, reserved;
+  float scale_attn, scale_linear;
+  const void *q_attn, *k_attn, *v_attn, *types_attn;
+  void* o_attn;
+  float* lse;
+  int32_t *block_indices, *n_blocks;
+  const void *q, *k, *v;
+  const float* g;
+  const void* beta;
+  const float* h0;
+  void* o;
+  float *ht, *h_block_start, *g_block_sum;
+  void *chunk_states, *chunk_v_new;
+  const void* types;
+  void* workspace;
+  size_t workspace_bytes;
+  const natsl_seq_row* seqs;
+  natsl_cast cast_in[NATSL_MIXED_CASTS], cast_out[NATSL_MIXED_CASTS];
+} natsl_mixed;
+int natsl_mixed_fwd(const natsl_mixed* m, int phases, natsl_stream_t stream, natsl_stream_t attn_stream);
+
 /* Decode: both operators of a step in one call and two launches -- what natsl_attn_masked_fwd and natsl_gdn_recurrent_fwd
  * (is_delta) or natsl_mamba_recurrent_fwd give on the same arguments, bf16, without the query-only form.  The attention runs
  * next to the recurrence and splits its keys over more workgroups; workspace of natsl_decode_workspace_bytes().

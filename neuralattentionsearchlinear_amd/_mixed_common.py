@@ -1,15 +1,38 @@
 """Shared host logic of the two mixed operators."""
 from __future__ import annotations
 
+import ctypes
 from typing import Optional
 
 import torch
 
 from . import _capi
-from .attns import parallel_attn_nats_fwd
-from .nats_util import CHUNK_SIZE, PackedSeqs, _seq_args, pack_sequences, route
+from .nats_util import CHUNK_SIZE, PackedSeqs, _seq_args, pack_sequences
 
 _attn_streams: dict = {}
+_cu_counts: dict = {}
+
+
+class _Cast(ctypes.Structure):
+    _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p), ("n", ctypes.c_int64)]
+
+
+_MAX_CASTS = 8
+_INTS = ("is_delta", "B", "T", "H", "HN", "K", "V", "TN", "block", "flags", "T_attn", "TN_attn", "HQ", "HKV", "KA", "VA", "same_block_visible",
+         "types_dtype", "n_seqs", "total_chunks", "total_qtiles", "n_cast_in", "n_cast_out", "reserved")
+_POINTERS = ("q_attn", "k_attn", "v_attn", "types_attn", "o_attn", "lse", "block_indices", "n_blocks", "q", "k", "v", "g", "beta", "h0", "o", "ht",
+             "h_block_start", "g_block_sum", "chunk_states", "chunk_v_new", "types", "workspace")
+
+
+class _Mixed(ctypes.Structure):
+    """natsl_mixed of include/natsl.h."""
+    _fields_ = ([(n, ctypes.c_int32) for n in _INTS] + [("scale_attn", ctypes.c_float), ("scale_linear", ctypes.c_float)] +
+                [(n, ctypes.c_void_p) for n in _POINTERS] +
+                [("workspace_bytes", ctypes.c_size_t), ("seqs", ctypes.c_void_p), ("cast_in", _Cast * _MAX_CASTS), ("cast_out", _Cast * _MAX_CASTS)])
+
+
+_CONVERT, _ROUTE, _SOFTMAX, _LINEAR, _JOIN = 1, 2, 4, 8, 16
+_ITEM_BYTES = {torch.bfloat16: 2, torch.float32: 4, torch.int32: 4, torch.uint8: 1}
 
 # Optional timing hook: when set to a callable(name, stream) it is invoked right before and right
 # after each branch is enqueued ("softmax:start", "softmax:end", "linear:start", "linear:end") so a
@@ -19,10 +42,13 @@ TIMING_HOOK = None
 # Where the softmax branch is launched.  True: on a side stream next to the linear branch (as the
 # reference's Mamba operator does); False: on the caller's stream, one branch after the other (as the
 # reference's GDN operator does); None: decide per call - side by side only when the linear branch's scan
-# cannot give every CU a workgroup even at its narrowest (one compute wave = 16 state columns per workgroup).
-# Both kernels take most of a CU's LDS (127 KiB / 159 KiB), so they never share a CU: when each fills the
-# machine alone, running them side by side gains nothing (measured) and only blurs timings.
+# cannot give every CU a workgroup even at its narrowest (one compute wave = 16 state columns per workgroup) and its chain is
+# long enough.  Both kernels take most of a CU's LDS (127 KiB / 159 KiB), so they never share a CU: when each fills the
+# machine alone, running them side by side gains nothing (measured) and only blurs timings.  Ordering two streams costs a call
+# about 40 us (36 us one after the other, 78 us side by side at T 256), which the overlap repays from a chain of 2048 tokens at
+# K = 128 on (4096 at K = 64): 87 -> 78 us at B1 T2048 H6, 154 -> 111 us at T 4096, but 56 -> 81 us at T 1024.
 CONCURRENT_BRANCHES = None
+_SIDE_BY_SIDE_TOKENS_X_K = 2048 * 128
 
 # What the differentiable operator keeps from its forward for the linear branch's backward.  Keeping means: the state entering
 # every chunk (bf16, K*V per chunk and head), v_new (64*V bf16) and the prep kernel's workspace (17 KiB) stay in device memory
@@ -38,10 +64,15 @@ _PREP_WORKSPACE_BYTES = 17 * 1024   # per chunk and head (csrc/natsl_linear.hip)
 _SCAN_COLUMNS_PER_WG = 16   # state columns of the scan's narrowest workgroup (csrc/natsl_linear.hip)
 
 
-def _run_side_by_side(dev, n_chains: int, V: int) -> bool:
+def _run_side_by_side(dev, n_chains: int, V: int, chain_tokens: int, K: int) -> bool:
     if CONCURRENT_BRANCHES is not None:
         return bool(CONCURRENT_BRANCHES)
-    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    if chain_tokens * K < _SIDE_BY_SIDE_TOKENS_X_K:
+        return False
+    index = dev.index if dev.index is not None else torch.cuda.current_device()
+    cus = _cu_counts.get(index)
+    if cus is None:
+        cus = _cu_counts[index] = torch.cuda.get_device_properties(index).multi_processor_count
     return n_chains * (V // _SCAN_COLUMNS_PER_WG) < cus
 
 
@@ -54,11 +85,6 @@ def _keep_chunk_states(q, v, cu_seqlens) -> bool:
     n_seq = B if cu_seqlens is None else len(cu_seqlens) - 1                     # (a host list here)
     chunks = -(-B * T // CHUNK_SIZE) + n_seq                       # upper bound on the chunks of all sequences
     return chunks * H * (2 * K * V + 2 * CHUNK_SIZE * V + _PREP_WORKSPACE_BYTES) <= SAVE_CHUNK_STATES_MAX_BYTES
-
-
-def _mark(name, stream):
-    if TIMING_HOOK is not None:
-        TIMING_HOOK(name, stream)
 
 
 def _get_attn_stream(device: torch.device) -> torch.cuda.Stream:
@@ -152,19 +178,76 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
     if io_dtype not in (torch.bfloat16, torch.float32):
         raise NotImplementedError(f"dtype {io_dtype} is not supported (bf16, or fp32 which is computed in bf16)")
 
-    def prep(t):
-        return None if t is None else t.detach().to(torch.bfloat16).contiguous()
+    m = _Mixed()
+    dev = q_lattn.device
+    # What only this call uses (conversions, routing tables, workspaces) lives in one allocation; what the backward keeps
+    # (return_aux) is made of tensors of its own.
+    scratch, total = [], 0
 
-    q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn, beta = map(prep, (q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn, beta))
+    def own(shape, dtype, set_pointer, hidden=True):
+        """A tensor of this call: a place in the scratch when nobody sees it afterwards (-> None), else a torch tensor."""
+        nonlocal total
+        if hidden and not return_aux:
+            scratch.append((set_pointer, total))
+            n = _ITEM_BYTES[dtype]
+            for d in shape:
+                n *= d
+            total += (n + 255) & ~255
+            return None
+        t = torch.empty(shape, dtype=dtype, device=dev)
+        set_pointer(t.data_ptr())
+        return t
+
+    copies = {}
+
+    def as_bf16(t, name):
+        """Names t (bf16, contiguous) in the call's arguments; an fp32 tensor's copy is filled by the call (one launch for all of
+        them).  -> the bf16 tensor, or t itself where its copy is in the scratch."""
+        if t is None:
+            return None
+        t = t.detach()
+        if t.dtype == torch.float32 and t.numel() > 0:
+            t = t.contiguous()
+            if t.data_ptr() % 16 == 0:
+                got = copies.get((t.data_ptr(), t.shape))
+                if got is None:
+                    c = m.cast_in[len(copies)]
+                    c.src, c.n = t.data_ptr(), t.numel()
+                    fields = [name]
+
+                    def point(at):
+                        c.dst = at
+                        for f in fields:
+                            setattr(m, f, at)
+                    got = copies[(t.data_ptr(), t.shape)] = (own(t.shape, torch.bfloat16, point, attn_prefix_valid is None), fields, t)
+                elif got[0] is None:
+                    got[1].append(name)
+                if got[0] is None:
+                    return t
+                setattr(m, name, got[0].data_ptr())
+                return got[0]
+        t = t if t.dtype == torch.bfloat16 else t.to(torch.bfloat16)
+        t = t.contiguous()
+        setattr(m, name, t.data_ptr())
+        return t
+
+    q_attn, k_attn, v_attn = as_bf16(q_attn, "q_attn"), as_bf16(k_attn, "k_attn"), as_bf16(v_attn, "v_attn")
+    q_lattn, k_lattn, v_lattn, beta = as_bf16(q_lattn, "q"), as_bf16(k_lattn, "k"), as_bf16(v_lattn, "v"), as_bf16(beta, "beta")
+    m.n_cast_in = len(copies)
     g = g.detach().to(torch.float32).contiguous()
     types = nats_block_types.detach()
     if types.dtype not in (torch.bfloat16, torch.float32):
         types = types.float()
     types = types.contiguous()
-    dev = q_lattn.device
-    T = q_lattn.shape[1]
+    B, T, H, K = q_lattn.shape
+    V = v_lattn.shape[-1]
+    if types.shape[-1] != 2:
+        raise NotImplementedError("routing is built for n_ops == 2")
+    TN, HN = types.shape[1], types.shape[2]
     seqs = pack_sequences(cu_seqlens, cu_seqlens_nats, nats_block_size, dev)
+    cur, L = _capi.stream_ptr(dev), _capi.lib()
 
+    n_prefix, types_attn = 0, types
     if attn_prefix_valid is not None:
         if not inference or seqs is not None:
             raise NotImplementedError("a key prefix is built for the prefill operators on unpacked input")
@@ -172,49 +255,92 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
         n_prefix = NP * nats_block_size
         if k_attn.shape[1] != q_attn.shape[1] + n_prefix or v_attn.shape[1] != k_attn.shape[1]:
             raise ValueError(f"with a prefix of {NP} blocks the keys must hold {q_attn.shape[1] + n_prefix} tokens, got {k_attn.shape[1]}")
+        if m.n_cast_in:                                   # the queries are put together below: their conversion comes first
+            _capi.check(L.natsl_mixed_fwd(ctypes.byref(m), _CONVERT, cur, cur), "natsl_mixed_fwd")
+            m.n_cast_in = 0
         pv = attn_prefix_valid.to(types.dtype)
         types_attn = torch.cat([torch.stack([pv, 1 - pv], -1), types], 1).contiguous()
         q_attn = torch.cat([q_attn.new_zeros(q_attn.shape[0], n_prefix, *q_attn.shape[2:]), q_attn], 1)
-        r = route(types_attn, T + n_prefix, nats_block_size, None)
-    else:
-        n_prefix, types_attn = 0, types
-        r = route(types, T, nats_block_size, seqs)
-    cur = torch.cuda.current_stream(dev)
-    n_chains = (seqs.n_seqs if seqs is not None else q_lattn.shape[0]) * q_lattn.shape[2]
-    side = _get_attn_stream(dev) if _run_side_by_side(dev, n_chains, v_lattn.shape[-1]) else cur
-    if side is not cur:
-        side.wait_stream(cur)
-    with torch.cuda.stream(side):
-        _mark("softmax:start", side)
-        o_attn, _lse, _ = parallel_attn_nats_fwd(
-            q_attn, k_attn, v_attn, types_attn, r['nats_block_indices'], None, scale_attn, nats_block_size,
-            compute_incomplete_chunk_scores=attn_same_block, n_nats_blocks=r['n_nats_blocks'], seqs=seqs)
-        if n_prefix:
-            o_attn = o_attn[:, n_prefix:]
-        _mark("softmax:end", side)
-    flags = (_capi.DECAY_NON_LINEAR if decay_non_linear else 0) | (_capi.QK_L2NORM if qk_l2norm else 0) | \
-            (_capi.INTRA_CHUNK if lin_intra else 0)
-    _mark("linear:start", cur)
+        m.q_attn = q_attn.data_ptr()
+    T_attn, HQ, KA = q_attn.shape[1:]
+    HKV, VA = k_attn.shape[2], v_attn.shape[3]
+
+    n_seqs = seqs.n_seqs if seqs is not None else B
+    total_chunks = seqs.total_chunks if seqs is not None else B * (-(-T // CHUNK_SIZE))
+    # every tensor below belongs to the caller's stream; the softmax branch's stream starts after what that stream holds and is
+    # waited for before the call returns, so memory that is freed later is only ever used again behind both
+    side = _get_attn_stream(dev) if _run_side_by_side(dev, n_seqs * H, V, T * B // n_seqs, K) else None
+    attn_stream = cur if side is None else side.cuda_stream
     want_start = inference and output_final_state
-    res = linear_chunk_fwd(kind, q_lattn, k_lattn, v_lattn, g, beta, initial_state, types, scale_lattn,
-                           nats_block_size, flags, output_final_state, seqs, block_start_state=want_start,
-                           chunk_states=keep_chunk_states and not want_start)
-    o_lin, ht = res[0], res[1]
-    _mark("linear:end", cur)
-    if side is not cur:
-        cur.wait_stream(side)
-        # tensors allocated on the caller's stream and read on the side stream, and the side stream's own output
-        # that the caller's stream goes on to use
-        for t in (q_attn, k_attn, v_attn, types_attn, r['nats_block_indices'], r['n_nats_blocks']):
-            t.record_stream(side)
-        o_attn.record_stream(cur)
-        _lse.record_stream(cur)
-    if io_dtype != torch.bfloat16:
-        o_lin, o_attn = o_lin.to(io_dtype), o_attn.to(io_dtype)
+    chunk_states = keep_chunk_states and not want_start
+    bf16, f32 = torch.bfloat16, torch.float32
+    point = lambda name: lambda at: setattr(m, name, at)
+    ws_bytes = L.natsl_linear_workspace_bytes(total_chunks, H)
+    idx = own((B, types_attn.shape[1], HN, 2), torch.int32, point("block_indices"))
+    nblk = own((n_seqs, HN, 2), torch.int32, point("n_blocks"))
+    lse = own((B, T_attn, HQ), f32, point("lse"))
+    ws = own((ws_bytes,), torch.uint8, point("workspace"))
+    o_attn = torch.empty(B, T_attn, HQ, VA, dtype=io_dtype, device=dev)
+    o_lin = torch.empty(B, T, H, V, dtype=io_dtype, device=dev)
+    o_attn16, o_lin16 = o_attn, o_lin
+    if io_dtype == bf16:
+        m.o_attn, m.o = o_attn.data_ptr(), o_lin.data_ptr()
+    else:
+        def out(c, name, dst):
+            c.dst, c.n = dst.data_ptr(), dst.numel()
+
+            def set_both(at):
+                c.src = at
+                setattr(m, name, at)
+            return own(dst.shape, bf16, set_both)
+        o_attn16, o_lin16 = out(m.cast_out[0], "o_attn", o_attn), out(m.cast_out[1], "o", o_lin)
+        m.n_cast_out = 2
+    ht = torch.empty(n_seqs, H, K, V, dtype=f32, device=dev) if output_final_state else None
+    hs = torch.empty(n_seqs, H, K, V, dtype=f32, device=dev) if want_start else None
+    gs = torch.empty(n_seqs, H, dtype=f32, device=dev) if want_start else None
+    sc = torch.empty(total_chunks, H, V, K, dtype=bf16, device=dev) if chunk_states else None
+    vn = torch.empty_like(v_lattn) if chunk_states and kind == 'gdn' else None
+    if scratch:
+        block = torch.empty(total, dtype=torch.uint8, device=dev)
+        base = block.data_ptr()
+        for set_pointer, at in scratch:
+            set_pointer(base + at)
+    h0 = None
+    if initial_state is not None:
+        if tuple(initial_state.shape) != (n_seqs, H, K, V):
+            raise ValueError(f"initial state must have shape {(n_seqs, H, K, V)}, got {tuple(initial_state.shape)}")
+        h0 = initial_state.detach().to(f32).contiguous()
+    m.is_delta, m.B, m.T, m.H, m.HN, m.K, m.V, m.TN, m.block = int(kind == 'gdn'), B, T, H, HN, K, V, TN, nats_block_size
+    m.flags = (_capi.DECAY_NON_LINEAR if decay_non_linear else 0) | (_capi.QK_L2NORM if qk_l2norm else 0) | (_capi.INTRA_CHUNK if lin_intra else 0)
+    m.T_attn, m.TN_attn, m.HQ, m.HKV, m.KA, m.VA = T_attn, types_attn.shape[1], HQ, HKV, KA, VA
+    m.same_block_visible, m.types_dtype = int(attn_same_block), _capi.dtype_code(types.dtype)
+    m.scale_attn, m.scale_linear = scale_attn, scale_lattn
+    if seqs is not None:
+        m.seqs, m.n_seqs, m.total_chunks, m.total_qtiles = seqs.table.data_ptr(), seqs.n_seqs, seqs.total_chunks, seqs.total_qtiles
+    m.g, m.types, m.types_attn, m.workspace_bytes = g.data_ptr(), types.data_ptr(), types_attn.data_ptr(), ws_bytes
+    for name, t in (("h0", h0), ("ht", ht), ("h_block_start", hs), ("g_block_sum", gs), ("chunk_states", sc), ("chunk_v_new", vn)):
+        if t is not None:
+            setattr(m, name, t.data_ptr())
+    ref = ctypes.byref(m)
+    if TIMING_HOOK is None:
+        _capi.check(L.natsl_mixed_fwd(ref, _CONVERT | _ROUTE | _SOFTMAX | _LINEAR | _JOIN, cur, attn_stream), "natsl_mixed_fwd")
+    else:
+        here = torch.cuda.current_stream(dev)
+        step = lambda phases: _capi.check(L.natsl_mixed_fwd(ref, phases, cur, attn_stream), "natsl_mixed_fwd")
+        step(_CONVERT | _ROUTE)
+        TIMING_HOOK("softmax:start", here if side is None else side)
+        step(_SOFTMAX)
+        TIMING_HOOK("softmax:end", here if side is None else side)
+        TIMING_HOOK("linear:start", here)
+        step(_LINEAR)
+        TIMING_HOOK("linear:end", here)
+        step(_JOIN)
+    if n_prefix:
+        o_attn = o_attn[:, n_prefix:]
     if return_aux:
         aux = dict(q_attn=q_attn, k_attn=k_attn, v_attn=v_attn, q_lattn=q_lattn, k_lattn=k_lattn, v_lattn=v_lattn, beta=beta, g=g,
-                   types=types, lse=_lse, nats_block_indices=r['nats_block_indices'], n_nats_blocks=r['n_nats_blocks'],
-                   linear_saved=tuple(res[2:5]) if keep_chunk_states and not want_start else None)
+                   types=types, lse=lse, nats_block_indices=idx, n_nats_blocks=nblk, o_attn=o_attn16,
+                   linear_saved=(sc, vn if kind == 'gdn' else v_lattn, ws) if chunk_states else None)
         return o_lin, o_attn, ht, aux
     if not inference:
         return o_lin, o_attn, ht
@@ -224,7 +350,6 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
         # with an incomplete last block it is the state that entered that block; when the input ends on
         # a block boundary it is the state after the last block under its TRUE type -- the final state
         # if that type is linear, otherwise the entering state rolled forward by the block's decay.
-        hs, gs = res[2], res[3]
         if T % nats_block_size != 0:
             h_start = hs
         else:
@@ -261,7 +386,7 @@ class _MixedFunction(torch.autograd.Function):
         ctx.has_h0 = initial_state is not None
         saved = [aux[n] for n in ('q_attn', 'k_attn', 'v_attn', 'q_lattn', 'k_lattn', 'v_lattn', 'g', 'types', 'lse',
                                   'nats_block_indices', 'n_nats_blocks')]
-        saved += [o_attn.to(torch.bfloat16), aux['beta'] if aux['beta'] is not None else g.new_zeros(0),
+        saved += [aux['o_attn'], aux['beta'] if aux['beta'] is not None else g.new_zeros(0),
                   initial_state if initial_state is not None else g.new_zeros(0)]
         ctx.n_linear_saved = 0
         if aux['linear_saved'] is not None:

@@ -1032,8 +1032,8 @@ template <int DK, bool DELTA, int NW, bool PF, int NF = 0>
 static int launch_scan(const LinearParams& p, hipStream_t stream, const char* what) {
   using L = ScanLds<DK, NW, PF, PF && DELTA>;
   auto kern = linear_scan_kernel<DK, DELTA, NW, PF, NF>;
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, L::TOTAL);
-  if (e != hipSuccess) return fail(NATSL_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS: %s", what, L::TOTAL, hipGetErrorString(e));
+  static std::atomic<unsigned long long> reserved{0};
+  if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, L::TOTAL, what)) return rc;
   const int n_chains = (p.seqs ? p.n_seqs : p.B) * p.H;
   const int grid = 8 * cdiv(n_chains, 8) * (p.V / L::BVW);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * (NW + 2 + NF)), L::TOTAL, stream, p);

@@ -1115,8 +1115,8 @@ template <int DK, bool DELTA, int NW>
 static int launch_bwd_scan(const LinBwdParams& p, hipStream_t stream, const char* what) {
   using L = BwdScanLds<DK, NW>;
   auto kern = linear_bwd_scan_kernel<DK, DELTA, NW>;
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, L::TOTAL);
-  if (e != hipSuccess) return fail(NATSL_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS: %s", what, L::TOTAL, hipGetErrorString(e));
+  static std::atomic<unsigned long long> reserved{0};
+  if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, L::TOTAL, what)) return rc;
   const int n_chains = (p.seqs ? p.n_seqs : p.B) * p.H;
   hipLaunchKernelGGL(kern, dim3((unsigned)((n_chains + 7) / 8 * 8 * (p.V / (16 * NW)))), dim3(L::THREADS), L::TOTAL, stream, p);
   return check_launch(what);
@@ -1136,8 +1136,8 @@ static int launch_bwd(const LinBwdParams& p, hipStream_t stream, const char* wha
   {
     using L = BwdChunkLds<DK>;
     auto kern = linear_bwd_chunk_kernel<DK, DELTA>;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, L::TOTAL);
-    if (e != hipSuccess) return fail(NATSL_ERR_LAUNCH, "%s: cannot reserve %d bytes of LDS: %s", what, L::TOTAL, hipGetErrorString(e));
+    static std::atomic<unsigned long long> reserved{0};
+    if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, L::TOTAL, what)) return rc;
     hipLaunchKernelGGL(kern, dim3((unsigned)(p.total_chunks * p.H)), dim3(256), L::TOTAL, stream, p);
     return check_launch(what);
   }

@@ -1,0 +1,124 @@
+// The mixed operator's forward as one native call: dtype conversions, routing, the softmax branch and the linear branch, on one
+// stream or with the softmax branch on a second one.  At small sizes the operator's cost is launches and the host that issues
+// them (fp32 B1 T256 H2: 60 us of kernels behind 200 us of host time as separate calls with torch conversions), so all tensor
+// conversions of a side go out as one launch and nothing returns to the interpreter in between.
+#include <mutex>
+
+#include "natsl_device.h"
+#include "natsl_host.h"
+
+namespace natsl {
+
+// ---- fp32 <-> bf16 copies of several tensors in one launch: 2048 elements per workgroup, 8 per thread -----------------------
+struct CastSet {
+  natsl_cast seg[NATSL_MIXED_CASTS];
+  unsigned first[NATSL_MIXED_CASTS + 1];   // the segments' first workgroups
+  int n;
+};
+
+template <bool TO_BF16>
+__global__ __launch_bounds__(256) void cast_kernel(const CastSet p) {
+  int s = 0;
+#pragma unroll
+  for (int i = 1; i < NATSL_MIXED_CASTS; ++i) s = i < p.n && blockIdx.x >= p.first[i] ? i : s;
+  const natsl_cast c = p.seg[s];
+  const long long at = (long long)(blockIdx.x - p.first[s]) * 2048 + 8 * threadIdx.x;
+  if (at >= c.n) return;
+  if (at + 8 <= c.n) {
+    if constexpr (TO_BF16) {
+      const float* src = reinterpret_cast<const float*>(c.src) + at;
+      const f32x4 a = *reinterpret_cast<const f32x4*>(src), b = *reinterpret_cast<const f32x4*>(src + 4);
+      *reinterpret_cast<bf16x8*>(reinterpret_cast<bf16_t*>(c.dst) + at) = pack8(a, b);
+    } else {
+      const u32x4 w = *reinterpret_cast<const u32x4*>(reinterpret_cast<const bf16_t*>(c.src) + at);
+      float* dst = reinterpret_cast<float*>(c.dst) + at;
+      *reinterpret_cast<f32x4*>(dst) = (f32x4){__uint_as_float(w[0] << 16), __uint_as_float(w[0] & 0xffff0000u), __uint_as_float(w[1] << 16), __uint_as_float(w[1] & 0xffff0000u)};
+      *reinterpret_cast<f32x4*>(dst + 4) = (f32x4){__uint_as_float(w[2] << 16), __uint_as_float(w[2] & 0xffff0000u), __uint_as_float(w[3] << 16), __uint_as_float(w[3] & 0xffff0000u)};
+    }
+  } else {
+    for (long long i = at; i < c.n; ++i) {
+      if constexpr (TO_BF16) reinterpret_cast<bf16_t*>(c.dst)[i] = f32_to_bf16(reinterpret_cast<const float*>(c.src)[i]);
+      else reinterpret_cast<float*>(c.dst)[i] = bf16_to_f32(reinterpret_cast<const bf16_t*>(c.src)[i]);
+    }
+  }
+}
+
+template <bool TO_BF16>
+static int cast_all(const natsl_cast* seg, int n, hipStream_t s, const char* what) {
+  if (n <= 0) return NATSL_OK;
+  CastSet p;
+  p.n = n;
+  long long wgs = 0;
+  for (int i = 0; i < NATSL_MIXED_CASTS; ++i) {
+    if (i < n) {
+      if (!seg[i].src || !seg[i].dst || seg[i].n <= 0) return fail(NATSL_ERR_INVALID, "%s: bad conversion segment", what);
+      if (((uintptr_t)seg[i].src | (uintptr_t)seg[i].dst) & 15) return fail(NATSL_ERR_INVALID, "%s: converted tensors must start on 16 bytes", what);
+      p.seg[i] = seg[i];
+    }
+    p.first[i] = (unsigned)wgs;
+    if (i < n) wgs += (seg[i].n + 2047) / 2048;
+  }
+  p.first[NATSL_MIXED_CASTS] = (unsigned)wgs;
+  if (wgs > 0x7fffffffll) return fail(NATSL_ERR_UNSUPPORTED, "%s: too much to convert", what);
+  hipLaunchKernelGGL((cast_kernel<TO_BF16>), dim3((unsigned)wgs), dim3(256), 0, s, p);
+  return check_launch(what);
+}
+
+// `to` waits for what `from` holds so far.  One event per device; a wait takes the event's state at the call, so the pair is
+// made under a lock and the event can serve the next pair at once.
+static int order_streams(hipStream_t from, hipStream_t to, const char* what) {
+  constexpr int MAX_DEVICES = 64;
+  static hipEvent_t events[MAX_DEVICES];
+  static std::mutex mu;
+  int dev = -1;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return fail(NATSL_ERR_LAUNCH, "%s: cannot name the current device (%s)", what, hipGetErrorString(e));
+  std::lock_guard<std::mutex> lock(mu);
+  if (!events[dev]) e = hipEventCreateWithFlags(&events[dev], hipEventDisableTiming);
+  if (e == hipSuccess) e = hipEventRecord(events[dev], from);
+  if (e == hipSuccess) e = hipStreamWaitEvent(to, events[dev], 0);
+  return e == hipSuccess ? NATSL_OK : fail(NATSL_ERR_LAUNCH, "%s: cannot order the streams (%s)", what, hipGetErrorString(e));
+}
+
+}  // namespace natsl
+
+using namespace natsl;
+
+extern "C" int natsl_mixed_fwd(const natsl_mixed* m, int phases, natsl_stream_t stream, natsl_stream_t attn_stream) {
+  const char* what = "natsl_mixed_fwd";
+  if (!m) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
+  if (m->n_cast_in < 0 || m->n_cast_in > NATSL_MIXED_CASTS || m->n_cast_out < 0 || m->n_cast_out > NATSL_MIXED_CASTS)
+    return fail(NATSL_ERR_INVALID, "%s: conversion counts", what);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream), side = reinterpret_cast<hipStream_t>(attn_stream);
+  const bool fork = side != s;
+  int rc = NATSL_OK;
+  if ((phases & NATSL_MIXED_CONVERT) && (rc = cast_all<true>(m->cast_in, m->n_cast_in, s, what)) != NATSL_OK) return rc;
+  if (phases & NATSL_MIXED_ROUTE) {
+    if (fork && (rc = order_streams(s, side, what)) != NATSL_OK) return rc;
+    rc = natsl_route(m->types_attn, m->types_dtype, m->B, m->TN_attn, m->HN, m->T_attn, m->block, m->block_indices, m->n_blocks, nullptr, nullptr,
+                     nullptr, nullptr, m->seqs, m->n_seqs, 0, attn_stream);
+    if (rc != NATSL_OK) return rc;
+  }
+  if (phases & NATSL_MIXED_SOFTMAX) {
+    rc = natsl_softmax_sparse_fwd(m->q_attn, m->k_attn, m->v_attn, m->o_attn, m->lse, m->types_attn, m->types_dtype, m->block_indices,
+                                  m->n_blocks, m->B, m->T_attn, m->HQ, m->HKV, m->HN, m->KA, m->VA, m->TN_attn, m->block, m->scale_attn,
+                                  m->same_block_visible, NATSL_BF16, m->seqs, m->n_seqs, m->total_qtiles, attn_stream);
+    if (rc != NATSL_OK) return rc;
+  }
+  if (phases & NATSL_MIXED_LINEAR) {
+    if (m->is_delta)
+      rc = natsl_gdn_chunk_fwd(m->q, m->k, m->v, m->g, m->beta, m->h0, m->o, m->ht, m->h_block_start, m->g_block_sum, m->chunk_states,
+                               m->chunk_v_new, m->types, m->types_dtype, m->B, m->T, m->H, m->HN, m->K, m->V, m->TN, m->block, m->scale_linear,
+                               m->flags, m->workspace, m->workspace_bytes, NATSL_BF16, m->seqs, m->n_seqs, m->total_chunks, stream);
+    else
+      rc = natsl_mamba_chunk_fwd(m->q, m->k, m->v, m->g, m->h0, m->o, m->ht, m->h_block_start, m->g_block_sum, m->chunk_states, m->types,
+                                 m->types_dtype, m->B, m->T, m->H, m->HN, m->K, m->V, m->TN, m->block, m->scale_linear, m->flags, m->workspace,
+                                 m->workspace_bytes, NATSL_BF16, m->seqs, m->n_seqs, m->total_chunks, stream);
+    if (rc != NATSL_OK) return rc;
+  }
+  if (phases & NATSL_MIXED_JOIN) {
+    if (fork && (rc = order_streams(side, s, what)) != NATSL_OK) return rc;
+    rc = cast_all<false>(m->cast_out, m->n_cast_out, s, what);
+  }
+  return rc;
+}

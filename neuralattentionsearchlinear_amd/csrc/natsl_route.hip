@@ -157,19 +157,25 @@ __global__ __launch_bounds__(256) void route_kernel(const void* types, int dtype
     ca += rintf(load_as_f32(types, dtype, i)) == 1.f;
     cl += rintf(load_as_f32(types, dtype, i + 1)) == 1.f;
   }
-  __shared__ int sa[257], sl[257];
-  sa[threadIdx.x + 1] = ca;
-  sl[threadIdx.x + 1] = cl;
-  if (threadIdx.x == 0) sa[0] = sl[0] = 0;
+  // exclusive prefix of the segment counts: shuffles inside a wave, the four waves' totals through LDS (one thread walking the
+  // 256 counts was most of the launch: 8 us, 3 without)
+  __shared__ int wa[4], wl[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int ia = ca, il = cl;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int ua = __shfl_up(ia, d), ul = __shfl_up(il, d);
+    if (lane >= d) { ia += ua; il += ul; }
+  }
+  if (lane == 63) { wa[wave] = ia; wl[wave] = il; }
   __syncthreads();
-  if (threadIdx.x == 0)
-    for (int i = 1; i <= 256; ++i) {
-      sa[i] += sa[i - 1];
-      sl[i] += sl[i - 1];
-    }
-  __syncthreads();
-  int ra = sa[threadIdx.x], rl = sl[threadIdx.x];
-  const int na = sa[256], nl = sl[256];
+  int ra = ia - ca, rl = il - cl, na = 0, nl = 0;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    if (w < wave) { ra += wa[w]; rl += wl[w]; }
+    na += wa[w];
+    nl += wl[w];
+  }
   for (int c = lo; c < hi; ++c) {
     const size_t i = ((size_t)(bos_nats + c) * HN + hn) * 2;
     pa[c] = ra;

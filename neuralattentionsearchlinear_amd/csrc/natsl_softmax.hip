@@ -1444,19 +1444,6 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
 
 }
 
-// The LDS reservation of a kernel is an attribute of the function per device: set when a device first runs it.
-static int reserve_lds(const void* kern, std::atomic<unsigned long long>& done, size_t lds) {
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return fail(NATSL_ERR_LAUNCH, "softmax: cannot name the current device (%s)", hipGetErrorString(e));
-  const unsigned long long bit = 1ull << (dev & 63);
-  if (dev < 64 && (done.load(std::memory_order_acquire) & bit)) return NATSL_OK;
-  e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return fail(NATSL_ERR_LAUNCH, "softmax: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
-  if (dev < 64) done.fetch_or(bit, std::memory_order_release);
-  return NATSL_OK;
-}
-
 template <int DK, int DV, int NWAVES>
 static int launch_softmax(const SoftmaxParams& p, hipStream_t stream) {
   constexpr int KP = DK + 8, VP = DV + 8, QTILE = 32 * NWAVES;
@@ -1467,7 +1454,7 @@ static int launch_softmax(const SoftmaxParams& p, hipStream_t stream) {
   if (NWAVES == 8 && ring > lds) lds = ring;
   auto kern = softmax_sparse_fwd_kernel<DK, DV, NWAVES>;
   static std::atomic<unsigned long long> reserved{0};
-  if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, lds)) return rc;
+  if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, lds, "softmax")) return rc;
   const long long grid = p.seqs ? (long long)p.total_tiles * (QTILE_TABLE / QTILE) * p.HQ
                                 : (long long)8 * ((p.B * p.HQ + 7) / 8) * ((p.T + QTILE - 1) / QTILE);
   if (grid <= 0) return NATSL_OK;
@@ -1528,7 +1515,7 @@ static int launch_softmax_stream(const SoftmaxParams& p, const StreamDevice* d, 
   static std::atomic<unsigned long long> reserved{0};
   const size_t lds = ((size_t)4 * 64 * DK + (size_t)2 * 64 * DV + (size_t)3 * DV * VTP) * sizeof(bf16_t) + 1024;
   auto kern = softmax_stream_kernel<DK, DV>;
-  if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, lds)) return rc;
+  if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, lds, "softmax")) return rc;
   unsigned* queue = d->queues + (size_t)(launches.fetch_add(1) % STREAM_SLOTS) * STREAM_SLOT_WORDS;
   hipLaunchKernelGGL(stream_queue_clear_kernel, dim3(1), dim3(64), 0, stream, queue);
   hipLaunchKernelGGL(kern, dim3((unsigned)d->cus), dim3(512), lds, stream, p, queue);

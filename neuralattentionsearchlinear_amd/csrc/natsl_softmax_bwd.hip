@@ -832,16 +832,16 @@ static int launch_bwd(const SoftmaxBwdParams& p, hipStream_t stream) {
   {
     size_t lds = (size_t)2 * 64 * (KP + VP) * sizeof(bf16_t);
     auto kern = dq_kernel<DK, DV>;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return fail(NATSL_ERR_LAUNCH, "softmax bwd: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
+    static std::atomic<unsigned long long> reserved{0};
+    if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, lds, "softmax bwd")) return rc;
     const long long grid = p.seqs ? (long long)p.total_tiles * 2 * p.HQ : ((long long)p.B * p.HQ + 7) / 8 * 8 * ((p.T + 127) / 128);
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, stream, p);
   }
   {
     const size_t lds = DkdvLds<DK, DV>::TOTAL;   // the ring of three query tiles and the exchange buffers
     auto kern = dkdv_kernel<DK, DV>;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return fail(NATSL_ERR_LAUNCH, "softmax bwd: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
+    static std::atomic<unsigned long long> reserved{0};
+    if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, lds, "softmax bwd")) return rc;
     const long long units = p.seqs ? (long long)p.total_chunks * p.HKV : (long long)p.B * p.HKV * ((p.T + 63) / 64);
     long long grid = (cu_count() + 7) / 8 * 8;   // whole groups of 8: block index mod 8 names the XCD and its queue
     if (grid > units) grid = units;

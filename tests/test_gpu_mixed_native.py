@@ -1,0 +1,51 @@
+"""The mixed operator's one native call: fp32 tensors converted inside it give what tensors rounded beforehand give, bit for bit, at
+sizes where a conversion segment ends inside a thread's eight elements or a workgroup's 2048; and both placements of the softmax
+branch (same stream, side stream) agree."""
+import pytest
+import torch
+
+from tests._util import make_gates, make_qkv, make_types
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda:0'
+
+
+def _case(kind, B, T, H, K, V, seed):
+    q, k, v = make_qkv(B, T, H, K, V, seed, torch.float32)
+    g, beta = make_gates(B, T, H, seed + 1, torch.float32)
+    ty = make_types(B, -(-T // 64), H, 0.4, seed + 2)
+    return [t.to(DEV) for t in (q, k, v, g, beta, ty)]
+
+
+def _run(kind, q, k, v, g, beta, ty):
+    from neuralattentionsearchlinear_amd.mixed_attn_gdn import nats_mixed_attn_gdn
+    from neuralattentionsearchlinear_amd.mixed_attn_mamba import nats_mixed_attn_mamba
+    if kind == 'gdn':
+        return nats_mixed_attn_gdn(q, k, v, q, k, v, None, g, beta, ty, None, ops_for_incomplete_chunks='all',
+                                   output_final_state_gated_delta=True, decay_for_non_gdn_blocks=True)
+    return nats_mixed_attn_mamba(q, k, v, q, k, v, None, g, ty, None, output_final_state_mamba=True, decay_for_non_mamba_blocks=True)
+
+
+@pytest.mark.parametrize("kind,B,T,H,K,V", [('gdn', 1, 1, 1, 64, 64), ('gdn', 1, 67, 3, 64, 64), ('gdn', 2, 129, 5, 128, 128), ('mamba', 1, 100, 3, 128, 64)])
+@pytest.mark.parametrize("grad", [False, True])
+def test_fp32_tensors_equal_rounded_tensors(kind, B, T, H, K, V, grad):
+    q, k, v, g, beta, ty = _case(kind, B, T, H, K, V, T)
+    r16 = lambda t: t.bfloat16()
+    if grad:                                              # the differentiable operator keeps its copies as tensors of their own
+        q.requires_grad_(True)
+    out = _run(kind, q, k, v, g, beta, ty)
+    ref = _run(kind, r16(q.detach()), r16(k), r16(v), g, r16(beta), ty)
+    for name, a, b in zip(("o_linear", "o_attn", "state"), out, ref):
+        assert a.dtype == torch.float32
+        assert torch.equal(a.detach(), b.float()), name
+
+
+@pytest.mark.parametrize("kind,H,K,V", [('gdn', 2, 64, 64), ('mamba', 3, 128, 64)])
+def test_side_stream_and_one_stream_agree(kind, H, K, V, monkeypatch):
+    import neuralattentionsearchlinear_amd._mixed_common as MC
+    q, k, v, g, beta, ty = _case(kind, 1, 500, H, K, V, 9)
+    outs = []
+    for side in (False, True):
+        monkeypatch.setattr(MC, 'CONCURRENT_BRANCHES', side)
+        outs.append(_run(kind, q, k, v, g, beta, ty))
+    assert all(torch.equal(a, b) for a, b in zip(*outs))

@@ -235,6 +235,15 @@ int natsl_norm_gate_bwd(const void* x1, const void* x2, const void* gate, const 
                         float* dw2, void* workspace, size_t workspace_bytes, int64_t rows, int D, int dtype, float eps,
                         int w_dtype, natsl_stream_t stream);
 
+/* The same with the two mixing weights of a row given as logits (bf16): x_weights = softmax(x_logits) rounded to bf16, and the
+ * gradient comes back for the logits (bf16) -- the mixing layer's softmax (src/nats/layers/natsl_attn_gdn.py:492-494) without a pass
+ * of its own. */
+int natsl_norm_gate_logits_fwd(const void* x1, const void* x2, const void* gate, const void* x_logits, const void* w1, const void* w2, void* y,
+                               int64_t rows, int D, int dtype, float eps, int w_dtype, natsl_stream_t stream);
+int natsl_norm_gate_logits_bwd(const void* x1, const void* x2, const void* gate, const void* x_logits, const void* w1, const void* w2,
+                               const void* dy, void* dx1, void* dx2, void* dgate, void* dx_logits, float* dw1, float* dw2, void* workspace,
+                               size_t workspace_bytes, int64_t rows, int D, int dtype, float eps, int w_dtype, natsl_stream_t stream);
+
 /* Layer glue, depthwise causal short convolution with its activation, on the layer's token-major tensors:
  * y[b,t,d] = act(bias[d] + sum_j w[d,j] e[b, t-(W-1)+j, d]) where e is x preceded by the W-1 inputs before it: the last
  * W-1 entries of `state` [B,D,W] (the cache of a previous call, in `state_dtype`), or zeros when state is NULL.
@@ -349,6 +358,57 @@ int natsl_kv_compact(const void* src_k, const void* src_v, long long src_tokens,
                      long long dst_tokens, const void* types, int types_dtype, const int64_t* n_before, int B, int HKV,
                      int HN, int K, int V, int dtype, int block, int NB, int n_complete, int tail_dst, int tail_tokens,
                      natsl_stream_t stream);
+
+/* The layers' short convolutions with what follows them, for up to NATSL_CONV_SEGS bf16 tensors [B, T, D_i] in one launch:
+ *   y = act(conv(x)) (as natsl_short_conv_fwd; bf16 weights [D, W]), and, when y_norm is given, its rows of 8 * norm_lanes
+ *   channels (a power of two of lanes) normalised: y rsqrt(mean y^2 + eps) norm_weight, or y rsqrt(sum y^2 + eps) (norm_l2).
+ * The backward takes the gradients that meet at y (dy_a, dy_b, and dy_norm through the norm; each may be NULL) and one that
+ * meets at x (dx_add), and gives dx, dweight, dbias (bf16) and dnorm_weight (norm_dtype); sums in a fixed order.
+ * Takes the place of natsl_short_conv_* and natsl_row_norm_* inside the layers (src/nats/layers/natsl_attn_gdn.py:425-505). */
+#define NATSL_CONV_SEGS 3
+typedef struct natsl_conv_seg {
+  const void *x, *weight, *bias, *state, *norm_weight;
+  void *y, *y_norm, *state_out;
+  const void *dy_a, *dy_b, *dy_norm, *dx_add;
+  void *dx, *dweight, *dbias, *dnorm_weight;
+  int32_t D, norm_lanes, norm_l2;
+  float norm_eps;
+} natsl_conv_seg;
+int natsl_conv_norm_fwd(const natsl_conv_seg* seg, int n_seg, int B, int T, int W, int activation, int norm_dtype, natsl_stream_t stream);
+size_t natsl_conv_norm_bwd_workspace_bytes(const natsl_conv_seg* seg, int n_seg, int B, int T, int W);
+int natsl_conv_norm_bwd(const natsl_conv_seg* seg, int n_seg, int B, int T, int W, int activation, int norm_dtype, void* workspace,
+                        size_t workspace_bytes, natsl_stream_t stream);
+
+/* The layers' gates from one projection ab [rows, ld] (bf16; a in columns 0..H-1, b in H..2H-1 for the delta rule):
+ * g = -exp(a_log) softplus(a + dt_bias) fp32 [rows, H], beta = sigmoid(b) bf16 (doubled with neg_eigval; NULL for Mamba),
+ * dt = softplus(a + dt_bias) fp32 (or NULL); and the gradients (dab has zeros behind the used columns).
+ * src/nats/layers/natsl_attn_gdn.py:507-512, src/nats/layers/natsl_attn_mamba2.py:391-393. */
+int natsl_gates_fwd(const void* ab, const void* a_log, const void* dt_bias, float* g, void* beta, float* dt, int64_t rows, int H, int ld,
+                    int neg_eigval, int param_dtype, natsl_stream_t stream);
+size_t natsl_gates_bwd_workspace_bytes(int64_t rows, int H);
+int natsl_gates_bwd(const void* ab, const void* a_log, const void* dt_bias, const float* dg, const void* dbeta, const float* ddt, int delta,
+                    void* dab, void* da_log, void* ddt_bias, void* workspace, size_t workspace_bytes, int64_t rows, int H, int ld,
+                    int neg_eigval, int param_dtype, natsl_stream_t stream);
+
+/* dx [B, T, D] = dn [B*T, ld] w [N, D] (N a multiple of 16, 0 = none) + the block mean's gradient dpool [B, ceil(T/block), D] (or
+ * NULL) over the block's length, bf16: the terms of a layer's input gradient that are no wide product. */
+int natsl_dx_init(const void* dn, const void* w, const void* dpool, void* dx, int B, int T, int D, int N, int ld, int block,
+                  natsl_stream_t stream);
+
+/* Straight-through gradient of natsl_hard_select: the softmax's backward of dtypes, [B, TN, HN, 2] in one dtype; last_forced:
+ * the last block's types were constants (src/nats/layers/natsl_attn_gdn.py:47-61, :553-554). */
+int natsl_hard_select_bwd(const void* logits, const void* dtypes, void* dlogits, int B, int TN, int HN, int dtype, int last_forced,
+                          natsl_stream_t stream);
+
+/* Weight gradients of up to NATSL_WGRAD_SEGS projections that share their input: out_i [n_i, D] = dy_i^T x, bf16, sums in fp32;
+ * dy_i [T, ld_i] (n_i columns used), x [T, ldx] (D columns used); widths and row strides are multiples of 8, dy and x start on
+ * 16 bytes.  Deterministic.  Takes the place of the library products in the backward of the layers' projections
+ * (src/nats/layers/natsl_attn_gdn.py:425-491). */
+#define NATSL_WGRAD_SEGS 8
+typedef struct natsl_wgrad_seg { const void* dy; void* out; int32_t n, ld; } natsl_wgrad_seg;
+size_t natsl_wgrad_workspace_bytes(const natsl_wgrad_seg* segs, int n_seg, int64_t T, int D);
+int natsl_wgrad(const natsl_wgrad_seg* segs, int n_seg, const void* x, int64_t T, int D, int ldx, void* workspace,
+                size_t workspace_bytes, natsl_stream_t stream);
 
 /* The mixed operator's forward (src/nats/ops/mixed_ops/mixed_attn_gdn.py:47-191, src/nats/ops/mixed_ops/mixed_attn_mamba.py:51-192)
  * in one call: natsl_route, natsl_softmax_sparse_fwd and natsl_gdn_chunk_fwd (is_delta) or natsl_mamba_chunk_fwd with the

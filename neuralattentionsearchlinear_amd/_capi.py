@@ -49,6 +49,8 @@ _SIGNATURES = {
     "natsl_linear_chunk_bwd": (c_int, [c_int] + [c_void_p] * 9 + [c_int] + [c_void_p] * 12 + [c_int] * 8 + [c_float, c_int, c_int, c_void_p, c_int, c_int, c_void_p]),
     "natsl_norm_gate_bwd_workspace_bytes": (c_size_t, [c_int64, c_int]),
     "natsl_norm_gate_bwd": (c_int, [c_void_p] * 14 + [c_size_t, c_int64, c_int, c_int, c_float, c_int, c_void_p]),
+    "natsl_norm_gate_logits_fwd": (c_int, [c_void_p] * 7 + [c_int64, c_int, c_int, c_float, c_int, c_void_p]),
+    "natsl_norm_gate_logits_bwd": (c_int, [c_void_p] * 14 + [c_size_t, c_int64, c_int, c_int, c_float, c_int, c_void_p]),
     "natsl_row_norm_bwd_workspace_bytes": (c_size_t, [c_int64, c_int]),
     "natsl_row_norm_bwd": (c_int, [c_void_p] * 6 + [c_size_t, c_int64, c_int, c_float, c_int, c_int, c_int, c_void_p]),
     "natsl_short_conv_fwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
@@ -74,6 +76,16 @@ _SIGNATURES = {
     "natsl_decode_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
     "natsl_decode_fwd": (c_int, [c_int] + [c_void_p] * 5 + [c_int] * 8 + [c_float, c_int64, c_int64, c_void_p, c_size_t] + [c_void_p] * 11 +
                                 [c_int, c_void_p] + [c_int] * 6 + [c_float, c_int, c_void_p]),
+    "natsl_conv_norm_fwd": (c_int, [c_void_p] + [c_int] * 6 + [c_void_p]),
+    "natsl_conv_norm_bwd_workspace_bytes": (c_size_t, [c_void_p] + [c_int] * 4),
+    "natsl_conv_norm_bwd": (c_int, [c_void_p] + [c_int] * 6 + [c_void_p, c_size_t, c_void_p]),
+    "natsl_gates_fwd": (c_int, [c_void_p] * 6 + [c_int64] + [c_int] * 4 + [c_void_p]),
+    "natsl_gates_bwd_workspace_bytes": (c_size_t, [c_int64, c_int]),
+    "natsl_gates_bwd": (c_int, [c_void_p] * 6 + [c_int] + [c_void_p] * 4 + [c_size_t, c_int64] + [c_int] * 4 + [c_void_p]),
+    "natsl_dx_init": (c_int, [c_void_p] * 4 + [c_int] * 6 + [c_void_p]),
+    "natsl_hard_select_bwd": (c_int, [c_void_p] * 3 + [c_int] * 5 + [c_void_p]),
+    "natsl_wgrad_workspace_bytes": (c_size_t, [c_void_p, c_int, c_int64, c_int]),
+    "natsl_wgrad": (c_int, [c_void_p, c_int, c_void_p, c_int64, c_int, c_int, c_void_p, c_size_t, c_void_p]),
     "natsl_mixed_fwd": (c_int, [c_void_p, c_int, c_void_p, c_void_p]),
     "natsl_layer_step_workspace_bytes": (c_size_t, [c_void_p]),
     "natsl_layer_step_fwd": (c_int, [c_void_p, c_void_p, c_size_t, c_void_p]),

@@ -1,0 +1,423 @@
+"""What surrounds the mixed operator inside the two layers, as a few fused steps with their backward: the projections of one input,
+the short convolutions with the row norms behind them, the gates, the selector, the mixing logits and the output norm-gate.
+
+`fast_front` says whether a forward may take this path: bf16 tensors on the GPU and the layers' own, unhooked submodules.  What it
+declines runs through the submodules one by one (the layers' general path).  Per step the saving is passes over [B,T,D] tensors
+(gradients that meet at a tensor are added where they are used, norms and mixing softmax ride on their neighbours' passes),
+weight-gradient products that split the tokens (natsl_wgrad), and launches.
+"""
+from __future__ import annotations
+
+import ctypes
+
+import torch
+import torch.nn.functional as F
+
+from . import _capi
+from ._layer_step import _PARAMS, _parameters
+from .modules import _NORM_GATE_WIDTHS
+
+_NAMES = [p[0] for p in _PARAMS]
+_EITHER = {"norm_q", "norm_k", "a_log", "dt_bias", "out_norm1", "out_norm2"}
+_ab_rows = lambda n: -(-n // 16) * 16
+
+
+class _WgradSeg(ctypes.Structure):
+    _fields_ = [("dy", ctypes.c_void_p), ("out", ctypes.c_void_p), ("n", ctypes.c_int32), ("ld", ctypes.c_int32)]
+
+
+class _ConvSeg(ctypes.Structure):
+    _fields_ = ([(n, ctypes.c_void_p) for n in ("x", "weight", "bias", "state", "norm_weight", "y", "y_norm", "state_out", "dy_a", "dy_b", "dy_norm",
+                                                "dx_add", "dx", "dweight", "dbias", "dnorm_weight")] +
+                [("D", ctypes.c_int32), ("norm_lanes", ctypes.c_int32), ("norm_l2", ctypes.c_int32), ("norm_eps", ctypes.c_float)])
+
+
+def _p(t):
+    return None if t is None else t.data_ptr()
+
+
+def weight_grads(x2, dys):
+    """[dy_i^T x2 for dy_i [rows, n_i] in dys] (bf16; entries may be None): natsl_wgrad for widths that are multiples of 8, else torch."""
+    rows, D = x2.shape
+    out = [None] * len(dys)
+    todo = []
+    for i, dy in enumerate(dys):
+        if dy is None:
+            continue
+        if dy.shape[1] % 8 or D % 8 or x2.data_ptr() % 16 or dy.data_ptr() % 16 or dy.dtype != torch.bfloat16:
+            out[i] = torch.mm(dy.t(), x2)
+        else:
+            out[i] = torch.empty(dy.shape[1], D, dtype=torch.bfloat16, device=x2.device)
+            todo.append(i)
+    if todo:
+        segs = (_WgradSeg * len(todo))()
+        for s, i in zip(segs, todo):
+            s.dy, s.out, s.n, s.ld = dys[i].data_ptr(), out[i].data_ptr(), dys[i].shape[1], dys[i].shape[1]
+        L = _capi.lib()
+        n = L.natsl_wgrad_workspace_bytes(segs, len(todo), rows, D)
+        ws = torch.empty(n, dtype=torch.uint8, device=x2.device)
+        _capi.check(L.natsl_wgrad(segs, len(todo), x2.data_ptr(), rows, D, D, ws.data_ptr(), n, _capi.stream_ptr(x2.device)), "natsl_wgrad")
+    return out
+
+
+class _Linear(torch.autograd.Function):
+    """F.linear with the weight gradient of natsl_wgrad."""
+
+    @staticmethod
+    def forward(ctx, x, w):
+        ctx.save_for_backward(x, w)
+        return F.linear(x, w)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, w = ctx.saved_tensors
+        dy2 = dy.reshape(-1, dy.shape[-1]).contiguous()
+        dx = torch.mm(dy2, w).view(x.shape) if ctx.needs_input_grad[0] else None
+        dw = weight_grads(x.reshape(-1, x.shape[-1]), [dy2])[0] if ctx.needs_input_grad[1] else None
+        return dx, dw
+
+
+def linear(x, w):
+    if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
+        return _Linear.apply(x, w)
+    return F.linear(x, w)
+
+
+# ---- the projections of one input -----------------------------------------------------------------------------------------------
+def _project(x, wq, wk, wv, wg, wa, wb, pool_block):
+    """-> ((q, k, v, gate, ab, block means or None), the joint weight of a and b).  The narrow projections share one product: their
+    rows and enough others to make whole tiles of 16 (the columns behind a and b are never read)."""
+    narrow = (wa,) if wb is None else (wa, wb)
+    used = sum(w.shape[0] for w in narrow)
+    wab = torch.cat(narrow + (wq[:_ab_rows(used) - used],)) if used % 16 else torch.cat(narrow) if len(narrow) > 1 else wa
+    pooled = None
+    if pool_block:
+        from .nats_util import _mean_pooling_fwd
+        pooled = _mean_pooling_fwd(x.unsqueeze(-2), pool_block, None).squeeze(-2)
+    return (F.linear(x, wq), F.linear(x, wk), F.linear(x, wv), F.linear(x, wg), F.linear(x, wab), pooled), wab
+
+
+class _Project(torch.autograd.Function):
+    """dx starts as what is no wide product (natsl_dx_init) and the four wide ones accumulate onto it; all weight gradients are one
+    launch."""
+
+    @staticmethod
+    def forward(ctx, x, wq, wk, wv, wg, wa, wb, pool_block):
+        out, wab = _project(x, wq, wk, wv, wg, wa, wb, pool_block)
+        ctx.save_for_backward(x, wq, wk, wv, wg, wab)
+        ctx.block, ctx.n_a, ctx.n_b = pool_block, wa.shape[0], 0 if wb is None else wb.shape[0]
+        ctx.set_materialize_grads(False)
+        return out
+
+    @staticmethod
+    def backward(ctx, dq, dk, dv, dg, dab, dpool):
+        x, wq, wk, wv, wg, wab = ctx.saved_tensors
+        B, T, D = x.shape
+        rows = B * T
+        flat = lambda t: None if t is None else t.reshape(rows, t.shape[-1]).contiguous()
+        dys = [flat(t) for t in (dq, dk, dv, dg, dab)]
+        need = ctx.needs_input_grad
+        dx = None
+        if need[0]:
+            dx = torch.empty_like(x)
+            dp = None if dpool is None else dpool.contiguous()
+            n = 0 if dys[4] is None else wab.shape[0]
+            rc = _capi.lib().natsl_dx_init(_p(dys[4]), wab.data_ptr(), _p(dp), dx.data_ptr(), B, T, D, n, max(n, 16), ctx.block or T,
+                                           _capi.stream_ptr(x.device))
+            _capi.check(rc, "natsl_dx_init")
+            dx2 = dx.view(rows, D)
+            for dy, w in zip(dys, (wq, wk, wv, wg)):
+                if dy is not None:
+                    dx2.addmm_(dy, w)
+        wants = [need[1], need[2], need[3], need[4], need[5] or need[6]]
+        dws = weight_grads(x.view(rows, D), [dy if want else None for dy, want in zip(dys, wants)])
+        da = db = None
+        if dws[4] is not None:
+            da = dws[4][:ctx.n_a]
+            db = dws[4][ctx.n_a:ctx.n_a + ctx.n_b] if ctx.n_b else None
+        return dx, dws[0], dws[1], dws[2], dws[3], da, db, None
+
+
+# ---- convolutions, norms, mixing logits --------------------------------------------------------------------------------------------
+def _conv_segs(f, raw):
+    """The segments of natsl_conv_norm_*: q, k, v with their weights; f: the layer's FastFront."""
+    segs = (_ConvSeg * 3)()
+    for s, x, n in zip(segs, raw, "qkv"):
+        s.x, s.D, s.weight, s.bias = x.data_ptr(), x.shape[-1], _p(f.w["conv_w" + n]), _p(f.w["conv_b" + n])
+        if n != "v":
+            s.norm_lanes, s.norm_l2, s.norm_eps = f.norm_width // 8, int(f.l2), f.front_eps
+            s.norm_weight = None if f.l2 else f.w["norm_" + n].data_ptr()
+    return segs
+
+
+def _conv_norm(f, raw, states, want_states):
+    """-> (conv(q) or None, conv(k) or None, conv(v), normed q, normed k, new states)."""
+    B, T, _ = raw[0].shape
+    segs = _conv_segs(f, raw)
+    ys = [torch.empty_like(raw[0]), None if f.l2 else torch.empty_like(raw[1]), torch.empty_like(raw[2])]
+    ns = [torch.empty_like(raw[0]), torch.empty_like(raw[1])]
+    new = None
+    if want_states:
+        new = tuple([torch.empty(B, x.shape[-1], f.W, dtype=torch.bfloat16, device=x.device) for x in raw])
+    for i, s in enumerate(segs):
+        s.y = _p(ys[i])
+        if i < 2:
+            s.y_norm = ns[i].data_ptr()
+        if states is not None and states[i] is not None:
+            s.state = states[i].data_ptr()
+        if new is not None:
+            s.state_out = new[i].data_ptr()
+    _capi.check(_capi.lib().natsl_conv_norm_fwd(segs, 3, B, T, f.W, f.act, f.norm_dtype, _capi.stream_ptr(raw[0].device)), "natsl_conv_norm_fwd")
+    return ys, ns, new
+
+
+class _ConvNorm(torch.autograd.Function):
+    """(q, k, v projections) -> (conv(q), conv(k), conv(v), normed q, normed k, mixing logits, and the projections themselves); the last
+    three only carry the gradient of an attention view that takes them to where it is added (dx_add)."""
+
+    @staticmethod
+    def forward(ctx, f, q, k, v, wq, bq, wk, bk, wv, bv, nq, nk, w_mix):
+        ys, ns, _ = _conv_norm(f, (q, k, v), None, False)
+        ctx.f = f
+        # (the parameters are saved for the check that nobody changes them before the backward reads them through f)
+        ctx.save_for_backward(q, k, v, ys[0], w_mix, wq, bq, wk, bk, wv, bv, nq, nk)
+        ctx.set_materialize_grads(False)
+        raw = tuple(t.view(t.shape) for t in (q, k, v)) if f.raw_attention else (None, None, None)
+        return (ys[0], ys[1], ys[2], ns[0], ns[1], F.linear(ys[0], w_mix)) + raw
+
+    @staticmethod
+    def backward(ctx, dq, dk, dv, dqn, dkn, dlogits, dq_raw, dk_raw, dv_raw):
+        f = ctx.f
+        q, k, v, yq, w_mix = ctx.saved_tensors[:5]
+        B, T, _ = q.shape
+        dev = q.device
+        dw_mix = dq_mix = None
+        if dlogits is not None:
+            d2 = dlogits.reshape(B * T, -1).contiguous()
+            dq_mix = torch.mm(d2, w_mix)
+            dw_mix = weight_grads(yq.view(B * T, -1), [d2])[0]
+        hold = []
+
+        def at(t):
+            if t is None:
+                return None
+            t = t.contiguous()
+            hold.append(t)
+            return t.data_ptr()
+        segs = _conv_segs(f, (q, k, v))
+        grads = []
+        for s, x, n, da, db, dn, add in zip(segs, (q, k, v), "qkv", (dq, dk, dv), (dq_mix, None, None), (dqn, dkn, None), (dq_raw, dk_raw, dv_raw)):
+            w, b = f.w["conv_w" + n], f.w["conv_b" + n]
+            dx, dw = torch.empty_like(x), torch.empty_like(w)
+            dbias = None if b is None else torch.empty_like(b)
+            dnorm = torch.empty_like(f.w["norm_" + n]) if n != "v" and not f.l2 else None
+            s.dy_a, s.dy_b, s.dy_norm, s.dx_add = at(da), at(db), at(dn), at(add)
+            s.dx, s.dweight, s.dbias, s.dnorm_weight = dx.data_ptr(), dw.data_ptr(), _p(dbias), _p(dnorm)
+            if dn is None and dnorm is not None:
+                dnorm.zero_()
+            grads.append((dx, dw, dbias, dnorm))
+        L = _capi.lib()
+        n = L.natsl_conv_norm_bwd_workspace_bytes(segs, 3, B, T, f.W)
+        ws = torch.empty(n, dtype=torch.uint8, device=dev)
+        _capi.check(L.natsl_conv_norm_bwd(segs, 3, B, T, f.W, f.act, f.norm_dtype, ws.data_ptr(), n, _capi.stream_ptr(dev)), "natsl_conv_norm_bwd")
+        (dxq, dwq, dbq, dnq), (dxk, dwk, dbk, dnk), (dxv, dwv, dbv, _) = grads
+        return None, dxq, dxk, dxv, dwq, dbq, dwk, dbk, dwv, dbv, dnq, dnk, dw_mix
+
+
+# ---- gates ---------------------------------------------------------------------------------------------------------------------------
+def _gates(f, ab):
+    """-> (g fp32, beta bf16 or None, dt fp32 or None), each [B,T,H]."""
+    B, T, ld = ab.shape
+    g = torch.empty(B, T, f.H, dtype=torch.float32, device=ab.device)
+    beta = torch.empty(B, T, f.H, dtype=torch.bfloat16, device=ab.device) if f.delta else None
+    dt = None if f.delta else torch.empty_like(g)
+    rc = _capi.lib().natsl_gates_fwd(ab.data_ptr(), f.w["a_log"].data_ptr(), f.w["dt_bias"].data_ptr(), g.data_ptr(), _p(beta), _p(dt), B * T, f.H, ld,
+                                     f.neg, f.gate_dtype, _capi.stream_ptr(ab.device))
+    _capi.check(rc, "natsl_gates_fwd")
+    return g, beta, dt
+
+
+class _Gates(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, f, ab, a_log, dt_bias):
+        ctx.f = f
+        ctx.save_for_backward(ab, a_log, dt_bias)
+        ctx.set_materialize_grads(False)
+        return _gates(f, ab)
+
+    @staticmethod
+    def backward(ctx, dg, dbeta, ddt):
+        f, ab = ctx.f, ctx.saved_tensors[0]
+        B, T, ld = ab.shape
+        c = lambda t, dt: None if t is None else t.to(dt).contiguous()
+        dg, dbeta, ddt = c(dg, torch.float32), c(dbeta, torch.bfloat16), c(ddt, torch.float32)
+        dab = torch.empty_like(ab)
+        da_log, ddt_bias = torch.empty_like(f.w["a_log"]), torch.empty_like(f.w["dt_bias"])
+        L = _capi.lib()
+        n = L.natsl_gates_bwd_workspace_bytes(B * T, f.H)
+        ws = torch.empty(n, dtype=torch.uint8, device=ab.device)
+        rc = L.natsl_gates_bwd(ab.data_ptr(), f.w["a_log"].data_ptr(), f.w["dt_bias"].data_ptr(), _p(dg), _p(dbeta), _p(ddt), int(f.delta), dab.data_ptr(),
+                               da_log.data_ptr(), ddt_bias.data_ptr(), ws.data_ptr(), n, B * T, f.H, ld, f.neg, f.gate_dtype,
+                               _capi.stream_ptr(ab.device))
+        _capi.check(rc, "natsl_gates_bwd")
+        return None, dab, da_log, ddt_bias
+
+
+# ---- output norm-gate with the mixing logits -------------------------------------------------------------------------------------------
+def _tail(f, o_lin, o_attn, gate, logits):
+    y = torch.empty_like(o_attn)
+    D = o_attn.shape[-1]
+    rc = _capi.lib().natsl_norm_gate_logits_fwd(o_lin.data_ptr(), o_attn.data_ptr(), gate.data_ptr(), logits.data_ptr(), f.w["out_norm1"].data_ptr(),
+                                                f.w["out_norm2"].data_ptr(), y.data_ptr(), o_attn.numel() // D, D, _capi.BF16, f.out_eps, f.out_dtype,
+                                                _capi.stream_ptr(y.device))
+    _capi.check(rc, "natsl_norm_gate_logits_fwd")
+    return y
+
+
+class _Tail(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, f, o_lin, o_attn, gate, logits, w1, w2):
+        ctx.f = f
+        ctx.save_for_backward(o_lin, o_attn, gate, logits, w1, w2)
+        return _tail(f, o_lin, o_attn, gate, logits)
+
+    @staticmethod
+    def backward(ctx, dy):
+        f = ctx.f
+        a, b, g, lg = ctx.saved_tensors[:4]
+        D = b.shape[-1]
+        rows = b.numel() // D
+        dy = dy.contiguous()
+        w1, w2 = f.w["out_norm1"], f.w["out_norm2"]
+        da, db, dg, dl = torch.empty_like(a), torch.empty_like(b), torch.empty_like(g), torch.empty_like(lg)
+        dw = torch.empty(2, D, dtype=torch.float32, device=a.device)
+        L = _capi.lib()
+        n = L.natsl_norm_gate_bwd_workspace_bytes(rows, D)
+        ws = torch.empty(n, dtype=torch.uint8, device=a.device)
+        rc = L.natsl_norm_gate_logits_bwd(a.data_ptr(), b.data_ptr(), g.data_ptr(), lg.data_ptr(), w1.data_ptr(), w2.data_ptr(), dy.data_ptr(),
+                                          da.data_ptr(), db.data_ptr(), dg.data_ptr(), dl.data_ptr(), dw.data_ptr(), dw.data_ptr() + 4 * D,
+                                          ws.data_ptr(), n, rows, D, _capi.BF16, f.out_eps, f.out_dtype, _capi.stream_ptr(a.device))
+        _capi.check(rc, "natsl_norm_gate_logits_bwd")
+        dw = dw.to(w1.dtype)
+        return None, da, db, dg, dl, dw[0], dw[1]
+
+
+# ---- selector ------------------------------------------------------------------------------------------------------------------------
+class _Select(torch.autograd.Function):
+    """Hard selection with the straight-through gradient; the last block, forced to both ops, has none."""
+
+    @staticmethod
+    def forward(ctx, logits, force_last):
+        from .nats_util import hard_select
+        types, counts = hard_select(logits.detach(), force_last_block=force_last)
+        ctx.save_for_backward(logits)
+        ctx.force = force_last
+        ctx.mark_non_differentiable(counts)
+        return types, counts
+
+    @staticmethod
+    def backward(ctx, dtypes, _):
+        (logits,) = ctx.saved_tensors
+        lg, d = logits.contiguous(), dtypes.to(logits.dtype).contiguous()
+        out = torch.empty_like(lg)
+        B, TN, HN, _ = lg.shape
+        rc = _capi.lib().natsl_hard_select_bwd(lg.data_ptr(), d.data_ptr(), out.data_ptr(), B, TN, HN, _capi.dtype_code(lg.dtype), int(ctx.force),
+                                               _capi.stream_ptr(lg.device))
+        _capi.check(rc, "natsl_hard_select_bwd")
+        return out, None
+
+
+class FastFront:
+    """The layer's current parameters and constants for one forward (and the backward that follows it)."""
+
+    def __init__(self, layer, kind, params):
+        self.w = w = dict(zip(_NAMES, params))
+        self.delta = kind == 'gdn'
+        self.H, self.W = layer.num_heads, layer.conv_size
+        self.act = 0 if layer.q_conv1d.activation is None else 1
+        self.l2 = not self.delta
+        self.raw_attention = not self.delta
+        self.norm_width = layer.head_attn_k_dim if self.delta else layer.head_k_dim
+        self.front_eps = layer.q_norm.eps if self.delta else layer.q_norm2.eps
+        self.norm_dtype = _capi.dtype_code(w["norm_q"].dtype) if self.delta else _capi.BF16
+        self.gate_dtype, self.out_dtype = _capi.dtype_code(w["a_log"].dtype), _capi.dtype_code(w["out_norm1"].dtype)
+        self.neg = int(self.delta and layer.allow_neg_eigval)
+        self.out_eps = layer.o_norm.eps
+
+    def grad(self, *tensors):
+        return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
+
+    def project(self, x, pool_block):
+        w = self.w
+        args = (x, w["wq"], w["wk"], w["wv"], w["wg"], w["wa"], w["wb"] if self.delta else None, pool_block)
+        if self.grad(*args[:7]):
+            return _Project.apply(*args)
+        return _project(*args)[0]
+
+    def conv_norm(self, q, k, v, states, want_states):
+        """-> (conv(q), conv(k) or None, conv(v), normed q, normed k, mixing logits, raw q, k, v, new states)."""
+        w = self.w
+        args = (q, k, v, w["conv_wq"], w["conv_bq"], w["conv_wk"], w["conv_bk"], w["conv_wv"], w["conv_bv"],
+                w["norm_q"] if self.delta else None, w["norm_k"] if self.delta else None, w["w_mix"])
+        if self.grad(*args):
+            return _ConvNorm.apply(self, *args) + (None,)
+        ys, ns, new = _conv_norm(self, (q, k, v), states, want_states)
+        return ys[0], ys[1], ys[2], ns[0], ns[1], F.linear(ys[0], w["w_mix"]), q, k, v, new
+
+    def gates(self, ab):
+        if self.grad(ab, self.w["a_log"], self.w["dt_bias"]):
+            return _Gates.apply(self, ab, self.w["a_log"], self.w["dt_bias"])
+        return _gates(self, ab)
+
+    def select(self, logits, force_last):
+        if self.grad(logits):
+            return _Select.apply(logits, force_last)
+        from .nats_util import hard_select
+        return hard_select(logits, force_last_block=force_last)
+
+    def tail(self, o_lin, o_attn, gate, logits):
+        args = (o_lin.contiguous(), o_attn.contiguous(), gate.contiguous(), logits.contiguous())
+        w1, w2 = self.w["out_norm1"], self.w["out_norm2"]
+        y = _Tail.apply(self, *args, w1, w2) if self.grad(*args, w1, w2) else _tail(self, *args)
+        return linear(y.flatten(-2), self.w["wo"])
+
+
+def fast_front(layer, kind, x, cache, cu_seqlens):
+    """The layer's FastFront for this forward, or None where the general path has to run."""
+    if not x.is_cuda or x.dtype != torch.bfloat16 or cu_seqlens is not None or not x.is_contiguous() or x.numel() == 0 or \
+            torch.is_autocast_enabled():
+        return None
+    params = _parameters(layer)
+    if params is None or not layer.use_short_conv or layer.num_v_heads != layer.num_heads:
+        return None
+    delta = kind == 'gdn'
+    if layer.attn_with_short_conv != delta or (delta and not layer.attn_qk_norm):
+        return None
+    w = dict(zip(_NAMES, params))
+    for n, t in w.items():
+        if t is None:
+            if n.startswith("conv_b") or (not delta and n in ("wb", "norm_q", "norm_k")):
+                continue
+            return None
+        if t.device != x.device or not t.is_contiguous() or (t.dtype != torch.bfloat16 and (n not in _EITHER or t.dtype != torch.float32)):
+            return None
+    if w["a_log"].dtype != w["dt_bias"].dtype or w["out_norm1"].dtype != w["out_norm2"].dtype or (delta and w["norm_q"].dtype != w["norm_k"].dtype):
+        return None
+    convs = (layer.q_conv1d, layer.k_conv1d, layer.v_conv1d)
+    if any(c.kernel_size[0] != layer.conv_size or (c.activation is None) != (convs[0].activation is None) for c in convs) or layer.conv_size not in (2, 3, 4):
+        return None
+    if any(layer._modules[m].bias is not None for m in ("q_proj", "k_proj", "v_proj", "g_proj", "a_proj", "nats_out_weights_layer", "o_proj")) or \
+            (delta and layer.b_proj.bias is not None):
+        return None
+    norms = (layer.q_norm, layer.k_norm) if delta else (layer.q_norm2, layer.k_norm2)
+    width = layer.head_attn_k_dim if delta else layer.head_k_dim
+    if norms[0].eps != norms[1].eps or width not in (32, 64, 128, 256, 512) or layer.head_attn_v_dim not in _NORM_GATE_WIDTHS or \
+            layer.hidden_size % 8 or layer.num_heads > 256 or layer.value_dim % 8:
+        return None
+    if cache is not None:
+        if torch.is_grad_enabled() and (x.requires_grad or any(t is not None and t.requires_grad for t in params)):
+            return None
+        st = cache.conv_state
+        if st is not None and any(s is not None and (s.dtype != torch.bfloat16 or not s.is_contiguous() or s.shape[0] != x.shape[0]) for s in st):
+            return None
+    return FastFront(layer, kind, params)

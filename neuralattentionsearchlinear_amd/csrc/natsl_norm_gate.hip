@@ -14,10 +14,22 @@ NATSL_DEVICE void unpack8(const u32x4 w, float* f) {
   }
 }
 
+// The mixing weights of a row: as given, or the softmax of the two given logits rounded to bf16 (what the mixing layer's separate
+// softmax returns; taken here, it costs no pass of its own)
+NATSL_DEVICE void mix_weights(const bf16_t* xw, const long long row, const int logits, float& a, float& b) {
+  a = bf16_to_f32(xw[row * 2]);
+  b = bf16_to_f32(xw[row * 2 + 1]);
+  if (logits) {
+    const float mx = fmaxf(a, b), e0 = __expf(a - mx), e1 = __expf(b - mx), inv = 1.f / (e0 + e1);
+    a = bf16_to_f32(f32_to_bf16(e0 * inv));
+    b = bf16_to_f32(f32_to_bf16(e1 * inv));
+  }
+}
+
 template <int LANES, int PER>  // a row is handled by LANES adjacent lanes, PER 16-byte pieces each: D = 8 LANES PER
 __global__ __launch_bounds__(256) void norm_gate_kernel(const bf16_t* x1, const bf16_t* x2, const bf16_t* gate, const bf16_t* xw,
                                                         const void* w1, const void* w2, bf16_t* y, long long rows, float eps,
-                                                        int w_dtype) {
+                                                        int w_dtype, int logits) {
   constexpr int D = LANES * PER * 8;
   const long long row = ((long long)blockIdx.x * 256 + threadIdx.x) / LANES;
   const int seg = threadIdx.x % LANES;
@@ -41,8 +53,10 @@ __global__ __launch_bounds__(256) void norm_gate_kernel(const bf16_t* x1, const 
     sa += __shfl_xor(sa, d);
     sb += __shfl_xor(sb, d);
   }
-  const float ra = rsqrtf(sa / D + eps) * bf16_to_f32(xw[row * 2]);
-  const float rb = rsqrtf(sb / D + eps) * bf16_to_f32(xw[row * 2 + 1]);
+  float ra, rb;
+  mix_weights(xw, row, logits, ra, rb);
+  ra *= rsqrtf(sa / D + eps);
+  rb *= rsqrtf(sb / D + eps);
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
     const int col = (u * LANES + seg) * 8;
@@ -85,7 +99,7 @@ __global__ __launch_bounds__(256) void norm_gate_kernel(const bf16_t* x1, const 
 template <int LANES, int PER>
 __global__ __launch_bounds__(256) void norm_gate_bwd_kernel(const bf16_t* x1, const bf16_t* x2, const bf16_t* gate, const bf16_t* xw,
                                                             const void* w1, const void* w2, const bf16_t* dy, bf16_t* dx1, bf16_t* dx2,
-                                                            bf16_t* dgate, float* dxw, float* part, long long rows, int rows_per_wg,
+                                                            bf16_t* dgate, float* dxw, bf16_t* dlogits, float* part, long long rows, int rows_per_wg,
                                                             float eps, int w_dtype) {
   constexpr int D = LANES * PER * 8, G = 256 / LANES;
   __shared__ float acc_s[G][2][D];
@@ -133,7 +147,8 @@ __global__ __launch_bounds__(256) void norm_gate_bwd_kernel(const bf16_t* x1, co
       sb += __shfl_xor(sb, dd);
     }
     const float ra = rsqrtf(sa / D + eps), rb = rsqrtf(sb / D + eps);
-    const float xa = bf16_to_f32(xw[row * 2]), xb = bf16_to_f32(xw[row * 2 + 1]);
+    float xa, xb;
+    mix_weights(xw, row, dlogits != nullptr, xa, xb);
     // pass 2: a, b become the normalised inputs, d becomes dmix, g becomes dgate / mix's factor
     float pa = 0.f, pb = 0.f;
 #pragma unroll
@@ -158,8 +173,13 @@ __global__ __launch_bounds__(256) void norm_gate_bwd_kernel(const bf16_t* x1, co
       pb += __shfl_xor(pb, dd);
     }
     if (seg == 0) {
-      dxw[row * 2] = pa;
-      dxw[row * 2 + 1] = pb;
+      if (dlogits) {
+        const float m = pa * xa + pb * xb;
+        reinterpret_cast<unsigned*>(dlogits)[row] = pack_bf16x2(xa * (pa - m), xb * (pb - m));
+      } else {
+        dxw[row * 2] = pa;
+        dxw[row * 2 + 1] = pb;
+      }
     }
     const float ma = xa * pa / D, mb = xb * pb / D;   // mean_d(a1 n1), mean_d(a2 n2)
 #pragma unroll
@@ -238,9 +258,8 @@ constexpr int NG_BWD_ROWS = 128;   // rows per workgroup of the backward
 
 using namespace natsl;
 
-extern "C" int natsl_norm_gate_fwd(const void* x1, const void* x2, const void* gate, const void* x_weights, const void* w1,
-                                   const void* w2, void* y, int64_t rows, int D, int dtype, float eps, int w_dtype,
-                                   natsl_stream_t stream) {
+static int norm_gate_fwd(const void* x1, const void* x2, const void* gate, const void* x_weights, const void* w1, const void* w2, void* y,
+                         int64_t rows, int D, int dtype, float eps, int w_dtype, int logits, natsl_stream_t stream) {
   if (!x1 || !x2 || !gate || !x_weights || !w1 || !w2 || !y) return fail(NATSL_ERR_INVALID, "norm_gate: null pointer argument");
   if (dtype != NATSL_BF16) return fail(NATSL_ERR_UNSUPPORTED, "norm_gate: only bf16 activations are supported");
   if (w_dtype != NATSL_BF16 && w_dtype != NATSL_F32) return fail(NATSL_ERR_UNSUPPORTED, "norm_gate: weights must be f32 or bf16");
@@ -251,7 +270,7 @@ extern "C" int natsl_norm_gate_fwd(const void* x1, const void* x2, const void* g
     const long long threads = rows * (L);                                                                                   \
     hipLaunchKernelGGL((norm_gate_kernel<L, P>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, (const bf16_t*)x1,    \
                        (const bf16_t*)x2, (const bf16_t*)gate, (const bf16_t*)x_weights, w1, w2, (bf16_t*)y, (long long)rows, \
-                       eps, w_dtype);                                                                                       \
+                       eps, w_dtype, logits);                                                                               \
     return check_launch("natsl_norm_gate_fwd");                                                                             \
   }
   switch (D) {
@@ -268,17 +287,28 @@ extern "C" int natsl_norm_gate_fwd(const void* x1, const void* x2, const void* g
 #undef NATSL_NG
 }
 
+extern "C" int natsl_norm_gate_fwd(const void* x1, const void* x2, const void* gate, const void* x_weights, const void* w1,
+                                   const void* w2, void* y, int64_t rows, int D, int dtype, float eps, int w_dtype,
+                                   natsl_stream_t stream) {
+  return norm_gate_fwd(x1, x2, gate, x_weights, w1, w2, y, rows, D, dtype, eps, w_dtype, 0, stream);
+}
+extern "C" int natsl_norm_gate_logits_fwd(const void* x1, const void* x2, const void* gate, const void* x_logits, const void* w1,
+                                          const void* w2, void* y, int64_t rows, int D, int dtype, float eps, int w_dtype,
+                                          natsl_stream_t stream) {
+  return norm_gate_fwd(x1, x2, gate, x_logits, w1, w2, y, rows, D, dtype, eps, w_dtype, 1, stream);
+}
+
 extern "C" size_t natsl_norm_gate_bwd_workspace_bytes(int64_t rows, int D) {
   if (rows <= 0 || D <= 0) return 0;
   return (size_t)((rows + NG_BWD_ROWS - 1) / NG_BWD_ROWS) * 2 * (size_t)D * sizeof(float);
 }
 
-extern "C" int natsl_norm_gate_bwd(const void* x1, const void* x2, const void* gate, const void* x_weights, const void* w1,
-                                   const void* w2, const void* dy, void* dx1, void* dx2, void* dgate, float* dx_weights, float* dw1,
-                                   float* dw2, void* workspace, size_t workspace_bytes, int64_t rows, int D, int dtype, float eps,
-                                   int w_dtype, natsl_stream_t stream) {
+static int norm_gate_bwd(const void* x1, const void* x2, const void* gate, const void* x_weights, const void* w1, const void* w2,
+                         const void* dy, void* dx1, void* dx2, void* dgate, float* dx_weights, bf16_t* dlogits, float* dw1, float* dw2,
+                         void* workspace, size_t workspace_bytes, int64_t rows, int D, int dtype, float eps, int w_dtype,
+                         natsl_stream_t stream) {
   const char* what = "natsl_norm_gate_bwd";
-  if (!x1 || !x2 || !gate || !x_weights || !w1 || !w2 || !dy || !dx1 || !dx2 || !dgate || !dx_weights || !dw1 || !dw2)
+  if (!x1 || !x2 || !gate || !x_weights || !w1 || !w2 || !dy || !dx1 || !dx2 || !dgate || (!dx_weights && !dlogits) || !dw1 || !dw2)
     return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
   if (dtype != NATSL_BF16) return fail(NATSL_ERR_UNSUPPORTED, "%s: only bf16 activations are supported", what);
   if (w_dtype != NATSL_BF16 && w_dtype != NATSL_F32) return fail(NATSL_ERR_UNSUPPORTED, "%s: weights must be f32 or bf16", what);
@@ -292,7 +322,7 @@ extern "C" int natsl_norm_gate_bwd(const void* x1, const void* x2, const void* g
 #define NATSL_NGB(L, P)                                                                                                          \
   hipLaunchKernelGGL((norm_gate_bwd_kernel<L, P>), dim3(wgs), dim3(256), 0, s, (const bf16_t*)x1, (const bf16_t*)x2,              \
                      (const bf16_t*)gate, (const bf16_t*)x_weights, w1, w2, (const bf16_t*)dy, (bf16_t*)dx1, (bf16_t*)dx2,       \
-                     (bf16_t*)dgate, dx_weights, part, (long long)rows, NG_BWD_ROWS, eps, w_dtype);                              \
+                     (bf16_t*)dgate, dx_weights, dlogits, part, (long long)rows, NG_BWD_ROWS, eps, w_dtype);                              \
   break;
   switch (D) {
     case 32: NATSL_NGB(4, 1)
@@ -310,4 +340,19 @@ extern "C" int natsl_norm_gate_bwd(const void* x1, const void* x2, const void* g
   if (rc != NATSL_OK) return rc;
   hipLaunchKernelGGL(colsum_reduce_kernel, dim3((unsigned)((2 * D + 63) / 64)), dim3(1024), 0, s, part, dw1, (int)wgs, 2 * D);
   return check_launch(what);
+}
+
+extern "C" int natsl_norm_gate_bwd(const void* x1, const void* x2, const void* gate, const void* x_weights, const void* w1,
+                                   const void* w2, const void* dy, void* dx1, void* dx2, void* dgate, float* dx_weights, float* dw1,
+                                   float* dw2, void* workspace, size_t workspace_bytes, int64_t rows, int D, int dtype, float eps,
+                                   int w_dtype, natsl_stream_t stream) {
+  return norm_gate_bwd(x1, x2, gate, x_weights, w1, w2, dy, dx1, dx2, dgate, dx_weights, nullptr, dw1, dw2, workspace, workspace_bytes, rows, D,
+                       dtype, eps, w_dtype, stream);
+}
+extern "C" int natsl_norm_gate_logits_bwd(const void* x1, const void* x2, const void* gate, const void* x_logits, const void* w1,
+                                          const void* w2, const void* dy, void* dx1, void* dx2, void* dgate, void* dx_logits, float* dw1,
+                                          float* dw2, void* workspace, size_t workspace_bytes, int64_t rows, int D, int dtype, float eps,
+                                          int w_dtype, natsl_stream_t stream) {
+  return norm_gate_bwd(x1, x2, gate, x_logits, w1, w2, dy, dx1, dx2, dgate, nullptr, (bf16_t*)dx_logits, dw1, dw2, workspace, workspace_bytes, rows,
+                       D, dtype, eps, w_dtype, stream);
 }

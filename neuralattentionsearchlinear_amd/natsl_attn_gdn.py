@@ -21,6 +21,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import nats_util
+from ._front import fast_front
 from ._layer_step import layer_step
 from .cache import NAtSCache, NAtSLayerCache
 from .mixed_attn_gdn import nats_mixed_attn_gdn, nats_mixed_attn_gdn_chunk_inference, nats_mixed_attn_gdn_recurrent
@@ -132,6 +133,49 @@ class NeuralAttentionSearchLinearAttnGDN(nn.Module):
                                                   op_for_incomplete_chunk=self.ops_for_incomplete_chunks)
         return past_key_values[self.layer_idx]
 
+    def _general_front(self, hidden_states, selector_input, conv_states, use_cache, cu_seqlens):
+        """Selector, projections, convolutions, norms and gates through the submodules one by one."""
+        if selector_input is not None:
+            raw_types, _, _ = self.select_ops(selector_input, cu_seqlens, force_last_block=False)
+        else:
+            raw_types = torch.ones(hidden_states.shape[0], 1, self.num_nats_head, self.n_ops, device=hidden_states.device, dtype=hidden_states.dtype)
+
+        new_conv_states = []
+
+        def conv_or_act(x, conv, state):
+            if self.use_short_conv:
+                y, final = conv(x=x, cache=state, output_final_state=bool(use_cache), cu_seqlens=cu_seqlens)
+                new_conv_states.append(final)
+                return y
+            return F.silu(x)
+
+        if self.attn_with_short_conv:
+            q = conv_or_act(self.q_proj(hidden_states), getattr(self, 'q_conv1d', None), conv_states[0])
+            k = conv_or_act(self.k_proj(hidden_states), getattr(self, 'k_conv1d', None), conv_states[1])
+            v = conv_or_act(self.v_proj(hidden_states), getattr(self, 'v_conv1d', None), conv_states[2])
+            q_attn, k_attn, v_attn = q, k, v
+        else:
+            q_attn, k_attn, v_attn = self.q_proj(hidden_states), self.k_proj(hidden_states), self.v_proj(hidden_states)
+            q = conv_or_act(q_attn, getattr(self, 'q_conv1d', None), conv_states[0])
+            k = conv_or_act(k_attn, getattr(self, 'k_conv1d', None), conv_states[1])
+            v = conv_or_act(v_attn, getattr(self, 'v_conv1d', None), conv_states[2])
+        o_weights = self.nats_out_weights_layer(q).unflatten(-1, (self.num_attn_heads, self.n_ops)).softmax(-1)
+
+        q, k = (x.unflatten(-1, (-1, self.head_k_dim)) for x in (q, k))
+        v = v.unflatten(-1, (-1, self.head_v_dim))
+        q_attn, k_attn = (x.unflatten(-1, (-1, self.head_attn_k_dim)) for x in (q_attn, k_attn))
+        v_attn = v_attn.unflatten(-1, (-1, self.head_attn_v_dim))
+        if self.num_v_heads > self.num_heads:
+            q, k = (x.repeat_interleave(self.num_v_heads // self.num_heads, dim=-2) for x in (q, k))
+        if self.attn_qk_norm:
+            q_attn, k_attn = self.q_norm(q_attn), self.k_norm(k_attn)
+
+        beta = self.b_proj(hidden_states).sigmoid()
+        if self.allow_neg_eigval:
+            beta = beta * 2.
+        g = -self.A_log.float().exp() * F.softplus(self.a_proj(hidden_states).float() + self.dt_bias)
+        return q, k, v, q_attn, k_attn, v_attn, o_weights, g, beta, raw_types, tuple(new_conv_states) if self.use_short_conv else None
+
     def forward(self, hidden_states: torch.Tensor, attention_mask: Optional[torch.Tensor] = None, past_key_values=None,
                 use_cache: Optional[bool] = False, output_attentions: Optional[bool] = False, **kwargs):
         if attention_mask is not None:
@@ -172,46 +216,29 @@ class NeuralAttentionSearchLinearAttnGDN(nn.Module):
             selector_input = cache.update_attn_types(input_hidden_states=hidden_states)
         else:
             selector_input = hidden_states
-        if selector_input is not None:
-            raw_types, _, _ = self.select_ops(selector_input, cu_seqlens, force_last_block=False)
-        else:
-            raw_types = torch.ones(B, 1, self.num_nats_head, self.n_ops, device=hidden_states.device, dtype=hidden_states.dtype)
-
+        fast = fast_front(self, 'gdn', hidden_states, cache, cu_seqlens) if mode == 'chunk' and selector_input is not None else None
+        types = n_nats_blocks = None
         conv_states = cache.conv_state if cache is not None and cache.conv_state is not None else (None, None, None)
-        new_conv_states = []
-
-        def conv_or_act(x, conv, state):
-            if self.use_short_conv:
-                y, final = conv(x=x, cache=state, output_final_state=bool(use_cache), cu_seqlens=cu_seqlens)
-                new_conv_states.append(final)
-                return y
-            return F.silu(x)
-
-        if self.attn_with_short_conv:
-            q = conv_or_act(self.q_proj(hidden_states), getattr(self, 'q_conv1d', None), conv_states[0])
-            k = conv_or_act(self.k_proj(hidden_states), getattr(self, 'k_conv1d', None), conv_states[1])
-            v = conv_or_act(self.v_proj(hidden_states), getattr(self, 'v_conv1d', None), conv_states[2])
-            q_attn, k_attn, v_attn = q, k, v
+        if fast is not None:
+            whole = selector_input is hidden_states
+            q, k, v, gate, ab, pooled = fast.project(hidden_states, self.nats_block_size if whole else 0)
+            if not whole:
+                pooled = nats_util.mean_pooling(selector_input, self.nats_block_size)
+            logits = self.nats_layer(pooled).unflatten(-1, (self.num_nats_head, self.n_ops))
+            types, n_nats_blocks = fast.select(logits, True)
+            # (the types before the last block is forced are only needed where states are handed on)
+            raw_types = fast.select(logits, False)[0] if use_cache or cache is not None else types
+            q, k, v, q_attn, k_attn, o_mix, _, _, _, new_conv_states = fast.conv_norm(q, k, v, conv_states, bool(use_cache))
+            v_attn = v
+            g, beta, _ = fast.gates(ab)
+            q, k = (x.unflatten(-1, (-1, self.head_k_dim)) for x in (q, k))
+            v = v.unflatten(-1, (-1, self.head_v_dim))
+            q_attn, k_attn = (x.unflatten(-1, (-1, self.head_attn_k_dim)) for x in (q_attn, k_attn))
+            v_attn = v_attn.unflatten(-1, (-1, self.head_attn_v_dim))
         else:
-            q_attn, k_attn, v_attn = self.q_proj(hidden_states), self.k_proj(hidden_states), self.v_proj(hidden_states)
-            q = conv_or_act(q_attn, getattr(self, 'q_conv1d', None), conv_states[0])
-            k = conv_or_act(k_attn, getattr(self, 'k_conv1d', None), conv_states[1])
-            v = conv_or_act(v_attn, getattr(self, 'v_conv1d', None), conv_states[2])
-        o_weights = self.nats_out_weights_layer(q).unflatten(-1, (self.num_attn_heads, self.n_ops)).softmax(-1)
-
-        q, k = (x.unflatten(-1, (-1, self.head_k_dim)) for x in (q, k))
-        v = v.unflatten(-1, (-1, self.head_v_dim))
-        q_attn, k_attn = (x.unflatten(-1, (-1, self.head_attn_k_dim)) for x in (q_attn, k_attn))
-        v_attn = v_attn.unflatten(-1, (-1, self.head_attn_v_dim))
-        if self.num_v_heads > self.num_heads:
-            q, k = (x.repeat_interleave(self.num_v_heads // self.num_heads, dim=-2) for x in (q, k))
-        if self.attn_qk_norm:
-            q_attn, k_attn = self.q_norm(q_attn), self.k_norm(k_attn)
-
-        beta = self.b_proj(hidden_states).sigmoid()
-        if self.allow_neg_eigval:
-            beta = beta * 2.
-        g = -self.A_log.float().exp() * F.softplus(self.a_proj(hidden_states).float() + self.dt_bias)
+            q, k, v, q_attn, k_attn, v_attn, o_mix, g, beta, raw_types, new_conv_states = self._general_front(
+                hidden_states, selector_input, conv_states, use_cache, cu_seqlens)
+            gate = None
 
         state, state_block_start, g_cumsum = None, None, None
         k_new, v_new, g_new = k_attn, v_attn, g
@@ -243,11 +270,12 @@ class NeuralAttentionSearchLinearAttnGDN(nn.Module):
                       lattn_use_qk_l2norm_in_kernel=True)
         if mode == 'chunk':
             # the last block runs both ops so that its state is recorded (reference :547-555, :577-583)
-            types = raw_types.clone()
-            last_type = types[:, -1].clone()
-            types[:, -1] = 1
-            n_nats_blocks = types.to(torch.int32).sum(1)
-            self.attn_fraction = (n_nats_blocks.float()[..., 0] / types.shape[1]).mean(0).detach()
+            last_type = raw_types[:, -1].clone() if types is None else raw_types[:, -1]
+            if types is None:
+                types = raw_types.clone()
+                types[:, -1] = 1
+                n_nats_blocks = types.to(torch.int32).sum(1)
+            self.attn_fraction = n_nats_blocks[..., 0].sum(0).float() / (types.shape[1] * B)
             if self.training:
                 o_lin, o_attn, state = nats_mixed_attn_gdn(
                     initial_state_gated_delta=state, nats_block_types=types, n_nats_blocks=n_nats_blocks,
@@ -270,10 +298,12 @@ class NeuralAttentionSearchLinearAttnGDN(nn.Module):
 
         if cache is not None:
             cache.update(recurrent_state=state, recurrent_state_block_start=state_block_start, attn_state=(k_new, v_new),
-                         conv_state=tuple(new_conv_states) if self.use_short_conv else None, nats_block_types=raw_types,
+                         conv_state=new_conv_states, nats_block_types=raw_types,
                          l_attn_state=(k, v), g=g_new, n_new_tokens=q_len)
 
+        if fast is not None:
+            return fast.tail(o_lin.reshape(o_attn.shape), o_attn, gate.view(o_attn.shape), o_mix), None, past_key_values
         gate = self.g_proj(hidden_states).unflatten(-1, (-1, self.head_v_dim))
-        o = self.o_norm(o_lin.reshape(o_attn.shape), o_attn, gate.reshape(o_attn.shape), o_weights)
+        o = self.o_norm(o_lin.reshape(o_attn.shape), o_attn, gate.reshape(o_attn.shape), o_mix)
         o = self.o_proj(o.flatten(-2))
         return o, None, past_key_values

@@ -1,0 +1,95 @@
+"""The layers' fused front and tail (_front.FastFront) against their general path of single submodules: outputs, gradients and caches;
+and the weight-gradient kernel against an fp32 product at the edges of its tiles."""
+import pytest
+import torch
+
+from tests._util import rel_l2
+from tests.test_gpu_layer_step import _generate, _layer
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda:0'
+
+
+def _general(monkeypatch):
+    from neuralattentionsearchlinear_amd import natsl_attn_gdn, natsl_attn_mamba2
+    for mod in (natsl_attn_gdn, natsl_attn_mamba2):
+        monkeypatch.setattr(mod, 'fast_front', lambda *a: None)
+
+
+@pytest.mark.parametrize("kind,geometry,B,T,more", [
+    ('gdn', None, 1, 64, {}), ('gdn', '340M', 2, 333, {}), ('gdn', '760M', 1, 200, dict(allow_neg_eigval=True, conv_bias=True)),
+    ('gdn', None, 3, 130, dict(conv_size=3, conv_activation=None)), ('gdn', None, 2, 65, dict(conv_size=2)),
+    ('mamba', None, 2, 257, {}), ('mamba', None, 1, 100, dict(attn_qk_norm=True, conv_bias=True)),
+])
+def test_front_matches_the_general_path(kind, geometry, B, T, more, monkeypatch):
+    layer = _layer(kind, geometry, 'all', **more).train()
+    torch.manual_seed(T)
+    x0 = torch.randn(B, T, layer.hidden_size, device=DEV).bfloat16()
+    do = torch.randn_like(x0)
+
+    def run():
+        x = x0.clone().requires_grad_(True)
+        layer.zero_grad(set_to_none=True)
+        o = layer(x)
+        o = o[0] if isinstance(o, tuple) else o
+        o.backward(do)
+        return dict({n: p.grad for n, p in layer.named_parameters()}, x=x.grad, out=o.detach(), fraction=layer.attn_fraction)
+    fast = run()
+    _general(monkeypatch)
+    slow = run()
+    for n, b in slow.items():
+        a = fast[n]
+        assert a is not None and a.shape == b.shape and a.dtype == b.dtype, n
+        # Both sides round to bf16 on the way (2^-9 relative each time); sums that the fused steps keep in fp32 are rounded once
+        # more in the general path.  The selector's gradient is a sum of terms that largely cancel: ten times that.
+        tol = 5e-2 if n == 'nats_layer.weight' else 1e-2
+        assert rel_l2(a.float(), b.float()) <= tol, f"{n}: rel-L2 {rel_l2(a.float(), b.float()):.3e}"
+
+
+@pytest.mark.parametrize("kind,T0,sizes", [('gdn', 128, (1, 70)), ('gdn', 100, (64,)), ('mamba', 131, (2, 100))])
+def test_front_on_a_cache(kind, T0, sizes, monkeypatch):
+    """Prefill and a second prompt: the same outputs and convolution states as the general path."""
+    layer = _layer(kind, None, 'all')
+    torch.manual_seed(T0)
+    x = torch.randn(2, T0 + sum(sizes), layer.hidden_size, device=DEV).bfloat16()
+    fast, cf = _generate(layer, kind, x, T0, sizes)
+    _general(monkeypatch)
+    slow, cs = _generate(layer, kind, x, T0, sizes)
+    for a, b in zip(fast + list(cf.conv_state), slow + list(cs.conv_state)):
+        assert rel_l2(a.float(), b.float()) <= 5e-3
+    assert torch.equal(cf.n_attn_blocks, cs.n_attn_blocks)
+
+
+@pytest.mark.parametrize("T,D,widths", [(1, 8, (8,)), (31, 64, (16, 24)), (32, 256, (256,)), (33, 264, (264, 8)), (129, 72, (512,)), (5000, 128, (136,))])
+def test_weight_grads(T, D, widths):
+    """natsl_wgrad at the edges of its 32-token stages, 256-wide tiles and token slices."""
+    from neuralattentionsearchlinear_amd._front import weight_grads
+    torch.manual_seed(T)
+    x = torch.randn(T, D, device=DEV).bfloat16()
+    dys = [torch.randn(T, n, device=DEV).bfloat16() for n in widths]
+    out = weight_grads(x, dys)
+    again = weight_grads(x, dys)
+    for dy, a, b in zip(dys, out, again):
+        ref = dy.double().t() @ x.double()
+        # exact products, fp32 sums (T 2^-24 of the sum of magnitudes, far below), one rounding to bf16
+        assert bool(((a.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * T ** 0.5).all()), float((a.double() - ref).abs().max())
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("B,T,D,N,block,pool", [(1, 1, 8, 16, 64, True), (2, 100, 264, 32, 64, True), (1, 70, 1032, 0, 256, True), (3, 33, 64, 16, 64, False)])
+def test_dx_init(B, T, D, N, block, pool):
+    from neuralattentionsearchlinear_amd import _capi
+    torch.manual_seed(D)
+    nb = -(-T // block)
+    dn, w = torch.randn(B * T, max(N, 16), device=DEV).bfloat16(), torch.randn(max(N, 1), D, device=DEV).bfloat16()
+    dp = torch.randn(B, nb, D, device=DEV).bfloat16()
+    dx = torch.full((B, T, D), float('nan'), device=DEV).bfloat16()
+    P = _capi.ptr
+    _capi.check(_capi.lib().natsl_dx_init(P(dn) if N else None, P(w) if N else None, P(dp) if pool else None, P(dx), B, T, D, N, max(N, 16), block,
+                                          _capi.stream_ptr(dx.device)), "natsl_dx_init")
+    ref = (dn[:, :N].double() @ w[:N].double()).view(B, T, D) if N else torch.zeros(B, T, D, device=DEV, dtype=torch.float64)
+    if pool:
+        lens = torch.full((nb,), block, device=DEV, dtype=torch.float64)
+        lens[-1] = T - (nb - 1) * block
+        ref = ref + (dp.double() / lens.view(1, nb, 1)).repeat_interleave(block, 1)[:, :T]
+    assert bool(((dx.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5).all())

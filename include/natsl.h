@@ -359,6 +359,14 @@ int natsl_kv_compact(const void* src_k, const void* src_v, long long src_tokens,
                      int HN, int K, int V, int dtype, int block, int NB, int n_complete, int tail_dst, int tail_tokens,
                      natsl_stream_t stream);
 
+/* The cache's bookkeeping around natsl_kv_compact: n_after [B, HN] = n_before (or 0) + the attention-typed blocks among the first
+ * n_complete of types [B, NB, HN, 2], with the largest of them written to *host_max (HOST memory that the GPU can write); and the
+ * validity flags valid [B, blocks, HN] of n_after kept blocks plus the incomplete block at tail_block (-1 = none).
+ * src/nats/models/utils.py:509-588. */
+int natsl_kv_counts(const void* types, int types_dtype, const int64_t* n_before, int64_t* n_after, int32_t* host_max, int B, int HN, int NB,
+                    int n_complete, natsl_stream_t stream);
+int natsl_kv_flags(const int64_t* n_after, uint8_t* valid, int B, int blocks, int HN, int tail_block, natsl_stream_t stream);
+
 /* The layers' short convolutions with what follows them, for up to NATSL_CONV_SEGS bf16 tensors [B, T, D_i] in one launch:
  *   y = act(conv(x)) (as natsl_short_conv_fwd; bf16 weights [D, W]), and, when y_norm is given, its rows of 8 * norm_lanes
  *   channels (a power of two of lanes) normalised: y rsqrt(mean y^2 + eps) norm_weight, or y rsqrt(sum y^2 + eps) (norm_l2).

@@ -14,7 +14,7 @@ import torch
 import torch.nn.functional as F
 
 from . import _capi
-from ._layer_step import _PARAMS, _parameters
+from ._layer_step import _PARAMS, watch
 from .modules import _NORM_GATE_WIDTHS
 
 _NAMES = [p[0] for p in _PARAMS]
@@ -328,7 +328,7 @@ class _Select(torch.autograd.Function):
 
 
 class FastFront:
-    """The layer's current parameters and constants for one forward (and the backward that follows it)."""
+    """A layer's parameters and constants, as long as it holds these parameters (_layer_step.watch)."""
 
     def __init__(self, layer, kind, params):
         self.w = w = dict(zip(_NAMES, params))
@@ -382,24 +382,19 @@ class FastFront:
         return linear(y.flatten(-2), self.w["wo"])
 
 
-def fast_front(layer, kind, x, cache, cu_seqlens):
-    """The layer's FastFront for this forward, or None where the general path has to run."""
-    if not x.is_cuda or x.dtype != torch.bfloat16 or cu_seqlens is not None or not x.is_contiguous() or x.numel() == 0 or \
-            torch.is_autocast_enabled():
-        return None
-    params = _parameters(layer)
-    if params is None or not layer.use_short_conv or layer.num_v_heads != layer.num_heads:
-        return None
+def _front_plan(layer, kind, seen):
+    """The layer's FastFront, or None where its weights or options are not what the fused steps are built for."""
+    w = dict(zip(_NAMES, seen.tensors))
     delta = kind == 'gdn'
-    if layer.attn_with_short_conv != delta or (delta and not layer.attn_qk_norm):
+    if not layer.use_short_conv or layer.num_v_heads != layer.num_heads or layer.attn_with_short_conv != delta or (delta and not layer.attn_qk_norm):
         return None
-    w = dict(zip(_NAMES, params))
     for n, t in w.items():
         if t is None:
             if n.startswith("conv_b") or (not delta and n in ("wb", "norm_q", "norm_k")):
                 continue
             return None
-        if t.device != x.device or not t.is_contiguous() or (t.dtype != torch.bfloat16 and (n not in _EITHER or t.dtype != torch.float32)):
+        if not t.is_cuda or t.device != w["wq"].device or not t.is_contiguous() or \
+                (t.dtype != torch.bfloat16 and (n not in _EITHER or t.dtype != torch.float32)):
             return None
     if w["a_log"].dtype != w["dt_bias"].dtype or w["out_norm1"].dtype != w["out_norm2"].dtype or (delta and w["norm_q"].dtype != w["norm_k"].dtype):
         return None
@@ -414,10 +409,26 @@ def fast_front(layer, kind, x, cache, cu_seqlens):
     if norms[0].eps != norms[1].eps or width not in (32, 64, 128, 256, 512) or layer.head_attn_v_dim not in _NORM_GATE_WIDTHS or \
             layer.hidden_size % 8 or layer.num_heads > 256 or layer.value_dim % 8:
         return None
+    return FastFront(layer, kind, seen.tensors)
+
+
+def fast_front(layer, kind, x, cache, cu_seqlens):
+    """The layer's FastFront for this forward, or None where the general path has to run."""
+    if not x.is_cuda or x.dtype != torch.bfloat16 or cu_seqlens is not None or not x.is_contiguous() or x.numel() == 0 or \
+            torch.is_autocast_enabled():
+        return None
+    seen = watch(layer)
+    if seen is None:
+        return None
+    if seen.front_plan is None:
+        seen.front_plan = (_front_plan(layer, kind, seen),)
+    f = seen.front_plan[0]
+    if f is None or f.w["wq"].device != x.device:
+        return None
     if cache is not None:
-        if torch.is_grad_enabled() and (x.requires_grad or any(t is not None and t.requires_grad for t in params)):
+        if torch.is_grad_enabled() and (x.requires_grad or any(t is not None and t.requires_grad for t in seen.tensors)):
             return None
         st = cache.conv_state
         if st is not None and any(s is not None and (s.dtype != torch.bfloat16 or not s.is_contiguous() or s.shape[0] != x.shape[0]) for s in st):
             return None
-    return FastFront(layer, kind, params)
+    return f

@@ -10,6 +10,7 @@ general path runs.
 from __future__ import annotations
 
 import ctypes
+import weakref
 
 import torch
 import torch.nn as nn
@@ -50,30 +51,68 @@ _OPTIONAL = {"wb", "norm_q", "norm_k", "conv_bq", "conv_bk", "conv_bv"}
 _EITHER_DTYPE = {"norm_q", "norm_k", "a_log", "dt_bias", "out_norm1", "out_norm2"}       # the others are bf16
 
 
-def _parameters(layer):
-    """The current weight tensors by field (None where the layer has none), or None when a submodule is not the plain one."""
-    mods, own = layer._modules, layer._parameters
-    out = []
-    for _, mod, name, kind in _PARAMS:
-        if mod is None:
-            out.append(own.get(name))
-            continue
-        m = mods.get(mod)
-        if m is None:
-            out.append(None)
-            continue
-        if kind is not None and (type(m) is not kind or m._forward_hooks or m._forward_pre_hooks or 'forward' in m.__dict__):
-            return None
-        out.append(m._parameters.get(name))
-    return out
+# by layer, outside of it: a copied or saved layer takes nothing of this along
+_watches = weakref.WeakKeyDictionary()
+
+
+class _Watch:
+    """A layer's weight tensors by field, and a quick way to see that they are still the ones: same submodules, unhooked, holding
+    the same tensors at the same addresses."""
+
+    def __init__(self, layer):
+        mods = layer._modules
+        self.tensors, self.plain = [], True
+        self.mods, self.held = {}, []
+        for _, mod, name, kind in _PARAMS:
+            if mod is None:
+                where = layer._parameters
+            else:
+                m = mods.get(mod)
+                self.mods[mod] = m
+                if m is None:
+                    self.tensors.append(None)
+                    continue
+                if kind is not None and type(m) is not kind:
+                    self.plain = False
+                where = m._parameters
+            t = where.get(name)
+            self.tensors.append(t)
+            self.held.append((where, name, t, 0 if t is None else t.data_ptr()))
+        self.unhooked = [(m._forward_hooks, m._forward_pre_hooks, m.__dict__) for m in self.mods.values() if m is not None]
+        self.step_plan = self.front_plan = None
+
+    def holds(self, layer):
+        mods = layer._modules
+        for n, m in self.mods.items():
+            if mods.get(n) is not m:
+                return False
+        for where, name, t, at in self.held:
+            if where.get(name) is not t or (t is not None and t.data_ptr() != at):
+                return False
+        return True
+
+    def hooked(self):
+        for a, b, d in self.unhooked:
+            if a or b or 'forward' in d:
+                return True
+        return False
+
+
+def watch(layer):
+    """The layer's _Watch, made anew when a weight or submodule has been replaced; None when a submodule is not the plain one."""
+    w = _watches.get(layer)
+    if w is None or not w.holds(layer):
+        w = _watches[layer] = _Watch(layer)
+    return None if not w.plain or w.hooked() else w
 
 
 class _Plan:
     """What stays the same from step to step: the weights' addresses, the geometry and the mode."""
 
-    def __init__(self, layer, kind, key, params):
-        self.key = key
+    def __init__(self, layer, kind, seen):
         self.built = False
+        self.ws_bytes = {}
+        params = seen.tensors
         s = self.fixed = LayerStep()
         by = dict(zip((p[0] for p in _PARAMS), params))
         delta = kind == 'gdn'
@@ -133,13 +172,12 @@ def layer_step(layer, kind, x, cache):
     B, T, D = x.shape
     if B * T > MAX_ROWS or T < 1 or x.dtype != torch.bfloat16 or torch.is_grad_enabled() and _wants_grad(layer, x) or torch.is_autocast_enabled():
         return None
-    params = _parameters(layer)
-    if params is None:
+    seen = watch(layer)
+    if seen is None:
         return None
-    key = tuple([None if t is None else (t.data_ptr(), t.dtype) for t in params])
-    plan = layer.__dict__.get('_step_plan')
-    if plan is None or plan.key != key:
-        plan = layer.__dict__['_step_plan'] = _Plan(layer, kind, key, params)
+    plan = seen.step_plan
+    if plan is None:
+        plan = seen.step_plan = _Plan(layer, kind, seen)
     if not plan.built:
         return None
     bs, n_in, n_kept = cache.nats_block_size, cache._n_tokens_in_nats_block, cache.n_attn_blocks_max
@@ -159,7 +197,8 @@ def layer_step(layer, kind, x, cache):
     if n_in + T == bs:
         types, _, _ = layer.select_ops(cache.update_attn_types(input_hidden_states=x), None, force_last_block=False)
         types = types.contiguous()
-    cache._grow(cache.n_attn_tokens_max + T)
+    if cache.attn_k.shape[1] < cache.n_attn_tokens_max + T:
+        cache._grow(cache.n_attn_tokens_max + T)
     x = x.contiguous()
     dev = x.device
     s = LayerStep.from_buffer_copy(f)
@@ -188,14 +227,21 @@ def layer_step(layer, kind, x, cache):
         s.types, s.types_dtype = types.data_ptr(), _capi.dtype_code(types.dtype)
     L = _capi.lib()
     ref = ctypes.byref(s)
-    ws = torch.empty(L.natsl_layer_step_workspace_bytes(ref), dtype=torch.uint8, device=dev)
-    _capi.check(L.natsl_layer_step_fwd(ref, ws.data_ptr(), ws.numel(), _capi.stream_ptr(dev)), "natsl_layer_step_fwd")
+    ws_bytes = plan.ws_bytes.get((B, T))
+    if ws_bytes is None:
+        # (enough for every state of the cache: the attention's splits are bounded)
+        ws_bytes = plan.ws_bytes[(B, T)] = L.natsl_layer_step_workspace_bytes(ref)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    rc = L.natsl_layer_step_fwd(ref, ws.data_ptr(), ws_bytes, _capi.stream_ptr(dev))
+    if rc:
+        _capi.check(rc, "natsl_layer_step_fwd")
     if types is None:
         cache.note_step(state_out, start, new_conv, g_out, T)
     else:
         cache.update(recurrent_state=state_out, recurrent_state_block_start=start, attn_state=(cache.attn_k, cache.attn_v), conv_state=new_conv,
                      nats_block_types=types, g=cache.lattn_g, n_new_tokens=T)
-    layer.last_recurrent_state, layer.last_block_start_state = state_out, start
+    attrs = layer.__dict__
+    attrs['last_recurrent_state'], attrs['last_block_start_state'] = state_out, start
     return out
 
 

@@ -17,6 +17,7 @@ blocks, so the cache never holds the blocks the selector dropped.
 """
 from __future__ import annotations
 
+import threading
 from typing import Any, Dict, List, Optional, Tuple
 
 import torch
@@ -26,6 +27,26 @@ from . import _capi
 
 def _cdiv(a: int, b: int) -> int:
     return -(-a // b)
+
+
+class _HostNumbers:
+    """Numbers that kernels write for the host: a few words of pinned memory per device, handed out in turn (one is in use from
+    foresee() to the _compact() that follows it)."""
+    SLOTS = 256
+
+    def __init__(self):
+        self.lock, self.words, self.next = threading.Lock(), {}, 0
+
+    def take(self, device: torch.device):
+        with self.lock:
+            words = self.words.get(device)
+            if words is None:
+                words = self.words[device] = torch.zeros(self.SLOTS, dtype=torch.int32, pin_memory=True)
+            self.next = (self.next + 1) % self.SLOTS
+            return words[self.next:self.next + 1]
+
+
+_host_numbers = _HostNumbers()
 
 
 class NAtSLayerCache:
@@ -66,6 +87,7 @@ class NAtSLayerCache:
         self.g_cumsum = None                             # [B, 1, H]: sum of g over the incomplete block
         self.n_observed_tokens = 0
         self._pending_first = None                       # K/V of the first forward, kept until update() has the types
+        self._foreseen = None                            # counts on their way to the host (foresee)
 
     # ------------------------------------------------------------------------------------------------
     def update_attn_types(self, input_hidden_states: torch.Tensor) -> Optional[torch.Tensor]:
@@ -142,6 +164,8 @@ class NAtSLayerCache:
             buf = torch.zeros(old.shape[0], new_cap, *old.shape[2:], dtype=old.dtype, device=old.device)
             buf[:, :cap] = old
             setattr(self, name, buf)
+        if self.valid_attn_tokens is None:
+            return
         flags = torch.zeros(self.valid_attn_tokens.shape[0], new_cap // bs, self.valid_attn_tokens.shape[2], dtype=torch.bool,
                             device=self.valid_attn_tokens.device)
         flags[:, :self.valid_attn_tokens.shape[1]] = self.valid_attn_tokens
@@ -212,10 +236,13 @@ class NAtSLayerCache:
             types = types.float()
         types = types.contiguous()
         B, NB, HN, _ = types.shape
-        new_blocks = (torch.round(types[:, :n_complete, :, self.attn_offset].float()) == 1).sum(1)                     # int64 [B, HN]
         before = self.n_attn_blocks
-        after = new_blocks if before is None else before + new_blocks
-        new_max = int(after.max()) if after.numel() else 0                                        # one host sync per completed block
+        foreseen, self._foreseen = self._foreseen, None
+        if foreseen is None or foreseen[0] is not nats_block_types or foreseen[1] != n_complete:
+            foreseen = self._count(nats_block_types, types, n_complete)
+        _, _, after, host, ready = foreseen
+        ready.synchronize()                                                     # the host needs the largest count to size the cache
+        new_max = int(host)
         tail_dst = new_max if tail_tokens else -1
         if self.attn_k is None:
             src_k, src_v = (t.contiguous() for t in (self._pending_first if self._pending_first is not None else attn_state))
@@ -223,7 +250,6 @@ class NAtSLayerCache:
             cap = (new_max + 2) * bs
             self.attn_k = torch.zeros(B, cap, *src_k.shape[2:], dtype=src_k.dtype, device=src_k.device)
             self.attn_v = torch.zeros(B, cap, *src_v.shape[2:], dtype=src_v.dtype, device=src_v.device)
-            self.valid_attn_tokens = torch.zeros(B, cap // bs, HN, dtype=torch.bool, device=src_k.device)
             src_block0 = 0
         else:
             src_k, src_v, src_block0 = self.attn_k, self.attn_v, self.n_attn_blocks_max
@@ -242,10 +268,33 @@ class NAtSLayerCache:
         _capi.check(rc, "natsl_kv_compact")
         self.n_attn_blocks = after
         self.n_attn_blocks_max = new_max
-        idx = torch.arange(self.valid_attn_tokens.shape[1], device=after.device).view(1, -1, 1)
-        self.valid_attn_tokens = idx < after.unsqueeze(1)
-        if tail_tokens:
-            self.valid_attn_tokens[:, new_max] = True
+        blocks = self.attn_k.shape[1] // bs
+        self.valid_attn_tokens = torch.empty(B, blocks, HN, dtype=torch.bool, device=after.device)
+        rc = _capi.lib().natsl_kv_flags(_capi.ptr(after), _capi.ptr(self.valid_attn_tokens), B, blocks, HN, tail_dst, _capi.stream_ptr(after.device))
+        _capi.check(rc, "natsl_kv_flags")
+
+    def _count(self, key, types, n_complete: int):
+        """Enqueue the kept-block counts after this update; -> (key, n_complete, counts, the largest one's place on the host, event)."""
+        B, NB, HN, _ = types.shape
+        before = self.n_attn_blocks
+        if before is not None:
+            before = before.to(torch.int64).contiguous()
+        after = torch.empty(B, HN, dtype=torch.int64, device=types.device)
+        host = _host_numbers.take(types.device)
+        rc = _capi.lib().natsl_kv_counts(_capi.ptr(types), _capi.dtype_code(types.dtype), _capi.ptr(before), after.data_ptr(), host.data_ptr(), B, HN, NB,
+                                         n_complete, _capi.stream_ptr(types.device))
+        _capi.check(rc, "natsl_kv_counts")
+        ready = torch.cuda.Event()
+        ready.record(torch.cuda.current_stream(types.device))
+        return key, n_complete, after, host, ready
+
+    def foresee(self, nats_block_types: torch.Tensor, n_new_tokens: int):
+        """Called by a forward as soon as it knows the new blocks' types: the counts update() needs on the host are enqueued here, so
+        that update() waits for the selector only and not for everything enqueued since."""
+        total, bs = n_new_tokens + self._n_tokens_in_nats_block, self.nats_block_size
+        ok = nats_block_types.is_cuda and nats_block_types.is_contiguous() and nats_block_types.dtype in (torch.float32, torch.bfloat16)
+        if ok and total >= bs and nats_block_types.shape[1] == _cdiv(total, bs):
+            self._foreseen = self._count(nats_block_types, nats_block_types.detach(), total // bs)
 
     def note_step(self, recurrent_state, recurrent_state_block_start, conv_state, g_cumsum, n_new_tokens: int):
         """What update() does for tokens that stay inside the incomplete block, where the step itself has written the cache's
@@ -309,7 +358,7 @@ class NAtSLayerCache:
             self.block_type_state_logits = None
             self.recurrent_state = self.recurrent_state_block_start
             self.recurrent_state_block_start = None
-        elif self.valid_attn_tokens is not None:
+        elif total < bs and self.valid_attn_tokens is not None:
             self.valid_attn_tokens[:, self.n_attn_blocks_max] = True
         if conv_state is not None:
             self.conv_state = conv_state

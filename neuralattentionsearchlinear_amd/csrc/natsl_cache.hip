@@ -110,6 +110,45 @@ __global__ __launch_bounds__(256) void kv_compact_kernel(KvCompactParams p) {
   }
 }
 
+// ---- bookkeeping of the kept blocks ----------------------------------------------------------------------------------------
+// after[b][hn] = before + attention-typed blocks among the first n_complete, and the largest of them to *host_max (host memory the
+// GPU can write: the host needs that one number to size the cache and would otherwise wait for everything enqueued before it asks).
+// One workgroup; a wave takes a (sequence, head) pair at a time, its lanes the blocks.
+__global__ __launch_bounds__(1024) void kv_counts_kernel(const void* types, const int dtype, const int64_t* before, int64_t* after, int* host_max,
+                                                         const int pairs, const int HN, const int NB, const int n_complete) {
+  __shared__ int top[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int most = 0;
+  for (int i = wave; i < pairs; i += 16) {
+    const int b = i / HN, hn = i % HN;
+    int n = 0;
+    for (int c = lane; c < n_complete; c += 64) {
+      const size_t at = (((size_t)b * NB + c) * HN + hn) * 2;
+      const float t = dtype == NATSL_F32 ? reinterpret_cast<const float*>(types)[at] : bf16_to_f32(reinterpret_cast<const bf16_t*>(types)[at]);
+      n += rintf(t) == 1.f;
+    }
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) n += __shfl_xor(n, d);
+    const int64_t total = n + (before ? before[i] : 0);
+    if (lane == 0) after[i] = total;
+    most = max(most, (int)total);
+  }
+  if (lane == 0) top[wave] = most;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; ++w) most = max(most, top[w]);
+    *host_max = most;
+    __threadfence_system();
+  }
+}
+// valid[b][i][hn]: kept blocks, and the incomplete block at `tail` (-1: none)
+__global__ __launch_bounds__(256) void kv_flags_kernel(const int64_t* after, uint8_t* valid, const long long n, const int HN, const int blocks, const int tail) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int hn = (int)(i % HN), blk = (int)(i / HN % blocks), b = (int)(i / ((long long)HN * blocks));
+  valid[i] = blk < after[(size_t)b * HN + hn] || blk == tail;
+}
+
 }  // namespace natsl
 
 using namespace natsl;
@@ -148,5 +187,26 @@ extern "C" int natsl_kv_compact(const void* src_k, const void* src_v, long long 
   p.tail_dst = tail_dst; p.tail_tokens = tail_tokens;
   p.wgs[0] = cdiv(block * (p.row[0] / 16), 256); p.wgs[1] = cdiv(block * (p.row[1] / 16), 256);
   hipLaunchKernelGGL(kv_compact_kernel, dim3(p.wgs[0] + p.wgs[1], B * HKV), dim3(256), 0, (hipStream_t)stream, p);
+  return check_launch(what);
+}
+
+extern "C" int natsl_kv_counts(const void* types, int types_dtype, const int64_t* n_before, int64_t* n_after, int32_t* host_max, int B, int HN, int NB,
+                               int n_complete, natsl_stream_t stream) {
+  const char* what = "natsl_kv_counts";
+  if (!types || !n_after || !host_max) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
+  if (B <= 0 || HN <= 0 || NB <= 0 || n_complete < 0 || n_complete > NB) return fail(NATSL_ERR_INVALID, "%s: bad dimension", what);
+  if (types_dtype != NATSL_BF16 && types_dtype != NATSL_F32) return fail(NATSL_ERR_UNSUPPORTED, "%s: block types must be f32 or bf16", what);
+  hipLaunchKernelGGL(kv_counts_kernel, dim3(1), dim3(1024), 0, reinterpret_cast<hipStream_t>(stream), types, types_dtype, n_before, n_after, host_max,
+                     B * HN, HN, NB, n_complete);
+  return check_launch(what);
+}
+
+extern "C" int natsl_kv_flags(const int64_t* n_after, uint8_t* valid, int B, int blocks, int HN, int tail_block, natsl_stream_t stream) {
+  const char* what = "natsl_kv_flags";
+  if (!n_after || !valid) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
+  if (B <= 0 || HN <= 0 || blocks <= 0) return fail(NATSL_ERR_INVALID, "%s: non-positive dimension", what);
+  const long long n = (long long)B * blocks * HN;
+  hipLaunchKernelGGL(kv_flags_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), n_after, valid, n, HN, blocks,
+                     tail_block);
   return check_launch(what);
 }

@@ -66,7 +66,7 @@ __global__ __launch_bounds__(256) void attend_and_recur_kernel(const AttnParams 
 int attend_splits(int queries, int TK) {
   int want = cdiv(1024, queries), most = cdiv(TK, 4 * KEYS_PER_CHUNK);
   if (want > most) want = most;
-  return want < 1 ? 1 : want > 16 ? 16 : want;
+  return want < 1 ? 1 : want > ATTEND_MAX_SPLITS ? ATTEND_MAX_SPLITS : want;
 }
 
 int launch_attend_and_recur(const char* what, const AttnParams& a, const RecurrentParams& r, bool delta, int K, int KA, int VA, hipStream_t s) {

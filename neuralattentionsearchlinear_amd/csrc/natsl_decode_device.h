@@ -200,22 +200,35 @@ NATSL_DEVICE void attend(const AttnParams& p, const int b, const int tq, const i
   for (int j = 0; j < CPL; ++j) st_any(p.o, F32 ? NATSL_F32 : NATSL_BF16, row * DV + CPL * lane + j, o[j] * inv);
 }
 
-// (m, l, acc) of the splits of one query row, written by one workgroup each as [2 + DV] floats: the joined, normalised
-// columns CPL*lane.. of the row; a row that saw no key gives 0
+// (m, l, acc) of the splits (at most 64) of one query row, written by one workgroup each as [2 + DV] floats: the joined, normalised
+// columns CPL*lane.. of the row; a row that saw no key gives 0.  Lane s holds split s's weight, so that the maxima are one round
+// trip to memory and the partial rows another.
 template <int DV>
 NATSL_DEVICE void join_splits(const float* src, const int nsplit, float* o) {
-  constexpr int CPL = DV / 64;
+  constexpr int CPL = DV / 64, U = 4;
   const int lane = threadIdx.x & 63;
-  float m = -INFINITY, l = 0.f;
-  for (int s = 0; s < nsplit; ++s) m = fmaxf(m, src[s * (2 + DV)]);
+  const float ms = lane < nsplit ? src[lane * (2 + DV)] : -INFINITY, ls = lane < nsplit ? src[lane * (2 + DV) + 1] : 0.f;
+  float m = ms;
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
+  const float f = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - m);
+  float l = f * ls;
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) l += __shfl_xor(l, d);
 #pragma unroll
   for (int j = 0; j < CPL; ++j) o[j] = 0.f;
-  for (int s = 0; s < nsplit; ++s) {
-    const float* ps = src + s * (2 + DV);
-    const float f = ps[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ps[0] - m);
-    l += f * ps[1];
+  for (int s = 0; s < nsplit; s += U) {
+    float v[U][CPL];
 #pragma unroll
-    for (int j = 0; j < CPL; ++j) o[j] += f * ps[2 + CPL * lane + j];
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < CPL; ++j) v[u][j] = src[min(s + u, nsplit - 1) * (2 + DV) + 2 + CPL * lane + j];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float fu = s + u < nsplit ? __shfl(f, s + u) : 0.f;
+#pragma unroll
+      for (int j = 0; j < CPL; ++j) o[j] += fu * v[u][j];
+    }
   }
   const float inv = l > 0.f ? 1.f / l : 0.f;
 #pragma unroll
@@ -396,6 +409,7 @@ NATSL_DEVICE void recurrent_columns(const RecurrentParams& p, const int nh, cons
 
 // Both halves of a decode step in one launch (natsl_decode.hip); K, V: the linear branch's widths in r, KA, VA the attention's.
 int launch_attend_and_recur(const char* what, const AttnParams& a, const RecurrentParams& r, bool delta, int K, int KA, int VA, hipStream_t s);
-int attend_splits(int queries, int TK);   // splits per query of that launch
+constexpr int ATTEND_MAX_SPLITS = 16;
+int attend_splits(int queries, int TK);   // splits per query of that launch, at most ATTEND_MAX_SPLITS
 
 }  // namespace natsl

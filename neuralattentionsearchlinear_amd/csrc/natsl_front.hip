@@ -104,46 +104,48 @@ __global__ __launch_bounds__(256) void conv_norm_kernel(const ConvNormParams p) 
       for (int c = 0; c < 8; ++c) so[((size_t)b * D + d0 + c) * W + j] = f32_to_bf16(e[c]);
     }
   }
+  auto one_row = [&](const u32x4 in, const int t) __attribute__((always_inline)) {
+    float y[8], ss = 0.f, none = 0.f;
+    up8(in, win[W - 1]);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      float acc = bs[c];
+#pragma unroll
+      for (int j = 0; j < W; ++j) acc += wt[j][c] * win[j][c];
+      y[c] = p.silu ? acc / (1.f + __expf(-acc)) : acc;
+    }
+    const u32x4 packed = down8(y);
+    const size_t at = base + (size_t)t * D;
+    if (s.y) *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(s.y) + at) = packed;
+    if (s.y_norm) {
+      up8(packed, y);
+#pragma unroll
+      for (int c = 0; c < 8; ++c) ss += y[c] * y[c];
+      group_sum2(ss, none, s.norm_lanes);
+      const float rs = rsqrtf((s.norm_l2 ? ss : ss / (8 * s.norm_lanes)) + s.norm_eps);
+#pragma unroll
+      for (int c = 0; c < 8; ++c) y[c] *= rs * nw[c];
+      *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(s.y_norm) + at) = down8(y);
+    }
+#pragma unroll
+    for (int j = 0; j < W - 1; ++j)
+#pragma unroll
+      for (int c = 0; c < 8; ++c) win[j][c] = win[j + 1][c];
+  };
   constexpr int AHEAD = 8;
-  for (int tb = t0; tb < t1; tb += AHEAD) {
+  int tb = t0;
+  for (; tb + AHEAD <= t1; tb += AHEAD) {   // (no way out between a batch's loads and their use: they all go out together)
     u32x4 rows[AHEAD];
 #pragma unroll
-    for (int a = 0; a < AHEAD; ++a) rows[a] = *row8(s.x, base + (size_t)min(tb + a, t1 - 1) * D);
+    for (int a = 0; a < AHEAD; ++a) rows[a] = *row8(s.x, base + (size_t)(tb + a) * D);
 #pragma unroll
-    for (int a = 0; a < AHEAD; ++a) {
-      if (tb + a >= t1) break;
-      float y[8], ss = 0.f, none = 0.f;
-      up8(rows[a], win[W - 1]);
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        float acc = bs[c];
-#pragma unroll
-        for (int j = 0; j < W; ++j) acc += wt[j][c] * win[j][c];
-        y[c] = p.silu ? acc / (1.f + __expf(-acc)) : acc;
-      }
-      const u32x4 packed = down8(y);
-      const size_t at = base + (size_t)(tb + a) * D;
-      if (s.y) *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(s.y) + at) = packed;
-      if (s.y_norm) {
-        up8(packed, y);
-#pragma unroll
-        for (int c = 0; c < 8; ++c) ss += y[c] * y[c];
-        group_sum2(ss, none, s.norm_lanes);
-        const float rs = rsqrtf((s.norm_l2 ? ss : ss / (8 * s.norm_lanes)) + s.norm_eps);
-#pragma unroll
-        for (int c = 0; c < 8; ++c) y[c] *= rs * nw[c];
-        *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(s.y_norm) + at) = down8(y);
-      }
-#pragma unroll
-      for (int j = 0; j < W - 1; ++j)
-#pragma unroll
-        for (int c = 0; c < 8; ++c) win[j][c] = win[j + 1][c];
-    }
+    for (int a = 0; a < AHEAD; ++a) one_row(rows[a], tb + a);
   }
+  for (; tb < t1; ++tb) one_row(*row8(s.x, base + (size_t)tb * D), tb);
 }
 
 // Backward: dy = dy_a + dy_b + (norm's backward of dy_norm), then dpre = dy act'(pre), dx[s] = sum_i w[W-1-i] dpre[s+i] + dx_add[s],
-// dw[j] = sum dpre[t] x[t-(W-1)+j].  pre and y are recomputed from x; four rows of every input are requested at a time.  A thread
+// dw[j] = sum dpre[t] x[t-(W-1)+j].  pre and y are recomputed from x; two rows of every input are requested at a time.  A thread
 // reads W-1 rows past its run (for dx of the run's last tokens) without adding them to its sums.
 template <int W>
 __global__ __launch_bounds__(256) void conv_norm_bwd_kernel(const ConvNormParams p) {
@@ -177,94 +179,97 @@ __global__ __launch_bounds__(256) void conv_norm_bwd_kernel(const ConvNormParams
       for (int c = 0; c < 8; ++c) win[j][c] = st ? bf16_to_f32(st[((size_t)b * D + d0 + c) * W + (W + q)]) : 0.f;
     }
   }
-  constexpr int AHEAD = 4;
-  const int t_end = t1 + W - 1;                          // one past the last row whose dpre this run's dx needs
+  // row t: its gradient at y, its sums (rows of the next run, t >= t1, have none), and dx of row t - (W-1)
+  auto one_row = [&](const u32x4 rx, const u32x4 ra, const u32x4 rb, const u32x4 rn, const int t, const bool own) __attribute__((always_inline)) {
+    float dp[8], g[8], g2[8], y[8], da[8];
+    up8(rx, win[W - 1]);
+    up8(ra, g);
+    up8(rb, g2);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      float acc = bs[c];
+#pragma unroll
+      for (int j = 0; j < W; ++j) acc += wt[j][c] * win[j][c];
+      y[c] = acc;
+      da[c] = 1.f;
+      if (p.silu) {
+        const float sg = 1.f / (1.f + __expf(-acc));
+        y[c] = acc * sg;
+        da[c] = sg * (1.f + acc * (1.f - sg));
+      }
+      g[c] += g2[c];
+    }
+    if (s.dy_norm) {
+      float dn[8], ss = 0.f, an = 0.f;
+      up8(down8(y), y);                                 // the rounded activation, as the forward normalised it
+      up8(rn, dn);
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        ss += y[c] * y[c];
+        an += dn[c] * nw[c] * y[c];
+      }
+      group_sum2(ss, an, s.norm_lanes);
+      const float inv_n = s.norm_l2 ? 1.f : 1.f / (8 * s.norm_lanes);
+      const float rs = rsqrtf(ss * inv_n + s.norm_eps);
+      const float m = an * rs * inv_n;                  // mean (sum) of a n
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const float n = y[c] * rs;
+        g[c] += rs * (dn[c] * nw[c] - n * m);
+        if (own) dws[W + 1][c] += dn[c] * n;
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      dp[c] = t < T ? g[c] * da[c] : 0.f;
+      if (own) {
+#pragma unroll
+        for (int j = 0; j < W; ++j) dws[j][c] += dp[c] * win[j][c];
+        dws[W][c] += dp[c];
+      }
+      dwin[W - 1][c] = dp[c];
+    }
+    const int sx = t - (W - 1);
+    if (sx >= t0) {
+      float o[8];
+      const size_t at = base + (size_t)sx * D;
+      if (s.dx_add) {
+        up8(*row8(s.dx_add, at), o);
+      } else {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) o[c] = 0.f;
+      }
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+#pragma unroll
+        for (int i = 0; i < W; ++i) o[c] += wt[W - 1 - i][c] * dwin[i][c];
+      *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(s.dx) + at) = down8(o);
+    }
+#pragma unroll
+    for (int j = 0; j < W - 1; ++j)
+#pragma unroll
+      for (int c = 0; c < 8; ++c) { win[j][c] = win[j + 1][c]; dwin[j][c] = dwin[j + 1][c]; }
+  };
+  constexpr int AHEAD = 2;
   const u32x4 zero = {0u, 0u, 0u, 0u};
-  for (int tb = t0; tb < t_end; tb += AHEAD) {
+  int tb = t0;
+  for (; tb + AHEAD <= t1; tb += AHEAD) {
     u32x4 rx[AHEAD], ra[AHEAD], rb[AHEAD], rn[AHEAD];
 #pragma unroll
     for (int a = 0; a < AHEAD; ++a) {
-      const size_t at = base + (size_t)min(tb + a, T - 1) * D;
+      const size_t at = base + (size_t)(tb + a) * D;
       rx[a] = *row8(s.x, at);
       ra[a] = s.dy_a ? *row8(s.dy_a, at) : zero;
       rb[a] = s.dy_b ? *row8(s.dy_b, at) : zero;
       rn[a] = s.dy_norm ? *row8(s.dy_norm, at) : zero;
     }
 #pragma unroll
-    for (int a = 0; a < AHEAD; ++a) {
-      const int t = tb + a;
-      if (t >= t_end) break;
-      float dp[8], g[8], g2[8];
-      up8(rx[a], win[W - 1]);
-      up8(ra[a], g);
-      up8(rb[a], g2);
-      float y[8], da[8];
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        float acc = bs[c];
-#pragma unroll
-        for (int j = 0; j < W; ++j) acc += wt[j][c] * win[j][c];
-        y[c] = acc;
-        da[c] = 1.f;
-        if (p.silu) {
-          const float sg = 1.f / (1.f + __expf(-acc));
-          y[c] = acc * sg;
-          da[c] = sg * (1.f + acc * (1.f - sg));
-        }
-        g[c] += g2[c];
-      }
-      const bool own = t < t1;                            // (t >= t1: the next run's tokens, without their sums)
-      if (s.dy_norm) {
-        float dn[8], ss = 0.f, an = 0.f;
-        up8(down8(y), y);                                 // the rounded activation, as the forward normalised it
-        up8(rn[a], dn);
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          ss += y[c] * y[c];
-          an += dn[c] * nw[c] * y[c];
-        }
-        group_sum2(ss, an, s.norm_lanes);
-        const float inv_n = s.norm_l2 ? 1.f : 1.f / (8 * s.norm_lanes);
-        const float rs = rsqrtf(ss * inv_n + s.norm_eps);
-        const float m = an * rs * inv_n;                  // mean (sum) of a n
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          const float n = y[c] * rs;
-          g[c] += rs * (dn[c] * nw[c] - n * m);
-          if (own) dws[W + 1][c] += dn[c] * n;
-        }
-      }
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        dp[c] = t < T ? g[c] * da[c] : 0.f;
-        if (own) {
-#pragma unroll
-          for (int j = 0; j < W; ++j) dws[j][c] += dp[c] * win[j][c];
-          dws[W][c] += dp[c];
-        }
-        dwin[W - 1][c] = dp[c];
-      }
-      const int sx = t - (W - 1);
-      if (sx >= t0 && sx < t1) {
-        float o[8];
-        const size_t at = base + (size_t)sx * D;
-        if (s.dx_add) {
-          up8(*row8(s.dx_add, at), o);
-        } else {
-#pragma unroll
-          for (int c = 0; c < 8; ++c) o[c] = 0.f;
-        }
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-#pragma unroll
-          for (int i = 0; i < W; ++i) o[c] += wt[W - 1 - i][c] * dwin[i][c];
-        *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(s.dx) + at) = down8(o);
-      }
-#pragma unroll
-      for (int j = 0; j < W - 1; ++j)
-#pragma unroll
-        for (int c = 0; c < 8; ++c) { win[j][c] = win[j + 1][c]; dwin[j][c] = dwin[j + 1][c]; }
-    }
+    for (int a = 0; a < AHEAD; ++a) one_row(rx[a], ra[a], rb[a], rn[a], tb + a, true);
+  }
+#pragma unroll 1
+  for (; tb < t1 + W - 1; ++tb) {                         // the run's odd row, and the W-1 rows behind it that its dx needs
+    const size_t at = base + (size_t)min(tb, T - 1) * D;
+    one_row(*row8(s.x, at), s.dy_a ? *row8(s.dy_a, at) : zero, s.dy_b ? *row8(s.dy_b, at) : zero, s.dy_norm ? *row8(s.dy_norm, at) : zero, tb, tb < t1);
   }
   float* pr = p.part[si] + ((size_t)(b * runs + r) * (W + 2)) * D + d0;
 #pragma unroll
@@ -420,30 +425,41 @@ struct DxInit {
   long long rows;
   int D, N, ld, T, block, nb;     // dn [rows][ld], w [N][D] (N a multiple of 16, or 0); dpool [B][nb][D] or null
 };
+constexpr int DX_TILES = 4;
+// columns d0.. (one per lane%32) of rows k.. of the narrow weight, as the A operand of W^T
+NATSL_DEVICE bf16x8 dx_operand(const DxInit& p, const int k, const int d0) {
+  const int lane = threadIdx.x & 63;
+  bf16_t wv[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) wv[j] = p.w[(size_t)(k + 8 * (lane >> 5) + j) * p.D + min(d0 + (lane & 31), p.D - 1)];
+  u32x4 a;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) a[j] = (unsigned)wv[2 * j] | ((unsigned)wv[2 * j + 1] << 16);
+  return __builtin_bit_cast(bf16x8, a);
+}
 __global__ __launch_bounds__(256) void dx_init_kernel(const DxInit p) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const long long t = (long long)blockIdx.x * 32 + (lane & 31);
-  const long long tc = t < p.rows ? t : p.rows - 1;
   const int half = lane >> 5;
+  // a wave keeps its 64 columns for DX_TILES tiles of tokens: the first 16 rows of W^T stay in registers
+  bf16x8 w0[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) w0[u] = p.N > 0 ? dx_operand(p, 0, ((int)blockIdx.y * 4 + wave) * 64 + 32 * u) : zero8();
+#pragma unroll 1
+  for (int it = 0; it < DX_TILES; ++it) {
+  const long long t = ((long long)blockIdx.x * DX_TILES + it) * 32 + (lane & 31);
+  const long long tc = t < p.rows ? t : p.rows - 1;
   const int b = (int)(tc / p.T), tt = (int)(tc - (long long)b * p.T);
   const int blk = tt / p.block;
   const float inv = 1.f / (float)(min(p.T, (blk + 1) * p.block) - blk * p.block);
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     const int d0 = ((int)blockIdx.y * 4 + wave) * 64 + 32 * u;
-    if (d0 >= p.D) return;
+    if (d0 >= p.D) break;
     f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    for (int k = 0; k < p.N; k += 16) {
-      bf16_t wv[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) wv[j] = p.w[(size_t)(k + 8 * half + j) * p.D + min(d0 + (lane & 31), p.D - 1)];
-      u32x4 a;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) a[j] = (unsigned)wv[2 * j] | ((unsigned)wv[2 * j + 1] << 16);
-      acc = mfma32(__builtin_bit_cast(bf16x8, a), ld8(p.dn + tc * p.ld + k + 8 * half), acc);
-    }
+    if (p.N > 0) acc = mfma32(w0[u], ld8(p.dn + tc * p.ld + 8 * half), acc);
+    for (int k = 16; k < p.N; k += 16) acc = mfma32(dx_operand(p, k, d0), ld8(p.dn + tc * p.ld + k + 8 * half), acc);
     if (t >= p.rows) continue;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -461,6 +477,7 @@ __global__ __launch_bounds__(256) void dx_init_kernel(const DxInit p) {
       }
       *reinterpret_cast<u32x2*>(p.dx + (size_t)t * p.D + d) = (u32x2){pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
     }
+  }
   }
 }
 
@@ -644,7 +661,7 @@ extern "C" int natsl_dx_init(const void* dn, const void* w, const void* dpool, v
   DxInit p;
   p.dn = (const bf16_t*)dn; p.w = (const bf16_t*)w; p.dpool = (const bf16_t*)dpool; p.dx = (bf16_t*)dx; p.rows = (long long)B * T; p.D = D; p.N = N;
   p.ld = ld; p.T = T; p.block = block; p.nb = cdiv(T, block);
-  hipLaunchKernelGGL(dx_init_kernel, dim3((unsigned)((p.rows + 31) / 32), (unsigned)cdiv(D, 256)), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), p);
+  hipLaunchKernelGGL(dx_init_kernel, dim3((unsigned)((p.rows + 32 * DX_TILES - 1) / (32 * DX_TILES)), (unsigned)cdiv(D, 256)), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), p);
   return check_launch(what);
 }
 

@@ -43,22 +43,25 @@ __global__ __launch_bounds__(256) void mean_pool_kernel(const void* x, void* out
     if (d8 >= D) return;
     float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     const bf16_t* xp = reinterpret_cast<const bf16_t*>(x) + (size_t)(bos + lo) * D + d8;
-    // sixteen rows are requested before the first is added (a thread's loads one by one: 2.2 TB/s); added in order all the same
+    // sixteen rows are requested before the first is added, in order all the same (a loop that may leave in the middle of a batch
+    // makes the compiler ask for them one by one)
     constexpr int AHEAD = 16;
-    for (int t = lo; t < hi; t += AHEAD, xp += (size_t)AHEAD * D) {
+    auto add = [&](const u32x4 w) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        s[2 * j] += __uint_as_float(w[j] << 16);
+        s[2 * j + 1] += __uint_as_float(w[j] & 0xffff0000u);
+      }
+    };
+    int t = lo;
+    for (; t + AHEAD <= hi; t += AHEAD) {
       u32x4 w[AHEAD];
 #pragma unroll
-      for (int a = 0; a < AHEAD; ++a) w[a] = *reinterpret_cast<const u32x4*>(xp + (size_t)min(a, hi - 1 - t) * D);
+      for (int a = 0; a < AHEAD; ++a, xp += D) w[a] = *reinterpret_cast<const u32x4*>(xp);
 #pragma unroll
-      for (int a = 0; a < AHEAD; ++a) {
-        if (t + a >= hi) break;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          s[2 * j] += __uint_as_float(w[a][j] << 16);
-          s[2 * j + 1] += __uint_as_float(w[a][j] & 0xffff0000u);
-        }
-      }
+      for (int a = 0; a < AHEAD; ++a) add(w[a]);
     }
+    for (; t < hi; ++t, xp += D) add(*reinterpret_cast<const u32x4*>(xp));
     u32x4 o;
 #pragma unroll
     for (int j = 0; j < 4; ++j) o[j] = pack_bf16x2(s[2 * j] * inv, s[2 * j + 1] * inv);

@@ -305,7 +305,7 @@ static StepLayout step_layout(const natsl_layer_step& s) {
   l.q_attn = take((size_t)M * KD * 2);
   l.o_lin = take((size_t)M * VD * 2);
   l.y = take((size_t)M * VD * 2);
-  l.partials = take((size_t)M * s.HQ * l.nsplit * (2 + VD / s.HQ) * 4);
+  l.partials = take((size_t)M * s.HQ * ATTEND_MAX_SPLITS * (2 + VD / s.HQ) * 4);   // (the size does not follow the cache's)
   l.bytes = at;
   return l;
 }

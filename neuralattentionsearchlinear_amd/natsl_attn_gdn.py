@@ -228,6 +228,8 @@ class NeuralAttentionSearchLinearAttnGDN(nn.Module):
             types, n_nats_blocks = fast.select(logits, True)
             # (the types before the last block is forced are only needed where states are handed on)
             raw_types = fast.select(logits, False)[0] if use_cache or cache is not None else types
+            if cache is not None:
+                cache.foresee(raw_types, q_len)
             q, k, v, q_attn, k_attn, o_mix, _, _, _, new_conv_states = fast.conv_norm(q, k, v, conv_states, bool(use_cache))
             v_attn = v
             g, beta, _ = fast.gates(ab)

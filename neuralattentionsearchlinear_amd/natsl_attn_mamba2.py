@@ -195,6 +195,8 @@ class NeuralAttentionSearchLinearAttnMamba(nn.Module):
             types, n_nats_blocks = fast.select(logits, True)
             # (the types before the last block is forced are only needed where states are handed on)
             raw_types = fast.select(logits, False)[0] if use_cache or cache is not None else types
+            if cache is not None:
+                cache.foresee(raw_types, q_len)
             _, _, v, q, k, o_mix, q_attn, k_attn, v_attn, new_conv_states = fast.conv_norm(q, k, v, conv_states, bool(use_cache))
             g, _, dt = fast.gates(a)
             q, k = (x.unflatten(-1, (-1, self.head_k_dim)) for x in (q, k))

@@ -10,13 +10,15 @@ general path runs.
 from __future__ import annotations
 
 import ctypes
+import operator
 import weakref
 
 import torch
 import torch.nn as nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import _capi
-from .modules import FusedMultiInputRMSNormGated, RMSNorm, ShortConvolution
+from .modules import FusedMultiInputRMSNormGated, L2Norm, RMSNorm, ShortConvolution
 
 MAX_ROWS = 64
 
@@ -55,51 +57,90 @@ _EITHER_DTYPE = {"norm_q", "norm_k", "a_log", "dt_bias", "out_norm1", "out_norm2
 _watches = weakref.WeakKeyDictionary()
 
 
+# what the plans are made from besides the weights: a layer's options, and those of its submodules
+_OPTIONS = ("hidden_size", "head_k_dim", "head_v_dim", "head_attn_k_dim", "head_attn_v_dim", "num_heads", "num_v_heads", "num_attn_heads",
+            "num_nats_head", "nats_block_size", "ops_for_incomplete_chunks", "use_short_conv", "conv_size", "attn_with_short_conv", "attn_qk_norm",
+            "allow_neg_eigval", "decay_for_non_gdn_blocks", "decay_for_non_mamba_blocks", "value_dim")
+_SUB_OPTIONS = ("eps", "kernel_size", "activation")
+_SUBMODULES = tuple((p[1], p[3]) for p in _PARAMS if p[1] is not None and p[3] is not None) + (("q_norm2", L2Norm), ("k_norm2", L2Norm))
+_dtype_of = operator.attrgetter('dtype')
+
+
 class _Watch:
-    """A layer's weight tensors by field, and a quick way to see that they are still the ones: same submodules, unhooked, holding
-    the same tensors at the same addresses."""
+    """A layer's weight tensors by field, and a quick way to see that what the plans were made from still holds: the same
+    submodules with the same options, holding the same tensors at the same addresses in the same types and layouts."""
 
     def __init__(self, layer):
         mods = layer._modules
-        self.tensors, self.plain = [], True
-        self.mods, self.held = {}, []
-        for _, mod, name, kind in _PARAMS:
-            if mod is None:
-                where = layer._parameters
-            else:
-                m = mods.get(mod)
-                self.mods[mod] = m
-                if m is None:
-                    self.tensors.append(None)
-                    continue
-                if kind is not None and type(m) is not kind:
-                    self.plain = False
-                where = m._parameters
-            t = where.get(name)
+        self.mods = [(n, mods.get(n)) for n, _ in _SUBMODULES]
+        self.plain = all(m is None or type(m) is kind for (_, m), (_, kind) in zip(self.mods, _SUBMODULES))
+        self.tensors, self.held = [], []
+        for _, mod, name, _ in _PARAMS:
+            m = layer if mod is None else mods.get(mod)
+            t = None if m is None else m._parameters.get(name)
             self.tensors.append(t)
-            self.held.append((where, name, t, 0 if t is None else t.data_ptr()))
-        self.unhooked = [(m._forward_hooks, m._forward_pre_hooks, m.__dict__) for m in self.mods.values() if m is not None]
+            if m is not None:
+                self._hold(m._parameters, name, t)
+            if type(m) is nn.Linear:
+                self._hold(m._parameters, 'bias', m.bias)
+        self.options = [(layer.__dict__, _OPTIONS, self._read(layer.__dict__, _OPTIONS))]
+        self.hooks = []
+        for _, m in self.mods:
+            if m is not None:
+                d = m.__dict__
+                names = tuple(n for n in _SUB_OPTIONS if n in d)
+                if names:
+                    self.options.append((d, names, self._read(d, names)))
+                self.hooks.append((m._forward_hooks, m._forward_pre_hooks, m._backward_hooks, m._backward_pre_hooks, d))
+        self.weights = [t for _, _, t in self.held if t is not None]
+        self.layouts = self._layouts() if self.plain else None
         self.step_plan = self.front_plan = None
+
+    def _layouts(self):
+        w = self.weights
+        return [*map(torch.Tensor.data_ptr, w), *map(_dtype_of, w), *map(torch.Tensor.is_contiguous, w), *map(torch.Tensor.numel, w)]
+
+    @staticmethod
+    def _read(where, names):
+        return tuple(map(where.get, names))
+
+    def _hold(self, where, name, t):
+        if t is None:
+            self.held.append((where, name, None))
+        elif type(t) not in (nn.Parameter, torch.Tensor):
+            self.plain = False
+        else:
+            self.held.append((where, name, t))
 
     def holds(self, layer):
         mods = layer._modules
-        for n, m in self.mods.items():
+        for n, m in self.mods:
             if mods.get(n) is not m:
                 return False
-        for where, name, t, at in self.held:
-            if where.get(name) is not t or (t is not None and t.data_ptr() != at):
+        for where, name, t in self.held:
+            if where.get(name) is not t:
+                return False
+        if self._layouts() != self.layouts:
+            return False
+        for where, names, values in self.options:
+            if tuple(map(where.get, names)) != values:
                 return False
         return True
 
     def hooked(self):
-        for a, b, d in self.unhooked:
-            if a or b or 'forward' in d:
+        if _has_any_global_hook():
+            return True
+        for a, b, c, e, d in self.hooks:
+            if a or b or c or e or 'forward' in d:
                 return True
         return False
 
 
 def watch(layer):
-    """The layer's _Watch, made anew when a weight or submodule has been replaced; None when a submodule is not the plain one."""
+    """The layer's _Watch, made anew when a weight, a submodule or an option has changed; None when a submodule or a weight is not a
+    plain one, when something is hooked, or under forward-mode differentiation (whose tangents only the general path's products carry)."""
+    if torch.autograd.forward_ad._current_level >= 0:
+        return None
     w = _watches.get(layer)
     if w is None or not w.holds(layer):
         w = _watches[layer] = _Watch(layer)
@@ -135,7 +176,8 @@ class _Plan:
         W, act = convs[0].kernel_size[0], convs[0].activation
         if any(c.kernel_size[0] != W or (c.activation is None) != (act is None) for c in convs) or W not in (2, 3, 4):
             return
-        if any(layer._modules[m].bias is not None for m in ("q_proj", "k_proj", "v_proj", "g_proj", "a_proj", "nats_out_weights_layer", "o_proj")):
+        if any(layer._modules[m].bias is not None for m in ("q_proj", "k_proj", "v_proj", "g_proj", "a_proj", "nats_out_weights_layer", "o_proj")) \
+                or (delta and layer._modules["b_proj"].bias is not None):
             return
         D, KA, VA = layer.hidden_size, layer.head_attn_k_dim, layer.head_attn_v_dim
         if K not in (64, 128, 192) or KA not in (64, 128) or VA not in (64, 128) or K % KA or HQ % H or HQ % layer.num_nats_head or \

@@ -121,3 +121,36 @@ def test_chunk_state_saving_follows_the_byte_budget():
         assert not MC._keep_chunk_states(small, small, None)
     finally:
         MC.SAVE_CHUNK_STATES = old
+
+
+def test_layer_plans_notice_every_change():
+    """What the layers' fused paths remember about a layer is dropped when a weight, an option or a hook changes."""
+    import torch
+    from neuralattentionsearchlinear_amd._layer_step import watch
+    from neuralattentionsearchlinear_amd.natsl_attn_gdn import NeuralAttentionSearchLinearAttnGDN
+    layer = NeuralAttentionSearchLinearAttnGDN(hidden_size=64, expand_v=2, head_dim=64, num_heads=2, num_attn_heads=2, layer_idx=0)
+    seen = watch(layer)
+    assert seen is not None and watch(layer) is seen
+
+    def new_after(change):
+        nonlocal seen
+        change()
+        before, seen = seen, watch(layer)
+        return seen is not before
+
+    w = layer.q_conv1d.weight
+    assert new_after(lambda: setattr(w, 'data', w.data.clone()))                       # another address
+    assert new_after(lambda: setattr(w, 'data', w.data.view(torch.int32)))             # the same memory as another type
+    assert new_after(lambda: setattr(w, 'data', w.data.view(torch.float32)))
+    q = layer.nats_out_weights_layer.weight
+    assert new_after(lambda: setattr(q, 'data', q.data.t().contiguous().t()))          # another layout
+    assert new_after(lambda: setattr(layer, 'decay_for_non_gdn_blocks', not layer.decay_for_non_gdn_blocks))
+    assert new_after(lambda: setattr(layer.o_norm, 'eps', 1e-3))
+    assert new_after(lambda: setattr(layer.b_proj, 'bias', torch.nn.Parameter(torch.zeros(2))))
+    handle = layer.q_proj.register_full_backward_hook(lambda *a: None)
+    assert watch(layer) is None
+    handle.remove()
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda *a: None)
+    assert watch(layer) is None
+    handle.remove()
+    assert watch(layer) is seen

@@ -137,7 +137,8 @@ int natsl_softmax_fwd_variant(int B, int T, int HQ, int HKV, int block, int pack
  * with respect to a bias on that block's scores as later blocks see them; blocks not typed attention keep 0 unless
  * flags bit 1 is set (the reference's compute_dnats_for_invalid_blocks_attn, attns.py:1318-1325): then they get
  * sum min(exp2(s - lse), 1) (dP - delta) over the same (keys) x (later queries), what their keys would contribute if
- * they were visible.  flags bit 0: same_block_visible, as in the forward.  The caller sums dnats over the query heads
+ * they were visible.  flags bit 0: same_block_visible, as in the forward; bits 2, 3, 4: add to what is in dq, dk, dv
+ * (rounded to bf16 twice, as an elementwise addition of the two gradients would) instead of overwriting it.  The caller sums dnats over the query heads
  * of a selector head.  o, lse are the forward's outputs, d_o the gradient of o.  workspace: natsl_softmax_bwd_workspace_bytes()
  * bytes (delta = rowsum(d_o * o), then the work-queue counters of the dk/dv kernel; nothing to initialise: every call resets
  * them, so calls that share a workspace must not overlap).  T * HQ * max(K, V) * 2 must stay below 2^32 (32-bit row offsets
@@ -215,6 +216,17 @@ int natsl_linear_chunk_bwd(int delta_rule, const void* q, const void* k, const v
                            void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0, float* d_gate, float* d_rollback, int B, int T,
                            int H, int HN, int K, int V, int TN, int block, float scale, int flags, int dtype,
                            const natsl_seq_row* seqs, int n_seqs, int total_chunks, natsl_stream_t stream);
+
+/* What is per selector block around natsl_linear_chunk_bwd.  natsl_linear_block_sums fills its g_block_sums from the forward's
+ * workspace.  natsl_block_grads, after it: d_types [B,TN,HN,2] (f32 or bf16) = the selector's straight-through gradients --
+ * [..., 1] d_gate summed over a block's chunks and a selector head's heads where the block is typed linear (others: 0, or with
+ * `invalid` their last chunk's), [..., 0] dnats [B,TN,HQ] f32 of natsl_softmax_sparse_bwd summed over the query heads (NULL: 0) --
+ * and, where d_rollback is given, dg [B*T][H] += the rolled-back decay's share. */
+int natsl_linear_block_sums(const void* workspace, float* g_block_sums, int B, int T, int H, int TN, int block, const natsl_seq_row* seqs, int n_seqs,
+                            int total_chunks, natsl_stream_t stream);
+int natsl_block_grads(const void* types, int types_dtype, const float* d_gate, const float* d_rollback, const float* dnats, int HQ, float* dg,
+                      void* d_types, int d_types_dtype, int invalid, int B, int T, int H, int HN, int TN, int block, const natsl_seq_row* seqs,
+                      int n_seqs, natsl_stream_t stream);
 
 /* Layer tail: y = (rms(x1)*w1*xw[...,0] + rms(x2)*w2*xw[...,1]) * gate*sigmoid(gate) with
  * rms(x) = x*rsqrt(mean(x^2)+eps); x1, x2, gate, y [rows, D] and x_weights [rows, 2] in `dtype`,

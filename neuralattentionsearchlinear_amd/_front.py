@@ -172,8 +172,8 @@ def _conv_norm(f, raw, states, want_states):
 
 
 class _ConvNorm(torch.autograd.Function):
-    """(q, k, v projections) -> (conv(q), conv(k), conv(v), normed q, normed k, mixing logits, and the projections themselves); the last
-    three only carry the gradient of an attention view that takes them to where it is added (dx_add)."""
+    """(q, k, v projections) -> (conv(q), conv(k), conv(v), normed q, normed k, mixing logits, and what attention takes:
+    the projections themselves, or only conv(v) once more); the last three only carry attention's gradient to where it is added (dx_add, dy_b)."""
 
     @staticmethod
     def forward(ctx, f, q, k, v, wq, bq, wk, bk, wv, bv, nq, nk, w_mix):
@@ -182,7 +182,7 @@ class _ConvNorm(torch.autograd.Function):
         # (the parameters are saved for the check that nobody changes them before the backward reads them through f)
         ctx.save_for_backward(q, k, v, ys[0], w_mix, wq, bq, wk, bk, wv, bv, nq, nk)
         ctx.set_materialize_grads(False)
-        raw = tuple(t.view(t.shape) for t in (q, k, v)) if f.raw_attention else (None, None, None)
+        raw = tuple(t.view(t.shape) for t in (q, k, v)) if f.raw_attention else (None, None, ys[2].detach())
         return (ys[0], ys[1], ys[2], ns[0], ns[1], F.linear(ys[0], w_mix)) + raw
 
     @staticmethod
@@ -205,8 +205,11 @@ class _ConvNorm(torch.autograd.Function):
             hold.append(t)
             return t.data_ptr()
         segs = _conv_segs(f, (q, k, v))
+        dv_conv = None
+        if not f.raw_attention:
+            dv_conv, dv_raw = dv_raw, None
         grads = []
-        for s, x, n, da, db, dn, add in zip(segs, (q, k, v), "qkv", (dq, dk, dv), (dq_mix, None, None), (dqn, dkn, None), (dq_raw, dk_raw, dv_raw)):
+        for s, x, n, da, db, dn, add in zip(segs, (q, k, v), "qkv", (dq, dk, dv), (dq_mix, None, dv_conv), (dqn, dkn, None), (dq_raw, dk_raw, dv_raw)):
             w, b = f.w["conv_w" + n], f.w["conv_b" + n]
             dx, dw = torch.empty_like(x), torch.empty_like(w)
             dbias = None if b is None else torch.empty_like(b)
@@ -355,14 +358,15 @@ class FastFront:
         return _project(*args)[0]
 
     def conv_norm(self, q, k, v, states, want_states):
-        """-> (conv(q), conv(k) or None, conv(v), normed q, normed k, mixing logits, raw q, k, v, new states)."""
+        """-> (conv(q), conv(k) or None, conv(v), normed q, normed k, mixing logits, raw q, k, v
+        (or None, None, conv(v) again: attention's), new states)."""
         w = self.w
         args = (q, k, v, w["conv_wq"], w["conv_bq"], w["conv_wk"], w["conv_bk"], w["conv_wv"], w["conv_bv"],
                 w["norm_q"] if self.delta else None, w["norm_k"] if self.delta else None, w["w_mix"])
         if self.grad(*args):
             return _ConvNorm.apply(self, *args) + (None,)
         ys, ns, new = _conv_norm(self, (q, k, v), states, want_states)
-        return ys[0], ys[1], ys[2], ns[0], ns[1], F.linear(ys[0], w["w_mix"]), q, k, v, new
+        return ys[0], ys[1], ys[2], ns[0], ns[1], F.linear(ys[0], w["w_mix"]), *((q, k, v) if self.raw_attention else (None, None, ys[2])), new
 
     def gates(self, ab):
         if self.grad(ab, self.w["a_log"], self.w["dt_bias"]):

@@ -120,12 +120,15 @@ def hip_backward_is_built(K: int, V: int) -> bool:
 
 
 def linear_chunk_backward(kind, q, k, v, g, beta, h0, types, scale, block, decay, l2norm, intra, do, dht,
-                          dnats_for_invalid_blocks, seqs=None, saved=None):
+                          dnats_for_invalid_blocks, seqs=None, saved=None, later=None):
     """Gradients of the chunked linear branch: -> (dq, dk, dv, dg fp32, dbeta or None, dh0 or None, dnats fp32 [B,NB,HN]).
     types [B,NB,HN,2]; do [B,T,H,V]; dht [N,H,K,V] or None; seqs: packed sequences (B = 1) or None; saved: what
     linear_chunk_fwd(..., chunk_states=True) returned after (o, final_state) on these same inputs, if the caller kept it.  The
     HIP kernels (natsl_linear_chunk_bwd) for K in 64/128/192 -- V a multiple of 64 as it is, other multiples of 16 behind zero
     columns --, else the torch formulation below, one sequence at a time.
+
+    later (a list): where the kernels run on the tensors as they are, dg and dnats are left unfinished, dnats comes back as None and the list
+    receives a function that ends them, given the softmax branch's dnats [B,NB,HQ] fp32 -> the gradient of types [B,NB,HN,2].
 
     dnats_for_invalid_blocks with block > 64 raises NotImplementedError: for a block of several chunks that is not typed
     linear the reference sums a virtual key gradient v . dh over EVERY chunk of the block
@@ -139,7 +142,7 @@ def linear_chunk_backward(kind, q, k, v, g, beta, h0, types, scale, block, decay
     K, V = q.shape[-1], v.shape[-1]
     if hip_backward_is_built(K, V):
         return linear_chunk_backward_hip(kind, q, k, v, g, beta, h0, types, scale, block, decay, l2norm, intra, do, dht,
-                                         dnats_for_invalid_blocks, seqs, saved)
+                                         dnats_for_invalid_blocks, seqs, saved, later)
     if hip_backward_is_built(K, 64) and V % 16 == 0:
         # Value widths the kernels are not built for (16..48, 96, ..): zero columns up to the next multiple of 64.  The state's
         # columns never mix, a zero column of v and dO stays zero through the whole recurrence and adds nothing to any sum
@@ -165,49 +168,11 @@ def linear_chunk_backward(kind, q, k, v, g, beta, h0, types, scale, block, decay
     return cat(0, 1), cat(1, 1), cat(2, 1), cat(3, 1), cat(4, 1), cat(5, 0), cat(6, 1)
 
 
-_MAPS = {}
-
-
-def _block_maps(B, T, block, seqs, dev):
-    """Index tensors that tie tokens and chunks to selector blocks, flat over the sequences: for every block the first / one
-    past the last token and chunk, the index of its last chunk, and for every token its block."""
-    key = (B, T, block, None if seqs is None else tuple(seqs.cu_seqlens), str(dev))
-    m = _MAPS.get(key)
-    if m is not None:
-        return m
-    per = block // C
-    bounds = [(i * T, (i + 1) * T) for i in range(B)] if seqs is None else list(zip(seqs.cu_seqlens[:-1], seqs.cu_seqlens[1:]))
-    t0s, t1s, c0s, c1s, toks = [], [], [], [], []
-    coff, boff = 0, 0
-    for a, b in bounds:
-        n = b - a
-        nb, nc = -(-n // block), -(-n // C)
-        j = torch.arange(nb)
-        t0s.append(a + j * block)
-        t1s.append(torch.clamp(a + (j + 1) * block, max=b))
-        c0s.append(coff + j * per)
-        c1s.append(torch.clamp(coff + (j + 1) * per, max=coff + nc))
-        toks.append(boff + torch.arange(n) // block)
-        coff += nc
-        boff += nb
-    m = tuple(torch.cat(x).to(dev) for x in (t0s, t1s, c0s, c1s, toks))
-    if len(_MAPS) > 16:
-        _MAPS.clear()
-    _MAPS[key] = m
-    return m
-
-
-def _range_sums(x, first, end):
-    """Sums of x[first[j]:end[j]] along dim 0 for every j (fp64 running sums: the same result every time)."""
-    xt = x.double().t().contiguous()                      # [H, n]: the running sum along the contiguous dimension
-    cs = torch.cat([xt.new_zeros(xt.shape[0], 1), xt.cumsum(1)], 1)
-    return (cs[:, end] - cs[:, first]).t().float().contiguous()
-
-
 def linear_chunk_backward_hip(kind, q, k, v, g, beta, h0, types, scale, block, decay, l2norm, intra, do, dht,
-                              dnats_for_invalid_blocks, seqs=None, saved=None):
+                              dnats_for_invalid_blocks, seqs=None, saved=None, later=None):
     """The backward as kernels: the forward once more (storing every chunk's entering state and v_new) unless the caller kept
-    those from its own forward (`saved`), then the reverse scan and the per-chunk gradients (csrc/natsl_linear_bwd.hip)."""
+    those from its own forward (`saved`), then the reverse scan and the per-chunk gradients (csrc/natsl_linear_bwd.hip).  later: a list that receives
+    the call that ends the work (see linear_chunk_backward)."""
     from . import _capi
     from ._mixed_common import linear_chunk_fwd
     from .nats_util import _seq_args
@@ -232,14 +197,10 @@ def linear_chunk_backward_hip(kind, q, k, v, g, beta, h0, types, scale, block, d
         else:
             _, _, states, v_new, ws = linear_chunk_fwd(kind, qb, kb, vb, gf, bb, h0f, ty, scale, block, flags, False, seqs,
                                                        chunk_states=True)
-        tok0, tok1, ch0, ch1, tok_blk = _block_maps(B, T, block, seqs, dev)
-        # sum of g over every selector block [all blocks, H], from the chunk sums the forward left in its workspace (behind
-        # the TmB and P areas: four vectors of 64 floats per chunk and head, the fourth {e^G, G, is_linear, ..}; they are
-        # what the forward's own roll-back decay was made of)
-        units = NTtot * H
-        g_chunk = ws[units * (2 * C * C * 2):].view(f32).view(units, 4 * C)[:, 3 * C + 1].reshape(NTtot, H)
-        one_chunk_blocks = block == C
-        gsum = g_chunk.contiguous() if one_chunk_blocks else _range_sums(g_chunk, ch0, ch1).contiguous()
+        sp, ns, tot = _seq_args(seqs, NTtot)
+        P, L, stream = _capi.ptr, _capi.lib(), _capi.stream_ptr(dev)
+        gsum = torch.empty(B * NB, H, dtype=f32, device=dev)
+        _capi.check(L.natsl_linear_block_sums(P(ws), P(gsum), B, T, H, NB, block, sp, ns, tot, stream), "natsl_linear_block_sums")
         d_states = torch.empty_like(states)
         dq, dk, dv = torch.empty_like(qb), torch.empty_like(kb), torch.empty_like(vb)
         dg = torch.empty(B, T, H, dtype=f32, device=dev)
@@ -250,22 +211,24 @@ def linear_chunk_backward_hip(kind, q, k, v, g, beta, h0, types, scale, block, d
         rb = torch.empty(NTtot, H, dtype=f32, device=dev)
         dof = do.detach().to(bf16).contiguous()
         dhtf = None if dht is None else dht.detach().to(f32).contiguous()
-        P = _capi.ptr
-        sp, ns, tot = _seq_args(seqs, NTtot)
-        rc = _capi.lib().natsl_linear_chunk_bwd(
+        rc = L.natsl_linear_chunk_bwd(
             1 if delta else 0, P(qb), P(kb), P(v_new), P(gf), P(bb), P(dof), P(dhtf), P(states), P(ty), _capi.dtype_code(ty.dtype),
             P(gsum), P(ws), P(d_states), P(dbeta_parts), P(dq), P(dk), P(dv), P(dg), P(dbeta), P(dh0), P(gate), P(rb),
-            B, T, H, HN, K, V, NB, block, float(scale), flags, _capi.dtype_code(bf16), sp, ns, tot, _capi.stream_ptr(dev))
+            B, T, H, HN, K, V, NB, block, float(scale), flags, _capi.dtype_code(bf16), sp, ns, tot, stream)
         _capi.check(rc, "natsl_linear_chunk_bwd")
-        if decay:
-            # the decay of a rolled-back block acts on every token of the block (rb is non-zero at such a block's last chunk)
-            dg.view(B * T, H).add_(rb[ch1 - 1][tok_blk])
-        lin = (torch.round(ty[..., 1].float()) == 1).repeat_interleave(H // HN, dim=2).view(-1, H)          # [all blocks, H]
-        dn = torch.where(lin, gate if one_chunk_blocks else _range_sums(gate, ch0, ch1), torch.zeros_like(gsum))
-        if dnats_for_invalid_blocks:
-            # the (zero-valued) gate on the update a block that is not typed linear would have made (one chunk per block here)
-            dn = dn + torch.where(lin, torch.zeros_like(gsum), gate[ch1 - 1])
-        dn = dn.view(B, NB, HN, H // HN).sum(3)
+
+    def finish(dnats_attn=None):
+        d_types = torch.empty(B, NB, HN, 2, dtype=f32 if dnats_attn is None else ty.dtype, device=dev)
+        rc = L.natsl_block_grads(P(ty), _capi.dtype_code(ty.dtype), P(gate), P(rb) if decay else None, P(dnats_attn),
+                                 0 if dnats_attn is None else dnats_attn.shape[-1], P(dg), P(d_types), _capi.dtype_code(d_types.dtype),
+                                 int(bool(dnats_for_invalid_blocks)), B, T, H, HN, NB, block, sp, ns, _capi.stream_ptr(dev))
+        _capi.check(rc, "natsl_block_grads")
+        return d_types
+    dn = None
+    if later is None:
+        dn = finish()[..., 1]
+    else:
+        later.append(finish)
     return (dq.to(q.dtype), dk.to(k.dtype), dv.to(v.dtype), dg, None if dbeta is None else dbeta.to(beta.dtype), dh0, dn)
 
 

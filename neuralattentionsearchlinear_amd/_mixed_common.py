@@ -384,6 +384,9 @@ class _MixedFunction(torch.autograd.Function):
         ctx.in_dtypes = tuple(None if t is None else t.dtype for t in (q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
                                                                        initial_state, g, beta, nats_block_types))
         ctx.has_h0 = initial_state is not None
+        # a tensor given to both branches gets one gradient, added up by the softmax branch's kernels (bf16: the same sum, rounded the
+        # same way, as autograd's)
+        ctx.shared = tuple(a is l and a.dtype == torch.bfloat16 for a, l in ((q_attn, q_lattn), (k_attn, k_lattn), (v_attn, v_lattn)))
         saved = [aux[n] for n in ('q_attn', 'k_attn', 'v_attn', 'q_lattn', 'k_lattn', 'v_lattn', 'g', 'types', 'lse',
                                   'nats_block_indices', 'n_nats_blocks')]
         saved += [aux['o_attn'], aux['beta'] if aux['beta'] is not None else g.new_zeros(0),
@@ -409,22 +412,26 @@ class _MixedFunction(torch.autograd.Function):
         h0 = h0 if ctx.has_h0 else None
         B, NB, HN, _ = types.shape
         seqs = pack_sequences(cfg['cu_seqlens'], cfg['cu_seqlens_nats'], cfg['block'], types.device)
-        if do_attn is not None:
-            dq_a, dk_a, dv_a, _, dn_attn = parallel_attn_nats_bwd(
-                q_a, k_a, v_a, o_attn, types, idx, nblk, None, lse, do_attn.to(torch.bfloat16).contiguous(), scale=cfg['scale_attn'],
-                NAtS_block_size=cfg['block'], compute_incomplete_chunk_scores=cfg['attn_same_block'],
-                compute_dnats_for_invalid_blocks_attn=cfg['dnats_invalid_attn'], seqs=seqs)
-        else:
-            dq_a, dk_a, dv_a = torch.zeros_like(q_a), torch.zeros_like(k_a), torch.zeros_like(v_a)
-            dn_attn = torch.zeros(B, NB, HN, dtype=torch.float32, device=types.device)
         if do_lin is None:
             do_lin = torch.zeros(*q_l.shape[:3], v_l.shape[-1], dtype=torch.float32, device=q_l.device)
         lin_args = (cfg['scale_lattn'], cfg['block'], cfg['decay_non_linear'], cfg['qk_l2norm'], cfg['lin_intra'])
+        later = []
         dq_l, dk_l, dv_l, dg, dbeta, dh0, dn_lin = linear_chunk_backward(
             cfg['kind'], q_l, k_l, v_l, g, beta, h0, types, *lin_args, do_lin, dht, cfg['dnats_invalid_linear'], seqs,
-            saved=linear_saved)
-        d_types = torch.stack([dn_attn.float(), dn_lin.float()], -1)
-        grads = [dq_a, dk_a, dv_a, dq_l, dk_l, dv_l, dh0, dg, dbeta, d_types]
+            saved=linear_saved, later=later)
+        lin = [dq_l, dk_l, dv_l]
+        if do_attn is not None:
+            onto = tuple(t if both and t.dtype == torch.bfloat16 and t.is_contiguous() else None for t, both in zip(lin, ctx.shared))
+            dq_a, dk_a, dv_a, _, dn_attn = parallel_attn_nats_bwd(
+                q_a, k_a, v_a, o_attn, types, idx, nblk, None, lse, do_attn.to(torch.bfloat16).contiguous(), scale=cfg['scale_attn'],
+                NAtS_block_size=cfg['block'], compute_incomplete_chunk_scores=cfg['attn_same_block'],
+                compute_dnats_for_invalid_blocks_attn=cfg['dnats_invalid_attn'], seqs=seqs, onto=onto, sum_heads=not later)
+            lin = [None if have is not None else t for t, have in zip(lin, onto)]
+        else:
+            dq_a, dk_a, dv_a = torch.zeros_like(q_a), torch.zeros_like(k_a), torch.zeros_like(v_a)
+            dn_attn = torch.zeros(B, NB, q_a.shape[2] if later else HN, dtype=torch.float32, device=types.device)
+        d_types = later[0](dn_attn) if later else torch.stack([dn_attn.float(), dn_lin.float()], -1)
+        grads = [dq_a, dk_a, dv_a, *lin, dh0, dg, dbeta, d_types]
         grads = [None if (t is None or dt is None) else t.to(dt) for t, dt in zip(grads, ctx.in_dtypes)]
         return (None, *grads)
 

@@ -53,7 +53,7 @@ def parallel_attn_nats_bwd(
         NAtS_block_size: int = 64, OFFSET_ATTN: int = 0, compute_incomplete_chunk_scores: bool = False,
         compute_dnats_for_invalid_blocks_attn: bool = False, sliding_window_size: Optional[int] = None,
         cu_seqlens=None, cu_seqlens_nats=None, is_causal: bool = True, chunk_indices_attn_nats=None,
-        seqs: Optional[PackedSeqs] = None):
+        seqs: Optional[PackedSeqs] = None, onto=(None, None, None), sum_heads: bool = True):
     """Backward of the softmax branch (host-side mirror of parallel_attn_nats_bwd, src/nats/ops/attns/attns.py:1562-1759)
     -> (dq [B,T,HQ,K], dk [B,T,H,K], dv [B,T,H,V], None, dnats [B,TNAtS,HNAtS]).
 
@@ -61,7 +61,8 @@ def parallel_attn_nats_bwd(
     straight-through gradient of the selector, attns.py:946-961); the other blocks get 0, or, with
     compute_dnats_for_invalid_blocks_attn, what their keys would contribute if they were visible (probabilities against
     the queries' lse, clamped to 1: attns.py:1318-1325).  Packed sequences: cu_seqlens (and cu_seqlens_nats), or the table
-    `seqs` built from them; n_nats_blocks is then [n_seqs,HN,2].  g_cumsum and sliding windows are not built."""
+    `seqs` built from them; n_nats_blocks is then [n_seqs,HN,2].  onto: gradients (contiguous bf16) that dq, dk, dv are added to in
+    place.  sum_heads=False: dnats per query head [B,TNAtS,HQ].  g_cumsum and sliding windows are not built."""
     if g_cumsum is not None or sliding_window_size is not None or not is_causal or OFFSET_ATTN != 0:
         raise NotImplementedError("only the causal backward without g_cumsum / sliding window is built")
     if seqs is None and cu_seqlens is not None:
@@ -77,7 +78,11 @@ def parallel_attn_nats_bwd(
     B, T, HQ, K = q.shape
     H, V = k.shape[2], v.shape[-1]
     TN, HN = ty.shape[1], ty.shape[2]
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    dq, dk, dv = (torch.empty_like(t) if have is None else have for t, have in zip((q, k, v), onto))
+    for t, have in zip((q, k, v), onto):
+        if have is not None and (have.shape != t.shape or have.dtype != t.dtype or not have.is_contiguous()):
+            raise ValueError("a gradient to add to must be like its tensor")
+    add = sum(4 << i for i, have in enumerate(onto) if have is not None)
     dnats = torch.zeros(B, TN, HQ, dtype=torch.float32, device=q.device)
     L = _capi.lib()
     sp, ns, tot = _seq_args(seqs, seqs.total_qtiles if seqs is not None else 0)
@@ -87,10 +92,11 @@ def parallel_attn_nats_bwd(
         _capi.ptr(q), _capi.ptr(k), _capi.ptr(v), _capi.ptr(o), _capi.ptr(lse.contiguous()), _capi.ptr(do), _capi.ptr(dq),
         _capi.ptr(dk), _capi.ptr(dv), _capi.ptr(dnats), _capi.ptr(ty), _capi.dtype_code(ty.dtype), _capi.ptr(nats_block_indices),
         _capi.ptr(n_nats_blocks), B, T, HQ, H, HN, K, V, TN, NAtS_block_size, float(scale),
-        int(bool(compute_incomplete_chunk_scores)) | (2 if compute_dnats_for_invalid_blocks_attn else 0), _capi.dtype_code(q.dtype),
+        int(bool(compute_incomplete_chunk_scores)) | (2 if compute_dnats_for_invalid_blocks_attn else 0) | add, _capi.dtype_code(q.dtype),
         _capi.ptr(ws), ws_bytes, sp, ns, tot, seqs.total_chunks if seqs is not None else 0, _capi.stream_ptr(q.device))
     _capi.check(rc, "natsl_softmax_sparse_bwd")
-    dnats = dnats.view(B, TN, HN, HQ // HN).sum(-1)          # over the query heads of a selector head (attns.py:1755)
+    if sum_heads:
+        dnats = dnats.view(B, TN, HN, HQ // HN).sum(-1)      # over the query heads of a selector head (attns.py:1755)
     return dq, dk, dv, None, dnats
 
 

@@ -1099,6 +1099,101 @@ __global__ __launch_bounds__(256, DK <= 128 ? 2 : 1) void linear_bwd_chunk_kerne
   }
 }
 
+// ---- what is per selector block: a few hundred KB next to the kernels above, so what counts is the number of launches -------------
+struct BlockParams {
+  const float* ws_sc;     // the forward's scale vectors (the fourth: {e^G, G, ..} of the chunk)
+  float* gsum;            // [blocks][H]
+  const void* types;
+  int types_dtype;
+  const float* gate;      // [chunk][H]
+  const float* rb;        // [chunk][H] or null (no decay)
+  const float* dnats;     // [blocks][HQ] or null: the softmax branch's share
+  float* dg;              // [tokens][H]
+  void* d_types;          // [blocks][HN][2]
+  int d_types_dtype;
+  const SeqRow* seqs;
+  int n_seqs, blocks, T, TN, nt, H, HN, HQ, per, invalid, pair_wgs;
+  long long tokens;
+};
+
+// chunks [first, end) of flat block j
+NATSL_DEVICE void block_chunks(const BlockParams& p, const int j, int& first, int& end) {
+  int j0 = j / p.TN * p.TN, c0 = j / p.TN * p.nt, nc = p.nt;
+  if (p.seqs) {
+    int n = 0;
+    for (int i = 1; i < p.n_seqs; ++i)
+      if (p.seqs[i].bos_nats <= j) n = i;
+    j0 = p.seqs[n].bos_nats;
+    c0 = p.seqs[n].chunk_off;
+    nc = (p.seqs[n].eos - p.seqs[n].bos + CB - 1) / CB;
+  }
+  first = c0 + (j - j0) * p.per;
+  end = min(first + p.per, c0 + nc);
+}
+
+// sum of g over every selector block, in fp64 (what the forward's roll-back decay was made of)
+__global__ __launch_bounds__(256) void block_sums_kernel(const BlockParams p) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (long long)p.blocks * p.H) return;
+  const int j = (int)(i / p.H), h = (int)(i % p.H);
+  int first, end;
+  block_chunks(p, j, first, end);
+  double sum = 0.;
+  for (int c = first; c < end; ++c) sum += (double)p.ws_sc[((size_t)c * p.H + h) * (4 * CB) + 3 * CB + 1];
+  p.gsum[i] = (float)sum;
+}
+
+// The first pair_wgs workgroups: a wave per (block, selector head) sums what the selector's gradient is made of.  The others: the
+// decay of a rolled-back block acts on every token of the block (rb is non-zero at such a block's last chunk).
+__global__ __launch_bounds__(256) void block_grads_kernel(const BlockParams p) {
+  if ((int)blockIdx.x >= p.pair_wgs) {
+    const long long i = ((long long)blockIdx.x - p.pair_wgs) * 256 + threadIdx.x;
+    if (i >= p.tokens * p.H) return;
+    const int t = (int)(i / p.H), h = (int)(i % p.H);
+    int bos = t / p.T * p.T, c0 = t / p.T * p.nt, nc = p.nt;
+    if (p.seqs) {
+      int n = 0;
+      for (int s = 1; s < p.n_seqs; ++s)
+        if (p.seqs[s].bos <= t) n = s;
+      bos = p.seqs[n].bos;
+      if (t >= p.seqs[n].eos) return;
+      c0 = p.seqs[n].chunk_off;
+      nc = (p.seqs[n].eos - bos + CB - 1) / CB;
+    }
+    const int last = min(((t - bos) / (p.per * CB) + 1) * p.per, nc) - 1;
+    p.dg[i] += p.rb[(size_t)(c0 + last) * p.H + h];
+    return;
+  }
+  const int pair = (int)blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (pair >= p.blocks * p.HN) return;
+  const int j = pair / p.HN, hn = pair % p.HN, R = p.H / p.HN;
+  int first, end;
+  block_chunks(p, j, first, end);
+  const bool lin = lin_type_b(p.types, p.types_dtype, (size_t)pair * 2 + 1);
+  // a block that is not typed linear: the zero-valued gate on the update it would have made (its last chunk's), where asked for
+  if (!lin) first = p.invalid ? end - 1 : end;
+  double sum = 0., soft = 0.;
+  for (int i = lane; i < (end - first) * R; i += 64) sum += (double)p.gate[(size_t)(first + i / R) * p.H + hn * R + i % R];
+  if (p.dnats)
+    for (int i = lane; i < p.HQ / p.HN; i += 64) soft += (double)p.dnats[(size_t)j * p.HQ + hn * (p.HQ / p.HN) + i];
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    sum += __shfl_xor(sum, d);
+    soft += __shfl_xor(soft, d);
+  }
+  if (lane == 0) {
+    if (p.d_types_dtype == NATSL_F32) {
+      float* o = reinterpret_cast<float*>(p.d_types) + (size_t)pair * 2;
+      o[0] = (float)soft;
+      o[1] = (float)sum;
+    } else {
+      bf16_t* o = reinterpret_cast<bf16_t*>(p.d_types) + (size_t)pair * 2;
+      o[0] = f32_to_bf16((float)soft);
+      o[1] = f32_to_bf16((float)sum);
+    }
+  }
+}
+
 static int bwd_cu_count() {
   static int cached[64];
   int dev = 0;
@@ -1191,4 +1286,50 @@ extern "C" int natsl_linear_chunk_bwd(int delta_rule, const void* q, const void*
     if (K == 192) return launch_bwd<192, false>(p, s, what);
   }
   return fail(NATSL_ERR_UNSUPPORTED, "%s: key dim K=%d not built (supported: 64, 128, 192)", what, K);
+}
+
+static int block_params(BlockParams& p, int B, int T, int H, int HN, int TN, int block, const natsl_seq_row* seqs, int n_seqs, const char* what) {
+  if (B <= 0 || T <= 0 || H <= 0 || HN <= 0 || TN <= 0) return fail(NATSL_ERR_INVALID, "%s: non-positive dimension", what);
+  if (H % HN) return fail(NATSL_ERR_INVALID, "%s: H=%d must be a multiple of HN=%d", what, H, HN);
+  if (block < 64 || block % 64) return fail(NATSL_ERR_UNSUPPORTED, "%s: block size %d must be a multiple of 64", what, block);
+  if (seqs ? (B != 1 || n_seqs <= 0) : (TN != cdiv(T, block)))
+    return fail(NATSL_ERR_INVALID, "%s: TN=%d does not match T=%d, block=%d (or bad packed-input arguments)", what, TN, T, block);
+  if ((long long)B * T > 0x7fffffffll || (long long)B * TN * HN > 0x7fffffffll) return fail(NATSL_ERR_UNSUPPORTED, "%s: problem too large", what);
+  p = BlockParams{};
+  p.seqs = reinterpret_cast<const SeqRow*>(seqs); p.n_seqs = seqs ? n_seqs : 0;
+  p.blocks = B * TN; p.T = T; p.TN = TN; p.nt = cdiv(T, CB); p.H = H; p.HN = HN; p.per = block / CB; p.tokens = (long long)B * T;
+  return NATSL_OK;
+}
+
+extern "C" int natsl_linear_block_sums(const void* workspace, float* g_block_sums, int B, int T, int H, int TN, int block, const natsl_seq_row* seqs,
+                                       int n_seqs, int total_chunks, natsl_stream_t stream) {
+  const char* what = "natsl_linear_block_sums";
+  if (!workspace || !g_block_sums) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
+  BlockParams p;
+  if (const int rc = block_params(p, B, T, H, 1, TN, block, seqs, n_seqs, what)) return rc;
+  const size_t units = (size_t)(seqs ? total_chunks : B * p.nt) * (size_t)H;
+  p.ws_sc = reinterpret_cast<const float*>(reinterpret_cast<const bf16_t*>(workspace) + 2 * units * (CB * CB));
+  p.gsum = g_block_sums;
+  const long long n = (long long)p.blocks * H;
+  hipLaunchKernelGGL(block_sums_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), p);
+  return check_launch(what);
+}
+
+extern "C" int natsl_block_grads(const void* types, int types_dtype, const float* d_gate, const float* d_rollback, const float* dnats, int HQ, float* dg,
+                                 void* d_types, int d_types_dtype, int invalid, int B, int T, int H, int HN, int TN, int block,
+                                 const natsl_seq_row* seqs, int n_seqs, natsl_stream_t stream) {
+  const char* what = "natsl_block_grads";
+  if (!types || !d_gate || !d_types || (d_rollback && !dg)) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
+  if ((types_dtype != NATSL_BF16 && types_dtype != NATSL_F32) || (d_types_dtype != NATSL_BF16 && d_types_dtype != NATSL_F32))
+    return fail(NATSL_ERR_UNSUPPORTED, "%s: block types must be f32 or bf16", what);
+  BlockParams p;
+  if (const int rc = block_params(p, B, T, H, HN, TN, block, seqs, n_seqs, what)) return rc;
+  if (dnats && (HQ <= 0 || HQ % HN)) return fail(NATSL_ERR_INVALID, "%s: HQ=%d must be a multiple of HN=%d", what, HQ, HN);
+  p.types = types; p.types_dtype = types_dtype; p.gate = d_gate; p.rb = d_rollback; p.dnats = dnats; p.HQ = HQ; p.dg = dg;
+  p.d_types = d_types; p.d_types_dtype = d_types_dtype; p.invalid = invalid;
+  p.pair_wgs = (int)(((long long)p.blocks * HN + 3) / 4);
+  const long long grid = p.pair_wgs + (d_rollback ? (p.tokens * H + 255) / 256 : 0);
+  if (grid > 0x7fffffffll) return fail(NATSL_ERR_UNSUPPORTED, "%s: problem too large", what);
+  hipLaunchKernelGGL(block_grads_kernel, dim3((unsigned)grid), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), p);
+  return check_launch(what);
 }

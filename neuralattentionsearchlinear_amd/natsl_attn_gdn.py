@@ -230,8 +230,7 @@ class NeuralAttentionSearchLinearAttnGDN(nn.Module):
             raw_types = fast.select(logits, False)[0] if use_cache or cache is not None else types
             if cache is not None:
                 cache.foresee(raw_types, q_len)
-            q, k, v, q_attn, k_attn, o_mix, _, _, _, new_conv_states = fast.conv_norm(q, k, v, conv_states, bool(use_cache))
-            v_attn = v
+            q, k, v, q_attn, k_attn, o_mix, _, _, v_attn, new_conv_states = fast.conv_norm(q, k, v, conv_states, bool(use_cache))
             g, beta, _ = fast.gates(ab)
             q, k = (x.unflatten(-1, (-1, self.head_k_dim)) for x in (q, k))
             v = v.unflatten(-1, (-1, self.head_v_dim))

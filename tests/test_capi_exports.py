@@ -140,7 +140,7 @@ def test_layer_plans_notice_every_change():
 
     w = layer.q_conv1d.weight
     assert new_after(lambda: setattr(w, 'data', w.data.clone()))                       # another address
-    assert new_after(lambda: setattr(w, 'data', w.data.view(torch.int32)))             # the same memory as another type
+    assert new_after(lambda: setattr(w, 'data', w.data.view(torch.complex64)))         # the same memory as another type
     assert new_after(lambda: setattr(w, 'data', w.data.view(torch.float32)))
     q = layer.nats_out_weights_layer.weight
     assert new_after(lambda: setattr(q, 'data', q.data.t().contiguous().t()))          # another layout

@@ -253,3 +253,35 @@ def test_kept_chunk_states_give_the_recomputed_gradients(kind, packed):
     kept, again = grads(True), grads(False)
     for i, (a, b) in enumerate(zip(kept, again)):
         assert torch.equal(a, b), f"tensor {i} differs between the kept and the recomputed chunk states"
+
+
+@pytest.mark.parametrize("kind,T,V,block,packed", [('gdn', 130, 128, 64, False), ('gdn', 500, 64, 128, True), ('mamba', 64, 128, 64, False),
+                                                   ('mamba', 321, 64, 256, False), ('gdn', 200, 48, 64, False)])
+def test_one_gradient_of_a_tensor_given_to_both_branches(kind, T, V, block, packed):
+    """A tensor that both branches take gets, bit for bit, the sum of the gradients that two tensors would get."""
+    from neuralattentionsearchlinear_amd._mixed_common import mixed_forward
+    B, H, K = 1 if packed else 2, 4, 128
+    V_attn = 64 if V == 48 else V
+    gen = torch.Generator().manual_seed(T)
+    bounds = [0, 1, 193, T] if packed else [0, T]
+    cu = torch.tensor(bounds, dtype=torch.int32, device=DEV) if packed else None
+    q, k, v = make_qkv(B, T, H, K, V, 5)
+    g, beta = make_gates(B, T, H, 6)
+    NB = sum(-(-(b - a) // block) for a, b in zip(bounds[:-1], bounds[1:]))
+    ty = make_types(B, NB, 2, 0.4, 7, torch.bfloat16).to(DEV)
+    do_l, do_a = torch.randn(B, T, H, V, generator=gen).bfloat16().to(DEV), torch.randn(B, T, H, V_attn, generator=gen).bfloat16().to(DEV)
+    v_other = torch.randn(B, T, H, V_attn, generator=gen).bfloat16()
+
+    def grads(shared):
+        one = [t.to(DEV).requires_grad_(True) for t in (q, k, v)]
+        two = one if shared else [t.to(DEV).requires_grad_(True) for t in (q, k, v)]
+        va = one[2] if V == V_attn else v_other.to(DEV).requires_grad_(True)
+        gd, bd = g.to(DEV).requires_grad_(True), beta.to(DEV).requires_grad_(True) if kind == 'gdn' else None
+        o_l, o_a, _ = mixed_forward(kind, one[0], one[1], va, *two, None, gd, bd, ty, 0.1, 0.1, cu, None, block, None, True, True, True, True, True,
+                                    False, kind == 'gdn')
+        torch.autograd.backward([o_l, o_a], [do_l, do_a])
+        if shared or V != V_attn:
+            return [one[0].grad, one[1].grad, two[2].grad] if shared else [one[0].grad + two[0].grad, one[1].grad + two[1].grad, two[2].grad]
+        return [a.grad + b.grad for a, b in zip(one, two)]
+    for a, b in zip(grads(True), grads(False)):
+        assert torch.equal(a, b)

@@ -836,12 +836,6 @@ __global__ NATSL_SCAN_ATTR(DK, NW + NF) void linear_scan_kernel(const LinearPara
     bf16x8 SB[KS];
 #pragma unroll
     for (int s = 0; s < KS; ++s) SB[s] = pack8(S[2 * s], S[2 * s + 1]);
-    if (p.s_out) {
-      // a B operand is eight consecutive K rows of this lane's column: 16 contiguous bytes of S^T [V][K]
-      bf16_t* so = p.s_out + (((size_t)(chunk_off + c) * p.H + h) * p.V + col) * DK + 8 * g4;
-#pragma unroll
-      for (int s = 0; s < KS; ++s) *reinterpret_cast<bf16x8*>(so + 32 * s) = SB[s];
-    }
     const float dec_c = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, dec_v)));
     const float glast_c = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, glast_v)));
     const float linf_c = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, linf_v)));
@@ -923,15 +917,6 @@ __global__ NATSL_SCAN_ATTR(DK, NW + NF) void linear_scan_kernel(const LinearPara
     }
     // (3) state update / roll-back (the next step waits for it: before the output)
     const bf16x8 VB[2] = {pack8(VN[0], VN[1]), pack8(VN[2], VN[3])};
-    if (DELTA && p.vn_out) {
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int tok = 16 * t + 4 * g4 + r;
-          if (tok < nvalid) p.vn_out[((size_t)(bos + c * C + tok) * p.H + h) * p.V + col] = f32_to_bf16(VN[t][r]);
-        }
-    }
     if (keep) {
       f32x4 W[4];
 #pragma unroll
@@ -992,6 +977,30 @@ __global__ NATSL_SCAN_ATTR(DK, NW + NF) void linear_scan_kernel(const LinearPara
         w[0] = pack_bf16x2(O[t][0], O[t][1]);
         w[1] = pack_bf16x2(O[t][2], O[t][3]);
         *reinterpret_cast<__attribute__((address_space(3))) u32x2*>(ob + a_o + 32 * t) = w;
+      }
+    }
+    // (5) what a backward keeps, at the end of the step: right after the barrier the CU's memory pipe is busy with the requests for
+    // the next chunks, and a store would wait behind them
+    if (p.s_out) {
+      // a B operand is eight consecutive K rows of this lane's column: 16 contiguous bytes of S^T [V][K]
+      bf16_t* so = p.s_out + (((size_t)(chunk_off + c) * p.H + h) * p.V + col) * DK + 8 * g4;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) *reinterpret_cast<bf16x8*>(so + 32 * s) = SB[s];
+    }
+    if (DELTA && p.vn_out) {
+      // A lane holds four tokens of a column, memory wants a token's columns side by side: 4 x 4 transposition within the four lanes
+      // of a quad, then one 8-byte store per token tile (single values took 16 stores a step, 1.4 us of its 3.7)
+      const u32x4 vw[2] = {__builtin_bit_cast(u32x4, VB[0]), __builtin_bit_cast(u32x4, VB[1])};
+      const unsigned sel = (i16 & 1) ? 0x03020706u : 0x05040100u;   // pairs of columns: of tokens 0, 2 (even lanes) or 1, 3
+      bf16_t* vo = p.vn_out + ((size_t)(bos + c * C + 4 * g4 + (i16 & 3)) * p.H + h) * p.V + vcol0 + 16 * wave + (i16 & 12);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const unsigned w0 = vw[t >> 1][2 * (t & 1)], w1 = vw[t >> 1][2 * (t & 1) + 1];
+        const unsigned a0 = __builtin_amdgcn_perm(__builtin_amdgcn_mov_dpp(w0, 0xB1, 0xf, 0xf, true), w0, sel);
+        const unsigned a1 = __builtin_amdgcn_perm(__builtin_amdgcn_mov_dpp(w1, 0xB1, 0xf, 0xf, true), w1, sel);
+        const unsigned y = __builtin_amdgcn_mov_dpp((i16 & 2) ? a0 : a1, 0x4E, 0xf, 0xf, true);
+        const u32x2 w = (i16 & 2) ? (u32x2){y, a1} : (u32x2){a0, y};
+        if (16 * t + 4 * g4 + (i16 & 3) < nvalid) *reinterpret_cast<u32x2*>(vo + (size_t)(16 * t) * p.H * p.V) = w;
       }
     }
     // every wave is done with this stage and has written its part of the output tile; the data-movement wave has

@@ -61,7 +61,16 @@ _SIDE_BY_SIDE_TOKENS_X_K = 2048 * 128
 SAVE_CHUNK_STATES = None
 SAVE_CHUNK_STATES_MAX_BYTES = 1 << 30
 _PREP_WORKSPACE_BYTES = 17 * 1024   # per chunk and head (csrc/natsl_linear.hip)
+_BWD_SCAN_COLUMNS_PER_WG = 64   # of the reverse scan (csrc/natsl_linear_bwd.hip)
 _SCAN_COLUMNS_PER_WG = 16   # state columns of the scan's narrowest workgroup (csrc/natsl_linear.hip)
+
+
+def _cu_count(dev) -> int:
+    index = dev.index if dev.index is not None else torch.cuda.current_device()
+    cus = _cu_counts.get(index)
+    if cus is None:
+        cus = _cu_counts[index] = torch.cuda.get_device_properties(index).multi_processor_count
+    return cus
 
 
 def _run_side_by_side(dev, n_chains: int, V: int, chain_tokens: int, K: int) -> bool:
@@ -69,11 +78,19 @@ def _run_side_by_side(dev, n_chains: int, V: int, chain_tokens: int, K: int) -> 
         return bool(CONCURRENT_BRANCHES)
     if chain_tokens * K < _SIDE_BY_SIDE_TOKENS_X_K:
         return False
-    index = dev.index if dev.index is not None else torch.cuda.current_device()
-    cus = _cu_counts.get(index)
-    if cus is None:
-        cus = _cu_counts[index] = torch.cuda.get_device_properties(index).multi_processor_count
-    return n_chains * (V // _SCAN_COLUMNS_PER_WG) < cus
+    return n_chains * (V // _SCAN_COLUMNS_PER_WG) < _cu_count(dev)
+
+
+def _bwd_side_stream(dev, n_chains: int, V: int, chain_tokens: int, K: int):
+    """The stream on which the softmax branch's backward runs next to the linear branch's, or None: one after the other.  The reverse
+    scan has a workgroup of 64 (for few chains 32) state columns per chain and walks the chunks one by one, so where it takes at most
+    half of the CUs the softmax kernels have the others meanwhile (B2 T3000 H6 K192 V384: 72 workgroups for 0.25 ms)."""
+    if CONCURRENT_BRANCHES is None:
+        if chain_tokens * K < _SIDE_BY_SIDE_TOKENS_X_K or 2 * n_chains * max(1, V // _BWD_SCAN_COLUMNS_PER_WG) > _cu_count(dev):
+            return None
+    elif not CONCURRENT_BRANCHES:
+        return None
+    return _get_attn_stream(dev)
 
 
 def _keep_chunk_states(q, v, cu_seqlens) -> bool:
@@ -404,7 +421,7 @@ class _MixedFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, do_lin, do_attn, dht):
         from ._linear_bwd import linear_chunk_backward
-        from .attns import parallel_attn_nats_bwd
+        from .attns import prepare_attn_nats_bwd
         cfg = ctx.cfg
         (q_a, k_a, v_a, q_l, k_l, v_l, g, types, lse, idx, nblk, o_attn, beta, h0) = ctx.saved_tensors[:14]
         linear_saved = tuple(ctx.saved_tensors[14:]) if ctx.n_linear_saved else None
@@ -414,19 +431,41 @@ class _MixedFunction(torch.autograd.Function):
         seqs = pack_sequences(cfg['cu_seqlens'], cfg['cu_seqlens_nats'], cfg['block'], types.device)
         if do_lin is None:
             do_lin = torch.zeros(*q_l.shape[:3], v_l.shape[-1], dtype=torch.float32, device=q_l.device)
+        if do_attn is not None:
+            do_attn = do_attn.to(torch.bfloat16).contiguous()
+        prepare = lambda *onto: prepare_attn_nats_bwd(q_a, k_a, v_a, o_attn, types, idx, nblk, None, lse, do_attn, cfg['scale_attn'], cfg['block'], 0,
+                                                      cfg['attn_same_block'], cfg['dnats_invalid_attn'], None, None, None, True, seqs, *onto)
+        # side by side: the softmax branch's tensors are made first, on this stream, and live until this stream has waited for the
+        # other one (nothing that is allocated in between can share their memory)
+        side = attn = None
+        if do_attn is not None and not any(ctx.shared):
+            n_seqs = B if seqs is None else seqs.n_seqs
+            side = _bwd_side_stream(q_l.device, n_seqs * q_l.shape[2], v_l.shape[-1], q_l.shape[1] * B // n_seqs, q_l.shape[-1])
+            if side is not None:
+                here = torch.cuda.current_stream(q_l.device)
+                attn = prepare()
+                side.wait_stream(here)
         lin_args = (cfg['scale_lattn'], cfg['block'], cfg['decay_non_linear'], cfg['qk_l2norm'], cfg['lin_intra'])
         later = []
-        dq_l, dk_l, dv_l, dg, dbeta, dh0, dn_lin = linear_chunk_backward(
-            cfg['kind'], q_l, k_l, v_l, g, beta, h0, types, *lin_args, do_lin, dht, cfg['dnats_invalid_linear'], seqs,
-            saved=linear_saved, later=later)
+        try:
+            dq_l, dk_l, dv_l, dg, dbeta, dh0, dn_lin = linear_chunk_backward(
+                cfg['kind'], q_l, k_l, v_l, g, beta, h0, types, *lin_args, do_lin, dht, cfg['dnats_invalid_linear'], seqs,
+                saved=linear_saved, later=later)
+            if side is not None:
+                attn[0](side.cuda_stream)
+        finally:
+            if side is not None:
+                here.wait_stream(side)
         lin = [dq_l, dk_l, dv_l]
         if do_attn is not None:
-            onto = tuple(t if both and t.dtype == torch.bfloat16 and t.is_contiguous() else None for t, both in zip(lin, ctx.shared))
-            dq_a, dk_a, dv_a, _, dn_attn = parallel_attn_nats_bwd(
-                q_a, k_a, v_a, o_attn, types, idx, nblk, None, lse, do_attn.to(torch.bfloat16).contiguous(), scale=cfg['scale_attn'],
-                NAtS_block_size=cfg['block'], compute_incomplete_chunk_scores=cfg['attn_same_block'],
-                compute_dnats_for_invalid_blocks_attn=cfg['dnats_invalid_attn'], seqs=seqs, onto=onto, sum_heads=not later)
-            lin = [None if have is not None else t for t, have in zip(lin, onto)]
+            if side is None:
+                onto = tuple(t if both and t.dtype == torch.bfloat16 and t.is_contiguous() else None for t, both in zip(lin, ctx.shared))
+                lin = [None if have is not None else t for t, have in zip(lin, onto)]
+                attn = prepare(onto)
+                attn[0](_capi.stream_ptr(q_l.device))
+            dq_a, dk_a, dv_a, dn_attn = attn[1]
+            if not later:
+                dn_attn = dn_attn.view(B, NB, HN, -1).sum(-1)
         else:
             dq_a, dk_a, dv_a = torch.zeros_like(q_a), torch.zeros_like(k_a), torch.zeros_like(v_a)
             dn_attn = torch.zeros(B, NB, q_a.shape[2] if later else HN, dtype=torch.float32, device=types.device)

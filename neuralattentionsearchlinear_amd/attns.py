@@ -53,7 +53,7 @@ def parallel_attn_nats_bwd(
         NAtS_block_size: int = 64, OFFSET_ATTN: int = 0, compute_incomplete_chunk_scores: bool = False,
         compute_dnats_for_invalid_blocks_attn: bool = False, sliding_window_size: Optional[int] = None,
         cu_seqlens=None, cu_seqlens_nats=None, is_causal: bool = True, chunk_indices_attn_nats=None,
-        seqs: Optional[PackedSeqs] = None, onto=(None, None, None), sum_heads: bool = True):
+        seqs: Optional[PackedSeqs] = None):
     """Backward of the softmax branch (host-side mirror of parallel_attn_nats_bwd, src/nats/ops/attns/attns.py:1562-1759)
     -> (dq [B,T,HQ,K], dk [B,T,H,K], dv [B,T,H,V], None, dnats [B,TNAtS,HNAtS]).
 
@@ -61,8 +61,21 @@ def parallel_attn_nats_bwd(
     straight-through gradient of the selector, attns.py:946-961); the other blocks get 0, or, with
     compute_dnats_for_invalid_blocks_attn, what their keys would contribute if they were visible (probabilities against
     the queries' lse, clamped to 1: attns.py:1318-1325).  Packed sequences: cu_seqlens (and cu_seqlens_nats), or the table
-    `seqs` built from them; n_nats_blocks is then [n_seqs,HN,2].  onto: gradients (contiguous bf16) that dq, dk, dv are added to in
-    place.  sum_heads=False: dnats per query head [B,TNAtS,HQ].  g_cumsum and sliding windows are not built."""
+    `seqs` built from them; n_nats_blocks is then [n_seqs,HN,2].  g_cumsum and sliding windows are not built."""
+    launch, (dq, dk, dv, dnats) = prepare_attn_nats_bwd(
+        q, k, v, o, nats_block_types, nats_block_indices, n_nats_blocks, g_cumsum, lse, do, scale, NAtS_block_size, OFFSET_ATTN,
+        compute_incomplete_chunk_scores, compute_dnats_for_invalid_blocks_attn, sliding_window_size, cu_seqlens, cu_seqlens_nats, is_causal, seqs)
+    launch(_capi.stream_ptr(q.device))
+    dnats = dnats.view(*dnats.shape[:2], nats_block_types.shape[2], -1).sum(-1)          # over the query heads of a selector head (attns.py:1755)
+    return dq, dk, dv, None, dnats
+
+
+def prepare_attn_nats_bwd(q, k, v, o, nats_block_types, nats_block_indices, n_nats_blocks, g_cumsum, lse, do, scale, NAtS_block_size, OFFSET_ATTN,
+                          compute_incomplete_chunk_scores, compute_dnats_for_invalid_blocks_attn, sliding_window_size, cu_seqlens, cu_seqlens_nats,
+                          is_causal, seqs, onto=(None, None, None)):
+    """parallel_attn_nats_bwd up to its kernels: everything is allocated and converted on the current stream -> (launch, (dq, dk, dv, dnats
+    per query head)); launch(stream) enqueues the kernels.  launch holds what they use: keep it until the current stream waits for
+    `stream`.  onto: gradients (contiguous bf16) that dq, dk, dv are added to in place."""
     if g_cumsum is not None or sliding_window_size is not None or not is_causal or OFFSET_ATTN != 0:
         raise NotImplementedError("only the causal backward without g_cumsum / sliding window is built")
     if seqs is None and cu_seqlens is not None:
@@ -88,16 +101,17 @@ def parallel_attn_nats_bwd(
     sp, ns, tot = _seq_args(seqs, seqs.total_qtiles if seqs is not None else 0)
     ws_bytes = L.natsl_softmax_bwd_workspace_bytes(B, T, HQ)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-    rc = L.natsl_softmax_sparse_bwd(
-        _capi.ptr(q), _capi.ptr(k), _capi.ptr(v), _capi.ptr(o), _capi.ptr(lse.contiguous()), _capi.ptr(do), _capi.ptr(dq),
-        _capi.ptr(dk), _capi.ptr(dv), _capi.ptr(dnats), _capi.ptr(ty), _capi.dtype_code(ty.dtype), _capi.ptr(nats_block_indices),
-        _capi.ptr(n_nats_blocks), B, T, HQ, H, HN, K, V, TN, NAtS_block_size, float(scale),
-        int(bool(compute_incomplete_chunk_scores)) | (2 if compute_dnats_for_invalid_blocks_attn else 0) | add, _capi.dtype_code(q.dtype),
-        _capi.ptr(ws), ws_bytes, sp, ns, tot, seqs.total_chunks if seqs is not None else 0, _capi.stream_ptr(q.device))
-    _capi.check(rc, "natsl_softmax_sparse_bwd")
-    if sum_heads:
-        dnats = dnats.view(B, TN, HN, HQ // HN).sum(-1)      # over the query heads of a selector head (attns.py:1755)
-    return dq, dk, dv, None, dnats
+    lse, idx, nblk = lse.contiguous(), nats_block_indices, n_nats_blocks
+
+    def launch(stream):
+        rc = L.natsl_softmax_sparse_bwd(
+            _capi.ptr(q), _capi.ptr(k), _capi.ptr(v), _capi.ptr(o), _capi.ptr(lse), _capi.ptr(do), _capi.ptr(dq), _capi.ptr(dk), _capi.ptr(dv),
+            _capi.ptr(dnats), _capi.ptr(ty), _capi.dtype_code(ty.dtype), _capi.ptr(idx), _capi.ptr(nblk), B, T, HQ, H, HN, K, V, TN,
+            NAtS_block_size, float(scale),
+            int(bool(compute_incomplete_chunk_scores)) | (2 if compute_dnats_for_invalid_blocks_attn else 0) | add, _capi.dtype_code(q.dtype),
+            _capi.ptr(ws), ws_bytes, sp, ns, tot, seqs.total_chunks if seqs is not None else 0, stream)
+        _capi.check(rc, "natsl_softmax_sparse_bwd")
+    return launch, (dq, dk, dv, dnats)
 
 
 class AttentionNAtSFunction(torch.autograd.Function):

@@ -285,3 +285,32 @@ def test_one_gradient_of_a_tensor_given_to_both_branches(kind, T, V, block, pack
         return [a.grad + b.grad for a, b in zip(one, two)]
     for a, b in zip(grads(True), grads(False)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("kind,T,K,V,block", [('gdn', 700, 128, 128, 64), ('mamba', 513, 64, 128, 128), ('gdn', 330, 192, 64, 64)])
+def test_backward_branches_side_by_side(kind, T, K, V, block, monkeypatch):
+    """The two branches' backward on two streams gives the gradients of one after the other, call after call."""
+    from neuralattentionsearchlinear_amd import _mixed_common as MC
+    B, H, KA, VA = 2, 4, 128 if K != 192 else 64, 128
+    gen = torch.Generator().manual_seed(T)
+    ql, kl, vl = make_qkv(B, T, H, K, V, 5)
+    qa, ka, va = make_qkv(B, T, H, KA, VA, 8)
+    g, beta = make_gates(B, T, H, 6)
+    ty = make_types(B, -(-T // block), 2, 0.4, 7, torch.bfloat16)
+    do_l, do_a = torch.randn(B, T, H, V, generator=gen).bfloat16().to(DEV), torch.randn(B, T, H, VA, generator=gen).bfloat16().to(DEV)
+
+    def grads(side):
+        monkeypatch.setattr(MC, 'CONCURRENT_BRANCHES', side)
+        leaves = [t.to(DEV).requires_grad_(True) for t in (qa, ka, va, ql, kl, vl, g, ty)]
+        bd = beta.to(DEV).requires_grad_(True) if kind == 'gdn' else None
+        o_l, o_a, _ = MC.mixed_forward(kind, *leaves[:6], None, leaves[6], bd, leaves[7], 0.1, 0.1, None, None, block, None, True, True, True, True,
+                                       True, False, kind == 'gdn')
+        torch.autograd.backward([o_l, o_a], [do_l, do_a])
+        return [t.grad for t in leaves] + ([bd.grad] if bd is not None else [])
+    want = grads(False)
+    for _ in range(3):
+        for i, (a, b) in enumerate(zip(grads(True), want)):
+            if i == 7:                                   # (block types: one atomic addition per unit, in any order)
+                assert rel_l2(a, b) < 1e-2
+            else:
+                assert torch.equal(a, b), i

@@ -126,34 +126,29 @@ NATSL_DEVICE bf16x8 tr_operand(const bf16_t* base, const int pitch, const int ro
 
 // q^, k^ rows of a chunk: what a thread fetches (row tid / 4, 16-byte pieces tid % 4 + 4 i) and, normalised, puts into LDS
 template <int DK>
-struct QkRegs {
-  u32x4 a[DK / 32], b[DK / 32];
-};
-
-template <int DK>
-NATSL_DEVICE void load_qk(const LinBwdParams& p, const int tid, const size_t row0, const int nvalid, const int h, QkRegs<DK>& r) {
+NATSL_DEVICE void load_qk(const LinBwdParams& p, const int tid, const size_t row0, const int nvalid, const int h, u32x4* ra, u32x4* rb) {
   const int row = tid >> 2, sub = tid & 3;
   const bool ok = row < nvalid;
   const size_t off = ((row0 + row) * p.H + h) * DK;
   const u32x4 z = {0u, 0u, 0u, 0u};
 #pragma unroll
   for (int i = 0; i < DK / 32; ++i) {
-    r.a[i] = ok ? *reinterpret_cast<const u32x4*>(p.q + off + (sub + 4 * i) * 8) : z;
-    r.b[i] = ok ? *reinterpret_cast<const u32x4*>(p.k + off + (sub + 4 * i) * 8) : z;
+    ra[i] = ok ? *reinterpret_cast<const u32x4*>(p.q + off + (sub + 4 * i) * 8) : z;
+    rb[i] = ok ? *reinterpret_cast<const u32x4*>(p.k + off + (sub + 4 * i) * 8) : z;
   }
 }
 
 // rows past the end of the sequence arrive as zeros
 template <int DK>
-NATSL_DEVICE void store_qk(const QkRegs<DK>& r, const int tid, const bool l2, bf16_t* Qn, bf16_t* Kn, float* rq, float* rk) {
+NATSL_DEVICE void store_qk(const u32x4* ra, const u32x4* rb, const int tid, const bool l2, bf16_t* Qn, bf16_t* Kn, float* rq, float* rk) {
   constexpr int KP = DK + 8, KL = DK / 32;
   const int row = tid >> 2, sub = tid & 3;
   float sq = 0.f, sk = 0.f;
 #pragma unroll
   for (int i = 0; i < KL; ++i) {
     float fa[8], fb[8];
-    unpack8f(r.a[i], fa);
-    unpack8f(r.b[i], fb);
+    unpack8f(ra[i], fa);
+    unpack8f(rb[i], fb);
 #pragma unroll
     for (int e = 0; e < 8; ++e) { sq += fa[e] * fa[e]; sk += fb[e] * fb[e]; }
   }
@@ -165,8 +160,8 @@ NATSL_DEVICE void store_qk(const QkRegs<DK>& r, const int tid, const bool l2, bf
   for (int i = 0; i < KL; ++i) {
     const int seg = sub + 4 * i;
     float fa[8], fb[8];
-    unpack8f(r.a[i], fa);
-    unpack8f(r.b[i], fb);
+    unpack8f(ra[i], fa);
+    unpack8f(rb[i], fb);
     u32x4 wa, wb;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -829,10 +824,6 @@ __global__ __launch_bounds__(256, DK <= 128 ? 2 : 1) void linear_bwd_chunk_kerne
     const size_t gi = (row0 + lane) * p.H + h;
     store_scalars<DELTA>(lane, ok ? p.g[gi] : 0.f, DELTA && ok ? bf16_to_f32(p.beta[gi]) : 0.f, p.scale, gam, eg, ek, sqv, bet);
   }
-  // q^, k^ are requested now and put into LDS when phase 1 is done with it
-  QkRegs<DK> qk;
-  load_qk<DK>(p, tid, row0, nvalid, h, qk);
-
   // ---- phase 1 -------------------------------------------------------------------------------------------------------
   bf16_t* const DOs = sm + L::DO;
   bf16_t* const DXs = sm + L::DX;
@@ -851,47 +842,69 @@ __global__ __launch_bounds__(256, DK <= 128 ? 2 : 1) void linear_bwd_chunk_kerne
   const bf16_t* s_src = p.s_all + unit * p.V * DK;
   const bf16_t* ds_src = p.ds_all + unit * p.V * DK;
   const bf16_t* sf_src = p.s_all + ((size_t)(chunk_off + c_first) * p.H + h) * p.V * DK;
-  for (int vs = 0; vs < p.V / 64; ++vs) {
-    u32x4 w_do[2], w_vn[2], w_dx[2];
-    load_tokens64(p.d_o, tid, row0, nvalid, p.H, p.V, h, 64 * vs, w_do);
-    load_tokens64(p.vn, tid, row0, nvalid, p.H, p.V, h, 64 * vs, w_vn);
-    if (DELTA) load_tokens64(p.dv, tid, row0, nvalid, p.H, p.V, h, 64 * vs, w_dx);
+  // What a slice needs -- dO, v_new, dX; the state and its gradient as they lie in memory, [64 columns][K] -- is requested as a whole
+  // while the slice before it multiplies (behind the last one: the q, k rows), and waits in registers until the tiles are free.
+  // Requested piece by piece where it was used, a slice paid two memory latencies (K192 V384: six slices, one workgroup per CU).
+  // The delta rule at K = 128 has no registers for all of it (two workgroups per CU: 256): its token rows are requested at the top.
+  constexpr int NT3 = DELTA ? 6 : 4, NP = 64 * (DK / 8) / 256;
+  const int n_slices = p.V / 64;
+  u32x4 in[NT3 + 2 * NP];
+  constexpr int QK0 = 2 * (DK / 32) <= 2 * NP ? NT3 : 0;
+  static_assert(2 * (DK / 32) <= NT3 + 2 * NP - QK0, "the q, k rows fit the same registers");
+  constexpr bool TOKENS_AHEAD = !(DELTA && DK == 128);
+  auto request_tokens = [&](const int vs) __attribute__((always_inline)) {
+    load_tokens64(p.d_o, tid, row0, nvalid, p.H, p.V, h, 64 * vs, in);
+    load_tokens64(p.vn, tid, row0, nvalid, p.H, p.V, h, 64 * vs, in + 2);
+    if (DELTA) load_tokens64(p.dv, tid, row0, nvalid, p.H, p.V, h, 64 * vs, in + 4);
+  };
+  auto request_states = [&](const int vs) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      // (64 rows of K in a row: piece tid + 256 i of the slice lies at that place)
+      const size_t off = (size_t)64 * vs * DK + (size_t)(tid + 256 * i) * 8;
+      in[NT3 + i] = *reinterpret_cast<const u32x4*>(s_src + off);
+      in[NT3 + NP + i] = *reinterpret_cast<const u32x4*>(ds_src + off);
+    }
+  };
+  if (TOKENS_AHEAD) request_tokens(0);
+  request_states(0);
+  for (int vs = 0; vs < n_slices; ++vs) {
+    if (!TOKENS_AHEAD) request_tokens(vs);
     __syncthreads();   // the previous slice's tiles are dead
-    store_tokens64(w_do, tid, DOs);
-    store_tokens64(w_vn, tid, VNs);
-    if (DELTA) store_tokens64(w_dx, tid, DXs);
-    // the state and its gradient as they lie in memory: [64 columns][K]; a thread's pieces are all requested before the
-    // first of them is used
-    {
-      constexpr int NP = 64 * (DK / 8) / 256;
-      u32x4 ws[NP], wd[NP];
+    store_tokens64(in, tid, DOs);
+    store_tokens64(in + 2, tid, VNs);
+    if (DELTA) store_tokens64(in + 4, tid, DXs);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int pc = tid + 256 * i, v = pc / (DK / 8), seg = pc % (DK / 8);
+      *reinterpret_cast<u32x4*>(Sn + v * KP + seg * 8) = in[NT3 + i];
+      *reinterpret_cast<u32x4*>(DSn + v * KP + seg * 8) = in[NT3 + NP + i];
+      float fs[8], fd[8];
+      unpack8f(in[NT3 + i], fs);
+      unpack8f(in[NT3 + NP + i], fd);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sds += fs[e] * fd[e];
+    }
+    if (want_rb && c != c_first) {   // (at a block's first chunk the state that entered the block is the chunk's own)
+      u32x4 wf[NP];
+#pragma unroll
+      for (int i = 0; i < NP; ++i) wf[i] = *reinterpret_cast<const u32x4*>(sf_src + (size_t)64 * vs * DK + (size_t)(tid + 256 * i) * 8);
 #pragma unroll
       for (int i = 0; i < NP; ++i) {
-        const int pc = tid + 256 * i, v = pc / (DK / 8), seg = pc % (DK / 8);
-        const size_t off = (size_t)(64 * vs + v) * DK + seg * 8;
-        ws[i] = *reinterpret_cast<const u32x4*>(s_src + off);
-        wd[i] = *reinterpret_cast<const u32x4*>(ds_src + off);
-      }
+        float ff[8], fd[8];
+        unpack8f(wf[i], ff);
+        unpack8f(in[NT3 + NP + i], fd);
 #pragma unroll
-      for (int i = 0; i < NP; ++i) {
-        const int pc = tid + 256 * i, v = pc / (DK / 8), seg = pc % (DK / 8);
-        const size_t off = (size_t)(64 * vs + v) * DK + seg * 8;
-        *reinterpret_cast<u32x4*>(Sn + v * KP + seg * 8) = ws[i];
-        *reinterpret_cast<u32x4*>(DSn + v * KP + seg * 8) = wd[i];
-        float fs[8], fd[8];
-        unpack8f(ws[i], fs);
-        unpack8f(wd[i], fd);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sds += fs[e] * fd[e];
-        if (want_rb) {
-          float ff[8];
-          unpack8f(*reinterpret_cast<const u32x4*>(sf_src + off), ff);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) srb += ff[e] * fd[e];
-        }
+        for (int e = 0; e < 8; ++e) srb += ff[e] * fd[e];
       }
     }
     __syncthreads();
+    if (vs + 1 < n_slices) {
+      if (TOKENS_AHEAD) request_tokens(vs + 1);
+      request_states(vs + 1);
+    } else {
+      load_qk<DK>(p, tid, row0, nvalid, h, in + QK0, in + QK0 + DK / 32);
+    }
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const bf16x8 a_do = *reinterpret_cast<const bf16x8*>(DOs + (16 * wave + x16) * TP + 32 * s + 8 * g4);
@@ -917,7 +930,7 @@ __global__ __launch_bounds__(256, DK <= 128 ? 2 : 1) void linear_bwd_chunk_kerne
   }
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) { sds += __shfl_xor(sds, d); srb += __shfl_xor(srb, d); }
-  if (lane == 0) { red[wave] = sds; red[4 + wave] = srb; }
+  if (lane == 0) { red[wave] = sds; red[4 + wave] = c == c_first ? sds : srb; }
 
   // ---- phase 2 -------------------------------------------------------------------------------------------------------
   bf16_t* const Qn = sm + L::QN;
@@ -926,7 +939,7 @@ __global__ __launch_bounds__(256, DK <= 128 ? 2 : 1) void linear_bwd_chunk_kerne
   bf16_t* const GT = sm + L::GT;
   bf16_t* const Hs = sm + L::HS;
   __syncthreads();   // phase 1's tiles are dead
-  store_qk<DK>(qk, tid, l2, Qn, Kn, rq, rk);
+  store_qk<DK>(in + QK0, in + QK0 + DK / 32, tid, l2, Qn, Kn, rq, rk);
   if (DELTA)
     for (int i = tid; i < CB * TP / 8; i += 256) *reinterpret_cast<u32x4*>(Hs + 8 * i) = (u32x4){0u, 0u, 0u, 0u};
   __syncthreads();

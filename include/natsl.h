@@ -371,6 +371,12 @@ int natsl_kv_compact(const void* src_k, const void* src_v, long long src_tokens,
                      int HN, int K, int V, int dtype, int block, int NB, int n_complete, int tail_dst, int tail_tokens,
                      natsl_stream_t stream);
 
+/* natsl_kv_compact into a cache that is new (uninitialised) memory of whole blocks: the first region of a sequence, nothing kept
+ * before; every block of the cache that holds nothing is zeroed. */
+int natsl_kv_collect(const void* src_k, const void* src_v, long long src_tokens, void* dst_k, void* dst_v, long long dst_tokens, const void* types,
+                     int types_dtype, int B, int HKV, int HN, int K, int V, int dtype, int block, int NB, int n_complete, int tail_dst,
+                     int tail_tokens, natsl_stream_t stream);
+
 /* The cache's bookkeeping around natsl_kv_compact: n_after [B, HN] = n_before (or 0) + the attention-typed blocks among the first
  * n_complete of types [B, NB, HN, 2], with the largest of them written to *host_max (HOST memory that the GPU can write); and the
  * validity flags valid [B, blocks, HN] of n_after kept blocks plus the incomplete block at tail_block (-1 = none).

@@ -244,28 +244,33 @@ class NAtSLayerCache:
         ready.synchronize()                                                     # the host needs the largest count to size the cache
         new_max = int(host)
         tail_dst = new_max if tail_tokens else -1
-        if self.attn_k is None:
+        L, P = _capi.lib(), _capi.ptr
+        fresh = self.attn_k is None
+        if fresh:
             src_k, src_v = (t.contiguous() for t in (self._pending_first if self._pending_first is not None else attn_state))
             self._pending_first = None
             cap = (new_max + 2) * bs
-            self.attn_k = torch.zeros(B, cap, *src_k.shape[2:], dtype=src_k.dtype, device=src_k.device)
-            self.attn_v = torch.zeros(B, cap, *src_v.shape[2:], dtype=src_v.dtype, device=src_v.device)
+            fresh = before is None                                                   # (the kernel zeroes what it does not fill)
+            make = torch.empty if fresh else torch.zeros
+            self.attn_k = make(B, cap, *src_k.shape[2:], dtype=src_k.dtype, device=src_k.device)
+            self.attn_v = make(B, cap, *src_v.shape[2:], dtype=src_v.dtype, device=src_v.device)
             src_block0 = 0
         else:
-            src_k, src_v, src_block0 = self.attn_k, self.attn_v, self.n_attn_blocks_max
+            src_block0 = self.n_attn_blocks_max
             self._grow((new_max + 1) * bs)
             src_k, src_v = self.attn_k, self.attn_v
         if src_k.dtype != src_v.dtype:
             raise ValueError("attention keys and values must share a dtype")
         HKV = src_k.shape[2]
-        if before is not None:
-            before = before.to(torch.int64).contiguous()
-        rc = _capi.lib().natsl_kv_compact(
-            _capi.ptr(src_k), _capi.ptr(src_v), src_k.shape[1], src_block0, _capi.ptr(self.attn_k), _capi.ptr(self.attn_v),
-            self.attn_k.shape[1], _capi.ptr(types), _capi.dtype_code(types.dtype), _capi.ptr(before), B, HKV, HN,
-            src_k.shape[3], src_v.shape[3], _capi.dtype_code(src_k.dtype), bs, NB, n_complete, tail_dst, tail_tokens,
-            _capi.stream_ptr(src_k.device))
-        _capi.check(rc, "natsl_kv_compact")
+        dst = (P(self.attn_k), P(self.attn_v), self.attn_k.shape[1], P(types), _capi.dtype_code(types.dtype))
+        rest = (B, HKV, HN, src_k.shape[3], src_v.shape[3], _capi.dtype_code(src_k.dtype), bs, NB, n_complete, tail_dst, tail_tokens,
+                _capi.stream_ptr(src_k.device))
+        if fresh:
+            _capi.check(L.natsl_kv_collect(P(src_k), P(src_v), src_k.shape[1], *dst, *rest), "natsl_kv_collect")
+        else:
+            if before is not None:
+                before = before.to(torch.int64).contiguous()
+            _capi.check(L.natsl_kv_compact(P(src_k), P(src_v), src_k.shape[1], src_block0, *dst, P(before), *rest), "natsl_kv_compact")
         self.n_attn_blocks = after
         self.n_attn_blocks_max = new_max
         blocks = self.attn_k.shape[1] // bs

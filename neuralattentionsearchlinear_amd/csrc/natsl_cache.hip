@@ -33,6 +33,7 @@ struct KvCompactParams {
   int NB, n_complete;                     // blocks in the region / how many of them are complete
   int tail_dst, tail_tokens;              // destination block of the incomplete block (-1: none), tokens in it
   int wgs[2];                             // workgroups per (sequence, head) for K and for V
+  int zero_rest;                          // the destination is new memory: blocks that hold nothing get zeros
 };
 
 NATSL_DEVICE bool kv_is_attn(const KvCompactParams& p, int b, int s, int hn) {
@@ -108,6 +109,10 @@ __global__ __launch_bounds__(256) void kv_compact_kernel(KvCompactParams p) {
       *daddr(p.tail_dst) = x;
     }
   }
+  // (a cache made in one go costs its bytes once; zeroed as a whole before, the kept blocks' bytes were written twice)
+  if (p.zero_rest && active)
+    for (long blk = dst; blk < p.dst_cap / p.block; ++blk)
+      if (blk != p.tail_dst) *daddr(blk) = (u32x4){0u, 0u, 0u, 0u};
 }
 
 // ---- bookkeeping of the kept blocks ----------------------------------------------------------------------------------------
@@ -153,11 +158,9 @@ __global__ __launch_bounds__(256) void kv_flags_kernel(const int64_t* after, uin
 
 using namespace natsl;
 
-extern "C" int natsl_kv_compact(const void* src_k, const void* src_v, long long src_tokens, int src_block0, void* dst_k,
-                                void* dst_v, long long dst_tokens, const void* types, int types_dtype,
-                                const int64_t* n_before, int B, int HKV, int HN, int K, int V, int dtype, int block,
-                                int NB, int n_complete, int tail_dst, int tail_tokens, natsl_stream_t stream) {
-  const char* what = "natsl_kv_compact";
+static int kv_compact(const char* what, bool zero_rest, const void* src_k, const void* src_v, long long src_tokens, int src_block0, void* dst_k,
+                      void* dst_v, long long dst_tokens, const void* types, int types_dtype, const int64_t* n_before, int B, int HKV, int HN, int K,
+                      int V, int dtype, int block, int NB, int n_complete, int tail_dst, int tail_tokens, natsl_stream_t stream) {
   if (!src_k || !src_v || !dst_k || !dst_v || !types) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
   if (dtype != NATSL_BF16 && dtype != NATSL_F32) return fail(NATSL_ERR_UNSUPPORTED, "%s: tensors must be f32 or bf16", what);
   if (types_dtype != NATSL_BF16 && types_dtype != NATSL_F32) return fail(NATSL_ERR_UNSUPPORTED, "%s: block types must be f32 or bf16", what);
@@ -185,9 +188,28 @@ extern "C" int natsl_kv_compact(const void* src_k, const void* src_v, long long 
   p.types = types; p.types_dtype = types_dtype; p.n_before = n_before;
   p.B = B; p.HKV = HKV; p.HN = HN; p.block = block; p.src_block0 = src_block0; p.NB = NB; p.n_complete = n_complete;
   p.tail_dst = tail_dst; p.tail_tokens = tail_tokens;
+  p.zero_rest = zero_rest ? 1 : 0;
   p.wgs[0] = cdiv(block * (p.row[0] / 16), 256); p.wgs[1] = cdiv(block * (p.row[1] / 16), 256);
   hipLaunchKernelGGL(kv_compact_kernel, dim3(p.wgs[0] + p.wgs[1], B * HKV), dim3(256), 0, (hipStream_t)stream, p);
   return check_launch(what);
+}
+
+extern "C" int natsl_kv_compact(const void* src_k, const void* src_v, long long src_tokens, int src_block0, void* dst_k,
+                                void* dst_v, long long dst_tokens, const void* types, int types_dtype,
+                                const int64_t* n_before, int B, int HKV, int HN, int K, int V, int dtype, int block,
+                                int NB, int n_complete, int tail_dst, int tail_tokens, natsl_stream_t stream) {
+  return kv_compact("natsl_kv_compact", false, src_k, src_v, src_tokens, src_block0, dst_k, dst_v, dst_tokens, types, types_dtype, n_before, B, HKV, HN,
+                    K, V, dtype, block, NB, n_complete, tail_dst, tail_tokens, stream);
+}
+
+extern "C" int natsl_kv_collect(const void* src_k, const void* src_v, long long src_tokens, void* dst_k, void* dst_v, long long dst_tokens,
+                                const void* types, int types_dtype, int B, int HKV, int HN, int K, int V, int dtype, int block, int NB, int n_complete,
+                                int tail_dst, int tail_tokens, natsl_stream_t stream) {
+  const char* what = "natsl_kv_collect";
+  if (src_k == dst_k || src_v == dst_v) return fail(NATSL_ERR_INVALID, "%s: the cache must be new memory", what);
+  if (block <= 0 || dst_tokens <= 0 || dst_tokens % block) return fail(NATSL_ERR_INVALID, "%s: the cache must hold whole blocks", what);
+  return kv_compact(what, true, src_k, src_v, src_tokens, 0, dst_k, dst_v, dst_tokens, types, types_dtype, nullptr, B, HKV, HN, K, V, dtype, block, NB,
+                    n_complete, tail_dst, tail_tokens, stream);
 }
 
 extern "C" int natsl_kv_counts(const void* types, int types_dtype, const int64_t* n_before, int64_t* n_after, int32_t* host_max, int B, int HN, int NB,

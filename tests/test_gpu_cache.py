@@ -247,3 +247,25 @@ def test_long_continuation_on_a_filled_cache(kind, ops, T0, T1):
     if a2 is not None:
         assert ca.n_observed_tokens == cb.n_observed_tokens == T1 + 1
         assert rel_l2(a2.float(), b2.float()) <= 1e-2, f"the next token: rel-L2 {rel_l2(a2.float(), b2.float()):.3e}"
+
+
+@pytest.mark.parametrize("T,block,K,V,dtype", [(64, 64, 64, 128, torch.bfloat16), (300, 64, 128, 64, torch.bfloat16), (513, 128, 64, 64, torch.float32)])
+def test_a_cache_made_in_new_memory(T, block, K, V, dtype):
+    """natsl_kv_collect into memory that holds NaN = natsl_kv_compact into zeroed memory, every byte."""
+    from neuralattentionsearchlinear_amd import _capi
+    B, HKV, HN = 2, 4, 2
+    gen = torch.Generator().manual_seed(T)
+    NB, n_complete, tail = -(-T // block), T // block, T % block
+    types = (torch.rand(B, NB, HN, 2, generator=gen) < 0.5).to(torch.bfloat16).cuda()
+    k, v = torch.randn(B, T, HKV, K, generator=gen).to(dtype).cuda(), torch.randn(B, T, HKV, V, generator=gen).to(dtype).cuda()
+    most = int(types[:, :n_complete, :, 0].float().sum(1).max())
+    cap = (most + 2) * block
+    P, L, s = _capi.ptr, _capi.lib(), _capi.stream_ptr(k.device)
+    got = [torch.full((B, cap, HKV, n), float('nan'), dtype=dtype, device='cuda') for n in (K, V)]
+    want = [torch.zeros_like(t) for t in got]
+    head = (P(types), _capi.BF16)
+    rest = (B, HKV, HN, K, V, _capi.dtype_code(dtype), block, NB, n_complete, most if tail else -1, tail, s)
+    _capi.check(L.natsl_kv_collect(P(k), P(v), T, P(got[0]), P(got[1]), cap, *head, *rest), "natsl_kv_collect")
+    _capi.check(L.natsl_kv_compact(P(k), P(v), T, 0, P(want[0]), P(want[1]), cap, *head, None, *rest), "natsl_kv_compact")
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)

@@ -10,7 +10,6 @@ from . import _capi
 from .nats_util import CHUNK_SIZE, PackedSeqs, _seq_args, pack_sequences
 
 _attn_streams: dict = {}
-_cu_counts: dict = {}
 
 
 class _Cast(ctypes.Structure):
@@ -41,12 +40,12 @@ TIMING_HOOK = None
 
 # Where the softmax branch is launched.  True: on a side stream next to the linear branch (as the
 # reference's Mamba operator does); False: on the caller's stream, one branch after the other (as the
-# reference's GDN operator does); None: decide per call - side by side only when the linear branch's scan
-# cannot give every CU a workgroup even at its narrowest (one compute wave = 16 state columns per workgroup) and its chain is
-# long enough.  Both kernels take most of a CU's LDS (127 KiB / 159 KiB), so they never share a CU: when each fills the
-# machine alone, running them side by side gains nothing (measured) and only blurs timings.  Ordering two streams costs a call
-# about 40 us (36 us one after the other, 78 us side by side at T 256), which the overlap repays from a chain of 2048 tokens at
-# K = 128 on (4096 at K = 64): 87 -> 78 us at B1 T2048 H6, 154 -> 111 us at T 4096, but 56 -> 81 us at T 1024.
+# reference's GDN operator does); None: decide per call - side by side where the linear branch's chain is long enough.  Its scan
+# walks the chunks one by one with a few large workgroups, so the softmax kernel fills the CUs it leaves; both take most of a CU's
+# LDS (127 KiB / 159 KiB) and never share one, so a scan that fills the chip by itself neither gains nor loses (B8 T8192 H16: 1042
+# and 1045 us; B4 T8192 H8 400 -> 326, Mamba B4 T8192 H32 764 -> 699, four packed documents of 65536 tokens 2274 -> 2162).  Ordering two
+# streams costs a call about 40 us (36 us one after the other, 78 us side by side at T 256), which the overlap repays from a chain of
+# 2048 tokens at K = 128 on (4096 at K = 64): 87 -> 78 us at B1 T2048 H6, 154 -> 111 us at T 4096, but 56 -> 81 us at T 1024.
 CONCURRENT_BRANCHES = None
 _SIDE_BY_SIDE_TOKENS_X_K = 2048 * 128
 
@@ -61,36 +60,13 @@ _SIDE_BY_SIDE_TOKENS_X_K = 2048 * 128
 SAVE_CHUNK_STATES = None
 SAVE_CHUNK_STATES_MAX_BYTES = 1 << 30
 _PREP_WORKSPACE_BYTES = 17 * 1024   # per chunk and head (csrc/natsl_linear.hip)
-_BWD_SCAN_COLUMNS_PER_WG = 64   # of the reverse scan (csrc/natsl_linear_bwd.hip)
-_SCAN_COLUMNS_PER_WG = 16   # state columns of the scan's narrowest workgroup (csrc/natsl_linear.hip)
 
 
-def _cu_count(dev) -> int:
-    index = dev.index if dev.index is not None else torch.cuda.current_device()
-    cus = _cu_counts.get(index)
-    if cus is None:
-        cus = _cu_counts[index] = torch.cuda.get_device_properties(index).multi_processor_count
-    return cus
-
-
-def _run_side_by_side(dev, n_chains: int, V: int, chain_tokens: int, K: int) -> bool:
+def _run_side_by_side(chain_tokens: int, K: int) -> bool:
+    """Whether the softmax branch (forward or backward) goes to the side stream (see CONCURRENT_BRANCHES)."""
     if CONCURRENT_BRANCHES is not None:
         return bool(CONCURRENT_BRANCHES)
-    if chain_tokens * K < _SIDE_BY_SIDE_TOKENS_X_K:
-        return False
-    return n_chains * (V // _SCAN_COLUMNS_PER_WG) < _cu_count(dev)
-
-
-def _bwd_side_stream(dev, n_chains: int, V: int, chain_tokens: int, K: int):
-    """The stream on which the softmax branch's backward runs next to the linear branch's, or None: one after the other.  The reverse
-    scan has a workgroup of 64 (for few chains 32) state columns per chain and walks the chunks one by one, so where it takes at most
-    half of the CUs the softmax kernels have the others meanwhile (B2 T3000 H6 K192 V384: 72 workgroups for 0.25 ms)."""
-    if CONCURRENT_BRANCHES is None:
-        if chain_tokens * K < _SIDE_BY_SIDE_TOKENS_X_K or 2 * n_chains * max(1, V // _BWD_SCAN_COLUMNS_PER_WG) > _cu_count(dev):
-            return None
-    elif not CONCURRENT_BRANCHES:
-        return None
-    return _get_attn_stream(dev)
+    return chain_tokens * K >= _SIDE_BY_SIDE_TOKENS_X_K
 
 
 def _keep_chunk_states(q, v, cu_seqlens) -> bool:
@@ -286,7 +262,7 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
     total_chunks = seqs.total_chunks if seqs is not None else B * (-(-T // CHUNK_SIZE))
     # every tensor below belongs to the caller's stream; the softmax branch's stream starts after what that stream holds and is
     # waited for before the call returns, so memory that is freed later is only ever used again behind both
-    side = _get_attn_stream(dev) if _run_side_by_side(dev, n_seqs * H, V, T * B // n_seqs, K) else None
+    side = _get_attn_stream(dev) if _run_side_by_side(T * B // n_seqs, K) else None
     attn_stream = cur if side is None else side.cuda_stream
     want_start = inference and output_final_state
     chunk_states = keep_chunk_states and not want_start
@@ -439,8 +415,8 @@ class _MixedFunction(torch.autograd.Function):
         # other one (nothing that is allocated in between can share their memory)
         side = attn = None
         if do_attn is not None and not any(ctx.shared):
-            n_seqs = B if seqs is None else seqs.n_seqs
-            side = _bwd_side_stream(q_l.device, n_seqs * q_l.shape[2], v_l.shape[-1], q_l.shape[1] * B // n_seqs, q_l.shape[-1])
+            if _run_side_by_side(q_l.shape[1] * B // (B if seqs is None else seqs.n_seqs), q_l.shape[-1]):
+                side = _get_attn_stream(q_l.device)
             if side is not None:
                 here = torch.cuda.current_stream(q_l.device)
                 attn = prepare()

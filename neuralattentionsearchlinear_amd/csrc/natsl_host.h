@@ -38,6 +38,18 @@ inline int reserve_lds(const void* kern, std::atomic<unsigned long long>& done, 
   return NATSL_OK;
 }
 
+// Work on another stream that runs next to the linear branch's scan: ready(stream, other, what) is called between what the whole chip
+// does (the prep kernel) and the scan.
+struct BesideScan {
+  int (*ready)(hipStream_t, hipStream_t, const char*);
+  hipStream_t other;
+};
+// The two chunked linear branches behind their C entries (natsl_linear.hip); beside: null, or what the scan shares the chip with.
+int linear_fwd(bool delta, const void* q, const void* k, const void* v, const float* g, const void* beta, const float* h0, void* o, float* ht,
+               float* hs, float* gs, void* chunk_states, void* chunk_v_new, const void* types, int types_dtype, int B, int T, int H, int HN, int K,
+               int V, int TN, int block, float scale, int flags, void* workspace, size_t workspace_bytes, int dtype, const natsl_seq_row* seqs,
+               int n_seqs, int total_units, natsl_stream_t stream, const BesideScan* beside);
+
 inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 }  // namespace natsl

@@ -1050,7 +1050,7 @@ static int launch_scan(const LinearParams& p, hipStream_t stream, const char* wh
 }
 
 template <int DK, bool DELTA>
-static int launch_linear(const LinearParams& p, hipStream_t stream, const char* what) {
+static int launch_linear(const LinearParams& p, hipStream_t stream, const BesideScan* beside, const char* what) {
   const long long units = (long long)p.total_chunks * p.H;
   if (units <= 0) return NATSL_OK;
   // Waves per workgroup (16 state columns each).  A CU holds one workgroup (LDS), so a launch takes
@@ -1066,7 +1066,11 @@ static int launch_linear(const LinearParams& p, hipStream_t stream, const char* 
   // (K = 192: five waves of that size do not fit the registers of a CU without spilling; three do)
   const bool ok4 = DK <= 128 && p.V % 64 == 0, ok2 = p.V % 32 == 0;
   const double c1 = cost(1, 1.0), c2 = ok2 ? cost(2, 1.1) : 1e30, c4 = ok4 ? cost(4, 1.65) : 1e30;
-  const int nw = (c4 <= c2 && c4 <= c1) ? 4 : (c2 <= c1 ? 2 : 1);
+  int nw = (c4 <= c2 && c4 <= c1) ? 4 : (c2 <= c1 ? 2 : 1);
+  // With another kernel waiting for the CUs that the scan leaves, wider workgroups: 1, 1.1, 1.65 times the step on 1, 1/2, 1/4 of the
+  // CUs.  The narrowest that leaves that kernel three quarters of the chip (one wave) or half of it (two): both branches at
+  // B4 T8192 H8 one after the other (one wave, 256 workgroups) 400 us, side by side with two waves 326; Mamba B2 T8192 H32 480 -> 395.
+  if (beside) nw = 4 * n_chains * (p.V / 16) <= cus ? 1 : ok2 && (!ok4 || 2 * n_chains * (p.V / 32) <= cus) ? 2 : ok4 ? 4 : nw;
   // The delta rule's four-wave scan forms P itself and the prep reads k only, when the launch fills the machine: prep and scan
   // are then bound by their HBM traffic, which this cuts by a fifth (measured at B8 T8192 H16: 0.46 -> 0.43 ms), while a launch
   // that leaves CUs idle is bound by the scan's step and only gets slower from the extra work in it (B8 T4096 H6 V256:
@@ -1084,6 +1088,7 @@ static int launch_linear(const LinearParams& p, hipStream_t stream, const char* 
     hipLaunchKernelGGL(mamba_scale_kernel, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, stream, p);
   }
   int rc = check_launch(what);
+  if (rc == NATSL_OK && beside) rc = beside->ready(stream, beside->other, what);
   if (rc != NATSL_OK) return rc;
   if constexpr (!DELTA) {
     // the Mamba form's P is always formed by the data-movement waves (nothing about it comes from a prep kernel)
@@ -1104,10 +1109,10 @@ static int launch_linear(const LinearParams& p, hipStream_t stream, const char* 
   }
 }
 
-static int linear_fwd(bool delta, const void* q, const void* k, const void* v, const float* g, const void* beta,
+int linear_fwd(bool delta, const void* q, const void* k, const void* v, const float* g, const void* beta,
                       const float* h0, void* o, float* ht, float* hs, float* gs, void* chunk_states, void* chunk_v_new, const void* types, int types_dtype, int B, int T,
                       int H, int HN, int K, int V, int TN, int block, float scale, int flags, void* workspace, size_t workspace_bytes,
-                      int dtype, const natsl_seq_row* seqs, int n_seqs, int total_units, natsl_stream_t stream) {
+                      int dtype, const natsl_seq_row* seqs, int n_seqs, int total_units, natsl_stream_t stream, const BesideScan* beside) {
   const char* what = delta ? "natsl_gdn_chunk_fwd" : "natsl_mamba_chunk_fwd";
   if (!q || !k || !v || !g || !o || !types || (delta && !beta)) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
   if (dtype != NATSL_BF16) return fail(NATSL_ERR_UNSUPPORTED, "%s: only bf16 tensors are supported (got dtype %d)", what, dtype);
@@ -1135,13 +1140,13 @@ static int linear_fwd(bool delta, const void* q, const void* k, const void* v, c
   p.ws_sc = reinterpret_cast<float*>(p.ws_p + units * (C * C));
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (delta) {
-    if (K == 128) return launch_linear<128, true>(p, s, what);
-    if (K == 64) return launch_linear<64, true>(p, s, what);
-    if (K == 192) return launch_linear<192, true>(p, s, what);
+    if (K == 128) return launch_linear<128, true>(p, s, beside, what);
+    if (K == 64) return launch_linear<64, true>(p, s, beside, what);
+    if (K == 192) return launch_linear<192, true>(p, s, beside, what);
   } else {
-    if (K == 128) return launch_linear<128, false>(p, s, what);
-    if (K == 64) return launch_linear<64, false>(p, s, what);
-    if (K == 192) return launch_linear<192, false>(p, s, what);
+    if (K == 128) return launch_linear<128, false>(p, s, beside, what);
+    if (K == 64) return launch_linear<64, false>(p, s, beside, what);
+    if (K == 192) return launch_linear<192, false>(p, s, beside, what);
   }
   return fail(NATSL_ERR_UNSUPPORTED, "%s: key dim K=%d not built (supported: 64, 128, 192)", what, K);
 }
@@ -1162,7 +1167,7 @@ extern "C" int natsl_gdn_chunk_fwd(const void* q, const void* k, const void* v, 
                                    size_t workspace_bytes, int dtype, const natsl_seq_row* seqs, int n_seqs, int total_units,
                                    natsl_stream_t stream) {
   return linear_fwd(true, q, k, v, g, beta, h0, o, ht, h_block_start, g_block_sum, chunk_states, chunk_v_new, types, types_dtype, B, T, H, HN, K, V, TN, block, scale, flags,
-                    workspace, workspace_bytes, dtype, seqs, n_seqs, total_units, stream);
+                    workspace, workspace_bytes, dtype, seqs, n_seqs, total_units, stream, nullptr);
 }
 
 extern "C" int natsl_mamba_chunk_fwd(const void* q, const void* k, const void* v, const float* g, const float* h0, void* o,
@@ -1171,5 +1176,5 @@ extern "C" int natsl_mamba_chunk_fwd(const void* q, const void* k, const void* v
                                      int dtype, const natsl_seq_row* seqs, int n_seqs, int total_units,
                                      natsl_stream_t stream) {
   return linear_fwd(false, q, k, v, g, nullptr, h0, o, ht, h_block_start, g_block_sum, chunk_states, nullptr, types, types_dtype, B, T, H, HN, K, V, TN, block, scale,
-                    flags & ~NATSL_QK_L2NORM, workspace, workspace_bytes, dtype, seqs, n_seqs, total_units, stream);
+                    flags & ~NATSL_QK_L2NORM, workspace, workspace_bytes, dtype, seqs, n_seqs, total_units, stream, nullptr);
 }

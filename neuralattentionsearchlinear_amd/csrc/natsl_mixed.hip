@@ -99,23 +99,25 @@ extern "C" int natsl_mixed_fwd(const natsl_mixed* m, int phases, natsl_stream_t 
                      nullptr, nullptr, m->seqs, m->n_seqs, 0, attn_stream);
     if (rc != NATSL_OK) return rc;
   }
-  if (phases & NATSL_MIXED_SOFTMAX) {
-    rc = natsl_softmax_sparse_fwd(m->q_attn, m->k_attn, m->v_attn, m->o_attn, m->lse, m->types_attn, m->types_dtype, m->block_indices,
-                                  m->n_blocks, m->B, m->T_attn, m->HQ, m->HKV, m->HN, m->KA, m->VA, m->TN_attn, m->block, m->scale_attn,
-                                  m->same_block_visible, NATSL_BF16, m->seqs, m->n_seqs, m->total_qtiles, attn_stream);
-    if (rc != NATSL_OK) return rc;
-  }
+  auto softmax = [&]() {
+    return natsl_softmax_sparse_fwd(m->q_attn, m->k_attn, m->v_attn, m->o_attn, m->lse, m->types_attn, m->types_dtype, m->block_indices,
+                                    m->n_blocks, m->B, m->T_attn, m->HQ, m->HKV, m->HN, m->KA, m->VA, m->TN_attn, m->block, m->scale_attn,
+                                    m->same_block_visible, NATSL_BF16, m->seqs, m->n_seqs, m->total_qtiles, attn_stream);
+  };
+  // Side by side, the scan comes first and the softmax kernel right behind the prep kernel: its workgroups take a CU each for as long
+  // as there are tiles, so it has to find the scan's in place and fill the CUs they leave (the other way round the scan waits
+  // for it).
+  const bool both = fork && (phases & NATSL_MIXED_SOFTMAX) && (phases & NATSL_MIXED_LINEAR);
+  if ((phases & NATSL_MIXED_SOFTMAX) && !both && (rc = softmax()) != NATSL_OK) return rc;
   if (phases & NATSL_MIXED_LINEAR) {
-    if (m->is_delta)
-      rc = natsl_gdn_chunk_fwd(m->q, m->k, m->v, m->g, m->beta, m->h0, m->o, m->ht, m->h_block_start, m->g_block_sum, m->chunk_states,
-                               m->chunk_v_new, m->types, m->types_dtype, m->B, m->T, m->H, m->HN, m->K, m->V, m->TN, m->block, m->scale_linear,
-                               m->flags, m->workspace, m->workspace_bytes, NATSL_BF16, m->seqs, m->n_seqs, m->total_chunks, stream);
-    else
-      rc = natsl_mamba_chunk_fwd(m->q, m->k, m->v, m->g, m->h0, m->o, m->ht, m->h_block_start, m->g_block_sum, m->chunk_states, m->types,
-                                 m->types_dtype, m->B, m->T, m->H, m->HN, m->K, m->V, m->TN, m->block, m->scale_linear, m->flags, m->workspace,
-                                 m->workspace_bytes, NATSL_BF16, m->seqs, m->n_seqs, m->total_chunks, stream);
+    const BesideScan beside{order_streams, side};
+    rc = linear_fwd(m->is_delta != 0, m->q, m->k, m->v, m->g, m->is_delta ? m->beta : nullptr, m->h0, m->o, m->ht, m->h_block_start, m->g_block_sum,
+                    m->chunk_states, m->is_delta ? m->chunk_v_new : nullptr, m->types, m->types_dtype, m->B, m->T, m->H, m->HN, m->K, m->V, m->TN,
+                    m->block, m->scale_linear, m->is_delta ? m->flags : m->flags & ~NATSL_QK_L2NORM, m->workspace, m->workspace_bytes, NATSL_BF16,
+                    m->seqs, m->n_seqs, m->total_chunks, stream, both ? &beside : nullptr);
     if (rc != NATSL_OK) return rc;
   }
+  if (both && (rc = softmax()) != NATSL_OK) return rc;
   if (phases & NATSL_MIXED_JOIN) {
     if (fork && (rc = order_streams(side, s, what)) != NATSL_OK) return rc;
     rc = cast_all<false>(m->cast_out, m->n_cast_out, s, what);

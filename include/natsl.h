@@ -137,8 +137,7 @@ int natsl_softmax_fwd_variant(int B, int T, int HQ, int HKV, int block, int pack
  * with respect to a bias on that block's scores as later blocks see them; blocks not typed attention keep 0 unless
  * flags bit 1 is set (the reference's compute_dnats_for_invalid_blocks_attn, attns.py:1318-1325): then they get
  * sum min(exp2(s - lse), 1) (dP - delta) over the same (keys) x (later queries), what their keys would contribute if
- * they were visible.  flags bit 0: same_block_visible, as in the forward; bits 2, 3, 4: add to what is in dq, dk, dv
- * (rounded to bf16 twice, as an elementwise addition of the two gradients would) instead of overwriting it.  The caller sums dnats over the query heads
+ * they were visible.  flags bit 0: same_block_visible, as in the forward.  The caller sums dnats over the query heads
  * of a selector head.  o, lse are the forward's outputs, d_o the gradient of o.  workspace: natsl_softmax_bwd_workspace_bytes()
  * bytes (delta = rowsum(d_o * o), then the work-queue counters of the dk/dv kernel; nothing to initialise: every call resets
  * them, so calls that share a workspace must not overlap).  T * HQ * max(K, V) * 2 must stay below 2^32 (32-bit row offsets
@@ -216,6 +215,18 @@ int natsl_linear_chunk_bwd(int delta_rule, const void* q, const void* k, const v
                            void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0, float* d_gate, float* d_rollback, int B, int T,
                            int H, int HN, int K, int V, int TN, int block, float scale, int flags, int dtype,
                            const natsl_seq_row* seqs, int n_seqs, int total_chunks, natsl_stream_t stream);
+
+/* natsl_linear_chunk_bwd in its two steps, so that something can run next to the scan or be ready before the second step: steps 1 = the
+ * reverse scan (dv, d_chunk_states, dbeta_parts, dh0), 2 = the per-chunk gradients (dq, dk, dg, dbeta, d_gate, d_rollback), 3 = both; + 4: another
+ * kernel shares the chip with the scan (wider workgroups on fewer CUs).
+ * add (second step): 1, 2 = dq, dk are added to what is there; dv_sum, when given, [B*T][H][V]: dv is added to what is there.  (A tensor
+ * that another operator takes as well has one gradient; the sum is rounded as an elementwise bf16 addition would.) */
+int natsl_linear_chunk_bwd_steps(int steps, int add, void* dv_sum, int delta_rule, const void* q, const void* k, const void* v_new, const float* g,
+                                 const void* beta, const void* d_o, const float* dht, const void* chunk_states, const void* types,
+                                 int types_dtype, const float* g_block_sums, const void* workspace, void* d_chunk_states, float* dbeta_parts,
+                                 void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0, float* d_gate, float* d_rollback, int B, int T,
+                                 int H, int HN, int K, int V, int TN, int block, float scale, int flags, int dtype,
+                                 const natsl_seq_row* seqs, int n_seqs, int total_chunks, natsl_stream_t stream);
 
 /* What is per selector block around natsl_linear_chunk_bwd.  natsl_linear_block_sums fills its g_block_sums from the forward's
  * workspace.  natsl_block_grads, after it: d_types [B,TN,HN,2] (f32 or bf16) = the selector's straight-through gradients --

@@ -76,6 +76,8 @@ _SIGNATURES = {
     "natsl_decode_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
     "natsl_decode_fwd": (c_int, [c_int] + [c_void_p] * 5 + [c_int] * 8 + [c_float, c_int64, c_int64, c_void_p, c_size_t] + [c_void_p] * 11 +
                                 [c_int, c_void_p] + [c_int] * 6 + [c_float, c_int, c_void_p]),
+    "natsl_linear_chunk_bwd_steps": (c_int, [c_int, c_int, c_void_p, c_int] + [c_void_p] * 9 + [c_int] + [c_void_p] * 12 + [c_int] * 8 +
+                                     [c_float, c_int, c_int, c_void_p, c_int, c_int, c_void_p]),
     "natsl_linear_block_sums": (c_int, [c_void_p] * 2 + [c_int] * 5 + [c_void_p, c_int, c_int, c_void_p]),
     "natsl_block_grads": (c_int, [c_void_p, c_int] + [c_void_p] * 3 + [c_int, c_void_p, c_void_p] + [c_int] * 8 + [c_void_p, c_int, c_void_p]),
     "natsl_kv_collect": (c_int, [c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_longlong, c_void_p] + [c_int] * 12 + [c_void_p]),

@@ -120,7 +120,7 @@ def hip_backward_is_built(K: int, V: int) -> bool:
 
 
 def linear_chunk_backward(kind, q, k, v, g, beta, h0, types, scale, block, decay, l2norm, intra, do, dht,
-                          dnats_for_invalid_blocks, seqs=None, saved=None, later=None):
+                          dnats_for_invalid_blocks, seqs=None, saved=None, later=None, meanwhile=None, beside=0, onto=(None, None, None)):
     """Gradients of the chunked linear branch: -> (dq, dk, dv, dg fp32, dbeta or None, dh0 or None, dnats fp32 [B,NB,HN]).
     types [B,NB,HN,2]; do [B,T,H,V]; dht [N,H,K,V] or None; seqs: packed sequences (B = 1) or None; saved: what
     linear_chunk_fwd(..., chunk_states=True) returned after (o, final_state) on these same inputs, if the caller kept it.  The
@@ -129,6 +129,9 @@ def linear_chunk_backward(kind, q, k, v, g, beta, h0, types, scale, block, decay
 
     later (a list): where the kernels run on the tensors as they are, dg and dnats are left unfinished, dnats comes back as None and the list
     receives a function that ends them, given the softmax branch's dnats [B,NB,HQ] fp32 -> the gradient of types [B,NB,HN,2].
+    In that case, too: onto: gradients (bf16, like q, k, v) that dq, dk, dv are added to in place and that come back as them; and
+    meanwhile is called once, behind the reverse scan if anything is added (when it returns, this stream has what is added to),
+    else behind everything; beside: 4 if it puts a kernel next to the scan, else 0.
 
     dnats_for_invalid_blocks with block > 64 raises NotImplementedError: for a block of several chunks that is not typed
     linear the reference sums a virtual key gradient v . dh over EVERY chunk of the block
@@ -142,7 +145,7 @@ def linear_chunk_backward(kind, q, k, v, g, beta, h0, types, scale, block, decay
     K, V = q.shape[-1], v.shape[-1]
     if hip_backward_is_built(K, V):
         return linear_chunk_backward_hip(kind, q, k, v, g, beta, h0, types, scale, block, decay, l2norm, intra, do, dht,
-                                         dnats_for_invalid_blocks, seqs, saved, later)
+                                         dnats_for_invalid_blocks, seqs, saved, later, meanwhile, beside, onto)
     if hip_backward_is_built(K, 64) and V % 16 == 0:
         # Value widths the kernels are not built for (16..48, 96, ..): zero columns up to the next multiple of 64.  The state's
         # columns never mix, a zero column of v and dO stays zero through the whole recurrence and adds nothing to any sum
@@ -169,10 +172,10 @@ def linear_chunk_backward(kind, q, k, v, g, beta, h0, types, scale, block, decay
 
 
 def linear_chunk_backward_hip(kind, q, k, v, g, beta, h0, types, scale, block, decay, l2norm, intra, do, dht,
-                              dnats_for_invalid_blocks, seqs=None, saved=None, later=None):
+                              dnats_for_invalid_blocks, seqs=None, saved=None, later=None, meanwhile=None, beside=0, onto=(None, None, None)):
     """The backward as kernels: the forward once more (storing every chunk's entering state and v_new) unless the caller kept
     those from its own forward (`saved`), then the reverse scan and the per-chunk gradients (csrc/natsl_linear_bwd.hip).  later: a list that receives
-    the call that ends the work (see linear_chunk_backward)."""
+    the call that ends the work; meanwhile, beside, onto: see linear_chunk_backward."""
     from . import _capi
     from ._mixed_common import linear_chunk_fwd
     from .nats_util import _seq_args
@@ -202,7 +205,12 @@ def linear_chunk_backward_hip(kind, q, k, v, g, beta, h0, types, scale, block, d
         gsum = torch.empty(B * NB, H, dtype=f32, device=dev)
         _capi.check(L.natsl_linear_block_sums(P(ws), P(gsum), B, T, H, NB, block, sp, ns, tot, stream), "natsl_linear_block_sums")
         d_states = torch.empty_like(states)
-        dq, dk, dv = torch.empty_like(qb), torch.empty_like(kb), torch.empty_like(vb)
+        dq, dk = (torch.empty_like(t) if have is None else have for t, have in zip((qb, kb), onto))
+        dv, dv_sum = torch.empty_like(vb), onto[2]
+        for t, have in zip((qb, kb, vb), onto):
+            if have is not None and (have.shape != t.shape or have.dtype != bf16 or not have.is_contiguous()):
+                raise ValueError("a gradient to add to must be like its tensor")
+        add = (onto[0] is not None) + 2 * (onto[1] is not None)
         dg = torch.empty(B, T, H, dtype=f32, device=dev)
         dbeta = torch.empty(B, T, H, dtype=f32, device=dev) if delta else None
         dbeta_parts = torch.empty(B, T, H, V // 16, dtype=f32, device=dev) if delta else None
@@ -211,11 +219,22 @@ def linear_chunk_backward_hip(kind, q, k, v, g, beta, h0, types, scale, block, d
         rb = torch.empty(NTtot, H, dtype=f32, device=dev)
         dof = do.detach().to(bf16).contiguous()
         dhtf = None if dht is None else dht.detach().to(f32).contiguous()
-        rc = L.natsl_linear_chunk_bwd(
-            1 if delta else 0, P(qb), P(kb), P(v_new), P(gf), P(bb), P(dof), P(dhtf), P(states), P(ty), _capi.dtype_code(ty.dtype),
-            P(gsum), P(ws), P(d_states), P(dbeta_parts), P(dq), P(dk), P(dv), P(dg), P(dbeta), P(dh0), P(gate), P(rb),
-            B, T, H, HN, K, V, NB, block, float(scale), flags, _capi.dtype_code(bf16), sp, ns, tot, stream)
-        _capi.check(rc, "natsl_linear_chunk_bwd")
+        def steps(which):
+            rc = L.natsl_linear_chunk_bwd_steps(
+                which, add, P(dv_sum), 1 if delta else 0, P(qb), P(kb), P(v_new), P(gf), P(bb), P(dof), P(dhtf), P(states), P(ty),
+                _capi.dtype_code(ty.dtype), P(gsum), P(ws), P(d_states), P(dbeta_parts), P(dq), P(dk), P(dv), P(dg), P(dbeta), P(dh0), P(gate), P(rb),
+                B, T, H, HN, K, V, NB, block, float(scale), flags, _capi.dtype_code(bf16), sp, ns, tot, stream)
+            _capi.check(rc, "natsl_linear_chunk_bwd_steps")
+        if meanwhile is not None and (add or dv_sum is not None):
+            steps(1 + beside)
+            meanwhile()
+            steps(2)
+        else:
+            steps(3 + beside)
+            if meanwhile is not None:
+                meanwhile()
+        if dv_sum is not None:
+            dv = dv_sum
 
     def finish(dnats_attn=None):
         d_types = torch.empty(B, NB, HN, 2, dtype=f32 if dnats_attn is None else ty.dtype, device=dev)

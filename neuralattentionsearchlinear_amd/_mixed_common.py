@@ -377,7 +377,7 @@ class _MixedFunction(torch.autograd.Function):
         ctx.in_dtypes = tuple(None if t is None else t.dtype for t in (q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
                                                                        initial_state, g, beta, nats_block_types))
         ctx.has_h0 = initial_state is not None
-        # a tensor given to both branches gets one gradient, added up by the softmax branch's kernels (bf16: the same sum, rounded the
+        # a tensor given to both branches gets one gradient, added up by the linear branch's last kernel (bf16: the same sum, rounded the
         # same way, as autograd's)
         ctx.shared = tuple(a is l and a.dtype == torch.bfloat16 for a, l in ((q_attn, q_lattn), (k_attn, k_lattn), (v_attn, v_lattn)))
         saved = [aux[n] for n in ('q_attn', 'k_attn', 'v_attn', 'q_lattn', 'k_lattn', 'v_lattn', 'g', 'types', 'lse',
@@ -396,7 +396,7 @@ class _MixedFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, do_lin, do_attn, dht):
-        from ._linear_bwd import linear_chunk_backward
+        from ._linear_bwd import hip_backward_is_built, linear_chunk_backward
         from .attns import prepare_attn_nats_bwd
         cfg = ctx.cfg
         (q_a, k_a, v_a, q_l, k_l, v_l, g, types, lse, idx, nblk, o_attn, beta, h0) = ctx.saved_tensors[:14]
@@ -409,37 +409,41 @@ class _MixedFunction(torch.autograd.Function):
             do_lin = torch.zeros(*q_l.shape[:3], v_l.shape[-1], dtype=torch.float32, device=q_l.device)
         if do_attn is not None:
             do_attn = do_attn.to(torch.bfloat16).contiguous()
-        prepare = lambda *onto: prepare_attn_nats_bwd(q_a, k_a, v_a, o_attn, types, idx, nblk, None, lse, do_attn, cfg['scale_attn'], cfg['block'], 0,
-                                                      cfg['attn_same_block'], cfg['dnats_invalid_attn'], None, None, None, True, seqs, *onto)
-        # side by side: the softmax branch's tensors are made first, on this stream, and live until this stream has waited for the
-        # other one (nothing that is allocated in between can share their memory)
-        side = attn = None
-        if do_attn is not None and not any(ctx.shared):
+        # The softmax branch's tensors are made first, on this stream, and live until this stream has its kernels behind it (nothing
+        # that is allocated in between can share their memory).  Side by side, the reverse scan is enqueued first (see natsl_mixed_fwd) and
+        # the per-chunk kernel, which adds the branches' gradients of a tensor they share, behind both.
+        attn = side = None
+        if do_attn is not None:
+            attn = prepare_attn_nats_bwd(q_a, k_a, v_a, o_attn, types, idx, nblk, None, lse, do_attn, cfg['scale_attn'], cfg['block'], 0,
+                                         cfg['attn_same_block'], cfg['dnats_invalid_attn'], None, None, None, True, seqs)
+            here = torch.cuda.current_stream(q_l.device)
             if _run_side_by_side(q_l.shape[1] * B // (B if seqs is None else seqs.n_seqs), q_l.shape[-1]):
                 side = _get_attn_stream(q_l.device)
-            if side is not None:
-                here = torch.cuda.current_stream(q_l.device)
-                attn = prepare()
                 side.wait_stream(here)
+            else:
+                attn[0](here.cuda_stream)
+
+        def softmax_beside():
+            nonlocal side
+            if side is not None:
+                beside, side = side, None
+                try:
+                    attn[0](beside.cuda_stream)
+                finally:
+                    here.wait_stream(beside)
+        onto = (None, None, None)
+        if attn is not None and hip_backward_is_built(q_l.shape[-1], v_l.shape[-1]):
+            onto = tuple(t if both else None for t, both in zip(attn[1], ctx.shared))
         lin_args = (cfg['scale_lattn'], cfg['block'], cfg['decay_non_linear'], cfg['qk_l2norm'], cfg['lin_intra'])
         later = []
-        try:
-            dq_l, dk_l, dv_l, dg, dbeta, dh0, dn_lin = linear_chunk_backward(
-                cfg['kind'], q_l, k_l, v_l, g, beta, h0, types, *lin_args, do_lin, dht, cfg['dnats_invalid_linear'], seqs,
-                saved=linear_saved, later=later)
-            if side is not None:
-                attn[0](side.cuda_stream)
-        finally:
-            if side is not None:
-                here.wait_stream(side)
+        dq_l, dk_l, dv_l, dg, dbeta, dh0, dn_lin = linear_chunk_backward(
+            cfg['kind'], q_l, k_l, v_l, g, beta, h0, types, *lin_args, do_lin, dht, cfg['dnats_invalid_linear'], seqs,
+            saved=linear_saved, later=later, meanwhile=softmax_beside, beside=0 if side is None else 4, onto=onto)
+        softmax_beside()                                   # (where the linear branch did not call it)
         lin = [dq_l, dk_l, dv_l]
-        if do_attn is not None:
-            if side is None:
-                onto = tuple(t if both and t.dtype == torch.bfloat16 and t.is_contiguous() else None for t, both in zip(lin, ctx.shared))
-                lin = [None if have is not None else t for t, have in zip(lin, onto)]
-                attn = prepare(onto)
-                attn[0](_capi.stream_ptr(q_l.device))
+        if attn is not None:
             dq_a, dk_a, dv_a, dn_attn = attn[1]
+            lin = [None if have is not None else t for t, have in zip(lin, onto)]
             if not later:
                 dn_attn = dn_attn.view(B, NB, HN, -1).sum(-1)
         else:

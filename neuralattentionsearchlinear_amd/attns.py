@@ -72,10 +72,10 @@ def parallel_attn_nats_bwd(
 
 def prepare_attn_nats_bwd(q, k, v, o, nats_block_types, nats_block_indices, n_nats_blocks, g_cumsum, lse, do, scale, NAtS_block_size, OFFSET_ATTN,
                           compute_incomplete_chunk_scores, compute_dnats_for_invalid_blocks_attn, sliding_window_size, cu_seqlens, cu_seqlens_nats,
-                          is_causal, seqs, onto=(None, None, None)):
+                          is_causal, seqs):
     """parallel_attn_nats_bwd up to its kernels: everything is allocated and converted on the current stream -> (launch, (dq, dk, dv, dnats
     per query head)); launch(stream) enqueues the kernels.  launch holds what they use: keep it until the current stream waits for
-    `stream`.  onto: gradients (contiguous bf16) that dq, dk, dv are added to in place."""
+    `stream`."""
     if g_cumsum is not None or sliding_window_size is not None or not is_causal or OFFSET_ATTN != 0:
         raise NotImplementedError("only the causal backward without g_cumsum / sliding window is built")
     if seqs is None and cu_seqlens is not None:
@@ -91,11 +91,7 @@ def prepare_attn_nats_bwd(q, k, v, o, nats_block_types, nats_block_indices, n_na
     B, T, HQ, K = q.shape
     H, V = k.shape[2], v.shape[-1]
     TN, HN = ty.shape[1], ty.shape[2]
-    dq, dk, dv = (torch.empty_like(t) if have is None else have for t, have in zip((q, k, v), onto))
-    for t, have in zip((q, k, v), onto):
-        if have is not None and (have.shape != t.shape or have.dtype != t.dtype or not have.is_contiguous()):
-            raise ValueError("a gradient to add to must be like its tensor")
-    add = sum(4 << i for i, have in enumerate(onto) if have is not None)
+    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     dnats = torch.zeros(B, TN, HQ, dtype=torch.float32, device=q.device)
     L = _capi.lib()
     sp, ns, tot = _seq_args(seqs, seqs.total_qtiles if seqs is not None else 0)
@@ -108,7 +104,7 @@ def prepare_attn_nats_bwd(q, k, v, o, nats_block_types, nats_block_indices, n_na
             _capi.ptr(q), _capi.ptr(k), _capi.ptr(v), _capi.ptr(o), _capi.ptr(lse), _capi.ptr(do), _capi.ptr(dq), _capi.ptr(dk), _capi.ptr(dv),
             _capi.ptr(dnats), _capi.ptr(ty), _capi.dtype_code(ty.dtype), _capi.ptr(idx), _capi.ptr(nblk), B, T, HQ, H, HN, K, V, TN,
             NAtS_block_size, float(scale),
-            int(bool(compute_incomplete_chunk_scores)) | (2 if compute_dnats_for_invalid_blocks_attn else 0) | add, _capi.dtype_code(q.dtype),
+            int(bool(compute_incomplete_chunk_scores)) | (2 if compute_dnats_for_invalid_blocks_attn else 0), _capi.dtype_code(q.dtype),
             _capi.ptr(ws), ws_bytes, sp, ns, tot, seqs.total_chunks if seqs is not None else 0, stream)
         _capi.check(rc, "natsl_softmax_sparse_bwd")
     return launch, (dq, dk, dv, dnats)

@@ -70,6 +70,8 @@ struct LinBwdParams {
   int B, T, H, HN, V, TN, block, nt;
   float scale;
   int flags;
+  int add;                // 1, 2: the per-chunk kernel adds dq, dk to what is there
+  bf16_t* dv_sum;         // ... and dX to this, or null
 };
 
 constexpr int CB = 64;          // tokens per chunk
@@ -87,6 +89,15 @@ NATSL_DEVICE void unpack8f(const u32x4 w, float* f) {
     f[2 * j] = __uint_as_float(w[j] << 16);
     f[2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
   }
+}
+
+// Sums of eight bf16 pairs, rounded: what an elementwise bf16 addition of two gradients gives.
+NATSL_DEVICE u32x4 add8_bf16(const u32x4 a, const u32x4 b) {
+  u32x4 w;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    w[j] = pack_bf16x2(__uint_as_float(a[j] << 16) + __uint_as_float(b[j] << 16), __uint_as_float(a[j] & 0xffff0000u) + __uint_as_float(b[j] & 0xffff0000u));
+  return w;
 }
 
 // two 8-byte halves -> one operand: slots 0..3 from lo, 4..7 from hi
@@ -1101,13 +1112,37 @@ __global__ __launch_bounds__(256, DK <= 128 ? 2 : 1) void linear_bwd_chunk_kerne
       p.rb[unit] = want_rb ? __expf(p.gsum_blk[((size_t)blk0 + blk) * p.H + h]) * (red[4] + red[5] + red[6] + red[7]) : 0.f;
     }
   }
+  // dX joins another gradient of the same tensor; what dq, dk are added to, where they are, is fetched before the barrier
+  if (p.dv_sum) {
+#pragma unroll 2
+    for (int i = tid; i < CB * (p.V / 8); i += 256) {
+      const int row = i / (p.V / 8), seg = i % (p.V / 8);
+      if (row < nvalid) {
+        const size_t at = ((row0 + row) * p.H + h) * p.V + seg * 8;
+        *reinterpret_cast<u32x4*>(p.dv_sum + at) = add8_bf16(*reinterpret_cast<const u32x4*>(p.dv + at), *reinterpret_cast<const u32x4*>(p.dv_sum + at));
+      }
+    }
+  }
+  constexpr int NO = CB * (DK / 8) / 256;
+  u32x4 have_q[NO], have_k[NO];
+  auto out_at = [&](const int i) { const int pc = tid + 256 * i; return ((row0 + min(pc / (DK / 8), nvalid - 1)) * p.H + h) * DK + pc % (DK / 8) * 8; };
+  if (p.add) {
+#pragma unroll
+    for (int i = 0; i < NO; ++i) {
+      have_q[i] = *reinterpret_cast<const u32x4*>(p.dq + out_at(i));
+      have_k[i] = *reinterpret_cast<const u32x4*>(p.dk + out_at(i));
+    }
+  }
   __syncthreads();
-  for (int pc = tid; pc < CB * (DK / 8); pc += 256) {
-    const int row = pc / (DK / 8), seg = pc % (DK / 8);
+#pragma unroll
+  for (int i = 0; i < NO; ++i) {
+    const int pc = tid + 256 * i, row = pc / (DK / 8), seg = pc % (DK / 8);
+    u32x4 wq = *reinterpret_cast<const u32x4*>(Qn + row * KP + seg * 8), wk = *reinterpret_cast<const u32x4*>(Kn + row * KP + seg * 8);
+    if (p.add & 1) wq = add8_bf16(have_q[i], wq);
+    if (p.add & 2) wk = add8_bf16(have_k[i], wk);
     if (row < nvalid) {
-      const size_t off = ((row0 + row) * p.H + h) * DK + seg * 8;
-      *reinterpret_cast<u32x4*>(p.dq + off) = *reinterpret_cast<const u32x4*>(Qn + row * KP + seg * 8);
-      *reinterpret_cast<u32x4*>(p.dk + off) = *reinterpret_cast<const u32x4*>(Kn + row * KP + seg * 8);
+      *reinterpret_cast<u32x4*>(p.dq + out_at(i)) = wq;
+      *reinterpret_cast<u32x4*>(p.dk + out_at(i)) = wk;
     }
   }
 }
@@ -1231,17 +1266,18 @@ static int launch_bwd_scan(const LinBwdParams& p, hipStream_t stream, const char
 }
 
 template <int DK, bool DELTA>
-static int launch_bwd(const LinBwdParams& p, hipStream_t stream, const char* what) {
-  {
+static int launch_bwd(const LinBwdParams& p, const int steps, hipStream_t stream, const char* what) {
+  if (steps & 1) {
     // one workgroup per CU at most (LDS): 32-column workgroups (two compute waves) when the 64-column ones would leave
-    // half of the CUs without work
+    // half of the CUs without work, or, with another kernel waiting for the CUs the scan leaves, three quarters of them
+    const int spare = steps & 4 ? 4 : 2;
     const long long wgs64 = (long long)(p.seqs ? p.n_seqs : p.B) * p.H * (p.V / 64);
     int rc;
-    if constexpr (DK <= 128) rc = 2 * wgs64 <= bwd_cu_count() ? launch_bwd_scan<DK, DELTA, 2>(p, stream, what) : launch_bwd_scan<DK, DELTA, 4>(p, stream, what);
+    if constexpr (DK <= 128) rc = spare * wgs64 <= bwd_cu_count() ? launch_bwd_scan<DK, DELTA, 2>(p, stream, what) : launch_bwd_scan<DK, DELTA, 4>(p, stream, what);
     else rc = launch_bwd_scan<DK, DELTA, 4>(p, stream, what);
     if (rc != NATSL_OK) return rc;
   }
-  {
+  if (steps & 2) {
     using L = BwdChunkLds<DK>;
     auto kern = linear_bwd_chunk_kernel<DK, DELTA>;
     static std::atomic<unsigned long long> reserved{0};
@@ -1249,13 +1285,14 @@ static int launch_bwd(const LinBwdParams& p, hipStream_t stream, const char* wha
     hipLaunchKernelGGL(kern, dim3((unsigned)(p.total_chunks * p.H)), dim3(256), L::TOTAL, stream, p);
     return check_launch(what);
   }
+  return NATSL_OK;
 }
 
 }  // namespace natsl
 
 using namespace natsl;
 
-extern "C" int natsl_linear_chunk_bwd(int delta_rule, const void* q, const void* k, const void* v_new, const float* g, const void* beta,
+extern "C" int natsl_linear_chunk_bwd_steps(int steps, int add, void* dv_sum, int delta_rule, const void* q, const void* k, const void* v_new, const float* g, const void* beta,
                                       const void* d_o, const float* dht, const void* chunk_states, const void* types, int types_dtype,
                                       const float* g_block_sums, const void* workspace, void* d_chunk_states, float* dbeta_parts,
                                       void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0, float* d_gate, float* d_rollback, int B, int T,
@@ -1286,19 +1323,28 @@ extern "C" int natsl_linear_chunk_bwd(int delta_rule, const void* q, const void*
   p.dq = (bf16_t*)dq; p.dk = (bf16_t*)dk; p.dg = dg; p.dbeta = dbeta; p.dbeta_parts = dbeta_parts; p.gate = d_gate; p.rb = d_rollback;
   p.B = B; p.T = T; p.H = H; p.HN = HN; p.V = V; p.TN = TN; p.block = block; p.nt = cdiv(T, CB);
   p.seqs = reinterpret_cast<const SeqRow*>(seqs); p.n_seqs = seqs ? n_seqs : 0; p.total_chunks = seqs ? total_chunks : B * p.nt;
-  p.scale = scale; p.flags = flags;
+  p.scale = scale; p.flags = flags; p.add = add; p.dv_sum = (bf16_t*)dv_sum;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (delta_rule) {
-    if (K == 128) return launch_bwd<128, true>(p, s, what);
-    if (K == 64) return launch_bwd<64, true>(p, s, what);
-    if (K == 192) return launch_bwd<192, true>(p, s, what);
+    if (K == 128) return launch_bwd<128, true>(p, steps, s, what);
+    if (K == 64) return launch_bwd<64, true>(p, steps, s, what);
+    if (K == 192) return launch_bwd<192, true>(p, steps, s, what);
   } else {
     p.flags &= ~NATSL_QK_L2NORM;
-    if (K == 128) return launch_bwd<128, false>(p, s, what);
-    if (K == 64) return launch_bwd<64, false>(p, s, what);
-    if (K == 192) return launch_bwd<192, false>(p, s, what);
+    if (K == 128) return launch_bwd<128, false>(p, steps, s, what);
+    if (K == 64) return launch_bwd<64, false>(p, steps, s, what);
+    if (K == 192) return launch_bwd<192, false>(p, steps, s, what);
   }
   return fail(NATSL_ERR_UNSUPPORTED, "%s: key dim K=%d not built (supported: 64, 128, 192)", what, K);
+}
+
+extern "C" int natsl_linear_chunk_bwd(int delta_rule, const void* q, const void* k, const void* v_new, const float* g, const void* beta,
+                                      const void* d_o, const float* dht, const void* chunk_states, const void* types, int types_dtype,
+                                      const float* g_block_sums, const void* workspace, void* d_chunk_states, float* dbeta_parts,
+                                      void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0, float* d_gate, float* d_rollback, int B, int T,
+                                      int H, int HN, int K, int V, int TN, int block, float scale, int flags, int dtype,
+                                      const natsl_seq_row* seqs, int n_seqs, int total_chunks, natsl_stream_t stream) {
+  return natsl_linear_chunk_bwd_steps(3, 0, nullptr, delta_rule, q, k, v_new, g, beta, d_o, dht, chunk_states, types, types_dtype, g_block_sums, workspace, d_chunk_states, dbeta_parts, dq, dk, dv, dg, dbeta, dh0, d_gate, d_rollback, B, T, H, HN, K, V, TN, block, scale, flags, dtype, seqs, n_seqs, total_chunks, stream);
 }
 
 static int block_params(BlockParams& p, int B, int T, int H, int HN, int TN, int block, const natsl_seq_row* seqs, int n_seqs, const char* what) {

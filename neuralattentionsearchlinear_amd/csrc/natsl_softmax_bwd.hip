@@ -38,7 +38,6 @@ struct SoftmaxBwdParams {
   float scale, scale_log2;
   int same_block;
   int dnats_invalid;   // also give dnats to blocks that are not typed attention (what their keys would contribute, reference attns.py:1318-1325)
-  int add;                // 1, 2, 4: dq, dk, dv are added to what is there (a gradient that meets this one at the same tensor)
 };
 
 NATSL_DEVICE bool bwd_type_is_one(const void* types, int dtype, size_t i) {
@@ -99,15 +98,6 @@ NATSL_DEVICE bf16x8 pack8(const f32x16& x, const int ss) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) w[j] = pack_bf16x2(x[8 * ss + 2 * j], x[8 * ss + 2 * j + 1]);
   return __builtin_bit_cast(bf16x8, w);
-}
-
-// Sums of eight bf16 pairs, rounded: what an elementwise bf16 addition of two gradients gives.
-NATSL_DEVICE u32x4 add8_bf16(const u32x4 a, const u32x4 b) {
-  u32x4 w;
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    w[j] = pack_bf16x2(__uint_as_float(a[j] << 16) + __uint_as_float(b[j] << 16), __uint_as_float(a[j] & 0xffff0000u) + __uint_as_float(b[j] & 0xffff0000u));
-  return w;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -396,10 +386,8 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
     const int row = pass * RPP + lane / SEGS, seg = lane % SEGS;
     const int t = q0 + row;
     if (t < len) {
-      u32x4 w = *reinterpret_cast<const u32x4*>(Os + row * KP + seg * 8);
-      u32x4* at = reinterpret_cast<u32x4*>(p.dq + ((size_t)(bos + t) * p.HQ + hq) * DK + seg * 8);
-      if (p.add & 1) w = add8_bf16(*at, w);
-      *at = w;
+      const u32x4 w = *reinterpret_cast<const u32x4*>(Os + row * KP + seg * 8);
+      *reinterpret_cast<u32x4*>(p.dq + ((size_t)(bos + t) * p.HQ + hq) * DK + seg * 8) = w;
     }
   }
 }
@@ -803,16 +791,6 @@ NATSL_DEVICE void dkdv_role(const SoftmaxBwdParams& p, unsigned char* smem, Dkdv
       }
       const int t_base = jc * 64 + 32 * kh;
       bf16_t* out = ROLE == 0 ? p.dv : p.dk;
-      if (p.add & (ROLE == 0 ? 4 : 2)) {
-        u32x4 have[NS];
-#pragma unroll
-        for (int i = 0; i < NS; ++i) {
-          const int e = lane + 64 * i, row = min(e / (D2 / 8), len - 1 - t_base), seg = e % (D2 / 8);
-          have[i] = row < 0 ? w2[i] : *reinterpret_cast<const u32x4*>(out + ((size_t)(bos + t_base + row) * p.HKV + hkv) * D2 + seg * 8);
-        }
-#pragma unroll
-        for (int i = 0; i < NS; ++i) w2[i] = add8_bf16(have[i], w2[i]);
-      }
 #pragma unroll
       for (int i = 0; i < NS; ++i) {
         const int e = lane + 64 * i, row = e / (D2 / 8), seg = e % (D2 / 8);
@@ -914,7 +892,6 @@ extern "C" int natsl_softmax_sparse_bwd(const void* q, const void* k, const void
   p.seqs = reinterpret_cast<const SeqRow*>(seqs); p.n_seqs = seqs ? n_seqs : 0; p.total_tiles = total_tiles; p.total_chunks = total_chunks;
   p.scale = scale; p.scale_log2 = scale * 1.4426950408889634f; p.same_block = same_block_visible ? 1 : 0;
   p.dnats_invalid = (flags & 2) ? 1 : 0;
-  p.add = (flags >> 2) & 7;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
 #define NATSL_SB(KK, VV) \
   if (K == KK && V == VV) return launch_bwd<KK, VV>(p, s);

@@ -10,6 +10,7 @@ from . import _capi
 from .nats_util import CHUNK_SIZE, PackedSeqs, _seq_args, pack_sequences
 
 _attn_streams: dict = {}
+_cu_counts: dict = {}
 
 
 class _Cast(ctypes.Structure):
@@ -40,14 +41,15 @@ TIMING_HOOK = None
 
 # Where the softmax branch is launched.  True: on a side stream next to the linear branch (as the
 # reference's Mamba operator does); False: on the caller's stream, one branch after the other (as the
-# reference's GDN operator does); None: decide per call - side by side where the linear branch's chain is long enough.  Its scan
+# reference's GDN operator does); None: decide per call - side by side where the linear branch's chain is long enough and its scan leaves CUs.  The scan
 # walks the chunks one by one with a few large workgroups, so the softmax kernel fills the CUs it leaves; both take most of a CU's
-# LDS (127 KiB / 159 KiB) and never share one, so a scan that fills the chip by itself neither gains nor loses (B8 T8192 H16: 1042
-# and 1045 us; B4 T8192 H8 400 -> 326, Mamba B4 T8192 H32 764 -> 699, four packed documents of 65536 tokens 2274 -> 2162).  Ordering two
+# LDS (127 KiB / 159 KiB) and never share one, so a scan that fills the chip by itself gains nothing (B8 T8192 H16: 1042
+# and 1045 us); B4 T8192 H8 400 -> 326, Mamba B4 T8192 H32 764 -> 699, four packed documents of 65536 tokens 2274 -> 2162 us.  Ordering two
 # streams costs a call about 40 us (36 us one after the other, 78 us side by side at T 256), which the overlap repays from a chain of
 # 2048 tokens at K = 128 on (4096 at K = 64): 87 -> 78 us at B1 T2048 H6, 154 -> 111 us at T 4096, but 56 -> 81 us at T 1024.
 CONCURRENT_BRANCHES = None
 _SIDE_BY_SIDE_TOKENS_X_K = 2048 * 128
+_SCAN_COLUMNS_PER_WG = 64           # state columns of the scans' widest workgroup (csrc/natsl_linear.hip, natsl_linear_bwd.hip)
 
 # What the differentiable operator keeps from its forward for the linear branch's backward.  Keeping means: the state entering
 # every chunk (bf16, K*V per chunk and head), v_new (64*V bf16) and the prep kernel's workspace (17 KiB) stay in device memory
@@ -62,11 +64,21 @@ SAVE_CHUNK_STATES_MAX_BYTES = 1 << 30
 _PREP_WORKSPACE_BYTES = 17 * 1024   # per chunk and head (csrc/natsl_linear.hip)
 
 
-def _run_side_by_side(chain_tokens: int, K: int) -> bool:
+def _run_side_by_side(dev, seqs, B: int, T: int, H: int, K: int, V: int) -> bool:
     """Whether the softmax branch (forward or backward) goes to the side stream (see CONCURRENT_BRANCHES)."""
     if CONCURRENT_BRANCHES is not None:
         return bool(CONCURRENT_BRANCHES)
-    return chain_tokens * K >= _SIDE_BY_SIDE_TOKENS_X_K
+    n_seqs = B if seqs is None else seqs.n_seqs
+    if T * B // n_seqs * K < _SIDE_BY_SIDE_TOKENS_X_K:
+        return False
+    if seqs is not None:
+        return True                                # chains of different lengths
+    index = dev.index if dev.index is not None else torch.cuda.current_device()
+    cus = _cu_counts.get(index)
+    if cus is None:
+        cus = _cu_counts[index] = torch.cuda.get_device_properties(index).multi_processor_count
+    workgroups = n_seqs * H * max(1, V // _SCAN_COLUMNS_PER_WG)
+    return -workgroups % cus >= cus // 16          # CUs that the scan's last round leaves
 
 
 def _keep_chunk_states(q, v, cu_seqlens) -> bool:
@@ -262,7 +274,7 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
     total_chunks = seqs.total_chunks if seqs is not None else B * (-(-T // CHUNK_SIZE))
     # every tensor below belongs to the caller's stream; the softmax branch's stream starts after what that stream holds and is
     # waited for before the call returns, so memory that is freed later is only ever used again behind both
-    side = _get_attn_stream(dev) if _run_side_by_side(T * B // n_seqs, K) else None
+    side = _get_attn_stream(dev) if _run_side_by_side(dev, seqs, B, T, H, K, V) else None
     attn_stream = cur if side is None else side.cuda_stream
     want_start = inference and output_final_state
     chunk_states = keep_chunk_states and not want_start
@@ -417,7 +429,7 @@ class _MixedFunction(torch.autograd.Function):
             attn = prepare_attn_nats_bwd(q_a, k_a, v_a, o_attn, types, idx, nblk, None, lse, do_attn, cfg['scale_attn'], cfg['block'], 0,
                                          cfg['attn_same_block'], cfg['dnats_invalid_attn'], None, None, None, True, seqs)
             here = torch.cuda.current_stream(q_l.device)
-            if _run_side_by_side(q_l.shape[1] * B // (B if seqs is None else seqs.n_seqs), q_l.shape[-1]):
+            if _run_side_by_side(q_l.device, seqs, *q_l.shape, v_l.shape[-1]):
                 side = _get_attn_stream(q_l.device)
                 side.wait_stream(here)
             else:

@@ -546,31 +546,49 @@ __global__ __launch_bounds__((BwdScanLds<DK, NW>::THREADS)) void linear_bwd_scan
     }
     if (more) request(1, c - 1);
 
+    // Left to itself the compiler reads each LDS operand right before the matrix instruction that needs it and waits for it there (some 90
+    // round trips a step): every product below has its operands requested AHEAD instructions before, and what does not depend on the
+    // chain (scale vectors, dO, v_new, TmB) before the product in front of it.
+    s16x4 do_raw[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) do_raw[t] = lds_tr4_at(st + L::OFF_DO + a_v + t * 16 * L::VROW);
     // ---- Y1 = K~ dS' ----------------------------------------------------------------------------------------------------
     f32x4 DV[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) DV[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
     if (!(last && !lin)) {   // (behind a rolled-back block dS' is zero)
+      constexpr int NOP = 4 * KS, AHEAD = 6;
+      f32x4 e4[4];
 #pragma unroll
-      for (int s = 0; s < KS; ++s)
+      for (int t = 0; t < 4; ++t) e4[t] = *reinterpret_cast<lds_f4_t>(st + L::OFF_SC + 4 * (2 * CB) + a_sc + 64 * t);
+      bf16x8 op[NOP + AHEAD];
+      auto ld_k = [&](const int j) __attribute__((always_inline)) -> bf16x8 { return *reinterpret_cast<lds_b128_t>(st + L::OFF_K + a_kq[j >> 2] + (j & 3) * 16 * L::KROW); };
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-          DV[t] = mfma16(*reinterpret_cast<lds_b128_t>(st + L::OFF_K + a_kq[s] + t * 16 * L::KROW), DSB[s], DV[t]);
+      for (int j = 0; j < AHEAD; ++j) op[j] = ld_k(j);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const f32x4 e4 = *reinterpret_cast<lds_f4_t>(st + L::OFF_SC + 4 * (2 * CB) + a_sc + 64 * t);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) DV[t][r] *= e4[r];
+      for (int j = 0; j < NOP; ++j) {
+        if (j + AHEAD < NOP) op[j + AHEAD] = ld_k(j + AHEAD);
+        DV[j & 3] = mfma16(op[j], DSB[j >> 2], DV[j & 3]);
       }
+#pragma unroll
+      for (int j = 0; j < NOP; ++j) {
+        if (j + AHEAD < NOP) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) DV[t][r] *= e4[t][r];
     }
     if (more) request(2, c - 1);
     // ---- dO in accumulator layout (lane = column, registers = tokens 16 t + 4 g + r); zero past the end of the sequence ----
     f32x4 DOc[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const s16x4 w = lds_tr4_at(st + L::OFF_DO + a_v + t * 16 * L::VROW);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) DOc[t][r] = bf16_to_f32((bf16_t)w[r]);
+      for (int r = 0; r < 4; ++r) DOc[t][r] = bf16_to_f32((bf16_t)do_raw[t][r]);
     }
     if (__builtin_expect(nvalid < CB, 0)) {
       asm volatile("" ::: "memory");   // (keeps this a branch: it runs once per chain)
@@ -581,20 +599,38 @@ __global__ __launch_bounds__((BwdScanLds<DK, NW>::THREADS)) void linear_bwd_scan
           if (16 * t + 4 * g4 + r >= nvalid) DOc[t][r] = 0.f;
     }
     if (more) request(3, c - 1);
+    // operand i of TmB^T / P^T: (tj, s2) = (0, 0), (1, 0), (0, 1), (1, 1), (2, 1), (3, 1)
+    constexpr auto TRI_J = [](const int i) { return i < 2 ? i : i - 2; };
+    auto tri_t = [&](const unsigned off, const int i) __attribute__((always_inline)) -> bf16x8 {
+      const int tj = TRI_J(i), s2 = i >= 2;
+      return join4(lds_tr4_at(st + off + 1024 * tri_slot(2 * s2, tj >> 1) + a_tm + 8 * (tj & 1)),
+                   lds_tr4_at(st + off + 1024 * tri_slot(2 * s2 + 1, tj >> 1) + a_tm + 8 * (tj & 1)));
+    };
+    bf16x8 tm[6];
+    s16x4 vn_raw[4];
+    f32x4 sq4[4], se4[4];
+    if constexpr (DELTA) {
+#pragma unroll
+      for (int i = 0; i < 6; ++i) tm[i] = tri_t(L::OFF_T, i);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        vn_raw[t] = lds_tr4_at(st + L::OFF_VN + a_v + t * 16 * L::VROW);
+        se4[t] = *reinterpret_cast<lds_f4_t>(st + L::OFF_SC + a_sc + 64 * t);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) sq4[t] = *reinterpret_cast<lds_f4_t>(st + L::OFF_SC + 4 * CB + a_sc + 64 * t);
     // ---- Y2 = P^T dO ----------------------------------------------------------------------------------------------------
     if (intra) {
       const bf16x8 DOB[2] = {pack8(DOc[0], DOc[1]), pack8(DOc[2], DOc[3])};
       if constexpr (DELTA) {
         // P as the prep kernel stored it, read transposed (see a_tm): rows i = 32 s2 + 16 hf + 4 g + j of column 16 tj + x
+        bf16x8 op[6];
 #pragma unroll
-        for (int tj = 0; tj < 4; ++tj)
+        for (int i = 0; i < 6; ++i) op[i] = tri_t(L::OFF_P, i);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int s2 = 0; s2 < 2; ++s2)
-            if (2 * s2 + 1 >= tj) {
-              const unsigned lo = st + L::OFF_P + 1024 * tri_slot(2 * s2, tj >> 1) + a_tm + 8 * (tj & 1);
-              const unsigned hi = st + L::OFF_P + 1024 * tri_slot(2 * s2 + 1, tj >> 1) + a_tm + 8 * (tj & 1);
-              DV[tj] = mfma16(join4(lds_tr4_at(lo), lds_tr4_at(hi)), DOB[s2], DV[tj]);
-            }
+        for (int i = 0; i < 6; ++i) DV[TRI_J(i)] = mfma16(op[i], DOB[i >= 2], DV[TRI_J(i)]);
       } else {
         // P^T formed here, once per workgroup: Z = q k^T leaves lane (x, g) with key 16 tj + x against queries
         // 16 ti + 4 g + r, the four slots this lane holds of operand (tj, ti / 2), half ti % 2.  Operand (tj, s2) at index
@@ -643,17 +679,13 @@ __global__ __launch_bounds__((BwdScanLds<DK, NW>::THREADS)) void linear_bwd_scan
       const bf16x8 DVB[2] = {pack8_trunc(DV[0], DV[1]), pack8_trunc(DV[2], DV[3])};
       const bf16x8 DVR[2] = {pack8_rest(DV[0], DV[1]), pack8_rest(DV[2], DV[3])};
 #pragma unroll
-      for (int tj = 0; tj < 4; ++tj) {
-        DX[tj] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      for (int t = 0; t < 4; ++t) DX[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2)
-          if (2 * s2 + 1 >= tj) {
-            const unsigned lo = st + L::OFF_T + 1024 * tri_slot(2 * s2, tj >> 1) + a_tm + 8 * (tj & 1);
-            const unsigned hi = st + L::OFF_T + 1024 * tri_slot(2 * s2 + 1, tj >> 1) + a_tm + 8 * (tj & 1);
-            const bf16x8 a = join4(lds_tr4_at(lo), lds_tr4_at(hi));
-            DX[tj] = mfma16(a, DVR[s2], DX[tj]);
-            DX[tj] = mfma16(a, DVB[s2], DX[tj]);
-          }
+      for (int s2 = 0; s2 < 2; ++s2) {
+#pragma unroll
+        for (int i = 2 * s2; i < 2 + 4 * s2; ++i) DX[TRI_J(i)] = mfma16(tm[i], DVR[s2], DX[TRI_J(i)]);
+#pragma unroll
+        for (int i = 2 * s2; i < 2 + 4 * s2; ++i) DX[TRI_J(i)] = mfma16(tm[i], DVB[s2], DX[TRI_J(i)]);
       }
     } else {
 #pragma unroll
@@ -669,9 +701,8 @@ __global__ __launch_bounds__((BwdScanLds<DK, NW>::THREADS)) void linear_bwd_scan
       if constexpr (DELTA) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-          const s16x4 w = lds_tr4_at(st + L::OFF_VN + a_v + t * 16 * L::VROW);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) VNc[t][r] = bf16_to_f32((bf16_t)w[r]);
+          for (int r = 0; r < 4; ++r) VNc[t][r] = bf16_to_f32((bf16_t)vn_raw[t][r]);
         }
       }
 #pragma unroll
@@ -709,32 +740,42 @@ __global__ __launch_bounds__((BwdScanLds<DK, NW>::THREADS)) void linear_bwd_scan
       f32x4 A1[4], A2[4];
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const f32x4 s4 = *reinterpret_cast<lds_f4_t>(st + L::OFF_SC + 4 * CB + a_sc + 64 * t);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) A1[t][r] = DOc[t][r] * s4[r];
+        for (int r = 0; r < 4; ++r) A1[t][r] = DOc[t][r] * sq4[t][r];
         if constexpr (DELTA) {
-          const f32x4 e4 = *reinterpret_cast<lds_f4_t>(st + L::OFF_SC + a_sc + 64 * t);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) A2[t][r] = -DX[t][r] * e4[r];
+          for (int r = 0; r < 4; ++r) A2[t][r] = -DX[t][r] * se4[t][r];
         }
       }
-      const bf16x8 B1[2] = {pack8(A1[0], A1[1]), pack8(A1[2], A1[3])};
+      bf16x8 B1[2] = {pack8(A1[0], A1[1]), pack8(A1[2], A1[3])};
       bf16x8 B2[2];
       if constexpr (DELTA) { B2[0] = pack8(A2[0], A2[1]); B2[1] = pack8(A2[2], A2[3]); }
-      auto ld_t = [&](const int off, const int m, const int s2) __attribute__((always_inline)) -> bf16x8 {
+      // product j: state tile j % KT, of (q, first 32 tokens), (k, first), (q, last), (k, last)
+      constexpr int ND = DELTA ? 2 : 1, NOP = 2 * ND * KT, AHEAD = 6;
+      auto ld_t = [&](const int j) __attribute__((always_inline)) -> bf16x8 {
+        const int m = j % KT, s2 = j / (ND * KT), off = DELTA && (j / KT & 1) ? L::OFF_K : L::OFF_Q;
         const unsigned a = st + off + a_kt[m >> 1] + 8u * (m & 1) + (32 * s2) * L::KROW;
         return join4(lds_tr4_at(a), lds_tr4_at(a + 16 * L::KROW));
       };
+      bf16x8 op[NOP + AHEAD];
 #pragma unroll
-      for (int m = 0; m < KT; ++m) {
+      for (int j = 0; j < AHEAD; ++j) op[j] = ld_t(j);
+#pragma unroll
+      for (int m = 0; m < KT; ++m)
 #pragma unroll
         for (int r = 0; r < 4; ++r) dS[m][r] *= dec;
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-          dS[m] = mfma16(ld_t(L::OFF_Q, m, s2), B1[s2], dS[m]);
-          if constexpr (DELTA) dS[m] = mfma16(ld_t(L::OFF_K, m, s2), B2[s2], dS[m]);
-        }
+      for (int j = 0; j < NOP; ++j) {
+        if (j + AHEAD < NOP) op[j + AHEAD] = ld_t(j + AHEAD);
+        dS[j % KT] = mfma16(op[j], DELTA && (j / KT & 1) ? B2[j / (ND * KT)] : B1[j / (ND * KT)], dS[j % KT]);
       }
+#pragma unroll
+      for (int j = 0; j < NOP; ++j) {
+        if (j + AHEAD < NOP) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
     // ---- this step's global stores (and the one scalar the next step needs) -----------------------------------------------
     {

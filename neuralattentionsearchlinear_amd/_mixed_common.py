@@ -333,12 +333,19 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
         here = torch.cuda.current_stream(dev)
         step = lambda phases: _capi.check(L.natsl_mixed_fwd(ref, phases, cur, attn_stream), "natsl_mixed_fwd")
         step(_CONVERT | _ROUTE)
-        TIMING_HOOK("softmax:start", here if side is None else side)
-        step(_SOFTMAX)
-        TIMING_HOOK("softmax:end", here if side is None else side)
-        TIMING_HOOK("linear:start", here)
-        step(_LINEAR)
-        TIMING_HOOK("linear:end", here)
+        if side is None:
+            TIMING_HOOK("softmax:start", here)
+            step(_SOFTMAX)
+            TIMING_HOOK("softmax:end", here)
+            TIMING_HOOK("linear:start", here)
+            step(_LINEAR)
+            TIMING_HOOK("linear:end", here)
+        else:                                              # (side by side the order is the call's own; softmax includes its wait)
+            TIMING_HOOK("softmax:start", side)
+            TIMING_HOOK("linear:start", here)
+            step(_SOFTMAX | _LINEAR)
+            TIMING_HOOK("softmax:end", side)
+            TIMING_HOOK("linear:end", here)
         step(_JOIN)
     if n_prefix:
         o_attn = o_attn[:, n_prefix:]

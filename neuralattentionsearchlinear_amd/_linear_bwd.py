@@ -2,8 +2,8 @@
 
 linear_chunk_backward_hip is the product path: the forward's per-chunk state and v_new outputs (kept by the differentiable
 operator from its own forward, else the forward once more), then
-natsl_linear_chunk_bwd (csrc/natsl_linear_bwd.hip: a reverse scan over the chunks and a per-chunk gradient kernel), and the
-few lines of host glue around them (block sums of g, the per-block sums of the gate gradients).  It replaces
+natsl_linear_chunk_bwd_steps (csrc/natsl_linear_bwd.hip: a reverse scan over the chunks and a per-chunk gradient kernel), and
+around them natsl_linear_block_sums (sums of g per selector block) and natsl_block_grads (of the gate gradients).  It replaces
 chunk_gated_delta_rule_nats_bwd (src/nats/ops/gated_delta_rule/chunk.py:170-332) and the Mamba counterpart
 (src/nats/ops/mamba/chunk.py:112-260) in function.  linear_chunk_backward_torch is the same method as fp32 torch operations
 on the GPU, for key widths the kernels are not built for and as the method's plain statement; both follow the

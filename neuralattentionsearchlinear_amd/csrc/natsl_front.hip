@@ -500,6 +500,32 @@ __global__ __launch_bounds__(256) void select_bwd_kernel(const void* logits, con
   stf(dlogits, dtype, 2 * i + 1, y1 * (d1 - m));
 }
 
+static int conv_cus() {
+  static std::atomic<int> cached{0};
+  int n = cached.load();
+  if (n == 0) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cached.store(n);
+  }
+  return n;
+}
+
+// Tokens per thread: long runs read the fewest rows twice (and leave the fewest partial sums), but what counts first is that the
+// workgroups fill whole rounds of the chip -- registers admit three of them on a CU forward, two backward
+// (340M geometry, 8 x 4096: backward with runs of 64 in 1.5 rounds 233 us, of 98 in one 208; forward 32 -> 64 tokens 100 -> 94).
+static int conv_run(int B, int T, int W, int groups, bool bwd) {
+  const long long slots = (long long)conv_cus() * (bwd ? 2 : 3);
+  int best = 8;
+  double best_cost = 1e300;
+  for (int run = 8; run <= (bwd ? 128 : 64); run += bwd ? 2 : 8) {
+    const long long wgs = ((long long)B * cdiv(T, run) * groups + 255) / 256;
+    const double cost = (double)((wgs + slots - 1) / slots) * (run + W - 1 + (bwd ? 5 : 1));
+    if (cost <= best_cost) { best_cost = cost; best = run; }
+  }
+  return best;
+}
+
 static int conv_plan(ConvNormParams& p, const natsl_conv_seg* seg, int n_seg, int B, int T, int W, int silu, int norm_dtype, bool bwd, const char* what) {
   if (!seg || n_seg <= 0 || n_seg > NATSL_CONV_SEGS) return fail(NATSL_ERR_INVALID, "%s: 1 to %d tensors", what, NATSL_CONV_SEGS);
   if (B <= 0 || T <= 0) return fail(NATSL_ERR_INVALID, "%s: non-positive dimension", what);
@@ -516,9 +542,7 @@ static int conv_plan(ConvNormParams& p, const natsl_conv_seg* seg, int n_seg, in
     }
     all += s.D;
   }
-  // long runs read the fewest rows twice and leave the fewest partial sums; short ones give small inputs enough threads
-  int run = bwd ? 64 : 32;
-  while (run > 8 && (long long)B * cdiv(T, run) * (all / 8) < 512ll * 256) run >>= 1;
+  const int run = conv_run(B, T, W, all / 8, bwd);
   p.n_seg = n_seg; p.B = B; p.T = T; p.run = run; p.silu = silu; p.norm_dtype = norm_dtype;
   long long wgs = 0;
   for (int i = 0; i < NATSL_CONV_SEGS; ++i) {

@@ -20,6 +20,7 @@ def _general(monkeypatch):
     ('gdn', None, 1, 64, {}), ('gdn', '340M', 2, 333, {}), ('gdn', '760M', 1, 200, dict(allow_neg_eigval=True, conv_bias=True)),
     ('gdn', None, 3, 130, dict(conv_size=3, conv_activation=None)), ('gdn', None, 2, 65, dict(conv_size=2)),
     ('mamba', None, 2, 257, {}), ('mamba', None, 1, 100, dict(attn_qk_norm=True, conv_bias=True)),
+    ('gdn', '340M', 7, 1999, {}), ('gdn', None, 16, 4100, dict(conv_size=3)),             # long runs, the last one short
 ])
 def test_front_matches_the_general_path(kind, geometry, B, T, more, monkeypatch):
     layer = _layer(kind, geometry, 'all', **more).train()

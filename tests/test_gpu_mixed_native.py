@@ -40,10 +40,13 @@ def test_fp32_tensors_equal_rounded_tensors(kind, B, T, H, K, V, grad):
         assert torch.equal(a.detach(), b.float()), name
 
 
-@pytest.mark.parametrize("kind,H,K,V", [('gdn', 2, 64, 64), ('mamba', 3, 128, 64)])
-def test_side_stream_and_one_stream_agree(kind, H, K, V, monkeypatch):
+@pytest.mark.parametrize("kind,B,H,K,V", [('gdn', 1, 2, 64, 64), ('mamba', 1, 3, 128, 64),
+                                          # the scan's width depends on what it leaves: 1, 2, 4 waves, several rounds
+                                          ('gdn', 5, 13, 64, 64), ('gdn', 9, 15, 128, 128), ('gdn', 11, 24, 128, 64),
+                                          ('mamba', 5, 13, 128, 64), ('mamba', 9, 15, 64, 128)])
+def test_side_stream_and_one_stream_agree(kind, B, H, K, V, monkeypatch):
     import neuralattentionsearchlinear_amd._mixed_common as MC
-    q, k, v, g, beta, ty = _case(kind, 1, 500, H, K, V, 9)
+    q, k, v, g, beta, ty = _case(kind, B, 500 if B == 1 else 130, H, K, V, 9)
     outs = []
     for side in (False, True):
         monkeypatch.setattr(MC, 'CONCURRENT_BRANCHES', side)

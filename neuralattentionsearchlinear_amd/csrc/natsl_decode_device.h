@@ -98,15 +98,17 @@ struct AttnRow {
     for (int i = 0; i < KEY_PASSES; ++i) mx = fmaxf(mx, s[i]);
     mx = fmaxf(mx, __shfl_xor(mx, 16));
     mx = xhalf_max(mx);
-    const float mn = fmaxf(m, mx);                       // finite: some key is visible
-    const float alpha = __builtin_amdgcn_exp2f(m - mn);
+    // Scores can be -inf for keys that are visible (infinite entries, an overflow of q.k): such keys weigh 0.  While there is no
+    // other key the exponents are taken from 0, as -inf minus -inf would make NaN of everything that follows.
+    const float mn = fmaxf(m, mx), ref = mn == -INFINITY ? 0.f : mn;
+    const float alpha = __builtin_amdgcn_exp2f(m - ref);
     m = mn;
     l *= alpha;
 #pragma unroll
     for (int e = 0; e < EV; ++e) acc[e] *= alpha;
 #pragma unroll
     for (int i = 0; i < KEY_PASSES; ++i) {
-      const float p = __builtin_amdgcn_exp2f(s[i] - mn);
+      const float p = __builtin_amdgcn_exp2f(s[i] - ref);
       l += p;
 #pragma unroll
       for (int e = 0; e < EV; ++e) acc[e] += p * vr[i].at(e);

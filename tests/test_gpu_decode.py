@@ -82,6 +82,36 @@ def test_masked_attention_against_oracle(K, V, TQ, TK, HM, dtype):
     assert float(o[0, 0, :HQ // HM].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("pair,dtype", [(False, torch.bfloat16), (False, torch.float32), (True, torch.bfloat16)])  # attention alone; a whole decode step
+@pytest.mark.parametrize("first,last,TK", [(0, 32, 130), (0, 64, 64), (0, 64, 700), (256, 320, 3000), (5, 33, 100)])
+def test_masked_attention_with_scores_of_minus_infinity(first, last, TK, pair, dtype):
+    """Keys whose score is -inf (an infinite entry, an overflow of q.k) weigh 0 although they are visible, also where a wave meets no
+    other key before them; a query that has only such keys gives 0."""
+    from neuralattentionsearchlinear_amd.mixed_attn_gdn import masked_attention, nats_mixed_attn_gdn_recurrent
+    B, H, K, V, TQ = 2, 4, 64, 128, 2
+    gen = torch.Generator().manual_seed(TK + first)
+    q = torch.randn(B, TQ, H, K, generator=gen).to(dtype)
+    k = torch.randn(B, TK, H, K, generator=gen).to(dtype)
+    v = torch.randn(B, TK, H, V, generator=gen).to(dtype)
+    q[..., 3] = q[..., 3].abs() + 0.1
+    k[:, first:last, :, 3] = float('-inf')
+    mask = torch.ones(B, 1, TQ, TK, dtype=torch.bool)
+    mask[1, :, 0, last:] = False
+    mask[1, :, 0, :first] = False                          # only keys of score -inf
+    ref = D.attn_masked(q.float(), k.float(), v.float(), mask, K ** -0.5)
+    if pair:
+        ql, kl, vl = make_qkv(B, TQ, H, K, V, 3)
+        g, beta = make_gates(B, TQ, H, 4)
+        h0 = torch.zeros(B, H, K, V)
+        o = nats_mixed_attn_gdn_recurrent(*_dev(q, k, v, ql, kl, vl, mask, h0, h0.clone(), g, torch.zeros(B, H), beta), torch.ones(B, 1, H, 2).bfloat16().to(DEV),
+                                          n_tokens_in_current_block=0, nats_block_size=64, ops_for_incomplete_chunks='all')[1]
+    else:
+        o = masked_attention(*_dev(q, k, v, mask), K ** -0.5)
+    assert bool(torch.isfinite(o.float()).all())
+    assert_close(o.float(), ref, "o_attn")
+    assert float(o[1, 0].abs().max()) == 0.0
+
+
 def test_masked_attention_reads_a_cache_buffer_in_place():
     """Keys / values that are the front part of a larger cache buffer [B, capacity, H, D] are read where they are (batch
     stride = capacity * H * D): same result as on a dense copy, bit for bit, and the buffer's tail is never touched."""

@@ -34,9 +34,6 @@ NATSL_DEVICE u32x4 down8(const float* f) {
 }
 NATSL_DEVICE const u32x4* row8(const void* p, const size_t elem) { return reinterpret_cast<const u32x4*>(reinterpret_cast<const bf16_t*>(p) + elem); }
 
-// 1 / (1 + e^-x): the hardware's reciprocal (1 ulp, like its exponential) where a correctly rounded division takes ten instructions
-NATSL_DEVICE float sigmoid_1ulp(const float x) { return __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
-
 // sums over the `lanes` adjacent lanes (a power of two) that share a head row
 NATSL_DEVICE void group_sum2(float& a, float& b, const int lanes) {
   for (int d = 1; d < lanes; d <<= 1) {
@@ -115,7 +112,7 @@ __global__ __launch_bounds__(256) void conv_norm_kernel(const ConvNormParams p) 
       float acc = bs[c];
 #pragma unroll
       for (int j = 0; j < W; ++j) acc += wt[j][c] * win[j][c];
-      y[c] = p.silu ? acc * sigmoid_1ulp(acc) : acc;
+      y[c] = p.silu ? acc / (1.f + __expf(-acc)) : acc;
     }
     const u32x4 packed = down8(y);
     const size_t at = base + (size_t)t * D;
@@ -196,7 +193,7 @@ __global__ __launch_bounds__(256) void conv_norm_bwd_kernel(const ConvNormParams
       y[c] = acc;
       da[c] = 1.f;
       if (p.silu) {
-        const float sg = sigmoid_1ulp(acc);
+        const float sg = 1.f / (1.f + __expf(-acc));
         y[c] = acc * sg;
         da[c] = sg * (1.f + acc * (1.f - sg));
       }

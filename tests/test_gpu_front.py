@@ -61,6 +61,32 @@ def test_front_on_a_cache(kind, T0, sizes, monkeypatch):
     assert torch.equal(cf.n_attn_blocks, cs.n_attn_blocks)
 
 
+@pytest.mark.parametrize("W,bias", [(4, False), (3, True), (2, False)])
+def test_conv_arithmetic_is_the_single_kernels(W, bias):
+    """The fused convolution forms its activation, and the gradients behind it, with the arithmetic of natsl_short_conv_*: the same bits.
+    (A reciprocal in the place of the division moves about one rounding to bf16 in 2^15; a tensor here holds 2^22 values.)"""
+    from neuralattentionsearchlinear_amd import _front
+    from neuralattentionsearchlinear_amd._layer_step import watch
+    layer = _layer('gdn', None, 'all', conv_size=W, conv_bias=bias)
+    f = _front._front_plan(layer, 'gdn', watch(layer))
+    torch.manual_seed(W)
+    B, T = 4, 4096
+    raw = [torch.randn(B, T, c.hidden_size, device=DEV).bfloat16() for c in (layer.q_conv1d, layer.k_conv1d, layer.v_conv1d)]
+    ref = lambda i, x: (layer.q_conv1d, layer.k_conv1d, layer.v_conv1d)[i](x)[0]
+    with torch.no_grad():
+        for i, y in enumerate(_front._conv_norm(f, raw, None, False)[0]):
+            assert torch.equal(y, ref(i, raw[i])), "qkv"[i]
+    grads = []
+    for fused in (True, False):
+        x = [r.clone().requires_grad_(True) for r in raw]
+        ys = f.conv_norm(*x, (None,) * 3, False)[:3] if fused else [ref(i, t) for i, t in enumerate(x)]
+        torch.manual_seed(1)
+        torch.autograd.backward(ys, [torch.randn_like(y) for y in ys])
+        grads.append([t.grad for t in x])
+    for a, b, n in zip(*grads, "qkv"):
+        assert torch.equal(a, b), f"d{n}"
+
+
 @pytest.mark.parametrize("T,D,widths", [(1, 8, (8,)), (31, 64, (16, 24)), (32, 256, (256,)), (33, 264, (264, 8)), (129, 72, (512,)), (5000, 128, (136,))])
 def test_weight_grads(T, D, widths):
     """natsl_wgrad at the edges of its 32-token stages, 256-wide tiles and token slices."""

@@ -86,6 +86,11 @@ NATSL_DEVICE float xhalf_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// The layers' gates, shared by whole sequences and single steps: both write rows of the same cache, so both take the library's
+// exponential (the hardware's differs from it by up to its argument in ulps, and g is kept and summed up in fp32).
+NATSL_DEVICE float softplus_gate(const float x) { return x > 20.f ? x : log1pf(expf(x)); }
+NATSL_DEVICE float sigmoid_gate(const float x) { return 1.f / (1.f + expf(-x)); }
+
 // Per-sequence descriptor for packed (variable-length) input; one row per sequence.
 struct SeqRow {
   int bos;        // first token (flat index)

@@ -341,18 +341,17 @@ struct GatesParams {
   long long rows;
   int H, ld, dtype, neg;
 };
-NATSL_DEVICE float softplus_x(const float x) { return x > 20.f ? x : log1pf(expf(x)); }
 
 __global__ __launch_bounds__(256) void gates_kernel(const GatesParams p) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= p.rows * p.H) return;
   const long long row = i / p.H;
   const int h = (int)(i - row * p.H);
-  const float dt = softplus_x(bf16_to_f32(p.ab[row * p.ld + h]) + ldf(p.dt_bias, p.dtype, h));
+  const float dt = softplus_gate(bf16_to_f32(p.ab[row * p.ld + h]) + ldf(p.dt_bias, p.dtype, h));
   p.g[i] = -expf(ldf(p.a_log, p.dtype, h)) * dt;
   if (p.dt) p.dt[i] = dt;
   if (p.beta) {
-    float s = bf16_to_f32(f32_to_bf16(1.f / (1.f + expf(-bf16_to_f32(p.ab[row * p.ld + p.H + h])))));
+    float s = bf16_to_f32(f32_to_bf16(sigmoid_gate(bf16_to_f32(p.ab[row * p.ld + p.H + h]))));
     p.beta[i] = f32_to_bf16(p.neg ? 2.f * s : s);
   }
 }
@@ -369,7 +368,7 @@ __global__ __launch_bounds__(256) void gates_bwd_kernel(const GatesParams p) {
       const long long row = ((long long)blockIdx.x * GATES_ITERS + it) * in + ri;
       if (row >= p.rows) break;
       const float x = bf16_to_f32(p.ab[row * p.ld + h]) + bias;
-      const float dt = softplus_x(x), sg = x > 20.f ? 1.f : 1.f / (1.f + expf(-x));
+      const float dt = softplus_gate(x), sg = x > 20.f ? 1.f : sigmoid_gate(x);
       const float dg = p.dg ? p.dg[row * p.H + h] : 0.f;
       const float ddt = (p.ddt ? p.ddt[row * p.H + h] : 0.f) - A * dg;
       const float da = ddt * sg;
@@ -379,7 +378,7 @@ __global__ __launch_bounds__(256) void gates_bwd_kernel(const GatesParams p) {
       o[h] = f32_to_bf16(da);
       int used = p.H;
       if (p.beta || p.dbeta) {
-        const float s = bf16_to_f32(f32_to_bf16(1.f / (1.f + expf(-bf16_to_f32(p.ab[row * p.ld + p.H + h])))));
+        const float s = bf16_to_f32(f32_to_bf16(sigmoid_gate(bf16_to_f32(p.ab[row * p.ld + p.H + h]))));
         const float db = p.dbeta ? bf16_to_f32(p.dbeta[row * p.H + h]) : 0.f;
         o[p.H + h] = f32_to_bf16((p.neg ? 2.f : 1.f) * db * s * (1.f - s));
         used = 2 * p.H;

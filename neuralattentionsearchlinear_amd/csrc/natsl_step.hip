@@ -91,8 +91,6 @@ struct StepMix {
   bf16_t *q_conv, *q_lin, *q_attn;                    // [M][H*K]; q_lin == q_conv without L2-normalised rows
 };
 
-NATSL_DEVICE float softplus_f(const float x) { return x > 20.f ? x : log1pf(__expf(x)); }
-
 template <int W>
 struct ConvWindow {
   float e[W], w[W], b;      // e: the last W inputs
@@ -185,14 +183,14 @@ __global__ __launch_bounds__(256) void step_mix_kernel(const StepMix p) {
   }
   if (role == 2) {
     const int VD = H * V;
-    const float A = __expf(ld_any(s.a_log, s.gate_dtype, h)), bias = ld_any(s.dt_bias, s.gate_dtype, h);
+    const float A = expf(ld_any(s.a_log, s.gate_dtype, h)), bias = ld_any(s.dt_bias, s.gate_dtype, h);
     for (int t = tid; t < T; t += 256) {
       const size_t row = (size_t)b * T + t;
-      const float dt = softplus_f(bf16_to_f32(p.proj[row * p.ldp + p.ca + h]) + bias);
+      const float dt = softplus_gate(bf16_to_f32(p.proj[row * p.ldp + p.ca + h]) + bias);
       s.block_g[(block_row + t) * H + h] = -A * dt;
       if (s.is_delta) {
         const float be = bf16_to_f32(p.proj[row * p.ldp + p.cb + h]);
-        float sg = bf16_to_f32(f32_to_bf16(1.f / (1.f + __expf(-be))));
+        float sg = bf16_to_f32(f32_to_bf16(sigmoid_gate(be)));
         if (s.flags & NATSL_STEP_NEG_EIGVAL) sg *= 2.f;
         ((bf16_t*)s.block_beta)[(block_row + t) * H + h] = f32_to_bf16(sg);
       }
@@ -209,7 +207,7 @@ __global__ __launch_bounds__(256) void step_mix_kernel(const StepMix p) {
         const float x = bf16_to_f32(p.proj[row * p.ldp + p.cv + d]);
         const float y = win.next(x, silu);
         float lin = y;
-        if (!s.is_delta) lin = y * softplus_f(bf16_to_f32(p.proj[row * p.ldp + p.ca + h]) + bias);
+        if (!s.is_delta) lin = y * softplus_gate(bf16_to_f32(p.proj[row * p.ldp + p.ca + h]) + bias);
         ((bf16_t*)s.block_v)[(block_row + t) * VD + d] = f32_to_bf16(lin);
         ((bf16_t*)s.cache_v)[(cache_row + t) * VD + d] = f32_to_bf16(from_conv ? y : x);
       }

@@ -84,6 +84,38 @@ def test_layer_step_matches_the_general_path(kind, geometry, ops, B, T0, sizes, 
         assert a.shape == b.shape and rel_l2(a.float(), b.float()) <= 5e-3, f"cache tensor {i}: rel-L2 {rel_l2(a.float(), b.float()):.3e}"
 
 
+@pytest.mark.parametrize("kind", ['gdn', 'mamba'])
+@pytest.mark.parametrize("float_gates", [False, True])
+def test_layer_step_forms_the_general_paths_gates(kind, float_gates, monkeypatch):
+    """g (kept in fp32 and summed up) and beta of a step are those of the general path and of a prefill, bit for bit: the projections
+    that feed them pick single inputs, so that nothing before the gates rounds."""
+    from neuralattentionsearchlinear_amd import natsl_attn_gdn, natsl_attn_mamba2
+    layer = _layer(kind, None, 'all')
+    torch.manual_seed(5)
+    with torch.no_grad():
+        for i, name in enumerate(("a_proj", "b_proj")):
+            if hasattr(layer, name):
+                w = getattr(layer, name).weight
+                w.zero_()[torch.arange(w.shape[0]), 10 * i + torch.arange(w.shape[0])] = 4.0
+        layer.dt_bias.copy_(torch.randn_like(layer.dt_bias))
+        if float_gates:
+            layer.A_log.data, layer.dt_bias.data = layer.A_log.data.float() * 1.003, layer.dt_bias.data.float() * 1.003
+    sizes = (4,) * 15
+    x = torch.randn(16, 64 + sum(sizes), layer.hidden_size, device=DEV).bfloat16()
+    _, cf = _generate(layer, kind, x, 64, sizes)
+    for mod in (natsl_attn_gdn, natsl_attn_mamba2):
+        monkeypatch.setattr(mod, 'layer_step', lambda *a: None)
+    _, cs = _generate(layer, kind, x, 64, sizes)
+    n = cf._n_tokens_in_nats_block
+    assert n == sum(sizes) == cs._n_tokens_in_nats_block
+    assert torch.equal(cf.lattn_g[:, :n], cs.lattn_g[:, :n])
+    # the same tokens as the incomplete end of one prompt
+    _, cp = _generate(layer, kind, x, x.shape[1], ())
+    assert torch.equal(cf.lattn_g[:, :n], cp.lattn_g[:, :n])
+    if kind == 'gdn':
+        assert torch.equal(cf.lattn_beta[:, :n], cs.lattn_beta[:, :n]) and torch.equal(cf.lattn_beta[:, :n], cp.lattn_beta[:, :n])
+
+
 def test_layer_step_follows_replaced_weights_and_declines_hooks():
     """The step reads the layer's current parameters, and a hooked submodule sends the layer down the general path."""
     import neuralattentionsearchlinear_amd._layer_step as LS

@@ -91,6 +91,13 @@ NATSL_DEVICE float xhalf_sum(float x) {
 NATSL_DEVICE float softplus_gate(const float x) { return x > 20.f ? x : log1pf(expf(x)); }
 NATSL_DEVICE float sigmoid_gate(const float x) { return 1.f / (1.f + expf(-x)); }
 
+// The softmax of a head's two mixing logits, rounded to bf16: what the mixing layer's separate softmax returns
+NATSL_DEVICE void mix_softmax(float& a, float& b) {
+  const float mx = fmaxf(a, b), e0 = expf(a - mx), e1 = expf(b - mx);
+  a = __uint_as_float(pack_bf16x2(e0 / (e0 + e1), 0.f) << 16);
+  b = __uint_as_float(pack_bf16x2(e1 / (e0 + e1), 0.f) << 16);
+}
+
 // Per-sequence descriptor for packed (variable-length) input; one row per sequence.
 struct SeqRow {
   int bos;        // first token (flat index)

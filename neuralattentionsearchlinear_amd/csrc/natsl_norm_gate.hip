@@ -14,16 +14,11 @@ NATSL_DEVICE void unpack8(const u32x4 w, float* f) {
   }
 }
 
-// The mixing weights of a row: as given, or the softmax of the two given logits rounded to bf16 (what the mixing layer's separate
-// softmax returns; taken here, it costs no pass of its own)
+// The mixing weights of a row: as given, or the softmax of the two given logits (taken here, it costs no pass of its own)
 NATSL_DEVICE void mix_weights(const bf16_t* xw, const long long row, const int logits, float& a, float& b) {
   a = bf16_to_f32(xw[row * 2]);
   b = bf16_to_f32(xw[row * 2 + 1]);
-  if (logits) {
-    const float mx = fmaxf(a, b), e0 = __expf(a - mx), e1 = __expf(b - mx), inv = 1.f / (e0 + e1);
-    a = bf16_to_f32(f32_to_bf16(e0 * inv));
-    b = bf16_to_f32(f32_to_bf16(e1 * inv));
-  }
+  if (logits) mix_softmax(a, b);
 }
 
 template <int LANES, int PER>  // a row is handled by LANES adjacent lanes, PER 16-byte pieces each: D = 8 LANES PER

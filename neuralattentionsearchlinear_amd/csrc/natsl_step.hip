@@ -270,9 +270,8 @@ __global__ __launch_bounds__(256) void step_tail_kernel(const StepTail p) {
   }
   d0 = bf16_to_f32(f32_to_bf16(d0));
   d1 = bf16_to_f32(f32_to_bf16(d1));
-  const float mx = fmaxf(d0, d1), e0 = __expf(d0 - mx), e1 = __expf(d1 - mx);
-  const float ra = rsqrtf(sa / VA + p.eps) * bf16_to_f32(f32_to_bf16(e0 / (e0 + e1)));
-  const float rb = rsqrtf(sb / VA + p.eps) * bf16_to_f32(f32_to_bf16(e1 / (e0 + e1)));
+  mix_softmax(d0, d1);
+  const float ra = rsqrtf(sa / VA + p.eps) * d0, rb = rsqrtf(sb / VA + p.eps) * d1;
 #pragma unroll
   for (int j = 0; j < CPL; ++j) {
     const float g = bf16_to_f32(p.proj[(size_t)row * p.ldp + p.cg + hq * VA + CPL * lane + j]);

@@ -87,6 +87,31 @@ def test_conv_arithmetic_is_the_single_kernels(W, bias):
         assert torch.equal(a, b), f"d{n}"
 
 
+def test_mixing_softmax_is_the_separate_ones():
+    """The norm-gate that takes mixing logits gives what it gives for the weights of torch's bf16 softmax, forward and backward: the same
+    bits.  (An exponential an ulp off moves about one weight in 2^15 across a rounding edge; here are 2^21 of them.)"""
+    from neuralattentionsearchlinear_amd import _capi
+    torch.manual_seed(2)
+    rows, D = 1 << 20, 32
+    a, b, g, dy = (torch.randn(rows, D, device=DEV).bfloat16() for _ in range(4))
+    logits = 3 * torch.randn(rows, 2, device=DEV).bfloat16()
+    w = torch.rand(2, D, device=DEV)
+    L, P, st = _capi.lib(), _capi.ptr, _capi.stream_ptr(a.device)
+    n = L.natsl_norm_gate_bwd_workspace_bytes(rows, D)
+    outs = []
+    for fused, xw in ((True, logits), (False, logits.softmax(-1))):
+        y, da, db, dg = (torch.empty_like(a) for _ in range(4))
+        dx = torch.empty(rows, 2, dtype=torch.bfloat16 if fused else torch.float32, device=DEV)
+        dw, ws = torch.empty(2, D, device=DEV), torch.empty(n, dtype=torch.uint8, device=DEV)
+        fwd, bwd = (L.natsl_norm_gate_logits_fwd, L.natsl_norm_gate_logits_bwd) if fused else (L.natsl_norm_gate_fwd, L.natsl_norm_gate_bwd)
+        _capi.check(fwd(P(a), P(b), P(g), P(xw), P(w[0]), P(w[1]), P(y), rows, D, _capi.BF16, 1e-5, _capi.F32, st), "forward")
+        _capi.check(bwd(P(a), P(b), P(g), P(xw), P(w[0]), P(w[1]), P(dy), P(da), P(db), P(dg), P(dx), P(dw[0]), P(dw[1]), P(ws), n, rows, D,
+                        _capi.BF16, 1e-5, _capi.F32, st), "backward")
+        outs.append((y, da, db, dg, dw))
+    for i, (p, q) in enumerate(zip(*outs)):
+        assert torch.equal(p, q), f"output {i}: {int((p != q).sum())} values differ"
+
+
 @pytest.mark.parametrize("T,D,widths", [(1, 8, (8,)), (31, 64, (16, 24)), (32, 256, (256,)), (33, 264, (264, 8)), (129, 72, (512,)), (5000, 128, (136,))])
 def test_weight_grads(T, D, widths):
     """natsl_wgrad at the edges of its 32-token stages, 256-wide tiles and token slices."""

@@ -216,7 +216,9 @@ class NeuralAttentionSearchLinearAttnGDN(nn.Module):
             selector_input = cache.update_attn_types(input_hidden_states=hidden_states)
         else:
             selector_input = hidden_states
-        fast = fast_front(self, 'gdn', hidden_states, cache, cu_seqlens) if mode == 'chunk' and selector_input is not None else None
+        fast = None
+        if mode == 'chunk' and selector_input is not None and getattr(self.select_ops, '__func__', None) is _SELECT_OPS:
+            fast = fast_front(self, 'gdn', hidden_states, cache, cu_seqlens)
         types = n_nats_blocks = None
         conv_states = cache.conv_state if cache is not None and cache.conv_state is not None else (None, None, None)
         if fast is not None:
@@ -308,3 +310,7 @@ class NeuralAttentionSearchLinearAttnGDN(nn.Module):
         o = self.o_norm(o_lin.reshape(o_attn.shape), o_attn, gate.reshape(o_attn.shape), o_mix)
         o = self.o_proj(o.flatten(-2))
         return o, None, past_key_values
+
+
+# the selector that the fused front contains; a layer whose select_ops is another one takes the general front, which calls it
+_SELECT_OPS = NeuralAttentionSearchLinearAttnGDN.select_ops

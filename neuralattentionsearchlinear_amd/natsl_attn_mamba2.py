@@ -183,7 +183,9 @@ class NeuralAttentionSearchLinearAttnMamba(nn.Module):
             if o is not None:
                 return o
         selector_input = cache.update_attn_types(input_hidden_states=hidden_states) if cache is not None else hidden_states
-        fast = fast_front(self, 'mamba', hidden_states, cache, cu_seqlens) if mode == 'chunk' and selector_input is not None else None
+        fast = None
+        if mode == 'chunk' and selector_input is not None and getattr(self.select_ops, '__func__', None) is _SELECT_OPS:
+            fast = fast_front(self, 'mamba', hidden_states, cache, cu_seqlens)
         types = n_nats_blocks = None
         conv_states = cache.conv_state if cache is not None and cache.conv_state is not None else (None, None, None)
         if fast is not None:
@@ -272,3 +274,7 @@ class NeuralAttentionSearchLinearAttnMamba(nn.Module):
         gate = self.g_proj(hidden_states).unflatten(-1, (-1, self.head_v_dim))
         o = self.o_norm(o_lin.reshape(o_attn.shape), o_attn, gate.reshape(o_attn.shape), o_mix)
         return self.o_proj(o.flatten(-2))
+
+
+# the selector that the fused front contains; a layer whose select_ops is another one takes the general front, which calls it
+_SELECT_OPS = NeuralAttentionSearchLinearAttnMamba.select_ops

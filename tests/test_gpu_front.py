@@ -61,6 +61,35 @@ def test_front_on_a_cache(kind, T0, sizes, monkeypatch):
     assert torch.equal(cf.n_attn_blocks, cs.n_attn_blocks)
 
 
+@pytest.mark.parametrize("kind", ['gdn', 'mamba'])
+@pytest.mark.parametrize("where", ['instance', 'subclass'])
+@pytest.mark.parametrize("train", [False, True])
+def test_an_overridden_selector_is_called(kind, where, train):
+    """A layer's select_ops decides in training and prefill too, also where a subclass or an instance has its own: here every block goes
+    to one operator, which the layer's own selector would not do."""
+    layer = _layer(kind, None, 'all')
+    own, calls = type(layer).select_ops, []
+
+    def only_linear(self, hidden_states, cu_seqlens=None, force_last_block=True):
+        calls.append(hidden_states.shape)
+        types, counts, last = own(self, hidden_states, cu_seqlens, force_last_block)
+        types, last = torch.zeros_like(types), torch.zeros_like(last)
+        types[..., 1] = last[..., 1] = 1
+        return types, counts, last
+    torch.manual_seed(4)
+    x = torch.randn(2, 8 * layer.nats_block_size, layer.hidden_size, device=DEV).bfloat16()
+    run = lambda: layer.train()(x) if train else _generate(layer.eval(), kind, x, x.shape[1], ())
+    run()
+    assert float(layer.attn_fraction.float().mean()) > 0.2           # (the layer's own choice)
+    if where == 'instance':
+        layer.select_ops = only_linear.__get__(layer)
+    else:
+        layer.__class__ = type('Other', (type(layer),), dict(select_ops=only_linear))
+    run()
+    assert calls == [x.shape]
+    assert torch.equal(layer.attn_fraction.float(), torch.full_like(layer.attn_fraction.float(), 1 / 8))     # the last block runs both
+
+
 @pytest.mark.parametrize("W,bias", [(4, False), (3, True), (2, False)])
 def test_conv_arithmetic_is_the_single_kernels(W, bias):
     """The fused convolution forms its activation, and the gradients behind it, with the arithmetic of natsl_short_conv_*: the same bits.

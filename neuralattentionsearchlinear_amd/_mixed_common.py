@@ -54,13 +54,14 @@ _SCAN_COLUMNS_PER_WG = 64           # state columns of the scans' widest workgro
 # What the differentiable operator keeps from its forward for the linear branch's backward.  Keeping means: the state entering
 # every chunk (bf16, K*V per chunk and head), v_new (64*V bf16) and the prep kernel's workspace (17 KiB) stay in device memory
 # until the backward, which then starts at its reverse scan - about 66 KiB per chunk and head at K = V = 128, 1.1 GB per call
-# at B8 T8192 H16 (a 24-layer model at the limit below keeps 24 of the card's 288 GB).  Not keeping means: only the inputs are saved and the backward runs the forward's two kernels once more, as
-# the reference's backward does (src/nats/ops/gated_delta_rule/chunk.py:170-332 recomputes h); a model that fits in memory
-# under the reference then fits here.  The gradients are the same bit for bit either way.
+# at B8 T8192 H16, for every layer of a model.  Not keeping means: only the inputs are saved and the backward runs the forward's two
+# kernels once more, as the reference's backward does (src/nats/ops/gated_delta_rule/chunk.py:170-332 recomputes h); a model that
+# fits in memory under the reference then fits here.  The gradients are the same bit for bit either way.  The default keeps what no
+# model misses (at most 1.5 GiB over 24 layers); more is the caller's trade and set by the caller.
 #   SAVE_CHUNK_STATES = None  (default) keep only when what would be kept is at most SAVE_CHUNK_STATES_MAX_BYTES per call
 #                     = True  always keep        = False  never keep
 SAVE_CHUNK_STATES = None
-SAVE_CHUNK_STATES_MAX_BYTES = 1 << 30
+SAVE_CHUNK_STATES_MAX_BYTES = 64 << 20
 _PREP_WORKSPACE_BYTES = 17 * 1024   # per chunk and head (csrc/natsl_linear.hip)
 
 

@@ -115,6 +115,9 @@ def test_chunk_state_saving_follows_the_byte_budget():
     try:
         MC.SAVE_CHUNK_STATES = None
         assert MC._keep_chunk_states(small, small, None) and not MC._keep_chunk_states(big, big, None)
+        # by default a layer's training step holds no more than 64 MiB per call that the backward could compute again: 340M geometry, 8 x 4096
+        assert not MC._keep_chunk_states(torch.empty(8, 4096, 6, 128, device='meta'), torch.empty(8, 4096, 6, 256, device='meta'), None)
+        assert MC.SAVE_CHUNK_STATES_MAX_BYTES == 64 << 20
         MC.SAVE_CHUNK_STATES = True
         assert MC._keep_chunk_states(big, big, None)
         MC.SAVE_CHUNK_STATES = False

@@ -433,6 +433,7 @@ def fast_front(layer, kind, x, cache, cu_seqlens):
         if torch.is_grad_enabled() and (x.requires_grad or any(t is not None and t.requires_grad for t in seen.tensors)):
             return None
         st = cache.conv_state
-        if st is not None and any(s is not None and (s.dtype != torch.bfloat16 or not s.is_contiguous() or s.shape[0] != x.shape[0]) for s in st):
+        if st is not None and any(s is not None and (s.dtype != torch.bfloat16 or not s.is_contiguous() or s.device != x.device or
+                                                     s.shape != (x.shape[0], f.w["conv_w" + n].shape[0], f.W)) for s, n in zip(st, "qkv")):
             return None
     return f

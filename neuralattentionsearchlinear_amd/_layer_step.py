@@ -204,8 +204,37 @@ class _Plan:
             s.l2_eps = layer.q_norm2.eps
         s.flags = flags
         self.device = params[0].device
-        self.conv_shapes = ((H * K, W), (H * K, W), (H * V, W))
+        # the cache's tensors as the kernels address them: (type, shape behind the batch); the attention keys and values by their rows
+        bs, bf16, f32 = layer.nats_block_size, torch.bfloat16, torch.float32
+        self.rows = ((HQ, KA), (HQ, VA))
+        self.buffers = [(bf16, (H * K, W)), (bf16, (H * K, W)), (bf16, (H * V, W)), (f32, (H, K, V)), (bf16, (bs, H, K)), (bf16, (bs, H, V)),
+                        (f32, (bs, H)), (bf16, (bs, D))] + [(bf16, (bs, H))] * delta
+        self.expected = {}
         self.built = True
+
+    def takes(self, cache, B, start):
+        """Whether the cache's tensors have the types, shapes and layouts that the kernels read and write (a cache filled under autocast
+        or by other code can hold others: the general path converts)."""
+        k, valid = cache.attn_k, cache.valid_attn_tokens
+        want = self.expected.get(B)
+        if want is None:
+            want = self.expected[B] = [(dt, (B, *tail)) for dt, tail in self.buffers]
+        have = [*cache.conv_state, cache.recurrent_state, cache.l_attn_k, cache.l_attn_v, cache.lattn_g, cache.block_type_state]
+        if self.fixed.is_delta:
+            have.append(cache.lattn_beta)
+        cap, HN, index = k.shape[1], self.fixed.HN, self.device.index
+        have += [k, cache.attn_v, valid]
+        want = want + [(torch.bfloat16, (B, cap, *self.rows[0])), (torch.bfloat16, (B, cap, *self.rows[1])), (torch.bool, (B, cap // self.fixed.block, HN))]
+        if start is not None:
+            have.append(start)
+            want.append(want[3])
+        g = cache.g_cumsum
+        if cap % self.fixed.block or len(have) != len(want) or (g is not None and (g.numel() != B * self.fixed.H or g.get_device() != index)):
+            return False
+        for t, (dtype, shape) in zip(have, want):
+            if t is None or t.dtype is not dtype or t.shape != shape or not t.is_contiguous() or t.get_device() != index:
+                return False
+        return True
 
 
 def layer_step(layer, kind, x, cache):
@@ -225,20 +254,16 @@ def layer_step(layer, kind, x, cache):
     bs, n_in, n_kept = cache.nats_block_size, cache._n_tokens_in_nats_block, cache.n_attn_blocks_max
     conv, state, start = cache.conv_state, cache.recurrent_state, cache.recurrent_state_block_start
     f = plan.fixed
-    if (cache.attn_k is None or cache.l_attn_k is None or cache.block_type_state is None or state is None or conv is None or
-            conv[0] is None or cache.valid_attn_tokens is None or bs != f.block or n_in + T > bs or x.device != plan.device or
-            cache.n_attn_blocks is None or (cache._linear_only == bool(f.flags & ATTN_OWN_BLOCK)) or cache.attn_k.dtype != torch.bfloat16 or
-            state.dtype != torch.float32 or cache.op_for_incomplete_chunk == 'attn'):
-        return None
-    for c, (ch, W) in zip(conv, plan.conv_shapes):
-        if c.dtype != torch.bfloat16 or c.shape != (B, ch, W) or not c.is_contiguous():
-            return None
-    if cache.attn_k.shape[0] != B or state.shape[0] != B or not state.is_contiguous():
+    if (cache.attn_k is None or state is None or conv is None or cache.valid_attn_tokens is None or bs != f.block or n_in + T > bs or
+            x.device != plan.device or cache.n_attn_blocks is None or (cache._linear_only == bool(f.flags & ATTN_OWN_BLOCK)) or
+            cache.op_for_incomplete_chunk == 'attn' or not plan.takes(cache, B, start)):
         return None
     types = None
     if n_in + T == bs:
         types, _, _ = layer.select_ops(cache.update_attn_types(input_hidden_states=x), None, force_last_block=False)
-        types = types.contiguous()
+        if types.shape != (B, 1, f.HN, 2) or types.device != x.device:
+            raise ValueError(f"select_ops must give types {(B, 1, f.HN, 2)} on {x.device}, got {tuple(types.shape)} on {types.device}")
+        types = (types if types.dtype in (torch.bfloat16, torch.float32) else types.float()).contiguous()
     if cache.attn_k.shape[1] < cache.n_attn_tokens_max + T:
         cache._grow(cache.n_attn_tokens_max + T)
     x = x.contiguous()

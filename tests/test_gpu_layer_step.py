@@ -116,6 +116,62 @@ def test_layer_step_forms_the_general_paths_gates(kind, float_gates, monkeypatch
         assert torch.equal(cf.lattn_beta[:, :n], cs.lattn_beta[:, :n]) and torch.equal(cf.lattn_beta[:, :n], cp.lattn_beta[:, :n])
 
 
+@pytest.mark.parametrize("kind", ['gdn', 'mamba'])
+def test_layer_step_after_a_prefill_under_autocast(kind, monkeypatch):
+    """fp32 hidden states under autocast leave a cache whose collected hidden states are fp32: bf16 steps on it fill it as the general
+    path does."""
+    from neuralattentionsearchlinear_amd import natsl_attn_gdn, natsl_attn_mamba2
+    layer = _layer(kind, None, 'all')
+    torch.manual_seed(6)
+    x = torch.randn(2, 75, layer.hidden_size, device=DEV)
+
+    def run():
+        from neuralattentionsearchlinear_amd.cache import NAtSCache, NAtSMamba2Cache
+        holder = NAtSCache() if kind == 'gdn' else NAtSMamba2Cache()
+        kw = dict(past_key_values=holder, use_cache=True) if kind == 'gdn' else dict(cache_params=holder, use_cache=True)
+        with torch.no_grad():
+            with torch.autocast('cuda', dtype=torch.bfloat16):
+                layer(x[:, :70], **kw)
+            outs = [layer(x[:, t:t + 1].bfloat16(), **kw) for t in range(70, 75)]
+        return [o[0] if isinstance(o, tuple) else o for o in outs], holder[0] if kind == 'gdn' else holder.nats_cache[0]
+    fast, cf = run()
+    for mod in (natsl_attn_gdn, natsl_attn_mamba2):
+        monkeypatch.setattr(mod, 'layer_step', lambda *a: None)
+    slow, cs = run()
+    assert cf.block_type_state.dtype == cs.block_type_state.dtype
+    n = cs._n_tokens_in_nats_block
+    assert n == 75 % layer.nats_block_size and torch.equal(cf.block_type_state[:, :n], cs.block_type_state[:, :n])
+    for a, b in zip(fast, slow):
+        assert rel_l2(a.float(), b.float()) <= 5e-3
+
+
+@pytest.mark.parametrize("name,change", [
+    ('block_type_state', 'float'), ('l_attn_k', 'float'), ('l_attn_v', 'float'), ('attn_v', 'float'), ('attn_k', 'half'), ('lattn_g', 'bfloat16'),
+    ('lattn_beta', 'float'), ('recurrent_state', 'bfloat16'), ('recurrent_state_block_start', 'bfloat16'), ('valid_attn_tokens', 'int'),
+    ('l_attn_k', 'short'), ('lattn_g', 'short'), ('attn_v', 'short'), ('valid_attn_tokens', 'short'), ('recurrent_state', 'strided'), ('attn_k', 'strided'),
+    ('g_cumsum', 'short'), ('conv_state', 'short')])
+def test_layer_step_declines_other_cache_tensors(name, change):
+    """A cache tensor of another type, shape or layout than the kernels address sends the step down the general path."""
+    import neuralattentionsearchlinear_amd._layer_step as LS
+    layer = _layer('gdn', None, 'all')
+    torch.manual_seed(7)
+    x = torch.randn(2, 102, 256, device=DEV).bfloat16()
+    with torch.no_grad():
+        _, cache = _generate(layer, 'gdn', x[:, :101], 100, (1,))
+        t = getattr(cache, name)
+        if change == 'short':
+            t = tuple(c[..., :2].contiguous() for c in t) if isinstance(t, tuple) else t[:, :-1].contiguous()
+        elif change == 'strided':
+            t = t.transpose(-1, -2).contiguous().transpose(-1, -2)
+        else:
+            t = getattr(t, change)()
+        own = getattr(cache, name)
+        setattr(cache, name, t)
+        assert LS.layer_step(layer, 'gdn', x[:, 101:], cache) is None
+        setattr(cache, name, own)
+        assert LS.layer_step(layer, 'gdn', x[:, 101:], cache) is not None
+
+
 def test_layer_step_follows_replaced_weights_and_declines_hooks():
     """The step reads the layer's current parameters, and a hooked submodule sends the layer down the general path."""
     import neuralattentionsearchlinear_amd._layer_step as LS

@@ -14,7 +14,7 @@ import torch
 import torch.nn.functional as F
 
 from . import _capi
-from ._layer_step import _PARAMS, watch
+from ._layer_step import _PARAMS, watch, weight_shapes
 from .modules import _NORM_GATE_WIDTHS
 
 _NAMES = [p[0] for p in _PARAMS]
@@ -388,7 +388,7 @@ class FastFront:
 
 def _front_plan(layer, kind, seen):
     """The layer's FastFront, or None where its weights or options are not what the fused steps are built for."""
-    w = dict(zip(_NAMES, seen.tensors))
+    w, shapes = dict(zip(_NAMES, seen.tensors)), weight_shapes(layer)
     delta = kind == 'gdn'
     if not layer.use_short_conv or layer.num_v_heads != layer.num_heads or layer.attn_with_short_conv != delta or (delta and not layer.attn_qk_norm):
         return None
@@ -397,7 +397,7 @@ def _front_plan(layer, kind, seen):
             if n.startswith("conv_b") or (not delta and n in ("wb", "norm_q", "norm_k")):
                 continue
             return None
-        if not t.is_cuda or t.device != w["wq"].device or not t.is_contiguous() or \
+        if not t.is_cuda or t.device != w["wq"].device or not t.is_contiguous() or t.shape != shapes[n] or \
                 (t.dtype != torch.bfloat16 and (n not in _EITHER or t.dtype != torch.float32)):
             return None
     if w["a_log"].dtype != w["dt_bias"].dtype or w["out_norm1"].dtype != w["out_norm2"].dtype or (delta and w["norm_q"].dtype != w["norm_k"].dtype):

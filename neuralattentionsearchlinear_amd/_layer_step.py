@@ -63,7 +63,18 @@ _OPTIONS = ("hidden_size", "head_k_dim", "head_v_dim", "head_attn_k_dim", "head_
             "allow_neg_eigval", "decay_for_non_gdn_blocks", "decay_for_non_mamba_blocks", "value_dim")
 _SUB_OPTIONS = ("eps", "kernel_size", "activation")
 _SUBMODULES = tuple((p[1], p[3]) for p in _PARAMS if p[1] is not None and p[3] is not None) + (("q_norm2", L2Norm), ("k_norm2", L2Norm))
-_dtype_of = operator.attrgetter('dtype')
+_dtype_of, _shape_of = operator.attrgetter('dtype'), operator.attrgetter('shape')
+
+
+def weight_shapes(layer):
+    """The weights' shapes under the layer's options, by field: what the kernels address.  A layer with others (a replaced projection, a
+    pruned head) is left to its submodules, which take or refuse them."""
+    D, qk, vd, H, W = layer.hidden_size, layer.num_heads * layer.head_k_dim, layer.value_dim, layer.num_heads, layer.conv_size
+    s = dict(wq=(qk, D), wk=(qk, D), wv=(vd, D), wg=(vd, D), wa=(H, D), wb=(H, D), w_mix=(2 * layer.num_attn_heads, qk), wo=(D, vd),
+             conv_wq=(qk, 1, W), conv_wk=(qk, 1, W), conv_wv=(vd, 1, W), conv_bq=(qk,), conv_bk=(qk,), conv_bv=(vd,), a_log=(H,), dt_bias=(H,))
+    s["norm_q"] = s["norm_k"] = (layer.head_attn_k_dim,)
+    s["out_norm1"] = s["out_norm2"] = (layer.head_attn_v_dim,)
+    return s
 
 
 class _Watch:
@@ -98,7 +109,7 @@ class _Watch:
 
     def _layouts(self):
         w = self.weights
-        return [*map(torch.Tensor.data_ptr, w), *map(_dtype_of, w), *map(torch.Tensor.is_contiguous, w), *map(torch.Tensor.numel, w)]
+        return [*map(torch.Tensor.data_ptr, w), *map(_dtype_of, w), *map(torch.Tensor.is_contiguous, w), *map(_shape_of, w)]
 
     @staticmethod
     def _read(where, names):
@@ -155,7 +166,7 @@ class _Plan:
         self.ws_bytes = {}
         params = seen.tensors
         s = self.fixed = LayerStep()
-        by = dict(zip((p[0] for p in _PARAMS), params))
+        by, shapes = dict(zip((p[0] for p in _PARAMS), params)), weight_shapes(layer)
         delta = kind == 'gdn'
         K, V, H, HQ = layer.head_k_dim, layer.head_v_dim, layer.num_heads, layer.num_attn_heads
         for n, t in by.items():
@@ -163,7 +174,7 @@ class _Plan:
                 if n not in _OPTIONAL or (n == "wb" and delta) or (n in ("norm_q", "norm_k") and layer.attn_qk_norm):
                     return
                 continue
-            if not (t.is_cuda and t.is_contiguous() and t.device == params[0].device and
+            if not (t.is_cuda and t.is_contiguous() and t.device == params[0].device and t.shape == shapes[n] and
                     (t.dtype == torch.bfloat16 or (n in _EITHER_DTYPE and t.dtype == torch.float32))):
                 return
             setattr(s, n, t.data_ptr())
@@ -173,7 +184,7 @@ class _Plan:
         if not layer.use_short_conv or layer.num_v_heads != H or layer.ops_for_incomplete_chunks == 'attn':
             return
         convs = [layer.q_conv1d, layer.k_conv1d, layer.v_conv1d]
-        W, act = convs[0].kernel_size[0], convs[0].activation
+        W, act = layer.conv_size, convs[0].activation
         if any(c.kernel_size[0] != W or (c.activation is None) != (act is None) for c in convs) or W not in (2, 3, 4):
             return
         if any(layer._modules[m].bias is not None for m in ("q_proj", "k_proj", "v_proj", "g_proj", "a_proj", "nats_out_weights_layer", "o_proj")) \

@@ -188,3 +188,24 @@ def test_layer_step_follows_replaced_weights_and_declines_hooks():
         layer.o_proj.weight = torch.nn.Parameter(torch.zeros_like(layer.o_proj.weight))
         out = LS.layer_step(layer, 'gdn', x[:, 101:102], cache)
     assert float(out.abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("where,shape", [('o_proj.weight', (128, 512)), ('v_proj.weight', (256, 512)), ('A_log', (1,)), ('dt_bias', (1,)),
+                                         ('o_norm.weight1', (64,)), ('k_conv1d.weight', (256, 1, 3)), ('q_norm.weight', (1,)),
+                                         ('nats_out_weights_layer.weight', (256, 8))])
+def test_layer_step_and_front_decline_other_weight_shapes(where, shape):
+    """A weight of another shape than the layer's options say is left to the submodules: the kernels would address the options' shape."""
+    import neuralattentionsearchlinear_amd._layer_step as LS
+    from neuralattentionsearchlinear_amd._front import fast_front
+    layer = _layer('gdn', None, 'all')
+    torch.manual_seed(8)
+    x = torch.randn(2, 102, 256, device=DEV).bfloat16()
+    with torch.no_grad():
+        _, cache = _generate(layer, 'gdn', x[:, :100], 100, ())
+        assert fast_front(layer, 'gdn', x, None, None) is not None
+        assert LS.layer_step(layer, 'gdn', x[:, 100:101], cache) is not None
+        p = layer.get_parameter(where)
+        assert p.shape != shape
+        p.data = torch.zeros(shape, dtype=p.dtype, device=DEV)
+        assert LS.layer_step(layer, 'gdn', x[:, 101:], cache) is None
+        assert fast_front(layer, 'gdn', x, None, None) is None

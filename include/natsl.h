@@ -452,7 +452,8 @@ int natsl_wgrad(const natsl_wgrad_seg* segs, int n_seg, const void* x, int64_t T
  * arguments those take, in bf16, and in front of and behind them the conversions of fp32 tensors (cast_in: fp32 -> bf16,
  * cast_out: bf16 -> fp32; tensors on 16 bytes).  `phases` says which steps to enqueue, so that a caller can time them one by
  * one.  attn_stream carries routing and the softmax branch: the same stream, or another one, which is then made to wait for
- * `stream` before (at ROUTE) and waited for after (at JOIN).  The attention view may hold other lengths (a prefix of cached
+ * `stream` before (at ROUTE) and waited for after (at JOIN).  Both belong to one device, which need not be the caller's current one.
+ * The attention view may hold other lengths (a prefix of cached
  * keys): T_attn tokens in TN_attn blocks. */
 #define NATSL_MIXED_CASTS 8
 enum natsl_mixed_phases { NATSL_MIXED_CONVERT = 1, NATSL_MIXED_ROUTE = 2, NATSL_MIXED_SOFTMAX = 4, NATSL_MIXED_LINEAR = 8, NATSL_MIXED_JOIN = 16 };

@@ -64,8 +64,30 @@ static int cast_all(const natsl_cast* seg, int n, hipStream_t s, const char* wha
   return check_launch(what);
 }
 
-// `to` waits for what `from` holds so far.  One event per device; a wait takes the event's state at the call, so the pair is
-// made under a lock and the event can serve the next pair at once.
+// The streams' device is the current one while a call runs: events, kernel attributes and null handles go by the current device, and
+// the caller's may be another.
+class OnDeviceOf {
+  int before = -1;
+
+ public:
+  int enter(const hipStream_t a, const hipStream_t b, const char* what) {
+    int now = 0, dev = 0, other = 0;
+    hipError_t e = hipGetDevice(&now);
+    dev = now;
+    if (e == hipSuccess && (a || b)) e = hipStreamGetDevice(a ? a : b, &dev);
+    other = dev;
+    if (e == hipSuccess && a && b) e = hipStreamGetDevice(b, &other);
+    if (e == hipSuccess && other != dev) return fail(NATSL_ERR_INVALID, "%s: streams of devices %d and %d", what, dev, other);
+    if (e == hipSuccess && dev != now && (e = hipSetDevice(dev)) == hipSuccess) before = now;
+    return e == hipSuccess ? NATSL_OK : fail(NATSL_ERR_LAUNCH, "%s: cannot enter the streams' device (%s)", what, hipGetErrorString(e));
+  }
+  ~OnDeviceOf() {
+    if (before >= 0) (void)hipSetDevice(before);
+  }
+};
+
+// `to` waits for what `from` holds so far (both of the current device).  One event per device; a wait takes the event's state at the
+// call, so the pair is made under a lock and the event can serve the next pair at once.
 static int order_streams(hipStream_t from, hipStream_t to, const char* what) {
   constexpr int MAX_DEVICES = 64;
   static hipEvent_t events[MAX_DEVICES];
@@ -91,7 +113,9 @@ extern "C" int natsl_mixed_fwd(const natsl_mixed* m, int phases, natsl_stream_t 
     return fail(NATSL_ERR_INVALID, "%s: conversion counts", what);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream), side = reinterpret_cast<hipStream_t>(attn_stream);
   const bool fork = side != s;
-  int rc = NATSL_OK;
+  OnDeviceOf device;
+  int rc = device.enter(s, side, what);
+  if (rc != NATSL_OK) return rc;
   if ((phases & NATSL_MIXED_CONVERT) && (rc = cast_all<true>(m->cast_in, m->n_cast_in, s, what)) != NATSL_OK) return rc;
   if (phases & NATSL_MIXED_ROUTE) {
     if (fork && (rc = order_streams(s, side, what)) != NATSL_OK) return rc;

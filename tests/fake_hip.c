@@ -1,0 +1,62 @@
+/* A HIP runtime that launches nothing: it notes the calls that order streams, and holds them to the rules a real one has (an event is
+ * recorded on a stream of its own device).  A stream handle's device is its bits 12 and up; the null stream is the current device's. */
+#include <stdarg.h>
+#include <stdio.h>
+#include <string.h>
+
+static char notes[1 << 16];
+static size_t used;
+static int current, next_event;
+static int event_device[256];
+
+static void note(const char* fmt, ...) {
+  va_list ap;
+  va_start(ap, fmt);
+  if (used < sizeof(notes) - 256) used += vsnprintf(notes + used, 256, fmt, ap);
+  va_end(ap);
+}
+static int device_of(const void* s) { return s ? (int)((size_t)s >> 12) : current; }
+
+const char* fake_notes(void) { return notes; }
+void fake_reset(int device) { used = 0; notes[0] = 0; current = device; }
+int fake_current(void) { return current; }
+
+int hipGetDevice(int* d) { *d = current; return 0; }
+int hipSetDevice(int d) { current = d; return 0; }
+int hipStreamGetDevice(void* s, int* d) { *d = device_of(s); return 0; }
+int hipEventCreateWithFlags(void** e, unsigned flags) {
+  (void)flags;
+  event_device[++next_event] = current;
+  *e = (void*)(size_t)next_event;
+  return 0;
+}
+int hipEventRecord(void* e, void* s) {
+  note("record %lx ", (unsigned long)(size_t)s);
+  return event_device[(size_t)e] == device_of(s) ? 0 : 400;   /* hipErrorInvalidHandle */
+}
+int hipStreamWaitEvent(void* s, void* e, unsigned flags) {
+  (void)e; (void)flags;
+  note("wait %lx ", (unsigned long)(size_t)s);
+  return 0;
+}
+typedef struct { unsigned x, y, z; } dim3_t;
+static struct { dim3_t grid, block; size_t lds; void* stream; } config;
+int __hipPushCallConfiguration(dim3_t grid, dim3_t block, size_t lds, void* s) {
+  config.grid = grid; config.block = block; config.lds = lds; config.stream = s;
+  return 0;
+}
+int __hipPopCallConfiguration(dim3_t* grid, dim3_t* block, size_t* lds, void** s) {
+  *grid = config.grid; *block = config.block; *lds = config.lds; *s = config.stream;
+  return 0;
+}
+int hipLaunchKernel(const void* f, dim3_t grid, dim3_t block, void** args, size_t lds, void* s) {
+  (void)f; (void)grid; (void)block; (void)args; (void)lds;
+  note("launch %lx:%d ", (unsigned long)(size_t)s, current);
+  return 0;
+}
+int hipFuncSetAttribute(const void* f, int attr, int value) { (void)f; (void)attr; (void)value; return 0; }
+int hipDeviceGetAttribute(int* v, int attr, int d) { (void)attr; (void)d; *v = 256; return 0; }
+int hipGetDevicePropertiesR0600(void* p, int d) { (void)p; (void)d; return 1; }
+int hipGetSymbolAddress(void** p, const void* symbol) { (void)symbol; *p = (void*)4096; return 0; }
+int hipGetLastError(void) { return 0; }
+const char* hipGetErrorString(int e) { return e ? "an error" : "none"; }

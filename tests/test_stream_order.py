@@ -1,0 +1,64 @@
+"""CPU-only: how the mixed operator's native call orders its two streams, run against a HIP runtime that launches nothing
+(tests/fake_hip.c) in a process of its own."""
+import json
+import os
+import re
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CONVERT, ROUTE, SOFTMAX, LINEAR, JOIN = 1, 2, 4, 8, 16
+ALL = CONVERT | ROUTE | SOFTMAX | LINEAR | JOIN
+CHILD = """
+import ctypes, json, sys
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+fake.fake_notes.restype = ctypes.c_char_p
+lib = ctypes.CDLL(sys.argv[2])
+call, out = ctypes.create_string_buffer(bytes.fromhex(sys.argv[3])), []
+for phases, stream, side, current in json.loads(sys.argv[4]):
+    fake.fake_reset(current)
+    rc = lib.natsl_mixed_fwd(call, phases, ctypes.c_void_p(stream), ctypes.c_void_p(side))
+    out.append([rc, fake.fake_notes().decode().strip(), fake.fake_current()])
+print(json.dumps(out))
+"""
+
+
+@pytest.fixture(scope="module")
+def fake_hip(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", os.path.join(HERE, "fake_hip.c"), "-o", lib], check=True)
+    return lib
+
+
+def _run(fake_hip, calls, **fields):
+    """[(return code, what was launched and ordered, the current device afterwards)] of calls (phases, stream, side, current device)."""
+    from neuralattentionsearchlinear_amd import _build, _capi
+    from neuralattentionsearchlinear_amd._mixed_common import _POINTERS, _Mixed
+    if not os.path.exists(_capi.LIB_PATH):
+        _build.build()
+    m = _Mixed()
+    for name in _POINTERS:
+        setattr(m, name, 1 << 20)
+    m.h0 = m.ht = m.h_block_start = m.g_block_sum = m.chunk_states = m.chunk_v_new = None
+    size = dict(is_delta=1, B=1, T=256, H=2, HN=2, K=64, V=64, TN=4, block=64, flags=7, T_attn=256, TN_attn=4, HQ=2, HKV=2, KA=64, VA=64,
+                same_block_visible=1, types_dtype=_capi.BF16, scale_attn=0.1, scale_linear=0.1, workspace_bytes=1 << 30)
+    for name, value in dict(size, **fields).items():
+        setattr(m, name, value)
+    r = subprocess.run([sys.executable, "-c", CHILD, fake_hip, _capi.LIB_PATH, bytes(m).hex(), json.dumps(calls)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    return json.loads(r.stdout)
+
+
+def test_streams_are_ordered_on_their_own_device(fake_hip):
+    """The caller's current device may be another than the streams': the call enters theirs and leaves the caller's as it was."""
+    calls = [(ALL, 0x2001, 0x2002, 0), (ALL, 0x1001, 0x1002, 1), (ALL, 0, 0x3002, 0), (ALL, 0x2001, 0x2001, 0)]
+    for (_, stream, side, current), (rc, notes, after) in zip(calls, _run(fake_hip, calls)):
+        device = (side or stream) >> 12
+        assert rc == 0 and after == current
+        launched = re.findall(r"launch (\w+):(\d+)", notes)
+        assert {int(s, 16) for s, _ in launched} == {stream, side} and {int(d) for _, d in launched} == {device}, notes
+        if side != stream:
+            assert notes.startswith(f"record {stream:x} wait {side:x} ") and notes.endswith(f"record {side:x} wait {stream:x}"), notes
+    assert _run(fake_hip, [(ALL, 0x1001, 0x2001, 0)])[0][0] == -1                    # streams of two devices

@@ -106,19 +106,15 @@ static int order_streams(hipStream_t from, hipStream_t to, const char* what) {
 
 using namespace natsl;
 
-extern "C" int natsl_mixed_fwd(const natsl_mixed* m, int phases, natsl_stream_t stream, natsl_stream_t attn_stream) {
-  const char* what = "natsl_mixed_fwd";
-  if (!m) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
-  if (m->n_cast_in < 0 || m->n_cast_in > NATSL_MIXED_CASTS || m->n_cast_out < 0 || m->n_cast_out > NATSL_MIXED_CASTS)
-    return fail(NATSL_ERR_INVALID, "%s: conversion counts", what);
+// What natsl_mixed_fwd enqueues, on the streams' device; forked: the side stream may hold work that nothing waits for yet.
+static int mixed_phases(const natsl_mixed* m, const int phases, natsl_stream_t stream, natsl_stream_t attn_stream, bool& forked, const char* what) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream), side = reinterpret_cast<hipStream_t>(attn_stream);
   const bool fork = side != s;
-  OnDeviceOf device;
-  int rc = device.enter(s, side, what);
-  if (rc != NATSL_OK) return rc;
+  int rc = NATSL_OK;
   if ((phases & NATSL_MIXED_CONVERT) && (rc = cast_all<true>(m->cast_in, m->n_cast_in, s, what)) != NATSL_OK) return rc;
   if (phases & NATSL_MIXED_ROUTE) {
     if (fork && (rc = order_streams(s, side, what)) != NATSL_OK) return rc;
+    forked = fork;
     rc = natsl_route(m->types_attn, m->types_dtype, m->B, m->TN_attn, m->HN, m->T_attn, m->block, m->block_indices, m->n_blocks, nullptr, nullptr,
                      nullptr, nullptr, m->seqs, m->n_seqs, 0, attn_stream);
     if (rc != NATSL_OK) return rc;
@@ -144,7 +140,24 @@ extern "C" int natsl_mixed_fwd(const natsl_mixed* m, int phases, natsl_stream_t 
   if (both && (rc = softmax()) != NATSL_OK) return rc;
   if (phases & NATSL_MIXED_JOIN) {
     if (fork && (rc = order_streams(side, s, what)) != NATSL_OK) return rc;
+    forked = false;
     rc = cast_all<false>(m->cast_out, m->n_cast_out, s, what);
   }
+  return rc;
+}
+
+extern "C" int natsl_mixed_fwd(const natsl_mixed* m, int phases, natsl_stream_t stream, natsl_stream_t attn_stream) {
+  const char* what = "natsl_mixed_fwd";
+  if (!m) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
+  if (m->n_cast_in < 0 || m->n_cast_in > NATSL_MIXED_CASTS || m->n_cast_out < 0 || m->n_cast_out > NATSL_MIXED_CASTS)
+    return fail(NATSL_ERR_INVALID, "%s: conversion counts", what);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream), side = reinterpret_cast<hipStream_t>(attn_stream);
+  OnDeviceOf device;
+  int rc = device.enter(s, side, what);
+  if (rc != NATSL_OK) return rc;
+  bool forked = side != s && !(phases & NATSL_MIXED_ROUTE);      // (by an earlier call)
+  rc = mixed_phases(m, phases, stream, attn_stream, forked, what);
+  // after an error too the caller may free what the side stream works on, as soon as its own stream allows
+  if (rc != NATSL_OK && forked) (void)order_streams(side, s, what);
   return rc;
 }

@@ -62,3 +62,20 @@ def test_streams_are_ordered_on_their_own_device(fake_hip):
         if side != stream:
             assert notes.startswith(f"record {stream:x} wait {side:x} ") and notes.endswith(f"record {side:x} wait {stream:x}"), notes
     assert _run(fake_hip, [(ALL, 0x1001, 0x2001, 0)])[0][0] == -1                    # streams of two devices
+
+
+@pytest.mark.parametrize("fields", [dict(K=96), dict(VA=96), dict(HQ=3), dict(workspace_bytes=16)])
+def test_an_error_leaves_nothing_unwaited_on_the_side_stream(fake_hip, fields):
+    """What the side stream got before a branch refused its arguments is waited for by the caller's stream all the same: the caller
+    frees what it works on."""
+    s, side = 0x1001, 0x1002
+    steps = [(ALL, s, side, 1), (CONVERT | ROUTE, s, side, 1), (SOFTMAX | LINEAR, s, side, 1), (CONVERT | ROUTE | SOFTMAX, s, side, 1), (LINEAR, s, side, 1)]
+    failed = 0
+    for rc, notes, _ in _run(fake_hip, steps, **fields):
+        if rc != 0:
+            failed += 1
+            assert notes.endswith(f"record {side:x} wait {s:x}"), notes
+    assert failed >= 2
+    # on one stream there is nothing to wait for
+    rc, notes, _ = _run(fake_hip, [(ALL, s, s, 1)], **fields)[0]
+    assert rc != 0 and "wait" not in notes

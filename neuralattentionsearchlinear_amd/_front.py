@@ -331,21 +331,11 @@ class _Select(torch.autograd.Function):
 
 
 class FastFront:
-    """A layer's parameters and constants, as long as it holds these parameters (_layer_step.watch)."""
+    """A layer's parameters at one forward, with the constants of its plan.  (The plan, which outlives the forward, holds no tensor.)"""
 
-    def __init__(self, layer, kind, params):
-        self.w = w = dict(zip(_NAMES, params))
-        self.delta = kind == 'gdn'
-        self.H, self.W = layer.num_heads, layer.conv_size
-        self.act = 0 if layer.q_conv1d.activation is None else 1
-        self.l2 = not self.delta
-        self.raw_attention = not self.delta
-        self.norm_width = layer.head_attn_k_dim if self.delta else layer.head_k_dim
-        self.front_eps = layer.q_norm.eps if self.delta else layer.q_norm2.eps
-        self.norm_dtype = _capi.dtype_code(w["norm_q"].dtype) if self.delta else _capi.BF16
-        self.gate_dtype, self.out_dtype = _capi.dtype_code(w["a_log"].dtype), _capi.dtype_code(w["out_norm1"].dtype)
-        self.neg = int(self.delta and layer.allow_neg_eigval)
-        self.out_eps = layer.o_norm.eps
+    def __init__(self, constants, w):
+        self.__dict__.update(constants)
+        self.w = w
 
     def grad(self, *tensors):
         return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
@@ -386,9 +376,9 @@ class FastFront:
         return linear(y.flatten(-2), self.w["wo"])
 
 
-def _front_plan(layer, kind, seen):
-    """The layer's FastFront, or None where its weights or options are not what the fused steps are built for."""
-    w, shapes = dict(zip(_NAMES, seen.tensors)), weight_shapes(layer)
+def _front_plan(layer, kind, w):
+    """A FastFront's constants, or None where the layer's weights (by field) or options are not what the fused steps are built for."""
+    shapes = weight_shapes(layer)
     delta = kind == 'gdn'
     if not layer.use_short_conv or layer.num_v_heads != layer.num_heads or layer.attn_with_short_conv != delta or (delta and not layer.attn_qk_norm):
         return None
@@ -413,7 +403,10 @@ def _front_plan(layer, kind, seen):
     if norms[0].eps != norms[1].eps or width not in (32, 64, 128, 256, 512) or layer.head_attn_v_dim not in _NORM_GATE_WIDTHS or \
             layer.hidden_size % 8 or layer.num_heads > 256 or layer.value_dim % 8:
         return None
-    return FastFront(layer, kind, seen.tensors)
+    code = lambda n: _capi.dtype_code(w[n].dtype)
+    return dict(delta=delta, H=layer.num_heads, W=layer.conv_size, act=0 if layer.q_conv1d.activation is None else 1, l2=not delta,
+                raw_attention=not delta, norm_width=width, front_eps=norms[0].eps, norm_dtype=code("norm_q") if delta else _capi.BF16,
+                gate_dtype=code("a_log"), out_dtype=code("out_norm1"), neg=int(delta and layer.allow_neg_eigval), out_eps=layer.o_norm.eps)
 
 
 def fast_front(layer, kind, x, cache, cu_seqlens):
@@ -424,13 +417,15 @@ def fast_front(layer, kind, x, cache, cu_seqlens):
     seen = watch(layer)
     if seen is None:
         return None
+    w = dict(zip(_NAMES, seen.weights(layer)))
     if seen.front_plan is None:
-        seen.front_plan = (_front_plan(layer, kind, seen),)
-    f = seen.front_plan[0]
-    if f is None or f.w["wq"].device != x.device:
+        seen.front_plan = (_front_plan(layer, kind, w),)
+    constants = seen.front_plan[0]
+    if constants is None or w["wq"].device != x.device:
         return None
+    f = FastFront(constants, w)
     if cache is not None:
-        if torch.is_grad_enabled() and (x.requires_grad or any(t is not None and t.requires_grad for t in seen.tensors)):
+        if torch.is_grad_enabled() and (x.requires_grad or any(t is not None and t.requires_grad for t in w.values())):
             return None
         st = cache.conv_state
         if st is not None and any(s is not None and (s.dtype != torch.bfloat16 or not s.is_contiguous() or s.device != x.device or

@@ -62,7 +62,8 @@ _OPTIONS = ("hidden_size", "head_k_dim", "head_v_dim", "head_attn_k_dim", "head_
             "num_nats_head", "nats_block_size", "ops_for_incomplete_chunks", "use_short_conv", "conv_size", "attn_with_short_conv", "attn_qk_norm",
             "allow_neg_eigval", "decay_for_non_gdn_blocks", "decay_for_non_mamba_blocks", "value_dim")
 _SUB_OPTIONS = ("eps", "kernel_size", "activation")
-_SUBMODULES = tuple((p[1], p[3]) for p in _PARAMS if p[1] is not None and p[3] is not None) + (("q_norm2", L2Norm), ("k_norm2", L2Norm))
+_SUBMODULES = tuple({p[1]: p[3] for p in _PARAMS if p[1] is not None and p[3] is not None}.items()) + (("q_norm2", L2Norm), ("k_norm2", L2Norm))
+_PLAIN_TENSORS = {nn.Parameter, torch.Tensor}
 _dtype_of, _shape_of = operator.attrgetter('dtype'), operator.attrgetter('shape')
 
 
@@ -78,73 +79,78 @@ def weight_shapes(layer):
 
 
 class _Watch:
-    """A layer's weight tensors by field, and a quick way to see that what the plans were made from still holds: the same
-    submodules with the same options, holding the same tensors at the same addresses in the same types and layouts."""
+    """What a layer's plans were made from besides its weights' values: which weights and plain submodules it has, the options, and the
+    weights' addresses, types and layouts.  No tensor or module is held: a replaced weight is freed when its owner lets go of it."""
 
     def __init__(self, layer):
         mods = layer._modules
-        self.mods = [(n, mods.get(n)) for n, _ in _SUBMODULES]
-        self.plain = all(m is None or type(m) is kind for (_, m), (_, kind) in zip(self.mods, _SUBMODULES))
-        self.tensors, self.held = [], []
-        for _, mod, name, _ in _PARAMS:
-            m = layer if mod is None else mods.get(mod)
-            t = None if m is None else m._parameters.get(name)
-            self.tensors.append(t)
-            if m is not None:
-                self._hold(m._parameters, name, t)
-            if type(m) is nn.Linear:
-                self._hold(m._parameters, 'bias', m.bias)
-        self.options = [(layer.__dict__, _OPTIONS, self._read(layer.__dict__, _OPTIONS))]
-        self.hooks = []
-        for _, m in self.mods:
-            if m is not None:
-                d = m.__dict__
-                names = tuple(n for n in _SUB_OPTIONS if n in d)
-                if names:
-                    self.options.append((d, names, self._read(d, names)))
-                self.hooks.append((m._forward_hooks, m._forward_pre_hooks, m._backward_hooks, m._backward_pre_hooks, d))
-        self.weights = [t for _, _, t in self.held if t is not None]
-        self.layouts = self._layouts() if self.plain else None
+        self.parts, weights, self.plain = [], [], True     # parts: (name, type or None, [(parameter, whether there is one)], options, their values)
+        for n, kind in _SUBMODULES:
+            m = mods.get(n)
+            if m is None:
+                self.parts.append((n, None, (), (), ()))
+                continue
+            self.plain &= type(m) is kind
+            names = {p[2] for p in _PARAMS if p[1] == n} | ({'bias'} if kind is nn.Linear else set())
+            d = m.__dict__
+            options = tuple(o for o in _SUB_OPTIONS if o in d)
+            self.parts.append((n, type(m), self._params(m, sorted(names), weights), options, tuple(map(d.get, options))))
+        self.own = self._params(layer, sorted(p[2] for p in _PARAMS if p[1] is None), weights)
+        self.options = tuple(map(layer.__dict__.get, _OPTIONS))
+        self.plain &= set(map(type, weights)) <= _PLAIN_TENSORS
+        self.layouts = self._layouts(weights) if self.plain else None
         self.step_plan = self.front_plan = None
 
-    def _layouts(self):
-        w = self.weights
-        return [*map(torch.Tensor.data_ptr, w), *map(_dtype_of, w), *map(torch.Tensor.is_contiguous, w), *map(_shape_of, w)]
+    @staticmethod
+    def _params(m, names, weights):
+        held = [(n, m._parameters.get(n)) for n in names]
+        weights += [t for _, t in held if t is not None]
+        return tuple((n, t is not None) for n, t in held)
 
     @staticmethod
-    def _read(where, names):
-        return tuple(map(where.get, names))
+    def _layouts(w):
+        return [*map(torch.Tensor.data_ptr, w), *map(_dtype_of, w), *map(torch.Tensor.is_contiguous, w), *map(_shape_of, w)]
 
-    def _hold(self, where, name, t):
-        if t is None:
-            self.held.append((where, name, None))
-        elif type(t) not in (nn.Parameter, torch.Tensor):
-            self.plain = False
-        else:
-            self.held.append((where, name, t))
+    def weights(self, layer):
+        """The weights by field, None where the layer has none."""
+        mods, out = layer._modules, []
+        for _, mod, name, _ in _PARAMS:
+            m = layer if mod is None else mods.get(mod)
+            out.append(None if m is None else m._parameters.get(name))
+        return out
 
     def holds(self, layer):
-        mods = layer._modules
-        for n, m in self.mods:
-            if mods.get(n) is not m:
-                return False
-        for where, name, t in self.held:
-            if where.get(name) is not t:
-                return False
-        if self._layouts() != self.layouts:
-            return False
-        for where, names, values in self.options:
-            if tuple(map(where.get, names)) != values:
-                return False
-        return True
-
-    def hooked(self):
-        if _has_any_global_hook():
-            return True
-        for a, b, c, e, d in self.hooks:
-            if a or b or c or e or 'forward' in d:
-                return True
-        return False
+        """-> (whether nothing has changed, whether a submodule has a hook or a forward of its own)"""
+        mods, weights, hooked = layer._modules, [], False
+        for n, kind, params, options, values in self.parts:
+            m = mods.get(n)
+            if m is None or kind is None:
+                if m is not None or kind is not None:
+                    return False, False
+                continue
+            if type(m) is not kind:
+                return False, False
+            d = m.__dict__
+            held = d['_parameters']
+            for name, there in params:
+                t = held.get(name)
+                if (t is not None) is not there:
+                    return False, False
+                if there:
+                    weights.append(t)
+            if options and tuple(map(d.get, options)) != values:
+                return False, False
+            if d['_forward_hooks'] or d['_forward_pre_hooks'] or d['_backward_hooks'] or d['_backward_pre_hooks'] or 'forward' in d:
+                hooked = True
+        held = layer._parameters
+        for name, there in self.own:
+            t = held.get(name)
+            if (t is not None) is not there:
+                return False, False
+            if there:
+                weights.append(t)
+        return (tuple(map(layer.__dict__.get, _OPTIONS)) == self.options and set(map(type, weights)) <= _PLAIN_TENSORS and
+                self._layouts(weights) == self.layouts), hooked
 
 
 def watch(layer):
@@ -153,9 +159,11 @@ def watch(layer):
     if torch.autograd.forward_ad._current_level >= 0:
         return None
     w = _watches.get(layer)
-    if w is None or not w.holds(layer):
+    same, hooked = (False, False) if w is None else w.holds(layer)
+    if not same:
         w = _watches[layer] = _Watch(layer)
-    return None if not w.plain or w.hooked() else w
+        hooked = w.holds(layer)[1] if w.plain else False
+    return None if not w.plain or hooked or _has_any_global_hook() else w
 
 
 class _Plan:
@@ -164,7 +172,7 @@ class _Plan:
     def __init__(self, layer, kind, seen):
         self.built = False
         self.ws_bytes = {}
-        params = seen.tensors
+        params = seen.weights(layer)
         s = self.fixed = LayerStep()
         by, shapes = dict(zip((p[0] for p in _PARAMS), params)), weight_shapes(layer)
         delta = kind == 'gdn'

@@ -157,3 +157,23 @@ def test_layer_plans_notice_every_change():
     assert watch(layer) is None
     handle.remove()
     assert watch(layer) is seen
+
+
+def test_layer_plans_keep_nothing_alive():
+    """What is remembered about a layer frees a replaced weight or submodule at once."""
+    import gc
+    import weakref
+    import torch
+    from neuralattentionsearchlinear_amd._layer_step import watch
+    from neuralattentionsearchlinear_amd.natsl_attn_mamba2 import NeuralAttentionSearchLinearAttnMamba
+    layer = NeuralAttentionSearchLinearAttnMamba(hidden_size=64, expand_v=1, head_dim=64, num_heads=2, num_attn_heads=2, layer_idx=0)
+    seen = watch(layer)
+    old = [weakref.ref(t) for t in (layer.A_log, layer.q_proj.weight, layer.o_proj, layer.o_proj.weight, layer.k_conv1d.weight)]
+    layer.A_log = torch.nn.Parameter(layer.A_log.detach().clone())
+    layer.q_proj.weight = torch.nn.Parameter(layer.q_proj.weight.detach().clone())
+    layer.k_conv1d.weight = torch.nn.Parameter(layer.k_conv1d.weight.detach().clone())
+    layer.o_proj = torch.nn.Linear(128, 64, bias=False)
+    gc.collect()
+    assert not any(r() is not None for r in old)
+    again = watch(layer)
+    assert again is not seen and again is not None and watch(layer) is again

@@ -95,11 +95,10 @@ def test_conv_arithmetic_is_the_single_kernels(W, bias):
     """The fused convolution forms its activation, and the gradients behind it, with the arithmetic of natsl_short_conv_*: the same bits.
     (A reciprocal in the place of the division moves about one rounding to bf16 in 2^15; a tensor here holds 2^22 values.)"""
     from neuralattentionsearchlinear_amd import _front
-    from neuralattentionsearchlinear_amd._layer_step import watch
     layer = _layer('gdn', None, 'all', conv_size=W, conv_bias=bias)
-    f = _front._front_plan(layer, 'gdn', watch(layer))
     torch.manual_seed(W)
     B, T = 4, 4096
+    f = _front.fast_front(layer, 'gdn', torch.zeros(B, T, layer.hidden_size, device=DEV).bfloat16(), None, None)
     raw = [torch.randn(B, T, c.hidden_size, device=DEV).bfloat16() for c in (layer.q_conv1d, layer.k_conv1d, layer.v_conv1d)]
     ref = lambda i, x: (layer.q_conv1d, layer.k_conv1d, layer.v_conv1d)[i](x)[0]
     with torch.no_grad():
@@ -139,6 +138,34 @@ def test_mixing_softmax_is_the_separate_ones():
         outs.append((y, da, db, dg, dw))
     for i, (p, q) in enumerate(zip(*outs)):
         assert torch.equal(p, q), f"output {i}: {int((p != q).sum())} values differ"
+
+
+@pytest.mark.parametrize("kind", ['gdn', 'mamba'])
+def test_replaced_weights_are_freed(kind):
+    """What the fused front and the step remember of a layer keeps no tensor alive: a replaced weight, and weights that a functional call
+    puts in for one forward, go with their last owner."""
+    import gc
+    import weakref
+    layer = _layer(kind, None, 'all')
+    torch.manual_seed(3)
+    x = torch.randn(2, 101, layer.hidden_size, device=DEV).bfloat16()
+    _generate(layer, kind, x, 100, (1,))
+    old = [weakref.ref(p) for p in layer.parameters()]
+    own = weakref.ref(layer.g_proj)
+    for name, p in list(layer.named_parameters()):
+        mod, _, leaf = name.rpartition('.')
+        setattr(layer.get_submodule(mod), leaf, torch.nn.Parameter(p.detach().clone()))
+    del p
+    layer.g_proj = torch.nn.Linear(layer.g_proj.in_features, layer.g_proj.out_features, bias=False, device=DEV, dtype=torch.bfloat16)
+    gc.collect()
+    assert own() is None and not any(r() is not None for r in old)
+    made = {n: p.detach().clone().requires_grad_(True) * 1.0 for n, p in layer.named_parameters()}
+    old = [weakref.ref(t) for t in made.values()]
+    o = torch.func.functional_call(layer.train(), made, (x[:, :100],))
+    (o[0] if isinstance(o, tuple) else o).sum().backward()
+    del made, o
+    gc.collect()
+    assert not any(r() is not None for r in old)
 
 
 @pytest.mark.parametrize("T,D,widths", [(1, 8, (8,)), (31, 64, (16, 24)), (32, 256, (256,)), (33, 264, (264, 8)), (129, 72, (512,)), (5000, 128, (136,))])

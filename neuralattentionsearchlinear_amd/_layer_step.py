@@ -223,37 +223,38 @@ class _Plan:
             s.l2_eps = layer.q_norm2.eps
         s.flags = flags
         self.device = params[0].device
-        # the cache's tensors as the kernels address them: (type, shape behind the batch); the attention keys and values by their rows
+        # the cache's tensors as the kernels address them: (type, shape behind the batch), but for those that follow the cache's capacity
         bs, bf16, f32 = layer.nats_block_size, torch.bfloat16, torch.float32
         self.rows = ((HQ, KA), (HQ, VA))
         self.buffers = [(bf16, (H * K, W)), (bf16, (H * K, W)), (bf16, (H * V, W)), (f32, (H, K, V)), (bf16, (bs, H, K)), (bf16, (bs, H, V)),
                         (f32, (bs, H)), (bf16, (bs, D))] + [(bf16, (bs, H))] * delta
-        self.expected = {}
+        self.expected = (0, 0, None, None)
         self.built = True
+
+    def _expect(self, B, cap):
+        """Types and shapes of takes()' tensors (the block-start state last) at this batch and capacity; the last pair is remembered."""
+        if self.expected[:2] != (B, cap):
+            want = self.buffers + [(torch.bfloat16, (cap, *self.rows[0])), (torch.bfloat16, (cap, *self.rows[1])),
+                                   (torch.bool, (cap // self.fixed.block, self.fixed.HN)), self.buffers[3]]
+            self.expected = (B, cap, [dt for dt, _ in want], [(B, *tail) for _, tail in want])
+        return self.expected[2:]
 
     def takes(self, cache, B, start):
         """Whether the cache's tensors have the types, shapes and layouts that the kernels read and write (a cache filled under autocast
         or by other code can hold others: the general path converts)."""
-        k, valid = cache.attn_k, cache.valid_attn_tokens
-        want = self.expected.get(B)
-        if want is None:
-            want = self.expected[B] = [(dt, (B, *tail)) for dt, tail in self.buffers]
-        have = [*cache.conv_state, cache.recurrent_state, cache.l_attn_k, cache.l_attn_v, cache.lattn_g, cache.block_type_state]
+        k, state = cache.attn_k, cache.recurrent_state
+        have = [*cache.conv_state, state, cache.l_attn_k, cache.l_attn_v, cache.lattn_g, cache.block_type_state]
         if self.fixed.is_delta:
             have.append(cache.lattn_beta)
-        cap, HN, index = k.shape[1], self.fixed.HN, self.device.index
-        have += [k, cache.attn_v, valid]
-        want = want + [(torch.bfloat16, (B, cap, *self.rows[0])), (torch.bfloat16, (B, cap, *self.rows[1])), (torch.bool, (B, cap // self.fixed.block, HN))]
-        if start is not None:
-            have.append(start)
-            want.append(want[3])
-        g = cache.g_cumsum
-        if cap % self.fixed.block or len(have) != len(want) or (g is not None and (g.numel() != B * self.fixed.H or g.get_device() != index)):
+        have += (k, cache.attn_v, cache.valid_attn_tokens, state if start is None else start)
+        g, cap, index = cache.g_cumsum, k.shape[1], self.device.index
+        dtypes, shapes = self._expect(B, cap)
+        try:
+            return ([*map(_dtype_of, have)] == dtypes and [*map(_shape_of, have)] == shapes and all(map(torch.Tensor.is_contiguous, have)) and
+                    {*map(torch.Tensor.get_device, have)} == {index} and cap % self.fixed.block == 0 and
+                    (g is None or (g.numel() == B * self.fixed.H and g.get_device() == index)))
+        except (AttributeError, TypeError):                # (one of them is None)
             return False
-        for t, (dtype, shape) in zip(have, want):
-            if t is None or t.dtype is not dtype or t.shape != shape or not t.is_contiguous() or t.get_device() != index:
-                return False
-        return True
 
 
 def layer_step(layer, kind, x, cache):

@@ -63,7 +63,8 @@ _OPTIONS = ("hidden_size", "head_k_dim", "head_v_dim", "head_attn_k_dim", "head_
             "allow_neg_eigval", "decay_for_non_gdn_blocks", "decay_for_non_mamba_blocks", "value_dim")
 _SUB_OPTIONS = ("eps", "kernel_size", "activation")
 _SUBMODULES = tuple({p[1]: p[3] for p in _PARAMS if p[1] is not None and p[3] is not None}.items()) + (("q_norm2", L2Norm), ("k_norm2", L2Norm))
-_PLAIN_TENSORS = {nn.Parameter, torch.Tensor}
+_PLAIN_TENSORS = {nn.Parameter, torch.Tensor, type(None)}
+_hooks_of = operator.itemgetter('_forward_hooks', '_forward_pre_hooks', '_backward_hooks', '_backward_pre_hooks')
 _dtype_of, _shape_of = operator.attrgetter('dtype'), operator.attrgetter('shape')
 
 
@@ -78,34 +79,37 @@ def weight_shapes(layer):
     return s
 
 
+def _getter(names):
+    """dict -> the tuple of its entries `names` (KeyError when one is gone)"""
+    if len(names) == 1:
+        return lambda d, n=names[0]: (d[n],)
+    return operator.itemgetter(*names) if names else lambda d: ()
+
+
 class _Watch:
     """What a layer's plans were made from besides its weights' values: which weights and plain submodules it has, the options, and the
     weights' addresses, types and layouts.  No tensor or module is held: a replaced weight is freed when its owner lets go of it."""
 
     def __init__(self, layer):
         mods = layer._modules
-        self.parts, weights, self.plain = [], [], True     # parts: (name, type or None, [(parameter, whether there is one)], options, their values)
+        self.absent = [n for n, _ in _SUBMODULES if mods.get(n) is None]
+        self.parts, self.plain = [], True                  # parts: (name, type, its parameters, its options, their values)
         for n, kind in _SUBMODULES:
             m = mods.get(n)
-            if m is None:
-                self.parts.append((n, None, (), (), ()))
-                continue
-            self.plain &= type(m) is kind
-            names = {p[2] for p in _PARAMS if p[1] == n} | ({'bias'} if kind is nn.Linear else set())
-            d = m.__dict__
-            options = tuple(o for o in _SUB_OPTIONS if o in d)
-            self.parts.append((n, type(m), self._params(m, sorted(names), weights), options, tuple(map(d.get, options))))
-        self.own = self._params(layer, sorted(p[2] for p in _PARAMS if p[1] is None), weights)
-        self.options = tuple(map(layer.__dict__.get, _OPTIONS))
-        self.plain &= set(map(type, weights)) <= _PLAIN_TENSORS
-        self.layouts = self._layouts(weights) if self.plain else None
+            if m is not None:
+                options = [o for o in _SUB_OPTIONS if o in m.__dict__]
+                self.parts.append((n, type(m), _getter([*m._parameters]), _getter(options) if options else None, _getter(options)(m.__dict__)))
+                self.plain &= type(m) is kind
+        self.own = _getter([*layer._parameters])
+        self.option_names = _getter([o for o in _OPTIONS if o in layer.__dict__])
+        self.options = self.option_names(layer.__dict__)
+        weights = [*self.own(layer._parameters)]
+        for n, _, params, _, _ in self.parts:
+            weights += params(mods[n]._parameters)
+        self.types = [*map(type, weights)]
+        self.plain &= {*self.types} <= _PLAIN_TENSORS
+        self.layouts = self._layouts([t for t in weights if t is not None]) if self.plain else None
         self.step_plan = self.front_plan = None
-
-    @staticmethod
-    def _params(m, names, weights):
-        held = [(n, m._parameters.get(n)) for n in names]
-        weights += [t for _, t in held if t is not None]
-        return tuple((n, t is not None) for n, t in held)
 
     @staticmethod
     def _layouts(w):
@@ -121,36 +125,27 @@ class _Watch:
 
     def holds(self, layer):
         """-> (whether nothing has changed, whether a submodule has a hook or a forward of its own)"""
-        mods, weights, hooked = layer._modules, [], False
-        for n, kind, params, options, values in self.parts:
-            m = mods.get(n)
-            if m is None or kind is None:
-                if m is not None or kind is not None:
+        mods, hooks = layer._modules, []
+        try:
+            weights = [*self.own(layer._parameters)]
+            for n, kind, params, options, values in self.parts:
+                m = mods[n]
+                if type(m) is not kind:
                     return False, False
-                continue
-            if type(m) is not kind:
-                return False, False
-            d = m.__dict__
-            held = d['_parameters']
-            for name, there in params:
-                t = held.get(name)
-                if (t is not None) is not there:
+                d = m.__dict__
+                weights += params(d['_parameters'])
+                hooks += _hooks_of(d)
+                if 'forward' in d:
+                    hooks.append(True)
+                if options is not None and options(d) != values:
                     return False, False
-                if there:
-                    weights.append(t)
-            if options and tuple(map(d.get, options)) != values:
-                return False, False
-            if d['_forward_hooks'] or d['_forward_pre_hooks'] or d['_backward_hooks'] or d['_backward_pre_hooks'] or 'forward' in d:
-                hooked = True
-        held = layer._parameters
-        for name, there in self.own:
-            t = held.get(name)
-            if (t is not None) is not there:
-                return False, False
-            if there:
-                weights.append(t)
-        return (tuple(map(layer.__dict__.get, _OPTIONS)) == self.options and set(map(type, weights)) <= _PLAIN_TENSORS and
-                self._layouts(weights) == self.layouts), hooked
+            same = self.option_names(layer.__dict__) == self.options
+        except KeyError:                                   # (a parameter, a submodule or an option is gone)
+            return False, False
+        for n in self.absent:
+            same &= mods.get(n) is None
+        return (same and [*map(type, weights)] == self.types and self.layouts is not None and
+                self._layouts([t for t in weights if t is not None]) == self.layouts), any(hooks)
 
 
 def watch(layer):

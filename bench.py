@@ -245,7 +245,7 @@ def bench_decode(args):
         metric="hybrid-layer decode tokens/sec (one new token per sequence) @ctx=8192,H=16,d=128 bf16", value=B / (ms * 1e-3),
         unit="tokens/s", n_gpus=1, steps=args.steps, warmup=args.warmup, ms_per_step=ms, higher_is_better=True, scaling="weak",
         vs_baseline=None, dtype="bf16", data="synthetic", config=dict(workload=args.workload, **w, cached_keys=TK),
-        roofline=dict(bound="hbm", kernel="gdn_recurrent_kernel+attn_masked_kernel", achieved=nbytes / (ms * 1e-3) / 1e9,
+        roofline=dict(bound="hbm", kernel="attend_and_recur_kernel+attn_masked_join_kernel", achieved=nbytes / (ms * 1e-3) / 1e9,
                       peak=PEAK_HBM_GBS, unit="GB/s", frac=nbytes / (ms * 1e-3) / 1e9 / PEAK_HBM_GBS, traffic=None,
                       algorithmic_bytes=nbytes, note="whole step incl. launch overheads of two kernels"))))
 

@@ -27,10 +27,11 @@ NATSL_DEVICE float row16_sum(float x) {
 // ---------------------------------------------------------------------------------------------
 // Bound by the bytes of K and V.  A wave takes chunks of KEYS_PER_CHUNK keys: 16 lanes share a row (16 or 8 bytes each in
 // bf16), four rows per instruction, and ALL loads of a chunk, keys and values, are issued before the first is used (16 KiB in
-// flight per wave at 128-wide bf16 heads; the earlier form requested four rows at a time and the values only after the
-// softmax, which kept the launch at 3.9 TB/s where plain reads reach 6.8).  A key row's four lane groups never meet until the
-// end: the score of key (pass, group) sits in all 16 lanes of its group, which are the lanes that hold that key's value row, so
-// neither scores nor probabilities go through LDS.  A chunk without a visible key is not loaded.
+// flight per wave at 128-wide bf16 heads).  8 sequences x 16 heads x 2066 keys with the recurrence beside it, 161 MB from HBM:
+// 36 us = 4.5 TB/s a decode step, against 57 us when four rows were requested at a time and the values only after the softmax.
+// A key row's four lane groups never meet until the end: the score of key (pass, group) sits in all 16 lanes of its group,
+// which are the lanes that hold that key's value row, so neither scores nor probabilities go through LDS.  A chunk without a
+// visible key is not loaded.
 constexpr int KEYS_PER_CHUNK = 32;
 constexpr int KEY_PASSES = KEYS_PER_CHUNK / 4;
 

@@ -5,11 +5,11 @@
 // rules, then every earlier block typed "attention" (taken from the sorted block list).
 // Scores are computed transposed, S^T = K Q^T, so that a lane owns one query column: the online-softmax
 // statistics are per-lane scalars and the probabilities already sit in the B-operand layout of the second
-// product O^T = V^T P^T.  V is staged transposed in LDS.
+// product O^T = V^T P^T.
 // Two ways through a tile: chunk_pipelined() (4 waves, and the ragged last tile of a sequence on 8 waves: K and V
-// staged through registers, double buffered, one chunk as one pipelined instruction stream per wave) and, for full
-// tiles on 8 waves, the three-phase schedule further down (K and V by LDS-DMA, the two waves of a SIMD half a chunk
-// apart).
+// staged through registers, V transposed on the way, double buffered, one chunk as one pipelined instruction stream per
+// wave) and, for full tiles on 8 waves, the three-phase schedule further down (K and V by LDS-DMA as they lie in memory, V
+// transposed by the operand reads, the two waves of a SIMD half a chunk apart).
 #include "natsl_device.h"
 #include "natsl_host.h"
 #include <atomic>
@@ -226,8 +226,8 @@ NATSL_DEVICE void chunk_pipelined(const bf16_t* Kb, const bf16_t* VTb, const bf1
 // segments of a row, applied on the way in by letting each lane fetch the segment that belongs at its LDS position.
 // The operand read is ds_read_b128, 16 lanes = 16 rows = 256 bytes per clock: with DK = 128 (one row = all 64 banks)
 // segment s of row r sits at s ^ (r & 15); with DK = 64 (two rows share the banks) at s ^ ((r >> 1) & 7).
-// V has to be transposed on the way (the matrix instruction wants 8 consecutive keys per lane, memory has 8
-// consecutive value columns), which the DMA cannot do: it passes through registers (4x8 transposes with v_perm_b32).
+// V takes the same way, row-major; the matrix instruction wants 8 consecutive keys per lane where memory has 8 consecutive value
+// columns, which the transposing LDS read gives (see pv_phase).
 // The two waves that share a SIMD run half a chunk apart (see the kernel), so a wave's vector phase (softmax_phase)
 // meets the other wave's matrix phases (pv_phase, qk_phase).
 
@@ -281,26 +281,40 @@ NATSL_DEVICE float dot2_ones(const unsigned w, const float acc) {
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w), ones, acc, false);
 }
 
-// O^T += V^T P^T for one chunk: PB[g] holds the probabilities of keys 16 g .. 16 g + 15.  V is staged transposed,
-// [DV][VTP] with the keys of a 16-key group stored in the order the probabilities are held (a lane's 8 k-slots are 16
-// contiguous bytes), so an operand is ONE ds_read_b128: the LDS pipe takes as long for an 8-byte read instruction as
-// for a 16-byte one, and two reads per operand made this phase LDS-bound.  vaddr: LDS byte address of the lane's row
-// (lane%32) of the tile plus 16*(lane>>5).  The row sums are taken from the same rounded probabilities, one v_dot2
-// under each matrix instruction.
-constexpr int VTP = 72;  // elements per row of that tile (64 keys + 8): conflict-free 16-byte reads and 8-byte transposed stores
+// O^T += V^T P^T for one chunk: PB[g] holds the probabilities of keys 16 g .. 16 g + 15.  V lies in LDS as in memory, [64 keys][DV],
+// and an operand is two transposing reads (4 keys x 32 columns each): a lane gets its column's keys in the order the probabilities
+// are held.  One clock serves 32 lanes of such a read, four rows x 64 bytes; the swizzle (v_swizzle) puts the four rows on different
+// banks: 1.0 - 1.25 ns an
+// instruction and CU, against 1.8 with two rows on the same banks and 3.4 with four (rows padded by 16 bytes).  (A pass that
+// transposed V from LDS to LDS, for operands of one 16-byte read, took 754 us a launch at B8 T8192 H16 against 746 now.)
+// vaddr: LDS byte address of the tile plus the lane's v_lane_addr(); XOR-ing it with 64 vt gives value tile vt.  The row sums are
+// taken from the same rounded probabilities, one v_dot2 under each matrix instruction.
+template <int DV>
+NATSL_DEVICE unsigned v_swizzle(const int row) {   // 16-byte segment s of key row `row` sits at s ^ v_swizzle
+  return DV == 128 ? (unsigned)(row & 3) << 2 : (unsigned)((row >> 1) & 1) << 2;
+}
+template <int DV>
+NATSL_DEVICE unsigned v_lane_addr(const int lane) {
+  const int i16 = lane & 15, row = 4 * (lane >> 5) + (i16 >> 2);
+  return (unsigned)(row * DV * 2) + 16u * ((unsigned)(2 * ((lane >> 4) & 1) + ((i16 >> 1) & 1)) ^ v_swizzle<DV>(row)) + 8u * (i16 & 1);
+}
 template <int DV>
 NATSL_DEVICE void pv_phase(const unsigned vaddr, const bf16x8 (&PB)[4], f32x16 (&acc)[DV / 32], float& l_run) {
   constexpr int VT = DV / 32, N = 4 * VT, A = OPERANDS_AHEAD, DOTS = 16 / N;  // 16 packed words per lane
   static_assert(16 % N == 0, "row sums ride on the matrix instructions");
-  typedef __attribute__((address_space(3))) const bf16x8* lds_op;
-  // (opaque to the compiler: it must stay ONE base register with the tile offsets in the instructions' offset fields;
-  // re-associated with the ring arithmetic of the caller, half of the offsets came out negative, each read got an
-  // address computation of its own and the reads were no longer issued ahead of their use)
-  unsigned base = vaddr;
-  asm("" : "+v"(base));
+  typedef __attribute__((address_space(3))) s16x4* lds_tr;
+  // (opaque to the compiler: one base register per value tile with the row offsets in the instructions' offset fields;
+  // re-associated with the ring arithmetic of the caller, each read got an address computation of its own)
+  unsigned base[VT];
+#pragma unroll
+  for (int vt = 0; vt < VT; ++vt) {
+    base[vt] = vaddr ^ (64u * vt);
+    asm("" : "+v"(base[vt]));
+  }
   auto ld_op = [&](const int i) __attribute__((always_inline)) -> bf16x8 {
-    const int g = i / VT, vt = i % VT;
-    return *reinterpret_cast<lds_op>(base + 32u * vt * (2u * VTP) + 32u * g);
+    const unsigned at = base[i % VT] + (unsigned)(16 * (i / VT) * DV * 2);
+    return join4(__builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_tr>(at)),
+                 __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_tr>(at + 8u * DV * 2)));
   };
   bf16x8 op[N + A];
 #pragma unroll
@@ -312,10 +326,10 @@ NATSL_DEVICE void pv_phase(const unsigned vaddr, const bf16x8 (&PB)[4], f32x16 (
 #pragma unroll
     for (int d = 0; d < DOTS; ++d) l_run = dot2_ones(__builtin_bit_cast(u32x4, PB[(i * DOTS + d) / 4])[(i * DOTS + d) % 4], l_run);
   }
-  __builtin_amdgcn_sched_group_barrier(0x100, A, 0);
+  __builtin_amdgcn_sched_group_barrier(0x100, 2 * A, 0);
 #pragma unroll
   for (int i = 0; i < N; ++i) {
-    if (i + A < N) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    if (i + A < N) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
   }
 }
@@ -573,89 +587,57 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
       //  * K(c) lives in ring buffer c % 4.  The early waves request K(k+4) by DMA right after sync(k): the buffer it
       //    overwrites, K(k), was last read before sync(k); it must have landed when they arrive at sync(k+2), so their
       //    wait before a barrier leaves exactly the newest request in flight.
-      //  * V(c) first lands row-major ("raw", buffer c % 2), also by DMA from the early waves: V(k+3) is requested right
-      //    after sync(k), ahead of K(k+4), and must have landed when they arrive at sync(k+1).  The late waves then
-      //    transpose it from LDS to LDS into ring buffer c % 3: V(k+2) is stored
-      //    after sync(k), into the buffer of V(k-1), last read before sync(k), and is visible from sync(k+1) on.
-      constexpr int KRING = 4, KTILE = 64 * DK * 2, VRING = 3, VTILE = DV * VTP * 2, RTILE = 64 * DV * 2;   // bytes
-      constexpr int KI = DK / 32, RI = DV / 32;                                          // DMA instructions per early wave and chunk
-      constexpr int KROWS_I = 512 / DK, RROWS_I = 512 / DV;                              // tile rows one instruction covers
+      //  * V(c) lives in ring buffer c % 4, row-major as it comes.  The late waves request V(k+3) at the end of their body k,
+      //    after sync(k): the buffer it overwrites, V(k-1), was last read before sync(k).  It must have landed when they arrive
+      //    at sync(k+2): they too leave exactly the newest request in flight.
+      constexpr int RING = 4, KTILE = 64 * DK * 2, VTILE = 64 * DV * 2;   // bytes
+      constexpr int KI = DK / 32, VI = DV / 32;                           // DMA instructions per wave and chunk: early waves K, late waves V
+      constexpr int KROWS_I = 512 / DK, VROWS_I = 512 / DV;               // tile rows one instruction covers
       // (the swizzled operand addresses are formed with XOR: the ring starts on a 1 KiB boundary)
-      const unsigned lds_k = ((unsigned)(size_t)smem + 1023u) & ~1023u, lds_r = lds_k + KRING * KTILE, lds_v = lds_r + 2 * RTILE;
+      const unsigned lds_k = ((unsigned)(size_t)smem + 1023u) & ~1023u, lds_v = lds_k + RING * KTILE;
       const bool late = wave >= 4;
       const int gw = wave & 3;  // wave within its group
-      // --- early waves: lane l of instruction i fills LDS row KROWS_I*i + l/segs, position l%segs, with the segment that belongs there
-      unsigned k_src[KI];
+      // --- lane l of instruction i fills LDS row rows_per_instr*i + l/segs, position l%segs, with the segment that belongs there
+      // (one array for both roles: a wave requests K or V, never both)
+      unsigned src[KI > VI ? KI : VI];
+      if (!late) {
 #pragma unroll
-      for (int j = 0; j < KI; ++j) {
-        const int r = KROWS_I * (KI * gw + j) + lane / (DK / 8), pos = lane % (DK / 8);
-        k_src[j] = (unsigned)((size_t)r * krow * sizeof(bf16_t)) + 16u * (pos ^ (DK == 128 ? (r & 15) : ((r >> 1) & 7)));
-      }
-      // raw V: segment s of row r sits at s ^ ((r >> 2) & 15), so that the 16 lanes of a transposing thread group (16
-      // key groups = rows 4 apart, one segment) read 16 different 16-byte slots
-      unsigned r_src[RI];
+        for (int j = 0; j < KI; ++j) {
+          const int r = KROWS_I * (KI * gw + j) + lane / (DK / 8), pos = lane % (DK / 8);
+          src[j] = (unsigned)((size_t)r * krow * sizeof(bf16_t)) + 16u * (pos ^ (DK == 128 ? (r & 15) : ((r >> 1) & 7)));
+        }
+      } else {
 #pragma unroll
-      for (int j = 0; j < RI; ++j) {
-        const int r = RROWS_I * (RI * gw + j) + lane / (DV / 8), pos = lane % (DV / 8);
-        r_src[j] = (unsigned)((size_t)r * vrow * sizeof(bf16_t)) + 16u * (pos ^ ((r >> 2) & (DV / 8 - 1)));
+        for (int j = 0; j < VI; ++j) {
+          const int r = VROWS_I * (VI * gw + j) + lane / (DV / 8), pos = lane % (DV / 8);
+          src[j] = (unsigned)((size_t)r * vrow * sizeof(bf16_t)) + 16u * ((unsigned)pos ^ v_swizzle<DV>(r));
+        }
       }
-      auto dma_r = [&](const int ks, const int c) __attribute__((always_inline)) {
+      auto dma_v = [&](const int ks, const int c) __attribute__((always_inline)) {
         const char* g = reinterpret_cast<const char*>(vp + (size_t)ks * vrow);
 #pragma unroll
-        for (int j = 0; j < RI; ++j) dma16(g, r_src[j], lds_r + (c & 1) * RTILE + (RI * gw + j) * 1024);
+        for (int j = 0; j < VI; ++j) dma16(g, src[j], lds_v + (c & 3) * VTILE + (VI * gw + j) * 1024);
       };
       auto dma_k = [&](const int ks, const int c) __attribute__((always_inline)) {
         const char* g = reinterpret_cast<const char*>(kp + (size_t)ks * krow);
 #pragma unroll
-        for (int j = 0; j < KI; ++j) dma16(g, k_src[j], lds_k + (c & 3) * KTILE + (KI * gw + j) * 1024);
-      };
-      // --- late waves: a thread owns keys 4 kg .. 4 kg + 3 of one 8-column segment.  16 consecutive lanes take the 16
-      // key groups of one segment: their transposed 8-byte stores fill one 128-byte row, the next 16 lanes' row lies
-      // 8 rows = 1152 bytes further, on the other half of the banks.
-      const int lt = tid & 255;
-      const int v_kg = lt & 15, v_sg = lt >> 4;
-      const bool v_on = v_sg < DV / 8;   // (DV = 64: half of the late waves have nothing to stage)
-      // raw tile: rows 4 kg .. 4 kg + 3, segment sg (swizzled)
-      const unsigned v_raw = (unsigned)(4 * v_kg * DV * 2) + 16u * ((v_on ? v_sg : 0) ^ (v_kg & (DV / 8 - 1)));
-      // keys 4 kg .. 4 kg + 3 sit at position 4 * slot of their 16-key group, slot = 2 (q & 1) + (q >> 1), q = kg % 4:
-      // a lane of half hf then finds its k-slots (keys 4 hf .. +3 and 8 + 4 hf .. +3 of the group) in bytes 16 hf .. 16 hf + 15
-      const unsigned v_dst = (unsigned)(8 * v_sg * VTP * 2) + 32u * (v_kg >> 2) + 8u * (2 * (v_kg & 1) + ((v_kg >> 1) & 1));
-      auto transpose_v = [&](const int c) __attribute__((always_inline)) {
-        if (v_on) {
-          typedef __attribute__((address_space(3))) const u32x4* lds_r4;
-          typedef __attribute__((address_space(3))) u32x2* lds_w;
-          unsigned src = lds_r + (c & 1) * RTILE + v_raw;
-          asm("" : "+v"(src));
-          u32x4 rv[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) rv[j] = *reinterpret_cast<lds_r4>(src + j * DV * 2);
-          const unsigned a = lds_v + (c % VRING) * VTILE + v_dst;
-#pragma unroll
-          for (int d = 0; d < 4; ++d) {
-            // value columns 2d (low halves) and 2d+1 (high halves) of the four keys
-            u32x2 lo, hi;
-            lo[0] = __builtin_amdgcn_perm(rv[1][d], rv[0][d], 0x05040100u);
-            lo[1] = __builtin_amdgcn_perm(rv[3][d], rv[2][d], 0x05040100u);
-            hi[0] = __builtin_amdgcn_perm(rv[1][d], rv[0][d], 0x07060302u);
-            hi[1] = __builtin_amdgcn_perm(rv[3][d], rv[2][d], 0x07060302u);
-            *reinterpret_cast<lds_w>(a + (2 * d) * VTP * 2) = lo;
-            *reinterpret_cast<lds_w>(a + (2 * d + 1) * VTP * 2) = hi;
-          }
-        }
+        for (int j = 0; j < KI; ++j) dma16(g, src[j], lds_k + (c & 3) * KTILE + (KI * gw + j) * 1024);
       };
       // operand addresses of this lane inside a tile (see qk_phase / pv_phase)
       const unsigned k_lane = (unsigned)(l32 * DK * 2) + 16u * (hf ^ (DK == 128 ? (l32 & 15) : ((l32 >> 1) & 7)));
-      const unsigned v_lane = (unsigned)(l32 * VTP * 2) + 16u * hf;
+      const unsigned v_lane = v_lane_addr<DV>(lane);
 
-      // The first four chunks are requested before anything else when their addresses need no block list (the usual
-      // case: four or more chunks from dstart on).
-      // Request order of the early waves: K(0), V(0), K(1), V(1); K(2) after the first barrier; V(2), K(3) after the second.
+      // The first two chunks are requested before anything else when their addresses need no block list (the usual
+      // case: four or more chunks from dstart on), the next ones behind the loads of the block list.
       const bool early_request = n_diag >= 4;
-      if (early_request && !late) {
-        dma_k(dstart, 0);
-        dma_r(dstart, 0);
-        dma_k(dstart + 64, 1);
-        dma_r(dstart + 64, 1);
+      if (early_request) {
+        if (late) {
+          dma_v(dstart, 0);
+          dma_v(dstart + 64, 1);
+        } else {
+          dma_k(dstart, 0);
+          dma_k(dstart + 64, 1);
+        }
       }
       // types of the blocks the chunks from dstart on fall into, as a bit mask (bit i = block dstart/Bs + i)
       unsigned long long diag_attn;
@@ -709,39 +691,20 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
         ++nx_it;
         return ks_cur;
       };
-      int ks_v = dstart;   // first key of the chunk whose raw V is requested next (one chunk behind the K requests)
-      if (!late) {
-        if (early_request) {
-          nx_it = 2;
-        } else {
-          int ks = next_chunk();
-          dma_k(ks, 0);
-          dma_r(ks, 0);
-          ks = next_chunk();
-          if (1 < n_iters) {
-            dma_k(ks, 1);
-            dma_r(ks, 1);
-          }
+      // the early waves' iterator runs four chunks ahead of the loop, the late waves' three
+      if (early_request) nx_it = 2;
+      for (int c = nx_it; c < (late ? 3 : 4); ++c) {
+        const int ks = next_chunk();
+        if (c < n_iters) {
+          if (late) dma_v(ks, c);
+          else dma_k(ks, c);
         }
-        // raw V(0), V(1) (and K(0), K(1)) must have landed for the transposition below
-        __builtin_amdgcn_s_waitcnt(0x0f70);
       }
-      __syncthreads();
-      if (!late) {
-        ks_v = next_chunk();                      // chunk 2
-        if (2 < n_iters) dma_k(ks_v, 2);
-      } else {
-        transpose_v(0);
-        if (1 < n_iters) transpose_v(1);
-      }
+      // K(0), K(1) and V(0) must have landed: the newer requests of a full set may stay in flight
+      if (n_iters < 4) __builtin_amdgcn_s_waitcnt(0x0f70);
+      else if (late) __builtin_amdgcn_s_waitcnt(0x0f70 | (2 * VI));
+      else __builtin_amdgcn_s_waitcnt(0x0f70 | (2 * KI));
       __syncthreads();                            // "sync(-1)"
-      if (!late) {
-        // raw V(2) only now: its buffer held raw V(0) until the barrier.  Like every later request pair it is followed
-        // by the K request that may stay in flight at the next barrier.
-        if (2 < n_iters) dma_r(ks_v, 2);
-        ks_v = next_chunk();                      // chunk 3
-        if (3 < n_iters) dma_k(ks_v, 3);
-      }
 
       // which of the chunks from dstart on this wave takes part in (bit it), and which one is its own, causal chunk:
       // lane i works it out for chunk i, once
@@ -777,34 +740,38 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
           if (cur_active) {
             softmax_phase<DV>(s0, s1, acc, m_ref, l_run, thr, lane, it == causal_it, qloc0, PB);
             __builtin_amdgcn_s_setprio(3);
-            pv_phase<DV>(lds_v + (it % VRING) * VTILE + v_lane, PB, acc, l_run);
+            pv_phase<DV>(lds_v + (it & 3) * VTILE + v_lane, PB, acc, l_run);
           }
           __builtin_amdgcn_s_setprio(3);
           if (nxt_active) qk_phase<DK>(lds_k + ((it + 1) & 3) * KTILE + k_lane, QB, m_ref, s0, s1);
           __builtin_amdgcn_s_setprio(0);
-          // K(it+2) and raw V(it+2) must have landed; the request for K(it+3), the newest, may stay in flight if there is one
+          // K(it+2) must have landed; the request for K(it+3), the newest, may stay in flight if there is one
           if (it + 3 < n_iters) __builtin_amdgcn_s_waitcnt(0x0f70 | KI);
           else __builtin_amdgcn_s_waitcnt(0x0f70);
           __syncthreads();                                  // sync(it)
-          if (it + 3 < n_iters) dma_r(ks_v, it + 3);        // raw V first: it has one interval to land, K has two
-          ks_v = next_chunk(ahead, true);
-          if (it + 4 < n_iters) dma_k(ks_v, it + 4);
+          const int ks = next_chunk(ahead, true);
+          if (it + 4 < n_iters) dma_k(ks, it + 4);
           cur_active = nxt_active;
         }
       } else {
         for (int it = 0; it < n_iters; ++it) {
           const bool nxt_active = is_active(it + 1);
+          const int ahead = list_ahead();
           bf16x8 PB[4];
           if (cur_active) softmax_phase<DV>(s0, s1, acc, m_ref, l_run, thr, lane, it == causal_it, qloc0, PB);
 #pragma unroll
           for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(PB[i]));   // the probabilities exist before the barrier
+          // V(it+1) must have landed; the request for V(it+2), the newest, may stay in flight if there is one
+          if (it + 2 < n_iters) __builtin_amdgcn_s_waitcnt(0x0f70 | VI);
+          else __builtin_amdgcn_s_waitcnt(0x0f70);
           __syncthreads();                                  // sync(it)
           __builtin_amdgcn_s_setprio(3);
-          if (cur_active) pv_phase<DV>(lds_v + (it % VRING) * VTILE + v_lane, PB, acc, l_run);
+          if (cur_active) pv_phase<DV>(lds_v + (it & 3) * VTILE + v_lane, PB, acc, l_run);
           if (nxt_active) qk_phase<DK>(lds_k + ((it + 1) & 3) * KTILE + k_lane, QB, m_ref, s0, s1);
           __builtin_amdgcn_s_setprio(0);
-          // the matrix phases come first, while the early waves are in their vector phase; the transposition follows
-          if (it + 2 < n_iters) transpose_v(it + 2);
+          // the matrix phases come first, while the early waves are in their vector phase; the requests follow
+          const int ks = next_chunk(ahead, true);
+          if (it + 3 < n_iters) dma_v(ks, it + 3);
           cur_active = nxt_active;
         }
       }
@@ -963,9 +930,8 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
 // to memory, two barriers, the first transposition) and ~3 800 of epilogue, against ~58 000 in the loop.  Here
 //  * the memory side is ONE stream of chunks across tiles.  Chunk c of a tile with n chunks has stream position sp0 + c,
 //    the next tile's chunk j has sp0 + n + j, and every ring slot is chosen by stream position.  The rules of the loop
-//    (after barrier k: request raw V(k+3), then K(k+4); the late waves transpose V(k+2)) simply run on into the next
-//    tile, whose first chunks need no block list: when a tile's loop ends, K(0..3) and V(0..2) of the next tile are on
-//    their way or already there, and V(0), V(1) are transposed;
+//    (after barrier k the early waves request K(k+4), the late waves V(k+3)) simply run on into the next tile, whose first
+//    chunks need no block list: when a tile's loop ends, K(0..3) and V(0..2) of the next tile are on their way or there;
 //  * the compute side makes a clean cut between tiles: output straight from the accumulators (no LDS), then one barrier
 //    that hands over what the late waves prepared for the new tile while the old one was running (its block types, its
 //    list of prior attention blocks in LDS, how many there are, and which tile comes after it), then QK(0);
@@ -997,8 +963,8 @@ template <int DK, int DV>
 __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
   constexpr int QW = 32, QTILE = 256, KSTEPS = DK / 16, VT = DV / 32;
-  constexpr int KTILE = 64 * DK * 2, VRING = 3, VTILE = DV * VTP * 2, RTILE = 64 * DV * 2;  // bytes
-  constexpr int KI = DK / 32, RI = DV / 32, KROWS_I = 512 / DK, RROWS_I = 512 / DV;
+  constexpr int KTILE = 64 * DK * 2, VTILE = 64 * DV * 2;  // bytes
+  constexpr int KI = DK / 32, VI = DV / 32, KROWS_I = 512 / DK, VROWS_I = 512 / DV;
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int rows[2][STREAM_ROWS];
   __shared__ __align__(16) StreamTile info[2];
@@ -1014,64 +980,42 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
   const size_t krow = (size_t)p.HKV * DK, vrow = (size_t)p.HKV * DV;
   const size_t list_stride = (size_t)p.HN * 2;
   constexpr int K_SHIFT = DK == 128 ? 8 : 7, V_SHIFT = DV == 128 ? 8 : 7;  // log2 of a K / V row in bytes
-  const unsigned lds_k = ((unsigned)(size_t)smem + 1023u) & ~1023u, lds_r = lds_k + 4 * KTILE, lds_v = lds_r + 2 * RTILE;
+  const unsigned lds_k = ((unsigned)(size_t)smem + 1023u) & ~1023u, lds_v = lds_k + 4 * KTILE, lds_o = lds_v + 4 * VTILE;
 
   // ---- lane constants of the data movement (as in the kernel above) ----------------------------------------------
   // Source offsets of the DMA instructions: lane l of instruction j fills LDS row rows_per_instr * j + l / segs, position
   // l % segs, with the segment that the swizzle puts there.  A chunk is named by the row index of its first key in the
   // [B*T*HKV] row space of K and V, (token * HKV + kv head): its address is the tensor base plus that index shifted.
-  unsigned k_src[KI], r_src[RI];
+  // (one array for both roles: a wave requests K or V, never both)
+  unsigned src[KI > VI ? KI : VI];
+  if (!late) {
 #pragma unroll
-  for (int j = 0; j < KI; ++j) {
-    const int r = KROWS_I * (KI * gw + j) + lane / (DK / 8), pos = lane % (DK / 8);
-    k_src[j] = (unsigned)((size_t)r * krow * sizeof(bf16_t)) + 16u * (pos ^ (DK == 128 ? (r & 15) : ((r >> 1) & 7)));
-  }
+    for (int j = 0; j < KI; ++j) {
+      const int r = KROWS_I * (KI * gw + j) + lane / (DK / 8), pos = lane % (DK / 8);
+      src[j] = (unsigned)((size_t)r * krow * sizeof(bf16_t)) + 16u * (pos ^ (DK == 128 ? (r & 15) : ((r >> 1) & 7)));
+    }
+  } else {
 #pragma unroll
-  for (int j = 0; j < RI; ++j) {
-    const int r = RROWS_I * (RI * gw + j) + lane / (DV / 8), pos = lane % (DV / 8);
-    r_src[j] = (unsigned)((size_t)r * vrow * sizeof(bf16_t)) + 16u * (pos ^ ((r >> 2) & (DV / 8 - 1)));
+    for (int j = 0; j < VI; ++j) {
+      const int r = VROWS_I * (VI * gw + j) + lane / (DV / 8), pos = lane % (DV / 8);
+      src[j] = (unsigned)((size_t)r * vrow * sizeof(bf16_t)) + 16u * ((unsigned)pos ^ v_swizzle<DV>(r));
+    }
   }
-  auto dma_r = [&](const int row, const unsigned sp) __attribute__((always_inline)) {
+  auto dma_v = [&](const int row, const unsigned sp) __attribute__((always_inline)) {
     const char* g = reinterpret_cast<const char*>(p.v) + ((size_t)(unsigned)row << V_SHIFT);
-    const unsigned l0 = lds_r + (sp & 1) * RTILE + RI * gw * 1024;
+    const unsigned l0 = lds_v + (sp & 3) * VTILE + VI * gw * 1024;
 #pragma unroll
-    for (int j = 0; j < RI; ++j) dma16(g, r_src[j], l0 + j * 1024);
+    for (int j = 0; j < VI; ++j) dma16(g, src[j], l0 + j * 1024);
   };
   auto dma_k = [&](const int row, const unsigned sp) __attribute__((always_inline)) {
     const char* g = reinterpret_cast<const char*>(p.k) + ((size_t)(unsigned)row << K_SHIFT);
     const unsigned l0 = lds_k + (sp & 3) * KTILE + KI * gw * 1024;
 #pragma unroll
-    for (int j = 0; j < KI; ++j) dma16(g, k_src[j], l0 + j * 1024);
+    for (int j = 0; j < KI; ++j) dma16(g, src[j], l0 + j * 1024);
   };
   const int lt = tid & 255;
-  const int v_kg = lt & 15, v_sg = lt >> 4;
-  const bool v_on = v_sg < DV / 8;
-  const unsigned v_raw = (unsigned)(4 * v_kg * DV * 2) + 16u * ((v_on ? v_sg : 0) ^ (v_kg & (DV / 8 - 1)));
-  const unsigned v_dst = (unsigned)(8 * v_sg * VTP * 2) + 32u * (v_kg >> 2) + 8u * (2 * (v_kg & 1) + ((v_kg >> 1) & 1));
-  auto transpose_v = [&](const unsigned sp) __attribute__((always_inline)) {
-    if (v_on) {
-      typedef __attribute__((address_space(3))) const u32x4* lds_r4;
-      typedef __attribute__((address_space(3))) u32x2* lds_w;
-      unsigned src = lds_r + (sp & 1) * RTILE + v_raw;
-      asm("" : "+v"(src));
-      u32x4 rv[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) rv[j] = *reinterpret_cast<lds_r4>(src + j * DV * 2);
-      const unsigned a = lds_v + (sp % VRING) * VTILE + v_dst;
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        u32x2 lo, hi;
-        lo[0] = __builtin_amdgcn_perm(rv[1][d], rv[0][d], 0x05040100u);
-        lo[1] = __builtin_amdgcn_perm(rv[3][d], rv[2][d], 0x05040100u);
-        hi[0] = __builtin_amdgcn_perm(rv[1][d], rv[0][d], 0x07060302u);
-        hi[1] = __builtin_amdgcn_perm(rv[3][d], rv[2][d], 0x07060302u);
-        *reinterpret_cast<lds_w>(a + (2 * d) * VTP * 2) = lo;
-        *reinterpret_cast<lds_w>(a + (2 * d + 1) * VTP * 2) = hi;
-      }
-    }
-  };
   const unsigned k_lane = (unsigned)(l32 * DK * 2) + 16u * (hf ^ (DK == 128 ? (l32 & 15) : ((l32 >> 1) & 7)));
-  const unsigned v_lane = (unsigned)(l32 * VTP * 2) + 16u * hf;
+  const unsigned v_lane = v_lane_addr<DV>(lane);
 
   // ---- work queues (wave 4 only) -----------------------------------------------------------------------------------
   const unsigned xcc = xcc_id();
@@ -1135,8 +1079,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
   unsigned sp0 = 0;   // stream position of its chunk 0
   bool cur_real = false;
   int c_n = 0, c_hq = 0, c_tile = 0, c_hkv = 0, c_hn = 0, dstart = 0, dblk = 0;
-  bool k_req = false;  // the early waves' newest request is a K request that may still be in flight at the next barrier
-  int row_v = 0;       // early waves: row index of the chunk whose K was requested last (its V is requested next)
+  bool req = false;  // this wave made a request in its last request step: that one may still be in flight at the next barrier
   if (wave == 4) {
     const int r0 = resolve_ticket(take_ticket(), &info[0]);
     if (lane == 0) {
@@ -1155,12 +1098,9 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
   // ---- a tile's output.  A lane holds, of its query, value columns 8 rg + 4 hf .. + 3 of every 32-column tile: stored
   // from there, an instruction would touch 64 separate 16-byte pieces.  The rows go through LDS instead, half of the
   // columns at a time (a wave's 32 rows x DV/2 columns; 16-byte segments XOR-swizzled by the row), and leave as whole
-  // lines.  The space is a raw V buffer, a quarter of it per wave.  The early waves use, right after their last chunk,
-  // the buffer whose next request (the next tile's chunk 2) they hold back until they are done: a wave's requests go
-  // to the same quarter as its rows, so no barrier is needed.  The late waves use the other buffer, whose contents (the
-  // next tile's chunk 1) all of them have transposed once the hand-over barrier of the next tile is behind them: they
-  // store there, before anything of the new tile touches the accumulators.  row0: flat (token, head) index of the
-  // wave's first query.
+  // lines.  The space is an area of its own, a quarter of it per wave of a group.  The early waves use it right after their last
+  // chunk; the late waves once the hand-over barrier of the next tile is behind them (all early waves have then read their rows
+  // back), before anything of the new tile touches their accumulators.  row0: flat (token, head) index of the wave's first query.
   auto store_tile = [&](const unsigned stage, const size_t row0) __attribute__((always_inline)) {
     constexpr int PW = DV / 2, RB = PW * 2, NSEG = RB / 16, RPI = 64 / NSEG;   // columns per pass, row bytes, segments, rows per instruction
     typedef __attribute__((address_space(3))) u32x2* lds_w8;
@@ -1289,14 +1229,11 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
     bool cur_active = act_mask & 1ull;
     if (cur_active) qk_phase<DK>(lds_k + (sp0 & 3) * KTILE + k_lane, QB, m_ref, s0, s1);
 
+    // Stream chunks requested during this tile: its own from chunk 4 (V: 3) on, the ones before were requested while the
+    // previous tile ran, and the next tile's first four (three), all by their entry in this tile's chunk table.
+    const int rq_lo = cur_real ? 0 : n_iters;
+    const unsigned rq_span = (unsigned)((n_valid ? n_iters + (late ? 3 : 4) : n_iters) - rq_lo);
     if (!late) {
-      // Stream chunks requested during this tile: its own from chunk 4 on (chunks 0..3 were requested while the previous
-      // tile ran) and the next tile's first four, all by their entry in this tile's chunk table.
-      // (the V request of the last iteration, the next tile's chunk 2, waits until the output code below is done with
-      // the buffer it goes to)
-      const int rq_lo = cur_real ? 0 : n_iters;
-      const unsigned rq_span = (unsigned)((n_valid ? n_iters + 4 : n_iters) - rq_lo);
-      const unsigned rv_span = (unsigned)((n_valid ? n_iters + 2 : n_iters) - rq_lo);
       typedef __attribute__((address_space(3))) const int* lds_row;
       const unsigned row_tab = (unsigned)(size_t)&rows[a][4];
       for (int it = 0; it < n_iters; ++it) {
@@ -1306,25 +1243,22 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
         if (cur_active) {
           softmax_phase<DV>(s0, s1, acc, m_ref, l_run, thr, lane, it == causal_it, qloc0, PB);
           __builtin_amdgcn_s_setprio(3);
-          pv_phase<DV>(lds_v + ((sp0 + it) % VRING) * VTILE + v_lane, PB, acc, l_run);
+          pv_phase<DV>(lds_v + ((sp0 + it) & 3) * VTILE + v_lane, PB, acc, l_run);
         }
         __builtin_amdgcn_s_setprio(3);
         if (nxt_active) qk_phase<DK>(lds_k + ((sp0 + it + 1) & 3) * KTILE + k_lane, QB, m_ref, s0, s1);
         __builtin_amdgcn_s_setprio(0);
-        // K(it+2) and raw V(it+2) must have landed; the newest K request, if the last request step made one, may stay
-        // in flight
-        if (k_req) __builtin_amdgcn_s_waitcnt(0x0f70 | KI);
-        else __builtin_amdgcn_s_waitcnt(0x0f70);
-        __syncthreads();                                  // sync(it)
-        // Requests: V(it+3), whose row index was found when its K was requested, then K(it+4).  (As few instructions
-        // as possible: the other wave of the SIMD runs its matrix phases at raised priority meanwhile, and every
-        // instruction of this one waits for an issue slot.)
-        if ((unsigned)(it + 3 - rq_lo) < rv_span) dma_r(row_v, sp0 + it + 3);
-        k_req = (unsigned)(it + 4 - rq_lo) < rq_span;
-        if (k_req) {
-          row_v = __builtin_amdgcn_readfirstlane(row_ahead);
-          dma_k(row_v, sp0 + it + 4);
+        // K(it+2) must have landed; the newest request, K(it+3), if the last request step made one, may stay in flight.  (In a
+        // tile's first iteration it has: the wait at the end of the tile before left K(3) only.)
+        if (it > 0) {
+          if (req) __builtin_amdgcn_s_waitcnt(0x0f70 | KI);
+          else __builtin_amdgcn_s_waitcnt(0x0f70);
         }
+        __syncthreads();                                  // sync(it)
+        // K(it+4).  (As few instructions as possible: the other wave of the SIMD runs its matrix phases at raised
+        // priority meanwhile, and every instruction of this one waits for an issue slot.)
+        req = (unsigned)(it + 4 - rq_lo) < rq_span;
+        if (req) dma_k(__builtin_amdgcn_readfirstlane(row_ahead), sp0 + it + 4);
         cur_active = nxt_active;
       }
     } else {
@@ -1338,9 +1272,8 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
       int pe[4] = {0, 0, 0, 0}, p_nattn = 0;
       float p_type = 0.f;
       int ev_it = n_valid ? 0 : -1;
-      // transpositions cover stream chunks tr_lo <= it + 2 < tr_lo + tr_span (this tile's, then the next tile's first two)
-      const int tr_lo = cur_real ? 0 : n_iters;
-      const unsigned tr_span = (unsigned)((n_valid ? n_iters + 2 : n_iters) - tr_lo);
+      typedef __attribute__((address_space(3))) const int* lds_row;
+      const unsigned row_tab = (unsigned)(size_t)&rows[a][3];
       for (int it = 0; it < n_iters; ++it) {
         const bool nxt_active = is_active(it + 1);
         const bool last = it == n_iters - 1;
@@ -1402,37 +1335,49 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
         if (cur_active) softmax_phase<DV>(s0, s1, acc, m_ref, l_run, thr, lane, it == causal_it, qloc0, PB);
 #pragma unroll
         for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(PB[i]));   // the probabilities exist before the barrier
+        // V(it+1) must have landed; the newest request, V(it+2), if there was one, may stay in flight (the first iteration: as
+        // for the early waves)
+        if (it > 0) {
+          if (req) __builtin_amdgcn_s_waitcnt(0x0f70 | VI);
+          else __builtin_amdgcn_s_waitcnt(0x0f70);
+        }
         __syncthreads();                                  // sync(it)
+        const int row_ahead = *reinterpret_cast<lds_row>(row_tab + 4u * it);   // chunk it + 3
         __builtin_amdgcn_s_setprio(3);
-        if (cur_active) pv_phase<DV>(lds_v + ((sp0 + it) % VRING) * VTILE + v_lane, PB, acc, l_run);
+        if (cur_active) pv_phase<DV>(lds_v + ((sp0 + it) & 3) * VTILE + v_lane, PB, acc, l_run);
         if (nxt_active) qk_phase<DK>(lds_k + ((sp0 + it + 1) & 3) * KTILE + k_lane, QB, m_ref, s0, s1);
         __builtin_amdgcn_s_setprio(0);
-        if ((unsigned)(it + 2 - tr_lo) < tr_span) transpose_v(sp0 + it + 2);
+        req = (unsigned)(it + 3 - rq_lo) < rq_span;
+        if (req) dma_v(__builtin_amdgcn_readfirstlane(row_ahead), sp0 + it + 3);
         cur_active = nxt_active;
       }
     }
 
-    // ---- end of the tile: output (early waves now, late waves after the next hand-over barrier), the request held back,
-    // the next tile's queries
+    // ---- end of the tile: the next tile's queries, output (early waves now, late waves after the next hand-over barrier)
     {
       const size_t row0 = (size_t)(bos + q0) * p.HQ + c_hq;
-      const unsigned stage_e = lds_r + ((sp0 + n_iters) & 1) * RTILE + gw * (32 * DV);
-      const unsigned stage_l = lds_r + ((sp0 + n_iters + 1) & 1) * RTILE + gw * (32 * DV);
+      const unsigned stage = lds_o + gw * (32 * DV);
+      load_next_q();   // (ahead of the stores: what waits for the queries later does not wait for the stores then)
+      // What the first barrier of the next tile needs, K(2) and V(1) of that tile, has landed: newer than those are one request
+      // and the queries.  (Behind the stores that wait would last until the output has left.)
+      static_assert(KSTEPS + KI <= 15 && KSTEPS + VI <= 15, "fits the low field of the wait");
       if (!late) {
-        load_next_q();   // (ahead of the stores: what waits for the queries later does not wait for the stores then)
-        if (cur_real) store_tile(stage_e, row0);
+        __builtin_amdgcn_s_waitcnt(0x0f70 | (KSTEPS + KI));
+        if (cur_real) store_tile(stage, row0);
         __builtin_amdgcn_s_waitcnt(0xc07f);   // the staged rows have been read
-        if (!n_valid) break;
-        dma_r(__builtin_amdgcn_readfirstlane(rows[a][n_iters + 2]), sp0 + n_iters + 2);
-        k_req = false;   // the newest request is now a V request: everything has to land before the next barrier but one
-      } else {
-        load_next_q();
         if (!n_valid) {
-          if (cur_real) store_tile(stage_l, row0);   // (no next tile: nothing was transposed after this tile's own chunks)
+          __syncthreads();   // the late waves take the staging area over
+          break;
+        }
+      } else {
+        __builtin_amdgcn_s_waitcnt(0x0f70 | (KSTEPS + VI));
+        if (!n_valid) {
+          __syncthreads();
+          if (cur_real) store_tile(stage, row0);
           break;
         }
         pend_store = cur_real;
-        pend_stage = stage_l;
+        pend_stage = stage;
         pend_row0 = row0;
       }
     }
@@ -1450,7 +1395,7 @@ static int launch_softmax(const SoftmaxParams& p, hipStream_t stream) {
   size_t lds = (size_t)2 * (64 * KP + DV * VT_PITCH) * sizeof(bf16_t);
   const size_t epi = (size_t)QTILE * VP * sizeof(bf16_t);
   if (epi > lds) lds = epi;
-  const size_t ring = ((size_t)4 * 64 * DK + (size_t)2 * 64 * DV + (size_t)3 * DV * VTP) * sizeof(bf16_t) + 1024;  // 8 waves: four K tiles, two raw and three transposed V tiles, 1 KiB aligned
+  const size_t ring = (size_t)4 * 64 * (DK + DV) * sizeof(bf16_t) + 1024;  // 8 waves: four K and four V tiles, 1 KiB aligned
   if (NWAVES == 8 && ring > lds) lds = ring;
   auto kern = softmax_sparse_fwd_kernel<DK, DV, NWAVES>;
   static std::atomic<unsigned long long> reserved{0};
@@ -1513,7 +1458,7 @@ template <int DK, int DV>
 static int launch_softmax_stream(const SoftmaxParams& p, const StreamDevice* d, hipStream_t stream) {
   static std::atomic<unsigned> launches{0};
   static std::atomic<unsigned long long> reserved{0};
-  const size_t lds = ((size_t)4 * 64 * DK + (size_t)2 * 64 * DV + (size_t)3 * DV * VTP) * sizeof(bf16_t) + 1024;
+  const size_t lds = (size_t)(4 * 64 * (DK + DV) + 64 * DV) * sizeof(bf16_t) + 1024;  // four K and four V tiles, the output's staging area; 1 KiB aligned
   auto kern = softmax_stream_kernel<DK, DV>;
   if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, lds, "softmax")) return rc;
   unsigned* queue = d->queues + (size_t)(launches.fetch_add(1) % STREAM_SLOTS) * STREAM_SLOT_WORDS;

@@ -47,15 +47,15 @@ NATSL_DEVICE bool bwd_type_is_one(const void* types, int dtype, size_t i) {
 
 constexpr int BWD_MAX_LDS_LIST = 2048;
 
-// Position swizzle of the dkdv kernel's query tiles (rows of D bf16, unpadded): 16-byte segment s of row r is stored at
-// s ^ bwd_swizzle<D>(r).  A bijection over the 16 rows that one clock of a 16-byte row read serves (conflict-free), and
-// two of four consecutive rows never differ by 1, so the 4 rows x 2 segments of a transposing read's 16 lanes
-// fall on different banks as well.
+// Position swizzle of tiles that are read both by rows and transposed (rows of D bf16, unpadded): 16-byte segment s of row r is
+// stored at s ^ bwd_swizzle<D>(r).  A bijection over the 16 rows that one clock of a 16-byte row read serves; and of a transposing
+// read one clock serves 32 lanes, 4 consecutive rows x 64 bytes, which land on the four quarters of the banks: 1.0 - 1.25 ns an
+// instruction and CU against 1.8 where two of the rows share banks and 3.4 in rows padded by 16 bytes.
 template <int D>
 NATSL_DEVICE int bwd_swizzle(const int r) {
-  if constexpr (D == 128) return ((r & 7) << 1) | ((r >> 3) & 1);
+  if constexpr (D == 128) return ((r & 3) << 2) | ((r >> 2) & 3);
   const int y = (r >> 1) & 7;
-  return ((y & 3) << 1) | (y >> 2);
+  return ((y & 1) << 2) | (y >> 1);
 }
 
 // one DMA instruction: lane l copies 16 (4) bytes from base + voff to LDS byte address lds + 16 l (4 l)
@@ -82,15 +82,6 @@ NATSL_DEVICE void dma4_if(const void* base, const unsigned voff, const unsigned 
       : "=&s"(saved)
       : "v"(voff), "s"(base), "s"(lds), "s"(__builtin_amdgcn_readfirstlane(on))
       : "memory", "m0", "scc");
-}
-
-// A operand of a 32x32x16 product taken TRANSPOSED from a row-major LDS tile: A[m = lane%32][k-slot (hf, j)] =
-// tile[row_base + 8(j/4) + 4hf + j%4][col_base + m].  ds_read_b64_tr_b16: within each group of 16 lanes, lane i supplies
-// the address of a 4-element row R_i and receives { R_{4j + i/4}[i%4] : j < 4 }.
-NATSL_DEVICE bf16x8 tr_operand(const bf16_t* tile, const int pitch, const int row_base, const int col_base, const int lane) {
-  const int i16 = lane & 15, colsel = 16 * ((lane >> 4) & 1), hf = lane >> 5;
-  const bf16_t* p = tile + (row_base + 4 * hf + (i16 >> 2)) * pitch + col_base + colsel + 4 * (i16 & 3);
-  return join4(lds_tr4(p), lds_tr4(p + 8 * pitch));
 }
 
 NATSL_DEVICE bf16x8 pack8(const f32x16& x, const int ss) {
@@ -124,32 +115,14 @@ __global__ __launch_bounds__(256) void delta_kernel(const SoftmaxBwdParams p) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// 256 threads stage a [64][D] tile row-major (pitch D+8) from rows tok0.. of a [T][stride] tensor, rows clamped to len-1
-template <int D>
-struct RowStage {
-  static constexpr int SEGS = D / 8, ROWS = 256 / SEGS, PASSES = 64 / ROWS, PITCH = D + 8;
-  u32x4 r[PASSES];
-  NATSL_DEVICE void load(const bf16_t* base, const size_t row_stride, const int tok0, const int len, const int tid) {
-    const int row = tid / SEGS, seg = tid % SEGS;
-#pragma unroll
-    for (int i = 0; i < PASSES; ++i) {
-      const int tok = min(tok0 + row + ROWS * i, len - 1);
-      r[i] = *reinterpret_cast<const u32x4*>(base + (size_t)tok * row_stride + 8 * seg);
-    }
-  }
-  NATSL_DEVICE void store(bf16_t* tile, const int tid) const {
-    const int row = tid / SEGS, seg = tid % SEGS;
-#pragma unroll
-    for (int i = 0; i < PASSES; ++i) *reinterpret_cast<u32x4*>(tile + (row + ROWS * i) * PITCH + 8 * seg) = r[i];
-  }
-};
-
+// dQ.  What bounds it: the LDS pipe and the matrix pipe of a SIMD's two waves are about equally busy (per 64-key chunk and wave: K and V by
+// rows, K once more transposed; 2 KS + 2 VS + 4 DT matrix instructions).  K and V chunks come by DMA into two buffers, unpadded and
+// swizzled (bwd_swizzle), so that neither kind of read meets bank conflicts and no register stages them.
 template <int DK, int DV>
 __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
-  constexpr int KP = DK + 8, VP = DV + 8, KS = DK / 16, VS = DV / 16, DT = DK / 32, QTILE = 128;
-  extern __shared__ __align__(16) unsigned char smem[];
-  bf16_t* Ks = reinterpret_cast<bf16_t*>(smem);  // [2][64][KP]
-  bf16_t* Vs = Ks + 2 * 64 * KP;                 // [2][64][VP]
+  constexpr int KP = DK + 8, KS = DK / 16, VS = DV / 16, DT = DK / 32, QTILE = 128;
+  constexpr unsigned KROWB = DK * 2, VROWB = DV * 2, KTILE = 64 * KROWB, VTILE = 64 * VROWB;   // bytes
+  extern __shared__ __align__(1024) unsigned char smem[];   // K [2][64][DK], V [2][64][DV], swizzled
   __shared__ int lds_list[BWD_MAX_LDS_LIST];
   __shared__ int lds_count;
 
@@ -193,7 +166,7 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
 
   const bf16_t* kp = p.k + ((size_t)bos * p.HKV + hkv) * DK;
   const bf16_t* vp = p.v + ((size_t)bos * p.HKV + hkv) * DV;
-  const size_t krow = (size_t)p.HKV * DK, vrow = (size_t)p.HKV * DV;
+  const unsigned krow = (unsigned)p.HKV * KROWB, vrow = (unsigned)p.HKV * VROWB;   // bytes from token to token (T * HQ * D * 2 < 2^32 is checked on the host)
   const int32_t* list = p.idx + ((size_t)bos_nats * p.HN + hn) * 2;
   const size_t list_stride = (size_t)p.HN * 2;
   const int n_attn = p.nblk[((size_t)n * p.HN + hn) * 2];
@@ -217,11 +190,34 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
 
-  RowStage<DK> sk;
-  RowStage<DV> sv;
+  // ---- requests: lane l of instruction j fills row rows_per_instr * j + l / segs, position l % segs of a tile, with the segment that the
+  // swizzle puts there; rows past the end repeat the last one (such keys are hidden by the causal rule)
+  constexpr int KI = DK / 32, VI = DV / 32;   // instructions per wave and chunk
+  const unsigned lds_k = (unsigned)(size_t)smem, lds_v = lds_k + 2 * KTILE;
+  const int kr0 = KI * wave * (512 / DK) + lane / (DK / 8), vr0 = VI * wave * (512 / DV) + lane / (DV / 8);
+  auto request = [&](const int ks, const int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < KI; ++j) {
+      const int r = kr0 + (512 / DK) * j;
+      dma16(kp, (unsigned)min(ks + r, len - 1) * krow + 16u * ((lane % (DK / 8)) ^ bwd_swizzle<DK>(r)), lds_k + buf * KTILE + (KI * wave + j) * 1024);
+    }
+#pragma unroll
+    for (int j = 0; j < VI; ++j) {
+      const int r = vr0 + (512 / DV) * j;
+      dma16(vp, (unsigned)min(ks + r, len - 1) * vrow + 16u * ((lane % (DV / 8)) ^ bwd_swizzle<DV>(r)), lds_v + buf * VTILE + (VI * wave + j) * 1024);
+    }
+  };
+  // ---- the lane's operand addresses inside a tile: its row (XOR with 32 st: k-step st), and for the transposing reads the 4-element
+  // row piece it names (XOR with 64 t: columns 32 t ..; XOR with 32 and 8 rows further: the second read)
+  const unsigned k_lane = (unsigned)l32 * KROWB + 16u * (unsigned)(hf ^ bwd_swizzle<DK>(l32));
+  const unsigned v_lane = (unsigned)l32 * VROWB + 16u * (unsigned)(hf ^ bwd_swizzle<DV>(l32));
+  unsigned t_lane;
+  {
+    const int i16 = lane & 15, r = 4 * hf + (i16 >> 2);
+    t_lane = (unsigned)r * KROWB + 16u * (unsigned)((2 * ((lane >> 4) & 1) + ((i16 >> 1) & 1)) ^ bwd_swizzle<DK>(r)) + 8u * (unsigned)(i16 & 1);
+  }
   const int n_diag = (min(len, tile_start + QTILE) - dstart + 63) >> 6;
-  sk.load(kp, krow, dstart, len, tid);
-  sv.load(vp, vrow, dstart, len, tid);
+  request(dstart, 0);
   if (tid == 0) lds_count = 0;
   __syncthreads();
   {
@@ -242,8 +238,7 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
     const bool in_range = lane < n_diag && (size_t)blk * Bs < (size_t)min(len, tile_start + QTILE);
     diag_attn = __ballot(in_range && bwd_type_is_one(p.types, p.types_dtype, ((size_t)(bos_nats + blk) * p.HN + hn) * 2));
   }
-  sk.store(Ks, tid);
-  sv.store(Vs, tid);
+  __builtin_amdgcn_s_waitcnt(0x0f70);   // this wave's requests have landed
   __syncthreads();
   const int n_prior_chunks = __builtin_amdgcn_readfirstlane(lds_count) * per_blk;
   const int n_iters = n_diag + n_prior_chunks;
@@ -272,10 +267,7 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
 
   for (int it = 0; it < n_iters; ++it) {
     const int buf = it & 1;
-    if (it + 1 < n_iters) {
-      sk.load(kp, krow, ks_fetch, len, tid);
-      sv.load(vp, vrow, ks_fetch, len, tid);
-    }
+    if (it + 1 < n_iters) request(ks_fetch, buf ^ 1);   // (that buffer was last read before the barrier just passed)
     bool active = wave_valid, causal = false;
     if (it < n_diag) {
       const int jc = (dstart >> 6) + it;
@@ -289,8 +281,10 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
       }
     }
     if (active) {
-      const bf16_t* Kb = Ks + buf * 64 * KP;
-      const bf16_t* Vb = Vs + buf * 64 * VP;
+      typedef __attribute__((address_space(3))) const bf16x8* lds_op;
+      typedef __attribute__((address_space(3))) s16x4* lds_tr;
+      unsigned ka = lds_k + buf * KTILE + k_lane, va = lds_v + buf * VTILE + v_lane, ta = lds_k + buf * KTILE + t_lane;
+      asm("" : "+v"(ka), "+v"(va), "+v"(ta));   // (three registers, the rest by XOR and offset fields)
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt) {
         // The LDS operands of the first two products form one stream (K row piece, V row piece, K, V, ...) that is
@@ -301,7 +295,7 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
         auto step_of = [&](const int j) __attribute__((always_inline)) { return j < 2 * NPAIR ? j >> 1 : j - NPAIR; };
         auto ld_op = [&](const int j) __attribute__((always_inline)) -> bf16x8 {
           const int st = step_of(j);
-          return is_v(j) ? ld8(Vb + (32 * kt + l32) * VP + 16 * st + 8 * hf) : ld8(Kb + (32 * kt + l32) * KP + 16 * st + 8 * hf);
+          return is_v(j) ? *reinterpret_cast<lds_op>((va ^ (32u * st)) + 32 * kt * VROWB) : *reinterpret_cast<lds_op>((ka ^ (32u * st)) + 32 * kt * KROWB);
         };
         bf16x8 op[NOPS + AHEAD];
 #pragma unroll
@@ -324,7 +318,9 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
         // dQ^T += K^T dS^T: the transposed K operands are read ahead as well, the first of them before the exponentials
         constexpr int N3 = 2 * DT, A3 = 4 < N3 ? 4 : N3;
         auto tr_op = [&](const int j) __attribute__((always_inline)) -> bf16x8 {
-          return tr_operand(Kb, KP, 32 * kt + 16 * (j / DT), 32 * (j % DT), lane);
+          const unsigned at = (32 * kt + 16 * (j / DT)) * KROWB, t64 = 64u * (j % DT);
+          return join4(__builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_tr>((ta ^ t64) + at)),
+                       __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_tr>((ta ^ (t64 + 32u)) + at + 8 * KROWB)));
         };
         bf16x8 at[N3 + A3];
 #pragma unroll
@@ -359,11 +355,8 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
         }
       }
     }
-    if (it + 1 < n_iters) {
-      sk.store(Ks + (buf ^ 1) * 64 * KP, tid);
-      sv.store(Vs + (buf ^ 1) * 64 * VP, tid);
-    }
     if (it + 2 < n_iters) ks_fetch = next_key_start();
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // this wave's requests of the next chunk have landed
     __syncthreads();
   }
 
@@ -825,12 +818,14 @@ static int cu_count() {
 
 template <int DK, int DV>
 static int launch_bwd(const SoftmaxBwdParams& p, hipStream_t stream) {
-  constexpr int KP = DK + 8, VP = DV + 8;
+  constexpr int KP = DK + 8;
   const long long rows = (long long)p.B * p.T * p.HQ;
   constexpr int RPB = 256 / (DV / 8);
   hipLaunchKernelGGL((delta_kernel<DV>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, stream, p);
   {
-    size_t lds = (size_t)2 * 64 * (KP + VP) * sizeof(bf16_t);
+    size_t lds = (size_t)2 * 64 * (DK + DV) * sizeof(bf16_t);                               // two buffers of K and V
+    const size_t epi = (size_t)128 * KP * sizeof(bf16_t);                                    // the output tile
+    if (epi > lds) lds = epi;
     auto kern = dq_kernel<DK, DV>;
     static std::atomic<unsigned long long> reserved{0};
     if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, lds, "softmax bwd")) return rc;

@@ -7,10 +7,10 @@
 //                  block, and every later chunk when the block is typed attention), for every query head of the group:
 //                  S = Q K^T, dP = dO V^T, dV^T += dO^T P, dK^T += Q^T dS, dnats += sum dS over later blocks (attns.py:719-983)
 //                  The query tiles (Q, dO, lse, delta) arrive by DMA in a ring of three LDS slots, two steps ahead.
-//                  One persistent workgroup per CU takes units from per-XCD work queues.  Eight waves in two roles:
-//                  four form S, P and dV, four form dP, dS and dK of the same (32 keys) x (32 queries) quarters; P
-//                  passes between the two in fp32 through LDS.  Each wave keeps one stationary operand and one
-//                  accumulator, so two waves fit a SIMD.
+//                  Persistent workgroups take units from per-XCD work queues.  K + V <= 192 (dkdv_whole_kernel): two
+//                  workgroups of four waves per CU, a wave forms everything of its (32 keys) x (32 queries) quarter.  K = V =
+//                  128: one of eight waves in two roles; four form S, P and dV, four form dP, dS and dK of the same
+//                  quarters, and P passes between the two in fp32 through LDS.
 //
 // Layouts follow the forward kernel: the stationary operand of a workgroup (Q, dO there; K, V here) sits in registers
 // as the B operand (lane = its row), the streamed tiles are row-major in LDS, the accumulators' own layout is the B
@@ -18,6 +18,7 @@
 // the transposing LDS read.
 #include "natsl_device.h"
 #include "natsl_host.h"
+#include <type_traits>
 
 namespace natsl {
 
@@ -386,7 +387,391 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// dk/dv.  Eight waves = 2 roles x 2 key halves x 2 query halves; a wave and its partner of the other role (wave + 4, on
+// Takes the next unit of the dk/dv kernels from the work queues.  Persistent workgroups take units = (sequence, kv head, key chunk):
+// starting a workgroup per unit left the CUs idle a quarter of the time.  Workgroups that run at the same time should stream the
+// same queries, so every XCD (block index mod 8) has a queue of its own with the key chunks of one (sequence, kv
+// head) after the other, earliest (heaviest) chunk first, and every unit walks the later query chunks from the last
+// one down: units started together stay together in L2.  A workgroup whose queue is empty takes from the other
+// XCDs' queues (q_probe: queues found empty so far; they stay empty).  Packed sequences: one queue, the units of a sequence (kv
+// head after kv head) after those of the one before.
+NATSL_DEVICE void dkdv_take_unit(const SoftmaxBwdParams& p, const bool packed, const bool per_xcd, const int n_queues, const int queue_len,
+                                 const int NT_reg, int& q_probe, int& pr, int& jj, int& seq) {
+  while (q_probe < n_queues) {
+    const int x = per_xcd ? ((int)blockIdx.x + q_probe) & 7 : 0;
+    const int i = atomicAdd(p.queue + x, 1);
+    if (i < queue_len) {
+      if (packed) {
+        int sn = 0;
+        for (int u = 1; u < p.n_seqs; ++u)
+          if (p.seqs[u].chunk_off * p.HKV <= i) sn = u;
+        const int r = i - p.seqs[sn].chunk_off * p.HKV, ntc = (p.seqs[sn].eos - p.seqs[sn].bos + 63) >> 6;
+        pr = r / ntc;   // the kv head
+        jj = r % ntc;
+        seq = sn;
+      } else {
+        pr = per_xcd ? (i / NT_reg) * 8 + x : i / NT_reg;
+        jj = i % NT_reg;
+      }
+      break;
+    }
+    ++q_probe;
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
+// dk/dv for K + V <= 192: a wave holds both stationary operands and both accumulators of its 32 keys (K 128, V 64: 144 registers), so
+// that it forms S, P, dP and dS of a 32 x 32 quarter and all four products by itself: nothing passes between waves inside a step.
+// Workgroups of four waves (2 key halves x 2 query halves), two per CU: each has its own ring and its own barrier, so one's
+// chain of LDS reads, exponentials and barrier runs under the others' matrix instructions, and so does what a unit costs besides its
+// steps (most units are a single step where a quarter of the blocks is attention).  Against the form with two roles below, which is
+// one workgroup of eight waves and 70 % more vector instructions a quarter: K 128, V 64, B4 T8192 H32, block 256, 25 % attention 1610
+// -> 1210 us; K 64, V 128, B8 T4096 H12, 50 % 600 -> 415; K = V = 64, B4 T4096 H32 330 -> 270.  What is left is the chain of a step
+// (about 2100 cycles a CU against 768 of matrix time): without the requests of the query tiles it is 15 % shorter, and fewer vector or
+// scalar instructions change it by 1 - 2 %.  Three workgroups per CU at K = V = 64 spill 36 registers a lane and take 390 us.
+constexpr int DKDV_WHOLE_WGS = 2;   // workgroups per CU (registers and LDS)
+
+template <int DK, int DV>
+struct DkdvWholeLds {
+  static constexpr unsigned DOFF = 64 * DK * 2, LOFF = DOFF + 64 * DV * 2, SLOT = LOFF + 512;   // slot: Q [64][DK], dO [64][DV], lse [64], delta [64]
+  static constexpr int TILES = DK / 32 + DV / 32, MINE = TILES / 2;                               // accumulator tiles; tiles a query half finishes
+  static constexpr unsigned SUMS = 2u * TILES * 4096;                                             // the unit's end: one query half's share of the other's tiles
+  static constexpr unsigned OROW = MINE * 64 + 16, OUT = 4u * 32 * OROW;                          // ... and the rows on their way out, per wave
+  static constexpr unsigned TOTAL = 3 * SLOT > SUMS + OUT ? 3 * SLOT : SUMS + OUT;
+};
+
+// INVALID: blocks that are not typed attention get dnats too (their units walk the later queries for nothing else)
+template <int DK, int DV, bool INVALID>
+__global__ __launch_bounds__(256, DKDV_WHOLE_WGS) void dkdv_whole_kernel(const SoftmaxBwdParams p) {
+  typedef DkdvWholeLds<DK, DV> L;
+  constexpr int KS = DK / 16, VS = DV / 16, KT = DK / 32, VT = DV / 32, KI = DK / 32, VI = DV / 32, NREQ = KI + VI + 1;
+  constexpr unsigned KROWB = DK * 2, VROWB = DV * 2, SLOT = L::SLOT;
+  extern __shared__ __align__(1024) unsigned char smem[];
+  __shared__ int unit[2][4];      // pair, chunk, sequence of the unit in work; in turn
+  __shared__ float red[4];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hf = lane >> 5;
+  const int kh = wave & 1, qh = wave >> 1;
+  const unsigned lds0 = (unsigned)(size_t)smem;
+  typedef __attribute__((address_space(3))) const bf16x8* lds_op;
+  typedef __attribute__((address_space(3))) const f32x4* lds_f4;
+  typedef __attribute__((address_space(3))) s16x4* lds_tr;
+
+  // requests: lane l of instruction j fills row rows_per_instr * j + l / segs, position l % segs of a tile, with the segment that the
+  // swizzle puts there (byte offsets from the tile's first row; the tail of a sequence clamps the rows)
+  const unsigned qrow = (unsigned)p.HQ * KROWB, drow = (unsigned)p.HQ * VROWB;
+  unsigned q_src[KI], d_src[VI];
+#pragma unroll
+  for (int j = 0; j < KI; ++j) {
+    const int r = (KI * wave + j) * (512 / DK) + lane / (DK / 8);
+    q_src[j] = (unsigned)r * qrow + 16u * (unsigned)((lane % (DK / 8)) ^ bwd_swizzle<DK>(r));
+  }
+#pragma unroll
+  for (int j = 0; j < VI; ++j) {
+    const int r = (VI * wave + j) * (512 / DV) + lane / (DV / 8);
+    d_src[j] = (unsigned)r * drow + 16u * (unsigned)((lane % (DV / 8)) ^ bwd_swizzle<DV>(r));
+  }
+  const unsigned l_src = (unsigned)lane * (unsigned)(p.HQ * 4);
+  // operand addresses inside a slot: the lane's query row (XOR with 32 st: k-step st), and the 4-element row piece it names in the
+  // transposing reads (XOR with 64 t: columns 32 t ..; XOR with 32 and 8 rows further: the second read)
+  const int i16 = lane & 15, trow = 32 * qh + 4 * hf + (i16 >> 2), tseg = 2 * ((lane >> 4) & 1) + ((i16 >> 1) & 1);
+  const unsigned q_lane = (unsigned)(32 * qh + l32) * KROWB + 16u * (unsigned)(hf ^ bwd_swizzle<DK>(l32));
+  const unsigned d_lane = L::DOFF + (unsigned)(32 * qh + l32) * VROWB + 16u * (unsigned)(hf ^ bwd_swizzle<DV>(l32));
+  const unsigned qt_lane = (unsigned)trow * KROWB + 16u * (unsigned)(tseg ^ bwd_swizzle<DK>(trow)) + 8u * (unsigned)(i16 & 1);
+  const unsigned dt_lane = L::DOFF + (unsigned)trow * VROWB + 16u * (unsigned)(tseg ^ bwd_swizzle<DV>(trow)) + 8u * (unsigned)(i16 & 1);
+
+  const bool packed = p.seqs != nullptr;
+  const int n_pairs = p.B * p.HKV;
+  // work queues as in the kernel below: one per XCD where the pairs divide evenly, else one
+  const int NT_reg = (p.T + 63) >> 6;
+  const bool per_xcd = !packed && n_pairs % 8 == 0;
+  const int n_queues = per_xcd ? 8 : 1;
+  const int queue_len = packed ? p.total_chunks * p.HKV : (per_xcd ? n_pairs / 8 : n_pairs) * NT_reg;
+  const float c = p.scale_log2;
+  int q_probe = 0;
+  for (int round = 0;; ++round) {
+    int* const un = unit[round & 1];
+    if (tid == 0) {
+      int pr = -1, jj = 0, sq = 0;
+      dkdv_take_unit(p, packed, per_xcd, n_queues, queue_len, NT_reg, q_probe, pr, jj, sq);
+      un[0] = pr;
+      un[1] = jj;
+      un[2] = sq;
+    }
+    __syncthreads();   // (also: the last unit's LDS is free)
+    const int pair = __builtin_amdgcn_readfirstlane(un[0]), jc = __builtin_amdgcn_readfirstlane(un[1]), seq = __builtin_amdgcn_readfirstlane(un[2]);
+    if (pair < 0) break;
+    const int n = packed ? seq : pair / p.HKV, hkv = packed ? pair : pair % p.HKV;
+    const int bos = packed ? p.seqs[n].bos : n * p.T, len = packed ? p.seqs[n].eos - bos : p.T;
+    const int bos_nats = packed ? p.seqs[n].bos_nats : n * p.TN;
+    const int NTc = (len + 63) >> 6;
+    const int Bs = p.block, per_blk = Bs >> 6;
+    const int G = p.HQ / p.HKV, GN = p.HQ / p.HN;
+    const int kb = (jc * 64) / Bs;
+    const int blk_end_chunk = min((kb + 1) * per_blk, NTc);
+
+    // the stationary operands: K and V of the wave's 32 keys (lane = key)
+    bf16x8 KB[KS], VB[VS];
+    {
+      const size_t krow0 = (size_t)(bos + min(jc * 64 + 32 * kh + l32, len - 1)) * p.HKV + hkv;
+      const bf16_t* kr = p.k + krow0 * DK + 8 * hf;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) KB[s] = ld8(kr + 16 * s);
+      const bf16_t* vr = p.v + krow0 * DV + 8 * hf;
+#pragma unroll
+      for (int s = 0; s < VS; ++s) VB[s] = ld8(vr + 16 * s);
+    }
+    f32x16 acc[KT + VT];   // dK tiles, then dV tiles
+#pragma unroll
+    for (int t = 0; t < KT + VT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+
+    for (int g = 0; g < G; ++g) {
+      const int hq = hkv * G + g, hn = hq / GN;
+      const bool attn = bwd_type_is_one(p.types, p.types_dtype, ((size_t)(bos_nats + kb) * p.HN + hn) * 2);
+      const int n_same = p.same_block ? blk_end_chunk - jc : 0;
+      const bool attn_u = __builtin_amdgcn_readfirstlane(attn ? 1 : 0) != 0;   // (the type was read by a vector load)
+      const int n_later = attn_u || INVALID ? max(NTc - blk_end_chunk, 0) : 0;
+      const int n_it = n_same + n_later;
+      float dn = 0.f;
+      // the query chunks from the last one that sees the keys down to the first: contiguous, the pointers below walk along
+      const int top = n_later > 0 ? NTc - 1 : blk_end_chunk - 1;
+      const size_t row0 = (size_t)(bos + top * 64) * p.HQ + hq;
+      const char* nq = reinterpret_cast<const char*>(p.q + row0 * DK);
+      const char* nd = reinterpret_cast<const char*>(p.dout + row0 * DV);
+      const char* nl = reinterpret_cast<const char*>((wave & 1 ? p.delta : p.lse) + row0);   // (two waves bring the same 256 bytes of either)
+      auto advance = [&]() __attribute__((always_inline)) {
+        nq -= 64ull * qrow;
+        nd -= 64ull * drow;
+        nl -= 256ull * p.HQ;
+      };
+      auto request = [&](const int slot) __attribute__((always_inline)) {
+        const unsigned sl = lds0 + slot * SLOT;
+#pragma unroll
+        for (int j = 0; j < KI; ++j) dma16(nq, q_src[j], sl + (KI * wave + j) * 1024);
+#pragma unroll
+        for (int j = 0; j < VI; ++j) dma16(nd, d_src[j], sl + L::DOFF + (VI * wave + j) * 1024);
+        dma4(nl, l_src, sl + L::LOFF + 256 * (wave & 1));
+        advance();
+      };
+      if (n_it > 0) {
+        const int last = len - 1 - top * 64;   // the first tile's last row of the sequence; all others are full
+        if (last >= 63) {
+          request(0);
+        } else {
+          int cl = lane;
+          asm volatile("" : "+v"(cl));   // (row numbers are not to be kept for this)
+#pragma unroll
+          for (int j = 0; j < KI; ++j) {
+            const int r = (KI * wave + j) * (512 / DK) + cl / (DK / 8);
+            dma16(nq, q_src[j] - (unsigned)(r - min(r, last)) * qrow, lds0 + (KI * wave + j) * 1024);
+          }
+#pragma unroll
+          for (int j = 0; j < VI; ++j) {
+            const int r = (VI * wave + j) * (512 / DV) + cl / (DV / 8);
+            dma16(nd, d_src[j] - (unsigned)(r - min(r, last)) * drow, lds0 + L::DOFF + (VI * wave + j) * 1024);
+          }
+          dma4(nl, (unsigned)min(cl, last) * (unsigned)(p.HQ * 4), lds0 + L::LOFF + 256 * (wave & 1));
+          advance();
+        }
+        if (n_it > 1) {
+          request(1);
+          __builtin_amdgcn_s_waitcnt(0x0f70 | NREQ);   // all but the newest tile's requests
+        } else {
+          __builtin_amdgcn_s_waitcnt(0x0f70);
+        }
+        __syncthreads();
+      }
+      int slot = 0;
+      for (int it = 0; it < n_it; ++it) {
+        const int jq = top - it;
+        const bool own = jq == jc;
+        // the tile two steps ahead goes into the slot of the previous step, which every wave has left
+        const bool ask = it + 2 < n_it;
+        if (ask) request(slot == 0 ? 2 : slot - 1);
+        // (in the own chunk the later keys see nothing of the earlier queries)
+        if (!(own && kh == 1 && qh == 0)) {
+          // keys the queries do not see: probabilities against the queries' lse, clamped to 1 as the reference does, enter
+          // dnats only (their products run on zeros)
+          const bool only_dn = INVALID && !attn_u && it < n_later;
+          const unsigned sb = lds0 + slot * SLOT;
+          unsigned qa = sb + q_lane, da = sb + d_lane, qt = sb + qt_lane, dt = sb + dt_lane;
+          asm("" : "+v"(qa), "+v"(da), "+v"(qt), "+v"(dt));   // (four registers, the rest by XOR and offset fields)
+          // ---- S = Q K^T and dP = dO V^T: one stream of row operands (Q, dO, Q, dO, ..., the longer one's rest), read ahead
+          constexpr int NOPS = KS + VS, AHEAD = 4, NPAIR = KS < VS ? KS : VS;
+          auto is_d = [&](const int j) __attribute__((always_inline)) { return j < 2 * NPAIR ? (j & 1) != 0 : VS > KS; };
+          auto step_of = [&](const int j) __attribute__((always_inline)) { return j < 2 * NPAIR ? j >> 1 : j - NPAIR; };
+          auto ld_op = [&](const int j) __attribute__((always_inline)) -> bf16x8 {
+            return *reinterpret_cast<lds_op>((is_d(j) ? da : qa) ^ (32u * step_of(j)));
+          };
+          bf16x8 op[NOPS + AHEAD];
+#pragma unroll
+          for (int j = 0; j < AHEAD; ++j) op[j] = ld_op(j);
+          f32x16 s, dp;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
+#pragma unroll
+          for (int j = 0; j < NOPS; ++j) {
+            if (j + AHEAD < NOPS) op[j + AHEAD] = ld_op(j + AHEAD);
+            if (is_d(j)) dp = mfma32(op[j], VB[step_of(j)], dp);
+            else s = mfma32(op[j], KB[step_of(j)], s);
+          }
+          __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+#pragma unroll
+          for (int j = 0; j < NOPS; ++j) {
+            if (j + AHEAD < NOPS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          }
+          // the rows' lse and delta, and the first transposed operands
+          const unsigned lb = sb + L::LOFF + 4u * (unsigned)(32 * qh + 4 * hf);
+          f32x4 ls[4], dl[4];
+#pragma unroll
+          for (int rg = 0; rg < 4; ++rg) ls[rg] = *reinterpret_cast<lds_f4>(lb + 32 * rg);
+          // ---- dV^T += dO^T P, dK^T += Q^T dS: operand j = (16-query group, tile), the dV tiles of both groups first
+          constexpr int NV = 2 * VT, N2 = NV + 2 * KT, A2 = 4;
+          auto tr_op = [&](const int j) __attribute__((always_inline)) -> bf16x8 {
+            const int ss = j < NV ? j / VT : (j - NV) / KT, t = j < NV ? j % VT : (j - NV) % KT;
+            const unsigned base = j < NV ? dt : qt, rowb = j < NV ? VROWB : KROWB, at = 16u * ss * rowb, t64 = 64u * t;
+            return join4(__builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_tr>((base ^ t64) + at)),
+                         __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<lds_tr>((base ^ (t64 + 32u)) + at + 8 * rowb)));
+          };
+          bf16x8 at[N2 + A2];
+#pragma unroll
+          for (int j = 0; j < A2; ++j) at[j] = tr_op(j);
+          __builtin_amdgcn_sched_barrier(0);
+          if (!own && jq * 64 + 64 <= len) {   // every (query, key) pair of the tile is visible: no masks
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], c, -ls[r >> 2][r & 3]));
+          } else {
+            // query 32 qh + 4 hf + 8 (r/4) + r%4 of the tile: from the lane's key on (own chunk), up to the sequence's end
+            int first = own ? 32 * kh + l32 - 32 * qh - 4 * hf : 0, end = len - jq * 64 - 32 * qh - 4 * hf;
+            asm volatile("" : "+v"(first), "+v"(end));   // (kept here: hoisted, the comparisons are held in registers through the loop)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+              const bool vis = 8 * (r >> 2) + (r & 3) >= first && 8 * (r >> 2) + (r & 3) < end;
+              s[r] = vis ? __builtin_amdgcn_exp2f(fmaf(s[r], c, -ls[r >> 2][r & 3])) : 0.f;
+            }
+          }
+          if constexpr (INVALID) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = only_dn ? fminf(s[r], 1.f) : s[r];
+          }
+#pragma unroll
+          for (int rg = 0; rg < 4; ++rg) dl[rg] = *reinterpret_cast<lds_f4>(lb + 256 + 32 * rg);
+          bf16x8 PB[4];
+          PB[0] = pack8(s, 0);
+          PB[1] = pack8(s, 1);
+          float dsum = 0.f;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            dp[r] = s[r] * (dp[r] - dl[r >> 2][r & 3]);
+            dsum += dp[r];
+          }
+          dn += it < n_later && jc * 64 + 32 * kh + l32 < len ? dsum : 0.f;
+          PB[2] = pack8(dp, 0);
+          PB[3] = pack8(dp, 1);
+          if constexpr (INVALID) {
+            const u32x4 on = only_dn ? u32x4{0u, 0u, 0u, 0u} : u32x4{~0u, ~0u, ~0u, ~0u};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) PB[i] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, PB[i]) & on);
+          }
+#pragma unroll
+          for (int j = 0; j < N2; ++j) {
+            if (j + A2 < N2) at[j + A2] = tr_op(j + A2);
+            if (j < NV) acc[KT + j % VT] = mfma32(at[j], PB[j / VT], acc[KT + j % VT]);
+            else acc[(j - NV) % KT] = mfma32(at[j], PB[2 + (j - NV) / KT], acc[(j - NV) % KT]);
+          }
+          // dS is formed under the dV products, its sum under the dK products
+          __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);   // delta
+          __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);   // P packed
+#pragma unroll
+          for (int j = 0; j < N2; ++j) {
+            if (j + A2 < N2) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (j < NV) __builtin_amdgcn_sched_group_barrier(0x002, 44 / NV, 0);
+            else __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+          }
+        }
+        // this wave's requests of the next tile have landed (those of the one after it may stay in flight)
+        if (ask) __builtin_amdgcn_s_waitcnt(0x0f70 | NREQ);
+        else __builtin_amdgcn_s_waitcnt(0x0f70);
+        __syncthreads();
+        slot = slot == 2 ? 0 : slot + 1;
+      }
+      // dnats of this (key block, query head): the sums of the four waves
+      if (n_later > 0) {
+#pragma unroll
+        for (int m = 32; m >= 1; m >>= 1) dn += __shfl_xor(dn, m);
+        if (lane == 0) red[wave] = dn;
+        __syncthreads();
+        if (tid == 0) atomicAdd(p.dnats + ((size_t)(bos_nats + kb)) * p.HQ + hq, red[0] + red[1] + red[2] + red[3]);
+        if (g + 1 < G) __syncthreads();
+      }
+    }
+
+    // ---- the two query halves of a key half are added through LDS, each half finishing the sum of half of the tiles, which then
+    // leave through LDS as whole rows.  (Every wave has left the ring: the last step ended with a barrier.)
+    constexpr int MINE = L::MINE;
+    int ol = lane;
+    asm volatile("" : "+v"(ol));   // (the lane's share of the addresses below is not to be kept through the steps)
+    const unsigned sums = lds0 + (unsigned)kh * (L::TILES * 4096u) + 16u * ol, outb = lds0 + L::SUMS + (unsigned)wave * (32u * L::OROW);
+    typedef __attribute__((address_space(3))) f32x4* lds_w4;
+    typedef __attribute__((address_space(3))) u32x2* lds_w2;
+    typedef __attribute__((address_space(3))) const u32x4* lds_r4;
+    auto finish = [&](auto first_c) __attribute__((always_inline)) {
+      constexpr int FIRST = decltype(first_c)::value, OTHER = FIRST == 0 ? MINE : 0;
+#pragma unroll
+      for (int t = 0; t < MINE; ++t)
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg)
+          *reinterpret_cast<lds_w4>(sums + (OTHER + t) * 4096u + rg * 1024u) =
+              f32x4{acc[OTHER + t][4 * rg], acc[OTHER + t][4 * rg + 1], acc[OTHER + t][4 * rg + 2], acc[OTHER + t][4 * rg + 3]};
+      __syncthreads();
+      f32x4 xs[MINE * 4];
+#pragma unroll
+      for (int i = 0; i < MINE * 4; ++i) xs[i] = *reinterpret_cast<lds_w4>(sums + (FIRST + i / 4) * 4096u + (i & 3) * 1024u);
+#pragma unroll
+      for (int t = 0; t < MINE; ++t) {
+        const float mul = FIRST + t < KT ? p.scale : 1.f;
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg) {
+          const f32x4 mine = {acc[FIRST + t][4 * rg], acc[FIRST + t][4 * rg + 1], acc[FIRST + t][4 * rg + 2], acc[FIRST + t][4 * rg + 3]};
+          const f32x4 sum = mine + xs[4 * t + rg];
+          u32x2 w;
+          w[0] = pack_bf16x2(sum[0] * mul, sum[1] * mul);
+          w[1] = pack_bf16x2(sum[2] * mul, sum[3] * mul);
+          *reinterpret_cast<lds_w2>(outb + (unsigned)(ol & 31) * L::OROW + 64u * t + 16u * rg + 8u * (unsigned)(ol >> 5)) = w;
+        }
+      }
+      __builtin_amdgcn_s_waitcnt(0xc07f);
+      __builtin_amdgcn_wave_barrier();
+      // lanes take the 16-byte pieces of the rows' dK part, then of their dV part
+      constexpr int NK = FIRST < KT ? (KT - FIRST < MINE ? KT - FIRST : MINE) : 0, NVT = MINE - NK;   // dK and dV tiles of this half
+      auto store_part = [&](auto tiles_c, const int tile0, bf16_t* out, const int width, const int col0) __attribute__((always_inline)) {
+        constexpr int TL = decltype(tiles_c)::value, SEGS = 4 * TL, PIECES = 32 * SEGS / 64;
+        u32x4 w[PIECES > 0 ? PIECES : 1];
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+          const int e = ol + 64 * i, row = e / SEGS, seg = e % SEGS;
+          w[i] = *reinterpret_cast<lds_r4>(outb + (unsigned)row * L::OROW + 64u * tile0 + 16u * seg);
+        }
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+          const int e = ol + 64 * i, row = e / SEGS, seg = e % SEGS, tk = jc * 64 + 32 * kh + row;
+          if (tk < len) *reinterpret_cast<u32x4*>(out + ((size_t)(bos + tk) * p.HKV + hkv) * width + col0 + 8 * seg) = w[i];
+        }
+      };
+      if constexpr (NK > 0) store_part(std::integral_constant<int, NK>{}, 0, p.dk, DK, 32 * FIRST);
+      if constexpr (NVT > 0) store_part(std::integral_constant<int, NVT>{}, NK, p.dv, DV, 32 * (FIRST + NK - KT));
+    };
+    if (qh == 0) finish(std::integral_constant<int, 0>{});
+    else finish(std::integral_constant<int, MINE>{});
+  }  // units
+}
+
+// ---------------------------------------------------------------------------------------------
+// dk/dv for K = V = 128, where a wave cannot hold both operands and both accumulators.  Eight waves = 2 roles x 2 key halves x 2 query halves; a wave and its partner of the other role (wave + 4, on
 // the same SIMD) work on the same 32 keys x 32 queries of every step:
 //   role 0: S = Q K^T, P = exp2(S c - lse) (masks, the clamp for blocks that only give dnats), dV^T += dO^T P
 //   role 1: dP = dO V^T, dS = P (dP - delta), dK^T += Q^T dS, dnats
@@ -425,13 +810,7 @@ NATSL_DEVICE void dkdv_role(const SoftmaxBwdParams& p, unsigned char* smem, Dkdv
   const int kh = quad & 1, qh = quad >> 1;
   const bool packed = p.seqs != nullptr;
   const int n_pairs = p.B * p.HKV;
-  // ---- Persistent workgroups (one per CU) take units = (sequence, kv head, key chunk) from work queues: starting a
-  // workgroup per unit left the CUs idle a quarter of the time.  Workgroups that run at the same time should stream the
-  // same queries, so every XCD (block index mod 8) has a queue of its own with the key chunks of one (sequence, kv
-  // head) after the other, earliest (heaviest) chunk first, and every unit walks the later query chunks from the last
-  // one down: units started together stay together in L2.  A workgroup whose queue is empty takes from the other
-  // XCDs' queues.  Packed sequences: one queue, the units of a sequence (kv head after kv head) after those of the one
-  // before.
+  // ---- persistent workgroups, one per CU (see dkdv_take_unit)
   const int NT_reg = (p.T + 63) >> 6;
   const bool per_xcd = !packed && n_pairs % 8 == 0;
   const int n_queues = per_xcd ? 8 : 1;
@@ -439,27 +818,9 @@ NATSL_DEVICE void dkdv_role(const SoftmaxBwdParams& p, unsigned char* smem, Dkdv
   int q_probe = 0;   // queues found empty so far (they stay empty)
   for (;;) {
     if (tid == 0) {
-      int pr = -1, jj = 0;
-      while (q_probe < n_queues) {
-        const int x = per_xcd ? ((int)blockIdx.x + q_probe) & 7 : 0;
-        const int i = atomicAdd(p.queue + x, 1);
-        if (i < queue_len) {
-          if (packed) {
-            int sn = 0;
-            for (int u = 1; u < p.n_seqs; ++u)
-              if (p.seqs[u].chunk_off * p.HKV <= i) sn = u;
-            const int r = i - p.seqs[sn].chunk_off * p.HKV, ntc = (p.seqs[sn].eos - p.seqs[sn].bos + 63) >> 6;
-            pr = r / ntc;   // the kv head
-            jj = r % ntc;
-            sh.unit_seq = sn;
-          } else {
-            pr = per_xcd ? (i / NT_reg) * 8 + x : i / NT_reg;
-            jj = i % NT_reg;
-          }
-          break;
-        }
-        ++q_probe;
-      }
+      int pr = -1, jj = 0, sq = 0;
+      dkdv_take_unit(p, packed, per_xcd, n_queues, queue_len, NT_reg, q_probe, pr, jj, sq);
+      sh.unit_seq = sq;
       sh.unit_pair = pr;
       sh.unit_jc = jj;
     }
@@ -832,16 +1193,24 @@ static int launch_bwd(const SoftmaxBwdParams& p, hipStream_t stream) {
     const long long grid = p.seqs ? (long long)p.total_tiles * 2 * p.HQ : ((long long)p.B * p.HQ + 7) / 8 * 8 * ((p.T + 127) / 128);
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, stream, p);
   }
-  {
-    const size_t lds = DkdvLds<DK, DV>::TOTAL;   // the ring of three query tiles and the exchange buffers
-    auto kern = dkdv_kernel<DK, DV>;
-    static std::atomic<unsigned long long> reserved{0};
+  const long long units = p.seqs ? (long long)p.total_chunks * p.HKV : (long long)p.B * p.HKV * ((p.T + 63) / 64);
+  auto dkdv = [&](auto kern, std::atomic<unsigned long long>& reserved, const size_t lds, const int threads, const int per_cu) -> int {
     if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, lds, "softmax bwd")) return rc;
-    const long long units = p.seqs ? (long long)p.total_chunks * p.HKV : (long long)p.B * p.HKV * ((p.T + 63) / 64);
-    long long grid = (cu_count() + 7) / 8 * 8;   // whole groups of 8: block index mod 8 names the XCD and its queue
+    long long grid = (long long)(cu_count() + 7) / 8 * 8 * per_cu;   // whole groups of 8: block index mod 8 names the XCD and its queue
     if (grid > units) grid = units;
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), lds, stream, p);
-  }
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(threads), lds, stream, p);
+    return NATSL_OK;
+  };
+  // (192: both operands, both accumulators and a quarter's scores fit the 256 registers that two waves a SIMD leave)
+  static std::atomic<unsigned long long> reserved{0};
+  int rc;
+  if constexpr (DK + DV <= 192) {
+    static std::atomic<unsigned long long> reserved_invalid{0};
+    constexpr size_t lds = DkdvWholeLds<DK, DV>::TOTAL;
+    rc = p.dnats_invalid ? dkdv(dkdv_whole_kernel<DK, DV, true>, reserved_invalid, lds, 256, DKDV_WHOLE_WGS)
+                         : dkdv(dkdv_whole_kernel<DK, DV, false>, reserved, lds, 256, DKDV_WHOLE_WGS);
+  } else rc = dkdv(dkdv_kernel<DK, DV>, reserved, DkdvLds<DK, DV>::TOTAL, 512, 1);   // the ring of three query tiles and the exchange buffers
+  if (rc != NATSL_OK) return rc;
   return check_launch("natsl_softmax_sparse_bwd");
 }
 

@@ -95,6 +95,17 @@ def test_softmax_bwd_many_pairs_and_long_walks():
     _run(1, 1000, 8, 8, 8, 128, 64, 128, 0.5, True, seed=22)     # ragged last tile, blocks of two chunks
 
 
+@pytest.mark.parametrize("T,HQ,H,block,dnats_invalid", [(2, 2, 2, 64, False), (63, 2, 2, 64, True), (65, 4, 2, 64, False),
+                                                        (191, 2, 2, 128, True), (256, 4, 4, 64, False), (449, 4, 1, 64, True)])
+@pytest.mark.parametrize("K,V", [(64, 64), (64, 128), (128, 64)])
+def test_softmax_bwd_whole_quarters(K, V, T, HQ, H, block, dnats_invalid):
+    """K + V <= 192: the dk/dv kernel whose waves form all four products.  Walks of one, two and three or more tiles (its ring holds
+    three), a ragged tile as the first of a walk, a block's own chunks behind the later ones, grouped query heads.  (Two tokens are the least: with one, dq and dk are exactly 0 and
+    what the kernel leaves is the fp32 rounding of dP - delta, 2e-7 measured, which has no relative error to speak of.)"""
+    for same_block in (True, False):
+        _run(1, T, HQ, H, H, K, V, block, 0.6, same_block, seed=40, dnats_invalid=dnats_invalid)
+
+
 def test_softmax_bwd_repeatable_and_workspace_reuse():
     """The dk/dv kernel takes its units from work queues in whatever order the workgroups arrive: dq, dk, dv must not
     depend on it (bit-identical from launch to launch; dnats is summed with float atomics and may differ in the last

@@ -1,8 +1,9 @@
 // Backward of the softmax branch for gfx950.
 //
-//   delta_kernel   delta[t] = sum_v dO[t,v] O[t,v]                                  (attns.py:357-372)
+//   delta_kernel   -delta[t] = -sum_v dO[t,v] O[t,v]                                (attns.py:357-372)
 //   dq_kernel      one workgroup per tile of 128 queries, the forward's walk over the visible key chunks:
-//                  S^T = K Q^T, P = exp2(S c - lse), dP^T = V dO^T, dS = P (dP - delta), dQ^T += K^T dS^T (attns.py:383-708)
+//                  S^T = K Q^T, P = exp2(S c - lse), dP^T - delta = V dO^T - delta (the accumulators start from -delta),
+//                  dS = P (dP - delta), dQ^T += K^T dS^T (attns.py:383-708)
 //   dkdv_kernel    unit = one 64-key chunk of a kv head, walking the query chunks that see it (the rest of its own
 //                  block, and every later chunk when the block is typed attention), for every query head of the group:
 //                  S = Q K^T, dP = dO V^T, dV^T += dO^T P, dK^T += Q^T dS, dnats += sum dS over later blocks (attns.py:719-983)
@@ -27,7 +28,7 @@ struct SoftmaxBwdParams {
   const float* lse;
   bf16_t *dq, *dk, *dv;
   float* dnats;   // [B, TN, HQ], zero on entry
-  float* delta;   // [B, T, HQ] workspace
+  float* ndelta;  // [B, T, HQ] workspace: -delta
   int* queue;     // [8] workspace: next unit of each XCD's list for the dk/dv kernel, zeroed by the delta kernel
   const void* types;
   int types_dtype;
@@ -112,7 +113,7 @@ __global__ __launch_bounds__(256) void delta_kernel(const SoftmaxBwdParams p) {
   }
 #pragma unroll
   for (int m = LPR / 2; m >= 1; m >>= 1) acc += __shfl_xor(acc, m);
-  if (row < rows && seg == 0) p.delta[row] = acc;
+  if (row < rows && seg == 0) p.ndelta[row] = -acc;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -183,7 +184,16 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
 #pragma unroll
     for (int s = 0; s < VS; ++s) DOB[s] = ld8(dr + 16 * s);
   }
-  const float lse_q = p.lse[(size_t)(bos + qi) * p.HQ + hq], delta_q = p.delta[(size_t)(bos + qi) * p.HQ + hq];
+  const float lse_q = p.lse[(size_t)(bos + qi) * p.HQ + hq];
+  // -delta of the lane's query: what the dP accumulators start from.  K = V = 64 subtracts it afterwards: with the sixteen registers
+  // that hold it, a third wave no longer fits the SIMD (153 -> 187 us at B4 T4096 H32).
+  constexpr bool FOLD = DK + DV > 128;
+  f32x16 ndelta;
+  {
+    const float d = p.ndelta[(size_t)(bos + qi) * p.HQ + hq];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) ndelta[r] = d;
+  }
 
   f32x16 acc[DT];
 #pragma unroll
@@ -307,7 +317,7 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
 #pragma unroll
         for (int j = 0; j < NOPS; ++j) {
           if (j + AHEAD < NOPS) op[j + AHEAD] = ld_op(j + AHEAD);
-          if (is_v(j)) dp = mfma32(op[j], DOB[step_of(j)], dp);
+          if (is_v(j)) dp = mfma32(op[j], DOB[step_of(j)], FOLD && step_of(j) == 0 ? ndelta : dp);
           else s = mfma32(op[j], QB[step_of(j)], s);
         }
         __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
@@ -330,14 +340,14 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
         f32x16 ds;
         if (!causal) {   // every key of the chunk is visible to every query of the wave: no masks
 #pragma unroll
-          for (int r = 0; r < 16; ++r) ds[r] = __builtin_amdgcn_exp2f(fmaf(s[r], c, -lse_q)) * (dp[r] - delta_q);
+          for (int r = 0; r < 16; ++r) ds[r] = __builtin_amdgcn_exp2f(fmaf(s[r], c, -lse_q)) * (FOLD ? dp[r] : dp[r] + ndelta[r]);
         } else {
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const int kloc = 32 * kt + 8 * (r >> 2) + 4 * hf + (r & 3);
             const bool vis = kloc <= qloc0 + l32;
             const float pr = vis ? __builtin_amdgcn_exp2f(fmaf(s[r], c, -lse_q)) : 0.f;
-            ds[r] = pr * (dp[r] - delta_q);
+            ds[r] = pr * (FOLD ? dp[r] : dp[r] + ndelta[r]);
           }
         }
         bf16x8 PB[2];
@@ -432,7 +442,7 @@ constexpr int DKDV_WHOLE_WGS = 2;   // workgroups per CU (registers and LDS)
 
 template <int DK, int DV>
 struct DkdvWholeLds {
-  static constexpr unsigned DOFF = 64 * DK * 2, LOFF = DOFF + 64 * DV * 2, SLOT = LOFF + 512;   // slot: Q [64][DK], dO [64][DV], lse [64], delta [64]
+  static constexpr unsigned DOFF = 64 * DK * 2, LOFF = DOFF + 64 * DV * 2, SLOT = LOFF + 512;   // slot: Q [64][DK], dO [64][DV], lse [64], -delta [64]
   static constexpr int TILES = DK / 32 + DV / 32, MINE = TILES / 2;                               // accumulator tiles; tiles a query half finishes
   static constexpr unsigned SUMS = 2u * TILES * 4096;                                             // the unit's end: one query half's share of the other's tiles
   static constexpr unsigned OROW = MINE * 64 + 16, OUT = 4u * 32 * OROW;                          // ... and the rows on their way out, per wave
@@ -540,7 +550,7 @@ __global__ __launch_bounds__(256, DKDV_WHOLE_WGS) void dkdv_whole_kernel(const S
       const size_t row0 = (size_t)(bos + top * 64) * p.HQ + hq;
       const char* nq = reinterpret_cast<const char*>(p.q + row0 * DK);
       const char* nd = reinterpret_cast<const char*>(p.dout + row0 * DV);
-      const char* nl = reinterpret_cast<const char*>((wave & 1 ? p.delta : p.lse) + row0);   // (two waves bring the same 256 bytes of either)
+      const char* nl = reinterpret_cast<const char*>((wave & 1 ? p.ndelta : p.lse) + row0);   // (two waves bring the same 256 bytes of either)
       auto advance = [&]() __attribute__((always_inline)) {
         nq -= 64ull * qrow;
         nd -= 64ull * drow;
@@ -608,24 +618,28 @@ __global__ __launch_bounds__(256, DKDV_WHOLE_WGS) void dkdv_whole_kernel(const S
           bf16x8 op[NOPS + AHEAD];
 #pragma unroll
           for (int j = 0; j < AHEAD; ++j) op[j] = ld_op(j);
-          f32x16 s, dp;
+          const unsigned lb = sb + L::LOFF + 4u * (unsigned)(32 * qh + 4 * hf);
+          f32x16 s, dp;   // dP starts from the rows' -delta
 #pragma unroll
-          for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
+          for (int rg = 0; rg < 4; ++rg) {
+            const f32x4 nd = *reinterpret_cast<lds_f4>(lb + 256 + 32 * rg);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) { s[4 * rg + r] = 0.f; dp[4 * rg + r] = nd[r]; }
+          }
 #pragma unroll
           for (int j = 0; j < NOPS; ++j) {
             if (j + AHEAD < NOPS) op[j + AHEAD] = ld_op(j + AHEAD);
             if (is_d(j)) dp = mfma32(op[j], VB[step_of(j)], dp);
             else s = mfma32(op[j], KB[step_of(j)], s);
           }
-          __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, AHEAD + 4, 0);
 #pragma unroll
           for (int j = 0; j < NOPS; ++j) {
             if (j + AHEAD < NOPS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
           }
-          // the rows' lse and delta, and the first transposed operands
-          const unsigned lb = sb + L::LOFF + 4u * (unsigned)(32 * qh + 4 * hf);
-          f32x4 ls[4], dl[4];
+          // the rows' lse, and the first transposed operands
+          f32x4 ls[4];
 #pragma unroll
           for (int rg = 0; rg < 4; ++rg) ls[rg] = *reinterpret_cast<lds_f4>(lb + 32 * rg);
           // ---- dV^T += dO^T P, dK^T += Q^T dS: operand j = (16-query group, tile), the dV tiles of both groups first
@@ -657,15 +671,13 @@ __global__ __launch_bounds__(256, DKDV_WHOLE_WGS) void dkdv_whole_kernel(const S
 #pragma unroll
             for (int r = 0; r < 16; ++r) s[r] = only_dn ? fminf(s[r], 1.f) : s[r];
           }
-#pragma unroll
-          for (int rg = 0; rg < 4; ++rg) dl[rg] = *reinterpret_cast<lds_f4>(lb + 256 + 32 * rg);
           bf16x8 PB[4];
           PB[0] = pack8(s, 0);
           PB[1] = pack8(s, 1);
           float dsum = 0.f;
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            dp[r] = s[r] * (dp[r] - dl[r >> 2][r & 3]);
+            dp[r] *= s[r];
             dsum += dp[r];
           }
           dn += it < n_later && jc * 64 + 32 * kh + l32 < len ? dsum : 0.f;
@@ -683,13 +695,12 @@ __global__ __launch_bounds__(256, DKDV_WHOLE_WGS) void dkdv_whole_kernel(const S
             else acc[(j - NV) % KT] = mfma32(at[j], PB[2 + (j - NV) / KT], acc[(j - NV) % KT]);
           }
           // dS is formed under the dV products, its sum under the dK products
-          __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);   // delta
           __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);   // P packed
 #pragma unroll
           for (int j = 0; j < N2; ++j) {
             if (j + A2 < N2) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (j < NV) __builtin_amdgcn_sched_group_barrier(0x002, 44 / NV, 0);
+            if (j < NV) __builtin_amdgcn_sched_group_barrier(0x002, 28 / NV, 0);
             else __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
           }
         }
@@ -786,7 +797,7 @@ struct DkdvShared {
 template <int DK, int DV>
 struct DkdvLds {
   static constexpr int QROWB = DK * 2, DROWB = DV * 2;
-  static constexpr unsigned DOFF = 64 * QROWB, LOFF = DOFF + 64 * DROWB, SLOT = LOFF + 512;   // slot: Q [64][DK], dO [64][DV], lse [64], delta [64]
+  static constexpr unsigned DOFF = 64 * QROWB, LOFF = DOFF + 64 * DROWB, SLOT = LOFF + 512;   // slot: Q [64][DK], dO [64][DV], lse [64], -delta [64]
   static constexpr unsigned XOFF = 3 * SLOT, XBUF = 4 * 4096;   // P exchange: [2][4 wave pairs][4][64 lanes] of 4 floats
   static constexpr unsigned RING = XOFF + 2 * XBUF;
   static constexpr unsigned RED = 2u * (DV / 32 + DK / 32) * 16 * 64 * sizeof(float);   // the unit's end: sums of the query halves
@@ -868,7 +879,7 @@ NATSL_DEVICE void dkdv_role(const SoftmaxBwdParams& p, unsigned char* smem, Dkdv
       r_seg[j] = 16u * (pos ^ bwd_swizzle<D1>(row));
     }
     const bf16_t* g_src = ROLE == 0 ? p.q : p.dout;
-    const float* l_src = ROLE == 0 ? p.lse : p.delta;
+    const float* l_src = ROLE == 0 ? p.lse : p.ndelta;
     // request piece r of tile jq of head hq into a slot
     auto piece = [&](const int r, const int hq, const int jq, const int slot, const void*& g, unsigned& voff, unsigned& dst) __attribute__((always_inline)) {
       const unsigned sl = lds0 + slot * SLOT;
@@ -982,7 +993,7 @@ NATSL_DEVICE void dkdv_role(const SoftmaxBwdParams& p, unsigned char* smem, Dkdv
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
           }
         }
-        // the rows' lse (role 0) or delta (role 1)
+        // the rows' lse (role 0) or -delta (role 1)
         const float* Lb = reinterpret_cast<const float*>(smem + slot * SLOT + LOFF) + 64 * ROLE;
         f32x4 l4[4];
 #pragma unroll
@@ -1054,7 +1065,7 @@ NATSL_DEVICE void dkdv_role(const SoftmaxBwdParams& p, unsigned char* smem, Dkdv
           f32x16 ds;
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            ds[r] = p4[r >> 2][r & 3] * (x[r] - l4[r >> 2][r & 3]);
+            ds[r] = p4[r >> 2][r & 3] * (x[r] + l4[r >> 2][r & 3]);
             dsum += ds[r];
           }
           if (it >= n_same && jc * 64 + 32 * kh + l32 < len) dn += dsum;
@@ -1218,7 +1229,7 @@ static int launch_bwd(const SoftmaxBwdParams& p, hipStream_t stream) {
 
 using namespace natsl;
 
-// delta [B, T, HQ] fp32, then the dk/dv kernel's 8 work-queue counters
+// -delta [B, T, HQ] fp32, then the dk/dv kernel's 8 work-queue counters
 static size_t bwd_queue_offset(int B, int T, int HQ) { return ((size_t)B * T * HQ * sizeof(float) + 255) / 256 * 256; }
 extern "C" size_t natsl_softmax_bwd_workspace_bytes(int B, int T, int HQ) { return bwd_queue_offset(B, T, HQ) + 256; }
 
@@ -1249,7 +1260,7 @@ extern "C" int natsl_softmax_sparse_bwd(const void* q, const void* k, const void
     return fail(NATSL_ERR_WORKSPACE, "%s: workspace of %zu bytes needed", what, natsl_softmax_bwd_workspace_bytes(B, T, HQ));
   SoftmaxBwdParams p;
   p.q = (const bf16_t*)q; p.k = (const bf16_t*)k; p.v = (const bf16_t*)v; p.o = (const bf16_t*)o; p.dout = (const bf16_t*)d_o;
-  p.lse = lse; p.dq = (bf16_t*)dq; p.dk = (bf16_t*)dk; p.dv = (bf16_t*)dv; p.dnats = dnats; p.delta = (float*)workspace;
+  p.lse = lse; p.dq = (bf16_t*)dq; p.dk = (bf16_t*)dk; p.dv = (bf16_t*)dv; p.dnats = dnats; p.ndelta = (float*)workspace;
   p.queue = reinterpret_cast<int*>(static_cast<char*>(workspace) + bwd_queue_offset(B, T, HQ));
   p.types = types; p.types_dtype = types_dtype; p.idx = nats_block_indices; p.nblk = n_nats_blocks;
   p.B = B; p.T = T; p.HQ = HQ; p.HKV = HKV; p.HN = HN; p.TN = TN; p.block = block;

@@ -674,6 +674,18 @@ __global__ __launch_bounds__(256, DKDV_WHOLE_WGS) void dkdv_whole_kernel(const S
           bf16x8 PB[4];
           PB[0] = pack8(s, 0);
           PB[1] = pack8(s, 1);
+          const u32x4 on = only_dn ? u32x4{0u, 0u, 0u, 0u} : u32x4{~0u, ~0u, ~0u, ~0u};
+          if constexpr (INVALID) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) PB[i] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, PB[i]) & on);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          // (three pieces that the scheduler keeps apart: left to itself it reads a transposed operand right before its product)
+#pragma unroll
+          for (int j = 0; j < NV; ++j) {
+            at[j + A2] = tr_op(j + A2);
+            acc[KT + j % VT] = mfma32(at[j], PB[j / VT], acc[KT + j % VT]);
+          }
           float dsum = 0.f;
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
@@ -684,24 +696,24 @@ __global__ __launch_bounds__(256, DKDV_WHOLE_WGS) void dkdv_whole_kernel(const S
           PB[2] = pack8(dp, 0);
           PB[3] = pack8(dp, 1);
           if constexpr (INVALID) {
-            const u32x4 on = only_dn ? u32x4{0u, 0u, 0u, 0u} : u32x4{~0u, ~0u, ~0u, ~0u};
 #pragma unroll
-            for (int i = 0; i < 4; ++i) PB[i] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, PB[i]) & on);
+            for (int i = 2; i < 4; ++i) PB[i] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, PB[i]) & on);
           }
 #pragma unroll
-          for (int j = 0; j < N2; ++j) {
+          for (int j = 0; j < NV; ++j) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int j = NV; j < N2; ++j) {
             if (j + A2 < N2) at[j + A2] = tr_op(j + A2);
-            if (j < NV) acc[KT + j % VT] = mfma32(at[j], PB[j / VT], acc[KT + j % VT]);
-            else acc[(j - NV) % KT] = mfma32(at[j], PB[2 + (j - NV) / KT], acc[(j - NV) % KT]);
+            acc[(j - NV) % KT] = mfma32(at[j], PB[2 + (j - NV) / KT], acc[(j - NV) % KT]);
           }
-          // dS is formed under the dV products, its sum under the dK products
-          __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);   // P packed
 #pragma unroll
-          for (int j = 0; j < N2; ++j) {
+          for (int j = NV; j < N2; ++j) {
             if (j + A2 < N2) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (j < NV) __builtin_amdgcn_sched_group_barrier(0x002, 28 / NV, 0);
-            else __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
           }
         }
         // this wave's requests of the next tile have landed (those of the one after it may stay in flight)

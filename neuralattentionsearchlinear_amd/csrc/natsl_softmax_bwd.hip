@@ -298,6 +298,7 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
       asm("" : "+v"(ka), "+v"(va), "+v"(ta));   // (three registers, the rest by XOR and offset fields)
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt) {
+        if (kt == 1 && causal && qloc0 == 0) break;   // (the chunk's later keys see nothing of its earlier queries)
         // The LDS operands of the first two products form one stream (K row piece, V row piece, K, V, ...) that is
         // read a few instructions ahead of its use: reading all of them up front needs 64 registers and spills.
         constexpr int NOPS = KS + VS, AHEAD = 4;

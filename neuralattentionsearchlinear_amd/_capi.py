@@ -13,11 +13,12 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "csrc", "libnatsl.so")
+STEP_CORE_PATH = os.path.join(_HERE, "_step_core.so")
 
 F32, BF16 = 0, 1
 DECAY_NON_LINEAR, QK_L2NORM, INTRA_CHUNK, QUERY_ONLY, FRESH_BLOCK_START = 1, 2, 4, 8, 16
 
-_lib = None
+_lib = _step_core = None
 
 _SIGNATURES = {
     "natsl_version": (c_int, []),
@@ -119,6 +120,17 @@ def lib():
                 fn.restype, fn.argtypes = res, args
         _lib = L
     return _lib
+
+
+def step_core():
+    """The native host side of the layers (csrc/host/step_core.cpp)."""
+    global _step_core
+    if _step_core is None:
+        if not os.path.exists(STEP_CORE_PATH):
+            raise NatslError(f"{STEP_CORE_PATH} is missing: build it with `python -m neuralattentionsearchlinear_amd._build`")
+        from . import _step_core as core
+        _step_core = core
+    return _step_core
 
 
 def exported_symbols():

@@ -3,14 +3,14 @@ states to the layer's output, with the cache's new rows written in place.
 
 A step of a layer is a few microseconds of memory traffic per kernel, so what it costs is launches and host time: the same step
 as separate torch operations and operator calls is forty launches and ~0.57 ms of host time (340M geometry), this is five
-launches behind one ctypes call.  `layer_step` declines (returns None) whatever the call is not built for -- other dtypes,
+launches behind one call of csrc/host/step_core.cpp, which also compares the layer with its plan, checks the cache's tensors and
+allocates the step's.  `layer_step` declines (returns None) whatever the call is not built for -- other dtypes,
 tensors that want gradients, replaced or hooked submodules, the 'attn' mode, more than 64 new tokens in all -- and the layers'
 general path runs.
 """
 from __future__ import annotations
 
 import ctypes
-import operator
 import weakref
 
 import torch
@@ -64,8 +64,6 @@ _OPTIONS = ("hidden_size", "head_k_dim", "head_v_dim", "head_attn_k_dim", "head_
 _SUB_OPTIONS = ("eps", "kernel_size", "activation")
 _SUBMODULES = tuple({p[1]: p[3] for p in _PARAMS if p[1] is not None and p[3] is not None}.items()) + (("q_norm2", L2Norm), ("k_norm2", L2Norm))
 _PLAIN_TENSORS = {nn.Parameter, torch.Tensor, type(None)}
-_hooks_of = operator.itemgetter('_forward_hooks', '_forward_pre_hooks', '_backward_hooks', '_backward_pre_hooks')
-_dtype_of, _shape_of = operator.attrgetter('dtype'), operator.attrgetter('shape')
 
 
 def weight_shapes(layer):
@@ -79,41 +77,27 @@ def weight_shapes(layer):
     return s
 
 
-def _getter(names):
-    """dict -> the tuple of its entries `names` (KeyError when one is gone)"""
-    if len(names) == 1:
-        return lambda d, n=names[0]: (d[n],)
-    return operator.itemgetter(*names) if names else lambda d: ()
-
-
 class _Watch:
     """What a layer's plans were made from besides its weights' values: which weights and plain submodules it has, the options, and the
     weights' addresses, types and layouts.  No tensor or module is held: a replaced weight is freed when its owner lets go of it."""
 
     def __init__(self, layer):
         mods = layer._modules
-        self.absent = [n for n, _ in _SUBMODULES if mods.get(n) is None]
-        self.parts, self.plain = [], True                  # parts: (name, type, its parameters, its options, their values)
+        absent = [n for n, _ in _SUBMODULES if mods.get(n) is None]
+        parts, self.plain = [], True                       # parts: (name, type, its parameters, its options, their values)
+        weights = [*layer._parameters.values()]
         for n, kind in _SUBMODULES:
             m = mods.get(n)
             if m is not None:
                 options = [o for o in _SUB_OPTIONS if o in m.__dict__]
-                self.parts.append((n, type(m), _getter([*m._parameters]), _getter(options) if options else None, _getter(options)(m.__dict__)))
+                parts.append((n, type(m), [*m._parameters], options, [m.__dict__[o] for o in options]))
+                weights += m._parameters.values()
                 self.plain &= type(m) is kind
-        self.own = _getter([*layer._parameters])
-        self.option_names = _getter([o for o in _OPTIONS if o in layer.__dict__])
-        self.options = self.option_names(layer.__dict__)
-        weights = [*self.own(layer._parameters)]
-        for n, _, params, _, _ in self.parts:
-            weights += params(mods[n]._parameters)
-        self.types = [*map(type, weights)]
-        self.plain &= {*self.types} <= _PLAIN_TENSORS
-        self.layouts = self._layouts([t for t in weights if t is not None]) if self.plain else None
+        options = [o for o in _OPTIONS if o in layer.__dict__]
+        self.plain &= {*map(type, weights)} <= _PLAIN_TENSORS
+        self.core = _capi.step_core().make_watch(parts, [*layer._parameters], absent, options, [layer.__dict__[o] for o in options],
+                                                 weights) if self.plain else None
         self.step_plan = self.front_plan = None
-
-    @staticmethod
-    def _layouts(w):
-        return [*map(torch.Tensor.data_ptr, w), *map(_dtype_of, w), *map(torch.Tensor.is_contiguous, w), *map(_shape_of, w)]
 
     def weights(self, layer):
         """The weights by field, None where the layer has none."""
@@ -124,28 +108,8 @@ class _Watch:
         return out
 
     def holds(self, layer):
-        """-> (whether nothing has changed, whether a submodule has a hook or a forward of its own)"""
-        mods, hooks = layer._modules, []
-        try:
-            weights = [*self.own(layer._parameters)]
-            for n, kind, params, options, values in self.parts:
-                m = mods[n]
-                if type(m) is not kind:
-                    return False, False
-                d = m.__dict__
-                weights += params(d['_parameters'])
-                hooks += _hooks_of(d)
-                if 'forward' in d:
-                    hooks.append(True)
-                if options is not None and options(d) != values:
-                    return False, False
-            same = self.option_names(layer.__dict__) == self.options
-        except KeyError:                                   # (a parameter, a submodule or an option is gone)
-            return False, False
-        for n in self.absent:
-            same &= mods.get(n) is None
-        return (same and [*map(type, weights)] == self.types and self.layouts is not None and
-                self._layouts([t for t in weights if t is not None]) == self.layouts), any(hooks)
+        """0: something has changed; 1: nothing has; 2: nothing has, and a submodule has a hook or a forward of its own."""
+        return _capi.step_core().holds(self.core, layer) if self.plain else 0
 
 
 def watch(layer):
@@ -154,11 +118,11 @@ def watch(layer):
     if torch.autograd.forward_ad._current_level >= 0:
         return None
     w = _watches.get(layer)
-    same, hooked = (False, False) if w is None else w.holds(layer)
-    if not same:
+    state = 0 if w is None else w.holds(layer)
+    if state == 0:
         w = _watches[layer] = _Watch(layer)
-        hooked = w.holds(layer)[1] if w.plain else False
-    return None if not w.plain or hooked or _has_any_global_hook() else w
+        state = w.holds(layer)
+    return w if state == 1 and not _has_any_global_hook() else None
 
 
 class _Plan:
@@ -166,7 +130,6 @@ class _Plan:
 
     def __init__(self, layer, kind, seen):
         self.built = False
-        self.ws_bytes = {}
         params = seen.weights(layer)
         s = self.fixed = LayerStep()
         by, shapes = dict(zip((p[0] for p in _PARAMS), params)), weight_shapes(layer)
@@ -218,38 +181,11 @@ class _Plan:
             s.l2_eps = layer.q_norm2.eps
         s.flags = flags
         self.device = params[0].device
-        # the cache's tensors as the kernels address them: (type, shape behind the batch), but for those that follow the cache's capacity
-        bs, bf16, f32 = layer.nats_block_size, torch.bfloat16, torch.float32
-        self.rows = ((HQ, KA), (HQ, VA))
-        self.buffers = [(bf16, (H * K, W)), (bf16, (H * K, W)), (bf16, (H * V, W)), (f32, (H, K, V)), (bf16, (bs, H, K)), (bf16, (bs, H, V)),
-                        (f32, (bs, H)), (bf16, (bs, D))] + [(bf16, (bs, H))] * delta
-        self.expected = (0, 0, None, None)
+        L = _capi.lib()
+        address = lambda f: ctypes.cast(f, ctypes.c_void_p).value
+        self.core = _capi.step_core().make_step(ctypes.addressof(s), ctypes.sizeof(s), address(L.natsl_layer_step_fwd),
+                                                address(L.natsl_layer_step_workspace_bytes), self.device.index)
         self.built = True
-
-    def _expect(self, B, cap):
-        """Types and shapes of takes()' tensors (the block-start state last) at this batch and capacity; the last pair is remembered."""
-        if self.expected[:2] != (B, cap):
-            want = self.buffers + [(torch.bfloat16, (cap, *self.rows[0])), (torch.bfloat16, (cap, *self.rows[1])),
-                                   (torch.bool, (cap // self.fixed.block, self.fixed.HN)), self.buffers[3]]
-            self.expected = (B, cap, [dt for dt, _ in want], [(B, *tail) for _, tail in want])
-        return self.expected[2:]
-
-    def takes(self, cache, B, start):
-        """Whether the cache's tensors have the types, shapes and layouts that the kernels read and write (a cache filled under autocast
-        or by other code can hold others: the general path converts)."""
-        k, state = cache.attn_k, cache.recurrent_state
-        have = [*cache.conv_state, state, cache.l_attn_k, cache.l_attn_v, cache.lattn_g, cache.block_type_state]
-        if self.fixed.is_delta:
-            have.append(cache.lattn_beta)
-        have += (k, cache.attn_v, cache.valid_attn_tokens, state if start is None else start)
-        g, cap, index = cache.g_cumsum, k.shape[1], self.device.index
-        dtypes, shapes = self._expect(B, cap)
-        try:
-            return ([*map(_dtype_of, have)] == dtypes and [*map(_shape_of, have)] == shapes and all(map(torch.Tensor.is_contiguous, have)) and
-                    {*map(torch.Tensor.get_device, have)} == {index} and cap % self.fixed.block == 0 and
-                    (g is None or (g.numel() == B * self.fixed.H and g.get_device() == index)))
-        except (AttributeError, TypeError):                # (one of them is None)
-            return False
 
 
 def layer_step(layer, kind, x, cache):
@@ -266,57 +202,33 @@ def layer_step(layer, kind, x, cache):
         plan = seen.step_plan = _Plan(layer, kind, seen)
     if not plan.built:
         return None
-    bs, n_in, n_kept = cache.nats_block_size, cache._n_tokens_in_nats_block, cache.n_attn_blocks_max
-    conv, state, start = cache.conv_state, cache.recurrent_state, cache.recurrent_state_block_start
-    f = plan.fixed
-    if (cache.attn_k is None or state is None or conv is None or cache.valid_attn_tokens is None or bs != f.block or n_in + T > bs or
-            x.device != plan.device or cache.n_attn_blocks is None or (cache._linear_only == bool(f.flags & ATTN_OWN_BLOCK)) or
-            cache.op_for_incomplete_chunk == 'attn' or not plan.takes(cache, B, start)):
+    bs, n_in, start = cache.nats_block_size, cache._n_tokens_in_nats_block, cache.recurrent_state_block_start
+    f, core = plan.fixed, _capi.step_core()
+    if (bs != f.block or n_in + T > bs or x.device != plan.device or cache.n_attn_blocks is None or cache.attn_k is None or
+            (cache._linear_only == bool(f.flags & ATTN_OWN_BLOCK)) or cache.op_for_incomplete_chunk == 'attn'):
         return None
+    completes = n_in + T == bs
+    full = cache.attn_k.shape[1] < cache.n_attn_tokens_max + T
+    tensors = lambda: (cache.conv_state, cache.recurrent_state, cache.l_attn_k, cache.l_attn_v, cache.lattn_g, cache.block_type_state,
+                       cache.lattn_beta, cache.attn_k, cache.attn_v, cache.valid_attn_tokens, start, cache.g_cumsum)
     types = None
-    if n_in + T == bs:
-        types, _, _ = layer.select_ops(cache.update_attn_types(input_hidden_states=x), None, force_last_block=False)
-        if types.shape != (B, 1, f.HN, 2) or types.device != x.device:
-            raise ValueError(f"select_ops must give types {(B, 1, f.HN, 2)} on {x.device}, got {tuple(types.shape)} on {types.device}")
-        types = (types if types.dtype in (torch.bfloat16, torch.float32) else types.float()).contiguous()
-    if cache.attn_k.shape[1] < cache.n_attn_tokens_max + T:
-        cache._grow(cache.n_attn_tokens_max + T)
-    x = x.contiguous()
-    dev = x.device
-    s = LayerStep.from_buffer_copy(f)
-    s.B, s.T, s.n_in, s.n_kept, s.cache_tokens = B, T, n_in, n_kept, cache.attn_k.shape[1]
-    new_conv = tuple([torch.empty_like(c) for c in conv])
-    state_out = torch.empty_like(state)
-    if start is None:
-        start = torch.empty_like(state)
-        s.flags |= FRESH_START
-    g_sum = cache.g_cumsum
-    if g_sum is not None and (g_sum.dtype != torch.float32 or not g_sum.is_contiguous()):
-        g_sum = g_sum.float().contiguous()
-    g_out = torch.empty((B, 1, f.H), dtype=torch.float32, device=dev)
-    out = torch.empty((B, T, D), dtype=torch.bfloat16, device=dev)
-    s.x, s.out, s.state, s.state_out, s.block_start = x.data_ptr(), out.data_ptr(), state.data_ptr(), state_out.data_ptr(), start.data_ptr()
-    s.conv_state_q, s.conv_state_k, s.conv_state_v = conv[0].data_ptr(), conv[1].data_ptr(), conv[2].data_ptr()
-    s.conv_out_q, s.conv_out_k, s.conv_out_v = new_conv[0].data_ptr(), new_conv[1].data_ptr(), new_conv[2].data_ptr()
-    s.g_cumsum, s.g_cumsum_out = None if g_sum is None else g_sum.data_ptr(), g_out.data_ptr()
-    s.cache_k, s.cache_v, s.cache_valid = cache.attn_k.data_ptr(), cache.attn_v.data_ptr(), cache.valid_attn_tokens.data_ptr()
-    s.block_k, s.block_v, s.block_g = cache.l_attn_k.data_ptr(), cache.l_attn_v.data_ptr(), cache.lattn_g.data_ptr()
-    if cache.lattn_beta is not None:
-        s.block_beta = cache.lattn_beta.data_ptr()
-    if types is None:
-        s.block_hidden = cache.block_type_state.data_ptr()
-    else:
-        s.types, s.types_dtype = types.data_ptr(), _capi.dtype_code(types.dtype)
-    L = _capi.lib()
-    ref = ctypes.byref(s)
-    ws_bytes = plan.ws_bytes.get((B, T))
-    if ws_bytes is None:
-        # (enough for every state of the cache: the attention's splits are bounded)
-        ws_bytes = plan.ws_bytes[(B, T)] = L.natsl_layer_step_workspace_bytes(ref)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    rc = L.natsl_layer_step_fwd(ref, ws.data_ptr(), ws_bytes, _capi.stream_ptr(dev))
-    if rc:
-        _capi.check(rc, "natsl_layer_step_fwd")
+    if completes or full:
+        if not core.takes(plan.core, B, *tensors()):       # (before anything of the cache changes)
+            return None
+        if completes:
+            types, _, _ = layer.select_ops(cache.update_attn_types(input_hidden_states=x), None, force_last_block=False)
+            if types.shape != (B, 1, f.HN, 2) or types.device != x.device:
+                raise ValueError(f"select_ops must give types {(B, 1, f.HN, 2)} on {x.device}, got {tuple(types.shape)} on {types.device}")
+            types = (types if types.dtype in (torch.bfloat16, torch.float32) else types.float()).contiguous()
+        if full:
+            cache._grow(cache.n_attn_tokens_max + T)
+    done = core.run(plan.core, x, n_in, cache.n_attn_blocks_max, _capi.stream_ptr(x.device), types,
+                    0 if types is None else _capi.dtype_code(types.dtype), *tensors())
+    if type(done) is not tuple:
+        if done is None:                                   # (the cache's tensors are not what the kernels address)
+            return None
+        _capi.check(done, "natsl_layer_step_fwd")
+    out, state_out, start, new_conv, g_out = done
     if types is None:
         cache.note_step(state_out, start, new_conv, g_out, T)
     else:

@@ -28,7 +28,7 @@ constexpr int MASKED_WAVES = 8;
 
 template <int DK, int DV, bool F32, int NW>
 __global__ __launch_bounds__(64 * NW) void attn_masked_kernel(const AttnParams p) {
-  attend<DK, DV, F32, NW>(p, blockIdx.z / p.nsplit, blockIdx.x, blockIdx.y, blockIdx.z % p.nsplit);
+  attend<DK, DV, F32, NW>(p, blockIdx.z / p.nsplit, blockIdx.x, blockIdx.y, blockIdx.z % p.nsplit, CachedRows());
 }
 
 // joins the splits of one query: one wave per (sequence, query, head)
@@ -53,7 +53,7 @@ __global__ __launch_bounds__(256) void attend_and_recur_kernel(const AttnParams 
     id /= a.nsplit;
     const int hq = id % a.HQ;
     id /= a.HQ;
-    attend<DKA, DVA, false, 4>(a, id / a.TQ, id % a.TQ, hq, split);
+    attend<DKA, DVA, false, 4>(a, id / a.TQ, id % a.TQ, hq, split, CachedRows());
     return;
   }
   id -= n_attn;

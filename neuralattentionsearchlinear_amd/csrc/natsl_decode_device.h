@@ -1,6 +1,8 @@
 // Device pieces of the decode-time kernels, shared by the operator entries (natsl_decode.hip) and the whole layer step
 // (natsl_step.hip): attention of one query row over cached keys, and the linear branch's token recurrence.
 #pragma once
+#include <type_traits>
+
 #include "natsl_device.h"
 #include "../../include/natsl.h"
 
@@ -21,6 +23,10 @@ NATSL_DEVICE float row16_sum(float x) {
 #undef NATSL_ROR
   return x;
 }
+
+// Values that waves of one launch hand to each other: stores that write through the XCD's own L2 and loads that do not trust it.
+NATSL_DEVICE void st_agent(float* p, const float x) { __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+NATSL_DEVICE float ld_agent(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 // ---------------------------------------------------------------------------------------------
 // attention of one query row over cached keys
@@ -60,20 +66,29 @@ struct AttnRow {
   static constexpr int EK = DK / 16, EV = DV / 16;      // elements of a key / value row per lane
   float q[EK], acc[EV], m, l;                            // m: running maximum (log2 units, the same in every lane); l, acc: this lane group's share
 
-  NATSL_DEVICE void init(const void* qs, const size_t row, const float scale_log2) {
+  NATSL_DEVICE void query(const void* qs, const size_t row, const float scale_log2) {
     const int sub = threadIdx.x & 15;
 #pragma unroll
     for (int e = 0; e < EK; ++e) q[e] = ld_any(qs, F32 ? NATSL_F32 : NATSL_BF16, row * DK + EK * sub + e) * scale_log2;
+  }
+  NATSL_DEVICE void clear() {
 #pragma unroll
     for (int e = 0; e < EV; ++e) acc[e] = 0.f;
     m = -INFINITY;
     l = 0.f;
   }
+  NATSL_DEVICE void init(const void* qs, const size_t row, const float scale_log2) {
+    query(qs, row, scale_log2);
+    clear();
+  }
 
   // keys k0 .. k0+31, rows of k_row / v_row elements behind element k_at / v_at; rows from n_keys on are not read (`vis` hides
   // them); vis: bit i = key k0+i visible, not all zero
+  // Own::STEP: own.ready() is called between the requests and their use; keys from own.first on are the row in own.k / own.v instead
+  // (a key that this launch itself adds to the cache).
+  template <class Own>
   NATSL_DEVICE void chunk(const void* k, const void* v, const size_t k_at, const size_t v_at, const size_t k_row, const size_t v_row,
-                          const int k0, const int n_keys, const unsigned vis) {
+                          const int k0, const int n_keys, const unsigned vis, Own& own) {
     const int sub = threadIdx.x & 15, grp = (threadIdx.x & 63) >> 4;
     RowPiece<EK, F32> kr[KEY_PASSES];
     RowPiece<EV, F32> vr[KEY_PASSES];
@@ -81,6 +96,17 @@ struct AttnRow {
     for (int i = 0; i < KEY_PASSES; ++i) kr[i].load(k, k_at + (size_t)min(k0 + 4 * i + grp, n_keys - 1) * k_row + EK * sub);
 #pragma unroll
     for (int i = 0; i < KEY_PASSES; ++i) vr[i].load(v, v_at + (size_t)min(k0 + 4 * i + grp, n_keys - 1) * v_row + EV * sub);
+    if constexpr (Own::STEP) {
+      own.ready(*this);
+      if (k0 + KEYS_PER_CHUNK > own.first) {
+#pragma unroll
+        for (int i = 0; i < KEY_PASSES; ++i)
+          if (k0 + 4 * i + grp >= own.first) {
+            kr[i].load(own.k, EK * sub);
+            vr[i].load(own.v, EV * sub);
+          }
+      }
+    }
     float s[KEY_PASSES];
     float mx = -INFINITY;
 #pragma unroll
@@ -140,36 +166,48 @@ struct AttnParams {
   const uint8_t* valid; int valid_bs, n_kept, block, n_in, own_visible;   // valid[b][block][HM], valid_bs bytes per sequence
 };
 
-// One workgroup of NW waves works on split `split` of query (b, tq, hq).
-template <int DK, int DV, bool F32, int NW>
-NATSL_DEVICE void attend(const AttnParams& p, const int b, const int tq, const int hq, const int split) {
+struct CachedRows { static constexpr bool STEP = false; };   // query and keys are all in memory
+
+// One workgroup of NW waves works on split `split` of query (b, tq, hq); wave 0 writes the result.  Own::STEP (above): the query comes
+// from own.ready(), called once with or without a visible chunk, memory holds the keys before own.first only, and the result goes to
+// the partials for another wave of this launch.
+template <int DK, int DV, bool F32, int NW, class Own>
+NATSL_DEVICE void attend(const AttnParams& p, const int b, const int tq, const int hq, const int split, Own&& own) {
+  constexpr bool STEP = std::remove_reference_t<Own>::STEP;
   constexpr int CPL = DV / 64, EV = DV / 16;
   __shared__ float sm_m[NW], sm_l[NW], sm_acc[NW][DV];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int hkv = hq / (p.HQ / p.HKV), hm = hq / (p.HQ / p.HM);
   const size_t row = ((size_t)b * p.TQ + tq) * p.HQ + hq;
   AttnRow<DK, DV, F32> r;
-  r.init(p.q, row, p.scale_log2);
+  if constexpr (STEP) r.clear();
+  else r.init(p.q, row, p.scale_log2);
   const uint8_t* mrow = p.mask ? p.mask + (((size_t)b * p.HM + hm) * p.TQ + tq) * p.TK : nullptr;
   const size_t k_at = (size_t)b * p.k_bs + (size_t)hkv * DK, v_at = (size_t)b * p.v_bs + (size_t)hkv * DV;
-  for (int k0 = KEYS_PER_CHUNK * (split * NW + wave); k0 < p.TK; k0 += KEYS_PER_CHUNK * NW * p.nsplit) {
-    unsigned vis;
-    if (mrow) {
+  const int first = KEYS_PER_CHUNK * (split * NW + wave), stride = KEYS_PER_CHUNK * NW * p.nsplit;   // the wave's chunks
+  auto chunk = [&](const int k0, const unsigned vis) __attribute__((always_inline)) {
+    r.chunk(p.k, p.v, k_at, v_at, (size_t)p.HKV * DK, (size_t)p.HKV * DV, k0, STEP ? max(p.TK - 1, 1) : p.TK, vis, own);
+  };
+  if (mrow) {
+    for (int k0 = first; k0 < p.TK; k0 += stride) {
       const int key = k0 + (lane & 31);
-      vis = (unsigned)__ballot(key < p.TK && mrow[min(key, p.TK - 1)] != 0);
-    } else {
-      const int own = p.n_kept * p.block;               // the incomplete block's first key
-      if (k0 < own) {
-        vis = p.valid[(size_t)b * p.valid_bs + (size_t)(k0 / p.block) * p.HM + hm] ? 0xffffffffu : 0u;
-      } else {
-        const int n = min(own + p.n_in + tq + 1, p.TK) - k0;
-        vis = !p.own_visible || n <= 0 ? 0u : n >= 32 ? 0xffffffffu : (1u << n) - 1u;
-      }
-      vis = __builtin_amdgcn_readfirstlane(vis);
+      const unsigned vis = (unsigned)__ballot(key < p.TK && mrow[min(key, p.TK - 1)] != 0);
+      if (vis != 0u) chunk(k0, vis);                     // (wave-uniform)
     }
-    if (vis == 0u) continue;                             // (wave-uniform)
-    r.chunk(p.k, p.v, k_at, v_at, (size_t)p.HKV * DK, (size_t)p.HKV * DV, k0, p.TK, vis);
+  } else {
+    // lane i looks at the i-th of the wave's next 64 chunks, so that their flags are one round trip
+    const int own_at = p.n_kept * p.block;              // the incomplete block's first key
+    const int end = min(own_at + p.n_in + tq + 1, p.TK);  // behind the last key that the query may see there
+    for (int base = first; base < p.TK; base += 64 * stride) {
+      const int mine = base + lane * stride;
+      const bool seen = mine < own_at ? p.valid[(size_t)b * p.valid_bs + (size_t)(mine / p.block) * p.HM + hm] != 0 : p.own_visible && mine < end;
+      for (unsigned long long todo = __ballot(seen); todo; todo &= todo - 1) {
+        const int k0 = base + __builtin_ctzll(todo) * stride, n = end - k0;
+        chunk(k0, k0 < own_at || n >= 32 ? 0xffffffffu : (1u << n) - 1u);
+      }
+    }
   }
+  if constexpr (STEP) own.ready(r);
   // the waves' shares together
   r.join_groups();
   if (lane == 0) { sm_m[wave] = r.m; sm_l[wave] = r.l; }
@@ -193,6 +231,12 @@ NATSL_DEVICE void attend(const AttnParams& p, const int b, const int tq, const i
   }
   if (p.partials) {
     float* dst = p.partials + (row * p.nsplit + split) * (2 + DV);
+    if constexpr (STEP) {
+      if (lane == 0) { st_agent(dst, m); st_agent(dst + 1, l); }
+#pragma unroll
+      for (int j = 0; j < CPL; ++j) st_agent(dst + 2 + CPL * lane + j, o[j]);
+      return;
+    }
     if (lane == 0) { dst[0] = m; dst[1] = l; }
 #pragma unroll
     for (int j = 0; j < CPL; ++j) dst[2 + CPL * lane + j] = o[j];
@@ -206,11 +250,21 @@ NATSL_DEVICE void attend(const AttnParams& p, const int b, const int tq, const i
 // (m, l, acc) of the splits (at most 64) of one query row, written by one workgroup each as [2 + DV] floats: the joined, normalised
 // columns CPL*lane.. of the row; a row that saw no key gives 0.  Lane s holds split s's weight, so that the maxima are one round
 // trip to memory and the partial rows another.
-template <int DV>
+// The first rows are requested with the maxima.  AGENT: the partials come from this launch.
+template <int DV, bool AGENT = false>
 NATSL_DEVICE void join_splits(const float* src, const int nsplit, float* o) {
-  constexpr int CPL = DV / 64, U = 4;
+  constexpr int CPL = DV / 64, U = AGENT ? 8 : 4;
   const int lane = threadIdx.x & 63;
-  const float ms = lane < nsplit ? src[lane * (2 + DV)] : -INFINITY, ls = lane < nsplit ? src[lane * (2 + DV) + 1] : 0.f;
+  auto ld = [](const float* p) __attribute__((always_inline)) { return AGENT ? ld_agent(p) : *p; };
+  const float ms = lane < nsplit ? ld(src + lane * (2 + DV)) : -INFINITY, ls = lane < nsplit ? ld(src + lane * (2 + DV) + 1) : 0.f;
+  float v[U][CPL];
+  auto rows = [&](const int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < CPL; ++j) v[u][j] = ld(src + min(s + u, nsplit - 1) * (2 + DV) + 2 + CPL * lane + j);
+  };
+  rows(0);
   float m = ms;
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
@@ -221,11 +275,7 @@ NATSL_DEVICE void join_splits(const float* src, const int nsplit, float* o) {
 #pragma unroll
   for (int j = 0; j < CPL; ++j) o[j] = 0.f;
   for (int s = 0; s < nsplit; s += U) {
-    float v[U][CPL];
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int j = 0; j < CPL; ++j) v[u][j] = src[min(s + u, nsplit - 1) * (2 + DV) + 2 + CPL * lane + j];
+    if (s > 0) rows(s);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const float fu = s + u < nsplit ? __shfl(f, s + u) : 0.f;
@@ -282,13 +332,33 @@ NATSL_DEVICE void ld_row(const void* p, const int dtype, const bool aligned, con
   }
 }
 
+// Where recurrent_columns takes a token from and puts its output: the tensors of the parameters.
+template <int DK>
+struct TokenRows {
+  static constexpr int R = DK / 4;
+  template <bool DELTA>
+  NATSL_DEVICE void token(const RecurrentParams& p, const int n, const int t, const int h, const int kq, const int vc, float* kk, float* qq, float& gt,
+                          float& bt, float& vt) const {
+    const size_t tok = (size_t)n * p.T + t, row = (size_t)n * p.kv_stride + p.kv_first + t;
+    ld_row<R>(p.k, p.dtype, p.aligned, (row * p.H + h) * DK + kq * R, kk);
+    ld_row<R>(p.q, p.dtype, p.aligned, (tok * p.H + h) * DK + kq * R, qq);
+    gt = p.g[row * p.H + h];
+    bt = DELTA ? ld_any(p.beta, p.dtype, row * p.H + h) : 1.f;
+    vt = ld_any(p.v, p.dtype, (row * p.H + h) * p.V + vc);
+  }
+  NATSL_DEVICE void out(const RecurrentParams& p, const int n, const int t, const int h, const int vc, const float x) const {
+    st_any(p.o, p.dtype, (((size_t)n * p.T + t) * p.H + h) * p.V + vc, x);
+  }
+  NATSL_DEVICE void done(int, int, int) const {}          // all outputs are written, the states are not
+};
+
 // One wave owns the state slice S[0:K][16 columns] of one (sequence, head): lane = (kq, col) with kq = lane/16 the quarter of
 // the K rows it keeps in registers (K/4 floats) and col = lane%16.  Sums over K are K/4 in-lane terms plus two cross-lane
 // steps; no LDS, no barriers.  Bound by the state's bytes (read and written once); the block-start state is only read by the
 // step that completes a block.  All of a lane's state loads are in flight before the token's k and q arrive.
 // DELTA = false is the Mamba form (src/nats/ops/mamba/fused_recurrent.py:150-178): S += k v^T, no beta, no norms.
-template <int DK, bool DELTA>
-NATSL_DEVICE void recurrent_columns(const RecurrentParams& p, const int nh, const int col16) {
+template <int DK, bool DELTA, class Tokens = TokenRows<DK>>
+NATSL_DEVICE void recurrent_columns(const RecurrentParams& p, const int nh, const int col16, Tokens&& tokens = Tokens()) {
   constexpr int R = DK / 4;  // state rows per lane
   const int lane = threadIdx.x & 63;
   const int kq = lane >> 4, col = lane & 15;
@@ -350,13 +420,8 @@ NATSL_DEVICE void recurrent_columns(const RecurrentParams& p, const int nh, cons
   }
 
   for (int t = 0; t < n_tok; ++t) {
-    const size_t tok = (size_t)n * p.T + t, row = (size_t)n * p.kv_stride + p.kv_first + t;
-    float kk[R], qq[R];
-    ld_row<R>(p.k, p.dtype, p.aligned, (row * p.H + h) * DK + kq * R, kk);
-    ld_row<R>(p.q, p.dtype, p.aligned, (tok * p.H + h) * DK + kq * R, qq);
-    const float gt = p.g[row * p.H + h];
-    const float bt = DELTA ? ld_any(p.beta, p.dtype, row * p.H + h) : 1.f;
-    const float vt = ld_any(p.v, p.dtype, (row * p.H + h) * p.V + vc);
+    float kk[R], qq[R], gt, bt, vt;
+    tokens.template token<DELTA>(p, n, t, h, kq, vc, kk, qq, gt, bt, vt);
     if (DELTA && p.l2norm) {
       float sk = 0.f, sq = 0.f;
 #pragma unroll
@@ -387,8 +452,9 @@ NATSL_DEVICE void recurrent_columns(const RecurrentParams& p, const int nh, cons
       hq += S[r] * qq[r];
     }
     hq += __shfl_xor(hq, 16); hq += __shfl_xor(hq, 32);
-    if (kq == 0) st_any(p.o, p.dtype, (tok * p.H + h) * p.V + vc, hq * p.scale);  // :199-201
+    if (kq == 0) tokens.out(p, n, t, h, vc, hq * p.scale);      // :199-201
   }
+  tokens.done(n, h, vc);
   if (p.g_cumsum_out && vc == 0 && kq == 0) p.g_cumsum_out[nh] = gcum;
   // the selector block is complete: a block not typed linear restores the state it started from
   // (times the block's total decay when asked), and that becomes the next block's start (:343-352)

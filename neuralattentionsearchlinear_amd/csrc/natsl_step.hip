@@ -1,12 +1,15 @@
 // A generation step of a whole hybrid layer: a few new tokens of each cached sequence, from the hidden states to the layer's
-// output, in five launches.  At this size a step is bound by launches and by the host that issues them (the same step as
-// separate operations was 40 launches, 0.2 ms of kernels and 0.57 ms of host time for one 340M-geometry layer), so each kernel
-// takes as much of the step as its data dependences allow:
+// output, in three launches for one token a sequence and five for several.  At this size a step is bound by launches and by the
+// host that issues them (the same step as separate operations was 40 launches, 0.2 ms of kernels and 0.57 ms of host time for one
+// 340M-geometry layer), so each kernel takes as much of the step as its data dependences allow:
 //   rows_gemm_kernel     q, k, v, gate, a (and beta) projections as one pass over all their weights; the output projection
+//   step_one_kernel      one token a sequence: all that the other three do
 //   step_mix_kernel      short convolutions, activations, row norms, gates; the new rows of every cache, written in place
 //   attend_and_recur     attention over the cached keys next to the token recurrence (natsl_decode.hip)
 //   step_tail_kernel     join of the attention's splits, mixing weights, two-input norm and gate
 // Roundings to bf16 are where the layer's separate operations round (projections, convolutions, norms, gates, branch outputs).
+#include <algorithm>
+
 #include "natsl_decode_device.h"
 #include "natsl_host.h"
 
@@ -24,6 +27,7 @@ struct RowsGemm {
   const bf16_t* x; bf16_t* out;
   int M, D, ldo, n_seg;
   GemmSeg seg[GEMM_SEGS];
+  unsigned* zero; int n_zero;   // cleared for a later launch of the step
 };
 
 template <int MT>
@@ -31,6 +35,8 @@ __global__ __launch_bounds__(512) void rows_gemm_kernel(const RowsGemm p) {
   constexpr int NW = 8, U = 4;
   __shared__ f32x4 red[NW][MT][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < p.n_zero; i += 512) p.zero[i] = 0u;
   int si = 0;
 #pragma unroll
   for (int i = 1; i < GEMM_SEGS; ++i) si = i < p.n_seg && (int)blockIdx.x >= p.seg[i].tile0 ? i : si;
@@ -101,6 +107,19 @@ struct ConvWindow {
       e[j] = bf16_to_f32(state[sd * W + j]);
       w[j] = bf16_to_f32(weight[d * W + j]);
     }
+  }
+  // W == 4, every pointer on 8 bytes
+  NATSL_DEVICE void init4(const void* state, const void* weight, const void* bias, const size_t d, const size_t sd) {
+    const u32x2 es = reinterpret_cast<const u32x2*>(state)[sd], ws = reinterpret_cast<const u32x2*>(weight)[d];
+    b = bias ? bf16_to_f32(reinterpret_cast<const bf16_t*>(bias)[d]) : 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      e[j] = __uint_as_float(j & 1 ? es[j >> 1] & 0xffff0000u : es[j >> 1] << 16);
+      w[j] = __uint_as_float(j & 1 ? ws[j >> 1] & 0xffff0000u : ws[j >> 1] << 16);
+    }
+  }
+  NATSL_DEVICE void save4(void* state, const size_t sd) const {
+    reinterpret_cast<u32x2*>(state)[sd] = (u32x2){pack_bf16x2(e[0], e[1]), pack_bf16x2(e[2], e[3])};
   }
   NATSL_DEVICE float next(const float x, const bool silu) {
 #pragma unroll
@@ -230,33 +249,29 @@ struct StepTail {
   float eps;
 };
 
+// the part of one wave: d0, d1 the head's two mixing logits, at the attention's columns CPL*lane.., x1 the linear branch's
 template <int VA>
-__global__ __launch_bounds__(256) void step_tail_kernel(const StepTail p) {
-  constexpr int CPL = VA / 64;
-  const int lane = threadIdx.x & 63;
-  const int rh = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (rh >= p.rows * p.HQ) return;
-  const int row = rh / p.HQ, hq = rh % p.HQ;
-  // the head's two mixing logits (rounded to bf16 as the projection's output is), their softmax
-  float d0 = 0.f, d1 = 0.f;
-  for (int i = 8 * lane; i < p.KD; i += 512) {
-    const u32x4 qv = *reinterpret_cast<const u32x4*>(p.q_conv + (size_t)row * p.KD + i);
-    const u32x4 a = *reinterpret_cast<const u32x4*>(p.w_mix + (size_t)(2 * hq) * p.KD + i);
-    const u32x4 c = *reinterpret_cast<const u32x4*>(p.w_mix + (size_t)(2 * hq + 1) * p.KD + i);
+struct TailRow {
+  static constexpr int CPL = VA / 64;
+  float g[CPL], w1[CPL], w2[CPL];
+  NATSL_DEVICE void load(const StepTail& p, const int row, const int hq) {
+    const int lane = threadIdx.x & 63;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float lo = __uint_as_float(qv[j] << 16), hi = __uint_as_float(qv[j] & 0xffff0000u);
-      d0 += lo * __uint_as_float(a[j] << 16) + hi * __uint_as_float(a[j] & 0xffff0000u);
-      d1 += lo * __uint_as_float(c[j] << 16) + hi * __uint_as_float(c[j] & 0xffff0000u);
+    for (int j = 0; j < CPL; ++j) {
+      g[j] = bf16_to_f32(p.proj[(size_t)row * p.ldp + p.cg + hq * VA + CPL * lane + j]);
+      w1[j] = ld_any(p.w1, p.w_dtype, CPL * lane + j);
+      w2[j] = ld_any(p.w2, p.w_dtype, CPL * lane + j);
     }
   }
-  float at[CPL];
-  join_splits<VA>(p.partials + (size_t)rh * p.nsplit * (2 + VA), p.nsplit, at);
-  float x1[CPL], x2[CPL], sa = 0.f, sb = 0.f;
-  const size_t base = (size_t)rh * VA + CPL * lane;
+  NATSL_DEVICE void finish(const StepTail& p, const int row, const int hq, float d0, float d1, const float* at, const float* x1) const;
+};
+
+template <int VA>
+NATSL_DEVICE void TailRow<VA>::finish(const StepTail& p, const int row, const int hq, float d0, float d1, const float* at, const float* x1) const {
+  const int lane = threadIdx.x & 63;
+  float x2[CPL], sa = 0.f, sb = 0.f;
 #pragma unroll
   for (int j = 0; j < CPL; ++j) {
-    x1[j] = bf16_to_f32(p.o_lin[base + j]);
     x2[j] = bf16_to_f32(f32_to_bf16(at[j]));
     sa += x1[j] * x1[j];
     sb += x2[j] * x2[j];
@@ -268,22 +283,398 @@ __global__ __launch_bounds__(256) void step_tail_kernel(const StepTail p) {
     sa += __shfl_xor(sa, o);
     sb += __shfl_xor(sb, o);
   }
-  d0 = bf16_to_f32(f32_to_bf16(d0));
+  d0 = bf16_to_f32(f32_to_bf16(d0));                   // (as the projection's output is)
   d1 = bf16_to_f32(f32_to_bf16(d1));
   mix_softmax(d0, d1);
   const float ra = rsqrtf(sa / VA + p.eps) * d0, rb = rsqrtf(sb / VA + p.eps) * d1;
+  const size_t base = ((size_t)row * p.HQ + hq) * VA + CPL * lane;
 #pragma unroll
   for (int j = 0; j < CPL; ++j) {
-    const float g = bf16_to_f32(p.proj[(size_t)row * p.ldp + p.cg + hq * VA + CPL * lane + j]);
-    const float mix = x1[j] * ra * ld_any(p.w1, p.w_dtype, CPL * lane + j) + x2[j] * rb * ld_any(p.w2, p.w_dtype, CPL * lane + j);
-    p.y[base + j] = f32_to_bf16(mix * g / (1.f + __expf(-g)));
+    const float mix = x1[j] * ra * w1[j] + x2[j] * rb * w2[j];
+    p.y[base + j] = f32_to_bf16(mix * g[j] / (1.f + __expf(-g[j])));
   }
 }
 
-struct StepLayout {
-  int ldp, cq, ck, cv, cg, ca, cb, tiles, nsplit;
-  size_t proj, q_conv, q_lin, q_attn, o_lin, y, partials, bytes;
+template <int VA>
+__global__ __launch_bounds__(256) void step_tail_kernel(const StepTail p) {
+  constexpr int CPL = VA / 64;
+  const int lane = threadIdx.x & 63;
+  const int rh = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (rh >= p.rows * p.HQ) return;
+  const int row = rh / p.HQ, hq = rh % p.HQ;
+  TailRow<VA> out;
+  out.load(p, row, hq);
+  float d0 = 0.f, d1 = 0.f;                            // the lane's share of the two logits
+  for (int i = 8 * lane; i < p.KD; i += 512) {
+    const u32x4 qv = *reinterpret_cast<const u32x4*>(p.q_conv + (size_t)row * p.KD + i);
+    const u32x4 a = *reinterpret_cast<const u32x4*>(p.w_mix + (size_t)(2 * hq) * p.KD + i);
+    const u32x4 c = *reinterpret_cast<const u32x4*>(p.w_mix + (size_t)(2 * hq + 1) * p.KD + i);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float lo = __uint_as_float(qv[j] << 16), hi = __uint_as_float(qv[j] & 0xffff0000u);
+      d0 += lo * __uint_as_float(a[j] << 16) + hi * __uint_as_float(a[j] & 0xffff0000u);
+      d1 += lo * __uint_as_float(c[j] << 16) + hi * __uint_as_float(c[j] & 0xffff0000u);
+    }
+  }
+  float at[CPL], x1[CPL];
+  join_splits<VA>(p.partials + (size_t)rh * p.nsplit * (2 + VA), p.nsplit, at);
+#pragma unroll
+  for (int j = 0; j < CPL; ++j) x1[j] = bf16_to_f32(p.o_lin[(size_t)rh * VA + CPL * lane + j]);
+  out.finish(p, row, hq, d0, d1, at, x1);
+}
+
+// ---- one token a sequence: everything between the two products in one launch --------------------------------------------
+// For one token the convolutions, norms and gates are a few operations on a few kilobytes, so every wave forms the ones that it
+// needs itself, and the tail of a (sequence, head) is done by whichever wave is the last to have written something for it: they
+// count themselves in on arrived[], which the projections' launch has cleared.  No wave waits for another.  Bound by round trips to
+// memory one behind another (arguments, windows and flags, keys, the count, the others' results); with many keys by their bytes.
+// Against the three launches: 340M geometry, one sequence of 800 tokens, 11.0 us for 4.3 + 5.4 + 4.8 and two gaps of 3.5; 16 heads of
+// 128/64 and eight sequences of 2000 tokens, 18 us for 5 + 13.6 + 5.3.  Workgroups:
+//   mixing logits   (sequence, 256 channels of q): their convolution, and their share of all heads' two logits
+//   recurrence      (sequence, head, 64 state columns), as in attend_and_recur
+//   attention       (sequence, head, split), as in attend_and_recur; the wave with the last chunk makes the new key and value
+//                   and writes them to the cache, which nothing else of the launch reads there
+// What leaves the launch besides y is written by one wave each: conv_out_q and block_hidden, cache_valid by the logits' waves,
+// conv_out_k, block_k, g and beta by the head's first recurrence wave, conv_out_v and block_v by the columns' own.
+struct StepOne {
+  StepMix m;
+  AttnParams a;
+  RecurrentParams r;
+  StepTail t;
+  float *o_lin, *logits;      // [B][H*V] rounded to bf16; [B][n_chunks][HQ][2]
+  unsigned* arrived;          // [B][HQ]
+  int n_chunks, n_logits, n_rec;
 };
+constexpr int LOGIT_CHUNK = 256;
+
+NATSL_DEVICE float wave_sum(float x) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) x += __shfl_xor(x, o);
+  return x;
+}
+
+// Everything that the wave handed over (stores that write through) has arrived before the lane with `on` counts it in; the
+// returned mask has the lanes that were their counter's last.
+NATSL_DEVICE unsigned long long arrive(const StepOne& p, const int b, const int hq, const bool on, const int expected) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  unsigned before = 0u;
+  if (on) before = __hip_atomic_fetch_add(p.arrived + (size_t)b * p.a.HQ + hq, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const unsigned long long last = __ballot(on && before + 1u == (unsigned)expected);
+  asm volatile("" ::: "memory");
+  return last;
+}
+
+template <int VA>
+NATSL_DEVICE void step_tail(const StepOne& p, const int b, const int hq) {
+  constexpr int CPL = VA / 64;
+  const int lane = threadIdx.x & 63;
+  const size_t rh = (size_t)b * p.a.HQ + hq;
+  TailRow<VA> out;
+  out.load(p.t, b, hq);
+  float at[CPL], x1[CPL];
+#pragma unroll
+  for (int j = 0; j < CPL; ++j) x1[j] = ld_agent(p.o_lin + rh * VA + CPL * lane + j);
+  const float* lg = p.logits + (((size_t)b * p.n_chunks + min(lane, p.n_chunks - 1)) * p.a.HQ + hq) * 2;
+  const float d0 = ld_agent(lg), d1 = ld_agent(lg + 1);
+  join_splits<VA, true>(p.a.partials + rh * p.a.nsplit * (2 + VA), p.a.nsplit, at);
+  out.finish(p.t, b, hq, lane < p.n_chunks ? d0 : 0.f, lane < p.n_chunks ? d1 : 0.f, at, x1);
+}
+
+template <int VA>
+NATSL_DEVICE void step_logits(const StepOne& p, const int b, const int chunk, const int expected) {
+  __shared__ __align__(16) bf16_t qs[LOGIT_CHUNK];
+  const natsl_layer_step& s = p.m.s;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int KD = s.H * s.K, d = LOGIT_CHUNK * chunk + tid;
+  constexpr int U = 4;                                  // four channels a lane, waves over the heads, four heads' rows in flight
+  const int c = LOGIT_CHUNK * chunk + 4 * lane;
+  const bf16_t* w = p.t.w_mix + min(c, KD - 4);
+  u32x2 r[2 * U];
+  auto load = [&](const int h0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 2 * U; ++u) r[u] = *reinterpret_cast<const u32x2*>(w + (size_t)(2 * min(h0 + 4 * (u >> 1), s.HQ - 1) + (u & 1)) * KD);
+  };
+  bf16_t y = 0;
+  if (d < KD) {
+    const size_t sd = (size_t)b * KD + d;
+    ConvWindow<4> win;
+    win.init4(s.conv_state_q, s.conv_wq, s.conv_bq, d, sd);
+    y = f32_to_bf16(win.next(bf16_to_f32(p.m.proj[(size_t)b * p.m.ldp + p.m.cq + d]), s.flags & NATSL_STEP_SILU));
+    win.save4(s.conv_out_q, sd);
+  }
+  load(wave);
+  qs[tid] = y;
+  if (s.block_hidden) {
+    const bf16_t* x = (const bf16_t*)s.x + (size_t)b * s.D;
+    bf16_t* to = (bf16_t*)s.block_hidden + ((size_t)b * s.block + s.n_in) * s.D;
+    for (int i = d; i < s.D; i += LOGIT_CHUNK * p.n_chunks) to[i] = x[i];
+  }
+  if (chunk == 0)
+    for (int i = tid; i < s.HN; i += 256) s.cache_valid[((size_t)b * (s.cache_tokens / s.block) + s.n_kept) * s.HN + i] = 1;
+  __syncthreads();
+  const u32x2 qv = *reinterpret_cast<const u32x2*>(qs + 4 * lane);
+  const float q0 = __uint_as_float(qv[0] << 16), q1 = __uint_as_float(qv[0] & 0xffff0000u), q2 = __uint_as_float(qv[1] << 16),
+              q3 = __uint_as_float(qv[1] & 0xffff0000u);
+  float* dst = p.logits + ((size_t)b * p.n_chunks + chunk) * s.HQ * 2;
+  for (int h0 = wave; h0 < s.HQ; h0 += 4 * U) {
+    if (h0 != wave) load(h0);
+#pragma unroll
+    for (int u = 0; u < 2 * U; ++u) {
+      float x = q0 * __uint_as_float(r[u][0] << 16) + q1 * __uint_as_float(r[u][0] & 0xffff0000u) + q2 * __uint_as_float(r[u][1] << 16) +
+                q3 * __uint_as_float(r[u][1] & 0xffff0000u);
+      x = wave_sum(c < KD ? x : 0.f);
+      const int h = h0 + 4 * (u >> 1);
+      if (lane == 0 && h < s.HQ) st_agent(dst + 2 * h + (u & 1), x);
+    }
+  }
+  for (int h0 = wave; h0 < s.HQ; h0 += 256) {           // lane i counts in for the wave's i-th head
+    const int h = h0 + 4 * lane;
+    for (unsigned long long last = arrive(p, b, h, h < s.HQ, expected); last; last &= last - 1) step_tail<VA>(p, b, h0 + 4 * __builtin_ctzll(last));
+  }
+}
+
+// The recurrence's token: q and k of the head go through the wave's own piece of LDS, the rest stays in registers.
+template <int DK>
+struct StepToken {
+  const StepOne& p;
+  bf16_t* rows;               // [2][DK], this wave's
+  const bool first;           // the head's first wave
+  const int expected, VA;
+  bool last = false;          // whether this wave is the one to do the tail
+  template <bool DELTA>
+  NATSL_DEVICE void token(const RecurrentParams& r, const int n, int, const int h, const int kq, const int vc, float* kk, float* qq, float& gt,
+                          float& bt, float& vt) const {
+    constexpr int R = DK / 4, C = DK / 64;
+    const natsl_layer_step& s = p.m.s;
+    const int lane = threadIdx.x & 63, KD = s.H * DK, VD = s.H * s.V;
+    const bool silu = s.flags & NATSL_STEP_SILU;
+    const bf16_t* proj = p.m.proj + (size_t)n * p.m.ldp;
+    const size_t block_row = (size_t)n * s.block + s.n_in;
+    ConvWindow<4> wq[C], wk[C], wv;
+    float xq[C], xk[C];
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      const int d = h * DK + 64 * i + lane;
+      wq[i].init4(s.conv_state_q, s.conv_wq, s.conv_bq, d, (size_t)n * KD + d);
+      wk[i].init4(s.conv_state_k, s.conv_wk, s.conv_bk, d, (size_t)n * KD + d);
+      xq[i] = bf16_to_f32(proj[p.m.cq + d]);
+      xk[i] = bf16_to_f32(proj[p.m.ck + d]);
+    }
+    const int dv = h * s.V + vc;
+    wv.init4(s.conv_state_v, s.conv_wv, s.conv_bv, dv, (size_t)n * VD + dv);
+    const float xv = bf16_to_f32(proj[p.m.cv + dv]);
+    const float A = expf(ld_any(s.a_log, s.gate_dtype, h));
+    const float dt = softplus_gate(bf16_to_f32(proj[p.m.ca + h]) + ld_any(s.dt_bias, s.gate_dtype, h));
+    gt = -A * dt;
+    bt = 1.f;
+    if (DELTA) {
+      float sg = bf16_to_f32(f32_to_bf16(sigmoid_gate(bf16_to_f32(proj[p.m.cb + h]))));
+      if (s.flags & NATSL_STEP_NEG_EIGVAL) sg *= 2.f;
+      bt = bf16_to_f32(f32_to_bf16(sg));
+    }
+    float ssq = 0.f, ssk = 0.f;
+    const bool l2 = s.flags & NATSL_STEP_L2_ROWS;
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      xq[i] = wq[i].next(xq[i], silu);
+      xk[i] = wk[i].next(xk[i], silu);
+      if (l2) {
+        ssq += wave_sum(xq[i] * xq[i]);
+        ssk += wave_sum(xk[i] * xk[i]);
+      }
+    }
+    const float rq = l2 ? rsqrtf(ssq + s.l2_eps) : 1.f, rk = l2 ? rsqrtf(ssk + s.l2_eps) : 1.f;
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      const bf16_t kb = f32_to_bf16(xk[i] * rk);
+      rows[64 * i + lane] = f32_to_bf16(xq[i] * rq);
+      rows[DK + 64 * i + lane] = kb;
+      if (first) {
+        const int d = h * DK + 64 * i + lane;
+        ((bf16_t*)s.block_k)[block_row * KD + d] = kb;
+        wk[i].save4(s.conv_out_k, (size_t)n * KD + d);
+      }
+    }
+    if (first && lane == 0) {
+      s.block_g[block_row * s.H + h] = gt;
+      if (DELTA) ((bf16_t*)s.block_beta)[block_row * s.H + h] = f32_to_bf16(bt);
+    }
+    float y = wv.next(xv, silu);
+    if (!DELTA) y = bf16_to_f32(f32_to_bf16(y * dt));
+    vt = y;
+    if (kq == 0) {
+      ((bf16_t*)s.block_v)[block_row * VD + dv] = f32_to_bf16(y);
+      wv.save4(s.conv_out_v, (size_t)n * VD + dv);
+    }
+    __builtin_amdgcn_wave_barrier();
+    ld_row<R>(rows, NATSL_BF16, true, kq * R, qq);
+    ld_row<R>(rows + DK, NATSL_BF16, true, kq * R, kk);
+  }
+  NATSL_DEVICE void out(const RecurrentParams& r, const int n, int, const int h, const int vc, const float x) const {
+    st_agent(p.o_lin + ((size_t)n * r.H + h) * r.V + vc, bf16_to_f32(f32_to_bf16(x)));
+  }
+  NATSL_DEVICE void done(const int n, const int h, const int vc) {   // (counted in before the states' stores are waited for)
+    last = arrive(p, n, (h * p.m.s.V + vc) / VA, (threadIdx.x & 63) == 0, expected) != 0;
+  }
+};
+
+// One head's row of the attention view of q, k or v (N channels), 64 i + lane in a lane: requested, then formed.
+template <int N>
+struct StepRow {
+  static constexpr int C = N / 64;
+  float x[C], nw[C];
+  ConvWindow<4> win[C];
+  NATSL_DEVICE void request(const natsl_layer_step& s, const bf16_t* proj, const void* state, const void* weight, const void* bias, const void* norm,
+                            const size_t seq, const int d0) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      const int d = d0 + 64 * i + lane;
+      x[i] = bf16_to_f32(proj[d]);
+      nw[i] = norm ? ld_any(norm, s.norm_dtype, 64 * i + lane) : 1.f;
+      if (s.flags & NATSL_STEP_ATTN_FROM_CONV) win[i].init4(state, weight, bias, d, seq + d);
+    }
+  }
+  NATSL_DEVICE void form(const natsl_layer_step& s, const bool norm, bf16_t* dst, bf16_t* also) {
+    const int lane = threadIdx.x & 63;
+    float ss = 0.f, r = 1.f;
+#pragma unroll
+    for (int i = 0; i < C; ++i)
+      if (s.flags & NATSL_STEP_ATTN_FROM_CONV) x[i] = win[i].next(x[i], s.flags & NATSL_STEP_SILU);
+    if (norm) {
+#pragma unroll
+      for (int i = 0; i < C; ++i) ss += wave_sum(x[i] * x[i]);
+      r = rsqrtf(ss / N + s.norm_eps);
+    }
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      const bf16_t y = f32_to_bf16(norm ? x[i] * r * nw[i] : x[i]);
+      dst[64 * i + lane] = y;
+      if (also) also[64 * i + lane] = y;
+    }
+  }
+};
+
+// What an attending wave of the step makes itself: its query, and in the wave with the last chunk (`mine`) the new key and value.  All
+// inputs are requested before the first chunk is, and used when that is on its way.
+template <int KA, int VA>
+struct StepKeys {
+  static constexpr bool STEP = true;
+  const StepOne& p;
+  bf16_t *q, *k, *v;             // LDS
+  const int b, hq, first;        // first: the new key's index
+  const bool mine;
+  bool done = false;
+  StepRow<KA> rq, rk;
+  StepRow<VA> rv;
+  NATSL_DEVICE StepKeys(const StepOne& p, bf16_t* q, bf16_t* k, bf16_t* v, const int b, const int hq, const bool mine)
+      : p(p), q(q), k(k), v(v), b(b), hq(hq), first(p.a.TK - 1), mine(mine) {
+    const natsl_layer_step& s = p.m.s;
+    const size_t KD = (size_t)s.H * s.K, VD = (size_t)s.H * s.V;
+    const bf16_t* proj = p.m.proj + (size_t)b * p.m.ldp;
+    const bool norm = s.flags & NATSL_STEP_ATTN_NORM;
+    rq.request(s, proj + p.m.cq, s.conv_state_q, s.conv_wq, s.conv_bq, norm ? s.norm_q : nullptr, b * KD, hq * KA);
+    if (mine) {
+      rk.request(s, proj + p.m.ck, s.conv_state_k, s.conv_wk, s.conv_bk, norm ? s.norm_k : nullptr, b * KD, hq * KA);
+      rv.request(s, proj + p.m.cv, s.conv_state_v, s.conv_wv, s.conv_bv, nullptr, b * VD, hq * VA);
+    }
+  }
+  NATSL_DEVICE void ready(AttnRow<KA, VA, false>& row) {
+    if (done) return;
+    done = true;
+    const natsl_layer_step& s = p.m.s;
+    const bool norm = s.flags & NATSL_STEP_ATTN_NORM;
+    rq.form(s, norm, q, nullptr);
+    if (mine) {
+      const size_t at = ((size_t)b * s.cache_tokens + first) * s.HQ + hq;
+      rk.form(s, norm, k, (bf16_t*)s.cache_k + at * KA);
+      rv.form(s, false, v, (bf16_t*)s.cache_v + at * VA);
+    }
+    __builtin_amdgcn_wave_barrier();
+    row.query(q, 0, p.a.scale_log2);
+  }
+};
+
+// The launch's only argument.  Read through a pointer that the optimiser cannot see through, so that each role loads the fields that it
+// needs where it needs them: as a plain argument the roles' fields are all loaded at the kernel's start and spill (70 scalar registers).
+NATSL_DEVICE const StepOne& step_one_args() {
+  typedef __attribute__((address_space(4))) const StepOne* arg_ptr;
+  unsigned long long at = (unsigned long long)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(at));
+  return *(const StepOne*)(arg_ptr)at;
+}
+
+template <int KA, int VA, int K, bool DELTA>
+__global__ __launch_bounds__(256) void step_one_kernel(const StepOne) {
+  const StepOne& p = step_one_args();
+  __shared__ __align__(16) bf16_t rows[4][2 * K > KA ? 2 * K : KA], own_k[KA], own_v[VA];
+  const natsl_layer_step& s = p.m.s;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int expected = p.a.nsplit + VA / 16 + p.n_chunks;
+  int id = blockIdx.x, b, hq;
+  if (id < p.n_logits) {
+    step_logits<VA>(p, id / p.n_chunks, id % p.n_chunks, expected);
+    return;
+  }
+  id -= p.n_logits;
+  if (id < p.n_rec) {
+    const int per = (s.V + 63) / 64, col16 = (id % per) * 4 + wave, nh = id / per;
+    if (col16 * 16 >= s.V) return;
+    StepToken<K> token{p, rows[wave], col16 == 0, expected, VA};
+    recurrent_columns<K, DELTA>(p.r, nh, col16, token);
+    if (!token.last) return;
+    b = nh / s.H;
+    hq = (nh % s.H * s.V + 16 * col16) / VA;
+  } else {
+    id -= p.n_rec;
+    const int split = id % p.a.nsplit;
+    hq = id / p.a.nsplit % s.HQ;
+    b = id / p.a.nsplit / s.HQ;
+    const bool mine = (p.a.TK - 1) / KEYS_PER_CHUNK % (4 * p.a.nsplit) == 4 * split + wave;
+    attend<KA, VA, false, 4>(p.a, b, 0, hq, split, StepKeys<KA, VA>(p, rows[wave], own_k, own_v, b, hq, mine));
+    if (wave != 0 || !arrive(p, b, hq, lane == 0, expected)) return;
+  }
+  step_tail<VA>(p, b, hq);
+}
+
+static int launch_step_one(const char* what, const StepOne& p, const int K, const int KA, const int VA, hipStream_t st) {
+  const natsl_layer_step& s = p.m.s;
+  const dim3 grid((unsigned)(p.n_logits + p.n_rec + s.B * s.HQ * p.a.nsplit));
+#define NATSL_S1(KK, VV, KL, DD)                                                              \
+  if (KA == KK && VA == VV && K == KL && (s.is_delta != 0) == DD) {                           \
+    hipLaunchKernelGGL((step_one_kernel<KK, VV, KL, DD>), grid, dim3(256), 0, st, p);         \
+    return check_launch(what);                                                                \
+  }
+#define NATSL_S3(KK, VV)                                                                                                     \
+  NATSL_S1(KK, VV, 64, true) NATSL_S1(KK, VV, 128, true) NATSL_S1(KK, VV, 192, true) NATSL_S1(KK, VV, 64, false)             \
+  NATSL_S1(KK, VV, 128, false) NATSL_S1(KK, VV, 192, false)
+  NATSL_S3(64, 64) NATSL_S3(64, 128) NATSL_S3(128, 64) NATSL_S3(128, 128)
+#undef NATSL_S3
+#undef NATSL_S1
+  return fail(NATSL_ERR_UNSUPPORTED, "%s: head dims %d (linear), %d / %d (attention) not built", what, K, KA, VA);
+}
+
+struct StepLayout {
+  int ldp, cq, ck, cv, cg, ca, cb, tiles, nsplit, n_chunks;
+  bool one;
+  size_t proj, q_conv, q_lin, q_attn, o_lin, y, partials, logits, arrived, bytes;
+};
+
+// One token a sequence: one launch between the two products.  That kernel is built for the layers' own convolution width and reads windows
+// and mixing rows 8 bytes at a time; a wave's lanes are its chunks of logits.
+static bool step_is_one(const natsl_layer_step& s, const int n_chunks) {
+  const uintptr_t at8 = (uintptr_t)s.conv_state_q | (uintptr_t)s.conv_state_k | (uintptr_t)s.conv_state_v | (uintptr_t)s.conv_out_q |
+                        (uintptr_t)s.conv_out_k | (uintptr_t)s.conv_out_v | (uintptr_t)s.conv_wq | (uintptr_t)s.conv_wk | (uintptr_t)s.conv_wv |
+                        (uintptr_t)s.w_mix;
+  return s.T == 1 && s.conv_width == 4 && n_chunks <= 64 && at8 % 8 == 0;
+}
+
+// As many splits as leave all of the launch's workgroups resident at once (its registers allow three a CU, two with 192-wide states):
+// eight sequences of the 128/64 geometry above take 17.9 us in one round of 4 splits, 19.3 in two rounds of 8.
+static int step_one_splits(const natsl_layer_step& s, const int n_chunks, const int most) {
+  const int slots = (s.K == 192 ? 2 : 3) * 256 - s.B * (n_chunks + s.H * cdiv(s.V, 64));
+  return std::max(1, std::min(most, slots / (s.B * s.HQ)));
+}
 
 static StepLayout step_layout(const natsl_layer_step& s) {
   StepLayout l;
@@ -293,16 +684,21 @@ static StepLayout step_layout(const natsl_layer_step& s) {
   l.cb = l.ca + up16(s.H);
   l.ldp = l.cb + (s.is_delta ? up16(s.H) : 0);
   l.tiles = l.ldp / 16;
+  l.n_chunks = cdiv(KD, LOGIT_CHUNK);
+  l.one = step_is_one(s, l.n_chunks);
   l.nsplit = attend_splits(M * s.HQ, s.n_kept * s.block + s.n_in + s.T);
+  if (l.one) l.nsplit = step_one_splits(s, l.n_chunks, l.nsplit);
   size_t at = 0;
   auto take = [&](size_t n) { const size_t r = at; at += (n + 255) / 256 * 256; return r; };
   l.proj = take((size_t)M * l.ldp * 2);
   l.q_conv = take((size_t)M * KD * 2);
   l.q_lin = s.flags & NATSL_STEP_L2_ROWS ? take((size_t)M * KD * 2) : l.q_conv;
   l.q_attn = take((size_t)M * KD * 2);
-  l.o_lin = take((size_t)M * VD * 2);
+  l.o_lin = take((size_t)M * VD * 4);
   l.y = take((size_t)M * VD * 2);
   l.partials = take((size_t)M * s.HQ * ATTEND_MAX_SPLITS * (2 + VD / s.HQ) * 4);   // (the size does not follow the cache's)
+  l.logits = take((size_t)M * l.n_chunks * s.HQ * 2 * 4);
+  l.arrived = take((size_t)M * s.HQ * 4);
   l.bytes = at;
   return l;
 }
@@ -363,6 +759,8 @@ extern "C" int natsl_layer_step_fwd(const natsl_layer_step* step, void* workspac
   const GemmSeg segs[GEMM_SEGS] = {{(const bf16_t*)s.wq, KD, 0, l.cq}, {(const bf16_t*)s.wk, KD, 0, l.ck}, {(const bf16_t*)s.wv, VD, 0, l.cv},
                                    {(const bf16_t*)s.wg, VD, 0, l.cg}, {(const bf16_t*)s.wa, s.H, 0, l.ca}, {(const bf16_t*)s.wb, s.H, 0, l.cb}};
   g.n_seg = s.is_delta ? 6 : 5;
+  unsigned* arrived = (unsigned*)(ws + l.arrived);
+  g.zero = arrived; g.n_zero = l.one ? M * s.HQ : 0;
   for (int i = 0; i < GEMM_SEGS; ++i) {
     g.seg[i] = segs[i];
     g.seg[i].tile0 = segs[i].col0 / 16;
@@ -372,12 +770,6 @@ extern "C" int natsl_layer_step_fwd(const natsl_layer_step* step, void* workspac
   StepMix m;
   m.s = s; m.proj = proj; m.ldp = l.ldp; m.cq = l.cq; m.ck = l.ck; m.cv = l.cv; m.ca = l.ca; m.cb = l.cb;
   m.q_conv = q_conv; m.q_lin = q_lin; m.q_attn = q_attn;
-  const dim3 mgrid(3 * s.H + (s.block_hidden ? cdiv(s.D, 256) : 0), s.B);
-  if (s.conv_width == 4) hipLaunchKernelGGL((step_mix_kernel<4>), mgrid, dim3(256), 0, st, m);
-  else if (s.conv_width == 3) hipLaunchKernelGGL((step_mix_kernel<3>), mgrid, dim3(256), 0, st, m);
-  else hipLaunchKernelGGL((step_mix_kernel<2>), mgrid, dim3(256), 0, st, m);
-  if ((rc = check_launch(what)) != NATSL_OK) return rc;
-
   AttnParams a;
   a.q = q_attn; a.k = s.cache_k; a.v = s.cache_v; a.mask = nullptr; a.o = nullptr;
   a.B = s.B; a.TQ = s.T; a.TK = s.n_kept * s.block + s.n_in + s.T; a.HQ = a.HKV = s.HQ; a.HM = s.HN; a.dtype = NATSL_BF16;
@@ -394,19 +786,32 @@ extern "C" int natsl_layer_step_fwd(const natsl_layer_step* step, void* workspac
   r.decay = (s.flags & NATSL_STEP_DECAY) != 0; r.l2norm = s.is_delta; r.query_only = 0;
   r.kv_stride = s.block; r.kv_first = s.n_in; r.fresh_start = (s.flags & NATSL_STEP_FRESH_START) != 0; r.aligned = 1;
   r.g_cumsum_out = s.g_cumsum_out;
-  if ((rc = launch_attend_and_recur(what, a, r, s.is_delta != 0, s.K, KA, VA, st)) != NATSL_OK) return rc;
-
   StepTail t;
   t.partials = partials; t.nsplit = l.nsplit; t.o_lin = o_lin; t.q_conv = q_conv; t.proj = proj; t.w_mix = (const bf16_t*)s.w_mix;
   t.w1 = s.out_norm1; t.w2 = s.out_norm2; t.w_dtype = s.out_norm_dtype; t.y = y; t.rows = M; t.HQ = s.HQ; t.KD = KD; t.ldp = l.ldp; t.cg = l.cg;
   t.eps = s.out_norm_eps;
+  RowsGemm o;
+  o.x = y; o.out = (bf16_t*)s.out; o.M = M; o.D = VD; o.ldo = s.D; o.n_seg = 1; o.zero = nullptr; o.n_zero = 0;
+  for (int i = 0; i < GEMM_SEGS; ++i) o.seg[i] = {(const bf16_t*)s.wo, s.D, 0, 0};
+  if (l.one) {
+    StepOne f;
+    f.m = m; f.a = a; f.r = r; f.t = t;
+    f.o_lin = (float*)(ws + l.o_lin); f.logits = (float*)(ws + l.logits); f.arrived = arrived;
+    f.n_chunks = l.n_chunks; f.n_logits = s.B * l.n_chunks; f.n_rec = s.B * s.H * cdiv(s.V, 64);
+    if ((rc = launch_step_one(what, f, s.K, KA, VA, st)) != NATSL_OK) return rc;
+    return gemm(o, cdiv(s.D, 16));
+  }
+
+  const dim3 mgrid(3 * s.H + (s.block_hidden ? cdiv(s.D, 256) : 0), s.B);
+  if (s.conv_width == 4) hipLaunchKernelGGL((step_mix_kernel<4>), mgrid, dim3(256), 0, st, m);
+  else if (s.conv_width == 3) hipLaunchKernelGGL((step_mix_kernel<3>), mgrid, dim3(256), 0, st, m);
+  else hipLaunchKernelGGL((step_mix_kernel<2>), mgrid, dim3(256), 0, st, m);
+  if ((rc = check_launch(what)) != NATSL_OK) return rc;
+  if ((rc = launch_attend_and_recur(what, a, r, s.is_delta != 0, s.K, KA, VA, st)) != NATSL_OK) return rc;
+
   const dim3 tgrid(cdiv(M * s.HQ, 4));
   if (VA == 128) hipLaunchKernelGGL((step_tail_kernel<128>), tgrid, dim3(256), 0, st, t);
   else hipLaunchKernelGGL((step_tail_kernel<64>), tgrid, dim3(256), 0, st, t);
   if ((rc = check_launch(what)) != NATSL_OK) return rc;
-
-  RowsGemm o;
-  o.x = y; o.out = (bf16_t*)s.out; o.M = M; o.D = VD; o.ldo = s.D; o.n_seg = 1;
-  for (int i = 0; i < GEMM_SEGS; ++i) o.seg[i] = {(const bf16_t*)s.wo, s.D, 0, 0};
   return gemm(o, cdiv(s.D, 16));
 }

@@ -84,6 +84,21 @@ def test_layer_step_matches_the_general_path(kind, geometry, ops, B, T0, sizes, 
         assert a.shape == b.shape and rel_l2(a.float(), b.float()) <= 5e-3, f"cache tensor {i}: rel-L2 {rel_l2(a.float(), b.float()):.3e}"
 
 
+@pytest.mark.parametrize("kind,B,T0,n,more", [
+    ('gdn', 1, 64, 3, {}),                                                # the first rows of a chunk
+    ('gdn', 2, 94, 4, dict(head_dim=64, num_heads=3, num_attn_heads=3)),  # over a chunk of keys; 192 channels of q in one chunk of 256; 3 heads
+    ('gdn', 1, 126, 4, dict(head_dim=64, num_heads=5, num_attn_heads=5)), # over a block and a split; 320 channels, 5 heads on 4 waves
+    ('gdn', 3, 253, 5, dict(head_dim=192, num_heads=1, num_attn_heads=3)),
+    ('gdn', 1, 2110, 2, dict(num_attn_heads=2, expand_v=1)),                          # 16 splits
+    ('mamba', 2, 95, 3, dict(head_dim=64, expand_v=1, num_heads=18, num_attn_heads=18)),   # more heads than a wave's four rounds of four
+    ('mamba', 1, 127, 2, dict(expand_v=1)),
+    ('mamba', 1, 257, 2, dict(attn_with_short_conv=False, conv_bias=True)),
+])
+def test_layer_step_of_one_token(kind, B, T0, n, more, monkeypatch):
+    """The launch that does everything between the products of a one-token step, at the edges of its chunks, splits and heads."""
+    test_layer_step_matches_the_general_path(kind, None, 'all', B, T0, (1,) * n, more, monkeypatch)
+
+
 @pytest.mark.parametrize("kind", ['gdn', 'mamba'])
 @pytest.mark.parametrize("float_gates", [False, True])
 def test_layer_step_forms_the_general_paths_gates(kind, float_gates, monkeypatch):

@@ -84,20 +84,32 @@ NATSL_DEVICE bool lin_type(const void* types, int dtype, size_t i) {
 // =============================================================================================
 // prep
 // =============================================================================================
+// acc + the squares of two bf16
+NATSL_DEVICE float sum_squares(const unsigned w, const float acc) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  const bf16x2 x = __builtin_bit_cast(bf16x2, w);
+  return __builtin_amdgcn_fdot2_f32_bf16(x, x, acc, false);
+}
+
 // PF ("P formed by the scan"): the kernel reads k only -- no q tile, no q k^T product, no P -- and leaves TmB and six scale
 // vectors; the two extra ones (in the first 512 bytes of the unit's P area) are the exponents the scan needs to form
 // P_ij = rq_i (q_i . k_j) exp2(gq_i - gk_j):   gk = gamma log2(e) - log2 rk,   gq = gamma log2(e) + log2 scale,
 // and sq comes without its 1/|q| factor (the scan takes the row norms of q from the tile it holds anyway).
+//
+// Bound by the instructions of its phases and by the barriers between them (63 % of the wave cycles wait; 2.2 TB/s), so what counts is
+// their number and how many workgroups share a CU: six with PF (26 KB of LDS, 78 registers).  B8 T8192 H16 d128: 124 us; with row
+// norms by separate conversions, branches around the exponentials, the substitution in 16 lanes of every wave and five workgroups a
+// CU 137.  A loop over units with the next rows requested ahead takes registers from it: 150 us at four workgroups.
 template <int DK, bool DELTA, bool PF>
 __global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams p) {
   static_assert(DELTA || !PF, "the Mamba form has its own prep");
   constexpr int KP = DK + 8;   // bf16 row pitch
   constexpr int KL = DK / 32;  // 16-byte loads per thread per tile
-  // The 64x64 fp32 matrices of the solve are kept as their ten lower 16x16 blocks, block (i, k) at
-  // index i(i+1)/2 + k, rows of BP floats.  A = strictly lower system matrix; X = (I+A)^-1 row-major;
-  // Xt = the four DIAGONAL blocks of X transposed (so that such a block serves as an MFMA B operand with one 16-byte read).
-  constexpr int BP = 20, BLK = 16 * BP, NBLK = 10;
-  constexpr int TILE_BYTES = (PF ? 1 : 2) * C * KP * 2, SOLVE_BYTES = (2 * NBLK + 4) * BLK * 4;
+  // The 64x64 fp32 matrices of the solve are kept as their lower 16x16 blocks, rows of BP floats.  A = strictly lower system matrix, ten
+  // blocks, (i, k) at index i(i+1)/2 + k; its diagonal blocks are replaced by those of X = (I+A)^-1.  Xb = the six others of X,
+  // (i, k) at i(i-1)/2 + k.  Xt = the diagonal blocks of X transposed (an MFMA B operand with one 16-byte read).
+  constexpr int BP = 20, BLK = 16 * BP, NBLK = 10, NOFF = 6;
+  constexpr int TILE_BYTES = (PF ? 1 : 2) * C * KP * 2, SOLVE_BYTES = (NBLK + NOFF + 4) * BLK * 4;
   // LDS: the q, k tiles are dead once the Gram products are done; the solve reuses their space
   constexpr int REGION0 = (DELTA && SOLVE_BYTES > TILE_BYTES) ? SOLVE_BYTES : TILE_BYTES;
   __shared__ __align__(16) unsigned char region0[REGION0];
@@ -106,10 +118,13 @@ __global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams 
   bf16_t* Ks = PF ? Qs : Qs + C * KP;   // (no q tile with PF)
   float* Ab = reinterpret_cast<float*>(region0);
   float* Xb = Ab + NBLK * BLK;
-  float* Xt = Xb + NBLK * BLK;
+  float* Xt = Xb + NOFF * BLK;
   auto bidx = [](int i, int k) { return i * (i + 1) / 2 + k; };
+  auto xblk = [&](int i, int k) { return i == k ? Ab + bidx(i, i) * BLK : Xb + (i * (i - 1) / 2 + k) * BLK; };
 
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  // the waves' shares differ: workgroups that are on a CU together give a share to different SIMDs
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = ((__builtin_amdgcn_readfirstlane(tid >> 6)) + (int)(blockIdx.x >> 8)) & 3;
   const int gc = blockIdx.x / p.H, h = blockIdx.x % p.H;
   int bos, len, c, bos_nats;
   if (p.seqs == nullptr) {
@@ -152,10 +167,8 @@ __global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams 
       *reinterpret_cast<u32x4*>(Ks + row * KP + (seg + 4 * i) * 8) = b;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const float a0 = __uint_as_float(a[j] << 16), a1 = __uint_as_float(a[j] & 0xffff0000u);
-        const float b0 = __uint_as_float(b[j] << 16), b1 = __uint_as_float(b[j] & 0xffff0000u);
-        sq += a0 * a0 + a1 * a1;
-        sk += b0 * b0 + b1 * b1;
+        if (!PF) sq = sum_squares(a[j], sq);
+        sk = sum_squares(b[j], sk);
       }
     }
     sq += __shfl_xor(sq, 1); sq += __shfl_xor(sq, 2);
@@ -246,8 +259,11 @@ __global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams 
           if ((i0 >> 4) >= (j >> 4)) {
             float* dst = Ab + bidx(i0 >> 4, j >> 4) * BLK + (i0 & 15) * BP + (j & 15);
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-              dst[e * BP] = i0 + e > j ? bi4[e] * ri4[e] * rkj * gk[4 * q4 + e] * __expf(gi4[e] - gj) : 0.f;
+            for (int e = 0; e < 4; ++e) {
+              float a = bi4[e] * ri4[e] * rkj * gk[4 * q4 + e] * __expf(gi4[e] - gj);
+              asm volatile("" : "+v"(a));               // (a select, no branch around the exponential)
+              dst[e * BP] = i0 + e > j ? a : 0.f;
+            }
           }
         }
       }
@@ -279,10 +295,11 @@ __global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams 
   __syncthreads();
 
   // ---- X = (I + A)^-1 in fp32, 4x4 blocks of 16x16 ------------------------------------------
-  // diagonal blocks by forward substitution: wave b owns block (b, b), one column per lane
+  // diagonal blocks by forward substitution: one wave, 16 lanes a block, one column per lane (16 lanes of each of the four waves
+  // cost the SIMDs four times the issue slots)
   const int x16 = lane & 15, g4 = lane >> 4;
-  if (lane < 16) {
-    const float* Ad = Ab + bidx(wave, wave) * BLK;
+  if (wave == 3) {
+    float* Ad = Ab + bidx(g4, g4) * BLK;
     f32x4 arow[16][4];
 #pragma unroll
     for (int r = 1; r < 16; ++r)
@@ -296,10 +313,9 @@ __global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams 
       for (int j = 0; j < r; ++j) acc -= arow[r][j >> 2][j & 3] * x[j];
       x[r] = acc;
     }
-    float* Xd = Xb + bidx(wave, wave) * BLK;
-    float* Xtd = Xt + wave * BLK;
+    float* Xtd = Xt + g4 * BLK;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) Xd[r * BP + x16] = x[r];
+    for (int r = 0; r < 16; ++r) Ad[r * BP + x16] = x[r];
 #pragma unroll
     for (int r4 = 0; r4 < 4; ++r4)
       *reinterpret_cast<f32x4*>(Xtd + x16 * BP + 4 * r4) = (f32x4){x[4 * r4], x[4 * r4 + 1], x[4 * r4 + 2], x[4 * r4 + 3]};
@@ -330,12 +346,12 @@ __global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams 
             for (int st = 0; st < 4; ++st) M = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[st], b4[st], M, 0, 0, 0);
           }
         }
-        const f32x4 d4 = *reinterpret_cast<const f32x4*>(Xb + bidx(i, i) * BLK + x16 * BP + 4 * g4);
+        const f32x4 d4 = *reinterpret_cast<const f32x4*>(xblk(i, i) + x16 * BP + 4 * g4);
         f32x4 Xa = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int st = 0; st < 4; ++st) Xa = __builtin_amdgcn_mfma_f32_16x16x4f32(d4[st], M[st], Xa, 0, 0, 0);
         Xcol[i] = (f32x4){-Xa[0], -Xa[1], -Xa[2], -Xa[3]};
-        float* Xo = Xb + bidx(i, k) * BLK;
+        float* Xo = Xb + (i * (i - 1) / 2 + k) * BLK;
 #pragma unroll
         for (int r = 0; r < 4; ++r) Xo[(4 * g4 + r) * BP + x16] = Xcol[i][r];
       }
@@ -351,7 +367,7 @@ __global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams 
       float x[16];
 #pragma unroll
       for (int e4 = 0; e4 < 4; ++e4) {
-        const f32x4 xv = cb <= (row >> 4) ? *reinterpret_cast<const f32x4*>(Xb + bidx(row >> 4, cb <= (row >> 4) ? cb : 0) * BLK + (row & 15) * BP + 4 * e4)
+        const f32x4 xv = cb <= (row >> 4) ? *reinterpret_cast<const f32x4*>(xblk(row >> 4, cb) + (row & 15) * BP + 4 * e4)
                                           : (f32x4){0.f, 0.f, 0.f, 0.f};
         const f32x4 bv = *reinterpret_cast<const f32x4*>(bet + 16 * cb + 4 * e4);
 #pragma unroll

@@ -438,13 +438,17 @@ NATSL_DEVICE void dma16(const void* base, const unsigned voff, const unsigned ld
 }
 
 // Swizzle of the k / q tiles in LDS (row-major, unpadded, rows of DK bf16): 16-byte segment s of row r sits at
-// s ^ kq_swizzle(r).  The A-operand read of a 16x16x32 instruction (16 lanes = 16 consecutive rows at one segment) and
-// the transposing read of k^T (16 lanes = 4 consecutive rows x 4 segments 0..3 of an aligned group) must both fall on
-// 16 different 16-byte slots of the 256-byte bank period.
+// s ^ kq_swizzle(r).  The 256-byte bank period has 16 such slots.  The A-operand read of a 16x16x32 instruction (16 consecutive
+// rows at segments 4 s .. 4 s + 3) is served 16 lanes at a time, rows 0..3 and 12..15 at one segment together with rows 4..11 at
+// its neighbour (s ^ 1): the slots of rows 4..11 have to come in such pairs.  The transposing read of k^T (4 consecutive rows x
+// segments 0..3 of an aligned group per 16 lanes, half a slot each) is served 32 lanes at a time: no more than two of rows 0..7
+// may share the bits above the lowest two.  Measured, ns an instruction and CU: 1.9 and 1.7, as without any conflict; with
+// (r & 3) << 2 | r >> 2 for DK = 128 the operand read takes 3.4, with (r >> 1) & 7 for the others the transposing read does.  The scan
+// of B8 T8192 H16 d128 with it: 333 -> 326 us.
 template <int DK>
 NATSL_DEVICE int kq_swizzle(const int r) {
-  if constexpr (DK == 128) return ((r & 3) << 2) | ((r >> 2) & 3);   // 16 segments per row, a row = one bank period
-  return (r >> 1) & 7;                                               // 8 or 24 segments per row: low three bits only
+  if constexpr (DK == 128) return ((r & 3) << 2) | (-(r >> 2) & 3);  // 16 segments per row, a row = one bank period
+  return (((r >> 1) & 1) << 2) | (-(r >> 2) & 3);                    // 8 or 24 segments per row: low three bits only, rows in pairs
 }
 
 typedef __attribute__((address_space(3))) const bf16x8* lds_b128_t;

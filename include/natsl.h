@@ -115,9 +115,10 @@ int natsl_softmax_sparse_fwd(const void* q, const void* k, const void* v, void* 
                              int V, int TN, int block, float scale, int same_block_visible, int dtype,
                              const natsl_seq_row* seqs, int n_seqs, int total_units, natsl_stream_t stream);
 
-/* The same operation with the same results bit for bit, always as one workgroup per query tile (what
- * natsl_softmax_sparse_fwd itself runs for packed input, ragged lengths and small problems): for callers that
- * want no library-owned device state in the launch, and the regression check of the persistent kernel.
+/* The same operation, always as one workgroup per query tile (what natsl_softmax_sparse_fwd itself runs for packed
+ * input and small problems): for callers that want no library-owned device state in the launch, and the regression
+ * check of the persistent kernel.  The same results bit for bit, except for the queries of a sequence's last 256-row
+ * tile where its length is no multiple of 64: those differ by the rounding of the probabilities in the row sums.
  * Same reference interface as natsl_softmax_sparse_fwd. */
 int natsl_softmax_sparse_fwd_per_tile(const void* q, const void* k, const void* v, void* o, float* lse,
                              const void* types, int types_dtype, const int32_t* nats_block_indices,

@@ -959,7 +959,12 @@ NATSL_DEVICE unsigned xcc_id() {
   return x & (STREAM_QUEUES - 1);
 }
 
-template <int DK, int DV>
+// RAGGED: T is not a whole number of tiles.  The last tile of a sequence keeps its full set of chunks (the rules of the rings do not
+// change); its chunks past the end are requested from the tile's first chunk and nobody takes part in them, the chunk that the end
+// cuts (marked in the chunk table: all bits of its row inverted) repeats the last row, waves behind the end stay idle, and rows
+// behind it are not stored.  Against a workgroup per tile: B8 T4095 H12 64/128 half attention 264 -> 212 us, B8 T8191 H16 128/128
+// 729 -> 661, B4 T8191 H32 128/64 593 -> 557, B4 T4095 H32 64/64 181 -> 161.
+template <int DK, int DV, bool RAGGED>
 __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
   constexpr int QW = 32, QTILE = 256, KSTEPS = DK / 16, VT = DV / 32;
@@ -975,7 +980,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
   const bool late = wave >= 4;
   const int gw = wave & 3;
   const int Bs = p.block, per_blk = Bs >> 6;
-  const unsigned NT = (unsigned)p.T / QTILE;
+  const unsigned NT = ((unsigned)p.T + (RAGGED ? QTILE - 1 : 0)) / QTILE;
   const unsigned n_pairs = (unsigned)(p.B * p.HQ);
   const size_t krow = (size_t)p.HKV * DK, vrow = (size_t)p.HKV * DV;
   const size_t list_stride = (size_t)p.HN * 2;
@@ -1001,17 +1006,45 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
       src[j] = (unsigned)((size_t)r * vrow * sizeof(bf16_t)) + 16u * ((unsigned)pos ^ v_swizzle<DV>(r));
     }
   }
-  auto dma_v = [&](const int row, const unsigned sp) __attribute__((always_inline)) {
+  auto dma_v = [&](const int entry, const unsigned sp) __attribute__((always_inline)) {
+    const int row = RAGGED ? entry ^ (entry >> 31) : entry;
     const char* g = reinterpret_cast<const char*>(p.v) + ((size_t)(unsigned)row << V_SHIFT);
     const unsigned l0 = lds_v + (sp & 3) * VTILE + VI * gw * 1024;
+    if (RAGGED && entry < 0) {
+      int ll = lane;
+      asm volatile("" : "+v"(ll));
+#pragma unroll
+      for (int j = 0; j < VI; ++j) {
+        const int r = VROWS_I * (VI * gw + j) + ll / (DV / 8), pos = ll % (DV / 8);
+        dma16(g, (unsigned)((size_t)min(r, (p.T & 63) - 1) * vrow * sizeof(bf16_t)) + 16u * ((unsigned)pos ^ v_swizzle<DV>(r)), l0 + j * 1024);
+      }
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < VI; ++j) dma16(g, src[j], l0 + j * 1024);
   };
-  auto dma_k = [&](const int row, const unsigned sp) __attribute__((always_inline)) {
+  auto dma_k = [&](const int entry, const unsigned sp) __attribute__((always_inline)) {
+    const int row = RAGGED ? entry ^ (entry >> 31) : entry;
     const char* g = reinterpret_cast<const char*>(p.k) + ((size_t)(unsigned)row << K_SHIFT);
     const unsigned l0 = lds_k + (sp & 3) * KTILE + KI * gw * 1024;
+    if (RAGGED && entry < 0) {
+      int ll = lane;
+      asm volatile("" : "+v"(ll));
+#pragma unroll
+      for (int j = 0; j < KI; ++j) {
+        const int r = KROWS_I * (KI * gw + j) + ll / (DK / 8), pos = ll % (DK / 8);
+        dma16(g, (unsigned)((size_t)min(r, (p.T & 63) - 1) * krow * sizeof(bf16_t)) + 16u * (pos ^ (DK == 128 ? (r & 15) : ((r >> 1) & 7))), l0 + j * 1024);
+      }
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < KI; ++j) dma16(g, src[j], l0 + j * 1024);
+  };
+  // table entry of chunk j of a tile's own: row0 the row of its first, dstart that one's token
+  auto own_entry = [&](const int row0, const int dstart, const int j) __attribute__((always_inline)) -> int {
+    if (!RAGGED) return row0 + 64 * j * p.HKV;
+    const int jj = dstart + 64 * j < p.T ? j : 0, row = row0 + 64 * jj * p.HKV;
+    return dstart + 64 * jj + 64 > p.T ? ~row : row;
   };
   const int lt = tid & 255;
   const unsigned k_lane = (unsigned)(l32 * DK * 2) + 16u * (hf ^ (DK == 128 ? (l32 & 15) : ((l32 >> 1) & 7)));
@@ -1029,8 +1062,8 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
   };
   // ticket t of the queue in use -> the tile it stands for, written as the "next tile" part of a record; moves on to the
   // other queues (one synchronous ticket each) when the queue in use has no tiles left.  Returns the row index of the
-  // tile's first chunk (-1: no tile left).
-  auto resolve_ticket = [&](unsigned t, StreamTile* out) -> int {
+  // tile's first chunk (-1: no tile left); first: that chunk's token.
+  auto resolve_ticket = [&](unsigned t, StreamTile* out, int& first) -> int {
     bool ok = false;
     unsigned qx = 0;
     while (cq < STREAM_QUEUES) {
@@ -1061,6 +1094,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
     const unsigned n = pair / (unsigned)p.HQ, hq = pair - n * (unsigned)p.HQ;
     const unsigned dstart = (tile * QTILE / (unsigned)Bs) * (unsigned)Bs;
     const unsigned hkv = hq / (unsigned)p.g_kv;
+    first = (int)dstart;
     if (lane == 0) {
       out->valid = 1;
       out->n = (int)n;
@@ -1081,12 +1115,13 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
   int c_n = 0, c_hq = 0, c_tile = 0, c_hkv = 0, c_hn = 0, dstart = 0, dblk = 0;
   bool req = false;  // this wave made a request in its last request step: that one may still be in flight at the next barrier
   if (wave == 4) {
-    const int r0 = resolve_ticket(take_ticket(), &info[0]);
+    int d0 = 0;
+    const int r0 = resolve_ticket(take_ticket(), &info[0], d0);
     if (lane == 0) {
       info[0].diag_lo = info[0].diag_hi = 0u;
       info[0].count[0] = info[0].count[1] = info[0].count[2] = info[0].count[3] = 0;
     }
-    if (r0 >= 0 && lane < 4) rows[0][4 + lane] = r0 + 64 * lane * p.HKV;   // the virtual tile has four chunks of its own
+    if (r0 >= 0 && lane < 4) rows[0][4 + lane] = own_entry(r0, d0, lane);   // the virtual tile has four chunks of its own
   }
 
   bf16x8 QB[KSTEPS];
@@ -1101,7 +1136,8 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
   // lines.  The space is an area of its own, a quarter of it per wave of a group.  The early waves use it right after their last
   // chunk; the late waves once the hand-over barrier of the next tile is behind them (all early waves have then read their rows
   // back), before anything of the new tile touches their accumulators.  row0: flat (token, head) index of the wave's first query.
-  auto store_tile = [&](const unsigned stage, const size_t row0) __attribute__((always_inline)) {
+  // n_rows: how many of the wave's queries there are (RAGGED).
+  auto store_tile = [&](const unsigned stage, const size_t row0, const int n_rows) __attribute__((always_inline)) {
     constexpr int PW = DV / 2, RB = PW * 2, NSEG = RB / 16, RPI = 64 / NSEG;   // columns per pass, row bytes, segments, rows per instruction
     typedef __attribute__((address_space(3))) u32x2* lds_w8;
     typedef __attribute__((address_space(3))) const u32x4* lds_r16;
@@ -1111,7 +1147,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
     int ol = lane;
     asm volatile("" : "+v"(ol));   // (the lane's share of the addresses below is not to be kept through the chunk loops)
     const int ol32 = ol & 31, ohf = ol >> 5;
-    if (ohf == 0) p.lse[row0 + (size_t)ol32 * p.HQ] = has ? m_ref + __builtin_amdgcn_logf(l_tot) : 0.f;
+    if (ohf == 0 && (!RAGGED || ol32 < n_rows)) p.lse[row0 + (size_t)ol32 * p.HQ] = has ? m_ref + __builtin_amdgcn_logf(l_tot) : 0.f;
     const unsigned wbase = stage + (unsigned)(ol32 * RB + 8 * ohf);
     const int rrow = ol / NSEG, rseg = ol % NSEG;
 #pragma unroll
@@ -1133,7 +1169,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
       for (int i = 0; i < 32 / RPI; ++i) {
         const int row = i * RPI + rrow;
         const u32x4 w = *reinterpret_cast<lds_r16>(stage + (unsigned)(row * RB) + 16u * ((unsigned)rseg ^ (unsigned)(row & (NSEG - 1))));
-        *reinterpret_cast<u32x4*>(p.o + (row0 + (size_t)row * p.HQ) * DV + ps * PW + rseg * 8) = w;
+        if (!RAGGED || row < n_rows) *reinterpret_cast<u32x4*>(p.o + (row0 + (size_t)row * p.HQ) * DV + ps * PW + rseg * 8) = w;
       }
       if (ps == 0) {
         __builtin_amdgcn_s_waitcnt(0xc07f);  // the rows have been read before the second half overwrites them
@@ -1156,6 +1192,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
   bool pend_store = false;   // late waves: the previous tile's output is still in the accumulators
   unsigned pend_stage = 0;
   size_t pend_row0 = 0;
+  int pend_rows = 0;
 
   for (;;) {
     // ---- hand-over barrier: the record and the list of the tile in work are complete ------------------------------
@@ -1189,12 +1226,13 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
       // (no next tile: this tile's rows are read again, so that the loads and the waits of the scaling below are on
       // every path -- with the loads under a condition the compiler assumes them pending wherever the queries are used)
       const size_t qrow = n_valid ? (size_t)(n_bos + n_tile_start) : (size_t)(bos + tile_start);
-      const bf16_t* qr = p.q + ((qrow + wave * QW + (ql & 31)) * p.HQ + (n_valid ? n_hq : c_hq)) * DK + 8 * (ql >> 5);
+      const int qi = wave * QW + (ql & 31), qmax = RAGGED ? p.T - 1 - (n_valid ? n_tile_start : tile_start) : QTILE;
+      const bf16_t* qr = p.q + ((qrow + (RAGGED ? min(qi, qmax) : qi)) * p.HQ + (n_valid ? n_hq : c_hq)) * DK + 8 * (ql >> 5);
 #pragma unroll
       for (int s = 0; s < KSTEPS; ++s) QB[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(qr + 16 * s));
     };
 
-    if (pend_store) store_tile(pend_stage, pend_row0);
+    if (pend_store) store_tile(pend_stage, pend_row0, pend_rows);
     scale_next_q();   // the queries requested at the end of the previous tile
 
     // which of the chunks from dstart on this wave takes part in, and which one is its own, causal chunk
@@ -1213,7 +1251,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
       } else {
         act = jc < my_chunk && kblk < my_blk && typed;
       }
-      act_mask = __ballot(act && al < n_diag);
+      act_mask = __ballot(act && al < n_diag && (!RAGGED || q0 < p.T));
       const unsigned long long cm = __ballot(cz && al < n_diag);
       causal_it = cm ? __builtin_ctzll(cm) : -1;
     }
@@ -1225,7 +1263,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
     l_run = 0.f;
     thr = -INFINITY;
     f32x16 s0, s1;
-    auto is_active = [&](const int it) -> bool { return it < n_diag ? (act_mask >> it) & 1ull : it < n_iters; };
+    auto is_active = [&](const int it) -> bool { return it < n_diag ? (act_mask >> it) & 1ull : it < n_iters && (!RAGGED || q0 < p.T); };
     bool cur_active = act_mask & 1ull;
     if (cur_active) qk_phase<DK>(lds_k + (sp0 & 3) * KTILE + k_lane, QB, m_ref, s0, s1);
 
@@ -1289,7 +1327,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
             p_nattn = p.nblk[((size_t)n_n * p.HN + n_hn) * 2];
             if (wave == 4) {
               const int blk = n_dblk + lane;
-              const bool in_range = lane < n_ndiag && (size_t)blk * Bs < (size_t)(n_tile_start + QTILE);
+              const bool in_range = lane < n_ndiag && (size_t)blk * Bs < (size_t)(n_tile_start + QTILE) && (!RAGGED || blk < p.TN);
               const size_t ti = ((size_t)(n_n * p.TN + (in_range ? blk : n_dblk)) * p.HN + n_hn) * 2;
               p_type = p.types_dtype == NATSL_F32 ? reinterpret_cast<const float*>(p.types)[ti]
                                                   : bf16_to_f32(reinterpret_cast<const bf16_t*>(p.types)[ti]);
@@ -1307,11 +1345,11 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
                 for (int sub = 0; sub < per_blk; ++sub)
                   rows[a ^ 1][n_ndiag + j * per_blk + sub] = (n_bos + pe[m] * Bs + 64 * sub) * p.HKV + n_hkv;
             }
-            if (lt < n_ndiag) rows[a ^ 1][lt] = (n_bos + n_dstart + 64 * lt) * p.HKV + n_hkv;
+            if (lt < n_ndiag) rows[a ^ 1][lt] = own_entry((n_bos + n_dstart) * p.HKV + n_hkv, n_dstart, lt);
             if (lane == 0) info[a ^ 1].count[gw] = cnt;
             if (wave == 4) {
               const int blk = n_dblk + lane;
-              const bool in_range = lane < n_ndiag && (size_t)blk * Bs < (size_t)(n_tile_start + QTILE);
+              const bool in_range = lane < n_ndiag && (size_t)blk * Bs < (size_t)(n_tile_start + QTILE) && (!RAGGED || blk < p.TN);
               const unsigned long long d = __ballot(in_range && rintf(p_type) == 1.0f);
               if (lane == 0) {
                 info[a ^ 1].diag_lo = (unsigned)d;
@@ -1323,10 +1361,11 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
             // the tile after the next: ticket asked for in the last chunk but one, turned into a tile in the last
             if (it == n_iters - 2 && cq < STREAM_QUEUES && lane == 0) t_ahead = atomicAdd(&queue[(xcc + (unsigned)cq) & 7u], 1u);
             if (last) {
-              const int r0 = resolve_ticket(__builtin_amdgcn_readfirstlane(t_ahead), &info[a ^ 1]);
+              int d0 = 0;
+              const int r0 = resolve_ticket(__builtin_amdgcn_readfirstlane(t_ahead), &info[a ^ 1], d0);
               // the next tile's table ends with the first four chunks of the tile after it
               const int nn_iters = n_ndiag + (info[a ^ 1].count[0] + info[a ^ 1].count[1] + info[a ^ 1].count[2] + info[a ^ 1].count[3]) * per_blk;
-              if (r0 >= 0 && lane < 4) rows[a ^ 1][nn_iters + lane] = r0 + 64 * lane * p.HKV;
+              if (r0 >= 0 && lane < 4) rows[a ^ 1][nn_iters + lane] = own_entry(r0, d0, lane);
             }
           }
           ev_it = it == 0 ? 1 : (it < n_iters - 2 ? n_iters - 2 : it + 1);
@@ -1356,6 +1395,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
     // ---- end of the tile: the next tile's queries, output (early waves now, late waves after the next hand-over barrier)
     {
       const size_t row0 = (size_t)(bos + q0) * p.HQ + c_hq;
+      const int n_rows = RAGGED ? p.T - q0 : QW;
       const unsigned stage = lds_o + gw * (32 * DV);
       load_next_q();   // (ahead of the stores: what waits for the queries later does not wait for the stores then)
       // What the first barrier of the next tile needs, K(2) and V(1) of that tile, has landed: newer than those are one request
@@ -1363,7 +1403,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
       static_assert(KSTEPS + KI <= 15 && KSTEPS + VI <= 15, "fits the low field of the wait");
       if (!late) {
         __builtin_amdgcn_s_waitcnt(0x0f70 | (KSTEPS + KI));
-        if (cur_real) store_tile(stage, row0);
+        if (cur_real) store_tile(stage, row0, n_rows);
         __builtin_amdgcn_s_waitcnt(0xc07f);   // the staged rows have been read
         if (!n_valid) {
           __syncthreads();   // the late waves take the staging area over
@@ -1373,12 +1413,13 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
         __builtin_amdgcn_s_waitcnt(0x0f70 | (KSTEPS + VI));
         if (!n_valid) {
           __syncthreads();
-          if (cur_real) store_tile(stage, row0);
+          if (cur_real) store_tile(stage, row0, n_rows);
           break;
         }
         pend_store = cur_real;
         pend_stage = stage;
         pend_row0 = row0;
+        pend_rows = n_rows;
       }
     }
     c_n = n_n; c_hq = n_hq; c_tile = n_tile; c_hkv = n_hkv; c_hn = n_hn; dstart = n_dstart; dblk = n_dblk;
@@ -1416,6 +1457,7 @@ static int launch_softmax(const SoftmaxParams& p, hipStream_t stream) {
 // other's tickets and leave tiles uncomputed, so keep fewer than STREAM_SLOTS launches of this entry in flight per GPU
 // and replay captured launches on the stream that also carries the eager ones.
 constexpr int STREAM_SLOTS = 64;
+static std::atomic<unsigned> stream_launches{0};   // of all forms of the kernel: they share the slots
 static __device__ __align__(256) unsigned stream_queues[STREAM_SLOTS * STREAM_SLOT_WORDS];
 
 __global__ void stream_queue_clear_kernel(unsigned* slot) {
@@ -1454,30 +1496,29 @@ static const StreamDevice* stream_device(int* rc) {
   return &devs[dev];
 }
 
-template <int DK, int DV>
+template <int DK, int DV, bool RAGGED>
 static int launch_softmax_stream(const SoftmaxParams& p, const StreamDevice* d, hipStream_t stream) {
-  static std::atomic<unsigned> launches{0};
   static std::atomic<unsigned long long> reserved{0};
   const size_t lds = (size_t)(4 * 64 * (DK + DV) + 64 * DV) * sizeof(bf16_t) + 1024;  // four K and four V tiles, the output's staging area; 1 KiB aligned
-  auto kern = softmax_stream_kernel<DK, DV>;
+  auto kern = softmax_stream_kernel<DK, DV, RAGGED>;
   if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, lds, "softmax")) return rc;
-  unsigned* queue = d->queues + (size_t)(launches.fetch_add(1) % STREAM_SLOTS) * STREAM_SLOT_WORDS;
+  unsigned* queue = d->queues + (size_t)(stream_launches.fetch_add(1) % STREAM_SLOTS) * STREAM_SLOT_WORDS;
   hipLaunchKernelGGL(stream_queue_clear_kernel, dim3(1), dim3(64), 0, stream, queue);
   hipLaunchKernelGGL(kern, dim3((unsigned)d->cus), dim3(512), lds, stream, p, queue);
   return check_launch("natsl_softmax_sparse_fwd");
 }
 
-// Which kernel natsl_softmax_sparse_fwd runs for a problem: the persistent one for unpacked input of whole 256-query
-// tiles, at least two per compute unit (its per-tile saving needs a tile to follow); else one workgroup per tile, of 256
+// Which kernel natsl_softmax_sparse_fwd runs for a problem: the persistent one for unpacked input of at least two
+// 256-query tiles per compute unit (its per-tile saving needs a tile to follow); else one workgroup per tile, of 256
 // queries on 8 waves once there is at least one such tile per compute unit (measured: from there on that shape is the
 // faster one; below, 128-query tiles fill more compute units).
 static int softmax_variant(int B, int T, int HQ, int HKV, int block, bool packed, bool allow_persistent, const StreamDevice** sd, int* rc) {
   *sd = nullptr;
   *rc = NATSL_OK;
-  if (allow_persistent && !packed && T % 256 == 0 && T <= 65536 && block <= 2048 && (long long)B * T * HKV < (1ll << 31)) {
+  if (allow_persistent && !packed && T <= 65536 && block <= 2048 && (long long)B * T * HKV < (1ll << 31)) {
     const StreamDevice* d = stream_device(rc);
     if (!d) return -1;
-    if ((long long)B * HQ * (T / 256) >= 2ll * d->cus) {
+    if ((long long)B * HQ * cdiv(T, 256) >= 2ll * d->cus) {
       *sd = d;
       return NATSL_SOFTMAX_PERSISTENT;
     }
@@ -1524,7 +1565,7 @@ static int softmax_fwd(const void* q, const void* k, const void* v, void* o, flo
   p.variant = variant == NATSL_SOFTMAX_TILE_128 ? 4 : 8;
 #define NATSL_SM(KK, VV)                                              \
   if (K == KK && V == VV) {                                           \
-    if (sd) return launch_softmax_stream<KK, VV>(p, sd, s);           \
+    if (sd) return T % 256 ? launch_softmax_stream<KK, VV, true>(p, sd, s) : launch_softmax_stream<KK, VV, false>(p, sd, s); \
     return p.variant == 8 ? launch_softmax<KK, VV, 8>(p, s) : launch_softmax<KK, VV, 4>(p, s); \
   }
   NATSL_SM(128, 128)

@@ -77,6 +77,29 @@ def test_persistent_kernel_equals_the_per_tile_kernel(B, T, HQ, H, HN, K, V, blo
     assert torch.equal(l1, l2)
 
 
+@pytest.mark.parametrize("T", [769, 801, 831, 832, 833, 895, 897, 960, 1023, 3 * 256 + 224])
+@pytest.mark.parametrize("K,V,H,block,same_block", [(128, 128, 32, 64, True), (64, 64, 8, 128, True), (64, 128, 32, 512, True), (128, 64, 16, 64, False)])
+def test_persistent_kernel_with_a_cut_last_tile(T, K, V, H, block, same_block):
+    """Sequences that end inside a tile, a wave's queries or a chunk: bit for bit what the per-tile kernel gives for whole chunks (same
+    order, same arithmetic), also where the rows behind a sequence's end, the next one's first, hold NaNs.  The tile of a cut chunk
+    goes another way in that kernel (its row sums take the probabilities before their rounding): there both are held to the bound that
+    each is held to against the oracle."""
+    B, HQ, HN, dev = 4, 32, 8, torch.device('cuda:0')
+    _, _, _, _, qd, kd, vd, tyd = _inputs(B, T, HQ, H, HN, K, V, block, 0.4, 31, dev)
+    kd[2, :5] = float('nan')
+    vd[2, :5] = float('inf')
+    o1, l1 = _call(qd, kd, vd, tyd, K, block, same_block, persistent=False)
+    o2, l2 = _call(qd, kd, vd, tyd, K, block, same_block, persistent=True)
+    torch.cuda.synchronize()
+    for x, y in ((o1, o2), (l1, l2)):
+        assert bool(torch.isfinite(y[[0, 1, 3]]).all())
+        whole = T if T % 64 == 0 else T // 256 * 256
+        assert torch.equal(x[[0, 1, 3], :whole], y[[0, 1, 3], :whole])
+        assert torch.equal(x[2].isnan(), y[2].isnan())
+        if whole < T:
+            assert_close(y[[0, 1, 3], whole:].float(), x[[0, 1, 3], whole:].float(), "last tile")
+
+
 def test_persistent_kernel_queues_across_launches_and_streams():
     """The ticket counters are shared device state: one slot per launch in rotation, zeroed on the launch's stream right
     before it."""

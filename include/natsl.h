@@ -115,8 +115,8 @@ int natsl_softmax_sparse_fwd(const void* q, const void* k, const void* v, void* 
                              int V, int TN, int block, float scale, int same_block_visible, int dtype,
                              const natsl_seq_row* seqs, int n_seqs, int total_units, natsl_stream_t stream);
 
-/* The same operation, always as one workgroup per query tile (what natsl_softmax_sparse_fwd itself runs for packed
- * input and small problems): for callers that want no library-owned device state in the launch, and the regression
+/* The same operation, always as one workgroup per query tile (what natsl_softmax_sparse_fwd itself runs for small
+ * problems and for more than 64 packed sequences): for callers that want no library-owned device state in the launch, and the regression
  * check of the persistent kernel.  The same results bit for bit, except for the queries of a sequence's last 256-row
  * tile where its length is no multiple of 64: those differ by the rounding of the probabilities in the row sums.
  * Same reference interface as natsl_softmax_sparse_fwd. */
@@ -126,7 +126,8 @@ int natsl_softmax_sparse_fwd_per_tile(const void* q, const void* k, const void* 
                              int V, int TN, int block, float scale, int same_block_visible, int dtype,
                              const natsl_seq_row* seqs, int n_seqs, int total_units, natsl_stream_t stream);
 
-/* Which kernel natsl_softmax_sparse_fwd runs for a problem on the current device (host-side query, no launch;
+/* Which kernel natsl_softmax_sparse_fwd runs for a problem on the current device (host-side query, no launch; packed: the
+ * number of packed sequences, 0 for a batch;
  * the choice that src/nats/ops/attns/attns.py:1497-1512 leaves to Triton's autotuner). */
 enum natsl_softmax_variant { NATSL_SOFTMAX_TILE_128 = 0, NATSL_SOFTMAX_TILE_256 = 1, NATSL_SOFTMAX_PERSISTENT = 2 };
 int natsl_softmax_fwd_variant(int B, int T, int HQ, int HKV, int block, int packed);

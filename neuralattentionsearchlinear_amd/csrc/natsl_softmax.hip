@@ -944,13 +944,14 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
 // memory, zeroed on the launch's stream by a small fill kernel right before the launch (see launch_softmax_stream).
 constexpr int STREAM_ROWS = 1088;  // chunk table of a tile: up to 1024 + 32 chunks of its own and four of the next tile (two tiles' tables are resident)
 constexpr int STREAM_QUEUES = 8;
+constexpr int STREAM_SEQS = 64;    // packed sequences: a lane each
 constexpr int STREAM_SLOT_WORDS = 16;  // per launch slot: 8 ticket counters (one per XCD), the rest unused padding to a 64-byte line
 
 struct StreamTile {
   int valid, n, hq, tile, hkv, hn, dstart, dblk;  // the tile AFTER the one this record belongs to
   unsigned diag_lo, diag_hi;                      // this tile: which of the blocks from dstart on are typed attention
   int count[4];                                   // this tile: prior attention blocks found by each late wave
-  int pad[2];
+  int bos, len, nats, pad[3];                     // the tile after: its sequence's first token, length and first selector block
 };
 
 NATSL_DEVICE unsigned xcc_id() {
@@ -959,11 +960,13 @@ NATSL_DEVICE unsigned xcc_id() {
   return x & (STREAM_QUEUES - 1);
 }
 
-// RAGGED: T is not a whole number of tiles.  The last tile of a sequence keeps its full set of chunks (the rules of the rings do not
+// RAGGED: packed sequences (p.seqs; at most STREAM_SEQS, looked up from a copy of the table in LDS), or one length that is not a whole
+// number of tiles.  The last tile of a sequence keeps its full set of chunks (the rules of the rings do not
 // change); its chunks past the end are requested from the tile's first chunk and nobody takes part in them, the chunk that the end
 // cuts (marked in the chunk table: all bits of its row inverted) repeats the last row, waves behind the end stay idle, and rows
 // behind it are not stored.  Against a workgroup per tile: B8 T4095 H12 64/128 half attention 264 -> 212 us, B8 T8191 H16 128/128
-// 729 -> 661, B4 T8191 H32 128/64 593 -> 557, B4 T4095 H32 64/64 181 -> 161.
+// 729 -> 661, B4 T8191 H32 128/64 593 -> 557, B4 T4095 H32 64/64 181 -> 161; four packed sequences of 65536 tokens in all, H32
+// 128/128, 1410 -> 1280.
 template <int DK, int DV, bool RAGGED>
 __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
@@ -973,6 +976,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int rows[2][STREAM_ROWS];
   __shared__ __align__(16) StreamTile info[2];
+  __shared__ int seq_tab[RAGGED ? 4 : 1][STREAM_SEQS];   // first token, length, first selector block, first tile
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -980,8 +984,19 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
   const bool late = wave >= 4;
   const int gw = wave & 3;
   const int Bs = p.block, per_blk = Bs >> 6;
-  const unsigned NT = ((unsigned)p.T + (RAGGED ? QTILE - 1 : 0)) / QTILE;
+  const bool packed = RAGGED && p.seqs != nullptr;
+  const unsigned NT = packed ? (unsigned)p.total_tiles : ((unsigned)p.T + (RAGGED ? QTILE - 1 : 0)) / QTILE;   // tiles of a (batch, head) pair
   const unsigned n_pairs = (unsigned)(p.B * p.HQ);
+  if (packed) {
+    if (tid < p.n_seqs) {
+      const SeqRow s = p.seqs[tid];
+      seq_tab[0][tid] = s.bos;
+      seq_tab[RAGGED ? 1 : 0][tid] = s.eos - s.bos;
+      seq_tab[RAGGED ? 2 : 0][tid] = s.bos_nats;
+      seq_tab[RAGGED ? 3 : 0][tid] = s.qtile_off;
+    }
+    __syncthreads();
+  }
   const size_t krow = (size_t)p.HKV * DK, vrow = (size_t)p.HKV * DV;
   const size_t list_stride = (size_t)p.HN * 2;
   constexpr int K_SHIFT = DK == 128 ? 8 : 7, V_SHIFT = DV == 128 ? 8 : 7;  // log2 of a K / V row in bytes
@@ -1006,7 +1021,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
       src[j] = (unsigned)((size_t)r * vrow * sizeof(bf16_t)) + 16u * ((unsigned)pos ^ v_swizzle<DV>(r));
     }
   }
-  auto dma_v = [&](const int entry, const unsigned sp) __attribute__((always_inline)) {
+  auto dma_v = [&](const int entry, const unsigned sp, const int len) __attribute__((always_inline)) {
     const int row = RAGGED ? entry ^ (entry >> 31) : entry;
     const char* g = reinterpret_cast<const char*>(p.v) + ((size_t)(unsigned)row << V_SHIFT);
     const unsigned l0 = lds_v + (sp & 3) * VTILE + VI * gw * 1024;
@@ -1016,14 +1031,14 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
 #pragma unroll
       for (int j = 0; j < VI; ++j) {
         const int r = VROWS_I * (VI * gw + j) + ll / (DV / 8), pos = ll % (DV / 8);
-        dma16(g, (unsigned)((size_t)min(r, (p.T & 63) - 1) * vrow * sizeof(bf16_t)) + 16u * ((unsigned)pos ^ v_swizzle<DV>(r)), l0 + j * 1024);
+        dma16(g, (unsigned)((size_t)min(r, (len & 63) - 1) * vrow * sizeof(bf16_t)) + 16u * ((unsigned)pos ^ v_swizzle<DV>(r)), l0 + j * 1024);
       }
       return;
     }
 #pragma unroll
     for (int j = 0; j < VI; ++j) dma16(g, src[j], l0 + j * 1024);
   };
-  auto dma_k = [&](const int entry, const unsigned sp) __attribute__((always_inline)) {
+  auto dma_k = [&](const int entry, const unsigned sp, const int len) __attribute__((always_inline)) {
     const int row = RAGGED ? entry ^ (entry >> 31) : entry;
     const char* g = reinterpret_cast<const char*>(p.k) + ((size_t)(unsigned)row << K_SHIFT);
     const unsigned l0 = lds_k + (sp & 3) * KTILE + KI * gw * 1024;
@@ -1033,18 +1048,18 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
 #pragma unroll
       for (int j = 0; j < KI; ++j) {
         const int r = KROWS_I * (KI * gw + j) + ll / (DK / 8), pos = ll % (DK / 8);
-        dma16(g, (unsigned)((size_t)min(r, (p.T & 63) - 1) * krow * sizeof(bf16_t)) + 16u * (pos ^ (DK == 128 ? (r & 15) : ((r >> 1) & 7))), l0 + j * 1024);
+        dma16(g, (unsigned)((size_t)min(r, (len & 63) - 1) * krow * sizeof(bf16_t)) + 16u * (pos ^ (DK == 128 ? (r & 15) : ((r >> 1) & 7))), l0 + j * 1024);
       }
       return;
     }
 #pragma unroll
     for (int j = 0; j < KI; ++j) dma16(g, src[j], l0 + j * 1024);
   };
-  // table entry of chunk j of a tile's own: row0 the row of its first, dstart that one's token
-  auto own_entry = [&](const int row0, const int dstart, const int j) __attribute__((always_inline)) -> int {
+  // table entry of chunk j of a tile's own: row0 the row of its first, dstart that one's token, len the sequence's length
+  auto own_entry = [&](const int row0, const int dstart, const int len, const int j) __attribute__((always_inline)) -> int {
     if (!RAGGED) return row0 + 64 * j * p.HKV;
-    const int jj = dstart + 64 * j < p.T ? j : 0, row = row0 + 64 * jj * p.HKV;
-    return dstart + 64 * jj + 64 > p.T ? ~row : row;
+    const int jj = dstart + 64 * j < len ? j : 0, row = row0 + 64 * jj * p.HKV;
+    return dstart + 64 * jj + 64 > len ? ~row : row;
   };
   const int lt = tid & 255;
   const unsigned k_lane = (unsigned)(l32 * DK * 2) + 16u * (hf ^ (DK == 128 ? (l32 & 15) : ((l32 >> 1) & 7)));
@@ -1062,8 +1077,8 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
   };
   // ticket t of the queue in use -> the tile it stands for, written as the "next tile" part of a record; moves on to the
   // other queues (one synchronous ticket each) when the queue in use has no tiles left.  Returns the row index of the
-  // tile's first chunk (-1: no tile left); first: that chunk's token.
-  auto resolve_ticket = [&](unsigned t, StreamTile* out, int& first) -> int {
+  // tile's first chunk (-1: no tile left); first: that chunk's token, len: its sequence's length.
+  auto resolve_ticket = [&](unsigned t, StreamTile* out, int& first, int& len) -> int {
     bool ok = false;
     unsigned qx = 0;
     while (cq < STREAM_QUEUES) {
@@ -1081,7 +1096,8 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
     // Order of a queue: first every pair's NT - NL late (long) tiles, pair after pair, latest tile first; then every
     // pair's NL early (short) tiles the same way.  With the pairs' tiles simply one after the other, the last pair's
     // longest tile would start when only that pair's tiles are left, and the other CUs of the XCD idle while it runs.
-    const unsigned NL = NT / 3u, NH = NT - NL, heavy = (queue_units(qx) / NT) * NH;
+    // (Packed: a pair's tiles from the last sequence's last to the first one's first.)
+    const unsigned NL = packed ? 0u : NT / 3u, NH = NT - NL, heavy = (queue_units(qx) / NT) * NH;
     unsigned pidx, tile;
     if (t < heavy) {
       pidx = t / NH;
@@ -1091,7 +1107,19 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
       tile = NL - 1u - (t - heavy) % NL;
     }
     const unsigned pair = pidx * 8u + qx;
-    const unsigned n = pair / (unsigned)p.HQ, hq = pair - n * (unsigned)p.HQ;
+    unsigned n = pair / (unsigned)p.HQ;
+    const unsigned hq = pair - n * (unsigned)p.HQ;
+    unsigned bos = n * (unsigned)p.T, nats = n * (unsigned)p.TN;
+    len = p.T;
+    if (packed) {
+      const int off = seq_tab[RAGGED ? 3 : 0][lane & (STREAM_SEQS - 1)];
+      n = (unsigned)__popcll(__ballot(lane < p.n_seqs && (unsigned)off <= tile)) - 1u;
+      auto of = [&](const int f) __attribute__((always_inline)) { return __builtin_amdgcn_readfirstlane(seq_tab[RAGGED ? f : 0][n]); };
+      bos = (unsigned)of(0);
+      len = of(1);
+      nats = (unsigned)of(2);
+      tile -= (unsigned)of(3);
+    }
     const unsigned dstart = (tile * QTILE / (unsigned)Bs) * (unsigned)Bs;
     const unsigned hkv = hq / (unsigned)p.g_kv;
     first = (int)dstart;
@@ -1104,8 +1132,13 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
       out->hn = (int)(hq / (unsigned)p.g_n);
       out->dstart = (int)dstart;
       out->dblk = (int)(dstart / (unsigned)Bs);
+      if (RAGGED) {
+        out->bos = (int)bos;
+        out->len = len;
+        out->nats = (int)nats;
+      }
     }
-    return (int)((n * (unsigned)p.T + dstart) * (unsigned)p.HKV + hkv);
+    return (int)((bos + dstart) * (unsigned)p.HKV + hkv);
   };
 
   // ---- state of the tile in work; the kernel starts in a virtual tile (four chunks, nothing to compute) ------------
@@ -1113,15 +1146,16 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
   unsigned sp0 = 0;   // stream position of its chunk 0
   bool cur_real = false;
   int c_n = 0, c_hq = 0, c_tile = 0, c_hkv = 0, c_hn = 0, dstart = 0, dblk = 0;
+  int c_bos = 0, c_len = 1;   // (RAGGED; the virtual tile's: one row)
   bool req = false;  // this wave made a request in its last request step: that one may still be in flight at the next barrier
   if (wave == 4) {
-    int d0 = 0;
-    const int r0 = resolve_ticket(take_ticket(), &info[0], d0);
+    int d0 = 0, l0 = 0;
+    const int r0 = resolve_ticket(take_ticket(), &info[0], d0, l0);
     if (lane == 0) {
       info[0].diag_lo = info[0].diag_hi = 0u;
       info[0].count[0] = info[0].count[1] = info[0].count[2] = info[0].count[3] = 0;
     }
-    if (r0 >= 0 && lane < 4) rows[0][4 + lane] = own_entry(r0, d0, lane);   // the virtual tile has four chunks of its own
+    if (r0 >= 0 && lane < 4) rows[0][4 + lane] = own_entry(r0, d0, l0, lane);   // the virtual tile has four chunks of its own
   }
 
   bf16x8 QB[KSTEPS];
@@ -1209,12 +1243,12 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
     const int tile_start = c_tile * QTILE;
     const int n_diag = cur_real ? (tile_start + QTILE - dstart) >> 6 : 4;
     const int n_iters = n_diag + n_prior * per_blk;
-    const int bos = c_n * p.T;
+    const int bos = RAGGED ? c_bos : c_n * p.T, len = RAGGED ? c_len : p.T;
     const int q0 = tile_start + wave * QW;
     const int my_chunk = q0 >> 6, qloc0 = q0 & 63;
     const int my_blk = (int)((unsigned)q0 / (unsigned)Bs);
     // the tile after this one
-    const int n_bos = n_n * p.T;
+    const int n_bos = RAGGED ? rd(14) : n_n * p.T, n_len = RAGGED ? rd(15) : p.T, n_nats = RAGGED ? rd(16) : n_n * p.TN;
     const int n_tile_start = n_tile * QTILE;
 
     // queries of the next tile: raw into the query registers (issued during this tile's last chunk), scaled in place
@@ -1226,7 +1260,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
       // (no next tile: this tile's rows are read again, so that the loads and the waits of the scaling below are on
       // every path -- with the loads under a condition the compiler assumes them pending wherever the queries are used)
       const size_t qrow = n_valid ? (size_t)(n_bos + n_tile_start) : (size_t)(bos + tile_start);
-      const int qi = wave * QW + (ql & 31), qmax = RAGGED ? p.T - 1 - (n_valid ? n_tile_start : tile_start) : QTILE;
+      const int qi = wave * QW + (ql & 31), qmax = RAGGED ? (n_valid ? n_len - n_tile_start : len - tile_start) - 1 : QTILE;
       const bf16_t* qr = p.q + ((qrow + (RAGGED ? min(qi, qmax) : qi)) * p.HQ + (n_valid ? n_hq : c_hq)) * DK + 8 * (ql >> 5);
 #pragma unroll
       for (int s = 0; s < KSTEPS; ++s) QB[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(qr + 16 * s));
@@ -1251,7 +1285,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
       } else {
         act = jc < my_chunk && kblk < my_blk && typed;
       }
-      act_mask = __ballot(act && al < n_diag && (!RAGGED || q0 < p.T));
+      act_mask = __ballot(act && al < n_diag && (!RAGGED || q0 < len));
       const unsigned long long cm = __ballot(cz && al < n_diag);
       causal_it = cm ? __builtin_ctzll(cm) : -1;
     }
@@ -1263,7 +1297,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
     l_run = 0.f;
     thr = -INFINITY;
     f32x16 s0, s1;
-    auto is_active = [&](const int it) -> bool { return it < n_diag ? (act_mask >> it) & 1ull : it < n_iters && (!RAGGED || q0 < p.T); };
+    auto is_active = [&](const int it) -> bool { return it < n_diag ? (act_mask >> it) & 1ull : it < n_iters && (!RAGGED || q0 < len); };
     bool cur_active = act_mask & 1ull;
     if (cur_active) qk_phase<DK>(lds_k + (sp0 & 3) * KTILE + k_lane, QB, m_ref, s0, s1);
 
@@ -1296,7 +1330,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
         // K(it+4).  (As few instructions as possible: the other wave of the SIMD runs its matrix phases at raised
         // priority meanwhile, and every instruction of this one waits for an issue slot.)
         req = (unsigned)(it + 4 - rq_lo) < rq_span;
-        if (req) dma_k(__builtin_amdgcn_readfirstlane(row_ahead), sp0 + it + 4);
+        if (req) dma_k(__builtin_amdgcn_readfirstlane(row_ahead), sp0 + it + 4, it + 4 < n_iters ? len : n_len);
         cur_active = nxt_active;
       }
     } else {
@@ -1304,8 +1338,8 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
       // then of the prior attention blocks from the sorted list: a thread takes up to four list entries, which covers
       // the 1024 blocks the launcher admits), how many prior blocks there are, and the types of its own blocks.  Loads
       // are issued in the first chunk and used in the second, so that no wave waits for memory.
-      const int32_t* n_list = p.idx + ((size_t)(n_n * p.TN) * p.HN + n_hn) * 2;
-      const int jmax = min(n_dblk, p.TN);
+      const int32_t* n_list = p.idx + ((size_t)n_nats * p.HN + n_hn) * 2;
+      const int jmax = RAGGED ? n_dblk : min(n_dblk, p.TN);
       const int n_ndiag = (n_tile_start + QTILE - n_dstart) >> 6;
       int pe[4] = {0, 0, 0, 0}, p_nattn = 0;
       float p_type = 0.f;
@@ -1327,8 +1361,8 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
             p_nattn = p.nblk[((size_t)n_n * p.HN + n_hn) * 2];
             if (wave == 4) {
               const int blk = n_dblk + lane;
-              const bool in_range = lane < n_ndiag && (size_t)blk * Bs < (size_t)(n_tile_start + QTILE) && (!RAGGED || blk < p.TN);
-              const size_t ti = ((size_t)(n_n * p.TN + (in_range ? blk : n_dblk)) * p.HN + n_hn) * 2;
+              const bool in_range = lane < n_ndiag && (size_t)blk * Bs < (size_t)(n_tile_start + QTILE) && (!RAGGED || blk * Bs < n_len);
+              const size_t ti = ((size_t)(n_nats + (in_range ? blk : n_dblk)) * p.HN + n_hn) * 2;
               p_type = p.types_dtype == NATSL_F32 ? reinterpret_cast<const float*>(p.types)[ti]
                                                   : bf16_to_f32(reinterpret_cast<const bf16_t*>(p.types)[ti]);
             }
@@ -1345,11 +1379,11 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
                 for (int sub = 0; sub < per_blk; ++sub)
                   rows[a ^ 1][n_ndiag + j * per_blk + sub] = (n_bos + pe[m] * Bs + 64 * sub) * p.HKV + n_hkv;
             }
-            if (lt < n_ndiag) rows[a ^ 1][lt] = own_entry((n_bos + n_dstart) * p.HKV + n_hkv, n_dstart, lt);
+            if (lt < n_ndiag) rows[a ^ 1][lt] = own_entry((n_bos + n_dstart) * p.HKV + n_hkv, n_dstart, n_len, lt);
             if (lane == 0) info[a ^ 1].count[gw] = cnt;
             if (wave == 4) {
               const int blk = n_dblk + lane;
-              const bool in_range = lane < n_ndiag && (size_t)blk * Bs < (size_t)(n_tile_start + QTILE) && (!RAGGED || blk < p.TN);
+              const bool in_range = lane < n_ndiag && (size_t)blk * Bs < (size_t)(n_tile_start + QTILE) && (!RAGGED || blk * Bs < n_len);
               const unsigned long long d = __ballot(in_range && rintf(p_type) == 1.0f);
               if (lane == 0) {
                 info[a ^ 1].diag_lo = (unsigned)d;
@@ -1361,11 +1395,11 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
             // the tile after the next: ticket asked for in the last chunk but one, turned into a tile in the last
             if (it == n_iters - 2 && cq < STREAM_QUEUES && lane == 0) t_ahead = atomicAdd(&queue[(xcc + (unsigned)cq) & 7u], 1u);
             if (last) {
-              int d0 = 0;
-              const int r0 = resolve_ticket(__builtin_amdgcn_readfirstlane(t_ahead), &info[a ^ 1], d0);
+              int d0 = 0, l0 = 0;
+              const int r0 = resolve_ticket(__builtin_amdgcn_readfirstlane(t_ahead), &info[a ^ 1], d0, l0);
               // the next tile's table ends with the first four chunks of the tile after it
               const int nn_iters = n_ndiag + (info[a ^ 1].count[0] + info[a ^ 1].count[1] + info[a ^ 1].count[2] + info[a ^ 1].count[3]) * per_blk;
-              if (r0 >= 0 && lane < 4) rows[a ^ 1][nn_iters + lane] = own_entry(r0, d0, lane);
+              if (r0 >= 0 && lane < 4) rows[a ^ 1][nn_iters + lane] = own_entry(r0, d0, l0, lane);
             }
           }
           ev_it = it == 0 ? 1 : (it < n_iters - 2 ? n_iters - 2 : it + 1);
@@ -1387,7 +1421,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
         if (nxt_active) qk_phase<DK>(lds_k + ((sp0 + it + 1) & 3) * KTILE + k_lane, QB, m_ref, s0, s1);
         __builtin_amdgcn_s_setprio(0);
         req = (unsigned)(it + 3 - rq_lo) < rq_span;
-        if (req) dma_v(__builtin_amdgcn_readfirstlane(row_ahead), sp0 + it + 3);
+        if (req) dma_v(__builtin_amdgcn_readfirstlane(row_ahead), sp0 + it + 3, it + 3 < n_iters ? len : n_len);
         cur_active = nxt_active;
       }
     }
@@ -1395,7 +1429,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
     // ---- end of the tile: the next tile's queries, output (early waves now, late waves after the next hand-over barrier)
     {
       const size_t row0 = (size_t)(bos + q0) * p.HQ + c_hq;
-      const int n_rows = RAGGED ? p.T - q0 : QW;
+      const int n_rows = RAGGED ? len - q0 : QW;
       const unsigned stage = lds_o + gw * (32 * DV);
       load_next_q();   // (ahead of the stores: what waits for the queries later does not wait for the stores then)
       // What the first barrier of the next tile needs, K(2) and V(1) of that tile, has landed: newer than those are one request
@@ -1422,6 +1456,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
         pend_rows = n_rows;
       }
     }
+    if (RAGGED) { c_bos = n_bos; c_len = n_len; }
     c_n = n_n; c_hq = n_hq; c_tile = n_tile; c_hkv = n_hkv; c_hn = n_hn; dstart = n_dstart; dblk = n_dblk;
     cur_real = true;
     sp0 += (unsigned)n_iters;
@@ -1508,14 +1543,15 @@ static int launch_softmax_stream(const SoftmaxParams& p, const StreamDevice* d, 
   return check_launch("natsl_softmax_sparse_fwd");
 }
 
-// Which kernel natsl_softmax_sparse_fwd runs for a problem: the persistent one for unpacked input of at least two
-// 256-query tiles per compute unit (its per-tile saving needs a tile to follow); else one workgroup per tile, of 256
+// Which kernel natsl_softmax_sparse_fwd runs for a problem: the persistent one for at least two 256-query tiles per compute unit (its
+// per-tile saving needs a tile to follow) and what its tables hold; else one workgroup per tile, of 256
 // queries on 8 waves once there is at least one such tile per compute unit (measured: from there on that shape is the
 // faster one; below, 128-query tiles fill more compute units).
-static int softmax_variant(int B, int T, int HQ, int HKV, int block, bool packed, bool allow_persistent, const StreamDevice** sd, int* rc) {
+static int softmax_variant(int B, int T, int HQ, int HKV, int block, bool packed, bool allow_persistent, int n_seqs, const StreamDevice** sd,
+                           int* rc) {
   *sd = nullptr;
   *rc = NATSL_OK;
-  if (allow_persistent && !packed && T <= 65536 && block <= 2048 && (long long)B * T * HKV < (1ll << 31)) {
+  if (allow_persistent && (!packed || n_seqs <= STREAM_SEQS) && T <= 65536 && block <= 2048 && (long long)B * T * HKV < (1ll << 31)) {
     const StreamDevice* d = stream_device(rc);
     if (!d) return -1;
     if ((long long)B * HQ * cdiv(T, 256) >= 2ll * d->cus) {
@@ -1560,12 +1596,12 @@ static int softmax_fwd(const void* q, const void* k, const void* v, void* o, flo
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const StreamDevice* sd = nullptr;
   int rc;
-  const int variant = softmax_variant(B, T, HQ, HKV, block, seqs != nullptr, allow_persistent, &sd, &rc);
+  const int variant = softmax_variant(B, T, HQ, HKV, block, seqs != nullptr, allow_persistent, n_seqs, &sd, &rc);
   if (variant < 0) return rc;
   p.variant = variant == NATSL_SOFTMAX_TILE_128 ? 4 : 8;
 #define NATSL_SM(KK, VV)                                              \
   if (K == KK && V == VV) {                                           \
-    if (sd) return T % 256 ? launch_softmax_stream<KK, VV, true>(p, sd, s) : launch_softmax_stream<KK, VV, false>(p, sd, s); \
+    if (sd) return seqs || T % 256 ? launch_softmax_stream<KK, VV, true>(p, sd, s) : launch_softmax_stream<KK, VV, false>(p, sd, s); \
     return p.variant == 8 ? launch_softmax<KK, VV, 8>(p, s) : launch_softmax<KK, VV, 4>(p, s); \
   }
   NATSL_SM(128, 128)
@@ -1599,6 +1635,6 @@ extern "C" int natsl_softmax_sparse_fwd_per_tile(const void* q, const void* k, c
 extern "C" int natsl_softmax_fwd_variant(int B, int T, int HQ, int HKV, int block, int packed) {
   const StreamDevice* sd = nullptr;
   int rc;
-  const int variant = softmax_variant(B, T, HQ, HKV, block, packed != 0, true, &sd, &rc);
+  const int variant = softmax_variant(B, T, HQ, HKV, block, packed != 0, true, packed, &sd, &rc);
   return variant < 0 ? rc : variant;
 }

@@ -100,6 +100,44 @@ def test_persistent_kernel_with_a_cut_last_tile(T, K, V, H, block, same_block):
             assert_close(y[[0, 1, 3], whole:].float(), x[[0, 1, 3], whole:].float(), "last tile")
 
 
+@pytest.mark.parametrize("K,V,H,block,same_block", [(128, 128, 32, 64, True), (64, 128, 8, 256, True), (128, 64, 16, 64, False)])
+@pytest.mark.parametrize("lens", [[300, 64, 1, 1000, 257, 511, 2048, 63], [4096, 65], [65] * 64, [65] * 65])
+def test_persistent_kernel_on_packed_sequences(lens, K, V, H, block, same_block):
+    """Packed sequences, up to as many as the kernel's table holds and one more (which goes to the per-tile kernel), against that kernel as
+    above; one sequence holds NaNs."""
+    from neuralattentionsearchlinear_amd import _capi, nats_util
+    HQ, HN, dev = 32, 8, torch.device('cuda:0')
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    T, bad = cu[-1], 1
+    seqs = nats_util.pack_sequences(cu, None, block, dev)
+    q, k, v = make_qkv(1, T, H, K, V, 41, HQ=HQ)
+    ty = make_types(1, seqs.total_blocks, HN, 0.4, 42, torch.bfloat16)
+    k[0, cu[bad]], v[0, cu[bad]] = float('nan'), float('inf')
+    qd, kd, vd, tyd = q.to(dev), k.to(dev), v.to(dev), ty.to(dev)
+    r = nats_util.route(tyd, T, block, seqs)
+    L, out = _capi.lib(), []
+    assert L.natsl_softmax_fwd_variant(1, T, HQ, H, block, len(lens)) == (2 if len(lens) <= 64 else 1)
+    for fn in (L.natsl_softmax_sparse_fwd_per_tile, L.natsl_softmax_sparse_fwd):
+        o, lse = torch.empty(1, T, HQ, V, dtype=torch.bfloat16, device=dev), torch.empty(1, T, HQ, device=dev)
+        rc = fn(_capi.ptr(qd), _capi.ptr(kd), _capi.ptr(vd), _capi.ptr(o), _capi.ptr(lse), _capi.ptr(tyd), _capi.dtype_code(tyd.dtype),
+                _capi.ptr(r['nats_block_indices']), _capi.ptr(r['n_nats_blocks']), 1, T, HQ, H, HN, K, V, ty.shape[1], block, float(K ** -0.5),
+                int(same_block), _capi.dtype_code(qd.dtype), _capi.ptr(seqs.table), seqs.n_seqs, seqs.total_qtiles, _capi.stream_ptr(dev))
+        _capi.check(rc, "softmax")
+        out.append((o[0], lse[0]))
+    torch.cuda.synchronize()
+    for i, (a, b) in enumerate(zip(cu[:-1], cu[1:])):
+        whole = b if (b - a) % 64 == 0 else a + (b - a) // 256 * 256
+        for x, y in zip(*out):
+            assert torch.equal(x[a:b].isnan(), y[a:b].isnan())
+            if i == bad:
+                continue
+            assert bool(torch.isfinite(y[a:b]).all()) and torch.equal(x[a:whole], y[a:whole])
+            if whole < b:
+                assert_close(y[whole:b].float(), x[whole:b].float(), f"sequence {i}")
+
+
 def test_persistent_kernel_queues_across_launches_and_streams():
     """The ticket counters are shared device state: one slot per launch in rotation, zeroed on the launch's stream right
     before it."""

@@ -444,11 +444,13 @@ NATSL_DEVICE void dma16(const void* base, const unsigned voff, const unsigned ld
 // segments 0..3 of an aligned group per 16 lanes, half a slot each) is served 32 lanes at a time: no more than two of rows 0..7
 // may share the bits above the lowest two.  Measured, ns an instruction and CU: 1.9 and 1.7, as without any conflict; with
 // (r & 3) << 2 | r >> 2 for DK = 128 the operand read takes 3.4, with (r >> 1) & 7 for the others the transposing read does.  The scan
-// of B8 T8192 H16 d128 with it: 333 -> 326 us.
-template <int DK>
+// of B8 T8192 H16 d128 with it: 333 -> 326 us.  A single compute wave does not notice the operand read's conflicts: with DK = 128 it keeps
+// the swizzle without them in mind (B1 T12000 H4: 231 us against 232).  Of the swizzles that meet all this for DK = 64, one that mixes the
+// row's low bits in is the better one there (168 us; 169 with (r >> 1) & 7, 173 without the mix).
+template <int DK, int NW>
 NATSL_DEVICE int kq_swizzle(const int r) {
-  if constexpr (DK == 128) return ((r & 3) << 2) | (-(r >> 2) & 3);  // 16 segments per row, a row = one bank period
-  return (((r >> 1) & 1) << 2) | (-(r >> 2) & 3);                    // 8 or 24 segments per row: low three bits only, rows in pairs
+  if constexpr (DK == 128) return ((r & 3) << 2) | ((NW == 1 ? r >> 2 : -(r >> 2) ^ r) & 3);   // 16 segments per row, a row = one bank period
+  return (((r >> 1) & 1) << 2) | (-(r >> 2) & 2) | ((-(r >> 2) ^ (r >> 1)) & 1);              // 8 or 24 per row: low three bits only, rows in pairs
 }
 
 typedef __attribute__((address_space(3))) const bf16x8* lds_b128_t;
@@ -553,7 +555,7 @@ __global__ NATSL_SCAN_ATTR(DK, NW + NF) void linear_scan_kernel(const LinearPara
     // (operand addresses of the k / q tiles and of a row of the scale vectors, as the compute waves use them below)
     unsigned a_kq[KS];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) a_kq[s] = (unsigned)(i16 * L::KROW) + 16u * (unsigned)((4 * s + g4) ^ kq_swizzle<DK>(i16));
+    for (int s = 0; s < KS; ++s) a_kq[s] = (unsigned)(i16 * L::KROW) + 16u * (unsigned)((4 * s + g4) ^ kq_swizzle<DK, NW>(i16));
     const unsigned a_sc = 16u * g4;
     const bool l2n = (p.flags & NATSL_QK_L2NORM) != 0;
     const float log2_scale_m = __builtin_amdgcn_logf(p.scale);
@@ -574,7 +576,7 @@ __global__ NATSL_SCAN_ATTR(DK, NW + NF) void linear_scan_kernel(const LinearPara
     constexpr int KQ_PIECES = L::KB / 1024, V_PIECES = L::VB / 1024;
     auto kq_src = [&](const int u, const int nvalid) -> unsigned {
       const int byte = 1024 * u + 16 * lane, row = byte / L::KROW, pos = (byte % L::KROW) / 16;
-      return (unsigned)((size_t)min(row, nvalid - 1) * qk_pitch) + 16u * (unsigned)(pos ^ kq_swizzle<DK>(row));
+      return (unsigned)((size_t)min(row, nvalid - 1) * qk_pitch) + 16u * (unsigned)(pos ^ kq_swizzle<DK, NW>(row));
     };
     auto v_src = [&](const int u, const int nvalid) -> unsigned {
       const int byte = 1024 * u + 16 * lane, row = byte / L::VROW, pos = (byte % L::VROW) / 16;
@@ -823,7 +825,7 @@ __global__ NATSL_SCAN_ATTR(DK, NW + NF) void linear_scan_kernel(const LinearPara
   // k / q as A operand (token tile t, k-step s): row 16 t + i16, segment 4 s + g4 (swizzled); t goes into the offset field
   unsigned a_kq[KS];
 #pragma unroll
-  for (int s = 0; s < KS; ++s) a_kq[s] = (unsigned)(i16 * L::KROW) + 16u * (unsigned)((4 * s + g4) ^ kq_swizzle<DK>(i16));
+  for (int s = 0; s < KS; ++s) a_kq[s] = (unsigned)(i16 * L::KROW) + 16u * (unsigned)((4 * s + g4) ^ kq_swizzle<DK, NW>(i16));
   // k^T as A operand (state tile m, token k-step s2, read rd): lane i16 addresses token 32 s2 + 16 rd + 4 g4 + i16 / 4,
   // the four K rows 32 (m / 2) + 8 (i16 % 4) + 4 (m % 2) ..: segment 4 (m / 2) + i16 % 4, half m % 2
   unsigned a_kt[KT / 2];
@@ -831,7 +833,7 @@ __global__ NATSL_SCAN_ATTR(DK, NW + NF) void linear_scan_kernel(const LinearPara
     const int tok = 4 * g4 + (i16 >> 2);
 #pragma unroll
     for (int mh = 0; mh < KT / 2; ++mh)
-      a_kt[mh] = (unsigned)(tok * L::KROW) + 16u * (unsigned)((4 * mh + (i16 & 3)) ^ kq_swizzle<DK>(tok));
+      a_kt[mh] = (unsigned)(tok * L::KROW) + 16u * (unsigned)((4 * mh + (i16 & 3)) ^ kq_swizzle<DK, NW>(tok));
   }
   // v through the transposing read (token tile t): lane i16 addresses token 16 t + 4 g4 + i16 / 4, columns 16 wave + 4 (i16 % 4)..
   unsigned a_v;

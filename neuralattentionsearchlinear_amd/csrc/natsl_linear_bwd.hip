@@ -232,12 +232,14 @@ NATSL_DEVICE void dma16(const void* base, const unsigned voff, const unsigned ld
 }
 
 // Swizzle of the raw k / q tiles (row-major, unpadded rows of DK bf16; the forward scan's): 16-byte segment s of row r sits at
-// s ^ kq_swz(r), with which neither the row reads nor the transposing reads meet in a bank (see kq_swizzle there).  K = 192, B2 T3000
-// H6 V384: 219.6 -> 201.9 us against (r >> 1) & 7, whose transposing reads met four times.
+// s ^ kq_swz(r), with which neither the row reads nor the transposing reads meet in a bank more than they have to (see kq_swizzle there).
+// K = 192, B2 T3000 H6 V384: 219.6 -> 202 us against (r >> 1) & 7, whose transposing reads meet four times; that one stays for K = 64, where
+// one or two compute waves do not notice (B1 T12000 H4: 368 us against 371).
 template <int DK>
 NATSL_DEVICE int kq_swz(const int r) {
-  if constexpr (DK == 128) return ((r & 3) << 2) | (-(r >> 2) & 3);
-  return (((r >> 1) & 1) << 2) | (-(r >> 2) & 3);
+  if constexpr (DK == 128) return ((r & 3) << 2) | ((-(r >> 2) ^ r) & 3);
+  if constexpr (DK == 64) return (r >> 1) & 7;
+  return (((r >> 1) & 1) << 2) | (-(r >> 2) & 2) | ((-(r >> 2) ^ (r >> 1)) & 1);
 }
 // the 64-column dO / v_new tiles (rows of 128 bytes): rows two apart share banks
 NATSL_DEVICE int v_swz(const int r) { return 2 * ((r >> 1) & 1); }

@@ -436,7 +436,8 @@ NATSL_DEVICE void dkdv_take_unit(const SoftmaxBwdParams& p, const bool packed, c
 // chain of LDS reads, exponentials and barrier runs under the others' matrix instructions, and so does what a unit costs besides its
 // steps (most units are a single step where a quarter of the blocks is attention).  Against the form with two roles below, which is
 // one workgroup of eight waves and 70 % more vector instructions a quarter: K 128, V 64, B4 T8192 H32, block 256, 25 % attention 1610
-// -> 1210 us; K 64, V 128, B8 T4096 H12, 50 % 600 -> 415; K = V = 64, B4 T4096 H32 330 -> 270.  What is left is the chain of a step
+// -> 1190 us; K 64, V 128, B8 T4096 H12, 50 % 600 -> 397; K = V = 64, B4 T4096 H32 330 -> 257 (415 and 270 of the last two without the
+// transposed operands read ahead).  What is left is the chain of a step
 // (about 2100 cycles a CU against 768 of matrix time): without the requests of the query tiles it is 15 % shorter, and fewer vector or
 // scalar instructions change it by 1 - 2 %.  Three workgroups per CU at K = V = 64 spill 36 registers a lane and take 390 us.
 constexpr int DKDV_WHOLE_WGS = 2;   // workgroups per CU (registers and LDS)

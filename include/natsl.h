@@ -103,8 +103,8 @@ int natsl_route(const void* types, int types_dtype, int B, int TN, int HN, int T
  * log2 units; rows that see no key give o = 0, lse = 0.
  * Replaces parallel_attn_nats_fwd (src/nats/ops/attns/attns.py:1421-1531, kernel :62-353) as
  * called at src/nats/ops/mixed_ops/mixed_attn_gdn.py:111-117.
- * K, V in {64, 128}.  Unpacked input of whole 256-query tiles, at least two per compute unit (T % 256 == 0,
- * T <= 65536, block <= 2048), runs as a persistent kernel whose work queues are ticket counters in device
+ * K, V in {64, 128}.  Problems with tiles enough for every compute unit (natsl_softmax_fwd_variant says which;
+ * T <= 65536, block <= 2048, at most 64 packed sequences) run as a persistent kernel whose work queues are ticket counters in device
  * memory owned by the library: 64 slots used in rotation, the launch's slot zeroed by a small fill kernel
  * enqueued on `stream` right before it (both kernels can be captured into a HIP graph).  Launches may overlap
  * across streams as long as fewer than 64 of them are in flight on one GPU; a captured launch keeps the slot it
@@ -116,7 +116,7 @@ int natsl_softmax_sparse_fwd(const void* q, const void* k, const void* v, void* 
                              const natsl_seq_row* seqs, int n_seqs, int total_units, natsl_stream_t stream);
 
 /* The same operation, always as one workgroup per query tile (what natsl_softmax_sparse_fwd itself runs for small
- * problems and for more than 64 packed sequences): for callers that want no library-owned device state in the launch, and the regression
+ * problems, short sequences and more than 64 packed sequences): for callers that want no library-owned device state in the launch, and the regression
  * check of the persistent kernel.  The same results bit for bit, except for the queries of a sequence's last 256-row
  * tile where its length is no multiple of 64: those differ by the rounding of the probabilities in the row sums.
  * Same reference interface as natsl_softmax_sparse_fwd. */

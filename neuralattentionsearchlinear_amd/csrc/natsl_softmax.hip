@@ -1543,10 +1543,17 @@ static int launch_softmax_stream(const SoftmaxParams& p, const StreamDevice* d, 
   return check_launch("natsl_softmax_sparse_fwd");
 }
 
-// Which kernel natsl_softmax_sparse_fwd runs for a problem: the persistent one for at least two 256-query tiles per compute unit (its
-// per-tile saving needs a tile to follow) and what its tables hold; else one workgroup per tile, of 256
-// queries on 8 waves once there is at least one such tile per compute unit (measured: from there on that shape is the
-// faster one; below, 128-query tiles fill more compute units).
+// Which kernel natsl_softmax_sparse_fwd runs for a problem.  The persistent one needs tiles to follow each other on its one workgroup
+// per CU: below that, two workgroups of a tile each per CU hide each other's ends and even out better.  Time per tile kernel / persistent
+// kernel, heads 64 and 128, 5 - 50 % attention, lengths of 333 .. 8256: 0.60 - 1.0 at two tiles per CU, 0.63 - 1.14 at four, 0.74 - 1.22
+// at six, 0.81 - 1.25 at eight, 0.94 - 1.3 at 16; the low ends are few attention blocks and K = V = 64, the high ends half attention and
+// lengths that cut a chunk.  So it takes eight tiles' worth of queries per CU.  Where sequences are shorter than a tile, what it does for
+// the missing queries costs more than it saves (100 queries: 0.42 - 0.8 up to 16 tiles per CU).  Whole tiles of at least 2048 queries
+// take it from two tiles per CU (0.69 - 1.02 there, 0.78 - 1.06 at four): its tests hold it at these small problems.
+// Long sequences that end inside a chunk take it from three: their last tile, the longest, goes the per-tile kernel's slow way (8191
+// queries at three tiles per CU: 1.04 - 1.12 with 25 % attention or more, 0.73 - 0.93 with 5 %, where there is little to lose; 4099: 0.69 - 0.87).
+// Of the others, one workgroup per tile, of 256 queries on 8 waves once there is at least one such tile per compute unit (measured:
+// from there on that shape is the faster one; below, 128-query tiles fill more compute units).
 static int softmax_variant(int B, int T, int HQ, int HKV, int block, bool packed, bool allow_persistent, int n_seqs, const StreamDevice** sd,
                            int* rc) {
   *sd = nullptr;
@@ -1554,7 +1561,10 @@ static int softmax_variant(int B, int T, int HQ, int HKV, int block, bool packed
   if (allow_persistent && (!packed || n_seqs <= STREAM_SEQS) && T <= 65536 && block <= 2048 && (long long)B * T * HKV < (1ll << 31)) {
     const StreamDevice* d = stream_device(rc);
     if (!d) return -1;
-    if ((long long)B * HQ * cdiv(T, 256) >= 2ll * d->cus) {
+    const long long tiles = (long long)B * HQ * T / 256;   // whole tiles' worth of queries
+    const bool whole = !packed && T % 256 == 0;
+    const bool cut = !packed && T % 64 && T >= 6144;
+    if (tiles >= (whole && T >= 2048 ? 2ll : cut ? 3ll : 8ll) * d->cus && T / (packed ? n_seqs : 1) >= 256) {
       *sd = d;
       return NATSL_SOFTMAX_PERSISTENT;
     }

@@ -8,9 +8,9 @@
 //                  block, and every later chunk when the block is typed attention), for every query head of the group:
 //                  S = Q K^T, dP = dO V^T, dV^T += dO^T P, dK^T += Q^T dS, dnats += sum dS over later blocks (attns.py:719-983)
 //                  The query tiles (Q, dO, lse, delta) arrive by DMA in a ring of three LDS slots, two steps ahead.
-//                  Persistent workgroups take units from per-XCD work queues.  K + V <= 192 (dkdv_whole_kernel): two
-//                  workgroups of four waves per CU, a wave forms everything of its (32 keys) x (32 queries) quarter.  K = V =
-//                  128: one of eight waves in two roles; four form S, P and dV, four form dP, dS and dK of the same
+//                  Persistent workgroups take units from per-XCD work queues.  K + V <= 192 and at
+//                  least ten chunks per CU (dkdv_whole_kernel): two workgroups of four waves per CU, a wave forms everything
+//                  of its (32 keys) x (32 queries) quarter.  Else one of eight waves in two roles; four form S, P and dV, four form dP, dS and dK of the same
 //                  quarters, and P passes between the two in fp32 through LDS.
 //
 // Layouts follow the forward kernel: the stationary operand of a workgroup (Q, dO there; K, V here) sits in registers
@@ -430,7 +430,7 @@ NATSL_DEVICE void dkdv_take_unit(const SoftmaxBwdParams& p, const bool packed, c
 }
 
 // ---------------------------------------------------------------------------------------------
-// dk/dv for K + V <= 192: a wave holds both stationary operands and both accumulators of its 32 keys (K 128, V 64: 144 registers), so
+// dk/dv for K + V <= 192 and many chunks: a wave holds both stationary operands and both accumulators of its 32 keys (K 128, V 64: 144 registers), so
 // that it forms S, P, dP and dS of a 32 x 32 quarter and all four products by itself: nothing passes between waves inside a step.
 // Workgroups of four waves (2 key halves x 2 query halves), two per CU: each has its own ring and its own barrier, so one's
 // chain of LDS reads, exponentials and barrier runs under the others' matrix instructions, and so does what a unit costs besides its
@@ -441,6 +441,10 @@ NATSL_DEVICE void dkdv_take_unit(const SoftmaxBwdParams& p, const bool packed, c
 // (about 2100 cycles a CU against 768 of matrix time): without the requests of the query tiles it is 15 % shorter, and fewer vector or
 // scalar instructions change it by 1 - 2 %.  Three workgroups per CU at K = V = 64 spill 36 registers a lane and take 390 us.
 constexpr int DKDV_WHOLE_WGS = 2;   // workgroups per CU (registers and LDS)
+// Chunks per CU from which this kernel runs: with fewer, each of its workgroups has a handful of units and takes twice as long over one
+// as the eight waves of the form below.  Whole backward (delta, dQ, dK/dV) of the other form against this one, T 192 .. 8256, 10 % and
+// 40 % attention: 0.83 - 0.95 of its time at seven or eight chunks per CU and short sequences, 0.97 - 1.1 at ten, 1.15 - 1.35 at 32.
+constexpr int DKDV_WHOLE_CHUNKS = 10;
 
 template <int DK, int DV>
 struct DkdvWholeLds {
@@ -1226,15 +1230,17 @@ static int launch_bwd(const SoftmaxBwdParams& p, hipStream_t stream) {
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(threads), lds, stream, p);
     return NATSL_OK;
   };
-  // (192: both operands, both accumulators and a quarter's scores fit the 256 registers that two waves a SIMD leave)
   static std::atomic<unsigned long long> reserved{0};
+  auto roles = [&] { return dkdv(dkdv_kernel<DK, DV>, reserved, DkdvLds<DK, DV>::TOTAL, 512, 1); };   // the ring of three query tiles and the exchange buffers
   int rc;
+  // (192: both operands, both accumulators and a quarter's scores fit the 256 registers that two waves a SIMD leave)
   if constexpr (DK + DV <= 192) {
-    static std::atomic<unsigned long long> reserved_invalid{0};
+    static std::atomic<unsigned long long> reserved_whole{0}, reserved_invalid{0};
     constexpr size_t lds = DkdvWholeLds<DK, DV>::TOTAL;
-    rc = p.dnats_invalid ? dkdv(dkdv_whole_kernel<DK, DV, true>, reserved_invalid, lds, 256, DKDV_WHOLE_WGS)
-                         : dkdv(dkdv_whole_kernel<DK, DV, false>, reserved, lds, 256, DKDV_WHOLE_WGS);
-  } else rc = dkdv(dkdv_kernel<DK, DV>, reserved, DkdvLds<DK, DV>::TOTAL, 512, 1);   // the ring of three query tiles and the exchange buffers
+    if (units < (long long)DKDV_WHOLE_CHUNKS * cu_count()) rc = roles();
+    else if (p.dnats_invalid) rc = dkdv(dkdv_whole_kernel<DK, DV, true>, reserved_invalid, lds, 256, DKDV_WHOLE_WGS);
+    else rc = dkdv(dkdv_whole_kernel<DK, DV, false>, reserved_whole, lds, 256, DKDV_WHOLE_WGS);
+  } else rc = roles();
   if (rc != NATSL_OK) return rc;
   return check_launch("natsl_softmax_sparse_bwd");
 }

@@ -17,7 +17,7 @@ def _close(a, b, what):
     assert rl <= 5e-3 and ma <= 2e-2 * max(top, 1.0), f"{what}: rel-L2 {rl:.3e}, max-abs {ma:.3e} (largest reference value {top:.3e})"
 
 
-def _run(B, T, HQ, H, HN, K, V, block, p_attn, same_block, seed, through_autograd=False, dnats_invalid=False):
+def _run(B, T, HQ, H, HN, K, V, block, p_attn, same_block, seed, through_autograd=False, dnats_invalid=False, copies=1):
     from neuralattentionsearchlinear_amd import nats_util
     from neuralattentionsearchlinear_amd.attns import parallel_attn_nats_bwd, parallel_attn_nats_fwd, parallel_nats_attn
     q, k, v = make_qkv(B, T, H, K, V, seed, HQ=HQ)
@@ -26,7 +26,7 @@ def _run(B, T, HQ, H, HN, K, V, block, p_attn, same_block, seed, through_autogra
     scale = K ** -0.5
     dq_r, dk_r, dv_r, dn_r, dn_mag = sb.softmax_branch_bwd(q, k, v, ty, do, scale, block, same_block, with_magnitude=True,
                                                            dnats_invalid=dnats_invalid)
-    qd, kd, vd, dod, tyd = (t.to(DEV) for t in (q, k, v, do, ty))
+    qd, kd, vd, dod, tyd = (t.to(DEV).repeat(copies, *[1] * (t.dim() - 1)) for t in (q, k, v, do, ty))
     r = nats_util.route(tyd, T, block)
     if through_autograd:
         qd, kd, vd = (t.requires_grad_() for t in (qd, kd, vd))
@@ -44,6 +44,9 @@ def _run(B, T, HQ, H, HN, K, V, block, p_attn, same_block, seed, through_autogra
                                                    scale=scale, NAtS_block_size=block, compute_incomplete_chunk_scores=same_block,
                                                    compute_dnats_for_invalid_blocks_attn=dnats_invalid)
     torch.cuda.synchronize()
+    if copies > 1:
+        assert torch.equal(dk, dk[-B:].repeat(copies, 1, 1, 1)) and torch.equal(dv, dv[-B:].repeat(copies, 1, 1, 1))
+        dq, dk, dv, dn = (t[-B:] for t in (dq, dk, dv, dn))
     _close(dq.float(), dq_r, "dq")
     _close(dk.float(), dk_r, "dk")
     _close(dv.float(), dv_r, "dv")
@@ -98,12 +101,18 @@ def test_softmax_bwd_many_pairs_and_long_walks():
 @pytest.mark.parametrize("T,HQ,H,block,dnats_invalid", [(2, 2, 2, 64, False), (63, 2, 2, 64, True), (65, 4, 2, 64, False),
                                                         (191, 2, 2, 128, True), (256, 4, 4, 64, False), (449, 4, 1, 64, True)])
 @pytest.mark.parametrize("K,V", [(64, 64), (64, 128), (128, 64)])
-def test_softmax_bwd_whole_quarters(K, V, T, HQ, H, block, dnats_invalid):
-    """K + V <= 192: the dk/dv kernel whose waves form all four products.  Walks of one, two and three or more tiles (its ring holds
+@pytest.mark.parametrize("chunks", [0, 9, 10])
+def test_softmax_bwd_whole_quarters(chunks, K, V, T, HQ, H, block, dnats_invalid):
+    """K + V <= 192: the two dk/dv kernels, on copies of a sequence that make so many chunks per CU (from ten on it is the one whose
+    waves form all four products).  Walks of one, two and three or more tiles (its ring holds
     three), a ragged tile as the first of a walk, a block's own chunks behind the later ones, grouped query heads.  (Two tokens are the least: with one, dq and dk are exactly 0 and
     what the kernel leaves is the fp32 rounding of dP - delta, 2e-7 measured, which has no relative error to speak of.)"""
+    units, cus = H * -(-T // 64), torch.cuda.get_device_properties(0).multi_processor_count
+    copies = max(1, -(-chunks * cus // units))
+    if chunks == 9:
+        copies = (10 * cus - 1) // units                 # the most that are below ten
     for same_block in (True, False):
-        _run(1, T, HQ, H, H, K, V, block, 0.6, same_block, seed=40, dnats_invalid=dnats_invalid)
+        _run(1, T, HQ, H, H, K, V, block, 0.6, same_block, seed=40, dnats_invalid=dnats_invalid, copies=copies)
 
 
 def test_softmax_bwd_repeatable_and_workspace_reuse():

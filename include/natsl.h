@@ -7,8 +7,8 @@
  * (src/nats/ops/mixed_ops/mixed_attn_gdn.py:49-50 makes its inputs contiguous).  Nothing here
  * allocates or synchronises with the host; work is enqueued on `stream`.  Two pieces of device
  * memory belong to the library and are shared by all calls on one GPU: the ticket counters of
- * natsl_softmax_sparse_fwd's persistent kernel (64 slots used in rotation, each zeroed on the
- * caller's stream ahead of the launch that uses it) and the scratch of
+ * natsl_softmax_sparse_fwd's persistent kernel on whole tiles (64 slots used in rotation, each zeroed
+ * on the caller's stream ahead of the launch that uses it) and the scratch of
  * natsl_attn_masked_fwd_static; their comments say what that means for overlapping calls.
  * Each function returns NATSL_OK or a negative natsl_status; natsl_last_error() gives the
  * message for the calling thread.
@@ -104,11 +104,12 @@ int natsl_route(const void* types, int types_dtype, int B, int TN, int HN, int T
  * Replaces parallel_attn_nats_fwd (src/nats/ops/attns/attns.py:1421-1531, kernel :62-353) as
  * called at src/nats/ops/mixed_ops/mixed_attn_gdn.py:111-117.
  * K, V in {64, 128}.  Problems with tiles enough for every compute unit (natsl_softmax_fwd_variant says which;
- * T <= 65536, block <= 2048, at most 64 packed sequences) run as a persistent kernel whose work queues are ticket counters in device
- * memory owned by the library: 64 slots used in rotation, the launch's slot zeroed by a small fill kernel
- * enqueued on `stream` right before it (both kernels can be captured into a HIP graph).  Launches may overlap
- * across streams as long as fewer than 64 of them are in flight on one GPU; a captured launch keeps the slot it
- * drew at capture, so replay it on the stream that also carries the eager launches. */
+ * T <= 65536, block <= 2048, at most 64 packed sequences) run as a persistent kernel.  On batches with T a multiple of 256 its work
+ * queues are ticket counters in device memory owned by the library: 64 slots used in rotation, the launch's slot zeroed by a small
+ * fill kernel enqueued on `stream` right before it (both kernels can be captured into a HIP graph).  Such launches may overlap across
+ * streams as long as fewer than 64 of them are in flight on one GPU; a captured one keeps the slot it drew at capture, so replay it
+ * on the stream that also carries the eager launches.  Packed sequences and other lengths use no device memory but what the
+ * arguments name, and may overlap and be replayed in any way. */
 int natsl_softmax_sparse_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
                              const void* types, int types_dtype, const int32_t* nats_block_indices,
                              const int32_t* n_nats_blocks, int B, int T, int HQ, int HKV, int HN, int K,
@@ -456,7 +457,10 @@ int natsl_wgrad(const natsl_wgrad_seg* segs, int n_seg, const void* x, int64_t T
  * one.  attn_stream carries routing and the softmax branch: the same stream, or another one, which is then made to wait for
  * `stream` before (at ROUTE) and waited for after (at JOIN).  Both belong to one device, which need not be the caller's current one.
  * The attention view may hold other lengths (a prefix of cached
- * keys): T_attn tokens in TN_attn blocks. */
+ * keys): T_attn tokens in TN_attn blocks.
+ * workspace: natsl_mixed_workspace_bytes(), for total_chunks as for natsl_linear_workspace_bytes; of the bytes behind the linear
+ * branch's the softmax branch makes its work queues, so that calls with workspaces of their own may overlap and be replayed in any way.
+ * With natsl_linear_workspace_bytes() alone that branch runs as natsl_softmax_sparse_fwd would. */
 #define NATSL_MIXED_CASTS 8
 enum natsl_mixed_phases { NATSL_MIXED_CONVERT = 1, NATSL_MIXED_ROUTE = 2, NATSL_MIXED_SOFTMAX = 4, NATSL_MIXED_LINEAR = 8, NATSL_MIXED_JOIN = 16 };
 typedef struct natsl_cast { const void* src; void* dst; int64_t n; } natsl_cast;
@@ -482,6 +486,7 @@ typedef struct natsl_mixed {
   const natsl_seq_row* seqs;
   natsl_cast cast_in[NATSL_MIXED_CASTS], cast_out[NATSL_MIXED_CASTS];
 } natsl_mixed;
+size_t natsl_mixed_workspace_bytes(int64_t total_chunks, int H);
 int natsl_mixed_fwd(const natsl_mixed* m, int phases, natsl_stream_t stream, natsl_stream_t attn_stream);
 
 /* Decode: both operators of a step in one call and two launches -- what natsl_attn_masked_fwd and natsl_gdn_recurrent_fwd

@@ -281,7 +281,7 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
     chunk_states = keep_chunk_states and not want_start
     bf16, f32 = torch.bfloat16, torch.float32
     point = lambda name: lambda at: setattr(m, name, at)
-    ws_bytes = L.natsl_linear_workspace_bytes(total_chunks, H)
+    ws_bytes = L.natsl_mixed_workspace_bytes(total_chunks, H)
     idx = own((B, types_attn.shape[1], HN, 2), torch.int32, point("block_indices"))
     nblk = own((n_seqs, HN, 2), torch.int32, point("n_blocks"))
     lse = own((B, T_attn, HQ), f32, point("lse"))

@@ -120,9 +120,14 @@ static int mixed_phases(const natsl_mixed* m, const int phases, natsl_stream_t s
     if (rc != NATSL_OK) return rc;
   }
   auto softmax = [&]() {
-    return natsl_softmax_sparse_fwd(m->q_attn, m->k_attn, m->v_attn, m->o_attn, m->lse, m->types_attn, m->types_dtype, m->block_indices,
-                                    m->n_blocks, m->B, m->T_attn, m->HQ, m->HKV, m->HN, m->KA, m->VA, m->TN_attn, m->block, m->scale_attn,
-                                    m->same_block_visible, NATSL_BF16, m->seqs, m->n_seqs, m->total_qtiles, attn_stream);
+    // the work queues lie behind the linear branch's part of the workspace
+    const long long chunks = m->seqs ? m->total_chunks : (long long)m->B * cdiv(m->T, 64);
+    const size_t at = natsl_linear_workspace_bytes(chunks, m->H);
+    unsigned* queue = nullptr;
+    if (m->workspace && m->workspace_bytes >= at + SOFTMAX_QUEUE_BYTES) queue = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(m->workspace) + at);
+    return softmax_fwd(m->q_attn, m->k_attn, m->v_attn, m->o_attn, m->lse, m->types_attn, m->types_dtype, m->block_indices, m->n_blocks, m->B,
+                       m->T_attn, m->HQ, m->HKV, m->HN, m->KA, m->VA, m->TN_attn, m->block, m->scale_attn, m->same_block_visible, NATSL_BF16,
+                       m->seqs, m->n_seqs, m->total_qtiles, attn_stream, true, queue);
   };
   // Side by side, the scan comes first and the softmax kernel right behind the prep kernel: its workgroups take a CU each for as long
   // as there are tiles, so it has to find the scan's in place and fill the CUs they leave (the other way round the scan waits
@@ -144,6 +149,10 @@ static int mixed_phases(const natsl_mixed* m, const int phases, natsl_stream_t s
     rc = cast_all<false>(m->cast_out, m->n_cast_out, s, what);
   }
   return rc;
+}
+
+extern "C" size_t natsl_mixed_workspace_bytes(int64_t total_chunks, int H) {
+  return natsl_linear_workspace_bytes(total_chunks, H) + SOFTMAX_QUEUE_BYTES;
 }
 
 extern "C" int natsl_mixed_fwd(const natsl_mixed* m, int phases, natsl_stream_t stream, natsl_stream_t attn_stream) {

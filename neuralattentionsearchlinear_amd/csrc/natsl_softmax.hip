@@ -942,6 +942,11 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
 // (batch, head) pairs x, x+8, ... pair after pair, heaviest tile first, so the tiles that share a pair's K/V run
 // together on one L2; a workgroup whose queue is used up takes from the others.  A queue is a ticket counter in device
 // memory, zeroed on the launch's stream by a small fill kernel right before the launch (see launch_softmax_stream).
+// DEALT (with RAGGED only) has no counters, the tiles are dealt out instead: all pairs' latest tiles first, then their next, and
+// so on, to the workgroups in turn, every other round in reverse.  Nothing is shared between launches then; what the workgroups
+// cannot do is even out.  By itself on the GPU that costs little (T8191 H8 64/64, half attention: 212 us with counters -> 180 at four
+// tiles a CU, 745 -> 764 at 17); next to another kernel a workgroup without a CU holds back its share, so the operators, whose scan
+// runs beside this, use counters.
 constexpr int STREAM_ROWS = 1088;  // chunk table of a tile: up to 1024 + 32 chunks of its own and four of the next tile (two tiles' tables are resident)
 constexpr int STREAM_QUEUES = 8;
 constexpr int STREAM_SEQS = 64;    // packed sequences: a lane each
@@ -967,7 +972,7 @@ NATSL_DEVICE unsigned xcc_id() {
 // behind it are not stored.  Against a workgroup per tile: B8 T4095 H12 64/128 half attention 264 -> 212 us, B8 T8191 H16 128/128
 // 729 -> 661, B4 T8191 H32 128/64 593 -> 557, B4 T4095 H32 64/64 181 -> 161; four packed sequences of 65536 tokens in all, H32
 // 128/128, 1410 -> 1280.
-template <int DK, int DV, bool RAGGED>
+template <int DK, int DV, bool RAGGED, bool DEALT>
 __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
   constexpr int QW = 32, QTILE = 256, KSTEPS = DK / 16, VT = DV / 32;
@@ -1070,7 +1075,13 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
   int cq = 0;  // queues used up so far; the queue in use is (xcc + cq) & 7
   unsigned t_ahead = 0;
   auto queue_units = [&](const unsigned qx) -> unsigned { return qx < n_pairs ? ((n_pairs - qx + 7u) / 8u) * NT : 0u; };
+  unsigned rounds = 0;   // (DEALT) tiles taken so far
+  auto next_dealt = [&]() -> unsigned {
+    const unsigned at = rounds & 1u ? gridDim.x - 1u - blockIdx.x : blockIdx.x;
+    return rounds++ * gridDim.x + at;
+  };
   auto take_ticket = [&]() -> unsigned {
+    if (DEALT) return next_dealt();
     unsigned t = 0;
     if (lane == 0) t = atomicAdd(&queue[(xcc + (unsigned)cq) & 7u], 1u);
     return __builtin_amdgcn_readfirstlane(t);
@@ -1083,6 +1094,11 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
     unsigned qx = 0;
     while (cq < STREAM_QUEUES) {
       qx = (xcc + (unsigned)cq) & 7u;
+      if (DEALT) {
+        ok = t < n_pairs * NT;
+        if (!ok) cq = STREAM_QUEUES;
+        break;
+      }
       if (t < queue_units(qx)) {
         ok = true;
         break;
@@ -1099,14 +1115,17 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
     // (Packed: a pair's tiles from the last sequence's last to the first one's first.)
     const unsigned NL = packed ? 0u : NT / 3u, NH = NT - NL, heavy = (queue_units(qx) / NT) * NH;
     unsigned pidx, tile;
-    if (t < heavy) {
+    if (DEALT) {
+      pidx = t % n_pairs;
+      tile = NT - 1u - t / n_pairs;
+    } else if (t < heavy) {
       pidx = t / NH;
       tile = NT - 1u - t % NH;
     } else {
       pidx = (t - heavy) / NL;   // (NL > 0 here: with NL = 0 every ticket is below `heavy`)
       tile = NL - 1u - (t - heavy) % NL;
     }
-    const unsigned pair = pidx * 8u + qx;
+    const unsigned pair = DEALT ? pidx : pidx * 8u + qx;
     unsigned n = pair / (unsigned)p.HQ;
     const unsigned hq = pair - n * (unsigned)p.HQ;
     unsigned bos = n * (unsigned)p.T, nats = n * (unsigned)p.TN;
@@ -1393,7 +1412,10 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
           }
           if (wave == 4) {
             // the tile after the next: ticket asked for in the last chunk but one, turned into a tile in the last
-            if (it == n_iters - 2 && cq < STREAM_QUEUES && lane == 0) t_ahead = atomicAdd(&queue[(xcc + (unsigned)cq) & 7u], 1u);
+            if (it == n_iters - 2 && cq < STREAM_QUEUES) {
+              if (DEALT) t_ahead = next_dealt();
+              else if (lane == 0) t_ahead = atomicAdd(&queue[(xcc + (unsigned)cq) & 7u], 1u);
+            }
             if (last) {
               int d0 = 0, l0 = 0;
               const int r0 = resolve_ticket(__builtin_amdgcn_readfirstlane(t_ahead), &info[a ^ 1], d0, l0);
@@ -1483,16 +1505,18 @@ static int launch_softmax(const SoftmaxParams& p, hipStream_t stream) {
   return check_launch("natsl_softmax_sparse_fwd");
 }
 
-// Ticket counters of the persistent kernel: library-owned device memory, STREAM_SLOTS slots of counters.  Consecutive
-// launches rotate through the slots, and each launch is preceded ON ITS STREAM by a fill kernel that zeroes its slot (a
-// kernel, not hipMemsetAsync, so that both can be captured into a HIP graph and replayed).  Nothing is left to set
-// back afterwards: a launch that was cut short cannot poison a later one.  Two launches use one slot at the same time
-// only if STREAM_SLOTS launches lie between them and both are still running, or if a captured graph (whose slot was
-// fixed at capture) is replayed next to an eager launch that drew the same slot; the launches would then share each
-// other's tickets and leave tiles uncomputed, so keep fewer than STREAM_SLOTS launches of this entry in flight per GPU
-// and replay captured launches on the stream that also carries the eager ones.
+// Ticket counters of the persistent kernel.  They are zeroed on the launch's stream by a fill kernel right before it (a kernel, not
+// hipMemsetAsync, so that both can be captured into a HIP graph and replayed); nothing is left to set back afterwards, so a launch
+// that was cut short cannot poison a later one.  Three homes:
+//  * the mixed operator's launches have theirs in the call's own workspace;
+//  * natsl_softmax_sparse_fwd has no workspace.  Its whole-tile launches rotate through STREAM_SLOTS slots of library-owned memory.
+//    Two of them use one slot at the same time only if STREAM_SLOTS launches lie between them and both are still running, or if a
+//    captured graph (whose slot was fixed at capture) is replayed next to an eager launch that drew the same slot; the launches would
+//    then share each other's tickets and leave tiles uncomputed, so keep fewer than STREAM_SLOTS launches of this entry in flight per
+//    GPU and replay captured launches on the stream that also carries the eager ones;
+//  * its launches on packed sequences and on other lengths have none: their tiles are dealt out, and they may overlap in any way.
 constexpr int STREAM_SLOTS = 64;
-static std::atomic<unsigned> stream_launches{0};   // of all forms of the kernel: they share the slots
+static std::atomic<unsigned> stream_launches{0};   // of all head widths: they share the slots
 static __device__ __align__(256) unsigned stream_queues[STREAM_SLOTS * STREAM_SLOT_WORDS];
 
 __global__ void stream_queue_clear_kernel(unsigned* slot) {
@@ -1531,14 +1555,14 @@ static const StreamDevice* stream_device(int* rc) {
   return &devs[dev];
 }
 
-template <int DK, int DV, bool RAGGED>
-static int launch_softmax_stream(const SoftmaxParams& p, const StreamDevice* d, hipStream_t stream) {
+template <int DK, int DV, bool RAGGED, bool DEALT>
+static int launch_softmax_stream(const SoftmaxParams& p, const StreamDevice* d, unsigned* queue, hipStream_t stream) {
   static std::atomic<unsigned long long> reserved{0};
   const size_t lds = (size_t)(4 * 64 * (DK + DV) + 64 * DV) * sizeof(bf16_t) + 1024;  // four K and four V tiles, the output's staging area; 1 KiB aligned
-  auto kern = softmax_stream_kernel<DK, DV, RAGGED>;
+  auto kern = softmax_stream_kernel<DK, DV, RAGGED, DEALT>;
   if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, lds, "softmax")) return rc;
-  unsigned* queue = d->queues + (size_t)(stream_launches.fetch_add(1) % STREAM_SLOTS) * STREAM_SLOT_WORDS;
-  hipLaunchKernelGGL(stream_queue_clear_kernel, dim3(1), dim3(64), 0, stream, queue);
+  if (!RAGGED && !queue) queue = d->queues + (size_t)(stream_launches.fetch_add(1) % STREAM_SLOTS) * STREAM_SLOT_WORDS;
+  if (queue) hipLaunchKernelGGL(stream_queue_clear_kernel, dim3(1), dim3(64), 0, stream, queue);
   hipLaunchKernelGGL(kern, dim3((unsigned)d->cus), dim3(512), lds, stream, p, queue);
   return check_launch("natsl_softmax_sparse_fwd");
 }
@@ -1572,14 +1596,12 @@ static int softmax_variant(int B, int T, int HQ, int HKV, int block, bool packed
   return (long long)B * HQ * cdiv(T, 256) >= 256 ? NATSL_SOFTMAX_TILE_256 : NATSL_SOFTMAX_TILE_128;
 }
 
-}  // namespace natsl
+static_assert(SOFTMAX_QUEUE_BYTES == STREAM_SLOT_WORDS * sizeof(unsigned), "the counters of one launch");
 
-using namespace natsl;
-
-static int softmax_fwd(const void* q, const void* k, const void* v, void* o, float* lse, const void* types, int types_dtype,
-                       const int32_t* nats_block_indices, const int32_t* n_nats_blocks, int B, int T, int HQ, int HKV, int HN, int K,
-                       int V, int TN, int block, float scale, int same_block_visible, int dtype, const natsl_seq_row* seqs,
-                       int n_seqs, int total_units, natsl_stream_t stream, bool allow_persistent) {
+int softmax_fwd(const void* q, const void* k, const void* v, void* o, float* lse, const void* types, int types_dtype,
+                const int32_t* nats_block_indices, const int32_t* n_nats_blocks, int B, int T, int HQ, int HKV, int HN, int K,
+                int V, int TN, int block, float scale, int same_block_visible, int dtype, const natsl_seq_row* seqs,
+                int n_seqs, int total_units, natsl_stream_t stream, bool allow_persistent, unsigned* queue) {
   if (!q || !k || !v || !o || !lse || !types || !nats_block_indices || !n_nats_blocks)
     return fail(NATSL_ERR_INVALID, "softmax: null pointer argument");
   if (dtype != NATSL_BF16) return fail(NATSL_ERR_UNSUPPORTED, "softmax: only bf16 tensors are supported (got dtype %d)", dtype);
@@ -1611,7 +1633,8 @@ static int softmax_fwd(const void* q, const void* k, const void* v, void* o, flo
   p.variant = variant == NATSL_SOFTMAX_TILE_128 ? 4 : 8;
 #define NATSL_SM(KK, VV)                                              \
   if (K == KK && V == VV) {                                           \
-    if (sd) return seqs || T % 256 ? launch_softmax_stream<KK, VV, true>(p, sd, s) : launch_softmax_stream<KK, VV, false>(p, sd, s); \
+    if (sd && !seqs && T % 256 == 0) return launch_softmax_stream<KK, VV, false, false>(p, sd, queue, s); \
+    if (sd) return queue ? launch_softmax_stream<KK, VV, true, false>(p, sd, queue, s) : launch_softmax_stream<KK, VV, true, true>(p, sd, nullptr, s); \
     return p.variant == 8 ? launch_softmax<KK, VV, 8>(p, s) : launch_softmax<KK, VV, 4>(p, s); \
   }
   NATSL_SM(128, 128)
@@ -1622,6 +1645,10 @@ static int softmax_fwd(const void* q, const void* k, const void* v, void* o, flo
   return fail(NATSL_ERR_UNSUPPORTED, "softmax: head dims K=%d, V=%d not built (supported: 64/128 x 64/128)", K, V);
 }
 
+}  // namespace natsl
+
+using namespace natsl;
+
 extern "C" int natsl_softmax_sparse_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
                                         const void* types, int types_dtype, const int32_t* nats_block_indices,
                                         const int32_t* n_nats_blocks, int B, int T, int HQ, int HKV, int HN, int K,
@@ -1629,7 +1656,7 @@ extern "C" int natsl_softmax_sparse_fwd(const void* q, const void* k, const void
                                         const natsl_seq_row* seqs, int n_seqs, int total_units,
                                         natsl_stream_t stream) {
   return softmax_fwd(q, k, v, o, lse, types, types_dtype, nats_block_indices, n_nats_blocks, B, T, HQ, HKV, HN, K, V, TN, block,
-                     scale, same_block_visible, dtype, seqs, n_seqs, total_units, stream, true);
+                     scale, same_block_visible, dtype, seqs, n_seqs, total_units, stream, true, nullptr);
 }
 
 extern "C" int natsl_softmax_sparse_fwd_per_tile(const void* q, const void* k, const void* v, void* o, float* lse,
@@ -1639,7 +1666,7 @@ extern "C" int natsl_softmax_sparse_fwd_per_tile(const void* q, const void* k, c
                                                  const natsl_seq_row* seqs, int n_seqs, int total_units,
                                                  natsl_stream_t stream) {
   return softmax_fwd(q, k, v, o, lse, types, types_dtype, nats_block_indices, n_nats_blocks, B, T, HQ, HKV, HN, K, V, TN, block,
-                     scale, same_block_visible, dtype, seqs, n_seqs, total_units, stream, false);
+                     scale, same_block_visible, dtype, seqs, n_seqs, total_units, stream, false, nullptr);
 }
 
 extern "C" int natsl_softmax_fwd_variant(int B, int T, int HQ, int HKV, int block, int packed) {

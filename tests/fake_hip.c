@@ -8,6 +8,10 @@ static char notes[1 << 16];
 static size_t used;
 static int current, next_event;
 static int event_device[256];
+static char launches[1 << 16];   /* a line per launch: kernel, stream, grid, and for kernels of the softmax queues their address */
+static size_t launched;
+static struct { const void* f; const char* name; } kernels[512];
+static int n_kernels;
 
 static void note(const char* fmt, ...) {
   va_list ap;
@@ -18,7 +22,8 @@ static void note(const char* fmt, ...) {
 static int device_of(const void* s) { return s ? (int)((size_t)s >> 12) : current; }
 
 const char* fake_notes(void) { return notes; }
-void fake_reset(int device) { used = 0; notes[0] = 0; current = device; }
+const char* fake_launches(void) { return launches; }
+void fake_reset(int device) { used = 0; notes[0] = 0; launched = 0; launches[0] = 0; current = device; }
 int fake_current(void) { return current; }
 
 int hipGetDevice(int* d) { *d = current; return 0; }
@@ -49,9 +54,21 @@ int __hipPopCallConfiguration(dim3_t* grid, dim3_t* block, size_t* lds, void** s
   *grid = config.grid; *block = config.block; *lds = config.lds; *s = config.stream;
   return 0;
 }
+void __hipRegisterFunction(void** modules, const void* f, char* device_function, const char* name, unsigned limit, void* tid, void* bid, void* block, void* grid, int* size) {
+  (void)modules; (void)device_function; (void)limit; (void)tid; (void)bid; (void)block; (void)grid; (void)size;
+  if (n_kernels < 512) { kernels[n_kernels].f = f; kernels[n_kernels++].name = name; }
+}
 int hipLaunchKernel(const void* f, dim3_t grid, dim3_t block, void** args, size_t lds, void* s) {
-  (void)f; (void)grid; (void)block; (void)args; (void)lds;
+  const char* name = "?";
+  const void* queue = 0;
+  (void)block; (void)lds;
+  for (int i = 0; i < n_kernels; ++i)
+    if (kernels[i].f == f) name = kernels[i].name;
+  if (strstr(name, "stream_queue_clear_kernel")) queue = *(void**)args[0];
+  if (strstr(name, "softmax_stream_kernel")) queue = *(void**)args[1];
   note("launch %lx:%d ", (unsigned long)(size_t)s, current);
+  if (launched < sizeof(launches) - 256)
+    launched += snprintf(launches + launched, 256, "%s %lx %u %lx\n", name, (unsigned long)(size_t)s, grid.x, (unsigned long)(size_t)queue);
   return 0;
 }
 int hipFuncSetAttribute(const void* f, int attr, int value) { (void)f; (void)attr; (void)value; return 0; }

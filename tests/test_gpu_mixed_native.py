@@ -52,3 +52,34 @@ def test_side_stream_and_one_stream_agree(kind, B, H, K, V, monkeypatch):
         monkeypatch.setattr(MC, 'CONCURRENT_BRANCHES', side)
         outs.append(_run(kind, q, k, v, g, beta, ty))
     assert all(torch.equal(a, b) for a, b in zip(*outs))
+
+
+@pytest.mark.parametrize("T,seqs", [(1023, 17), (1024, 17)])
+def test_captured_operator_replays_beside_other_launches(T, seqs):
+    """A captured forward whose softmax branch is the persistent kernel, replayed while eager launches of that kernel run on another
+    stream (more of them than the library has slots): the operator's work queues are its own."""
+    from neuralattentionsearchlinear_amd import _capi
+    from tests.test_gpu_softmax_stream import _call, _inputs
+    H = 32
+    assert _capi.lib().natsl_softmax_fwd_variant(seqs, T, H, H, 64, 0) == 2, "shape does not reach the persistent kernel on this GPU"
+    q, k, v, g, beta, ty = _case('gdn', seqs, T, H, 64, 64, 3)
+    args = [t.bfloat16() for t in (q, k, v)] + [g, beta.bfloat16(), ty.bfloat16()]
+    _, _, _, _, qe, ke, ve, te = _inputs(4, 4096, 16, 16, 16, 64, 64, 64, 0.25, 5, torch.device(DEV))
+    with torch.no_grad():
+        ref = [t.clone() for t in _run('gdn', *args)]
+        other_ref = _call(qe, ke, ve, te, 64, 64, True)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = _run('gdn', *args)
+        other = torch.cuda.Stream()                       # default priority
+        for i in range(3):
+            for t in out:
+                t.fill_(float('nan'))
+            torch.cuda.synchronize()
+            with torch.cuda.stream(other):
+                o = [_call(qe, ke, ve, te, 64, 64, True) for _ in range(35)]
+            graph.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(out, ref)), f"replay {i}"
+            assert all(torch.equal(a, b) for pair in o for a, b in zip(pair, other_ref)), f"beside replay {i}"

@@ -119,7 +119,7 @@ int natsl_softmax_sparse_fwd(const void* q, const void* k, const void* v, void* 
 /* The same operation, always as one workgroup per query tile (what natsl_softmax_sparse_fwd itself runs for small
  * problems, short sequences and more than 64 packed sequences): for callers that want no library-owned device state in the launch, and the regression
  * check of the persistent kernel.  The same results bit for bit, except for the queries of a sequence's last 256-row
- * tile where its length is no multiple of 64: those differ by the rounding of the probabilities in the row sums.
+ * tile where its length is no multiple of 64: there the two take other reference maxima, so the probabilities round differently.
  * Same reference interface as natsl_softmax_sparse_fwd. */
 int natsl_softmax_sparse_fwd_per_tile(const void* q, const void* k, const void* v, void* o, float* lse,
                              const void* types, int types_dtype, const int32_t* nats_block_indices,

@@ -338,9 +338,11 @@ NATSL_DEVICE void pv_phase(const unsigned vaddr, const bf16x8 (&PB)[4], f32x16 (
 // order.  The common path is a maximum (for the check), 32 exp2 and the packing.  The reference moves, in a side
 // block, when a score outgrows it by more than `thr`: -inf while the row has seen no key yet (m_ref is then still the
 // arbitrary 0 and the first visible score sets the real one), RESCALE_SLACK afterwards.
-template <int DV>
+// sums (FP32_SUMS only; wave-uniform): the row sums are formed here, from the probabilities before their rounding, as chunk_pipelined
+// forms them, and pv_phase's are not to be used.
+template <int DV, bool FP32_SUMS = false>
 NATSL_DEVICE void softmax_phase(f32x16& s0, f32x16& s1, f32x16 (&acc)[DV / 32], float& m_ref, float& l_run, float& thr,
-                                const int lane, const bool causal, const int qloc0, bf16x8 (&PB)[4]) {
+                                const int lane, const bool causal, const int qloc0, bf16x8 (&PB)[4], const bool sums = false) {
   if (causal) {
     mask_half(s0, 0, lane, qloc0);
     mask_half(s1, 1, lane, qloc0);
@@ -369,6 +371,30 @@ NATSL_DEVICE void softmax_phase(f32x16& s0, f32x16& s1, f32x16 (&acc)[DV / 32], 
     for (int r = 0; r < 16; ++r) {
       s0[r] -= delta;
       s1[r] -= delta;
+    }
+  }
+  if constexpr (FP32_SUMS) {
+    if (sums) {
+      float rs = 0.f;
+      auto prob = [&](float x) __attribute__((always_inline)) -> float {
+        asm volatile("" : "+v"(x));   // (the same exponentials as below: shared, they are kept, and 128/128 heads spill)
+        x = __builtin_amdgcn_exp2f(x);
+        rs += x;
+        return x;
+      };
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x16& s = g < 2 ? s0 : s1;
+        u32x4 w;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float lo = prob(s[8 * (g & 1) + 2 * j]), hi = prob(s[8 * (g & 1) + 2 * j + 1]);
+          w[j] = pack_bf16x2(lo, hi);
+        }
+        PB[g] = __builtin_bit_cast(bf16x8, w);
+      }
+      l_run += rs;
+      return;
     }
   }
 #pragma unroll
@@ -969,7 +995,8 @@ NATSL_DEVICE unsigned xcc_id() {
 // number of tiles.  The last tile of a sequence keeps its full set of chunks (the rules of the rings do not
 // change); its chunks past the end are requested from the tile's first chunk and nobody takes part in them, the chunk that the end
 // cuts (marked in the chunk table: all bits of its row inverted) repeats the last row, waves behind the end stay idle, and rows
-// behind it are not stored.  Against a workgroup per tile: B8 T4095 H12 64/128 half attention 264 -> 212 us, B8 T8191 H16 128/128
+// behind it are not stored.  The tile of a cut chunk keeps the per-tile kernel's fp32 row sums (taken from the rounded probabilities,
+// its log-sum-exp was off by 1.6e-4 on average and 1.4e-3 at most, against 4e-7 and 1.5e-6).  Against a workgroup per tile: B8 T4095 H12 64/128 half attention 264 -> 212 us, B8 T8191 H16 128/128
 // 729 -> 661, B4 T8191 H32 128/64 593 -> 557, B4 T4095 H32 64/64 181 -> 161; four packed sequences of 65536 tokens in all, H32
 // 128/128, 1410 -> 1280.
 template <int DK, int DV, bool RAGGED, bool DEALT>
@@ -1317,6 +1344,12 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
     thr = -INFINITY;
     f32x16 s0, s1;
     auto is_active = [&](const int it) -> bool { return it < n_diag ? (act_mask >> it) & 1ull : it < n_iters && (!RAGGED || q0 < len); };
+    const bool cut = RAGGED && (len & 63) && tile_start + QTILE > len;   // this tile holds the chunk that the sequence's end cuts
+    auto pv = [&](const int it, const bf16x8 (&PB)[4]) __attribute__((always_inline)) {
+      float l = l_run;
+      pv_phase<DV>(lds_v + ((sp0 + it) & 3) * VTILE + v_lane, PB, acc, l);
+      if (!cut) l_run = l;
+    };
     bool cur_active = act_mask & 1ull;
     if (cur_active) qk_phase<DK>(lds_k + (sp0 & 3) * KTILE + k_lane, QB, m_ref, s0, s1);
 
@@ -1332,9 +1365,9 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
         const int row_ahead = *reinterpret_cast<lds_row>(row_tab + 4u * it);   // chunk it + 4, used after the barrier
         bf16x8 PB[4];
         if (cur_active) {
-          softmax_phase<DV>(s0, s1, acc, m_ref, l_run, thr, lane, it == causal_it, qloc0, PB);
+          softmax_phase<DV, RAGGED>(s0, s1, acc, m_ref, l_run, thr, lane, it == causal_it, qloc0, PB, cut);
           __builtin_amdgcn_s_setprio(3);
-          pv_phase<DV>(lds_v + ((sp0 + it) & 3) * VTILE + v_lane, PB, acc, l_run);
+          pv(it, PB);
         }
         __builtin_amdgcn_s_setprio(3);
         if (nxt_active) qk_phase<DK>(lds_k + ((sp0 + it + 1) & 3) * KTILE + k_lane, QB, m_ref, s0, s1);
@@ -1427,7 +1460,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
           ev_it = it == 0 ? 1 : (it < n_iters - 2 ? n_iters - 2 : it + 1);
         }
         bf16x8 PB[4];
-        if (cur_active) softmax_phase<DV>(s0, s1, acc, m_ref, l_run, thr, lane, it == causal_it, qloc0, PB);
+        if (cur_active) softmax_phase<DV, RAGGED>(s0, s1, acc, m_ref, l_run, thr, lane, it == causal_it, qloc0, PB, cut);
 #pragma unroll
         for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(PB[i]));   // the probabilities exist before the barrier
         // V(it+1) must have landed; the newest request, V(it+2), if there was one, may stay in flight (the first iteration: as
@@ -1439,7 +1472,7 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
         __syncthreads();                                  // sync(it)
         const int row_ahead = *reinterpret_cast<lds_row>(row_tab + 4u * it);   // chunk it + 3
         __builtin_amdgcn_s_setprio(3);
-        if (cur_active) pv_phase<DV>(lds_v + ((sp0 + it) & 3) * VTILE + v_lane, PB, acc, l_run);
+        if (cur_active) pv(it, PB);
         if (nxt_active) qk_phase<DK>(lds_k + ((sp0 + it + 1) & 3) * KTILE + k_lane, QB, m_ref, s0, s1);
         __builtin_amdgcn_s_setprio(0);
         req = (unsigned)(it + 3 - rq_lo) < rq_span;

@@ -82,8 +82,8 @@ def test_persistent_kernel_equals_the_per_tile_kernel(B, T, HQ, H, HN, K, V, blo
 def test_persistent_kernel_with_a_cut_last_tile(T, K, V, H, block, same_block):
     """Sequences that end inside a tile, a wave's queries or a chunk: bit for bit what the per-tile kernel gives for whole chunks (same
     order, same arithmetic), also where the rows behind a sequence's end, the next one's first, hold NaNs.  The tile of a cut chunk
-    goes another way in that kernel (its row sums take the probabilities before their rounding): there both are held to the bound that
-    each is held to against the oracle."""
+    goes another way in that kernel (other reference maxima): there both are held to the bound that each is held to against the
+    oracle."""
     from neuralattentionsearchlinear_amd import _capi
     B, HQ, HN, dev = 22, 32, 8, torch.device('cuda:0')
     g = torch.Generator(device=dev).manual_seed(31)
@@ -142,6 +142,44 @@ def test_persistent_kernel_on_packed_sequences(lens, K, V, H, block, same_block)
             assert bool(torch.isfinite(y[a:b]).all()) and torch.equal(x[a:whole], y[a:whole])
             if whole < b:
                 assert_close(y[whole:b].float(), x[whole:b].float(), f"sequence {i}")
+
+
+@pytest.mark.parametrize("K,V", [(128, 128), (64, 64), (64, 128), (128, 64)])
+@pytest.mark.parametrize("T", [769, 831, 897, 1023])
+def test_row_sums_of_a_cut_last_tile_are_fp32(K, V, T):
+    """The log-sum-exp of the tile that a sequence's end cuts inside a chunk, against 64-bit arithmetic on the scaled bf16 queries that
+    the kernel multiplies.  With fp32 probabilities in the sums it is off by the rounding of K products of a few units (K 2^-24 x 8 at
+    most, 6e-5 for 128 aligned signs, 1.5e-6 seen) and of at most T additions whose partial sums are below 2^3 of the result; 1e-5 lies
+    between that and probabilities rounded to bf16 (2^-9 each: 1.6e-4 on average, 5e-4 to 1.4e-3 at most)."""
+    import math
+    B, H, block, dev = 22, 32, 64, torch.device('cuda:0')
+    g = torch.Generator(device=dev).manual_seed(T)
+    q, k, v = (torch.randn(B, T, H, d, device=dev, generator=g).bfloat16() for d in (K, K, V))
+    ty = make_types(B, -(-T // block), H, 0.4, 33, torch.bfloat16).to(dev)
+    for persistent in (False, True):
+        _, lse = _call(q, k, v, ty, K, block, True, persistent)
+        b, whole = 3, T // 256 * 256
+        scale = torch.tensor(K ** -0.5, dtype=torch.float32, device=dev) * 1.4426950408889634
+        qs = (q[b].float() * scale).bfloat16().double()
+        s = torch.matmul(qs[whole:].transpose(0, 1).contiguous(), k[b].double().permute(1, 2, 0).contiguous())      # [H, queries, keys], log2 units
+        i, j = torch.arange(whole, T, device=dev)[:, None], torch.arange(T, device=dev)[None]
+        typed = (ty[b, :, :, 0] > 0.5).T[:, torch.arange(T, device=dev) // block][:, None, :]
+        seen = (j <= i) & ((j // block == i // block) | typed)
+        ref = torch.logsumexp(torch.where(seen, s * math.log(2), torch.full_like(s, -1e300)), -1) / math.log(2)
+        worst = float((lse[b, whole:].T.double() - ref).abs().max())
+        assert worst <= 1e-5, f"persistent {persistent}: {worst:.2e}"
+
+
+def test_operator_and_entry_agree_on_a_cut_length():
+    """The same tiles from work queues (the operators) and dealt out (the entry): the same bits."""
+    import torch.nn.functional as F
+    from neuralattentionsearchlinear_amd.mixed_attn_gdn import nats_mixed_attn_gdn
+    B, T, H, D, block, dev = 22, 1023, 32, 64, 64, torch.device('cuda:0')
+    _, _, _, _, q, k, v, ty = _inputs(B, T, H, H, H, D, D, block, 0.4, 8, dev)
+    beta, g = torch.sigmoid(torch.randn(B, T, H, device=dev)).bfloat16(), -F.softplus(torch.randn(B, T, H, device=dev))
+    with torch.no_grad():
+        out = nats_mixed_attn_gdn(q, k, v, q, k, v, None, g, beta, ty, None, ops_for_incomplete_chunks='all')
+    assert torch.equal(out[1], _call(q, k, v, ty, D, block, True)[0])
 
 
 def test_persistent_kernel_queues_across_launches_and_streams():

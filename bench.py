@@ -150,9 +150,9 @@ def clock_probe(torch, device):
 
 
 def softmax_kernel_name(B, T, H, block):
-    """The kernel natsl_softmax_sparse_fwd runs for this problem, as the library itself reports it."""
+    """The softmax kernel the operator runs for this problem, as the library itself reports it."""
     from neuralattentionsearchlinear_amd import _capi
-    v = _capi.lib().natsl_softmax_fwd_variant(B, T, H, H, block, 0)
+    v = _capi.lib().natsl_mixed_softmax_variant(B, T, H, H, block, 0)
     return {0: "softmax_sparse_fwd_kernel<4 waves>", 1: "softmax_sparse_fwd_kernel<8 waves>", 2: "softmax_stream_kernel"}.get(v, f"unknown ({v})")
 
 

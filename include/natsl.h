@@ -460,7 +460,8 @@ int natsl_wgrad(const natsl_wgrad_seg* segs, int n_seg, const void* x, int64_t T
  * keys): T_attn tokens in TN_attn blocks.
  * workspace: natsl_mixed_workspace_bytes(), for total_chunks as for natsl_linear_workspace_bytes; of the bytes behind the linear
  * branch's the softmax branch makes its work queues, so that calls with workspaces of their own may overlap and be replayed in any way.
- * With natsl_linear_workspace_bytes() alone that branch runs as natsl_softmax_sparse_fwd would. */
+ * With natsl_linear_workspace_bytes() alone it has the queues that natsl_softmax_sparse_fwd has.  (That entry takes the persistent kernel for
+ * smaller problems than this one.) */
 #define NATSL_MIXED_CASTS 8
 enum natsl_mixed_phases { NATSL_MIXED_CONVERT = 1, NATSL_MIXED_ROUTE = 2, NATSL_MIXED_SOFTMAX = 4, NATSL_MIXED_LINEAR = 8, NATSL_MIXED_JOIN = 16 };
 typedef struct natsl_cast { const void* src; void* dst; int64_t n; } natsl_cast;
@@ -487,6 +488,7 @@ typedef struct natsl_mixed {
   natsl_cast cast_in[NATSL_MIXED_CASTS], cast_out[NATSL_MIXED_CASTS];
 } natsl_mixed;
 size_t natsl_mixed_workspace_bytes(int64_t total_chunks, int H);
+int natsl_mixed_softmax_variant(int B, int T, int HQ, int HKV, int block, int packed);   /* natsl_softmax_fwd_variant of its softmax branch */
 int natsl_mixed_fwd(const natsl_mixed* m, int phases, natsl_stream_t stream, natsl_stream_t attn_stream);
 
 /* Decode: both operators of a step in one call and two launches -- what natsl_attn_masked_fwd and natsl_gdn_recurrent_fwd

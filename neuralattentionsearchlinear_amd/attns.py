@@ -38,7 +38,10 @@ def parallel_attn_nats_fwd(
     o = torch.empty(B, T, HQ, V, dtype=v.dtype, device=q.device)
     lse = torch.empty(B, T, HQ, dtype=torch.float32, device=q.device)
     sp, ns, tot = _seq_args(seqs, seqs.total_qtiles if seqs is not None else 0)
-    rc = _capi.lib().natsl_softmax_sparse_fwd(
+    # (whole tiles below six per CU: the library's entry takes the persistent kernel from two on, where it is the slower one)
+    L = _capi.lib()
+    few = q.is_cuda and seqs is None and T % 256 == 0 and B * HQ * (T // 256) < 6 * torch.cuda.get_device_properties(q.device).multi_processor_count
+    rc = (L.natsl_softmax_sparse_fwd_per_tile if few else L.natsl_softmax_sparse_fwd)(
         _capi.ptr(q), _capi.ptr(k), _capi.ptr(v), _capi.ptr(o), _capi.ptr(lse), _capi.ptr(ty), _capi.dtype_code(ty.dtype),
         _capi.ptr(nats_block_indices), _capi.ptr(n_nats_blocks), B, T, HQ, H, HN, K, V, TN, NAtS_block_size, float(scale),
         int(bool(compute_incomplete_chunk_scores)), _capi.dtype_code(q.dtype), sp, ns, tot, _capi.stream_ptr(q.device))

@@ -127,7 +127,7 @@ static int mixed_phases(const natsl_mixed* m, const int phases, natsl_stream_t s
     if (m->workspace && m->workspace_bytes >= at + SOFTMAX_QUEUE_BYTES) queue = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(m->workspace) + at);
     return softmax_fwd(m->q_attn, m->k_attn, m->v_attn, m->o_attn, m->lse, m->types_attn, m->types_dtype, m->block_indices, m->n_blocks, m->B,
                        m->T_attn, m->HQ, m->HKV, m->HN, m->KA, m->VA, m->TN_attn, m->block, m->scale_attn, m->same_block_visible, NATSL_BF16,
-                       m->seqs, m->n_seqs, m->total_qtiles, attn_stream, true, queue);
+                       m->seqs, m->n_seqs, m->total_qtiles, attn_stream, SOFTMAX_OPERATOR, queue);
   };
   // Side by side, the scan comes first and the softmax kernel right behind the prep kernel: its workgroups take a CU each for as long
   // as there are tiles, so it has to find the scan's in place and fill the CUs they leave (the other way round the scan waits

@@ -1600,28 +1600,33 @@ static int launch_softmax_stream(const SoftmaxParams& p, const StreamDevice* d, 
   return check_launch("natsl_softmax_sparse_fwd");
 }
 
-// Which kernel natsl_softmax_sparse_fwd runs for a problem.  The persistent one needs tiles to follow each other on its one workgroup
-// per CU: below that, two workgroups of a tile each per CU hide each other's ends and even out better.  Time per tile kernel / persistent
-// kernel, heads 64 and 128, 5 - 50 % attention, lengths of 333 .. 8256: 0.60 - 1.0 at two tiles per CU, 0.63 - 1.14 at four, 0.74 - 1.22
-// at six, 0.81 - 1.25 at eight, 0.94 - 1.3 at 16; the low ends are few attention blocks and K = V = 64, the high ends half attention and
-// lengths that cut a chunk.  So it takes eight tiles' worth of queries per CU.  Where sequences are shorter than a tile, what it does for
-// the missing queries costs more than it saves (100 queries: 0.42 - 0.8 up to 16 tiles per CU).  Whole tiles of at least 2048 queries
-// take it from two tiles per CU (0.69 - 1.02 there, 0.78 - 1.06 at four): its tests hold it at these small problems.
-// Long sequences that end inside a chunk take it from three: their last tile, the longest, goes the per-tile kernel's slow way (8191
-// queries at three tiles per CU: 1.04 - 1.12 with 25 % attention or more, 0.73 - 0.93 with 5 %, where there is little to lose; 4099: 0.69 - 0.87).
+// Which kernel runs for a problem.  The persistent one needs tiles to follow each other on its one workgroup per CU.  A workgroup of
+// either kernel fills a CU (eight waves, two a SIMD); what the persistent one pays is its start: the fill kernel, the first ticket and a
+// virtual tile, 12 - 17 us in all, and tiles in the order of their pairs instead of all long ones first.  Time per tile kernel /
+// persistent kernel with counters, by themselves, heads 64 and 128, 5 - 50 % attention, lengths of 333 .. 8256: 0.60 - 1.0 at two tiles
+// per CU, 0.63 - 1.14 at four, 0.74 - 1.22 at six, 0.81 - 1.25 at eight, 0.94 - 1.3 at 16; the low ends are few attention blocks and
+// K = V = 64, the high ends half attention and lengths that cut a chunk.  So it takes eight tiles' worth of queries per CU.  Where
+// sequences are shorter than a tile, what it does for the missing queries costs more than it saves (100 queries: 0.42 - 0.8 up to 16
+// tiles per CU).
+// Operators (the linear branch's scan runs beside it and hides a part of that): from six on whole tiles of 2048 queries or more and on
+// lengths from 6144 that cut a chunk.  Time of the whole operator, per tile / persistent, the four head shapes: whole tiles 0.79 - 1.02
+// at two, 0.86 - 1.02 at four, 0.92 - 1.03 at six, 0.94 - 1.04 at eight; cut lengths (6145 .. 33000) 0.87 - 1.02 at three, 0.91 - 1.07
+// at four, 0.94 - 1.09 at six, 0.96 - 1.08 at eight.
+// The entry by itself takes whole tiles of 2048 queries or more from two on and cut lengths from 6144 from three: its tests hold it at
+// these small problems (dealt out, cut lengths lose little there: 0.86 - 1.0 at three, 0.88 - 1.27 at four).
 // Of the others, one workgroup per tile, of 256 queries on 8 waves once there is at least one such tile per compute unit (measured:
-// from there on that shape is the faster one; below, 128-query tiles fill more compute units).
-static int softmax_variant(int B, int T, int HQ, int HKV, int block, bool packed, bool allow_persistent, int n_seqs, const StreamDevice** sd,
-                           int* rc) {
+// from there on that shape is the faster one; below, 128-query tiles, two workgroups of four waves a CU, fill more compute units).
+static int softmax_variant(int B, int T, int HQ, int HKV, int block, bool packed, SoftmaxUse use, int n_seqs, const StreamDevice** sd, int* rc) {
   *sd = nullptr;
   *rc = NATSL_OK;
-  if (allow_persistent && (!packed || n_seqs <= STREAM_SEQS) && T <= 65536 && block <= 2048 && (long long)B * T * HKV < (1ll << 31)) {
+  if (use != SOFTMAX_PER_TILE && (!packed || n_seqs <= STREAM_SEQS) && T <= 65536 && block <= 2048 && (long long)B * T * HKV < (1ll << 31)) {
     const StreamDevice* d = stream_device(rc);
     if (!d) return -1;
     const long long tiles = (long long)B * HQ * T / 256;   // whole tiles' worth of queries
-    const bool whole = !packed && T % 256 == 0;
+    const bool whole = !packed && T % 256 == 0 && T >= 2048;
     const bool cut = !packed && T % 64 && T >= 6144;
-    if (tiles >= (whole && T >= 2048 ? 2ll : cut ? 3ll : 8ll) * d->cus && T / (packed ? n_seqs : 1) >= 256) {
+    const long long line = use == SOFTMAX_OPERATOR ? (whole || cut ? 6 : 8) : whole ? 2 : cut ? 3 : 8;
+    if (tiles >= line * d->cus && T / (packed ? n_seqs : 1) >= 256) {
       *sd = d;
       return NATSL_SOFTMAX_PERSISTENT;
     }
@@ -1634,7 +1639,7 @@ static_assert(SOFTMAX_QUEUE_BYTES == STREAM_SLOT_WORDS * sizeof(unsigned), "the 
 int softmax_fwd(const void* q, const void* k, const void* v, void* o, float* lse, const void* types, int types_dtype,
                 const int32_t* nats_block_indices, const int32_t* n_nats_blocks, int B, int T, int HQ, int HKV, int HN, int K,
                 int V, int TN, int block, float scale, int same_block_visible, int dtype, const natsl_seq_row* seqs,
-                int n_seqs, int total_units, natsl_stream_t stream, bool allow_persistent, unsigned* queue) {
+                int n_seqs, int total_units, natsl_stream_t stream, SoftmaxUse use, unsigned* queue) {
   if (!q || !k || !v || !o || !lse || !types || !nats_block_indices || !n_nats_blocks)
     return fail(NATSL_ERR_INVALID, "softmax: null pointer argument");
   if (dtype != NATSL_BF16) return fail(NATSL_ERR_UNSUPPORTED, "softmax: only bf16 tensors are supported (got dtype %d)", dtype);
@@ -1661,7 +1666,7 @@ int softmax_fwd(const void* q, const void* k, const void* v, void* o, float* lse
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const StreamDevice* sd = nullptr;
   int rc;
-  const int variant = softmax_variant(B, T, HQ, HKV, block, seqs != nullptr, allow_persistent, n_seqs, &sd, &rc);
+  const int variant = softmax_variant(B, T, HQ, HKV, block, seqs != nullptr, use, n_seqs, &sd, &rc);
   if (variant < 0) return rc;
   p.variant = variant == NATSL_SOFTMAX_TILE_128 ? 4 : 8;
 #define NATSL_SM(KK, VV)                                              \
@@ -1689,7 +1694,7 @@ extern "C" int natsl_softmax_sparse_fwd(const void* q, const void* k, const void
                                         const natsl_seq_row* seqs, int n_seqs, int total_units,
                                         natsl_stream_t stream) {
   return softmax_fwd(q, k, v, o, lse, types, types_dtype, nats_block_indices, n_nats_blocks, B, T, HQ, HKV, HN, K, V, TN, block,
-                     scale, same_block_visible, dtype, seqs, n_seqs, total_units, stream, true, nullptr);
+                     scale, same_block_visible, dtype, seqs, n_seqs, total_units, stream, SOFTMAX_ENTRY, nullptr);
 }
 
 extern "C" int natsl_softmax_sparse_fwd_per_tile(const void* q, const void* k, const void* v, void* o, float* lse,
@@ -1699,12 +1704,18 @@ extern "C" int natsl_softmax_sparse_fwd_per_tile(const void* q, const void* k, c
                                                  const natsl_seq_row* seqs, int n_seqs, int total_units,
                                                  natsl_stream_t stream) {
   return softmax_fwd(q, k, v, o, lse, types, types_dtype, nats_block_indices, n_nats_blocks, B, T, HQ, HKV, HN, K, V, TN, block,
-                     scale, same_block_visible, dtype, seqs, n_seqs, total_units, stream, false, nullptr);
+                     scale, same_block_visible, dtype, seqs, n_seqs, total_units, stream, SOFTMAX_PER_TILE, nullptr);
 }
 
-extern "C" int natsl_softmax_fwd_variant(int B, int T, int HQ, int HKV, int block, int packed) {
+static int variant_of(int B, int T, int HQ, int HKV, int block, int packed, SoftmaxUse use) {
   const StreamDevice* sd = nullptr;
   int rc;
-  const int variant = softmax_variant(B, T, HQ, HKV, block, packed != 0, true, packed, &sd, &rc);
+  const int variant = softmax_variant(B, T, HQ, HKV, block, packed != 0, use, packed, &sd, &rc);
   return variant < 0 ? rc : variant;
+}
+extern "C" int natsl_softmax_fwd_variant(int B, int T, int HQ, int HKV, int block, int packed) {
+  return variant_of(B, T, HQ, HKV, block, packed, SOFTMAX_ENTRY);
+}
+extern "C" int natsl_mixed_softmax_variant(int B, int T, int HQ, int HKV, int block, int packed) {
+  return variant_of(B, T, HQ, HKV, block, packed, SOFTMAX_OPERATOR);
 }

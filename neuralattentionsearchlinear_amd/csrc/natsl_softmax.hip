@@ -1610,7 +1610,7 @@ static int launch_softmax_stream(const SoftmaxParams& p, const StreamDevice* d, 
 // tiles per CU).
 // Operators (the linear branch's scan runs beside it and hides a part of that): from six on whole tiles of 2048 queries or more and on
 // lengths from 6144 that cut a chunk.  Time of the whole operator, per tile / persistent, the four head shapes: whole tiles 0.79 - 1.02
-// at two, 0.86 - 1.02 at four, 0.92 - 1.03 at six, 0.94 - 1.04 at eight; cut lengths (6145 .. 33000) 0.87 - 1.02 at three, 0.91 - 1.07
+// at two (GDN B8 T2048 H8 64/64, 5 % attention: 85 us against 107), 0.86 - 1.02 at four, 0.92 - 1.03 at six, 0.94 - 1.04 at eight; cut lengths (6145 .. 33000) 0.87 - 1.02 at three, 0.91 - 1.07
 // at four, 0.94 - 1.09 at six, 0.96 - 1.08 at eight.
 // The entry by itself takes whole tiles of 2048 queries or more from two on and cut lengths from 6144 from three: its tests hold it at
 // these small problems (dealt out, cut lengths lose little there: 0.86 - 1.0 at three, 0.88 - 1.27 at four).

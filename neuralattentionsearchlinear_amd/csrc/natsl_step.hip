@@ -660,20 +660,37 @@ struct StepLayout {
   size_t proj, q_conv, q_lin, q_attn, o_lin, y, partials, logits, arrived, bytes;
 };
 
+// Workgroups of step_one_kernel that fit on the chip at once, less those of the logits and the recurrence: what its registers allow a CU
+// (195 - 228 with 192-wide states or 128-wide keys and values: two; 118 with 64-wide everything: four; else 147 - 168: three).
+static int step_one_slots(const natsl_layer_step& s, const int n_chunks) {
+  const int KA = s.H * s.K / s.HQ, VA = s.H * s.V / s.HQ;
+  const int per_cu = s.K == 192 || KA + VA == 256 ? 2 : KA + VA + s.K == 192 ? 4 : 3;
+  return per_cu * 256 - s.B * (n_chunks + s.H * cdiv(s.V, 64));
+}
+
 // One token a sequence: one launch between the two products.  That kernel is built for the layers' own convolution width and reads windows
-// and mixing rows 8 bytes at a time; a wave's lanes are its chunks of logits.
+// and mixing rows 8 bytes at a time; a wave's lanes are its chunks of logits.  With 128-wide attention values and more logits and
+// recurrence workgroups than fit at once the several launches are faster (340M geometry from 29 sequences, 760M from 13: mostly 0.89 - 1.0
+// of the time that the one launch takes at its best split, 1.09 at most, up to 64 sequences of 600 to 5000 cached tokens); with 64-wide
+// values the one launch is (0.89 - 1.0 of theirs, up to 64 sequences).
 static bool step_is_one(const natsl_layer_step& s, const int n_chunks) {
+  if (s.H * s.V == 128 * s.HQ && step_one_slots(s, n_chunks) < 0) return false;
   const uintptr_t at8 = (uintptr_t)s.conv_state_q | (uintptr_t)s.conv_state_k | (uintptr_t)s.conv_state_v | (uintptr_t)s.conv_out_q |
                         (uintptr_t)s.conv_out_k | (uintptr_t)s.conv_out_v | (uintptr_t)s.conv_wq | (uintptr_t)s.conv_wk | (uintptr_t)s.conv_wv |
                         (uintptr_t)s.w_mix;
   return s.T == 1 && s.conv_width == 4 && n_chunks <= 64 && at8 % 8 == 0;
 }
 
-// As many splits as leave all of the launch's workgroups resident at once (its registers allow three a CU, two with 192-wide states):
-// eight sequences of the 128/64 geometry above take 17.9 us in one round of 4 splits, 19.3 in two rounds of 8.
-static int step_one_splits(const natsl_layer_step& s, const int n_chunks, const int most) {
-  const int slots = (s.K == 192 ? 2 : 3) * 256 - s.B * (n_chunks + s.H * cdiv(s.V, 64));
-  return std::max(1, std::min(most, slots / (s.B * s.HQ)));
+// As many splits as leave all of the launch's workgroups resident at once, of 256 keys or more (two chunks a wave: 760M, one sequence,
+// 1333 tokens: a step of 24.5 us with 6 - 8 splits, 33 with 11).  Where that leaves fewer than four there is no one round to keep, and
+// what counts is that a wave walks few chunks one after the other: up to five splits of 768 keys (a step of 16 sequences of the 340M
+// geometry with 5421 cached tokens: 91 us with one split, 83 with five; 32 of the Mamba geometry with 3113: 129 and 113; five rather
+// than four or eight, which spread the heads worse over the XCDs).  Over seven geometries, 1 - 64 sequences and 400 - 10000 cached
+// tokens a step takes 1.015 times the best split's (geometric mean; 1.14 at most).
+static int step_one_splits(const natsl_layer_step& s, const int n_chunks) {
+  const int keys = s.n_kept * s.block + s.n_in + s.T, queries = s.B * s.HQ;
+  const int one_round = std::min({attend_splits(queries, keys), cdiv(keys, 256), step_one_slots(s, n_chunks) / queries});
+  return one_round >= 4 ? one_round : std::max({1, one_round, std::min(5, cdiv(keys, 768))});
 }
 
 static StepLayout step_layout(const natsl_layer_step& s) {
@@ -686,8 +703,7 @@ static StepLayout step_layout(const natsl_layer_step& s) {
   l.tiles = l.ldp / 16;
   l.n_chunks = cdiv(KD, LOGIT_CHUNK);
   l.one = step_is_one(s, l.n_chunks);
-  l.nsplit = attend_splits(M * s.HQ, s.n_kept * s.block + s.n_in + s.T);
-  if (l.one) l.nsplit = step_one_splits(s, l.n_chunks, l.nsplit);
+  l.nsplit = l.one ? step_one_splits(s, l.n_chunks) : attend_splits(M * s.HQ, s.n_kept * s.block + s.n_in + s.T);
   size_t at = 0;
   auto take = [&](size_t n) { const size_t r = at; at += (n + 255) / 256 * 256; return r; };
   l.proj = take((size_t)M * l.ldp * 2);

@@ -93,6 +93,10 @@ def test_layer_step_matches_the_general_path(kind, geometry, ops, B, T0, sizes, 
     ('mamba', 2, 95, 3, dict(head_dim=64, expand_v=1, num_heads=18, num_attn_heads=18)),   # more heads than a wave's four rounds of four
     ('mamba', 1, 127, 2, dict(expand_v=1)),
     ('mamba', 1, 257, 2, dict(attn_with_short_conv=False, conv_bias=True)),
+    ('mamba', 16, 2100, 2, dict(num_heads=16, num_attn_heads=16)),                    # more workgroups than fit at once: three splits
+    ('gdn', 16, 3000, 2, dict(num_heads=6, num_attn_heads=12)),
+    ('gdn', 8, 1300, 2, dict(num_heads=6, num_attn_heads=12)),                        # all of them fit: four splits
+    ('gdn', 30, 1200, 1, dict(num_heads=6, num_attn_heads=12)),                       # 128-wide values, too many: the several launches
 ])
 def test_layer_step_of_one_token(kind, B, T0, n, more, monkeypatch):
     """The launch that does everything between the products of a one-token step, at the edges of its chunks, splits and heads."""

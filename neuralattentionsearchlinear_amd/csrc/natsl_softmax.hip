@@ -996,9 +996,9 @@ NATSL_DEVICE unsigned xcc_id() {
 // change); its chunks past the end are requested from the tile's first chunk and nobody takes part in them, the chunk that the end
 // cuts (marked in the chunk table: all bits of its row inverted) repeats the last row, waves behind the end stay idle, and rows
 // behind it are not stored.  The tile of a cut chunk keeps the per-tile kernel's fp32 row sums (taken from the rounded probabilities,
-// its log-sum-exp was off by 1.6e-4 on average and 1.4e-3 at most, against 4e-7 and 1.5e-6).  Against a workgroup per tile: B8 T4095 H12 64/128 half attention 264 -> 212 us, B8 T8191 H16 128/128
-// 729 -> 661, B4 T8191 H32 128/64 593 -> 557, B4 T4095 H32 64/64 181 -> 161; four packed sequences of 65536 tokens in all, H32
-// 128/128, 1410 -> 1280.
+// its log-sum-exp was off by 1.6e-4 on average and 1.4e-3 at most, against 4e-7 and 1.5e-6).  Against a workgroup per tile, an
+// operator's launch by itself: B8 T4095 H12 64/128 half attention 251 -> 223 us, B8 T8191 H16 128/128 684 -> 636, B4 T8191 H32 128/64
+// 557 -> 505, B4 T4095 H32 64/64 181 -> 171; four packed sequences of 65536 tokens in all, H32 128/128, 1211 -> 1113.
 template <int DK, int DV, bool RAGGED, bool DEALT>
 __global__ __launch_bounds__(512, 1) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {

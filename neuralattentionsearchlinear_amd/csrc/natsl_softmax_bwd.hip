@@ -800,8 +800,9 @@ __global__ __launch_bounds__(256, DKDV_WHOLE_WGS) void dkdv_whole_kernel(const S
 }
 
 // ---------------------------------------------------------------------------------------------
-// dk/dv for K = V = 128, where a wave cannot hold both operands and both accumulators.  Eight waves = 2 roles x 2 key halves x 2 query halves; a wave and its partner of the other role (wave + 4, on
-// the same SIMD) work on the same 32 keys x 32 queries of every step:
+// dk/dv for K = V = 128, where a wave cannot hold both operands and both accumulators, and for every width below DKDV_WHOLE_CHUNKS
+// chunks per CU.  Eight waves = 2 roles x 2 key halves x 2 query halves; a wave and its partner of the other role (wave + 4, on the same
+// SIMD) work on the same 32 keys x 32 queries of every step:
 //   role 0: S = Q K^T, P = exp2(S c - lse) (masks, the clamp for blocks that only give dnats), dV^T += dO^T P
 //   role 1: dP = dO V^T, dS = P (dP - delta), dK^T += Q^T dS, dnats
 // P goes from role 0 to role 1 in fp32 through LDS (two buffers, written before the step's barrier and read after it).
@@ -1233,7 +1234,8 @@ static int launch_bwd(const SoftmaxBwdParams& p, hipStream_t stream) {
   static std::atomic<unsigned long long> reserved{0};
   auto roles = [&] { return dkdv(dkdv_kernel<DK, DV>, reserved, DkdvLds<DK, DV>::TOTAL, 512, 1); };   // the ring of three query tiles and the exchange buffers
   int rc;
-  // (192: both operands, both accumulators and a quarter's scores fit the 256 registers that two waves a SIMD leave)
+  // (192: both operands, both accumulators and a quarter's scores fit the 256 registers that two waves a SIMD leave; at K 64, V 128 seven
+  // or eight values that only a unit's start and end need lie in scratch memory, written once and read once a unit, none in its steps)
   if constexpr (DK + DV <= 192) {
     static std::atomic<unsigned long long> reserved_whole{0}, reserved_invalid{0};
     constexpr size_t lds = DkdvWholeLds<DK, DV>::TOTAL;

@@ -353,8 +353,11 @@ NATSL_DEVICE float wave_sum(float x) {
   return x;
 }
 
-// Everything that the wave handed over (stores that write through) has arrived before the lane with `on` counts it in; the
-// returned mask has the lanes that were their counter's last.
+// Everything that the wave handed over (stores that write through) has arrived before the lane with `on` counts it in.  What orders the two
+// is this machine, not the language: the atomics are relaxed, s_waitcnt vmcnt(0) holds the count back until every lane's
+// write-through store has been acknowledged by the memory that all XCDs see, the empty asm statements keep the compiler from moving
+// accesses across, and the last arriver's loads (ld_agent) go past its own L2.  Release and acquire would write back and drop whole L2s.
+// The returned mask has the lanes that were their counter's last.
 NATSL_DEVICE unsigned long long arrive(const StepOne& p, const int b, const int hq, const bool on, const int expected) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   unsigned before = 0u;

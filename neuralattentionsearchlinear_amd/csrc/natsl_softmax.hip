@@ -1608,10 +1608,14 @@ static int launch_softmax_stream(const SoftmaxParams& p, const StreamDevice* d, 
 // K = V = 64, the high ends half attention and lengths that cut a chunk.  So it takes eight tiles' worth of queries per CU.  Where
 // sequences are shorter than a tile, what it does for the missing queries costs more than it saves (100 queries: 0.42 - 0.8 up to 16
 // tiles per CU).
-// Operators (the linear branch's scan runs beside it and hides a part of that): from six on whole tiles of 2048 queries or more and on
-// lengths from 6144 that cut a chunk.  Time of the whole operator, per tile / persistent, the four head shapes: whole tiles 0.79 - 1.02
-// at two (GDN B8 T2048 H8 64/64, 5 % attention: 85 us against 107), 0.86 - 1.02 at four, 0.92 - 1.03 at six, 0.94 - 1.04 at eight; cut lengths (6145 .. 33000) 0.87 - 1.02 at three, 0.91 - 1.07
-// at four, 0.94 - 1.09 at six, 0.96 - 1.08 at eight.
+// Operators (the linear branch's scan runs beside it and hides a part of that), time of the whole operator, per tile / persistent, seven
+// head shapes and both published geometries: whole tiles of 2048 queries or more 0.79 - 1.03 at two tiles per CU (GDN B8 T2048 H8 64/64,
+// 5 % attention: 85 us against 107), 0.86 - 1.03 at four, 0.92 - 1.04 at six: six.  Lengths from 6144 that cut a chunk, 0.87 - 1.02 at
+// three, 0.91 - 1.02 at four, 0.94 - 1.03 at six: six; where the last tile has more than half of its queries, which the per-tile
+// kernel takes its slow way through, 0.90 - 1.04 at three, 0.95 - 1.08 at four: four.  But a per-tile workgroup stays on the XCD of its
+// (sequence, head) pair, and persistent ones take what the others have left: where the pairs leave a tenth or more of the XCDs' last
+// round empty (9 to 36 of them, not a multiple of 8), two and three: 0.91 - 1.17 and 0.95 - 1.16, mostly above 1 (760M geometry B1
+// T12392, 18 pairs, half attention, 3.4 tiles per CU: 1.12).
 // The entry by itself takes whole tiles of 2048 queries or more from two on and cut lengths from 6144 from three: its tests hold it at
 // these small problems (dealt out, cut lengths lose little there: 0.86 - 1.0 at three, 0.88 - 1.27 at four).
 // Of the others, one workgroup per tile, of 256 queries on 8 waves once there is at least one such tile per compute unit (measured:
@@ -1625,7 +1629,9 @@ static int softmax_variant(int B, int T, int HQ, int HKV, int block, bool packed
     const long long tiles = (long long)B * HQ * T / 256;   // whole tiles' worth of queries
     const bool whole = !packed && T % 256 == 0 && T >= 2048;
     const bool cut = !packed && T % 64 && T >= 6144;
-    const long long line = use == SOFTMAX_OPERATOR ? (whole || cut ? 6 : 8) : whole ? 2 : cut ? 3 : 8;
+    const int pairs = B * HQ;
+    const bool even = use == SOFTMAX_OPERATOR && cdiv(pairs, 8) * 80 < 11 * pairs;
+    const long long line = whole ? (even ? 6 : 2) : cut ? (even ? (T % 256 > 128 ? 4 : 6) : 3) : 8;
     if (tiles >= line * d->cus && T / (packed ? n_seqs : 1) >= 256) {
       *sd = d;
       return NATSL_SOFTMAX_PERSISTENT;

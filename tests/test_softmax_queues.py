@@ -83,11 +83,11 @@ def test_an_operators_queues_are_in_its_own_workspace(fake_hip, B, T, H, n_seqs)
         assert [n for n, _, _ in short] == ["stream_queue_clear", "softmax_stream"] and short[0][2] == short[1][2] and short[0][2] < WORKSPACE
 
 
-@pytest.mark.parametrize("T,per_cu", [(2048, 6), (4096, 6), (65536, 6), (8191, 6), (32769, 6), (3000, 8), (4160, 8), (512, 8)])
+@pytest.mark.parametrize("T,per_cu", [(2048, 6), (4096, 6), (16384, 6), (8191, 4), (32769, 6), (3000, 8), (4160, 8), (512, 8)])
 def test_operators_take_the_persistent_kernel_from_their_own_line_on(fake_hip, T, per_cu):  # noqa: F811
-    """Six tiles' worth of queries per CU on long whole or cut lengths, eight on others (256 CUs), whatever the softmax entry by itself is
-    held to by its tests."""
-    H = 4
+    """Six tiles' worth of queries per CU on long whole or cut lengths (four where the last tile is more than half full), eight on others
+    (256 CUs), whatever the softmax entry by itself is held to by its tests."""
+    H = 8
     from neuralattentionsearchlinear_amd import _capi
     calls, first = [], -(-per_cu * 256 * 256 // (H * T))                # batches that reach the line, and the largest that does not
     for B in (first - 1, first):
@@ -95,6 +95,16 @@ def test_operators_take_the_persistent_kernel_from_their_own_line_on(fake_hip, T
         calls.append(_mixed(B, T, H, 0, need))
     below, at = _launches(fake_hip, calls)
     assert [r[0] for r in below] == ["softmax_sparse"] and [r[0] for r in at] == ["stream_queue_clear", "softmax_stream"]
+
+
+@pytest.mark.parametrize("B,T,H,kernel", [
+    (1, 8192, 18, "softmax_stream"), (1, 12392, 18, "softmax_stream"), (1, 16385, 12, "softmax_stream"), (4, 4096, 9, "softmax_stream"),
+    (1, 8192, 24, "softmax_sparse"), (1, 12392, 24, "softmax_sparse"), (5, 4096, 9, "softmax_sparse"), (1, 4096, 18, "softmax_sparse")])
+def test_operators_with_pairs_that_leave_xcds_idle_take_it_earlier(fake_hip, B, T, H, kernel):  # noqa: F811
+    """(sequence, head) pairs that do not divide over the eight XCDs: from two tiles per CU on whole tiles, three on cut lengths."""
+    from neuralattentionsearchlinear_amd import _capi
+    (rows,) = _launches(fake_hip, [_mixed(B, T, H, 0, _capi.lib().natsl_mixed_workspace_bytes(B * -(-T // 64), H))])
+    assert rows[-1][0] == kernel
 
 
 def test_only_whole_tile_launches_of_the_softmax_entry_take_slots(fake_hip):  # noqa: F811

@@ -1614,10 +1614,10 @@ static int launch_softmax_stream(const SoftmaxParams& p, const StreamDevice* d, 
 // three, 0.91 - 1.02 at four, 0.94 - 1.03 at six: six; where the last tile has more than half of its queries, which the per-tile
 // kernel takes its slow way through, 0.90 - 1.04 at three, 0.95 - 1.08 at four: four.  But a per-tile workgroup stays on the XCD of its
 // (sequence, head) pair, and persistent ones take what the others have left: where the pairs leave a tenth or more of the XCDs' last
-// round empty (9 to 36 of them, not a multiple of 8), two and three: 0.91 - 1.17 and 0.95 - 1.16, mostly above 1 (760M geometry B1
+// round empty (9 to 36 of them, not a multiple of 8), two and three: 0.91 - 1.16 and 0.92 - 1.16, mostly above 1 (760M geometry B1
 // T12392, 18 pairs, half attention, 3.4 tiles per CU: 1.12).
 // The entry by itself takes whole tiles of 2048 queries or more from two on and cut lengths from 6144 from three: its tests hold it at
-// these small problems (dealt out, cut lengths lose little there: 0.86 - 1.0 at three, 0.88 - 1.27 at four).
+// these small problems (dealt out, cut lengths lose little there: 0.86 - 1.05 at three, 0.91 - 1.27 at four).
 // Of the others, one workgroup per tile, of 256 queries on 8 waves once there is at least one such tile per compute unit (measured:
 // from there on that shape is the faster one; below, 128-query tiles, two workgroups of four waves a CU, fill more compute units).
 static int softmax_variant(int B, int T, int HQ, int HKV, int block, bool packed, SoftmaxUse use, int n_seqs, const StreamDevice** sd, int* rc) {
@@ -1629,8 +1629,8 @@ static int softmax_variant(int B, int T, int HQ, int HKV, int block, bool packed
     const long long tiles = (long long)B * HQ * T / 256;   // whole tiles' worth of queries
     const bool whole = !packed && T % 256 == 0 && T >= 2048;
     const bool cut = !packed && T % 64 && T >= 6144;
-    const int pairs = B * HQ;
-    const bool even = use == SOFTMAX_OPERATOR && cdiv(pairs, 8) * 80 < 11 * pairs;
+    const long long pairs = (long long)B * HQ;
+    const bool even = use == SOFTMAX_OPERATOR && (pairs + 7) / 8 * 80 < 11 * pairs;
     const long long line = whole ? (even ? 6 : 2) : cut ? (even ? (T % 256 > 128 ? 4 : 6) : 3) : 8;
     if (tiles >= line * d->cus && T / (packed ? n_seqs : 1) >= 256) {
       *sd = d;

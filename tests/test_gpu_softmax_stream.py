@@ -16,11 +16,11 @@ def _inputs(B, T, HQ, H, HN, K, V, block, p_attn, seed, dev):
     return q, k, v, ty, q.to(dev), k.to(dev), v.to(dev), ty.to(dev)
 
 
-def _call(qd, kd, vd, tyd, K, block, same_block, persistent=True):
+def _call(qd, kd, vd, tyd, K, block, same_block, persistent=True, seqs=None):
     """The softmax branch through the C ABI: natsl_softmax_sparse_fwd (picks the persistent kernel for these shapes), or
     natsl_softmax_sparse_fwd_per_tile (one workgroup per query tile, the same results)."""
     from neuralattentionsearchlinear_amd import _capi, nats_util
-    r = nats_util.route(tyd, qd.shape[1], block)
+    r = nats_util.route(tyd, qd.shape[1], block, seqs)
     B, T, HQ, _ = qd.shape
     H, V = kd.shape[2], vd.shape[-1]
     TN, HN = tyd.shape[1], tyd.shape[2]
@@ -29,10 +29,11 @@ def _call(qd, kd, vd, tyd, K, block, same_block, persistent=True):
     L = _capi.lib()
     fn = L.natsl_softmax_sparse_fwd if persistent else L.natsl_softmax_sparse_fwd_per_tile
     if persistent:
-        assert L.natsl_softmax_fwd_variant(B, T, HQ, H, block, 0) == 2, "shape does not reach the persistent kernel on this GPU"
+        assert L.natsl_softmax_fwd_variant(B, T, HQ, H, block, seqs.n_seqs if seqs else 0) == 2, "shape does not reach the persistent kernel on this GPU"
     rc = fn(_capi.ptr(qd), _capi.ptr(kd), _capi.ptr(vd), _capi.ptr(o), _capi.ptr(lse), _capi.ptr(tyd), _capi.dtype_code(tyd.dtype),
             _capi.ptr(r['nats_block_indices']), _capi.ptr(r['n_nats_blocks']), B, T, HQ, H, HN, K, V, TN, block, float(K ** -0.5),
-            int(bool(same_block)), _capi.dtype_code(qd.dtype), None, 0, 0, _capi.stream_ptr(qd.device))
+            int(bool(same_block)), _capi.dtype_code(qd.dtype), *((_capi.ptr(seqs.table), seqs.n_seqs, seqs.total_qtiles) if seqs else (None, 0, 0)),
+            _capi.stream_ptr(qd.device))
     _capi.check(rc, "natsl_softmax_sparse_fwd")
     return o, lse
 
@@ -148,19 +149,26 @@ def test_persistent_kernel_on_packed_sequences(lens, K, V, H, block, same_block)
 
 
 @pytest.mark.parametrize("K,V", [(128, 128), (64, 64), (64, 128), (128, 64)])
-@pytest.mark.parametrize("T", [769, 831, 897, 1023])
-def test_row_sums_of_a_cut_last_tile_are_fp32(K, V, T):
+@pytest.mark.parametrize("T,packed", [(769, False), (831, False), (897, False), (1023, False), (831, True)])
+def test_row_sums_of_a_cut_last_tile_are_fp32(K, V, T, packed):
     """The log-sum-exp of the tile that a sequence's end cuts inside a chunk, against 64-bit arithmetic on the scaled bf16 queries that
     the kernel multiplies.  With fp32 probabilities in the sums it is off by the rounding of K products of a few units (K 2^-24 x 8 at
     most, 6e-5 for 128 aligned signs, 1.5e-6 seen) and of at most T additions whose partial sums are below 2^3 of the result; 1e-5 lies
     between that and probabilities rounded to bf16 (2^-9 each: 1.6e-4 on average, 5e-4 to 1.4e-3 at most)."""
     import math
+    from neuralattentionsearchlinear_amd import nats_util
     B, H, block, dev = 22, 32, 64, torch.device('cuda:0')
     g = torch.Generator(device=dev).manual_seed(T)
     q, k, v = (torch.randn(B, T, H, d, device=dev, generator=g).bfloat16() for d in (K, K, V))
     ty = make_types(B, -(-T // block), H, 0.4, 33, torch.bfloat16).to(dev)
+    one_row = lambda t: t.reshape(1, -1, *t.shape[2:])
     for persistent in (False, True):
-        _, lse = _call(q, k, v, ty, K, block, True, persistent)
+        if packed:
+            seqs = nats_util.pack_sequences([T * i for i in range(B + 1)], None, block, dev)
+            _, lse = _call(one_row(q), one_row(k), one_row(v), one_row(ty), K, block, True, persistent, seqs)
+            lse = lse.view(B, T, H)
+        else:
+            _, lse = _call(q, k, v, ty, K, block, True, persistent)
         b, whole = 3, T // 256 * 256
         scale = torch.tensor(K ** -0.5, dtype=torch.float32, device=dev) * 1.4426950408889634
         qs = (q[b].float() * scale).bfloat16().double()

@@ -81,6 +81,12 @@ int natsl_hard_select(const void* logits, void* types, int32_t* n_nats_blocks, i
                       int dtype, int force_last, const natsl_seq_row* seqs, int n_seqs,
                       int total_units, natsl_stream_t stream);
 
+/* What a layer's forward takes from its logits [B,TN,HN,2], in one launch: natsl_hard_select's types with the last block of every
+ * sequence forced, the types before that (raw_types, or NULL), n_nats_blocks [B,HN,2], and attn_fraction [HN] fp32, the attention
+ * blocks' share of all blocks (src/nats/layers/natsl_attn_gdn.py:553-554). */
+int natsl_layer_select(const void* logits, void* types, void* raw_types, int32_t* n_nats_blocks, float* attn_fraction, int B, int TN, int HN,
+                       int dtype, natsl_stream_t stream);
+
 /* Routing tables derived from types [B,TN,HN,2] (values rounded as the reference does at
  * src/nats/ops/mixed_ops/mixed_attn_gdn.py:88).  Any output may be NULL.
  *   nats_block_indices   int32 [B,TN,HN,2]   ascending ids of selected blocks, padded with TN
@@ -398,6 +404,25 @@ int natsl_kv_collect(const void* src_k, const void* src_v, long long src_tokens,
 int natsl_kv_counts(const void* types, int types_dtype, const int64_t* n_before, int64_t* n_after, int32_t* host_max, int B, int HN, int NB,
                     int n_complete, natsl_stream_t stream);
 int natsl_kv_flags(const int64_t* n_after, uint8_t* valid, int B, int blocks, int HN, int tail_block, natsl_stream_t stream);
+/* natsl_kv_flags, and g_sum [B, H] = the sum of g [B, T, H] over the last `rest` tokens (fp32; 0 for none). */
+int natsl_kv_note(const int64_t* n_after, uint8_t* valid, int B, int blocks, int HN, int tail_block, const float* g, float* g_sum, int T, int H,
+                  int rest, natsl_stream_t stream);
+
+/* The incomplete block's rows of a cache that was empty: for each of n tensors, dst [B, block, row] = the last `rest` tokens of
+ * src [B, T, row] and zeros behind them (dense, row_bytes a token). */
+#define NATSL_TAIL_SEGS 8
+typedef struct natsl_tail_seg {
+  const void* src;
+  void* dst;
+  int64_t row_bytes;
+} natsl_tail_seg;
+int natsl_block_tails(const natsl_tail_seg* segs, int n, int B, int T, int block, int rest, natsl_stream_t stream);
+
+/* out [B, H, state_elems] = ht where the last block's type is linear (last_types: element [b, hn, 1] at b * stride_b + hn * stride_h + 1),
+ * else hs, times exp(gs [B, H]) unless gs is NULL: the state the next block starts from when the input ends on a block's end
+ * (src/nats/ops/gated_delta_rule/chunk_fwd.py:178-206). */
+int natsl_roll_state(const float* ht, const float* hs, const float* gs, const void* last_types, int types_dtype, int64_t stride_b, int64_t stride_h,
+                     float* out, int B, int H, int HN, int64_t state_elems, natsl_stream_t stream);
 
 /* The layers' short convolutions with what follows them, for up to NATSL_CONV_SEGS bf16 tensors [B, T, D_i] in one launch:
  *   y = act(conv(x)) (as natsl_short_conv_fwd; bf16 weights [D, W]), and, when y_norm is given, its rows of 8 * norm_lanes

@@ -25,6 +25,7 @@ _SIGNATURES = {
     "natsl_last_error": (c_char_p, []),
     "natsl_mean_pool": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_void_p]),
     "natsl_hard_select": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_void_p]),
+    "natsl_layer_select": (c_int, [c_void_p] * 5 + [c_int] * 4 + [c_void_p]),
     "natsl_route": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
                             c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p]),
     "natsl_softmax_sparse_fwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
@@ -84,6 +85,9 @@ _SIGNATURES = {
     "natsl_kv_collect": (c_int, [c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_longlong, c_void_p] + [c_int] * 12 + [c_void_p]),
     "natsl_kv_counts": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p] + [c_int] * 4 + [c_void_p]),
     "natsl_kv_flags": (c_int, [c_void_p, c_void_p] + [c_int] * 4 + [c_void_p]),
+    "natsl_kv_note": (c_int, [c_void_p] * 2 + [c_int] * 4 + [c_void_p] * 2 + [c_int] * 3 + [c_void_p]),
+    "natsl_block_tails": (c_int, [c_void_p] + [c_int] * 5 + [c_void_p]),
+    "natsl_roll_state": (c_int, [c_void_p] * 4 + [c_int, c_int64, c_int64, c_void_p] + [c_int] * 3 + [c_int64, c_void_p]),
     "natsl_conv_norm_fwd": (c_int, [c_void_p] + [c_int] * 6 + [c_void_p]),
     "natsl_conv_norm_bwd_workspace_bytes": (c_size_t, [c_void_p] + [c_int] * 4),
     "natsl_conv_norm_bwd": (c_int, [c_void_p] + [c_int] * 6 + [c_void_p, c_size_t, c_void_p]),

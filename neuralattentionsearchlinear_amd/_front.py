@@ -306,25 +306,36 @@ class _Tail(torch.autograd.Function):
 
 
 # ---- selector ------------------------------------------------------------------------------------------------------------------------
+def _select(logits, want_raw):
+    """-> (types with the last block forced, counts, attention's share per head, types before that or None)."""
+    logits = logits.contiguous()
+    B, TN, HN, _ = logits.shape
+    types, raw = torch.empty_like(logits), torch.empty_like(logits) if want_raw else None
+    counts = torch.empty(B, HN, 2, dtype=torch.int32, device=logits.device)
+    fraction = torch.empty(HN, dtype=torch.float32, device=logits.device)
+    rc = _capi.lib().natsl_layer_select(logits.data_ptr(), types.data_ptr(), _p(raw), counts.data_ptr(), fraction.data_ptr(), B, TN, HN,
+                                        _capi.dtype_code(logits.dtype), _capi.stream_ptr(logits.device))
+    _capi.check(rc, "natsl_layer_select")
+    return types, counts, fraction, raw
+
+
 class _Select(torch.autograd.Function):
     """Hard selection with the straight-through gradient; the last block, forced to both ops, has none."""
 
     @staticmethod
-    def forward(ctx, logits, force_last):
-        from .nats_util import hard_select
-        types, counts = hard_select(logits.detach(), force_last_block=force_last)
+    def forward(ctx, logits, want_raw):
+        types, counts, fraction, raw = _select(logits.detach(), want_raw)
         ctx.save_for_backward(logits)
-        ctx.force = force_last
-        ctx.mark_non_differentiable(counts)
-        return types, counts
+        ctx.mark_non_differentiable(counts, fraction, *((raw,) if want_raw else ()))
+        return types, counts, fraction, raw
 
     @staticmethod
-    def backward(ctx, dtypes, _):
+    def backward(ctx, dtypes, *_):
         (logits,) = ctx.saved_tensors
         lg, d = logits.contiguous(), dtypes.to(logits.dtype).contiguous()
         out = torch.empty_like(lg)
         B, TN, HN, _ = lg.shape
-        rc = _capi.lib().natsl_hard_select_bwd(lg.data_ptr(), d.data_ptr(), out.data_ptr(), B, TN, HN, _capi.dtype_code(lg.dtype), int(ctx.force),
+        rc = _capi.lib().natsl_hard_select_bwd(lg.data_ptr(), d.data_ptr(), out.data_ptr(), B, TN, HN, _capi.dtype_code(lg.dtype), 1,
                                                _capi.stream_ptr(lg.device))
         _capi.check(rc, "natsl_hard_select_bwd")
         return out, None
@@ -363,11 +374,10 @@ class FastFront:
             return _Gates.apply(self, ab, self.w["a_log"], self.w["dt_bias"])
         return _gates(self, ab)
 
-    def select(self, logits, force_last):
-        if self.grad(logits):
-            return _Select.apply(logits, force_last)
-        from .nats_util import hard_select
-        return hard_select(logits, force_last_block=force_last)
+    def select(self, logits, want_raw):
+        """-> (types with the last block forced, counts, attention's share per head, types before that: the forced ones unless wanted)."""
+        types, counts, fraction, raw = _Select.apply(logits, want_raw) if self.grad(logits) else _select(logits, want_raw)
+        return types, counts, fraction, raw if want_raw else types
 
     def tail(self, o_lin, o_attn, gate, logits):
         args = (o_lin.contiguous(), o_attn.contiguous(), gate.contiguous(), logits.contiguous())

@@ -368,11 +368,18 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
         else:
             if op_type_last_chunk is None:
                 raise AssertionError("op_type_last_chunk is required when the input ends on a block boundary")
-            H = ht.shape[1]
-            lin = (op_type_last_chunk[..., 1] > 0)
-            lin = lin.repeat_interleave(H // lin.shape[1], dim=1).view(ht.shape[0], H, 1, 1)
-            rolled = hs * torch.exp(gs).view(ht.shape[0], H, 1, 1) if decay_non_linear else hs
-            h_start = torch.where(lin, ht, rolled)
+            last, n = op_type_last_chunk, ht.shape[0]
+            if last.is_cuda and last.device == dev and last.dtype in (torch.bfloat16, torch.float32) and last.dim() == 3 and last.shape[0] == n and \
+                    last.stride(2) == 1 and H % last.shape[1] == 0 and last.shape[2] > 1 and n * H <= 65535:
+                h_start = torch.empty_like(ht)
+                rc = L.natsl_roll_state(ht.data_ptr(), hs.data_ptr(), gs.data_ptr() if decay_non_linear else None, last.data_ptr(),
+                                        _capi.dtype_code(last.dtype), last.stride(0), last.stride(1), h_start.data_ptr(), n, H, last.shape[1], K * V, cur)
+                _capi.check(rc, "natsl_roll_state")
+            else:
+                lin = (last[..., 1] > 0)
+                lin = lin.repeat_interleave(H // lin.shape[1], dim=1).view(n, H, 1, 1)
+                rolled = hs * torch.exp(gs).view(n, H, 1, 1) if decay_non_linear else hs
+                h_start = torch.where(lin, ht, rolled)
     return o_lin, o_attn, ht, h_start
 
 

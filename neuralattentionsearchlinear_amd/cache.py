@@ -17,6 +17,7 @@ blocks, so the cache never holds the blocks the selector dropped.
 """
 from __future__ import annotations
 
+import ctypes
 import threading
 from typing import Any, Dict, List, Optional, Tuple
 
@@ -47,6 +48,27 @@ class _HostNumbers:
 
 
 _host_numbers = _HostNumbers()
+
+
+class _TailSeg(ctypes.Structure):
+    _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p), ("row_bytes", ctypes.c_int64)]
+
+
+def _block_tails(tensors, block: int, rest: int):
+    """For each x [B, T, ...] of `tensors`: a new tensor [B, block, ...] with the last `rest` tokens of x and zeros behind them, all of
+    them in one launch; None where a tensor is not what that launch reads (the caller fills and copies then)."""
+    for x in tensors:
+        if not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float32) or not x.is_contiguous() or x.device != tensors[0].device or \
+                x.shape[:2] != tensors[0].shape[:2] or x.numel() == 0 or (x.requires_grad and torch.is_grad_enabled()):
+            return None
+    x = tensors[0]
+    B, T = x.shape[:2]
+    out = [torch.empty(B, block, *t.shape[2:], dtype=t.dtype, device=t.device) for t in tensors]
+    segs = (_TailSeg * len(tensors))()
+    for s, t, o in zip(segs, tensors, out):
+        s.src, s.dst, s.row_bytes = t.data_ptr(), o.data_ptr(), t.numel() // (B * T) * t.element_size()
+    _capi.check(_capi.lib().natsl_block_tails(segs, len(segs), B, T, block, rest, _capi.stream_ptr(x.device)), "natsl_block_tails")
+    return out
 
 
 class NAtSLayerCache:
@@ -96,9 +118,14 @@ class NAtSLayerCache:
         (src/nats/models/utils.py:178-207)."""
         B, T, D = input_hidden_states.shape
         bs, n_in = self.nats_block_size, self._n_tokens_in_nats_block
-        if self.block_type_state is None:
-            self.block_type_state = torch.zeros(B, bs, D, dtype=input_hidden_states.dtype, device=input_hidden_states.device)
         total = n_in + T
+        if self.block_type_state is None:
+            if n_in == 0 and total >= bs:
+                made = _block_tails((input_hidden_states,), bs, total % bs)
+                if made is not None:
+                    self.block_type_state = made[0]
+                    return input_hidden_states
+            self.block_type_state = torch.zeros(B, bs, D, dtype=input_hidden_states.dtype, device=input_hidden_states.device)
         if total < bs:
             self.block_type_state[:, n_in:total] = input_hidden_states
             return None
@@ -201,6 +228,15 @@ class NAtSLayerCache:
         k, v = lattn_state
         T, bs, n_in = k.shape[1], self.nats_block_size, self._n_tokens_in_nats_block
         fresh = self.l_attn_k is None
+        if fresh and T >= bs and v.dtype == k.dtype:
+            made = _block_tails([t for t in (k, v, lattn_beta, lattn_g) if t is not None], bs, T % bs)
+            if made is not None:
+                self.l_attn_k, self.l_attn_v = made[:2]
+                if lattn_beta is not None:
+                    self.lattn_beta = made[2]
+                if lattn_g is not None:
+                    self.lattn_g = made[-1]
+                return k, v, lattn_beta, lattn_g
         if fresh:
             B, _, H, _ = k.shape
             self.l_attn_k = torch.zeros(B, bs, H, k.shape[3], dtype=k.dtype, device=k.device)
@@ -228,8 +264,9 @@ class NAtSLayerCache:
         return out
 
     # ------------------------------------------------------------------------------------------------
-    def _compact(self, nats_block_types: torch.Tensor, attn_state, n_complete: int, tail_tokens: int):
-        """Keep the attention-typed complete blocks of the region of new tokens; returns nothing, updates counts."""
+    def _compact(self, nats_block_types: torch.Tensor, attn_state, n_complete: int, tail_tokens: int, g: Optional[torch.Tensor] = None):
+        """Keep the attention-typed complete blocks of the region of new tokens; updates counts and, given the tokens' g, its sum over
+        the incomplete block."""
         bs = self.nats_block_size
         types = nats_block_types
         if types.dtype not in (torch.float32, torch.bfloat16):
@@ -275,8 +312,18 @@ class NAtSLayerCache:
         self.n_attn_blocks_max = new_max
         blocks = self.attn_k.shape[1] // bs
         self.valid_attn_tokens = torch.empty(B, blocks, HN, dtype=torch.bool, device=after.device)
-        rc = _capi.lib().natsl_kv_flags(_capi.ptr(after), _capi.ptr(self.valid_attn_tokens), B, blocks, HN, tail_dst, _capi.stream_ptr(after.device))
-        _capi.check(rc, "natsl_kv_flags")
+        flags = (_capi.ptr(after), _capi.ptr(self.valid_attn_tokens), B, blocks, HN, tail_dst)
+        if g is None:
+            _capi.check(L.natsl_kv_flags(*flags, _capi.stream_ptr(after.device)), "natsl_kv_flags")
+        elif g.is_cuda and g.dtype == torch.float32 and g.is_contiguous() and g.dim() == 3 and g.shape[0] == B and g.shape[1] >= max(tail_tokens, 1) and \
+                g.shape[2] > 0 and g.device == after.device and not (g.requires_grad and torch.is_grad_enabled()):
+            self.g_cumsum = torch.empty(B, 1, g.shape[2], dtype=torch.float32, device=g.device)
+            rc = L.natsl_kv_note(*flags, g.data_ptr(), self.g_cumsum.data_ptr(), g.shape[1], g.shape[2], tail_tokens, _capi.stream_ptr(after.device))
+            _capi.check(rc, "natsl_kv_note")
+        else:
+            _capi.check(L.natsl_kv_flags(*flags, _capi.stream_ptr(after.device)), "natsl_kv_flags")
+            self.g_cumsum = g[:, -tail_tokens:].sum(1, keepdim=True) if tail_tokens else torch.zeros(g.shape[0], 1, g.shape[2], dtype=g.dtype,
+                                                                                                     device=g.device)
 
     def _count(self, key, types, n_complete: int):
         """Enqueue the kept-block counts after this update; -> (key, n_complete, counts, the largest one's place on the host, event)."""
@@ -332,12 +379,9 @@ class NAtSLayerCache:
             if NB != _cdiv(total, bs):
                 raise ValueError(f"nats_block_types holds {NB} blocks, the cached and new tokens make {_cdiv(total, bs)}")
             rest = total % bs
-            self._compact(nats_block_types, attn_state, NB - 1 if rest else NB, rest)
+            self._compact(nats_block_types, attn_state, NB - 1 if rest else NB, rest, g)
             self._n_tokens_in_nats_block = rest
             self.n_attn_tokens_max = self.n_attn_blocks_max * bs + rest
-            if g is not None:
-                self.g_cumsum = g[:, -rest:].sum(1, keepdim=True) if rest else torch.zeros(g.shape[0], 1, g.shape[2], dtype=g.dtype,
-                                                                                           device=g.device)
         else:
             if self.attn_k is None:
                 # fewer tokens than one block on an empty cache: they are the incomplete block

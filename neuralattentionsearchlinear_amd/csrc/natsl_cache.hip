@@ -146,12 +146,75 @@ __global__ __launch_bounds__(1024) void kv_counts_kernel(const void* types, cons
     __threadfence_system();
   }
 }
-// valid[b][i][hn]: kept blocks, and the incomplete block at `tail` (-1: none)
-__global__ __launch_bounds__(256) void kv_flags_kernel(const int64_t* after, uint8_t* valid, const long long n, const int HN, const int blocks, const int tail) {
-  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  const int hn = (int)(i % HN), blk = (int)(i / HN % blocks), b = (int)(i / ((long long)HN * blocks));
-  valid[i] = blk < after[(size_t)b * HN + hn] || blk == tail;
+// valid[b][i][hn]: kept blocks, and the incomplete block at `tail` (-1: none).  The workgroups behind those of the flags, a wave per
+// (sequence, head) each, leave the sum of g [B, T, H] over the incomplete block's tokens (the last `rest`; 0 where there are none).
+__global__ __launch_bounds__(256) void kv_flags_kernel(const int64_t* after, uint8_t* valid, const long long n, const int HN, const int blocks, const int tail,
+                                                       const unsigned flag_wgs, const float* g, float* g_sum, const int B, const int T, const int H,
+                                                       const int rest) {
+  if (blockIdx.x < flag_wgs) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const int hn = (int)(i % HN), blk = (int)(i / HN % blocks), b = (int)(i / ((long long)HN * blocks));
+    valid[i] = blk < after[(size_t)b * HN + hn] || blk == tail;
+    return;
+  }
+  const long long pair = (long long)(blockIdx.x - flag_wgs) * 4 + (threadIdx.x >> 6);
+  if (pair >= (long long)B * H) return;
+  const int b = (int)(pair / H), h = (int)(pair % H);
+  float s = 0.f;
+  for (int t = threadIdx.x & 63; t < rest; t += 64) s += g[((size_t)b * T + T - rest + t) * H + h];
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) s += __shfl_xor(s, d);
+  if ((threadIdx.x & 63) == 0) g_sum[pair] = s;
+}
+
+// ---- a cache's first prompt -------------------------------------------------------------------------------------------------
+// dst [B, block, row] = the last `rest` tokens of src [B, T, row], zeros behind them, for several tensors in one launch: the incomplete
+// block's rows of a cache that was empty before.  Fills and strided copies of their own were eleven launches of a prompt (six where it
+// ends on a block's end), 4.7 us each where the GPU is the limit and about 10 us of host time.  `unit`: bytes a thread moves, what the
+// row's length and the addresses allow.
+struct TailParams {
+  natsl_tail_seg seg[NATSL_TAIL_SEGS];
+  int unit[NATSL_TAIL_SEGS];
+  unsigned first[NATSL_TAIL_SEGS + 1];   // the segments' first workgroups
+  int n, B, T, block, rest;
+};
+template <typename U>
+NATSL_DEVICE void tail_unit(const natsl_tail_seg& s, const long long i, const TailParams& p) {
+  const int per_row = (int)(s.row_bytes / sizeof(U));
+  const long long token = i / per_row;
+  const int at = (int)(i - token * per_row), b = (int)(token / p.block), t = (int)(token - (long long)b * p.block);
+  if (b >= p.B) return;
+  U x{};
+  if (t < p.rest) x = reinterpret_cast<const U*>(s.src)[((size_t)b * p.T + p.T - p.rest + t) * per_row + at];
+  reinterpret_cast<U*>(s.dst)[i] = x;
+}
+__global__ __launch_bounds__(256) void block_tails_kernel(const TailParams p) {
+  int k = 0;
+  while (k + 1 < p.n && blockIdx.x >= p.first[k + 1]) ++k;
+  const long long i = (long long)(blockIdx.x - p.first[k]) * 256 + threadIdx.x;
+  if (p.unit[k] == 16) tail_unit<u32x4>(p.seg[k], i, p);
+  else if (p.unit[k] == 4) tail_unit<unsigned>(p.seg[k], i, p);
+  else tail_unit<uint16_t>(p.seg[k], i, p);
+}
+
+// The state that the next block starts from where a prompt ends on a block's end: the final state where the last block's own type is
+// linear, else the state that entered it, decayed by the block's g where asked for (src/nats/ops/gated_delta_rule/chunk_fwd.py:178-206).
+__global__ __launch_bounds__(256) void roll_state_kernel(const float* ht, const float* hs, const float* gs, const void* last, const int dtype,
+                                                         const long long stride_b, const long long stride_h, float* out, const int H, const int HN,
+                                                         const int n4) {
+  const int b = blockIdx.y / H, h = blockIdx.y % H;
+  const long long at = b * stride_b + (h / (H / HN)) * stride_h + 1;
+  const float t = dtype == NATSL_F32 ? reinterpret_cast<const float*>(last)[at] : bf16_to_f32(reinterpret_cast<const bf16_t*>(last)[at]);
+  const bool linear = t > 0.f;
+  const float f = linear || !gs ? 1.f : expf(gs[blockIdx.y]);
+  const f32x4* src = reinterpret_cast<const f32x4*>(linear ? ht : hs) + (size_t)blockIdx.y * n4;
+  f32x4* dst = reinterpret_cast<f32x4*>(out) + (size_t)blockIdx.y * n4;
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n4; i += gridDim.x * 256) {
+    f32x4 x = src[i];
+    x *= f;
+    dst[i] = x;
+  }
 }
 
 }  // namespace natsl
@@ -223,12 +286,66 @@ extern "C" int natsl_kv_counts(const void* types, int types_dtype, const int64_t
   return check_launch(what);
 }
 
-extern "C" int natsl_kv_flags(const int64_t* n_after, uint8_t* valid, int B, int blocks, int HN, int tail_block, natsl_stream_t stream) {
-  const char* what = "natsl_kv_flags";
+static int kv_flags(const char* what, const int64_t* n_after, uint8_t* valid, int B, int blocks, int HN, int tail_block, const float* g, float* g_sum,
+                    int T, int H, int rest, natsl_stream_t stream) {
   if (!n_after || !valid) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
   if (B <= 0 || HN <= 0 || blocks <= 0) return fail(NATSL_ERR_INVALID, "%s: non-positive dimension", what);
   const long long n = (long long)B * blocks * HN;
-  hipLaunchKernelGGL(kv_flags_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), n_after, valid, n, HN, blocks,
-                     tail_block);
+  const unsigned flag_wgs = (unsigned)((n + 255) / 256), sum_wgs = g_sum ? (unsigned)(((long long)B * H + 3) / 4) : 0u;
+  hipLaunchKernelGGL(kv_flags_kernel, dim3(flag_wgs + sum_wgs), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), n_after, valid, n, HN, blocks,
+                     tail_block, flag_wgs, g, g_sum, B, T, H, rest);
+  return check_launch(what);
+}
+
+extern "C" int natsl_kv_flags(const int64_t* n_after, uint8_t* valid, int B, int blocks, int HN, int tail_block, natsl_stream_t stream) {
+  return kv_flags("natsl_kv_flags", n_after, valid, B, blocks, HN, tail_block, nullptr, nullptr, 0, 0, 0, stream);
+}
+
+extern "C" int natsl_kv_note(const int64_t* n_after, uint8_t* valid, int B, int blocks, int HN, int tail_block, const float* g, float* g_sum, int T, int H,
+                             int rest, natsl_stream_t stream) {
+  const char* what = "natsl_kv_note";
+  if (!g || !g_sum) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
+  if (T <= 0 || H <= 0 || rest < 0 || rest > T) return fail(NATSL_ERR_INVALID, "%s: %d of %d tokens, %d heads", what, rest, T, H);
+  return kv_flags(what, n_after, valid, B, blocks, HN, tail_block, g, g_sum, T, H, rest, stream);
+}
+
+extern "C" int natsl_block_tails(const natsl_tail_seg* segs, int n, int B, int T, int block, int rest, natsl_stream_t stream) {
+  const char* what = "natsl_block_tails";
+  if (!segs) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
+  if (n <= 0 || n > NATSL_TAIL_SEGS) return fail(NATSL_ERR_INVALID, "%s: %d tensors (1 to %d)", what, n, NATSL_TAIL_SEGS);
+  if (B <= 0 || T <= 0 || block <= 0 || rest < 0 || rest > T || rest > block)
+    return fail(NATSL_ERR_INVALID, "%s: B=%d T=%d block=%d rest=%d", what, B, T, block, rest);
+  TailParams p{};
+  long long wgs = 0;
+  for (int i = 0; i < n; ++i) {
+    const natsl_tail_seg& s = segs[i];
+    if (!s.src || !s.dst) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
+    const size_t bits = (size_t)s.src | (size_t)s.dst | (size_t)s.row_bytes;
+    if (s.row_bytes <= 0 || s.row_bytes > (1ll << 30) || bits % 2)
+      return fail(NATSL_ERR_UNSUPPORTED, "%s: rows of %lld bytes at odd places", what, (long long)s.row_bytes);
+    p.seg[i] = s;
+    p.unit[i] = bits % 16 == 0 ? 16 : bits % 4 == 0 ? 4 : 2;
+    p.first[i] = (unsigned)wgs;
+    wgs += ((long long)B * block * (s.row_bytes / p.unit[i]) + 255) / 256;
+    if (wgs >= (1ll << 31)) return fail(NATSL_ERR_UNSUPPORTED, "%s: too many rows", what);
+  }
+  p.first[n] = (unsigned)wgs;
+  p.n = n; p.B = B; p.T = T; p.block = block; p.rest = rest;
+  hipLaunchKernelGGL(block_tails_kernel, dim3((unsigned)wgs), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), p);
+  return check_launch(what);
+}
+
+extern "C" int natsl_roll_state(const float* ht, const float* hs, const float* gs, const void* last_types, int types_dtype, int64_t stride_b,
+                                int64_t stride_h, float* out, int B, int H, int HN, int64_t state_elems, natsl_stream_t stream) {
+  const char* what = "natsl_roll_state";
+  if (!ht || !hs || !last_types || !out) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
+  if (B <= 0 || H <= 0 || HN <= 0 || H % HN || state_elems <= 0 || (long long)B * H > 65535)
+    return fail(NATSL_ERR_INVALID, "%s: B=%d H=%d HN=%d", what, B, H, HN);
+  if (types_dtype != NATSL_BF16 && types_dtype != NATSL_F32) return fail(NATSL_ERR_UNSUPPORTED, "%s: block types must be f32 or bf16", what);
+  if (state_elems % 4 || state_elems >= (1ll << 31) || ((size_t)ht | (size_t)hs | (size_t)out) % 16)
+    return fail(NATSL_ERR_UNSUPPORTED, "%s: states must be multiples of four elements, aligned to 16 bytes", what);
+  const int n4 = (int)(state_elems / 4);
+  hipLaunchKernelGGL(roll_state_kernel, dim3((unsigned)cdiv(n4, 256 * 8), (unsigned)(B * H)), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), ht, hs, gs,
+                     last_types, types_dtype, (long long)stride_b, (long long)stride_h, out, H, HN, n4);
   return check_launch(what);
 }

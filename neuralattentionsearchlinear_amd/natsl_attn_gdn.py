@@ -227,9 +227,8 @@ class NeuralAttentionSearchLinearAttnGDN(nn.Module):
             if not whole:
                 pooled = nats_util.mean_pooling(selector_input, self.nats_block_size)
             logits = self.nats_layer(pooled).unflatten(-1, (self.num_nats_head, self.n_ops))
-            types, n_nats_blocks = fast.select(logits, True)
             # (the types before the last block is forced are only needed where states are handed on)
-            raw_types = fast.select(logits, False)[0] if use_cache or cache is not None else types
+            types, n_nats_blocks, attn_fraction, raw_types = fast.select(logits, bool(use_cache) or cache is not None)
             if cache is not None:
                 cache.foresee(raw_types, q_len)
             q, k, v, q_attn, k_attn, o_mix, _, _, v_attn, new_conv_states = fast.conv_norm(q, k, v, conv_states, bool(use_cache))
@@ -278,7 +277,7 @@ class NeuralAttentionSearchLinearAttnGDN(nn.Module):
                 types = raw_types.clone()
                 types[:, -1] = 1
                 n_nats_blocks = types.to(torch.int32).sum(1)
-            self.attn_fraction = n_nats_blocks[..., 0].sum(0).float() / (types.shape[1] * B)
+            self.attn_fraction = attn_fraction if fast is not None else n_nats_blocks[..., 0].sum(0).float() / (types.shape[1] * B)
             if self.training:
                 o_lin, o_attn, state = nats_mixed_attn_gdn(
                     initial_state_gated_delta=state, nats_block_types=types, n_nats_blocks=n_nats_blocks,

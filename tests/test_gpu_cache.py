@@ -269,3 +269,52 @@ def test_a_cache_made_in_new_memory(T, block, K, V, dtype):
     _capi.check(L.natsl_kv_compact(P(k), P(v), T, 0, P(want[0]), P(want[1]), cap, *head, None, *rest), "natsl_kv_compact")
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T,rest", [(64, 0), (777, 9), (127, 63)])
+@pytest.mark.parametrize("dtype,inner", [(torch.bfloat16, (3, 64)), (torch.bfloat16, (1,)), (torch.float32, (6,)), (torch.float32, (5, 12)), (torch.bfloat16, (8, 2))])
+def test_block_tails(T, rest, dtype, inner):
+    """Rows of 2, 12, 24, 32, 240 and 384 bytes (moved 2, 4 or 16 at a time), next to each other in one launch, against copies."""
+    from neuralattentionsearchlinear_amd import cache
+    torch.manual_seed(T)
+    xs = [torch.randn(3, T, *s, device=DEV).to(d) for s, d in (((4, 64), torch.bfloat16), (inner, dtype), ((6,), torch.bfloat16))]
+    for x, got in zip(xs, cache._block_tails(xs, 64, rest)):
+        want = torch.zeros(3, 64, *x.shape[2:], dtype=x.dtype, device=DEV)
+        if rest:
+            want[:, :rest] = x[:, -rest:]
+        assert torch.equal(got, want)
+    assert cache._block_tails([xs[0], xs[0].transpose(0, 1)], 64, rest) is None
+    assert cache._block_tails([xs[0].half()], 64, rest) is None
+
+
+@pytest.mark.parametrize("H,HN,K,V,decay,dtype", [(6, 6, 128, 256, True, torch.bfloat16), (4, 2, 64, 16, True, torch.float32), (3, 1, 192, 384, False, torch.bfloat16)])
+def test_rolled_state(H, HN, K, V, decay, dtype):
+    """The state the next block starts from, bit for bit what torch's exp, product and choice give."""
+    from neuralattentionsearchlinear_amd import _capi
+    torch.manual_seed(H)
+    ht, hs, gs = torch.randn(2, H, K, V, device=DEV), torch.randn(2, H, K, V, device=DEV), -torch.rand(2, H, device=DEV) * 20
+    last = (torch.rand(2, 5, HN, 2, device=DEV) > 0.5).to(dtype)[:, -1]
+    out = torch.full_like(ht, float('nan'))
+    rc = _capi.lib().natsl_roll_state(ht.data_ptr(), hs.data_ptr(), gs.data_ptr() if decay else None, last.data_ptr(), _capi.dtype_code(dtype), last.stride(0),
+                                      last.stride(1), out.data_ptr(), 2, H, HN, K * V, _capi.stream_ptr(ht.device))
+    _capi.check(rc, "natsl_roll_state")
+    lin = (last[..., 1] > 0).repeat_interleave(H // HN, 1).view(2, H, 1, 1)
+    assert torch.equal(out, torch.where(lin, ht, hs * torch.exp(gs).view(2, H, 1, 1) if decay else hs))
+
+
+@pytest.mark.parametrize("T,rest", [(64, 0), (200, 8), (127, 63), (2047, 1023)])
+def test_kept_block_notes(T, rest):
+    """The validity flags, and the sum of g over the incomplete block: 1e-6 of the terms' sum is ten fp32 roundings of it."""
+    from neuralattentionsearchlinear_amd import _capi
+    torch.manual_seed(T)
+    B, HN, H, blocks = 3, 2, 5, 7
+    after = torch.randint(0, 6, (B, HN), device=DEV)
+    g, out = -torch.rand(B, T, H, device=DEV), torch.full((B, 1, H), float('nan'), device=DEV)
+    valid = torch.empty(B, blocks, HN, dtype=torch.bool, device=DEV)
+    rc = _capi.lib().natsl_kv_note(after.data_ptr(), valid.data_ptr(), B, blocks, HN, 5 if rest else -1, g.data_ptr(), out.data_ptr(), T, H, rest,
+                                   _capi.stream_ptr(g.device))
+    _capi.check(rc, "natsl_kv_note")
+    at = torch.arange(blocks, device=DEV).view(1, -1, 1)
+    assert torch.equal(valid, (at < after.unsqueeze(1)) | (at == (5 if rest else -1)))
+    want = g[:, T - rest:].double().sum(1, keepdim=True)
+    assert float((out.double() - want).abs().max()) <= 1e-6 * max(rest, 1)

@@ -97,3 +97,19 @@ def test_route_known_answer():
     assert got['linear_chunk_offsets'].tolist() == [0, 2]
     assert got['starting_h_idx'][0, :, 0].tolist() == [0, 0, 1, 1]
     assert got['attn_n_iters'][0, :, 0].tolist() == [0, 1]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,TN,HN", [(1, 1, 1), (3, 1025, 2), (513, 3, 5), (8, 64, 6)])     # around a workgroup's threads and sequences
+def test_layer_select(B, TN, HN, dtype):
+    """One launch gives what the two selections and torch's arithmetic on the counts give, bit for bit."""
+    from neuralattentionsearchlinear_amd import _front, nats_util
+    g = torch.Generator().manual_seed(B)
+    logits = torch.randn(B, TN, HN, 2, generator=g).to(dtype)
+    raw = R.hard_select(logits)
+    forced = R.force_last_block(raw)
+    for want in (True, False):
+        types, counts, fraction, before = _front._select(logits.to(_dev()), want)
+        assert torch.equal(types.cpu(), forced) and torch.equal(counts.cpu(), R.n_blocks(forced))
+        assert torch.equal(before.cpu(), raw) if want else before is None
+        assert torch.equal(fraction, nats_util.hard_select(logits.to(_dev()), True)[1][..., 0].sum(0).float() / (TN * B))

@@ -475,6 +475,17 @@ size_t natsl_wgrad_workspace_bytes(const natsl_wgrad_seg* segs, int n_seg, int64
 int natsl_wgrad(const natsl_wgrad_seg* segs, int n_seg, const void* x, int64_t T, int D, int ldx, void* workspace,
                 size_t workspace_bytes, natsl_stream_t stream);
 
+/* The wide products of up to NATSL_PROJECT_SEGS projections that share their input, one launch, bf16 with fp32 sums and one rounding.
+ * natsl_project: y_i [rows, ld_i] (n_i columns written) = x [rows, ldx] w_i^T, w_i [n_i, D] contiguous; D a multiple of 32 from 128 on.
+ * natsl_project_bwd: dx [B*T, D] = sum_i dy_i w_i + the block mean's gradient dpool [B, ceil(T/block), D] (or NULL) over the block's
+ * length; every n_i a multiple of 32, 128 or more in all.  Widths and row strides are multiples of
+ * 8, tensors start on 16 bytes; nothing else is taken.  (src/nats/layers/natsl_attn_gdn.py:425-491) */
+#define NATSL_PROJECT_SEGS 8
+typedef struct natsl_project_seg { const void* y; const void* w; int32_t n, ld; } natsl_project_seg;
+int natsl_project(const natsl_project_seg* segs, int n_seg, const void* x, int64_t rows, int D, int ldx, natsl_stream_t stream);
+int natsl_project_bwd(const natsl_project_seg* segs, int n_seg, const void* dpool, void* dx, int B, int T, int D, int block,
+                      natsl_stream_t stream);
+
 /* The mixed operator's forward (src/nats/ops/mixed_ops/mixed_attn_gdn.py:47-191, src/nats/ops/mixed_ops/mixed_attn_mamba.py:51-192)
  * in one call: natsl_route, natsl_softmax_sparse_fwd and natsl_gdn_chunk_fwd (is_delta) or natsl_mamba_chunk_fwd with the
  * arguments those take, in bf16, and in front of and behind them the conversions of fp32 tensors (cast_in: fp32 -> bf16,

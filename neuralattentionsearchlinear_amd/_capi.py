@@ -96,6 +96,8 @@ _SIGNATURES = {
     "natsl_gates_bwd": (c_int, [c_void_p] * 6 + [c_int] + [c_void_p] * 4 + [c_size_t, c_int64] + [c_int] * 4 + [c_void_p]),
     "natsl_dx_init": (c_int, [c_void_p] * 4 + [c_int] * 6 + [c_void_p]),
     "natsl_hard_select_bwd": (c_int, [c_void_p] * 3 + [c_int] * 5 + [c_void_p]),
+    "natsl_project": (c_int, [c_void_p, c_int, c_void_p, c_int64, c_int, c_int, c_void_p]),
+    "natsl_project_bwd": (c_int, [c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 4 + [c_void_p]),
     "natsl_wgrad_workspace_bytes": (c_size_t, [c_void_p, c_int, c_int64, c_int]),
     "natsl_wgrad": (c_int, [c_void_p, c_int, c_void_p, c_int64, c_int, c_int, c_void_p, c_size_t, c_void_p]),
     "natsl_mixed_softmax_variant": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int]),

@@ -9,6 +9,7 @@ weight-gradient products that split the tokens (natsl_wgrad), and launches.
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 import torch.nn.functional as F
@@ -19,11 +20,15 @@ from .modules import _NORM_GATE_WIDTHS
 
 _NAMES = [p[0] for p in _PARAMS]
 _EITHER = {"norm_q", "norm_k", "a_log", "dt_bias", "out_norm1", "out_norm2"}
-_ab_rows = lambda n: -(-n // 16) * 16
+_ab_rows = lambda n: -(-n // 32) * 32
 
 
 class _WgradSeg(ctypes.Structure):
     _fields_ = [("dy", ctypes.c_void_p), ("out", ctypes.c_void_p), ("n", ctypes.c_int32), ("ld", ctypes.c_int32)]
+
+
+class _ProjectSeg(ctypes.Structure):
+    _fields_ = [("y", ctypes.c_void_p), ("w", ctypes.c_void_p), ("n", ctypes.c_int32), ("ld", ctypes.c_int32)]
 
 
 class _ConvSeg(ctypes.Structure):
@@ -84,9 +89,42 @@ def linear(x, w):
 
 
 # ---- the projections of one input -----------------------------------------------------------------------------------------------
+@functools.lru_cache(maxsize=512)
+def _joint_pays(rows, D, widths, cus):
+    """Whether one launch for all projections (natsl_project) beats the library's products one by one: where it takes fewer rounds of
+    256 x 256 tiles over the CUs.  Measured (one by one / joint, us): 340M geometry 8 x 4096 tokens, 10 / 9 rounds: 273-318 / 265-289;
+    760M 8 x 2048, 10 / 7: 352 / 303; 760M 1 x 4096, 4 / 2: 109 / 81; but Mamba 4 x 8192, 12 / 12: 325 / 366.  Short prompts
+    take one round either way and the library's four launches: 1 x 777 78 / 16."""
+    tiles = [-(-rows // 256) * -(-n // 256) for n in widths]
+    return D % 32 == 0 and D >= 128 and all(n % 8 == 0 for n in widths) and -(-sum(tiles) // cus) < sum(-(-t // cus) for t in tiles)
+
+
+def _project_segs(ys, ws):
+    segs = (_ProjectSeg * len(ys))()
+    for s, y, w in zip(segs, ys, ws):
+        s.y, s.w, s.n, s.ld = y.data_ptr(), w.data_ptr(), w.shape[0], y.shape[-1]
+    return segs
+
+
+def _on_16(*tensors):
+    return not any(t.data_ptr() & 15 for t in tensors)
+
+
+def _wide(x, ws):
+    """[F.linear(x, w) for w in ws]"""
+    D = x.shape[-1]
+    rows = x.numel() // D
+    cus = torch.cuda.get_device_properties(x.device).multi_processor_count
+    if not _joint_pays(rows, D, tuple([w.shape[0] for w in ws]), cus) or not _on_16(x, *ws):
+        return [F.linear(x, w) for w in ws]
+    ys = [torch.empty(*x.shape[:-1], w.shape[0], dtype=x.dtype, device=x.device) for w in ws]
+    _capi.check(_capi.lib().natsl_project(_project_segs(ys, ws), len(ws), x.data_ptr(), rows, D, D, _capi.stream_ptr(x.device)), "natsl_project")
+    return ys
+
+
 def _project(x, wq, wk, wv, wg, wa, wb, pool_block):
     """-> ((q, k, v, gate, ab, block means or None), the joint weight of a and b).  The narrow projections share one product: their
-    rows and enough others to make whole tiles of 16 (the columns behind a and b are never read)."""
+    rows and enough others to make whole stages of 32 (the columns behind a and b are never read)."""
     narrow = (wa,) if wb is None else (wa, wb)
     used = sum(w.shape[0] for w in narrow)
     wab = torch.cat(narrow + (wq[:_ab_rows(used) - used],)) if used % 16 else torch.cat(narrow) if len(narrow) > 1 else wa
@@ -94,12 +132,12 @@ def _project(x, wq, wk, wv, wg, wa, wb, pool_block):
     if pool_block:
         from .nats_util import _mean_pooling_fwd
         pooled = _mean_pooling_fwd(x.unsqueeze(-2), pool_block, None).squeeze(-2)
-    return (F.linear(x, wq), F.linear(x, wk), F.linear(x, wv), F.linear(x, wg), F.linear(x, wab), pooled), wab
+    return (*_wide(x, (wq, wk, wv, wg)), F.linear(x, wab), pooled), wab
 
 
 class _Project(torch.autograd.Function):
-    """dx starts as what is no wide product (natsl_dx_init) and the four wide ones accumulate onto it; all weight gradients are one
-    launch."""
+    """dx is one launch (natsl_project_bwd), or starts as what is no wide product (natsl_dx_init) and the wide ones accumulate onto it;
+    all weight gradients are one launch."""
 
     @staticmethod
     def forward(ctx, x, wq, wk, wv, wg, wa, wb, pool_block):
@@ -121,6 +159,15 @@ class _Project(torch.autograd.Function):
         if need[0]:
             dx = torch.empty_like(x)
             dp = None if dpool is None else dpool.contiguous()
+            some = [(dy, w) for dy, w in zip(dys, (wq, wk, wv, wg, wab)) if dy is not None]
+            joint = sum(w.shape[0] for _, w in some) >= 128 and all(w.shape[0] % 32 == 0 for _, w in some) and \
+                _on_16(dx, *([] if dp is None else [dp]), *[t for pair in some for t in pair])
+        if need[0] and joint:
+            # one pass over dx where four accumulating products and dx_init made five (340M geometry, 8 x 4096 tokens: 412 -> 260 us)
+            rc = _capi.lib().natsl_project_bwd(_project_segs(*zip(*some)), len(some), _p(dp), dx.data_ptr(), B, T, D, ctx.block or T,
+                                               _capi.stream_ptr(x.device))
+            _capi.check(rc, "natsl_project_bwd")
+        elif need[0]:
             n = 0 if dys[4] is None else wab.shape[0]
             rc = _capi.lib().natsl_dx_init(_p(dys[4]), wab.data_ptr(), _p(dp), dx.data_ptr(), B, T, D, n, max(n, 16), ctx.block or T,
                                            _capi.stream_ptr(x.device))

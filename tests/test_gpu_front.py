@@ -201,3 +201,41 @@ def test_dx_init(B, T, D, N, block, pool):
         lens[-1] = T - (nb - 1) * block
         ref = ref + (dp.double() / lens.view(1, nb, 1)).repeat_interleave(block, 1)[:, :T]
     assert bool(((dx.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5).all())
+
+
+# (tokens, input width, projections): rows and columns behind the last tile, tiles of each height, more tiles than workgroups
+@pytest.mark.parametrize("B,T,D,widths,block", [
+    (1, 1, 128, (8,), 64), (1, 129, 160, (264, 32), 64), (3, 100, 416, (256, 64, 512, 32), 64), (2, 8200, 128, (520, 1024), 256),
+    (1, 16320, 768, (96, 32), 64), (1, 16320, 160, (512, 256), 64), (2, 8191, 1024, (64, 64), 128), (1, 40000, 264, (96, 128), 64), (1, 9000, 1032, (768, 768, 1536, 1536, 32), 64)])
+def test_joint_projections(B, T, D, widths, block):
+    """natsl_project and natsl_project_bwd: exact products, fp32 sums and one rounding to bf16."""
+    from neuralattentionsearchlinear_amd import _capi
+    from neuralattentionsearchlinear_amd._front import _project_segs
+    torch.manual_seed(T)
+    L, P, rows, nb = _capi.lib(), _capi.ptr, B * T, -(-T // block)
+    x, ws = torch.randn(rows, D, device=DEV).bfloat16(), [torch.randn(n, D, device=DEV).bfloat16() for n in widths]
+    close = lambda a, ref: bool(((a.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * sum(widths + (D,)) ** 0.5).all())
+    if D % 32 == 0:
+        guard = [torch.full((rows + 1, n), 7., device=DEV).bfloat16() for n in widths]
+        ys = [g[:rows] for g in guard]
+        _capi.check(L.natsl_project(_project_segs(ys, ws), len(ws), P(x), rows, D, D, _capi.stream_ptr(x.device)), "natsl_project")
+        for y, w, g in zip(ys, ws, guard):
+            assert close(y, x.double() @ w.double().t())
+            assert bool((g[rows] == 7).all())
+    else:
+        assert L.natsl_project(_project_segs([x], ws[:1]), 1, P(x), rows, D, D, _capi.stream_ptr(x.device)) != 0
+    dys = [torch.randn(rows, n, device=DEV).bfloat16() for n in widths]
+    dp = torch.randn(B, nb, D, device=DEV).bfloat16()
+    lens = torch.full((nb,), block, device=DEV, dtype=torch.float64)
+    lens[-1] = T - (nb - 1) * block
+    spread = (dp.double() / lens.view(1, nb, 1)).repeat_interleave(block, 1)[:, :T].reshape(rows, D)
+    for pool in (None, dp):
+        dx = torch.full((rows + 1, D), 7., device=DEV).bfloat16()
+        rc = L.natsl_project_bwd(_project_segs(dys, ws), len(ws), P(pool) if pool is not None else None, P(dx), B, T, D, block, _capi.stream_ptr(x.device))
+        if sum(widths) < 128 or any(n % 32 for n in widths):
+            assert rc != 0                                                  # (refused: the caller's other path)
+            continue
+        _capi.check(rc, "natsl_project_bwd")
+        ref = sum(dy.double() @ w.double() for dy, w in zip(dys, ws))
+        assert close(dx[:rows], ref if pool is None else ref + spread)
+        assert bool((dx[rows] == 7).all())

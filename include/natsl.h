@@ -44,7 +44,8 @@ enum natsl_flags {
   NATSL_QK_L2NORM = 2,        /* lattn_use_qk_l2norm_in_kernel */
   NATSL_INTRA_CHUNK = 4,      /* the linear op also scores its own incomplete block ('all', 'gated_delta_net', 'mamba') */
   NATSL_QUERY_ONLY = 8,       /* recurrent entries: outputs from the decayed block-start state, nothing updated ('attn') */
-  NATSL_FRESH_BLOCK_START = 16 /* recurrent entries: h_block_start is written only; the block starts from h0 (zeros if NULL) */
+  NATSL_FRESH_BLOCK_START = 16, /* recurrent entries: h_block_start is written only; the block starts from h0 (zeros if NULL) */
+  NATSL_STATES_ONLY = 32      /* chunked entries: no outputs (o is NULL), for a backward that forms chunk_states and chunk_v_new again */
 };
 
 /* One row per packed sequence (cu_seqlens / cu_seqlens_nats of the reference, plus prefix
@@ -177,7 +178,8 @@ size_t natsl_linear_workspace_bytes(int64_t total_chunks, int H);
  * uses it, bf16 [total_chunks][H][V][K] (total_chunks as for natsl_linear_workspace_bytes; the reference keeps the same
  * per-chunk states as `h`, src/nats/ops/common/chunk_delta_h.py:681-683); NULL = not stored.
  * chunk_v_new (optional, for a backward): the delta rule's corrected values v_new of every token, bf16 [B*T][H][V] (the
- * reference's `v_new`, chunk_delta_h.py:684); NULL = not stored.
+ * reference's `v_new`, chunk_delta_h.py:684); NULL = not stored.  With NATSL_STATES_ONLY o is NULL and chunk_states is not: q is read
+ * for the workspace only (the delta rule's P and norms).
  * The workspace is scratch between the entry's two kernels and its contents are the entry's own business, except after a call
  * with chunk_states: then it holds what natsl_linear_chunk_bwd reads (per chunk and head TmB, P and four scale vectors).  A
  * call without chunk_states may leave P out (a launch that fills the GPU forms it inside its second kernel).

@@ -16,7 +16,7 @@ LIB_PATH = os.path.join(_HERE, "csrc", "libnatsl.so")
 STEP_CORE_PATH = os.path.join(_HERE, "_step_core.so")
 
 F32, BF16 = 0, 1
-DECAY_NON_LINEAR, QK_L2NORM, INTRA_CHUNK, QUERY_ONLY, FRESH_BLOCK_START = 1, 2, 4, 8, 16
+DECAY_NON_LINEAR, QK_L2NORM, INTRA_CHUNK, QUERY_ONLY, FRESH_BLOCK_START, STATES_ONLY = 1, 2, 4, 8, 16, 32
 
 _lib = _step_core = None
 

@@ -199,7 +199,7 @@ def linear_chunk_backward_hip(kind, q, k, v, g, beta, h0, types, scale, block, d
             states, v_new, ws = saved
         else:
             _, _, states, v_new, ws = linear_chunk_fwd(kind, qb, kb, vb, gf, bb, h0f, ty, scale, block, flags, False, seqs,
-                                                       chunk_states=True)
+                                                       chunk_states=True, outputs=False)
         sp, ns, tot = _seq_args(seqs, NTtot)
         P, L, stream = _capi.ptr, _capi.lib(), _capi.stream_ptr(dev)
         gsum = torch.empty(B * NB, H, dtype=f32, device=dev)

@@ -108,11 +108,11 @@ def _wants_grad(*tensors) -> bool:
 
 def linear_chunk_fwd(kind: str, q, k, v, g, beta, h0, types, scale: float, block: int, flags: int,
                      output_final_state: bool, seqs: Optional[PackedSeqs], block_start_state: bool = False,
-                     chunk_states: bool = False):
+                     chunk_states: bool = False, outputs: bool = True):
     """Launch the chunked linear branch ('gdn' or 'mamba'); returns (o, final_state or None), or with
     block_start_state (o, final_state, state entering the last block, sum of g over the last block), or with chunk_states
     (o, final_state, the state entering every chunk as bf16 [total_chunks, H, V, K], v_new [B, T, H, V] (for 'mamba': v),
-    the workspace)."""
+    the workspace); with outputs=False (chunk_states only) o is None and costs nothing."""
     B, T, H, K = q.shape
     V = v.shape[-1]
     TN, HN = types.shape[1], types.shape[2]
@@ -121,7 +121,9 @@ def linear_chunk_fwd(kind: str, q, k, v, g, beta, h0, types, scale: float, block
     total_chunks = seqs.total_chunks if seqs is not None else B * (-(-T // CHUNK_SIZE))
     L = _capi.lib()
     ws = torch.empty(L.natsl_linear_workspace_bytes(total_chunks, H), dtype=torch.uint8, device=dev)
-    o = torch.empty(B, T, H, V, dtype=q.dtype, device=dev)
+    o = torch.empty(B, T, H, V, dtype=q.dtype, device=dev) if outputs else None
+    if not outputs:
+        flags |= _capi.STATES_ONLY
     ht = torch.empty(n, H, K, V, dtype=torch.float32, device=dev) if output_final_state else None
     hs = torch.empty(n, H, K, V, dtype=torch.float32, device=dev) if block_start_state else None
     gs = torch.empty(n, H, dtype=torch.float32, device=dev) if block_start_state else None

@@ -465,18 +465,19 @@ NATSL_DEVICE s16x4 lds_tr4_at(const unsigned addr) {
 }
 
 // LDS layout of the scan kernel: two or three stages and two output tiles.
-template <int DK, int NW, bool PF = false, bool XVEC = false>
+template <int DK, int NW, bool PF = false, bool XVEC = false, bool OUT = true, bool DELTA = true>
 struct ScanLds {
   static constexpr int BVW = 16 * NW;                 // state columns of the workgroup
   static constexpr int KROW = DK * 2;                 // bytes per k / q row
   static constexpr int VROW = BVW * 2;                // bytes per v row
   // (with PF, P is formed and used within one step: one area for all stages, behind them; XVEC: two more scale vectors arrive)
-  static constexpr int KB = 64 * KROW, VB = 64 * VROW, TB = 6 * 1024, PB = PF ? 0 : 6 * 1024, SCB = XVEC ? 2048 : 1024;
+  // (without outputs: no q, no P, no output tiles, for Mamba no TmB either)
+  static constexpr int KB = 64 * KROW, QB = OUT ? KB : 0, VB = 64 * VROW, TB = OUT || DELTA ? 6 * 1024 : 0, PB = PF || !OUT ? 0 : 6 * 1024, SCB = XVEC ? 2048 : 1024;
   static constexpr int PSHARED = PF ? 6 * 1024 : 0;
-  static constexpr int OFF_K = 0, OFF_Q = OFF_K + KB, OFF_V = OFF_Q + KB, OFF_T = OFF_V + VB, OFF_P = OFF_T + TB, OFF_SC = OFF_P + PB;
+  static constexpr int OFF_K = 0, OFF_Q = OFF_K + KB, OFF_V = OFF_Q + QB, OFF_T = OFF_V + VB, OFF_P = OFF_T + TB, OFF_SC = OFF_P + PB;
   static constexpr int STAGE = OFF_SC + SCB;
   static constexpr int OROW = VROW + 16;              // output tile row pitch (bytes)
-  static constexpr int OB = 64 * OROW;
+  static constexpr int OB = OUT ? 64 * OROW : 0;
   // Stages: chunk c lives in stage c % NSTAGE.  Three when they fit (narrow workgroups): the requests of chunk c + 2
   // are issued in step c and have a whole step more to land; two otherwise (requests of chunk c + 1 in step c).
   static constexpr int NSTAGE = 3 * STAGE + PSHARED + 2 * OB <= 160 * 1024 ? 3 : 2;
@@ -505,12 +506,16 @@ NATSL_DEVICE constexpr int tri_slot(const int t, const int s) { return t < 2 ? t
 // NF = 2 (with four compute waves): two more waves that do nothing but form P (waves NW + 2, NW + 3), so that this work sits on
 // the two SIMDs that host no data-movement wave; with NF = 0 the data-movement waves form P themselves (they have a SIMD of
 // their own when there are one or two compute waves).
-template <int DK, bool DELTA, int NW, bool PF, int NF = 0>
+// OUT = false: the states that enter the chunks and v_new only, for a backward that forms them again: q is not read, P neither read nor formed,
+// no output is formed or written, and the smaller stages leave room for three of them at every width.  By itself, with outputs and
+// without, us: Mamba B4 T8192 H32 128/64 285 -> 147, delta rule B8 T4096 H6 128/256 204 -> 146, B2 T3000 H6 192/384 126 -> 90.
+template <int DK, bool DELTA, int NW, bool PF, int NF = 0, bool OUT = true>
 __global__ NATSL_SCAN_ATTR(DK, NW + NF) void linear_scan_kernel(const LinearParams p) {
   static_assert(NF == 0 || (NF == 2 && PF), "the extra waves only form P");
   static_assert(!PF || !DELTA || NW == 4, "the delta rule's P is formed by the data-movement waves only in the four-wave shape");
-  static_assert(PF || DELTA, "the Mamba form's P is always formed by the data-movement waves");
-  using L = ScanLds<DK, NW, PF, PF && DELTA>;
+  static_assert(PF || DELTA || !OUT, "the Mamba form's P is always formed by the data-movement waves");
+  static_assert(OUT || !PF, "P is for the outputs");
+  using L = ScanLds<DK, NW, PF, PF && DELTA, OUT, DELTA>;
   constexpr int KS = DK / 32;   // matrix k-steps over the key dimension
   constexpr int KT = DK / 16;   // 16-row state tiles
   extern __shared__ __align__(1024) unsigned char smem[];
@@ -541,7 +546,7 @@ __global__ NATSL_SCAN_ATTR(DK, NW + NF) void linear_scan_kernel(const LinearPara
   // Output tile, TRANSPOSED in LDS: [column][64 tokens], rows of OT_ROW bytes: a compute lane writes the four tokens
   // 16 t + 4 g4 .. of its column with one 8-byte store; the data-movement wave reads it back with the transposing read.
   constexpr int OT_ROW = 2 * C + 16;
-  static_assert(L::BVW * OT_ROW <= L::OB, "the transposed output tile fits the space of the row-major one");
+  static_assert(!OUT || L::BVW * OT_ROW <= L::OB, "the transposed output tile fits the space of the row-major one");
 
   if (wave >= NW) {
     // ======================= the two data-movement waves ========================================================
@@ -563,7 +568,7 @@ __global__ NATSL_SCAN_ATTR(DK, NW + NF) void linear_scan_kernel(const LinearPara
     const char* kb = reinterpret_cast<const char*>(p.k + ((size_t)bos * p.H + h) * DK);
     const ptrdiff_t q_minus_k = reinterpret_cast<const char*>(p.q) - reinterpret_cast<const char*>(p.k);
     const char* vb = reinterpret_cast<const char*>(p.v + ((size_t)bos * p.H + h) * p.V + vcol0);
-    char* ob_g = reinterpret_cast<char*>(p.o + ((size_t)bos * p.H + h) * p.V + vcol0);
+    char* ob_g = OUT ? reinterpret_cast<char*>(p.o + ((size_t)bos * p.H + h) * p.V + vcol0) : nullptr;
     const size_t unit0 = (size_t)chunk_off * p.H + h;
     const char* tb = reinterpret_cast<const char*>(p.ws_tm + unit0 * (C * C));
     const ptrdiff_t p_minus_t = reinterpret_cast<const char*>(p.ws_p) - reinterpret_cast<const char*>(p.ws_tm);
@@ -610,8 +615,10 @@ __global__ NATSL_SCAN_ATTR(DK, NW + NF) void linear_scan_kernel(const LinearPara
         if (PF && DELTA) dma16(pb, 16u * lane, st + L::OFF_SC + 1024);   // the two exponent vectors (and 512 bytes nobody reads)
 #pragma unroll
         for (int u = 0; u < KQ_PIECES; ++u) dma16(kb, kq_off[u], st + L::OFF_K + 1024 * u);
+        if constexpr (OUT) {
 #pragma unroll
-        for (int u = 0; u < KQ_PIECES; ++u) dma16(qb, kq_off[u], st + L::OFF_Q + 1024 * u);
+          for (int u = 0; u < KQ_PIECES; ++u) dma16(qb, kq_off[u], st + L::OFF_Q + 1024 * u);
+        }
       } else {
 #pragma unroll
         for (int u = 0; u < V_PIECES; ++u) dma16(vb, v_off[u], st + L::OFF_V + 1024 * u);
@@ -619,7 +626,7 @@ __global__ NATSL_SCAN_ATTR(DK, NW + NF) void linear_scan_kernel(const LinearPara
 #pragma unroll
           for (int v = 0; v < 6; ++v) dma16(tb, ws_off[v], st + L::OFF_T + 1024 * v);
         }
-        if (DELTA && !PF) {
+        if (DELTA && !PF && OUT) {
 #pragma unroll
           for (int v = 0; v < 6; ++v) dma16(pb, ws_off[v], st + L::OFF_P + 1024 * v);
         }
@@ -665,7 +672,8 @@ __global__ NATSL_SCAN_ATTR(DK, NW + NF) void linear_scan_kernel(const LinearPara
     // stores issued after them) may still be in flight at the barrier: vector memory operations complete in the order
     // they were issued, so allowing as many outstanding as one step issues leaves exactly the older step's complete.
     constexpr int AHEAD = L::NSTAGE - 1;
-    constexpr int PER_STEP_FIRST = 1 + (PF && DELTA ? 1 : 0) + 2 * KQ_PIECES, PER_STEP_SECOND = V_PIECES + (DELTA ? (PF ? 6 : 12) : 0) + O_PASSES;
+    constexpr int PER_STEP_FIRST = 1 + (PF && DELTA ? 1 : 0) + (OUT ? 2 : 1) * KQ_PIECES;
+    constexpr int PER_STEP_SECOND = V_PIECES + (DELTA ? (PF || !OUT ? 6 : 12) : 0) + (OUT ? O_PASSES : 0);
     static_assert(PER_STEP_FIRST <= 63 && PER_STEP_SECOND <= 63, "the wait counter has six bits");
     constexpr int VM_FIRST = (PER_STEP_FIRST & 15) | ((PER_STEP_FIRST >> 4) << 14) | 0x0f70;
     constexpr int VM_SECOND = (PER_STEP_SECOND & 15) | ((PER_STEP_SECOND >> 4) << 14) | 0x0f70;
@@ -788,7 +796,7 @@ __global__ NATSL_SCAN_ATTR(DK, NW + NF) void linear_scan_kernel(const LinearPara
         // into the stage that step c - 1 read: every wave is past the barrier that ended it
         const bool more = c + AHEAD < NT;
         if (more) request(c + AHEAD);
-        if (c > 0 && !first) store_out(c - 1);
+        if (OUT && c > 0 && !first) store_out(c - 1);
         if (AHEAD == 2 && more) {
           if (first) __builtin_amdgcn_s_waitcnt(VM_FIRST);
           else __builtin_amdgcn_s_waitcnt(VM_SECOND);
@@ -798,7 +806,7 @@ __global__ NATSL_SCAN_ATTR(DK, NW + NF) void linear_scan_kernel(const LinearPara
         __syncthreads();
       }
     }
-    if (NT > 0 && !first && moves) store_out(NT - 1);
+    if (OUT && NT > 0 && !first && moves) store_out(NT - 1);
     return;
   }
 
@@ -881,14 +889,18 @@ __global__ NATSL_SCAN_ATTR(DK, NW + NF) void linear_scan_kernel(const LinearPara
 #pragma unroll
     for (int t = 0; t < 4; ++t) { R[t] = (f32x4){0.f, 0.f, 0.f, 0.f}; O1[t] = (f32x4){0.f, 0.f, 0.f, 0.f}; }
     {
-      constexpr int NOP = (DELTA ? 2 : 1) * 4 * KS, AHEAD = 4, NS = 4 * KT, PER = (NS + NOP - 1) / NOP;
+      constexpr int NOP = ((DELTA ? 1 : 0) + (OUT ? 1 : 0)) * 4 * KS, AHEAD = 4, NS = 4 * KT, PER = NOP ? (NS + NOP - 1) / (NOP ? NOP : 1) : 0;
+      if constexpr (NOP == 0) {
+#pragma unroll
+        for (int e = 0; e < NS; ++e) S[e >> 2][e & 3] *= dec_c;
+      }
       auto ld_op = [&](const int j) __attribute__((always_inline)) -> bf16x8 {
         const int which = DELTA ? j / (4 * KS) : 1, jj = j % (4 * KS), s = jj / 4, t = jj % 4;
         return *reinterpret_cast<lds_b128_t>(st + (which ? L::OFF_Q : L::OFF_K) + a_kq[s] + t * 16 * L::KROW);
       };
       bf16x8 opnd[NOP + AHEAD];
 #pragma unroll
-      for (int j = 0; j < AHEAD; ++j) opnd[j] = ld_op(j);
+      for (int j = 0; j < (NOP ? AHEAD : 0); ++j) opnd[j] = ld_op(j);
 #pragma unroll
       for (int j = 0; j < NOP; ++j) {
         if (j + AHEAD < NOP) opnd[j + AHEAD] = ld_op(j + AHEAD);
@@ -971,7 +983,7 @@ __global__ NATSL_SCAN_ATTR(DK, NW + NF) void linear_scan_kernel(const LinearPara
     }
     // (4) o = sq * O1 + P v_new, into the (transposed) output tile: the four token tiles side by side
     if constexpr (PF) __syncthreads();   // P and sq of this step are complete
-    {
+    if constexpr (OUT) {
       const unsigned ob = lds0 + L::OFF_OUT + (c & 1) * L::OB;
       f32x4 O[4];
       bf16x8 PA[6];
@@ -1059,10 +1071,10 @@ inline int cu_count_linear() {
   return n;
 }
 
-template <int DK, bool DELTA, int NW, bool PF, int NF = 0>
+template <int DK, bool DELTA, int NW, bool PF, int NF = 0, bool OUT = true>
 static int launch_scan(const LinearParams& p, hipStream_t stream, const char* what) {
-  using L = ScanLds<DK, NW, PF, PF && DELTA>;
-  auto kern = linear_scan_kernel<DK, DELTA, NW, PF, NF>;
+  using L = ScanLds<DK, NW, PF, PF && DELTA, OUT, DELTA>;
+  auto kern = linear_scan_kernel<DK, DELTA, NW, PF, NF, OUT>;
   static std::atomic<unsigned long long> reserved{0};
   if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, L::TOTAL, what)) return rc;
   const int n_chains = (p.seqs ? p.n_seqs : p.B) * p.H;
@@ -1112,6 +1124,11 @@ static int launch_linear(const LinearParams& p, hipStream_t stream, const Beside
   int rc = check_launch(what);
   if (rc == NATSL_OK && beside) rc = beside->ready(stream, beside->other, what);
   if (rc != NATSL_OK) return rc;
+  if (!p.o) {   // the chunk states only
+    if (nw == 4) return launch_scan<DK <= 128 ? DK : 128, DELTA, 4, false, 0, false>(p, stream, what);
+    if (nw == 2) return launch_scan<DK, DELTA, 2, false, 0, false>(p, stream, what);
+    return launch_scan<DK, DELTA, 1, false, 0, false>(p, stream, what);
+  }
   if constexpr (!DELTA) {
     // the Mamba form's P is always formed by the data-movement waves (nothing about it comes from a prep kernel)
     // (four compute waves: two of them share their SIMD with a data-movement wave, so two more waves, on the other two
@@ -1136,7 +1153,8 @@ int linear_fwd(bool delta, const void* q, const void* k, const void* v, const fl
                       int H, int HN, int K, int V, int TN, int block, float scale, int flags, void* workspace, size_t workspace_bytes,
                       int dtype, const natsl_seq_row* seqs, int n_seqs, int total_units, natsl_stream_t stream, const BesideScan* beside) {
   const char* what = delta ? "natsl_gdn_chunk_fwd" : "natsl_mamba_chunk_fwd";
-  if (!q || !k || !v || !g || !o || !types || (delta && !beta)) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
+  if (!q || !k || !v || !g || (!o && !(flags & NATSL_STATES_ONLY)) || !types || (delta && !beta)) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
+  if ((flags & NATSL_STATES_ONLY) && (!chunk_states || o)) return fail(NATSL_ERR_INVALID, "%s: states only: chunk_states and no output", what);
   if (dtype != NATSL_BF16) return fail(NATSL_ERR_UNSUPPORTED, "%s: only bf16 tensors are supported (got dtype %d)", what, dtype);
   if (types_dtype != NATSL_BF16 && types_dtype != NATSL_F32) return fail(NATSL_ERR_UNSUPPORTED, "%s: block types must be f32 or bf16", what);
   if (B <= 0 || T <= 0 || H <= 0 || HN <= 0 || TN <= 0) return fail(NATSL_ERR_INVALID, "%s: non-positive dimension", what);

@@ -156,3 +156,23 @@ def test_gdn_p_formed_by_the_scan_agrees_with_p_from_the_prep(K):
     assert torch.equal(s1, s2)
     rl = float((o1.float() - o2.float()).norm() / o2.float().norm())
     assert 0 < rl <= 5e-4, rl          # (0 would mean both calls took the same path)
+
+
+@pytest.mark.parametrize("kind,B,T,H,K,V,block", [
+    ('gdn', 1, 64, 2, 64, 16, 64), ('gdn', 2, 200, 3, 128, 32, 64), ('gdn', 8, 130, 16, 128, 128, 128), ('gdn', 3, 449, 2, 192, 64, 64),
+    ('mamba', 1, 1, 1, 64, 16, 64), ('mamba', 2, 321, 3, 128, 32, 64), ('mamba', 8, 300, 16, 128, 128, 256), ('mamba', 2, 190, 2, 192, 96, 64)])
+def test_states_without_outputs(kind, B, T, H, K, V, block):
+    """A call that forms the chunk states only (one, two and four compute waves, every key width) gives the same bits as one with outputs."""
+    from neuralattentionsearchlinear_amd import _capi
+    from neuralattentionsearchlinear_amd._mixed_common import linear_chunk_fwd
+    q, k, v = make_qkv(B, T, H, K, V, 50)
+    g, beta = make_gates(B, T, H, 51)
+    ty = make_types(B, -(-T // block), H, 0.3, 52, torch.bfloat16)
+    h0 = torch.randn(B, H, K, V, generator=torch.Generator().manual_seed(53)) * 0.5
+    flags = _capi.DECAY_NON_LINEAR | _capi.INTRA_CHUNK | (_capi.QK_L2NORM if kind == 'gdn' else 0)
+    args = [kind] + [t.to(DEV) for t in (q, k, v, g)] + [beta.to(DEV) if kind == 'gdn' else None, h0.to(DEV), ty.to(DEV), K ** -0.5, block, flags, True, None]
+    _, s1, states1, vn1, _ = linear_chunk_fwd(*args, chunk_states=True)
+    o, s2, states2, vn2, _ = linear_chunk_fwd(*args, chunk_states=True, outputs=False)
+    assert o is None and torch.equal(s1, s2) and torch.equal(states1, states2) and torch.equal(vn1, vn2)
+    with pytest.raises(ValueError):
+        linear_chunk_fwd(*args, outputs=False)                              # neither states nor outputs

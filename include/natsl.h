@@ -229,13 +229,13 @@ int natsl_linear_chunk_bwd(int delta_rule, const void* q, const void* k, const v
 
 /* natsl_linear_chunk_bwd in its two steps, so that something can run next to the scan or be ready before the second step: steps 1 = the
  * reverse scan (dv, d_chunk_states, dbeta_parts, dh0), 2 = the per-chunk gradients (dq, dk, dg, dbeta, d_gate, d_rollback), 3 = both; + 4: another
- * kernel shares the chip with the scan (wider workgroups on fewer CUs).
+ * kernel shares the chip with the scan (wider workgroups on fewer CUs); + 8: dbeta is bf16.
  * add (second step): 1, 2 = dq, dk are added to what is there; dv_sum, when given, [B*T][H][V]: dv is added to what is there.  (A tensor
  * that another operator takes as well has one gradient; the sum is rounded as an elementwise bf16 addition would.) */
 int natsl_linear_chunk_bwd_steps(int steps, int add, void* dv_sum, int delta_rule, const void* q, const void* k, const void* v_new, const float* g,
                                  const void* beta, const void* d_o, const float* dht, const void* chunk_states, const void* types,
                                  int types_dtype, const float* g_block_sums, const void* workspace, void* d_chunk_states, float* dbeta_parts,
-                                 void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0, float* d_gate, float* d_rollback, int B, int T,
+                                 void* dq, void* dk, void* dv, float* dg, void* dbeta, float* dh0, float* d_gate, float* d_rollback, int B, int T,
                                  int H, int HN, int K, int V, int TN, int block, float scale, int flags, int dtype,
                                  const natsl_seq_row* seqs, int n_seqs, int total_chunks, natsl_stream_t stream);
 
@@ -487,6 +487,12 @@ typedef struct natsl_project_seg { const void* y; const void* w; int32_t n, ld; 
 int natsl_project(const natsl_project_seg* segs, int n_seg, const void* x, int64_t rows, int D, int ldx, natsl_stream_t stream);
 int natsl_project_bwd(const natsl_project_seg* segs, int n_seg, const void* dpool, void* dx, int B, int T, int D, int block,
                       natsl_stream_t stream);
+
+/* Products with a narrow weight w [N, D] (N a multiple of 4 up to 64, D of 128, N D up to 81920), bf16 with fp32 sums:
+ * y [rows, N] = x [rows, D] w^T, and dx [rows, D] = dy [rows, N] w.  Contiguous, on 16 bytes.  (The mixing logits' layer,
+ * src/nats/layers/natsl_attn_gdn.py:425-491.) */
+int natsl_narrow_linear(const void* x, const void* w, void* y, int64_t rows, int D, int N, natsl_stream_t stream);
+int natsl_narrow_linear_bwd(const void* dy, const void* w, void* dx, int64_t rows, int D, int N, natsl_stream_t stream);
 
 /* The mixed operator's forward (src/nats/ops/mixed_ops/mixed_attn_gdn.py:47-191, src/nats/ops/mixed_ops/mixed_attn_mamba.py:51-192)
  * in one call: natsl_route, natsl_softmax_sparse_fwd and natsl_gdn_chunk_fwd (is_delta) or natsl_mamba_chunk_fwd with the

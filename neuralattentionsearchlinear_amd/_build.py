@@ -13,7 +13,7 @@ CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB = os.path.join(CSRC, "libnatsl.so")
 BENCH_LIB = os.path.join(CSRC, "libnatsl_bench.so")
 STEP_CORE = os.path.join(os.path.dirname(CSRC), "_step_core.so")
-SOURCES = ["natsl_route.hip", "natsl_softmax.hip", "natsl_softmax_bwd.hip", "natsl_linear.hip", "natsl_linear_bwd.hip", "natsl_norm_gate.hip", "natsl_conv.hip", "natsl_decode.hip", "natsl_step.hip", "natsl_mixed.hip", "natsl_wgrad.hip", "natsl_project.hip", "natsl_front.hip", "natsl_cache.hip"]
+SOURCES = ["natsl_route.hip", "natsl_softmax.hip", "natsl_softmax_bwd.hip", "natsl_linear.hip", "natsl_linear_bwd.hip", "natsl_norm_gate.hip", "natsl_conv.hip", "natsl_decode.hip", "natsl_step.hip", "natsl_mixed.hip", "natsl_wgrad.hip", "natsl_project.hip", "natsl_narrow.hip", "natsl_front.hip", "natsl_cache.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17",
     # keep the compiler from forming packed-fp32 VALU ops

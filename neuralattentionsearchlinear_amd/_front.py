@@ -185,6 +185,34 @@ class _Project(torch.autograd.Function):
         return dx, dws[0], dws[1], dws[2], dws[3], da, db, None
 
 
+# ---- a narrow weight: the mixing logits' layer ------------------------------------------------------------------------------------
+def _narrow_built(N, D, *tensors):
+    return N % 4 == 0 and N <= 64 and D % 128 == 0 and N * D <= 81920 and _on_16(*tensors)
+
+
+def _narrow(x, w):
+    """F.linear(x, w).  natsl_narrow_linear from 2^24 elements of x on (a layer's times, library / it, us: 24 x 768 over 32768 tokens
+    23 / 12, 32 x 2048 over 16000 29 / 21; 36 x 1152 over 6000 9.3 / 11.3)."""
+    N, D = w.shape
+    if x.numel() < 1 << 24 or not _narrow_built(N, D, x, w):
+        return F.linear(x, w)
+    y = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
+    _capi.check(_capi.lib().natsl_narrow_linear(x.data_ptr(), w.data_ptr(), y.data_ptr(), x.numel() // D, D, N, _capi.stream_ptr(x.device)),
+                "natsl_narrow_linear")
+    return y
+
+
+def _narrow_bwd(dy, w):
+    """dy [rows, N] w (24 x 768 over 32768 tokens 36 -> 14 us, 36 x 1152 over 6000 16 -> 9)"""
+    N, D = w.shape
+    if not _narrow_built(N, D, dy, w):
+        return torch.mm(dy, w)
+    dx = torch.empty(dy.shape[0], D, dtype=dy.dtype, device=dy.device)
+    _capi.check(_capi.lib().natsl_narrow_linear_bwd(dy.data_ptr(), w.data_ptr(), dx.data_ptr(), dy.shape[0], D, N, _capi.stream_ptr(dy.device)),
+                "natsl_narrow_linear_bwd")
+    return dx
+
+
 # ---- convolutions, norms, mixing logits --------------------------------------------------------------------------------------------
 def _conv_segs(f, raw):
     """The segments of natsl_conv_norm_*: q, k, v with their weights; f: the layer's FastFront."""
@@ -230,7 +258,7 @@ class _ConvNorm(torch.autograd.Function):
         ctx.save_for_backward(q, k, v, ys[0], w_mix, wq, bq, wk, bk, wv, bv, nq, nk)
         ctx.set_materialize_grads(False)
         raw = tuple(t.view(t.shape) for t in (q, k, v)) if f.raw_attention else (None, None, ys[2].detach())
-        return (ys[0], ys[1], ys[2], ns[0], ns[1], F.linear(ys[0], w_mix)) + raw
+        return (ys[0], ys[1], ys[2], ns[0], ns[1], _narrow(ys[0], w_mix)) + raw
 
     @staticmethod
     def backward(ctx, dq, dk, dv, dqn, dkn, dlogits, dq_raw, dk_raw, dv_raw):
@@ -241,7 +269,7 @@ class _ConvNorm(torch.autograd.Function):
         dw_mix = dq_mix = None
         if dlogits is not None:
             d2 = dlogits.reshape(B * T, -1).contiguous()
-            dq_mix = torch.mm(d2, w_mix)
+            dq_mix = _narrow_bwd(d2, w_mix)
             dw_mix = weight_grads(yq.view(B * T, -1), [d2])[0]
         hold = []
 
@@ -374,10 +402,13 @@ class _Select(torch.autograd.Function):
         types, counts, fraction, raw = _select(logits.detach(), want_raw)
         ctx.save_for_backward(logits)
         ctx.mark_non_differentiable(counts, fraction, *((raw,) if want_raw else ()))
+        ctx.set_materialize_grads(False)               # (zeros for the counts and shares would be two launches)
         return types, counts, fraction, raw
 
     @staticmethod
     def backward(ctx, dtypes, *_):
+        if dtypes is None:
+            return None, None
         (logits,) = ctx.saved_tensors
         lg, d = logits.contiguous(), dtypes.to(logits.dtype).contiguous()
         out = torch.empty_like(lg)
@@ -414,7 +445,7 @@ class FastFront:
         if self.grad(*args):
             return _ConvNorm.apply(self, *args) + (None,)
         ys, ns, new = _conv_norm(self, (q, k, v), states, want_states)
-        return ys[0], ys[1], ys[2], ns[0], ns[1], F.linear(ys[0], w["w_mix"]), *((q, k, v) if self.raw_attention else (None, None, ys[2])), new
+        return ys[0], ys[1], ys[2], ns[0], ns[1], _narrow(ys[0], w["w_mix"]), *((q, k, v) if self.raw_attention else (None, None, ys[2])), new
 
     def gates(self, ab):
         if self.grad(ab, self.w["a_log"], self.w["dt_bias"]):

@@ -212,7 +212,8 @@ def linear_chunk_backward_hip(kind, q, k, v, g, beta, h0, types, scale, block, d
                 raise ValueError("a gradient to add to must be like its tensor")
         add = (onto[0] is not None) + 2 * (onto[1] is not None)
         dg = torch.empty(B, T, H, dtype=f32, device=dev)
-        dbeta = torch.empty(B, T, H, dtype=f32, device=dev) if delta else None
+        dbeta_bf16 = delta and beta.dtype == bf16
+        dbeta = torch.empty(B, T, H, dtype=bf16 if dbeta_bf16 else f32, device=dev) if delta else None
         dbeta_parts = torch.empty(B, T, H, V // 16, dtype=f32, device=dev) if delta else None
         dh0 = torch.empty(N, H, K, V, dtype=f32, device=dev) if h0 is not None else None
         gate = torch.empty(NTtot, H, dtype=f32, device=dev)
@@ -221,7 +222,7 @@ def linear_chunk_backward_hip(kind, q, k, v, g, beta, h0, types, scale, block, d
         dhtf = None if dht is None else dht.detach().to(f32).contiguous()
         def steps(which):
             rc = L.natsl_linear_chunk_bwd_steps(
-                which, add, P(dv_sum), 1 if delta else 0, P(qb), P(kb), P(v_new), P(gf), P(bb), P(dof), P(dhtf), P(states), P(ty),
+                which + (8 if dbeta_bf16 else 0), add, P(dv_sum), 1 if delta else 0, P(qb), P(kb), P(v_new), P(gf), P(bb), P(dof), P(dhtf), P(states), P(ty),
                 _capi.dtype_code(ty.dtype), P(gsum), P(ws), P(d_states), P(dbeta_parts), P(dq), P(dk), P(dv), P(dg), P(dbeta), P(dh0), P(gate), P(rb),
                 B, T, H, HN, K, V, NB, block, float(scale), flags, _capi.dtype_code(bf16), sp, ns, tot, stream)
             _capi.check(rc, "natsl_linear_chunk_bwd_steps")

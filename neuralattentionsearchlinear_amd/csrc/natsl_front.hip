@@ -356,7 +356,7 @@ __global__ __launch_bounds__(256) void gates_kernel(const GatesParams p) {
   }
 }
 
-constexpr int GATES_ITERS = 8;
+constexpr int GATES_ITERS = 2;
 // thread = (row of the workgroup's batch, head); the rows' shares of the two parameter gradients are added through LDS in order
 __global__ __launch_bounds__(256) void gates_bwd_kernel(const GatesParams p) {
   __shared__ float red[2][256];

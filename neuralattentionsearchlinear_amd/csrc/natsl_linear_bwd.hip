@@ -61,7 +61,8 @@ struct LinBwdParams {
   bf16_t* dq;
   bf16_t* dk;
   float* dg;              // [tokens][H]
-  float* dbeta;           // [tokens][H]
+  void* dbeta;            // [tokens][H], fp32 or (dbeta_bf16) bf16
+  int dbeta_bf16;
   float* dbeta_parts;     // [tokens][H][V / 16]: <dX, v_new> over each wave's 16 columns (scan -> per-chunk kernel)
   float* gate;            // [chunk][H]: derivative with respect to a gate on the chunk's state update
   float* rb;              // [chunk][H]: f <dS', S_blockstart> behind a rolled-back block's last chunk (the decay's share of dg)
@@ -1136,7 +1137,10 @@ __global__ __launch_bounds__(256, DK <= 128 ? 2 : 1) void linear_bwd_chunk_kerne
     const float* pp = p.dbeta_parts + ((row0 + lane) * p.H + h) * (p.V / 16);
     float sum = 0.f;
     for (int i = 0; i < p.V / 16; ++i) sum += pp[i];
-    p.dbeta[(row0 + lane) * p.H + h] = sum / (bet[lane] * bet[lane]);
+    const float db = sum / (bet[lane] * bet[lane]);
+    const size_t at = (row0 + lane) * p.H + h;
+    if (p.dbeta_bf16) reinterpret_cast<bf16_t*>(p.dbeta)[at] = f32_to_bf16(db);
+    else reinterpret_cast<float*>(p.dbeta)[at] = db;
   }
   if (wave == 0) {
     // dg_t = sum_{i >= t} dgamma_i + dG
@@ -1338,7 +1342,7 @@ using namespace natsl;
 extern "C" int natsl_linear_chunk_bwd_steps(int steps, int add, void* dv_sum, int delta_rule, const void* q, const void* k, const void* v_new, const float* g, const void* beta,
                                       const void* d_o, const float* dht, const void* chunk_states, const void* types, int types_dtype,
                                       const float* g_block_sums, const void* workspace, void* d_chunk_states, float* dbeta_parts,
-                                      void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0, float* d_gate, float* d_rollback, int B, int T,
+                                      void* dq, void* dk, void* dv, float* dg, void* dbeta, float* dh0, float* d_gate, float* d_rollback, int B, int T,
                                       int H, int HN, int K, int V, int TN, int block, float scale, int flags, int dtype,
                                       const natsl_seq_row* seqs, int n_seqs, int total_chunks, natsl_stream_t stream) {
   const char* what = "natsl_linear_chunk_bwd";
@@ -1363,7 +1367,7 @@ extern "C" int natsl_linear_chunk_bwd_steps(int steps, int add, void* dv_sum, in
     p.ws_p = p.ws_tm + units * (CB * CB);
     p.ws_sc = reinterpret_cast<const float*>(p.ws_p + units * (CB * CB));
   } p.types_dtype = types_dtype;
-  p.dq = (bf16_t*)dq; p.dk = (bf16_t*)dk; p.dg = dg; p.dbeta = dbeta; p.dbeta_parts = dbeta_parts; p.gate = d_gate; p.rb = d_rollback;
+  p.dq = (bf16_t*)dq; p.dk = (bf16_t*)dk; p.dg = dg; p.dbeta = dbeta; p.dbeta_bf16 = steps >> 3 & 1; p.dbeta_parts = dbeta_parts; p.gate = d_gate; p.rb = d_rollback;
   p.B = B; p.T = T; p.H = H; p.HN = HN; p.V = V; p.TN = TN; p.block = block; p.nt = cdiv(T, CB);
   p.seqs = reinterpret_cast<const SeqRow*>(seqs); p.n_seqs = seqs ? n_seqs : 0; p.total_chunks = seqs ? total_chunks : B * p.nt;
   p.scale = scale; p.flags = flags; p.add = add; p.dv_sum = (bf16_t*)dv_sum;

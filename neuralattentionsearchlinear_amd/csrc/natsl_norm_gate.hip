@@ -218,31 +218,35 @@ __global__ __launch_bounds__(256) void norm_gate_bwd_kernel(const bf16_t* x1, co
   }
 }
 
-// out[c] = sum over k of part[k][c]: 64 adjacent columns per workgroup, 16 thread rows that each add up every 16th k
-// (eight loads in flight), the 16 row sums added in a fixed order.
+// out[c] = sum over k of part[k][c]: 16 adjacent columns per workgroup, 64 thread rows that each add up every 64th k (sixteen loads in
+// flight), the 64 row sums added in a fixed order.  A CU takes some 50 KB a microsecond: with 64 columns a workgroup four of them read
+// 3072 rows of 256 columns in 16 us.
+constexpr int COLSUM_COLS = 16;
 __global__ __launch_bounds__(1024) void colsum_reduce_kernel(const float* part, float* out, const int n_part, const int n_col) {
-  __shared__ float sums[16][64];
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  const int i = blockIdx.x * 64 + tx;
+  constexpr int TY = 1024 / COLSUM_COLS;
+  __shared__ float sums[TY][COLSUM_COLS];
+  const int tx = threadIdx.x % COLSUM_COLS, ty = threadIdx.x / COLSUM_COLS;
+  const int i = blockIdx.x * COLSUM_COLS + tx;
   float acc = 0.f;
   if (i < n_col) {
     const float* src = part + i;
     int k = ty;
-    for (; k + 7 * 16 < n_part; k += 8 * 16) {
-      float v[8];
+    for (; k + 15 * TY < n_part; k += 16 * TY) {
+      float v[16];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = src[(size_t)(k + 16 * u) * n_col];
+      for (int u = 0; u < 16; ++u) v[u] = src[(size_t)(k + TY * u) * n_col];
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int u = 0; u < 8; ++u) acc += v[u];
+      for (int u = 0; u < 16; ++u) acc += v[u];
     }
-    for (; k < n_part; k += 16) acc += src[(size_t)k * n_col];
+    for (; k < n_part; k += TY) acc += src[(size_t)k * n_col];
   }
   sums[ty][tx] = acc;
   __syncthreads();
   if (ty == 0 && i < n_col) {
     float t = 0.f;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) t += sums[r][tx];
+    for (int r = 0; r < TY; ++r) t += sums[r][tx];
     out[i] = t;
   }
 }
@@ -333,7 +337,7 @@ static int norm_gate_bwd(const void* x1, const void* x2, const void* gate, const
 #undef NATSL_NGB
   int rc = check_launch(what);
   if (rc != NATSL_OK) return rc;
-  hipLaunchKernelGGL(colsum_reduce_kernel, dim3((unsigned)((2 * D + 63) / 64)), dim3(1024), 0, s, part, dw1, (int)wgs, 2 * D);
+  hipLaunchKernelGGL(colsum_reduce_kernel, dim3((unsigned)((2 * D + COLSUM_COLS - 1) / COLSUM_COLS)), dim3(1024), 0, s, part, dw1, (int)wgs, 2 * D);
   return check_launch(what);
 }
 

@@ -55,6 +55,8 @@ __global__ __launch_bounds__(256, 1) void wgrad_kernel(const WgradParams p) {
   const long long t_first = (long long)split * p.slice;
   const int n_tok = (int)(p.T - t_first < p.slice ? p.T - t_first : p.slice);
   const int n_st = (n_tok + WG_T - 1) / WG_T;
+  // 32-row blocks of this wave's 128 that the weight has: a narrow weight's others are neither multiplied nor stored
+  const int blocks = min(4, max(0, (sg.n - n0 - 128 * (wave >> 1) + 31) / 32));
 
   // what this wave requests of a stage: rows 8*wave .. +7 of either tile, two rows per instruction.  16-byte segment s of row r
   // sits at slot s ^ 4*(r%4): the four rows of a transposing read then meet four different quarters of the banks.  Columns past
@@ -143,8 +145,8 @@ __global__ __launch_bounds__(256, 1) void wgrad_kernel(const WgradParams p) {
   // One stage's products.  AHEAD: stage st + 3 is a whole one, and its eight requests go out one behind every four products (issued
   // together they took 290 cycles in which the matrix cores had nothing: 4608 + 2 x 6 rows x 1024 columns over 32768 tokens 321 -> 264 us,
   // 1.2 PFLOP/s); else they are all in front, if there are any.
-  auto stage = [&](auto ahead, const int st) __attribute__((always_inline)) {
-    constexpr bool AHEAD = decltype(ahead)::value;
+  auto stage = [&](auto ahead, auto whole, const int st) __attribute__((always_inline)) {
+    constexpr bool AHEAD = decltype(ahead)::value, WHOLE = decltype(whole)::value;
     const unsigned here = (unsigned)(st & (WG_STAGES - 1)) * WG_STAGE, next = (unsigned)((st + 1) & (WG_STAGES - 1)) * WG_STAGE;
     const bool more = AHEAD || st + 3 < n_st;
     if (!AHEAD && more) request(st + 3);       // into the buffer of stage st-1, which every wave has read
@@ -159,8 +161,10 @@ __global__ __launch_bounds__(256, 1) void wgrad_kernel(const WgradParams p) {
       for (int a = 0; a < 4; ++a) {
         A[kk ^ 1][a] = operand(oa[a] + at);
         B[kk ^ 1][a] = operand(ob[a] + at);
+        if (WHOLE || a < blocks) {
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = mfma32(A[kk][a], B[kk][b], acc[a][b]);
+          for (int b = 0; b < 4; ++b) acc[a][b] = mfma32(A[kk][a], B[kk][b], acc[a][b]);
+        }
         // one read next to each product: the scheduler otherwise saves registers by reading an operand right before its use
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -181,8 +185,11 @@ __global__ __launch_bounds__(256, 1) void wgrad_kernel(const WgradParams p) {
     if (!AHEAD) finish_partial(st + 2);
   };
   int st = 0;
-  for (; (st + 4) * WG_T <= n_tok; ++st) stage(std::true_type{}, st);
-  for (; st < n_st; ++st) stage(std::false_type{}, st);
+  if (sg.n - n0 > WG_N / 2)
+    for (; (st + 4) * WG_T <= n_tok; ++st) stage(std::true_type{}, std::true_type{}, st);
+  else
+    for (; (st + 4) * WG_T <= n_tok; ++st) stage(std::true_type{}, std::false_type{}, st);
+  for (; st < n_st; ++st) stage(std::false_type{}, std::false_type{}, st);
 
   // lane: column d = lane%32 of each 32x32 tile, rows 8*(r/4) + 4*(lane/32) + r%4: four rows of a column per 16-byte store
   float* dst = p.part + ((size_t)u * 4 + wave) * (size_t)(WG_N * WG_N / 4) + lane * 4;
@@ -192,7 +199,7 @@ __global__ __launch_bounds__(256, 1) void wgrad_kernel(const WgradParams p) {
     for (int b = 0; b < 4; ++b)
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<f32x4*>(dst + ((a * 4 + b) * 4 + q) * 256) = (f32x4){acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]};
+        if (a < blocks) *reinterpret_cast<f32x4*>(dst + ((a * 4 + b) * 4 + q) * 256) = (f32x4){acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]};
 }
 
 // Adds the slices' partial tiles in order and writes the gradient: a workgroup takes one 32 x 32 block of a tile per wave.
@@ -210,11 +217,24 @@ __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const WgradParams p) 
   f32x4 sum[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) sum[q] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < p.splits; ++s) {
-    const float* src = p.part + (((size_t)s * p.tiles + tile) * 4 + wave) * (size_t)(WG_N * WG_N / 4) + (size_t)ab * 1024 + lane * 4;
+  const float* src = p.part + ((size_t)tile * 4 + wave) * (size_t)(WG_N * WG_N / 4) + (size_t)ab * 1024 + lane * 4;
+  const size_t step = (size_t)p.tiles * (WG_N * WG_N);
+  int s = 0;
+  for (; s + 6 <= p.splits; s += 6) {          // (six slices on their way at a time; one by one a slice takes a round trip, 0.4 us)
+    f32x4 v[6][4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) sum[q] += *reinterpret_cast<const f32x4*>(src + q * 256);
+    for (int i = 0; i < 6; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[i][q] = *reinterpret_cast<const f32x4*>(src + (s + i) * step + q * 256);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) sum[q] += v[i][q];
   }
+  for (; s < p.splits; ++s)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sum[q] += *reinterpret_cast<const f32x4*>(src + s * step + q * 256);
   if (d >= p.D) return;
 #pragma unroll
   for (int q = 0; q < 4; ++q)
@@ -237,15 +257,17 @@ static int wgrad_cus() {
 }
 
 // Slices of the tokens: a CU holds one unit at a time, so the launch takes ceil(tiles * slices / CUs) rounds of T / slices tokens
-// (measured: 17 ns a token), and every slice writes and reads its partial tiles once more (0.1 us a tile).
-static int wgrad_splits(long long T, int tiles) {
+// (measured: 17 ns a token), and every slice writes and reads its partial tiles once more (0.1 us a whole tile; full: whole tiles'
+// worth of rows.  24 rows x 768 columns over 32768 tokens: 45 us with
+// 32 slices of whole tiles, 28 with 85 of the blocks that there are).
+static int wgrad_splits(long long T, int tiles, double full) {
   const int cus = wgrad_cus();
   int best = 1;
   double best_cost = 1e300;
-  for (int s = 1; s <= 32; ++s) {
+  for (int s = 1; s <= 128; ++s) {
     if (s > 1 && T < 64ll * s) break;
     const double rounds = (double)(((long long)tiles * s + cus - 1) / cus);
-    const double cost = rounds * (4.0 + 0.017 * (double)T / s) + 0.1 * tiles * s;
+    const double cost = rounds * (4.0 + 0.017 * (double)T / s) + 0.1 * full * s;
     if (cost < best_cost) { best_cost = cost; best = s; }
   }
   return best;
@@ -258,6 +280,7 @@ static int wgrad_plan(WgradParams& p, const natsl_wgrad_seg* segs, int n_seg, co
   p.x = (const bf16_t*)x; p.ldx = ldx; p.D = D; p.n_seg = n_seg; p.T = T;
   p.tiles_d = cdiv(D, WG_N);
   int rows = 0;
+  double full = 0.;
   for (int i = 0; i < NATSL_WGRAD_SEGS; ++i) {
     if (i >= n_seg) { p.seg[i] = {nullptr, nullptr, 0, 0, 1 << 30}; continue; }
     const natsl_wgrad_seg& s = segs[i];
@@ -265,9 +288,10 @@ static int wgrad_plan(WgradParams& p, const natsl_wgrad_seg* segs, int n_seg, co
     if ((long long)WG_T * s.ld * 2 > 0x7fffffffll || (long long)WG_T * ldx * 2 > 0x7fffffffll) return fail(NATSL_ERR_UNSUPPORTED, "%s: rows too long", what);
     p.seg[i] = {(const bf16_t*)s.dy, (bf16_t*)s.out, s.n, s.ld, rows};
     rows += cdiv(s.n, WG_N);
+    full += cdiv(s.n, 32) / 8. * p.tiles_d;
   }
   p.tiles = rows * p.tiles_d;
-  const int splits = wgrad_splits(T, p.tiles);
+  const int splits = wgrad_splits(T, p.tiles, full);
   p.slice = (T + splits - 1) / splits;
   p.slice = (p.slice + WG_T - 1) / WG_T * WG_T;
   p.splits = (int)((T + p.slice - 1) / p.slice);

@@ -168,7 +168,7 @@ def test_replaced_weights_are_freed(kind):
     assert not any(r() is not None for r in old)
 
 
-@pytest.mark.parametrize("T,D,widths", [(1, 8, (8,)), (31, 64, (16, 24)), (32, 256, (256,)), (33, 264, (264, 8)), (129, 72, (512,)), (5000, 128, (136,))])
+@pytest.mark.parametrize("T,D,widths", [(1, 8, (8,)), (31, 64, (16, 24)), (32, 256, (256,)), (33, 264, (264, 8)), (129, 72, (512,)), (5000, 128, (136,)), (9000, 768, (24,)), (9001, 128, (264, 32))])
 def test_weight_grads(T, D, widths):
     """natsl_wgrad at the edges of its 32-token stages, 256-wide tiles and token slices."""
     from neuralattentionsearchlinear_amd._front import weight_grads
@@ -239,3 +239,20 @@ def test_joint_projections(B, T, D, widths, block):
         ref = sum(dy.double() @ w.double() for dy, w in zip(dys, ws))
         assert close(dx[:rows], ref if pool is None else ref + spread)
         assert bool((dx[rows] == 7).all())
+
+
+@pytest.mark.parametrize("rows,D,N", [(1, 128, 4), (33, 768, 24), (63, 1152, 36), (64, 2048, 32), (65, 1280, 64), (257, 384, 60), (4099, 256, 16)])
+def test_narrow_products(rows, D, N):
+    """natsl_narrow_linear and its backward at the edges of their tiles of tokens, columns and weight rows."""
+    from neuralattentionsearchlinear_amd import _capi
+    torch.manual_seed(rows)
+    L, P = _capi.lib(), _capi.ptr
+    x, w, dy = torch.randn(rows, D, device=DEV).bfloat16(), torch.randn(N, D, device=DEV).bfloat16(), torch.randn(rows, N, device=DEV).bfloat16()
+    y, dx = (torch.full((rows + 1, n), 7., device=DEV).bfloat16() for n in (N, D))
+    _capi.check(L.natsl_narrow_linear(P(x), P(w), P(y), rows, D, N, _capi.stream_ptr(x.device)), "natsl_narrow_linear")
+    _capi.check(L.natsl_narrow_linear_bwd(P(dy), P(w), P(dx), rows, D, N, _capi.stream_ptr(x.device)), "natsl_narrow_linear_bwd")
+    for a, ref in ((y, x.double() @ w.double().t()), (dx, dy.double() @ w.double())):
+        # exact products, fp32 sums, one rounding to bf16
+        assert bool(((a[:rows].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * D ** 0.5).all())
+        assert bool((a[rows] == 7).all())
+    assert L.natsl_narrow_linear(P(x), P(w), P(y), rows, D, N + 2, _capi.stream_ptr(x.device)) != 0

@@ -270,7 +270,7 @@ NATSL_DEVICE constexpr int tri_slot(const int t, const int s) { return t < 2 ? t
 // LDS of the reverse scan: two stages, each one chunk's inputs exactly as they lie in memory (filled by LDS-DMA).
 template <int DK, int NW>
 struct BwdScanLds {
-  static_assert(NW == 4 || (NW == 2 && DK <= 128), "four compute waves, or two where a fifth wave moves the data");
+  static_assert(NW == 4 || NW == 2, "two or four compute waves");
   static constexpr int KROW = DK * 2, VROW = 32 * NW;    // bytes per k / q row, per dO / v_new row (16 NW columns)
   static constexpr int KB = CB * KROW, VB = CB * VROW, TB = 6 * 1024, SCB = 1024;
   static constexpr int OFF_K = 0, OFF_Q = OFF_K + KB, OFF_DO = OFF_Q + KB, OFF_VN = OFF_DO + VB, OFF_T = OFF_VN + VB,
@@ -278,8 +278,9 @@ struct BwdScanLds {
   static constexpr int STAGE = OFF_SC + SCB;
   // Up to K = 128 a fifth wave does nothing but issue the requests (it shares a SIMD with a compute wave, so every wave has
   // to fit 256 registers: for K = 128 the held-back state gradient of a rolled-back block waits in LDS instead of
-  // registers); K = 192 has neither the registers nor the LDS for that, and its compute waves issue the requests themselves.
-  static constexpr bool DMAW = DK <= 128, PEND_LDS = DK == 128;
+  // registers); K = 192 with four compute waves has neither the registers nor the LDS for that, and its compute waves issue the requests
+  // themselves; with two a wave has a SIMD to itself, and 512 registers.
+  static constexpr bool DMAW = DK <= 128 || NW == 2, PEND_LDS = DK == 128;
   static constexpr int PEND = (DK / 16) * 4 * 64 * 4;    // bytes per wave
   static constexpr int TOTAL = 2 * STAGE + (PEND_LDS ? NW * PEND : 0);
   static constexpr int THREADS = 64 * (DMAW ? NW + 1 : NW);
@@ -1321,7 +1322,10 @@ static int launch_bwd(const LinBwdParams& p, const int steps, hipStream_t stream
     const long long wgs64 = (long long)(p.seqs ? p.n_seqs : p.B) * p.H * (p.V / 64);
     int rc;
     if constexpr (DK <= 128) rc = spare * wgs64 <= bwd_cu_count() ? launch_bwd_scan<DK, DELTA, 2>(p, stream, what) : launch_bwd_scan<DK, DELTA, 4>(p, stream, what);
-    else rc = launch_bwd_scan<DK, DELTA, 4>(p, stream, what);
+    // (K = 192: the four-wave form has no wave to spare for the requests and its step takes 206 us / 47, the two-wave one 147 / 47 at B2 T3000 H6
+    // V384; next to the softmax kernels as long as it leaves them a third of the CUs: a 760M layer's training step at B1 T5000 1635 -> 1560 us,
+    // but at B3 T4096, on 216 of 256 CUs, 2864 -> 2921)
+    else rc = (steps & 4 ? 3 : 2) * wgs64 <= bwd_cu_count() ? launch_bwd_scan<DK, DELTA, 2>(p, stream, what) : launch_bwd_scan<DK, DELTA, 4>(p, stream, what);
     if (rc != NATSL_OK) return rc;
   }
   if (steps & 2) {

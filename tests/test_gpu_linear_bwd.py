@@ -164,3 +164,17 @@ def test_value_widths_that_are_no_multiple_of_64(kind, K, V):
     torch.cuda.synchronize()
     assert out[2].shape[-1] == V and out[5].shape[-1] == V
     _check(out, ref, kind, True)
+
+
+@pytest.mark.parametrize("kind,B,H,V", [('gdn', 9, 6, 192), ('mamba', 9, 6, 192), ('gdn', 2, 3, 64), ('mamba', 1, 3, 128)])
+def test_key_width_192_with_four_and_two_compute_waves(kind, B, H, V):
+    """More 64-column slices than half of the CUs: four compute waves a workgroup; else two, with a wave of their own for the requests."""
+    from neuralattentionsearchlinear_amd import _linear_bwd as B_
+    T, K, block = 130, 192, 64
+    q, k, v, g, beta, ty, init, do, dht = _inputs(kind, B, T, H, H, K, V, block, 7)
+    scale, l2 = (K ** -0.5, True) if kind == 'gdn' else (1.0, False)
+    ref = LB.linear_branch_bwd(kind, q, k, v, g, beta if kind == 'gdn' else None, ty[..., 1], scale, do, dht, init, block, True, l2, True, False)
+    d = lambda t: t.to(DEV)
+    out = B_.linear_chunk_backward_hip(kind, d(q), d(k), d(v), d(g), d(beta) if kind == 'gdn' else None, d(init), d(ty), scale, block, True, l2, True, d(do),
+                                       d(dht), False)
+    _check(out, ref, kind, True)

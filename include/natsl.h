@@ -494,6 +494,14 @@ int natsl_project_bwd(const natsl_project_seg* segs, int n_seg, const void* dpoo
 int natsl_narrow_linear(const void* x, const void* w, void* y, int64_t rows, int D, int N, natsl_stream_t stream);
 int natsl_narrow_linear_bwd(const void* dy, const void* w, void* dx, int64_t rows, int D, int N, natsl_stream_t stream);
 
+/* natsl_gdn_chunk_fwd (is_delta) or natsl_mamba_chunk_fwd with NATSL_STATES_ONLY and no state of the last block.  beside: NULL, or
+ * another stream of the same device that is made to wait for `stream` up to the kernel in front of the scan, for work that shares the
+ * GPU with the scan. */
+int natsl_linear_chunk_states(int is_delta, const void* q, const void* k, const void* v, const float* g, const void* beta, const float* h0, float* ht,
+                              void* chunk_states, void* chunk_v_new, const void* types, int types_dtype, int B, int T, int H, int HN, int K, int V,
+                              int TN, int block, float scale, int flags, void* workspace, size_t workspace_bytes, int dtype, const natsl_seq_row* seqs,
+                              int n_seqs, int total_units, natsl_stream_t stream, natsl_stream_t beside);
+
 /* The mixed operator's forward (src/nats/ops/mixed_ops/mixed_attn_gdn.py:47-191, src/nats/ops/mixed_ops/mixed_attn_mamba.py:51-192)
  * in one call: natsl_route, natsl_softmax_sparse_fwd and natsl_gdn_chunk_fwd (is_delta) or natsl_mamba_chunk_fwd with the
  * arguments those take, in bf16, and in front of and behind them the conversions of fp32 tensors (cast_in: fp32 -> bf16,

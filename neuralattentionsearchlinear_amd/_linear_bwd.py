@@ -120,7 +120,8 @@ def hip_backward_is_built(K: int, V: int) -> bool:
 
 
 def linear_chunk_backward(kind, q, k, v, g, beta, h0, types, scale, block, decay, l2norm, intra, do, dht,
-                          dnats_for_invalid_blocks, seqs=None, saved=None, later=None, meanwhile=None, beside=0, onto=(None, None, None)):
+                          dnats_for_invalid_blocks, seqs=None, saved=None, later=None, release=None, meanwhile=None, beside=0,
+                          onto=(None, None, None)):
     """Gradients of the chunked linear branch: -> (dq, dk, dv, dg fp32, dbeta or None, dh0 or None, dnats fp32 [B,NB,HN]).
     types [B,NB,HN,2]; do [B,T,H,V]; dht [N,H,K,V] or None; seqs: packed sequences (B = 1) or None; saved: what
     linear_chunk_fwd(..., chunk_states=True) returned after (o, final_state) on these same inputs, if the caller kept it.  The
@@ -131,7 +132,8 @@ def linear_chunk_backward(kind, q, k, v, g, beta, h0, types, scale, block, decay
     receives a function that ends them, given the softmax branch's dnats [B,NB,HQ] fp32 -> the gradient of types [B,NB,HN,2].
     In that case, too: onto: gradients (bf16, like q, k, v) that dq, dk, dv are added to in place and that come back as them; and
     meanwhile is called once, behind the reverse scan if anything is added (when it returns, this stream has what is added to),
-    else behind everything; beside: 4 if it puts a kernel next to the scan, else 0.
+    else behind everything; beside: 4 if it puts a kernel next to the scan, else 0; release (without `saved`): the stream of that kernel, made
+    to wait for this one up to the forward scan.
 
     dnats_for_invalid_blocks with block > 64 raises NotImplementedError: for a block of several chunks that is not typed
     linear the reference sums a virtual key gradient v . dh over EVERY chunk of the block
@@ -145,7 +147,7 @@ def linear_chunk_backward(kind, q, k, v, g, beta, h0, types, scale, block, decay
     K, V = q.shape[-1], v.shape[-1]
     if hip_backward_is_built(K, V):
         return linear_chunk_backward_hip(kind, q, k, v, g, beta, h0, types, scale, block, decay, l2norm, intra, do, dht,
-                                         dnats_for_invalid_blocks, seqs, saved, later, meanwhile, beside, onto)
+                                         dnats_for_invalid_blocks, seqs, saved, later, release, meanwhile, beside, onto)
     if hip_backward_is_built(K, 64) and V % 16 == 0:
         # Value widths the kernels are not built for (16..48, 96, ..): zero columns up to the next multiple of 64.  The state's
         # columns never mix, a zero column of v and dO stays zero through the whole recurrence and adds nothing to any sum
@@ -172,10 +174,11 @@ def linear_chunk_backward(kind, q, k, v, g, beta, h0, types, scale, block, decay
 
 
 def linear_chunk_backward_hip(kind, q, k, v, g, beta, h0, types, scale, block, decay, l2norm, intra, do, dht,
-                              dnats_for_invalid_blocks, seqs=None, saved=None, later=None, meanwhile=None, beside=0, onto=(None, None, None)):
+                              dnats_for_invalid_blocks, seqs=None, saved=None, later=None, release=None, meanwhile=None, beside=0,
+                              onto=(None, None, None)):
     """The backward as kernels: the forward once more (storing every chunk's entering state and v_new) unless the caller kept
     those from its own forward (`saved`), then the reverse scan and the per-chunk gradients (csrc/natsl_linear_bwd.hip).  later: a list that receives
-    the call that ends the work; meanwhile, beside, onto: see linear_chunk_backward."""
+    the call that ends the work; release, meanwhile, beside, onto: see linear_chunk_backward."""
     from . import _capi
     from ._mixed_common import linear_chunk_fwd
     from .nats_util import _seq_args
@@ -199,7 +202,7 @@ def linear_chunk_backward_hip(kind, q, k, v, g, beta, h0, types, scale, block, d
             states, v_new, ws = saved
         else:
             _, _, states, v_new, ws = linear_chunk_fwd(kind, qb, kb, vb, gf, bb, h0f, ty, scale, block, flags, False, seqs,
-                                                       chunk_states=True, outputs=False)
+                                                       chunk_states=True, outputs=False, beside=release)
         sp, ns, tot = _seq_args(seqs, NTtot)
         P, L, stream = _capi.ptr, _capi.lib(), _capi.stream_ptr(dev)
         gsum = torch.empty(B * NB, H, dtype=f32, device=dev)

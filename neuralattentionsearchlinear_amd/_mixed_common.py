@@ -108,11 +108,12 @@ def _wants_grad(*tensors) -> bool:
 
 def linear_chunk_fwd(kind: str, q, k, v, g, beta, h0, types, scale: float, block: int, flags: int,
                      output_final_state: bool, seqs: Optional[PackedSeqs], block_start_state: bool = False,
-                     chunk_states: bool = False, outputs: bool = True):
+                     chunk_states: bool = False, outputs: bool = True, beside: Optional[int] = None):
     """Launch the chunked linear branch ('gdn' or 'mamba'); returns (o, final_state or None), or with
     block_start_state (o, final_state, state entering the last block, sum of g over the last block), or with chunk_states
     (o, final_state, the state entering every chunk as bf16 [total_chunks, H, V, K], v_new [B, T, H, V] (for 'mamba': v),
-    the workspace); with outputs=False (chunk_states only) o is None and costs nothing."""
+    the workspace); with outputs=False (chunk_states only) o is None and costs nothing, and beside names a stream that is made to wait for
+    this one up to the scan."""
     B, T, H, K = q.shape
     V = v.shape[-1]
     TN, HN = types.shape[1], types.shape[2]
@@ -122,8 +123,6 @@ def linear_chunk_fwd(kind: str, q, k, v, g, beta, h0, types, scale: float, block
     L = _capi.lib()
     ws = torch.empty(L.natsl_linear_workspace_bytes(total_chunks, H), dtype=torch.uint8, device=dev)
     o = torch.empty(B, T, H, V, dtype=q.dtype, device=dev) if outputs else None
-    if not outputs:
-        flags |= _capi.STATES_ONLY
     ht = torch.empty(n, H, K, V, dtype=torch.float32, device=dev) if output_final_state else None
     hs = torch.empty(n, H, K, V, dtype=torch.float32, device=dev) if block_start_state else None
     gs = torch.empty(n, H, dtype=torch.float32, device=dev) if block_start_state else None
@@ -134,6 +133,13 @@ def linear_chunk_fwd(kind: str, q, k, v, g, beta, h0, types, scale: float, block
         h0 = h0.to(torch.float32).contiguous()
     sp, ns, tot = _seq_args(seqs, total_chunks)
     vn = torch.empty_like(v) if chunk_states and kind == 'gdn' else None
+    if not outputs:
+        rc = L.natsl_linear_chunk_states(
+            int(kind == 'gdn'), _capi.ptr(q), _capi.ptr(k), _capi.ptr(v), _capi.ptr(g), _capi.ptr(beta), _capi.ptr(h0), _capi.ptr(ht), _capi.ptr(sc), _capi.ptr(vn),
+            _capi.ptr(types), _capi.dtype_code(types.dtype), B, T, H, HN, K, V, TN, block, float(scale), flags, _capi.ptr(ws), ws.numel(),
+            _capi.dtype_code(q.dtype), sp, ns, tot, _capi.stream_ptr(dev), beside)
+        _capi.check(rc, "natsl_linear_chunk_states")
+        return None, ht, sc, (vn if kind == 'gdn' else v), ws
     common = (_capi.ptr(h0), _capi.ptr(o), _capi.ptr(ht), _capi.ptr(hs), _capi.ptr(gs), _capi.ptr(sc),
               *((_capi.ptr(vn),) if kind == 'gdn' else ()), _capi.ptr(types), _capi.dtype_code(types.dtype), B, T, H, HN, K, V, TN,
               block, float(scale), flags, _capi.ptr(ws), ws.numel(), _capi.dtype_code(q.dtype), sp, ns, tot,
@@ -439,16 +445,20 @@ class _MixedFunction(torch.autograd.Function):
         if do_attn is not None:
             do_attn = do_attn.to(torch.bfloat16).contiguous()
         # The softmax branch's tensors are made first, on this stream, and live until this stream has its kernels behind it (nothing
-        # that is allocated in between can share their memory).  Side by side, the reverse scan is enqueued first (see natsl_mixed_fwd) and
-        # the per-chunk kernel, which adds the branches' gradients of a tensor they share, behind both.
-        attn = side = None
+        # that is allocated in between can share their memory).  Side by side, both scans are enqueued first (see natsl_mixed_fwd), with the
+        # softmax branch behind the kernel in front of the first, and the per-chunk kernel, which adds the branches' gradients of a
+        # tensor they share, behind both.
+        attn = side = release = None
         if do_attn is not None:
             attn = prepare_attn_nats_bwd(q_a, k_a, v_a, o_attn, types, idx, nblk, None, lse, do_attn, cfg['scale_attn'], cfg['block'], 0,
                                          cfg['attn_same_block'], cfg['dnats_invalid_attn'], None, None, None, True, seqs)
             here = torch.cuda.current_stream(q_l.device)
             if _run_side_by_side(q_l.device, seqs, *q_l.shape, v_l.shape[-1]):
                 side = _get_attn_stream(q_l.device)
-                side.wait_stream(here)
+                if linear_saved is None and hip_backward_is_built(q_l.shape[-1], v_l.shape[-1]):
+                    release = side.cuda_stream
+                else:
+                    side.wait_stream(here)
             else:
                 attn[0](here.cuda_stream)
 
@@ -467,7 +477,7 @@ class _MixedFunction(torch.autograd.Function):
         later = []
         dq_l, dk_l, dv_l, dg, dbeta, dh0, dn_lin = linear_chunk_backward(
             cfg['kind'], q_l, k_l, v_l, g, beta, h0, types, *lin_args, do_lin, dht, cfg['dnats_invalid_linear'], seqs,
-            saved=linear_saved, later=later, meanwhile=softmax_beside, beside=0 if side is None else 4, onto=onto)
+            saved=linear_saved, later=later, release=release, meanwhile=softmax_beside, beside=0 if side is None else 4, onto=onto)
         softmax_beside()                                   # (where the linear branch did not call it)
         lin = [dq_l, dk_l, dv_l]
         if attn is not None:

@@ -151,6 +151,27 @@ static int mixed_phases(const natsl_mixed* m, const int phases, natsl_stream_t s
   return rc;
 }
 
+// The linear branch's chunk states for a backward, next to whose scan the caller puts the softmax branch's backward: the other stream goes
+// on behind the prep kernel, for the reason given above.  Forward and backward of an operator against the dQ kernel free to start at
+// once and the scan behind its workgroups: B4 T4096 H12 128/128 1034 -> 969 us, B1 T32768 H2 4586 -> 3964 (50 % attention); the Mamba
+// operators, where the softmax branch is the longer one anyway, within 1 %.  Behind the whole scan instead, so that the reverse scan
+// follows at once as well: 1799 -> 1581 at B1 T16384 H8, where the linear branch is the longer one, but 1158 -> 1247 at B1 T8192 H16 with
+// 50 % attention and 1022 -> 1109 for Mamba B2 T8192 H16: which one it is the routing decides, on the GPU.
+extern "C" int natsl_linear_chunk_states(int is_delta, const void* q, const void* k, const void* v, const float* g, const void* beta, const float* h0,
+                                         float* ht, void* chunk_states, void* chunk_v_new, const void* types, int types_dtype, int B, int T, int H, int HN, int K,
+                                         int V, int TN, int block, float scale, int flags, void* workspace, size_t workspace_bytes, int dtype,
+                                         const natsl_seq_row* seqs, int n_seqs, int total_units, natsl_stream_t stream, natsl_stream_t beside) {
+  const char* what = "natsl_linear_chunk_states";
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream), other = reinterpret_cast<hipStream_t>(beside);
+  OnDeviceOf device;
+  if (const int rc = device.enter(s, other, what)) return rc;
+  const BesideScan side{order_streams, other};
+  flags |= NATSL_STATES_ONLY;
+  return linear_fwd(is_delta != 0, q, k, v, g, is_delta ? beta : nullptr, h0, nullptr, ht, nullptr, nullptr, chunk_states, is_delta ? chunk_v_new : nullptr,
+                    types, types_dtype, B, T, H, HN, K, V, TN, block, scale, is_delta ? flags : flags & ~NATSL_QK_L2NORM, workspace, workspace_bytes,
+                    dtype, seqs, n_seqs, total_units, stream, other ? &side : nullptr);
+}
+
 extern "C" size_t natsl_mixed_workspace_bytes(int64_t total_chunks, int H) {
   return natsl_linear_workspace_bytes(total_chunks, H) + SOFTMAX_QUEUE_BYTES;
 }

@@ -1,7 +1,7 @@
 // Backward of the softmax branch for gfx950.
 //
-//   delta_kernel   -delta[t] = -sum_v dO[t,v] O[t,v]                                (attns.py:357-372)
-//   dq_kernel      one workgroup per tile of 128 queries, the forward's walk over the visible key chunks:
+//   dq_kernel      one workgroup per tile of 128 queries: -delta[t] = -sum_v dO[t,v] O[t,v] (attns.py:357-372), kept for the
+//                  dk/dv kernel, then the forward's walk over the visible key chunks:
 //                  S^T = K Q^T, P = exp2(S c - lse), dP^T - delta = V dO^T - delta (the accumulators start from -delta),
 //                  dS = P (dP - delta), dQ^T += K^T dS^T (attns.py:383-708)
 //   dkdv_kernel    unit = one 64-key chunk of a kv head, walking the query chunks that see it (the rest of its own
@@ -28,8 +28,8 @@ struct SoftmaxBwdParams {
   const float* lse;
   bf16_t *dq, *dk, *dv;
   float* dnats;   // [B, TN, HQ], zero on entry
-  float* ndelta;  // [B, T, HQ] workspace: -delta
-  int* queue;     // [8] workspace: next unit of each XCD's list for the dk/dv kernel, zeroed by the delta kernel
+  float* ndelta;  // [B, T, HQ] workspace: -delta (written by the dQ kernel, read by the dk/dv kernel)
+  int* queue;     // [8] workspace: next unit of each XCD's list for the dk/dv kernel, zeroed by the dQ kernel
   const void* types;
   int types_dtype;
   const int32_t* idx;
@@ -94,29 +94,6 @@ NATSL_DEVICE bf16x8 pack8(const f32x16& x, const int ss) {
 }
 
 // ---------------------------------------------------------------------------------------------
-template <int DV>
-__global__ __launch_bounds__(256) void delta_kernel(const SoftmaxBwdParams p) {
-  constexpr int LPR = DV / 8, RPB = 256 / LPR;   // lanes per row, rows per workgroup
-  const long long rows = (long long)p.B * p.T * p.HQ;
-  const long long row = (long long)blockIdx.x * RPB + threadIdx.x / LPR;
-  const int seg = threadIdx.x % LPR;
-  if (blockIdx.x == 0 && threadIdx.x < 8) p.queue[threadIdx.x] = 0;   // the dk/dv kernel's work queues (it runs after this kernel)
-  float acc = 0.f;
-  if (row < rows) {
-    const u32x4 a = *reinterpret_cast<const u32x4*>(p.o + row * DV + 8 * seg);
-    const u32x4 b = *reinterpret_cast<const u32x4*>(p.dout + row * DV + 8 * seg);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      acc += __uint_as_float(a[j] << 16) * __uint_as_float(b[j] << 16);
-      acc += __uint_as_float(a[j] & 0xffff0000u) * __uint_as_float(b[j] & 0xffff0000u);
-    }
-  }
-#pragma unroll
-  for (int m = LPR / 2; m >= 1; m >>= 1) acc += __shfl_xor(acc, m);
-  if (row < rows && seg == 0) p.ndelta[row] = -acc;
-}
-
-// ---------------------------------------------------------------------------------------------
 // dQ.  What bounds it: the LDS pipe and the matrix pipe of a SIMD's two waves are about equally busy (per 64-key chunk and wave: K and V by
 // rows, K once more transposed; 2 KS + 2 VS + 4 DT matrix instructions).  K and V chunks come by DMA into two buffers, unpadded and
 // swizzled (bwd_swizzle), so that neither kind of read meets bank conflicts and no register stages them.
@@ -131,6 +108,7 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hf = lane >> 5;
+  if (blockIdx.x == 0 && tid < 8) p.queue[tid] = 0;   // the dk/dv kernel's work queues (it runs after this kernel)
   int n, hq, tile, len, bos, bos_nats;
   if (p.seqs == nullptr) {
     const int nq_tiles = (p.T + QTILE - 1) / QTILE;
@@ -173,7 +151,8 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
   const size_t list_stride = (size_t)p.HN * 2;
   const int n_attn = p.nblk[((size_t)n * p.HN + hn) * 2];
 
-  // Q and dO as B operands (lane = query), lse and delta of the lane's query
+  // Q and dO as B operands (lane = query), lse and delta of the lane's query.  delta is formed here, where dO is in registers anyway: a
+  // kernel of its own read dO once more and stood in front of the two (72 us at B8 T4096 H12 V128, 110 at B4 T8192 H32 V64).
   bf16x8 QB[KS], DOB[VS];
   const int qi = min(q0 + l32, len - 1);
   {
@@ -190,7 +169,19 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
   constexpr bool FOLD = DK + DV > 128;
   f32x16 ndelta;
   {
-    const float d = p.ndelta[(size_t)(bos + qi) * p.HQ + hq];
+    const bf16_t* orow = p.o + ((size_t)(bos + qi) * p.HQ + hq) * DV + 8 * hf;
+    float d = 0.f;
+#pragma unroll
+    for (int s = 0; s < VS; ++s) {
+      const u32x4 a = *reinterpret_cast<const u32x4*>(orow + 16 * s), b = __builtin_bit_cast(u32x4, DOB[s]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        d += __uint_as_float(a[j] << 16) * __uint_as_float(b[j] << 16);
+        d += __uint_as_float(a[j] & 0xffff0000u) * __uint_as_float(b[j] & 0xffff0000u);
+      }
+    }
+    d = -(d + __shfl_xor(d, 32));   // (the lane's half of the columns and the other half of the wave's)
+    if (hf == 0 && q0 + l32 < len) p.ndelta[(size_t)(bos + qi) * p.HQ + hq] = d;
 #pragma unroll
     for (int r = 0; r < 16; ++r) ndelta[r] = d;
   }
@@ -442,7 +433,7 @@ NATSL_DEVICE void dkdv_take_unit(const SoftmaxBwdParams& p, const bool packed, c
 // scalar instructions change it by 1 - 2 %.  Three workgroups per CU at K = V = 64 spill 36 registers a lane and take 390 us.
 constexpr int DKDV_WHOLE_WGS = 2;   // workgroups per CU (registers and LDS)
 // Chunks per CU from which this kernel runs: with fewer, each of its workgroups has a handful of units and takes twice as long over one
-// as the eight waves of the form below.  Whole backward (delta, dQ, dK/dV) of the other form against this one, T 192 .. 8256, 10 % and
+// as the eight waves of the form below.  Whole backward (dQ, dK/dV) of the other form against this one, T 192 .. 8256, 10 % and
 // 40 % attention: 0.83 - 0.95 of its time at seven or eight chunks per CU and short sequences, 0.97 - 1.1 at ten, 1.15 - 1.35 at 32.
 constexpr int DKDV_WHOLE_CHUNKS = 10;
 
@@ -1210,9 +1201,6 @@ static int cu_count() {
 template <int DK, int DV>
 static int launch_bwd(const SoftmaxBwdParams& p, hipStream_t stream) {
   constexpr int KP = DK + 8;
-  const long long rows = (long long)p.B * p.T * p.HQ;
-  constexpr int RPB = 256 / (DV / 8);
-  hipLaunchKernelGGL((delta_kernel<DV>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, stream, p);
   {
     size_t lds = (size_t)2 * 64 * (DK + DV) * sizeof(bf16_t);                               // two buffers of K and V
     const size_t epi = (size_t)128 * KP * sizeof(bf16_t);                                    // the output tile

@@ -79,3 +79,30 @@ def test_an_error_leaves_nothing_unwaited_on_the_side_stream(fake_hip, fields):
     # on one stream there is nothing to wait for
     rc, notes, _ = _run(fake_hip, [(ALL, s, s, 1)], **fields)[0]
     assert rc != 0 and "wait" not in notes
+
+
+def test_chunk_states_release_the_other_stream_before_the_scan(fake_hip):
+    """The linear branch's states for a backward: the other stream waits for what is in front of the scan and not for the scan; without one
+    nothing is ordered, and what is refused has ordered nothing."""
+    child = """
+import ctypes, json, sys
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+fake.fake_notes.restype = ctypes.c_char_p
+f = ctypes.CDLL(sys.argv[2]).natsl_linear_chunk_states
+p, n, i, out = ctypes.c_void_p(1 << 20), ctypes.c_void_p(None), ctypes.c_int, []
+for kind, K, side in ((1, 64, 0x1002), (0, 128, 0x1002), (1, 192, 0), (1, 96, 0x1002)):
+    fake.fake_reset(0)
+    rc = f(i(kind), p, p, p, p, p, n, n, p, p, p, i(1), i(1), i(256), i(2), i(2), i(K), i(64), i(4), i(64), ctypes.c_float(0.1), i(7), p,
+           ctypes.c_size_t(1 << 30), i(1), n, i(0), i(4), ctypes.c_void_p(0x1001), ctypes.c_void_p(side))
+    out.append([rc, fake.fake_notes().decode().strip(), fake.fake_current()])
+print(json.dumps(out))
+"""
+    from neuralattentionsearchlinear_amd import _build, _capi
+    if not os.path.exists(_capi.LIB_PATH):
+        _build.build()
+    assert _capi.BF16 == 1
+    r = subprocess.run([sys.executable, "-c", child, fake_hip, _capi.LIB_PATH], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    beside, ordered = "launch 1001:1 record 1001 wait 1002 launch 1001:1", "launch 1001:1 launch 1001:1"
+    got = json.loads(r.stdout)
+    assert [g[1] for g in got] == [beside, beside, ordered, ""] and [g[0] == 0 for g in got] == [True] * 3 + [False] and {g[2] for g in got} == {0}

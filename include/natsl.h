@@ -63,6 +63,11 @@ typedef struct natsl_seq_row {
   int32_t pad[3];
 } natsl_seq_row;
 
+/* Stores n rows of host memory into a table on the stream's device, in ceil(n / NATSL_SEQ_TABLE_ROWS) launches: the rows are read before the
+ * call returns, and it does not wait for the device.  table starts on 16 bytes. */
+#define NATSL_SEQ_TABLE_ROWS 64
+int natsl_seq_table(const natsl_seq_row* rows, int n, natsl_seq_row* table, natsl_stream_t stream);
+
 int natsl_version(void);
 const char* natsl_last_error(void);
 

@@ -48,6 +48,7 @@ _SIGNATURES = {
                                       c_void_p, c_void_p, c_int,
                                       c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_void_p, c_size_t,
                                       c_int, c_void_p, c_int, c_int, c_void_p]),
+    "natsl_seq_table": (c_int, [c_void_p, c_int, c_void_p, c_void_p]),
     "natsl_linear_chunk_states": (c_int, [c_int] + [c_void_p] * 10 + [c_int] * 9 + [c_float, c_int, c_void_p, c_size_t, c_int, c_void_p, c_int, c_int, c_void_p, c_void_p]),
     "natsl_linear_chunk_bwd": (c_int, [c_int] + [c_void_p] * 9 + [c_int] + [c_void_p] * 12 + [c_int] * 8 + [c_float, c_int, c_int, c_void_p, c_int, c_int, c_void_p]),
     "natsl_norm_gate_bwd_workspace_bytes": (c_size_t, [c_int64, c_int]),

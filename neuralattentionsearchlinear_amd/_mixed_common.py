@@ -65,14 +65,13 @@ SAVE_CHUNK_STATES_MAX_BYTES = 64 << 20
 _PREP_WORKSPACE_BYTES = 17 * 1024   # per chunk and head (csrc/natsl_linear.hip)
 
 
-def _run_side_by_side(dev, seqs, B: int, T: int, H: int, K: int, V: int) -> bool:
+def _run_side_by_side(dev, packed: bool, n_seqs: int, B: int, T: int, H: int, K: int, V: int) -> bool:
     """Whether the softmax branch (forward or backward) goes to the side stream (see CONCURRENT_BRANCHES)."""
     if CONCURRENT_BRANCHES is not None:
         return bool(CONCURRENT_BRANCHES)
-    n_seqs = B if seqs is None else seqs.n_seqs
     if T * B // n_seqs * K < _SIDE_BY_SIDE_TOKENS_X_K:
         return False
-    if seqs is not None:
+    if packed:
         return True                                # chains of different lengths
     index = dev.index if dev.index is not None else torch.cuda.current_device()
     cus = _cu_counts.get(index)
@@ -258,12 +257,15 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
     if types.shape[-1] != 2:
         raise NotImplementedError("routing is built for n_ops == 2")
     TN, HN = types.shape[1], types.shape[2]
-    seqs = pack_sequences(cu_seqlens, cu_seqlens_nats, nats_block_size, dev)
+    # Boundaries that lie on the GPU are read behind everything that can be made without them: the host waits there for the work before this
+    # call, and what it does afterwards the GPU waits for.
+    late = torch.is_tensor(cu_seqlens) and cu_seqlens.dim() == 1 and cu_seqlens.numel() > 1 and not keep_chunk_states
+    seqs = None if late else pack_sequences(cu_seqlens, cu_seqlens_nats, nats_block_size, dev)
     cur, L = _capi.stream_ptr(dev), _capi.lib()
 
     n_prefix, types_attn = 0, types
     if attn_prefix_valid is not None:
-        if not inference or seqs is not None:
+        if not inference or cu_seqlens is not None:
             raise NotImplementedError("a key prefix is built for the prefill operators on unpacked input")
         NP = attn_prefix_valid.shape[1]
         n_prefix = NP * nats_block_size
@@ -279,11 +281,15 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
     T_attn, HQ, KA = q_attn.shape[1:]
     HKV, VA = k_attn.shape[2], v_attn.shape[3]
 
-    n_seqs = seqs.n_seqs if seqs is not None else B
-    total_chunks = seqs.total_chunks if seqs is not None else B * (-(-T // CHUNK_SIZE))
+    if late:
+        n_seqs = cu_seqlens.numel() - 1
+        total_chunks = B * T // CHUNK_SIZE + n_seqs            # (no sequences of T tokens have more)
+    else:
+        n_seqs = seqs.n_seqs if seqs is not None else B
+        total_chunks = seqs.total_chunks if seqs is not None else B * (-(-T // CHUNK_SIZE))
     # every tensor below belongs to the caller's stream; the softmax branch's stream starts after what that stream holds and is
     # waited for before the call returns, so memory that is freed later is only ever used again behind both
-    side = _get_attn_stream(dev) if _run_side_by_side(dev, seqs, B, T, H, K, V) else None
+    side = _get_attn_stream(dev) if _run_side_by_side(dev, cu_seqlens is not None, n_seqs, B, T, H, K, V) else None
     attn_stream = cur if side is None else side.cuda_stream
     want_start = inference and output_final_state
     chunk_states = keep_chunk_states and not want_start
@@ -329,12 +335,14 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
     m.T_attn, m.TN_attn, m.HQ, m.HKV, m.KA, m.VA = T_attn, types_attn.shape[1], HQ, HKV, KA, VA
     m.same_block_visible, m.types_dtype = int(attn_same_block), _capi.dtype_code(types.dtype)
     m.scale_attn, m.scale_linear = scale_attn, scale_lattn
-    if seqs is not None:
-        m.seqs, m.n_seqs, m.total_chunks, m.total_qtiles = seqs.table.data_ptr(), seqs.n_seqs, seqs.total_chunks, seqs.total_qtiles
     m.g, m.types, m.types_attn, m.workspace_bytes = g.data_ptr(), types.data_ptr(), types_attn.data_ptr(), ws_bytes
     for name, t in (("h0", h0), ("ht", ht), ("h_block_start", hs), ("g_block_sum", gs), ("chunk_states", sc), ("chunk_v_new", vn)):
         if t is not None:
             setattr(m, name, t.data_ptr())
+    if late:
+        seqs = pack_sequences(cu_seqlens, cu_seqlens_nats, nats_block_size, dev)
+    if seqs is not None:
+        m.seqs, m.n_seqs, m.total_chunks, m.total_qtiles = seqs.table.data_ptr(), seqs.n_seqs, seqs.total_chunks, seqs.total_qtiles
     ref = ctypes.byref(m)
     if TIMING_HOOK is None:
         _capi.check(L.natsl_mixed_fwd(ref, _CONVERT | _ROUTE | _SOFTMAX | _LINEAR | _JOIN, cur, attn_stream), "natsl_mixed_fwd")
@@ -453,7 +461,7 @@ class _MixedFunction(torch.autograd.Function):
             attn = prepare_attn_nats_bwd(q_a, k_a, v_a, o_attn, types, idx, nblk, None, lse, do_attn, cfg['scale_attn'], cfg['block'], 0,
                                          cfg['attn_same_block'], cfg['dnats_invalid_attn'], None, None, None, True, seqs)
             here = torch.cuda.current_stream(q_l.device)
-            if _run_side_by_side(q_l.device, seqs, *q_l.shape, v_l.shape[-1]):
+            if _run_side_by_side(q_l.device, seqs is not None, B if seqs is None else seqs.n_seqs, *q_l.shape, v_l.shape[-1]):
                 side = _get_attn_stream(q_l.device)
                 if linear_saved is None and hip_backward_is_built(q_l.shape[-1], v_l.shape[-1]):
                     release = side.cuda_stream

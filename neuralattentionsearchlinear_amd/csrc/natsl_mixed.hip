@@ -2,6 +2,7 @@
 // stream or with the softmax branch on a second one.  At small sizes the operator's cost is launches and the host that issues
 // them (fp32 B1 T256 H2: 60 us of kernels behind 200 us of host time as separate calls with torch conversions), so all tensor
 // conversions of a side go out as one launch and nothing returns to the interpreter in between.
+#include <cstring>
 #include <mutex>
 
 #include "natsl_device.h"
@@ -62,6 +63,16 @@ static int cast_all(const natsl_cast* seg, int n, hipStream_t s, const char* wha
   if (wgs > 0x7fffffffll) return fail(NATSL_ERR_UNSUPPORTED, "%s: too much to convert", what);
   hipLaunchKernelGGL((cast_kernel<TO_BF16>), dim3((unsigned)wgs), dim3(256), 0, s, p);
   return check_launch(what);
+}
+
+// Rows of the table of packed sequences travel as arguments of the launch that stores them: a copy from host memory makes the host wait
+// (40 us in front of an operator, 5 for the launch).  64 rows are 2 KiB of arguments.
+struct SeqTableArgs {
+  int4 part[NATSL_SEQ_TABLE_ROWS * 2];   // (a row is 32 bytes)
+};
+__global__ __launch_bounds__(NATSL_SEQ_TABLE_ROWS * 2) void seq_table_kernel(const SeqTableArgs a, int4* table, const int parts) {
+  const int i = threadIdx.x;
+  if (i < parts) table[i] = a.part[i];
 }
 
 // The streams' device is the current one while a call runs: events, kernel attributes and null handles go by the current device, and
@@ -170,6 +181,25 @@ extern "C" int natsl_linear_chunk_states(int is_delta, const void* q, const void
   return linear_fwd(is_delta != 0, q, k, v, g, is_delta ? beta : nullptr, h0, nullptr, ht, nullptr, nullptr, chunk_states, is_delta ? chunk_v_new : nullptr,
                     types, types_dtype, B, T, H, HN, K, V, TN, block, scale, is_delta ? flags : flags & ~NATSL_QK_L2NORM, workspace, workspace_bytes,
                     dtype, seqs, n_seqs, total_units, stream, other ? &side : nullptr);
+}
+
+extern "C" int natsl_seq_table(const natsl_seq_row* rows, int n, natsl_seq_row* table, natsl_stream_t stream) {
+  const char* what = "natsl_seq_table";
+  static_assert(sizeof(natsl_seq_row) == 32, "a row is two pieces of 16 bytes");
+  if (!rows || !table) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
+  if (n <= 0) return fail(NATSL_ERR_INVALID, "%s: non-positive dimension", what);
+  if (reinterpret_cast<uintptr_t>(table) & 15) return fail(NATSL_ERR_INVALID, "%s: the table must start on 16 bytes", what);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  OnDeviceOf device;
+  int rc = device.enter(s, nullptr, what);
+  for (int at = 0; rc == NATSL_OK && at < n; at += NATSL_SEQ_TABLE_ROWS) {
+    const int here = n - at < NATSL_SEQ_TABLE_ROWS ? n - at : NATSL_SEQ_TABLE_ROWS;
+    SeqTableArgs a = {};
+    memcpy(a.part, rows + at, (size_t)here * sizeof(natsl_seq_row));
+    hipLaunchKernelGGL(seq_table_kernel, dim3(1), dim3(NATSL_SEQ_TABLE_ROWS * 2), 0, s, a, reinterpret_cast<int4*>(table + at), 2 * here);
+    rc = check_launch(what);
+  }
+  return rc;
 }
 
 extern "C" size_t natsl_mixed_workspace_bytes(int64_t total_chunks, int H) {

@@ -7,6 +7,7 @@ data dependent (exactly as in the reference).
 """
 from __future__ import annotations
 
+from array import array
 from dataclasses import dataclass
 from typing import Optional
 
@@ -16,6 +17,7 @@ from . import _capi
 
 CHUNK_SIZE = 64
 SOFTMAX_QUERY_TILE = 256
+_TABLE_BY_LAUNCH = 512               # rows of a table that launches carry (64 each, natsl_seq_table); more are copied, which waits for the device
 
 
 @dataclass
@@ -48,11 +50,17 @@ def pack_sequences(cu_seqlens, cu_seqlens_nats, block: int, device) -> Optional[
             raise ValueError("cu_seqlens must be strictly increasing")
         if cn[i + 1] - cn[i] != -(-(b - a) // block):
             raise ValueError("cu_seqlens_nats does not match cu_seqlens and nats_block_size")
-        rows.append([a, b, cn[i], coff, qoff, 0, 0, 0])
+        rows += (a, b, cn[i], coff, qoff, 0, 0, 0)
         coff += -(-(b - a) // CHUNK_SIZE)
         qoff += -(-(b - a) // SOFTMAX_QUERY_TILE)
-    table = torch.tensor(rows, dtype=torch.int32).to(device)
-    return PackedSeqs(table, len(rows), coff, qoff, cn[-1], cu, cn)
+    n = len(cu) - 1
+    rows, device = array('i', rows), torch.device(device)
+    if device.type == 'cuda' and 0 < n <= _TABLE_BY_LAUNCH and device.index in (None, torch.cuda.current_device()):
+        table = torch.empty(n, 8, dtype=torch.int32, device=device)
+        _capi.check(_capi.lib().natsl_seq_table(rows.buffer_info()[0], n, _capi.ptr(table), _capi.stream_ptr(table.device)), "natsl_seq_table")
+    else:
+        table = torch.tensor(rows, dtype=torch.int32).view(n, 8).to(device)
+    return PackedSeqs(table, n, coff, qoff, cn[-1], cu, cn)
 
 
 def _seq_args(seqs: Optional[PackedSeqs], total: int = 0):

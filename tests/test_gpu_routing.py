@@ -113,3 +113,36 @@ def test_layer_select(B, TN, HN, dtype):
         assert torch.equal(types.cpu(), forced) and torch.equal(counts.cpu(), R.n_blocks(forced))
         assert torch.equal(before.cpu(), raw) if want else before is None
         assert torch.equal(fraction, nats_util.hard_select(logits.to(_dev()), True)[1][..., 0].sum(0).float() / (TN * B))
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 512, 513])           # around a launch's 64 rows and the most that launches carry
+def test_table_of_packed_sequences(n):
+    from neuralattentionsearchlinear_amd import nats_util
+    lens = torch.randint(1, 400, (n,), generator=torch.Generator().manual_seed(n)).tolist()
+    cu = [0]
+    for x in lens:
+        cu.append(cu[-1] + x)
+    before = lambda unit: [sum(-(-x // unit) for x in lens[:i]) for i in range(n)]
+    ref = torch.tensor([[cu[i], cu[i + 1], b, c, t, 0, 0, 0] for i, (b, c, t) in enumerate(zip(before(128), before(64), before(256)))])
+    seqs = nats_util.pack_sequences(torch.tensor(cu, device=_dev()), None, 128, _dev())
+    assert seqs.table.dtype == torch.int32 and torch.equal(seqs.table.cpu().long(), ref)
+    assert (seqs.n_seqs, seqs.total_chunks, seqs.total_qtiles) == (n, before(64)[-1] + -(-lens[-1] // 64), before(256)[-1] + -(-lens[-1] // 256))
+
+
+@pytest.mark.parametrize("lens", [[1] * 70, [64, 128, 64], [65, 1, 127, 300], [2500, 700, 3, 1900]])
+def test_boundaries_on_the_gpu_or_on_the_host(lens):
+    """Boundaries that the call reads back behind its preparations (its workspace sized by what they can be at most) give the same bits."""
+    from neuralattentionsearchlinear_amd.mixed_attn_gdn import nats_mixed_attn_gdn
+    cu = [0]
+    for x in lens:
+        cu.append(cu[-1] + x)
+    g = torch.Generator(device=_dev()).manual_seed(3)
+    rn = lambda *s: torch.randn(*s, device=_dev(), generator=g)
+    T, NB = cu[-1], sum(-(-x // 64) for x in lens)
+    q, k, v, beta = rn(1, T, 2, 64).bfloat16(), rn(1, T, 2, 64).bfloat16(), rn(1, T, 2, 64).bfloat16(), torch.sigmoid(rn(1, T, 2)).bfloat16()
+    ty = torch.nn.functional.one_hot((rn(1, NB, 2) > 0).long(), 2).bfloat16()
+    out = [nats_mixed_attn_gdn(q, k, v, q, k, v, None, -torch.nn.functional.softplus(rn(1, T, 2) * 0 + 1), beta, ty, None, cu_seqlens=c, nats_block_size=64,
+                               ops_for_incomplete_chunks="all", output_final_state_gated_delta=True, decay_for_non_gdn_blocks=True)
+           for c in (cu, torch.tensor(cu, device=_dev()), torch.tensor(cu, dtype=torch.int32, device=_dev()))]
+    for o in out[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(o, out[0]))

@@ -18,9 +18,8 @@ struct NarrowParams {
   int D, N;
 };
 
-// Two waves take 32 tokens, half of the contraction each; the weight lies in LDS, row n's 16-byte segment s at s ^ (n % 16), so that the 32 rows that an operand read
-// names meet all banks.  A wave requests up to 24 of a
-// token's segments before the first is used.
+// Two waves take 32 tokens, half of the contraction each; the weight lies in LDS, row n's 16-byte segment s at s ^ (n % 16), so that the 32
+// rows that an operand read names meet all banks.  A wave requests up to 24 of a token's segments before the first is used.
 template <int NB>
 __global__ __launch_bounds__(256) void narrow_fwd_kernel(const NarrowParams p) {
   extern __shared__ __align__(1024) unsigned char smem[];

@@ -336,7 +336,7 @@ def bench_softmax_bwd(args):
         dtype="bf16", data="synthetic", config=dict(workload=args.workload, **w),
         roofline=dict(bound="mfma", kernel="dq_kernel+dkdv_kernel", achieved=flops / (ms * 1e-3) / 1e12, peak=PEAK_BF16_MFMA_TFLOPS,
                       unit="TFLOP/s", frac=flops / (ms * 1e-3) / 1e12 / PEAK_BF16_MFMA_TFLOPS, traffic=None, algorithmic_flops=flops,
-                      note="whole step: delta, dq and dk/dv kernels"))))
+                      note="whole step: dq (with delta) and dk/dv kernels"))))
 
 
 def bench_linear_bwd(args):

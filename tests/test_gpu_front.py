@@ -256,3 +256,27 @@ def test_narrow_products(rows, D, N):
         assert bool(((a[:rows].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * D ** 0.5).all())
         assert bool((a[rows] == 7).all())
     assert L.natsl_narrow_linear(P(x), P(w), P(y), rows, D, N + 2, _capi.stream_ptr(x.device)) != 0
+
+
+@pytest.mark.parametrize("n_a,n_b", [(16, 0), (6, 6), (16, 16), (8, 40), (24, 24), (32, 0)])
+def test_narrow_projections_of_any_count_join_the_backward(n_a, n_b):
+    """The narrow projections' joint weight is made of whole stages where a gradient is asked for, whatever their rows are: one natsl_project_bwd
+    and no natsl_dx_init.  Operands are bf16, sums fp32, one rounding each: 2^-8 in the norm at most."""
+    from neuralattentionsearchlinear_amd import _front
+    torch.manual_seed(n_a + n_b)
+    B, T, D = 2, 130, 256
+    x = torch.randn(B, T, D, device=DEV).bfloat16().requires_grad_(True)
+    ws = [(torch.randn(n, D, device=DEV) / 16).bfloat16().requires_grad_(True) if n else None for n in (128, 128, 256, 256, n_a, n_b)]
+    q, k, v, g, ab, pooled = _front._Project.apply(x, *ws, 64)
+    used = n_a + n_b
+    assert ab.shape[-1] % 32 == 0 and ab.shape[-1] - used < 32
+    dys = [torch.randn_like(t) for t in (q, k, v, g, ab, pooled)]
+    dys[4][..., used:] = 0
+    got = torch.autograd.grad((q, k, v, g, ab, pooled), [x] + [w for w in ws if w is not None], dys)
+    x32, w32 = x.detach().float().requires_grad_(True), [w.detach().float().requires_grad_(True) for w in ws if w is not None]
+    outs = [x32 @ w.t() for w in w32]
+    means = torch.stack([x32[:, t:t + 64].mean(1) for t in range(0, T, 64)], 1)
+    ups = [d.float() for d in dys[:4]] + [d.contiguous() for d in dys[4][..., :used].float().split([n for n in (n_a, n_b) if n], -1)] + [dys[5].float()]
+    want = torch.autograd.grad(outs + [means], [x32] + w32, ups)
+    for a, b in zip(got, want):
+        assert a.shape == b.shape and rel_l2(a.float(), b) <= 2 ** -8

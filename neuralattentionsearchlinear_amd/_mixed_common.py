@@ -7,7 +7,7 @@ from typing import Optional
 import torch
 
 from . import _capi
-from .nats_util import CHUNK_SIZE, PackedSeqs, _seq_args, pack_sequences
+from .nats_util import CHUNK_SIZE, PackedSeqs, _seq_args, pack_sequences_here
 
 _attn_streams: dict = {}
 _cu_counts: dict = {}
@@ -260,7 +260,7 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
     # Boundaries that lie on the GPU are read behind everything that can be made without them: the host waits there for the work before this
     # call, and what it does afterwards the GPU waits for.
     late = torch.is_tensor(cu_seqlens) and cu_seqlens.dim() == 1 and cu_seqlens.numel() > 1 and not keep_chunk_states
-    seqs = None if late else pack_sequences(cu_seqlens, cu_seqlens_nats, nats_block_size, dev)
+    seqs = None if late else pack_sequences_here(cu_seqlens, cu_seqlens_nats, nats_block_size, dev)
     cur, L = _capi.stream_ptr(dev), _capi.lib()
 
     n_prefix, types_attn = 0, types
@@ -340,7 +340,7 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
         if t is not None:
             setattr(m, name, t.data_ptr())
     if late:
-        seqs = pack_sequences(cu_seqlens, cu_seqlens_nats, nats_block_size, dev)
+        seqs = pack_sequences_here(cu_seqlens, cu_seqlens_nats, nats_block_size, dev)
     if seqs is not None:
         m.seqs, m.n_seqs, m.total_chunks, m.total_qtiles = seqs.table.data_ptr(), seqs.n_seqs, seqs.total_chunks, seqs.total_qtiles
     ref = ctypes.byref(m)
@@ -447,7 +447,7 @@ class _MixedFunction(torch.autograd.Function):
         beta = beta if beta.numel() else None
         h0 = h0 if ctx.has_h0 else None
         B, NB, HN, _ = types.shape
-        seqs = pack_sequences(cfg['cu_seqlens'], cfg['cu_seqlens_nats'], cfg['block'], types.device)
+        seqs = pack_sequences_here(cfg['cu_seqlens'], cfg['cu_seqlens_nats'], cfg['block'], types.device)
         if do_lin is None:
             do_lin = torch.zeros(*q_l.shape[:3], v_l.shape[-1], dtype=torch.float32, device=q_l.device)
         if do_attn is not None:

@@ -6,7 +6,7 @@ from typing import Optional
 import torch
 
 from . import _capi
-from .nats_util import PackedSeqs, _seq_args, pack_sequences
+from .nats_util import PackedSeqs, _seq_args, pack_sequences_here
 
 
 def parallel_attn_nats_fwd(
@@ -82,7 +82,7 @@ def prepare_attn_nats_bwd(q, k, v, o, nats_block_types, nats_block_indices, n_na
     if g_cumsum is not None or sliding_window_size is not None or not is_causal or OFFSET_ATTN != 0:
         raise NotImplementedError("only the causal backward without g_cumsum / sliding window is built")
     if seqs is None and cu_seqlens is not None:
-        seqs = pack_sequences(cu_seqlens, cu_seqlens_nats, NAtS_block_size, q.device)
+        seqs = pack_sequences_here(cu_seqlens, cu_seqlens_nats, NAtS_block_size, q.device)
     if seqs is not None and q.shape[0] != 1:
         raise ValueError("batch size must be 1 when cu_seqlens are provided")
     if scale is None:
@@ -122,7 +122,7 @@ class AttentionNAtSFunction(torch.autograd.Function):
                 compute_dnats_for_invalid_blocks_attn=False, is_causal=True, store_msk=False):
         if g is not None:
             raise NotImplementedError("use_g_for_attn is disabled in every reference layer and is not built")
-        seqs = pack_sequences(cu_seqlens, cu_seqlens_nats, NAtS_block_size, q.device)
+        seqs = pack_sequences_here(cu_seqlens, cu_seqlens_nats, NAtS_block_size, q.device)
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
         o, lse, _ = parallel_attn_nats_fwd(q, k, v, nats_block_types, nats_block_indices, None, scale, NAtS_block_size,
                                            offset_attn=offset_attn, compute_incomplete_chunk_scores=compute_incomplete_chunk_scores,

@@ -22,7 +22,8 @@ _TABLE_BY_LAUNCH = 512               # rows of a table that launches carry (64 e
 
 @dataclass
 class PackedSeqs:
-    """Device table describing packed sequences (cu_seqlens of the reference)."""
+    """Device table describing packed sequences (cu_seqlens of the reference).  pack_sequences' are complete when they are handed out: any
+    stream or thread may take them."""
     table: torch.Tensor          # int32 [N, 8] rows of natsl_seq_row
     n_seqs: int
     total_chunks: int
@@ -35,6 +36,16 @@ class PackedSeqs:
 def pack_sequences(cu_seqlens, cu_seqlens_nats, block: int, device) -> Optional[PackedSeqs]:
     """Build the per-sequence table (one host read of cu_seqlens; the reference's varlen helpers
     do the same at fla prepare_chunk_indices)."""
+    return _pack_sequences(cu_seqlens, cu_seqlens_nats, block, device, False)
+
+
+def pack_sequences_here(cu_seqlens, cu_seqlens_nats, block: int, device) -> Optional[PackedSeqs]:
+    """pack_sequences for a call that takes the table on the current stream, or on one that it orders behind it: a table of up to
+    _TABLE_BY_LAUNCH rows is stored by launches on that stream, without waiting for the device."""
+    return _pack_sequences(cu_seqlens, cu_seqlens_nats, block, device, True)
+
+
+def _pack_sequences(cu_seqlens, cu_seqlens_nats, block, device, by_launch):
     if cu_seqlens is None:
         return None
     cu = [int(x) for x in (cu_seqlens.tolist() if torch.is_tensor(cu_seqlens) else cu_seqlens)]
@@ -53,9 +64,11 @@ def pack_sequences(cu_seqlens, cu_seqlens_nats, block: int, device) -> Optional[
         rows += (a, b, cn[i], coff, qoff, 0, 0, 0)
         coff += -(-(b - a) // CHUNK_SIZE)
         qoff += -(-(b - a) // SOFTMAX_QUERY_TILE)
-    n = len(cu) - 1
+    n = len(rows) // 8
     rows, device = array('i', rows), torch.device(device)
-    if device.type == 'cuda' and 0 < n <= _TABLE_BY_LAUNCH and device.index in (None, torch.cuda.current_device()):
+    # (a captured graph takes launches, and no copy that is waited for)
+    if device.type == 'cuda' and 0 < n <= _TABLE_BY_LAUNCH and device.index in (None, torch.cuda.current_device()) and \
+            (by_launch or torch.cuda.is_current_stream_capturing()):
         table = torch.empty(n, 8, dtype=torch.int32, device=device)
         _capi.check(_capi.lib().natsl_seq_table(rows.buffer_info()[0], n, _capi.ptr(table), _capi.stream_ptr(table.device)), "natsl_seq_table")
     else:
@@ -107,7 +120,7 @@ def mean_pooling(x: torch.Tensor, chunk_size: int, cu_seqlens=None, seqs: Option
     if squeeze:
         x = x.unsqueeze(-2)
     if cu_seqlens is not None and seqs is None:
-        seqs = pack_sequences(cu_seqlens, None, chunk_size, x.device)
+        seqs = pack_sequences_here(cu_seqlens, None, chunk_size, x.device)
     if torch.is_grad_enabled() and x.requires_grad:
         if seqs is not None:
             raise NotImplementedError("the pooling backward is not built for packed sequences")

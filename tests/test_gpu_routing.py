@@ -124,9 +124,27 @@ def test_table_of_packed_sequences(n):
         cu.append(cu[-1] + x)
     before = lambda unit: [sum(-(-x // unit) for x in lens[:i]) for i in range(n)]
     ref = torch.tensor([[cu[i], cu[i + 1], b, c, t, 0, 0, 0] for i, (b, c, t) in enumerate(zip(before(128), before(64), before(256)))])
-    seqs = nats_util.pack_sequences(torch.tensor(cu, device=_dev()), None, 128, _dev())
-    assert seqs.table.dtype == torch.int32 and torch.equal(seqs.table.cpu().long(), ref)
-    assert (seqs.n_seqs, seqs.total_chunks, seqs.total_qtiles) == (n, before(64)[-1] + -(-lens[-1] // 64), before(256)[-1] + -(-lens[-1] // 256))
+    for make in (nats_util.pack_sequences, nats_util.pack_sequences_here):
+        seqs = make(torch.tensor(cu, device=_dev()), None, 128, _dev())
+        assert seqs.table.dtype == torch.int32 and torch.equal(seqs.table.cpu().long(), ref)
+        assert (seqs.n_seqs, seqs.total_chunks, seqs.total_qtiles) == (n, before(64)[-1] + -(-lens[-1] // 64), before(256)[-1] + -(-lens[-1] // 256))
+
+
+@pytest.mark.parametrize("n", [3, 512, 513])
+def test_a_packed_table_is_complete_when_it_is_handed_out(n):
+    """A table made on a stream that still has work in front of it is there for every other stream as soon as the call returns."""
+    from neuralattentionsearchlinear_amd import nats_util
+    cu = [100 * i for i in range(n + 1)]
+    maker, taker = torch.cuda.Stream(), torch.cuda.Stream()
+    for _ in range(3):
+        with torch.cuda.stream(maker):
+            torch.full((n, 8), -1, dtype=torch.int32, device=_dev())          # (what a table not yet written would hold)
+            torch.cuda._sleep(20_000_000)
+            seqs = nats_util.pack_sequences(cu, None, 64, _dev())
+        with torch.cuda.stream(taker):
+            got = seqs.table.cpu()
+        assert got[:, 0].tolist() == cu[:-1] and got[:, 1].tolist() == cu[1:]
+        torch.cuda.synchronize()
 
 
 @pytest.mark.parametrize("lens", [[1] * 70, [64, 128, 64], [65, 1, 127, 300], [2500, 700, 3, 1900]])

@@ -385,7 +385,9 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
             if op_type_last_chunk is None:
                 raise AssertionError("op_type_last_chunk is required when the input ends on a block boundary")
             last, n = op_type_last_chunk, ht.shape[0]
-            if last.is_cuda and last.device == dev and last.dtype in (torch.bfloat16, torch.float32) and last.dim() == 3 and last.shape[0] == n and \
+            # (a launch goes to the current device, torch's operations to their tensors')
+            if last.is_cuda and last.device == dev and dev.index in (None, torch.cuda.current_device()) and \
+                    last.dtype in (torch.bfloat16, torch.float32) and last.dim() == 3 and last.shape[0] == n and \
                     last.stride(2) == 1 and H % last.shape[1] == 0 and last.shape[2] > 1 and n * H <= 65535:
                 h_start = torch.empty_like(ht)
                 rc = L.natsl_roll_state(ht.data_ptr(), hs.data_ptr(), gs.data_ptr() if decay_non_linear else None, last.data_ptr(),

@@ -56,9 +56,10 @@ class _TailSeg(ctypes.Structure):
 
 def _block_tails(tensors, block: int, rest: int):
     """For each x [B, T, ...] of `tensors`: a new tensor [B, block, ...] with the last `rest` tokens of x and zeros behind them, all of
-    them in one launch; None where a tensor is not what that launch reads (the caller fills and copies then)."""
+    them in one launch on the current device; None where a tensor is not what that launch reads (the caller fills and copies then)."""
+    here = torch.cuda.current_device() if tensors[0].is_cuda else None
     for x in tensors:
-        if not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float32) or not x.is_contiguous() or x.device != tensors[0].device or \
+        if not x.is_cuda or x.device.index != here or x.dtype not in (torch.bfloat16, torch.float32) or not x.is_contiguous() or \
                 x.shape[:2] != tensors[0].shape[:2] or x.numel() == 0 or (x.requires_grad and torch.is_grad_enabled()):
             return None
     x = tensors[0]

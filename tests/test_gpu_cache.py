@@ -302,6 +302,27 @@ def test_rolled_state(H, HN, K, V, decay, dtype):
     assert torch.equal(out, torch.where(lin, ht, hs * torch.exp(gs).view(2, H, 1, 1) if decay else hs))
 
 
+def test_another_current_device_takes_torch(monkeypatch):
+    """Where the tensors' device is not the current one, what torch computes on the tensors' is not launched on the current one instead."""
+    from neuralattentionsearchlinear_amd import _capi, cache
+    from neuralattentionsearchlinear_amd.mixed_attn_gdn import nats_mixed_attn_gdn_chunk_inference
+    torch.manual_seed(0)
+    B, T, H, K = 2, 128, 2, 64
+    q, k, v = (torch.randn(B, T, H, K, device=DEV).bfloat16() for _ in range(3))
+    g, beta = -torch.rand(B, T, H, device=DEV), torch.rand(B, T, H, device=DEV).bfloat16()
+    ty = torch.nn.functional.one_hot(torch.randint(0, 2, (B, 2, H), device=DEV), 2).bfloat16()
+    call = lambda: nats_mixed_attn_gdn_chunk_inference(q, k, v, q, k, v, None, g, beta, ty, ty[:, -1], None, ops_for_incomplete_chunks='all',
+                                                       output_final_state_gated_delta=True, decay_for_non_gdn_blocks=True)
+    tails = lambda: cache._block_tails((k, v), 64, 5)
+    want = call()
+    assert tails() is not None
+    monkeypatch.setattr(_capi.lib(), 'natsl_roll_state', None)           # (a call would raise)
+    monkeypatch.setattr(torch.cuda, 'current_device', lambda: 1)
+    assert tails() is None
+    for a, b in zip(call(), want):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("T,rest", [(64, 0), (200, 8), (127, 63), (2047, 1023)])
 def test_kept_block_notes(T, rest):
     """The validity flags, and the sum of g over the incomplete block: 1e-6 of the terms' sum is ten fp32 roundings of it."""

@@ -98,6 +98,31 @@ NATSL_DEVICE void mix_softmax(float& a, float& b) {
   b = __uint_as_float(pack_bf16x2(e1 / (e0 + e1), 0.f) << 16);
 }
 
+// The sum of part[k][col] (n_col columns) over every TY-th k from `first` on, sixteen loads in flight: a thread's share of a column's sum.
+template <int TY>
+NATSL_DEVICE float column_share(const float* part, const int col, const int first, const int n_part, const int n_col) {
+  const float* src = part + col;
+  float acc = 0.f;
+  int k = first;
+  for (; k + 15 * TY < n_part; k += 16 * TY) {
+    float v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = src[(size_t)(k + TY * u) * n_col];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 16; ++u) acc += v[u];
+  }
+  for (; k + 3 * TY < n_part; k += 4 * TY) {
+    float v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = src[(size_t)(k + TY * u) * n_col];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) acc += v[u];
+  }
+  for (; k < n_part; k += TY) acc += src[(size_t)k * n_col];
+  return acc;
+}
+
 // Per-sequence descriptor for packed (variable-length) input; one row per sequence.
 struct SeqRow {
   int bos;        // first token (flat index)

@@ -339,7 +339,7 @@ struct GatesParams {
   const float* dg; const bf16_t* dbeta; const float* ddt;
   bf16_t* dab; float* part;
   long long rows;
-  int H, ld, dtype, neg;
+  int H, ld, dtype, neg, iters;                    // iters: batches of rows of a backward workgroup
 };
 
 __global__ __launch_bounds__(256) void gates_kernel(const GatesParams p) {
@@ -356,7 +356,10 @@ __global__ __launch_bounds__(256) void gates_kernel(const GatesParams p) {
   }
 }
 
-constexpr int GATES_ITERS = 2;
+// Batches of 256 / H rows of a backward workgroup: two, so that the launch fills the chip, and more where that makes more than GATES_WGS
+// workgroups, each of which leaves 2 H sums to be written and read again (32768 rows of 256 heads: 33 MB from two batches each; with at most
+// 1024, 2048, 4096 workgroups 67, 58, 58 us, 65536 rows of 64 heads 37, 33, 34).
+constexpr int GATES_WGS = 2048;
 // thread = (row of the workgroup's batch, head); the rows' shares of the two parameter gradients are added through LDS in order
 __global__ __launch_bounds__(256) void gates_bwd_kernel(const GatesParams p) {
   __shared__ float red[2][256];
@@ -364,8 +367,8 @@ __global__ __launch_bounds__(256) void gates_bwd_kernel(const GatesParams p) {
   float sa = 0.f, sb = 0.f;
   const float A = expf(ldf(p.a_log, p.dtype, h)), bias = ldf(p.dt_bias, p.dtype, h);
   if (ri < in) {
-    for (int it = 0; it < GATES_ITERS; ++it) {
-      const long long row = ((long long)blockIdx.x * GATES_ITERS + it) * in + ri;
+    for (int it = 0; it < p.iters; ++it) {
+      const long long row = ((long long)blockIdx.x * p.iters + it) * in + ri;
       if (row >= p.rows) break;
       const float x = bf16_to_f32(p.ab[row * p.ld + h]) + bias;
       const float dt = softplus_gate(x), sg = x > 20.f ? 1.f : sigmoid_gate(x);
@@ -399,19 +402,25 @@ __global__ __launch_bounds__(256) void gates_bwd_kernel(const GatesParams p) {
     p.part[(size_t)blockIdx.x * 2 * p.H + p.H + threadIdx.x] = tb;
   }
 }
+// 16 adjacent columns (sums for A_log, then for dt_bias) per workgroup, 64 thread rows.  With one workgroup for all columns and a load at a
+// time it is this kernel that decides from 16 heads on (both kernels, 32768 rows, such a one / this one, us: 6 heads 8.9 / 8.9, 16 15.3 / 9.7,
+// 32 41.5 / 13.1, 256 2276 / 58; 65536 rows of 64 heads 300 / 32).
+constexpr int GATES_COLS = 16;
 __global__ __launch_bounds__(1024) void gates_reduce_kernel(const float* part, void* da_log, void* ddt_bias, const int n_part, const int H, const int dtype) {
-  __shared__ float red[1024];
-  const int cols = 2 * H, in = 1024 / cols, c = threadIdx.x % cols, r = threadIdx.x / cols;
-  float t = 0.f;
-  if (r < in)
-    for (int k = r; k < n_part; k += in) t += part[(size_t)k * cols + c];
-  red[threadIdx.x] = t;
+  constexpr int TY = 1024 / GATES_COLS;
+  __shared__ float sums[16][GATES_COLS];
+  const int tx = threadIdx.x % GATES_COLS, ty = threadIdx.x / GATES_COLS, c = blockIdx.x * GATES_COLS + tx;
+  float t = c < 2 * H ? column_share<TY>(part, c, ty, n_part, 2 * H) : 0.f;
+  t += __shfl_xor(t, 16);                          // (a wave holds four thread rows)
+  t += __shfl_xor(t, 32);
+  if ((threadIdx.x & 63) < GATES_COLS) sums[threadIdx.x >> 6][tx] = t;
   __syncthreads();
-  if ((int)threadIdx.x < cols) {
-    float s = 0.f;
-    for (int k = 0; k < in; ++k) s += red[k * cols + threadIdx.x];
-    if (c < H) stf(da_log, dtype, c, s);
-    else stf(ddt_bias, dtype, c - H, s);
+  if (ty == 0 && c < 2 * H) {
+    t = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) t += sums[r][tx];
+    if (c < H) stf(da_log, dtype, c, t);
+    else stf(ddt_bias, dtype, c - H, t);
   }
 }
 
@@ -652,7 +661,11 @@ extern "C" int natsl_gates_fwd(const void* ab, const void* a_log, const void* dt
   return check_launch(what);
 }
 
-static long long gates_wgs(int64_t rows, int H) { const int in = 256 / H; return (rows + (long long)in * GATES_ITERS - 1) / ((long long)in * GATES_ITERS); }
+static int gates_iters(int64_t rows, int H) {
+  const long long batches = (rows + 256 / H - 1) / (256 / H), per = (batches + GATES_WGS - 1) / GATES_WGS;
+  return (int)(per < 2 ? 2 : per);
+}
+static long long gates_wgs(int64_t rows, int H) { const long long n = (long long)(256 / H) * gates_iters(rows, H); return (rows + n - 1) / n; }
 extern "C" size_t natsl_gates_bwd_workspace_bytes(int64_t rows, int H) {
   return rows > 0 && H > 0 && H <= 256 ? (size_t)gates_wgs(rows, H) * 2 * H * sizeof(float) : 0;
 }
@@ -668,11 +681,12 @@ extern "C" int natsl_gates_bwd(const void* ab, const void* a_log, const void* dt
   p.ab = (const bf16_t*)ab; p.a_log = a_log; p.dt_bias = dt_bias; p.dg = dg; p.dbeta = (const bf16_t*)dbeta; p.ddt = ddt; p.dab = (bf16_t*)dab;
   p.beta = delta ? (bf16_t*)dab : nullptr;      // (only tells the kernel that the rows hold b)
   p.part = reinterpret_cast<float*>(workspace); p.rows = rows; p.H = H; p.ld = ld; p.dtype = param_dtype; p.neg = neg_eigval;
+  p.iters = gates_iters(rows, H);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const long long wgs = gates_wgs(rows, H);
   hipLaunchKernelGGL(gates_bwd_kernel, dim3((unsigned)wgs), dim3(256), 0, s, p);
   if ((rc = check_launch(what)) != NATSL_OK) return rc;
-  hipLaunchKernelGGL(gates_reduce_kernel, dim3(1), dim3(1024), 0, s, p.part, da_log, ddt_bias, (int)wgs, H, param_dtype);
+  hipLaunchKernelGGL(gates_reduce_kernel, dim3((unsigned)cdiv(2 * H, GATES_COLS)), dim3(1024), 0, s, p.part, da_log, ddt_bias, (int)wgs, H, param_dtype);
   return check_launch(what);
 }
 

@@ -227,20 +227,7 @@ __global__ __launch_bounds__(1024) void colsum_reduce_kernel(const float* part, 
   __shared__ float sums[TY][COLSUM_COLS];
   const int tx = threadIdx.x % COLSUM_COLS, ty = threadIdx.x / COLSUM_COLS;
   const int i = blockIdx.x * COLSUM_COLS + tx;
-  float acc = 0.f;
-  if (i < n_col) {
-    const float* src = part + i;
-    int k = ty;
-    for (; k + 15 * TY < n_part; k += 16 * TY) {
-      float v[16];
-#pragma unroll
-      for (int u = 0; u < 16; ++u) v[u] = src[(size_t)(k + TY * u) * n_col];
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int u = 0; u < 16; ++u) acc += v[u];
-    }
-    for (; k < n_part; k += TY) acc += src[(size_t)k * n_col];
-  }
+  const float acc = i < n_col ? column_share<TY>(part, i, ty, n_part, n_col) : 0.f;
   sums[ty][tx] = acc;
   __syncthreads();
   if (ty == 0 && i < n_col) {

@@ -55,6 +55,14 @@ def test_argument_validation_needs_no_gpu():
     assert rc == -2 and b"32-bit" in L.natsl_last_error()
 
 
+def test_workspaces_stay_small():
+    """Partial sums are bounded by the chip and not by the tokens: a row of 2 H sums for each of 2048 workgroups of the gates' backward."""
+    L = _lib()
+    for rows in (1, 4096, 32768, 1 << 20, 1 << 24):
+        for H in (1, 6, 16, 33, 64, 256):
+            assert 0 < L.natsl_gates_bwd_workspace_bytes(rows, H) <= 2048 * 2 * H * 4
+
+
 def test_no_cpu_fallback():
     import torch
     from neuralattentionsearchlinear_amd import _capi

@@ -203,6 +203,40 @@ def test_dx_init(B, T, D, N, block, pool):
     assert bool(((dx.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5).all())
 
 
+# around a batch of 256 / H rows, a workgroup's batches and the most workgroups; columns that fill no group of the sums' kernel
+@pytest.mark.parametrize("rows,H,delta,neg", [(1, 1, True, False), (85, 6, True, True), (4099, 16, False, False), (9001, 100, True, False), (5000, 256, True, True),
+                                              (140001, 32, False, False), (50000, 200, True, False)])
+def test_gates_backward(rows, H, delta, neg):
+    """natsl_gates_bwd against 64 bits.  bf16 outputs are rounded once; a parameter's gradient is a sum of fp32 terms that are within 4e-6 of
+    exact ones (expf, log1pf, a few products) and loses a rounding where it is rounded to fp32."""
+    from neuralattentionsearchlinear_amd import _capi
+    torch.manual_seed(rows)
+    L, P = _capi.lib(), _capi.ptr
+    ld = 2 * H + 3 if delta else H + 5
+    ab, a_log, bias = torch.randn(rows, ld, device=DEV).bfloat16(), torch.randn(H, device=DEV), torch.randn(H, device=DEV)
+    dg, ddt = torch.randn(rows, H, device=DEV), None if delta else torch.randn(rows, H, device=DEV)
+    db = torch.randn(rows, H, device=DEV).bfloat16() if delta else None
+    dab, da, dd = torch.full_like(ab, 7.), torch.empty_like(a_log), torch.empty_like(bias)
+    n = L.natsl_gates_bwd_workspace_bytes(rows, H)
+    ws = torch.empty(n, dtype=torch.uint8, device=DEV)
+    rc = L.natsl_gates_bwd(P(ab), P(a_log), P(bias), P(dg), P(db) if delta else None, None if delta else P(ddt), int(delta), P(dab), P(da), P(dd), P(ws), n, rows, H,
+                           ld, int(neg), _capi.F32, _capi.stream_ptr(dg.device))
+    _capi.check(rc, "natsl_gates_bwd")
+    x, A = ab[:, :H].double() + bias.double(), a_log.double().exp()
+    dt = torch.nn.functional.softplus(x, threshold=1e9)
+    ta = dg.double() * -A * dt
+    tb = ((0. if delta else ddt.double()) - A * dg.double()) * x.sigmoid()
+    close = lambda got, ref, terms: bool(((got.double() - ref).abs() <= 2.0 ** -24 * ref.abs() + 4e-6 * terms.abs().sum(0)).all())
+    assert close(da, ta.sum(0), ta) and close(dd, tb.sum(0), tb)
+    assert bool(((dab[:, :H].double() - tb).abs() <= 2.0 ** -8 * tb.abs() + 1e-5).all())
+    if delta:
+        s = ab[:, H:2 * H].double().sigmoid().bfloat16().double()
+        ref = (2. if neg else 1.) * db.double() * s * (1 - s)
+        # (a sigmoid at the edge of two bf16 values may round to the other: s (1 - s) changes by less than 2^-8)
+        assert bool(((dab[:, H:2 * H].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2.0 ** -7 * db.double().abs()).all())
+    assert not bool(dab[:, (2 if delta else 1) * H:].any())
+
+
 # (tokens, input width, projections): rows and columns behind the last tile, tiles of each height, more tiles than workgroups
 @pytest.mark.parametrize("B,T,D,widths,block", [
     (1, 1, 128, (8,), 64), (1, 129, 160, (264, 32), 64), (3, 100, 416, (256, 64, 512, 32), 64), (2, 8200, 128, (520, 1024), 256),

@@ -26,17 +26,24 @@ constexpr int WG_TILE = WG_T * WG_ROW;         // 16 KiB per operand
 constexpr int WG_STAGE = 2 * WG_TILE;
 constexpr int WG_STAGES = 4;
 
-struct WgradSeg { const bf16_t* dy; bf16_t* out; int n, ld, tile0; };   // tile0: first row of tiles
+struct WgradSeg { const bf16_t* dy; bf16_t* out; int n, ld, tile0, block0; };   // tile0, block0: first row of tiles, of 32-row blocks
 struct WgradParams {
   const bf16_t* x;
   float* part;
-  int ldx, D, n_seg, tiles_d, tiles, splits, units;
+  int ldx, D, n_seg, tiles_d, tiles, blocks, splits, units;   // blocks: 32-row blocks of all weights
   long long T, slice;                          // tokens; tokens per slice (a multiple of WG_T)
   WgradSeg seg[NATSL_WGRAD_SEGS];
 };
 
 NATSL_DEVICE void wg_dma(const void* base, const unsigned voff, const unsigned lds) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(lds) : "memory", "m0");
+}
+
+// Partial sums lie as strips of 32 rows x 256 columns (wg_strip), those that the weights have and no others: whole tiles of a 24-row weight
+// would be eight times as much (24 x 768 over 32768 tokens: 59 MiB, 7.4 as strips).
+constexpr int WG_STRIP = 32 * WG_N;
+NATSL_DEVICE size_t wg_strip(const WgradParams& p, const int split, const int td, const int block) {
+  return (((size_t)split * p.tiles_d + td) * p.blocks + block) * WG_STRIP;
 }
 
 __global__ __launch_bounds__(256, 1) void wgrad_kernel(const WgradParams p) {
@@ -192,14 +199,14 @@ __global__ __launch_bounds__(256, 1) void wgrad_kernel(const WgradParams p) {
   for (; st < n_st; ++st) stage(std::false_type{}, std::false_type{}, st);
 
   // lane: column d = lane%32 of each 32x32 tile, rows 8*(r/4) + 4*(lane/32) + r%4: four rows of a column per 16-byte store
-  float* dst = p.part + ((size_t)u * 4 + wave) * (size_t)(WG_N * WG_N / 4) + lane * 4;
+  float* dst = p.part + wg_strip(p, split, td, sg.block0 + (tn - sg.tile0) * 8 + 4 * (wave >> 1)) + (wave & 1) * 4096 + lane * 4;
 #pragma unroll
   for (int a = 0; a < 4; ++a)
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        if (a < blocks) *reinterpret_cast<f32x4*>(dst + ((a * 4 + b) * 4 + q) * 256) = (f32x4){acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]};
+        if (a < blocks) *reinterpret_cast<f32x4*>(dst + a * WG_STRIP + (b * 4 + q) * 256) = (f32x4){acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]};
 }
 
 // Adds the slices' partial tiles in order and writes the gradient: a workgroup takes one 32 x 32 block of a tile per wave.
@@ -217,8 +224,8 @@ __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const WgradParams p) 
   f32x4 sum[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) sum[q] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  const float* src = p.part + ((size_t)tile * 4 + wave) * (size_t)(WG_N * WG_N / 4) + (size_t)ab * 1024 + lane * 4;
-  const size_t step = (size_t)p.tiles * (WG_N * WG_N);
+  const float* src = p.part + wg_strip(p, 0, td, sg.block0 + (tn - sg.tile0) * 8 + 4 * (wave >> 1) + (ab >> 2)) + (wave & 1) * 4096 + (ab & 3) * 1024 + lane * 4;
+  const size_t step = (size_t)p.tiles_d * p.blocks * WG_STRIP;
   int s = 0;
   for (; s + 6 <= p.splits; s += 6) {          // (six slices on their way at a time; one by one a slice takes a round trip, 0.4 us)
     f32x4 v[6][4];
@@ -257,9 +264,8 @@ static int wgrad_cus() {
 }
 
 // Slices of the tokens: a CU holds one unit at a time, so the launch takes ceil(tiles * slices / CUs) rounds of T / slices tokens
-// (measured: 17 ns a token), and every slice writes and reads its partial tiles once more (0.1 us a whole tile; full: whole tiles'
-// worth of rows.  24 rows x 768 columns over 32768 tokens: 45 us with
-// 32 slices of whole tiles, 28 with 85 of the blocks that there are).
+// (measured: 17 ns a token), and every slice writes and reads its partial sums once more (0.1 us a whole tile; full: whole tiles'
+// worth of rows.  24 rows x 768 columns over 32768 tokens: 37 us with 32 slices of whole tiles, 27 with 85 of the strips that there are).
 static int wgrad_splits(long long T, int tiles, double full) {
   const int cus = wgrad_cus();
   int best = 1;
@@ -280,18 +286,19 @@ static int wgrad_plan(WgradParams& p, const natsl_wgrad_seg* segs, int n_seg, co
   p.x = (const bf16_t*)x; p.ldx = ldx; p.D = D; p.n_seg = n_seg; p.T = T;
   p.tiles_d = cdiv(D, WG_N);
   int rows = 0;
-  double full = 0.;
+  long long blocks = 0;
   for (int i = 0; i < NATSL_WGRAD_SEGS; ++i) {
-    if (i >= n_seg) { p.seg[i] = {nullptr, nullptr, 0, 0, 1 << 30}; continue; }
+    if (i >= n_seg) { p.seg[i] = {nullptr, nullptr, 0, 0, 1 << 30, 0}; continue; }
     const natsl_wgrad_seg& s = segs[i];
     if (s.n <= 0 || s.ld < s.n || s.n % 8 || s.ld % 8) return fail(NATSL_ERR_UNSUPPORTED, "%s: a gradient's width and row stride must be multiples of 8", what);
     if ((long long)WG_T * s.ld * 2 > 0x7fffffffll || (long long)WG_T * ldx * 2 > 0x7fffffffll) return fail(NATSL_ERR_UNSUPPORTED, "%s: rows too long", what);
-    p.seg[i] = {(const bf16_t*)s.dy, (bf16_t*)s.out, s.n, s.ld, rows};
+    p.seg[i] = {(const bf16_t*)s.dy, (bf16_t*)s.out, s.n, s.ld, rows, (int)blocks};
     rows += cdiv(s.n, WG_N);
-    full += cdiv(s.n, 32) / 8. * p.tiles_d;
+    blocks += cdiv(s.n, 32);
   }
   p.tiles = rows * p.tiles_d;
-  const int splits = wgrad_splits(T, p.tiles, full);
+  p.blocks = (int)blocks;
+  const int splits = wgrad_splits(T, p.tiles, blocks / 8. * p.tiles_d);
   p.slice = (T + splits - 1) / splits;
   p.slice = (p.slice + WG_T - 1) / WG_T * WG_T;
   p.splits = (int)((T + p.slice - 1) / p.slice);
@@ -300,6 +307,8 @@ static int wgrad_plan(WgradParams& p, const natsl_wgrad_seg* segs, int n_seg, co
   return NATSL_OK;
 }
 
+static size_t wgrad_bytes(const WgradParams& p) { return (size_t)p.splits * p.tiles_d * p.blocks * WG_STRIP * sizeof(float); }
+
 }  // namespace natsl
 
 using namespace natsl;
@@ -307,7 +316,7 @@ using namespace natsl;
 extern "C" size_t natsl_wgrad_workspace_bytes(const natsl_wgrad_seg* segs, int n_seg, int64_t T, int D) {
   WgradParams p;
   if (wgrad_plan(p, segs, n_seg, nullptr, T, D, D, "natsl_wgrad") != NATSL_OK) return 0;
-  return (size_t)p.units * WG_N * WG_N * sizeof(float);
+  return wgrad_bytes(p);
 }
 
 extern "C" int natsl_wgrad(const natsl_wgrad_seg* segs, int n_seg, const void* x, int64_t T, int D, int ldx, void* workspace,
@@ -323,7 +332,7 @@ extern "C" int natsl_wgrad(const natsl_wgrad_seg* segs, int n_seg, const void* x
     low |= (uintptr_t)segs[i].dy;
   }
   if (low & 15) return fail(NATSL_ERR_INVALID, "%s: tensors must start on 16 bytes", what);
-  if (workspace_bytes < (size_t)p.units * WG_N * WG_N * sizeof(float)) return fail(NATSL_ERR_WORKSPACE, "%s: workspace too small", what);
+  if (workspace_bytes < wgrad_bytes(p)) return fail(NATSL_ERR_WORKSPACE, "%s: workspace too small", what);
   p.part = reinterpret_cast<float*>(workspace);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   static std::atomic<unsigned long long> reserved{0};

@@ -56,11 +56,17 @@ def test_argument_validation_needs_no_gpu():
 
 
 def test_workspaces_stay_small():
-    """Partial sums are bounded by the chip and not by the tokens: a row of 2 H sums for each of 2048 workgroups of the gates' backward."""
+    """Partial sums are bounded by the chip and not by the tokens: a row of 2 H sums for each of 2048 workgroups of the gates' backward; for a
+    weight's gradient its own rows, in blocks of 32, for each of 128 slices."""
     L = _lib()
     for rows in (1, 4096, 32768, 1 << 20, 1 << 24):
         for H in (1, 6, 16, 33, 64, 256):
             assert 0 < L.natsl_gates_bwd_workspace_bytes(rows, H) <= 2048 * 2 * H * 4
+    from neuralattentionsearchlinear_amd._front import _WgradSeg
+    up = lambda n, to: -(-n // to) * to
+    for rows, ns, D in ((32768, (24,), 768), (1 << 20, (8, 40), 256), (16000, (32,), 2048), (6000, (36,), 1152), (40, (8,), 8), (32768, (768, 1536, 200), 1000)):
+        segs = (_WgradSeg * len(ns))(*[_WgradSeg(None, None, n, n) for n in ns])
+        assert 0 < L.natsl_wgrad_workspace_bytes(segs, len(ns), rows, D) <= 128 * sum(up(n, 32) for n in ns) * up(D, 256) * 4
 
 
 def test_no_cpu_fallback():

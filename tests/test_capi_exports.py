@@ -64,7 +64,7 @@ def test_workspaces_stay_small():
             assert 0 < L.natsl_gates_bwd_workspace_bytes(rows, H) <= 2048 * 2 * H * 4
     from neuralattentionsearchlinear_amd._front import _WgradSeg
     up = lambda n, to: -(-n // to) * to
-    for rows, ns, D in ((32768, (24,), 768), (1 << 20, (8, 40), 256), (16000, (32,), 2048), (6000, (36,), 1152), (40, (8,), 8), (32768, (768, 1536, 200), 1000)):
+    for rows, ns, D in ((32768, (24,), 768), (1 << 20, (8, 40), 256), (16000, (32,), 2048), (6000, (40,), 1152), (40, (8,), 8), (32768, (768, 1536, 200), 1000)):
         segs = (_WgradSeg * len(ns))(*[_WgradSeg(None, None, n, n) for n in ns])
         assert 0 < L.natsl_wgrad_workspace_bytes(segs, len(ns), rows, D) <= 128 * sum(up(n, 32) for n in ns) * up(D, 256) * 4
 

@@ -493,10 +493,8 @@ int natsl_project(const natsl_project_seg* segs, int n_seg, const void* x, int64
 int natsl_project_bwd(const natsl_project_seg* segs, int n_seg, const void* dpool, void* dx, int B, int T, int D, int block,
                       natsl_stream_t stream);
 
-/* Products with a narrow weight w [N, D] (N a multiple of 4 up to 64, D of 128, N D up to 81920), bf16 with fp32 sums:
- * y [rows, N] = x [rows, D] w^T, and dx [rows, D] = dy [rows, N] w.  Contiguous, on 16 bytes.  (The mixing logits' layer,
- * src/nats/layers/natsl_attn_gdn.py:425-491.) */
-int natsl_narrow_linear(const void* x, const void* w, void* y, int64_t rows, int D, int N, natsl_stream_t stream);
+/* dx [rows, D] = dy [rows, N] w for a narrow weight w [N, D] (N a multiple of 4 up to 48, D of 128), bf16 with fp32 sums.  Contiguous, on 16
+ * bytes.  (The mixing logits' layer, src/nats/layers/natsl_attn_gdn.py:425-491.) */
 int natsl_narrow_linear_bwd(const void* dy, const void* w, void* dx, int64_t rows, int D, int N, natsl_stream_t stream);
 
 /* natsl_gdn_chunk_fwd (is_delta) or natsl_mamba_chunk_fwd with NATSL_STATES_ONLY and no state of the last block.  beside: NULL, or

@@ -188,26 +188,18 @@ class _Project(torch.autograd.Function):
 
 
 # ---- a narrow weight: the mixing logits' layer ------------------------------------------------------------------------------------
-def _narrow_built(N, D, *tensors):
-    return N % 4 == 0 and N <= 64 and D % 128 == 0 and N * D <= 81920 and _on_16(*tensors)
-
-
-def _narrow(x, w):
-    """F.linear(x, w).  natsl_narrow_linear from 2^24 elements of x on (a layer's times, library / it, us: 24 x 768 over 32768 tokens
-    23 / 12, 32 x 2048 over 16000 29 / 21; 36 x 1152 over 6000 9.3 / 11.3)."""
-    N, D = w.shape
-    if x.numel() < 1 << 24 or not _narrow_built(N, D, x, w):
-        return F.linear(x, w)
-    y = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
-    _capi.check(_capi.lib().natsl_narrow_linear(x.data_ptr(), w.data_ptr(), y.data_ptr(), x.numel() // D, D, N, _capi.stream_ptr(x.device)),
-                "natsl_narrow_linear")
-    return y
+def _narrow_pays(rows, N, D):
+    """Whether natsl_narrow_linear_bwd beats the library's product.  Measured (library / it, us, tensors in the cache): 8 x 512 over 16000
+    10.3 / 7.2, 24 x 768 over 2048 6.5 / 6.8, 6000 12.5 / 7.7, 32768 26.1 / 14.2, 36 x 1152 over 2048 7.3 / 7.9, 6000 11.1 / 9.2, 40 x 1024 over
+    6000 9.9 / 9.4 (from memory 10.2 / 10.7), 48 x 768 over 65536 39 / 29.  The library's kernels for 32 and 64 rows are as good or better
+    (32 x 512 over 6000 5.5 / 7.5, 64 x 1024 over 32768 20 / 27), 52 to 60 rows lose below 2^24 elements."""
+    return N % 32 != 0 and N <= 48 and rows * D >= (4 << 20 if N < 32 else 6 << 20)
 
 
 def _narrow_bwd(dy, w):
-    """dy [rows, N] w (24 x 768 over 32768 tokens 36 -> 14 us, 36 x 1152 over 6000 16 -> 9)"""
+    """dy [rows, N] w"""
     N, D = w.shape
-    if not _narrow_built(N, D, dy, w):
+    if N % 4 or D % 128 or not _narrow_pays(dy.shape[0], N, D) or not _on_16(dy, w):
         return torch.mm(dy, w)
     dx = torch.empty(dy.shape[0], D, dtype=dy.dtype, device=dy.device)
     _capi.check(_capi.lib().natsl_narrow_linear_bwd(dy.data_ptr(), w.data_ptr(), dx.data_ptr(), dy.shape[0], D, N, _capi.stream_ptr(dy.device)),
@@ -260,7 +252,7 @@ class _ConvNorm(torch.autograd.Function):
         ctx.save_for_backward(q, k, v, ys[0], w_mix, wq, bq, wk, bk, wv, bv, nq, nk)
         ctx.set_materialize_grads(False)
         raw = tuple(t.view(t.shape) for t in (q, k, v)) if f.raw_attention else (None, None, ys[2].detach())
-        return (ys[0], ys[1], ys[2], ns[0], ns[1], _narrow(ys[0], w_mix)) + raw
+        return (ys[0], ys[1], ys[2], ns[0], ns[1], F.linear(ys[0], w_mix)) + raw
 
     @staticmethod
     def backward(ctx, dq, dk, dv, dqn, dkn, dlogits, dq_raw, dk_raw, dv_raw):
@@ -447,7 +439,7 @@ class FastFront:
         if self.grad(*args):
             return _ConvNorm.apply(self, *args) + (None,)
         ys, ns, new = _conv_norm(self, (q, k, v), states, want_states)
-        return ys[0], ys[1], ys[2], ns[0], ns[1], _narrow(ys[0], w["w_mix"]), *((q, k, v) if self.raw_attention else (None, None, ys[2])), new
+        return ys[0], ys[1], ys[2], ns[0], ns[1], F.linear(ys[0], w["w_mix"]), *((q, k, v) if self.raw_attention else (None, None, ys[2])), new
 
     def gates(self, ab):
         if self.grad(ab, self.w["a_log"], self.w["dt_bias"]):

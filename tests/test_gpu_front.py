@@ -275,21 +275,31 @@ def test_joint_projections(B, T, D, widths, block):
         assert bool((dx[rows] == 7).all())
 
 
-@pytest.mark.parametrize("rows,D,N", [(1, 128, 4), (33, 768, 24), (63, 1152, 36), (64, 2048, 32), (65, 1280, 64), (257, 384, 60), (4099, 256, 16)])
-def test_narrow_products(rows, D, N):
-    """natsl_narrow_linear and its backward at the edges of their tiles of tokens, columns and weight rows."""
-    from neuralattentionsearchlinear_amd import _capi
+@pytest.mark.parametrize("rows,D,N", [(1, 128, 4), (33, 768, 24), (63, 1152, 36), (64, 2048, 32), (65, 1280, 48), (257, 384, 44), (4099, 256, 16), (16387, 1152, 40)])
+def test_narrow_product_backward(rows, D, N):
+    """natsl_narrow_linear_bwd at the edges of its tiles of tokens, columns and weight rows; what it is chosen for, and the library's else."""
+    from neuralattentionsearchlinear_amd import _capi, _front
     torch.manual_seed(rows)
     L, P = _capi.lib(), _capi.ptr
-    x, w, dy = torch.randn(rows, D, device=DEV).bfloat16(), torch.randn(N, D, device=DEV).bfloat16(), torch.randn(rows, N, device=DEV).bfloat16()
-    y, dx = (torch.full((rows + 1, n), 7., device=DEV).bfloat16() for n in (N, D))
-    _capi.check(L.natsl_narrow_linear(P(x), P(w), P(y), rows, D, N, _capi.stream_ptr(x.device)), "natsl_narrow_linear")
-    _capi.check(L.natsl_narrow_linear_bwd(P(dy), P(w), P(dx), rows, D, N, _capi.stream_ptr(x.device)), "natsl_narrow_linear_bwd")
-    for a, ref in ((y, x.double() @ w.double().t()), (dx, dy.double() @ w.double())):
-        # exact products, fp32 sums, one rounding to bf16
-        assert bool(((a[:rows].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * D ** 0.5).all())
-        assert bool((a[rows] == 7).all())
-    assert L.natsl_narrow_linear(P(x), P(w), P(y), rows, D, N + 2, _capi.stream_ptr(x.device)) != 0
+    w, dy = torch.randn(N, D, device=DEV).bfloat16(), torch.randn(rows, N, device=DEV).bfloat16()
+    dx = torch.full((rows + 1, D), 7., device=DEV).bfloat16()
+    _capi.check(L.natsl_narrow_linear_bwd(P(dy), P(w), P(dx), rows, D, N, _capi.stream_ptr(w.device)), "natsl_narrow_linear_bwd")
+    ref = dy.double() @ w.double()
+    # exact products, fp32 sums, one rounding to bf16
+    bound = 2.0 ** -8 * ref.abs() + 1e-5 * D ** 0.5
+    assert bool(((dx[:rows].double() - ref).abs() <= bound).all()) and bool((dx[rows] == 7).all())
+    for refused in (N + 2, 52):
+        assert L.natsl_narrow_linear_bwd(P(dy), P(w), P(dx), rows, D, refused, _capi.stream_ptr(w.device)) != 0
+    got = _front._narrow_bwd(dy, w)
+    assert torch.equal(got, dx[:rows]) if _front._narrow_pays(rows, N, D) else bool(((got.double() - ref).abs() <= bound).all())
+
+
+def test_narrow_product_only_where_it_pays():
+    """The line between natsl_narrow_linear_bwd and the library: rows of the weight, and elements of what is written."""
+    from neuralattentionsearchlinear_amd._front import _narrow_pays
+    assert _narrow_pays(6000, 24, 768) and _narrow_pays(6000, 36, 1152) and _narrow_pays(65536, 48, 768) and _narrow_pays(32768, 8, 512)
+    assert not any(_narrow_pays(rows, N, D) for rows in (1, 777, 65536) for N in (32, 52, 60, 64) for D in (128, 1280, 2048))
+    assert not _narrow_pays(2048, 24, 768) and not _narrow_pays(2048, 36, 1152) and not _narrow_pays(0, 24, 768)
 
 
 @pytest.mark.parametrize("n_a,n_b", [(16, 0), (6, 6), (16, 16), (8, 40), (24, 24), (32, 0)])

@@ -92,11 +92,13 @@ def linear(x, w):
 @functools.lru_cache(maxsize=512)
 def _joint_pays(rows, D, widths, cus):
     """Whether one launch for all projections (natsl_project) beats the library's products one by one: where it takes fewer rounds of
-    256 x 256 tiles over the CUs.  Measured (one by one / joint, us): 340M geometry 8 x 4096 tokens, 10 / 9 rounds: 273-318 / 265-289;
-    760M 8 x 2048, 10 / 7: 352 / 303; 760M 1 x 4096, 4 / 2: 109 / 81; but Mamba 4 x 8192, 12 / 12: 325 / 366.  Short prompts
-    take one round either way and the library's four launches: 1 x 777 78 / 16."""
+    256 x 256 tiles over the CUs.  Measured (one by one / joint, us): 340M geometry 8 x 4096 tokens, 10 / 9 rounds: 267 / 260, 1 x 777,
+    4 / 1: 39 / 17; 760M 8 x 2048, 10 / 7: 337 / 288, 1 x 4096, 4 / 2: 99 / 79; but Mamba 4 x 8192, 12 / 12: 341 / 350, 760M 8 x 8192, 28 / 28:
+    1065 / 1187.  From inputs wider than 1536 on a round of the library's is the shorter one (2048 columns in, 9216 out, 16384 tokens, 10 / 9:
+    461 / 502, 4096 tokens, 4 / 3: 138 / 141, 12000, 10 / 7: 407 / 390): there at most seven tenths of its rounds."""
     tiles = [-(-rows // 256) * -(-n // 256) for n in widths]
-    return D % 32 == 0 and D >= 128 and all(n % 8 == 0 for n in widths) and -(-sum(tiles) // cus) < sum(-(-t // cus) for t in tiles)
+    joint, alone = -(-sum(tiles) // cus), sum(-(-t // cus) for t in tiles)
+    return D % 32 == 0 and D >= 128 and all(n % 8 == 0 for n in widths) and (joint < alone if D <= 1536 else 0 < 10 * joint <= 7 * alone)
 
 
 def _project_segs(ys, ws):
@@ -165,7 +167,9 @@ class _Project(torch.autograd.Function):
             joint = sum(w.shape[0] for _, w in some) >= 128 and all(w.shape[0] % 32 == 0 for _, w in some) and \
                 _on_16(dx, *([] if dp is None else [dp]), *[t for pair in some for t in pair])
         if need[0] and joint:
-            # one pass over dx where four accumulating products and dx_init made five (340M geometry, 8 x 4096 tokens: 412 -> 260 us)
+            # one pass over dx where four accumulating products and dx_init made five (340M geometry, 8 x 4096 tokens: 342 -> 237 us, 1 x 777
+            # 56 -> 49).  Below some 500 tokens the one launch takes longer than the five (760M, 128 tokens: 54 / 68), but a step is the host's
+            # there, which issues one for five: the layer at 760M, 300 tokens 1.45 -> 1.2 ms
             rc = _capi.lib().natsl_project_bwd(_project_segs(*zip(*some)), len(some), _p(dp), dx.data_ptr(), B, T, D, ctx.block or T,
                                                _capi.stream_ptr(x.device))
             _capi.check(rc, "natsl_project_bwd")

@@ -294,6 +294,16 @@ def test_narrow_product_backward(rows, D, N):
     assert torch.equal(got, dx[:rows]) if _front._narrow_pays(rows, N, D) else bool(((got.double() - ref).abs() <= bound).all())
 
 
+def test_joint_projections_only_where_they_pay():
+    """The line between natsl_project and the library: fewer rounds of tiles, and for wide inputs many fewer."""
+    from neuralattentionsearchlinear_amd._front import _joint_pays
+    pays = lambda rows, D, *widths: _joint_pays(rows, D, widths, 256)
+    assert pays(32768, 1024, 768, 768, 1536, 1536) and pays(16384, 1536, 1152, 1152, 2304, 2304) and pays(1, 1024, 768, 768, 1536, 1536)
+    assert not pays(32768, 1024, 2048, 2048, 1024, 1024) and not pays(0, 1024, 768, 768, 1536, 1536) and not pays(777, 1032, 768, 768, 1536, 1536)
+    wide = 2048, 1536, 1536, 3072, 3072
+    assert pays(3000, *wide) and pays(12000, *wide) and not any(pays(rows, *wide) for rows in (0, 4096, 16384, 24000, 49152))
+
+
 def test_narrow_product_only_where_it_pays():
     """The line between natsl_narrow_linear_bwd and the library: rows of the weight, and elements of what is written."""
     from neuralattentionsearchlinear_amd._front import _narrow_pays

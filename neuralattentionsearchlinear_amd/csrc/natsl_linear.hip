@@ -1104,8 +1104,10 @@ static int launch_linear(const LinearParams& p, hipStream_t stream, const Beside
   // With another kernel waiting for the CUs that the scan leaves, wider workgroups: 1, 1.1, 1.65 times the step on 1, 1/2, 1/4 of the
   // CUs.  The narrowest that leaves that kernel three quarters of the chip (one wave) or half of it (two): both branches at
   // B4 T8192 H8 one after the other (one wave, 256 workgroups) 400 us, side by side with two waves 326; Mamba B2 T8192 H32 480 -> 395.
-  // (A scan for the chunk states alone is a third shorter and keeps its own width.)
-  if (beside && p.o) nw = 4 * n_chains * (p.V / 16) <= cus ? 1 : ok2 && (!ok4 || 2 * n_chains * (p.V / 32) <= cus) ? 2 : ok4 ? 4 : nw;
+  // A scan for the chunk states alone is a third shorter and gains from it all the same, next to the softmax branch's backward (whole passes,
+  // its own width / this, us): operator B4 T8192 H8 1675 / 1645, B1 T8192 H24 1160 / 1147, 760M layer 1 x 12000 3740 / 3638, 340M 2 x 9000
+  // 2628 / 2597; twenty other shapes within 1 %.
+  if (beside) nw = 4 * n_chains * (p.V / 16) <= cus ? 1 : ok2 && (!ok4 || 2 * n_chains * (p.V / 32) <= cus) ? 2 : ok4 ? 4 : nw;
   // The delta rule's four-wave scan forms P itself and the prep reads k only, when the launch fills the machine: prep and scan
   // are then bound by their HBM traffic, which this cuts by a fifth (measured at B8 T8192 H16: 0.46 -> 0.43 ms), while a launch
   // that leaves CUs idle is bound by the scan's step and only gets slower from the extra work in it (B8 T4096 H6 V256:

@@ -106,3 +106,29 @@ print(json.dumps(out))
     beside, ordered = "launch 1001:1 record 1001 wait 1002 launch 1001:1", "launch 1001:1 launch 1001:1"
     got = json.loads(r.stdout)
     assert [g[1] for g in got] == [beside, beside, ordered, ""] and [g[0] == 0 for g in got] == [True] * 3 + [False] and {g[2] for g in got} == {0}
+
+
+@pytest.mark.parametrize("kind,B,H,K,V,alone,beside", [(1, 4, 8, 128, 128, 256, 128), (1, 1, 8, 192, 384, 192, 96), (0, 2, 32, 128, 64, 256, 128), (1, 1, 2, 128, 128, 64, 64)])
+def test_a_scan_next_to_other_work_leaves_it_compute_units(fake_hip, kind, B, H, K, V, alone, beside):
+    """Workgroups of the scan, by itself and with the other stream's work behind the kernel in front of it (256 compute units)."""
+    child = """
+import ctypes, json, sys
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+fake.fake_launches.restype = ctypes.c_char_p
+f = ctypes.CDLL(sys.argv[2]).natsl_linear_chunk_states
+kind, B, H, K, V = json.loads(sys.argv[3])
+p, n, i, out = ctypes.c_void_p(1 << 20), ctypes.c_void_p(None), ctypes.c_int, []
+for side in (0, 0x1002):
+    fake.fake_reset(1)
+    rc = f(i(kind), p, p, p, p, p, n, n, p, p, p, i(1), i(B), i(4096), i(H), i(H), i(K), i(V), i(64), i(64), ctypes.c_float(0.1), i(7), p,
+           ctypes.c_size_t(1 << 40), i(1), n, i(0), i(B * 64), ctypes.c_void_p(0x1001), ctypes.c_void_p(side))
+    scan = [line.split() for line in fake.fake_launches().decode().splitlines() if "linear_scan_kernel" in line]
+    out.append([rc, len(scan), int(scan[0][2])])
+print(json.dumps(out))
+"""
+    from neuralattentionsearchlinear_amd import _build, _capi
+    if not os.path.exists(_capi.LIB_PATH):
+        _build.build()
+    r = subprocess.run([sys.executable, "-c", child, fake_hip, _capi.LIB_PATH, json.dumps([kind, B, H, K, V])], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    assert json.loads(r.stdout) == [[0, 1, alone], [0, 1, beside]]

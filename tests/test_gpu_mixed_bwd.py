@@ -314,3 +314,46 @@ def test_backward_branches_side_by_side(kind, T, K, V, block, monkeypatch):
                 assert rel_l2(a, b) < 1e-2
             else:
                 assert torch.equal(a, b), i
+
+
+@pytest.mark.parametrize("kind,T,K,V,block,shared,packed,released", [
+    ('gdn', 700, 128, 128, 64, False, False, True), ('gdn', 700, 128, 128, 64, True, False, True), ('gdn', 611, 128, 64, 128, True, True, True),
+    ('mamba', 513, 64, 128, 128, False, False, True), ('mamba', 450, 128, 64, 64, True, False, True), ('gdn', 330, 192, 64, 64, False, False, True),
+    ('gdn', 200, 128, 48, 64, False, False, False)])
+def test_recomputed_chunk_states_side_by_side(kind, T, K, V, block, shared, packed, released, monkeypatch):
+    """Chunk states formed again next to the softmax branch's backward, whose stream waits for the kernel in front of their scan (for the
+    whole stream where the value width is filled up): the gradients of one stream, with work still in front of the backward's first launch."""
+    from neuralattentionsearchlinear_amd import _linear_bwd, _mixed_common as MC
+    B, H = 1 if packed else 2, 4
+    KA, VA = (K, V) if shared else (128 if K != 192 else 64, 128)
+    gen = torch.Generator().manual_seed(T)
+    bounds = [0, 1, 193, T] if packed else [0, T]
+    cu = torch.tensor(bounds, dtype=torch.int32, device=DEV) if packed else None
+    NB = sum(-(-(b - a) // block) for a, b in zip(bounds[:-1], bounds[1:]))
+    ql, kl, vl = make_qkv(B, T, H, K, V, 5)
+    qa, ka, va = make_qkv(B, T, H, KA, VA, 8)
+    g, beta = make_gates(B, T, H, 6)
+    ty = make_types(B, NB, 2, 0.4, 7, torch.bfloat16)
+    do_l, do_a = torch.randn(B, T, H, V, generator=gen).bfloat16().to(DEV), torch.randn(B, T, H, VA, generator=gen).bfloat16().to(DEV)
+    streams, inner = [], _linear_bwd.linear_chunk_backward
+    monkeypatch.setattr(_linear_bwd, 'linear_chunk_backward', lambda *a, **kw: (streams.append(kw['release']), inner(*a, **kw))[1])
+
+    def grads(side, keep):
+        monkeypatch.setattr(MC, 'CONCURRENT_BRANCHES', side)
+        monkeypatch.setattr(MC, 'SAVE_CHUNK_STATES', keep)
+        del streams[:]
+        lin = [t.to(DEV).requires_grad_(True) for t in (ql, kl, vl)]
+        attn = lin if shared else [t.to(DEV).requires_grad_(True) for t in (qa, ka, va)]
+        rest = [t.to(DEV).requires_grad_(True) for t in ((g, ty, beta) if kind == 'gdn' else (g, ty))]
+        o_l, o_a, _ = MC.mixed_forward(kind, *attn, *lin, None, rest[0], rest[2] if kind == 'gdn' else None, rest[1], 0.1, 0.1, cu, None, block, None, True,
+                                       True, True, True, True, False, kind == 'gdn')
+        torch.cuda._sleep(20_000_000)
+        torch.autograd.backward([o_l, o_a], [do_l, do_a])
+        assert [s is not None for s in streams if s is not None] == [True] * (side and not keep and released)
+        return [t.grad for t in (lin if shared else lin + attn) + rest[:1] + rest[2:]] + [rest[1].grad]
+    want = grads(False, True)
+    for side, keep in ((True, False), (False, False), (True, True), (True, False)):
+        got = grads(side, keep)
+        for i, (a, b) in enumerate(zip(got[:-1], want[:-1])):
+            assert torch.equal(a, b), (i, side, keep)
+        assert rel_l2(got[-1], want[-1]) < 1e-2              # (block types: one atomic addition per unit, in any order)

@@ -164,3 +164,32 @@ def test_boundaries_on_the_gpu_or_on_the_host(lens):
            for c in (cu, torch.tensor(cu, device=_dev()), torch.tensor(cu, dtype=torch.int32, device=_dev()))]
     for o in out[1:]:
         assert all(torch.equal(a, b) for a, b in zip(o, out[0]))
+
+
+@pytest.mark.parametrize("lens", [[1] * 70, [65, 1, 127, 300], [2500, 700, 3, 1900]])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_boundaries_on_the_gpu_on_one_stream_and_two(lens, dtype, monkeypatch):
+    """The same with the branches on one stream and side by side (the table is stored behind what the side stream waits for), with a state
+    to start from, and with fp32 tensors, whose copies are laid out before the table is there."""
+    from neuralattentionsearchlinear_amd import _mixed_common as MC
+    from neuralattentionsearchlinear_amd.mixed_attn_gdn import nats_mixed_attn_gdn
+    cu = [0]
+    for x in lens:
+        cu.append(cu[-1] + x)
+    gen = torch.Generator(device=_dev()).manual_seed(3)
+    rn = lambda *s: torch.randn(*s, device=_dev(), generator=gen)
+    T, NB = cu[-1], sum(-(-x // 64) for x in lens)
+    q, k, v, beta = rn(1, T, 2, 64).to(dtype), rn(1, T, 2, 64).to(dtype), rn(1, T, 2, 64).to(dtype), torch.sigmoid(rn(1, T, 2)).to(dtype)
+    g, h0 = -torch.nn.functional.softplus(rn(1, T, 2)), rn(len(lens), 2, 64, 64)
+    ty = torch.nn.functional.one_hot((rn(1, NB, 2) > 0).long(), 2).bfloat16()
+
+    def outputs(c, side):
+        monkeypatch.setattr(MC, 'CONCURRENT_BRANCHES', side)
+        return nats_mixed_attn_gdn(q, k, v, q, k, v, h0, g, beta, ty, None, cu_seqlens=c, nats_block_size=64, ops_for_incomplete_chunks="all",
+                                   output_final_state_gated_delta=True, decay_for_non_gdn_blocks=True)
+    want = outputs(cu, False)
+    for c, side in ((cu, True), (torch.tensor(cu, device=_dev()), False), (torch.tensor(cu, device=_dev()), True), (torch.tensor(cu, dtype=torch.int32, device=_dev()), True)):
+        assert all(torch.equal(a, b) for a, b in zip(outputs(c, side), want))
+    with pytest.raises(ValueError):
+        nats_mixed_attn_gdn(q, k, v, q, k, v, h0[1:], g, beta, ty, None, cu_seqlens=torch.tensor(cu, device=_dev()), nats_block_size=64,
+                            ops_for_incomplete_chunks="all", output_final_state_gated_delta=True, decay_for_non_gdn_blocks=True)

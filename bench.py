@@ -7,6 +7,7 @@ softmax kernel, MFMA-bound) from HIP events recorded on the stream it is launche
 host-CPU baseline (the fp32 oracle on a bounded sample of the same workload).
 """
 import argparse
+import gc
 import json
 import math
 import os
@@ -495,6 +496,10 @@ def main():
         # The GPU leaves idle at reduced clocks and needs about 40 ms of load to settle (the first 30 steps of a cold
         # run take up to 15 % longer per kernel): load it for --prewarm-ms with the same step before the W warm-up
         # steps, so that a short run measures the steady state it would also reach after more steps.
+        # The interpreter's full collections (15 - 45 ms with torch loaded) fall inside the timed steps or not by how many objects were
+        # made before them (every block linear, 200 steps: 0.207 or 0.34 ms a step): what there is by now is looked at once, here.
+        gc.collect()
+        gc.freeze()
         t_pre = time.perf_counter()
         n_pre = 0
         while (time.perf_counter() - t_pre) * 1e3 < args.prewarm_ms:

@@ -6,14 +6,15 @@
 // Why not a library product each: a projection of 768 or 1152 columns leaves part of its last round of tiles idle, four products of a
 // short prompt are four launches, and the gradients of one input accumulate, so that dX is read and written once per projection.  Here the
 // tiles of all projections (forward) or the contraction over all of them (backward) follow each other in one launch.  340M geometry, 8 x 4096
-// tokens: backward 412 us (four accumulating products and the block mean's pass) -> 260, 1.2 PFLOP/s; forward 273-318 -> 265-289.
+// tokens: backward 342 us (four accumulating products and the block mean's pass) -> 237, 1.3 PFLOP/s; forward 267 -> 260.
 //
 // A tile is 256 tokens (or 192, 128) x 256 columns, four waves with 128 x 128 of it each: 256 accumulator registers, a wave per SIMD; an
 // operand pair from LDS serves 16 matrix instructions.  Stages of 32 contraction elements come by LDS-DMA into a ring of four; the
 // operands of the next 16 elements are requested while the current ones multiply, and the one barrier of a stage sits in its middle, where
 // the next stage's operands are about to be read.  A workgroup walks its tiles with the requests running on into the next one, so a tile
 // has no prologue.  1 190 - 1 220 cycles a stage against 1 024 of matrix time, 6 500 for a tile's way out (its stores: held back and
-// spread over the next tile's stages they cost the same there).  What bounds it then is the power limit (1.25 - 1.7 GHz).
+// spread over the next tile's stages they cost the same there).  What bounds it then is the power limit: 1.75 - 1.9 GHz in a training step,
+// where the passes around it run at 2.4, 1.25 - 1.7 back to back.
 #include <type_traits>
 
 #include "natsl_device.h"

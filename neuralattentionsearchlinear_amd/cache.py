@@ -249,14 +249,15 @@ class NAtSLayerCache:
             n_in = 0
         pairs = [(self.l_attn_k, k), (self.l_attn_v, v), (self.lattn_beta, lattn_beta), (self.lattn_g, lattn_g)]
         total = n_in + T
+        out = (k, v, lattn_beta, lattn_g)
+        # (the recurrent operator of the 'attn' mode takes the whole block's tokens once they complete it)
+        if not fresh and n_in and (mode == 'chunk' or (ops_for_incomplete_chunks == 'attn' and total >= bs)):
+            out = tuple(None if new is None else torch.cat([buf[:, :n_in], new], dim=1) for buf, new in pairs)
         if total < bs:
             for buf, new in pairs:
                 if new is not None:
                     buf[:, n_in:total] = new
-            return k, v, lattn_beta, lattn_g
-        out = (k, v, lattn_beta, lattn_g)
-        if not fresh and n_in and (mode == 'chunk' or ops_for_incomplete_chunks == 'attn'):
-            out = tuple(None if new is None else torch.cat([buf[:, :n_in], new], dim=1) for buf, new in pairs)
+            return out
         rest = total % bs
         if rest:
             for buf, new in pairs:

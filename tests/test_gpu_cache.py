@@ -249,6 +249,33 @@ def test_long_continuation_on_a_filled_cache(kind, ops, T0, T1):
         assert rel_l2(a2.float(), b2.float()) <= 1e-2, f"the next token: rel-L2 {rel_l2(a2.float(), b2.float()):.3e}"
 
 
+@pytest.mark.parametrize("kind,ops,block,pieces", [('gdn', 'all', 128, (12, 64, 1, 130)), ('gdn', 'all', 256, (270, 100, 64, 3, 90)), ('mamba', 'all', 256, (100, 90, 64, 80)),
+                                                   ('gdn', 'gated_delta_net', 256, (300, 64, 70, 90)), ('mamba', 'mamba', 128, (128, 64, 64, 64)),
+                                                   ('gdn', 'attn', 256, (140, 64, 100))])
+def test_long_continuation_inside_a_block(kind, ops, block, pieces):
+    """64 or more new tokens that do not complete the incomplete block (a block of 128 tokens or more): outputs close to the forward over all tokens
+    so far, whose last block is the same incomplete one."""
+    from neuralattentionsearchlinear_amd.cache import NAtSCache, NAtSMamba2Cache
+    layer, cfg, _, _ = _layer_case(kind, None, ops)
+    layer.layer_idx, layer.nats_block_size = 0, block
+    layer = layer.to(DEV).to(torch.bfloat16).eval()
+    torch.manual_seed(block)
+    x = torch.randn(2, sum(pieces), cfg['hidden_size']).to(DEV).bfloat16()
+    first = lambda out: out[0] if isinstance(out, tuple) else out
+    holder = NAtSCache() if kind == 'gdn' else NAtSMamba2Cache()
+    kw = dict(past_key_values=holder, use_cache=True) if kind == 'gdn' else dict(cache_params=holder, use_cache=True)
+    t = 0
+    with torch.no_grad():
+        for n in pieces:
+            got = first(layer(x[:, t:t + n], **kw))
+            t += n
+            if n >= 64:
+                want = first(layer(x[:, :t]))[:, t - n:]
+                assert rel_l2(got.float(), want.float()) <= 2e-2, f"tokens {t - n}..{t}: rel-L2 {rel_l2(got.float(), want.float()):.3e}"
+    cache = holder[0] if kind == 'gdn' else holder.nats_cache[0]
+    assert cache.n_observed_tokens == t and cache._n_tokens_in_nats_block == t % block
+
+
 @pytest.mark.parametrize("T,block,K,V,dtype", [(64, 64, 64, 128, torch.bfloat16), (300, 64, 128, 64, torch.bfloat16), (513, 128, 64, 64, torch.float32)])
 def test_a_cache_made_in_new_memory(T, block, K, V, dtype):
     """natsl_kv_collect into memory that holds NaN = natsl_kv_compact into zeroed memory, every byte."""

@@ -82,3 +82,22 @@ def test_next_query_mask():
             c = int(st['n_attn_blocks'][b, hn])
             assert int(m[b, hn, 0].sum()) == c * bs + 10
             assert bool(m[b, hn, 0, :c * bs].all()) and bool(m[b, hn, 0, st['n_max'] * bs:].all())
+
+
+@pytest.mark.parametrize("bs,pieces", [(128, (10, 64, 50)), (256, (70, 90, 64, 65)), (64, (30, 64)), (128, (128, 64, 64)), (256, (7, 64, 249, 300))])
+def test_a_chunked_forward_gets_the_block_from_its_first_token(bs, pieces):
+    """What NAtSLayerCache.update_lattn_cache hands a chunked forward: the incomplete block's cached tokens and the new ones, also where these
+    stay inside the block (a block of 128 tokens or more): the layers put as many zero queries in front."""
+    from neuralattentionsearchlinear_amd.cache import NAtSLayerCache
+    torch.manual_seed(bs)
+    rows = [torch.randn(2, sum(pieces), 3, 4), torch.randn(2, sum(pieces), 3, 5), torch.randn(2, sum(pieces), 3), torch.randn(2, sum(pieces), 3)]
+    cache, t = NAtSLayerCache(nats_block_size=bs, op_for_incomplete_chunk='all'), 0
+    for n in pieces:
+        new = [x[:, t:t + n].contiguous() for x in rows]
+        got = cache.update_lattn_cache((new[0], new[1]), new[2], new[3], 'chunk', 'all')
+        for x, y in zip(got, rows):
+            assert torch.equal(x, y[:, t - t % bs:t + n])
+        t += n
+        cache._n_tokens_in_nats_block = t % bs
+        for buf, y in zip((cache.l_attn_k, cache.l_attn_v, cache.lattn_beta, cache.lattn_g), rows):
+            assert torch.equal(buf[:, :t % bs], y[:, t - t % bs:t])

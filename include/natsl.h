@@ -451,6 +451,20 @@ size_t natsl_conv_norm_bwd_workspace_bytes(const natsl_conv_seg* seg, int n_seg,
 int natsl_conv_norm_bwd(const natsl_conv_seg* seg, int n_seg, int B, int T, int W, int activation, int norm_dtype, void* workspace,
                         size_t workspace_bytes, natsl_stream_t stream);
 
+/* The narrow products of one input in one pass over it (bf16): ab [B T, ld] = x [wa; wb]^T (columns behind NA + NB are zero), and, where asked
+ * for: wn -> the means of x over blocks of 64 tokens (pooled [B, cdiv(T,64), D]; may be NULL) and logits [B, cdiv(T,64), NL] = means wn^T; g -> the
+ * gates of natsl_gates_fwd from ab's rounded values (NA heads; ab itself may then be NULL); wab [wab_rows, D] = [wa; wb; zeros].  D a multiple of 32,
+ * NA + NB <= 64 (32 with logits), NL <= 64.  src/nats/layers/natsl_attn_gdn.py:411-420, 507-512, src/nats/layers/natsl_attn_mamba2.py:391-393. */
+typedef struct natsl_front {
+  const void *x, *wa, *wb, *wn, *a_log, *dt_bias;
+  void *ab, *pooled, *logits, *beta, *wab;
+  float *g, *dt;
+  int32_t B, T, D, NA, NB, NL, ld, neg_eigval, param_dtype, wab_rows;
+} natsl_front;
+int natsl_layer_front(const natsl_front* a, natsl_stream_t stream);
+/* dw [N, D] = dy [rows, N]^T x [rows, D] (bf16, N up to 64, D even) for a narrow weight over few rows: the selector's over the block means. */
+int natsl_narrow_wgrad(const void* dy, const void* x, void* dw, int64_t rows, int D, int N, natsl_stream_t stream);
+
 /* The layers' gates from one projection ab [rows, ld] (bf16; a in columns 0..H-1, b in H..2H-1 for the delta rule):
  * g = -exp(a_log) softplus(a + dt_bias) fp32 [rows, H], beta = sigmoid(b) bf16 (doubled with neg_eigval; NULL for Mamba),
  * dt = softplus(a + dt_bias) fp32 (or NULL); and the gradients (dab has zeros behind the used columns).

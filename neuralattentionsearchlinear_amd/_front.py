@@ -31,6 +31,12 @@ class _ProjectSeg(ctypes.Structure):
     _fields_ = [("y", ctypes.c_void_p), ("w", ctypes.c_void_p), ("n", ctypes.c_int32), ("ld", ctypes.c_int32)]
 
 
+class _FrontArgs(ctypes.Structure):
+    """natsl_front of include/natsl.h."""
+    _fields_ = ([(n, ctypes.c_void_p) for n in ("x", "wa", "wb", "wn", "a_log", "dt_bias", "ab", "pooled", "logits", "beta", "wab", "g", "dt")] +
+                [(n, ctypes.c_int32) for n in ("B", "T", "D", "NA", "NB", "NL", "ld", "neg_eigval", "param_dtype", "wab_rows")])
+
+
 class _ConvSeg(ctypes.Structure):
     _fields_ = ([(n, ctypes.c_void_p) for n in ("x", "weight", "bias", "state", "norm_weight", "y", "y_norm", "state_out", "dy_a", "dy_b", "dy_norm",
                                                 "dx_add", "dx", "dweight", "dbias", "dnorm_weight")] +
@@ -124,6 +130,38 @@ def _wide(x, ws):
     return ys
 
 
+def _narrow(f, x, want_selector, keep):
+    """The narrow products of one input, the gates behind them and the selector's logits over the means of 64 tokens, one pass over x:
+    -> (g fp32, beta bf16 or None, dt fp32 or None [B,T,H], logits [B,TN,NL] or None, what the backward needs if `keep`: (a and b of every token,
+    their joint weight in whole stages of 32 rows, the block means or None)).  As separate products and passes it is four launches, two of them the
+    library's (340M geometry, 8 x 4096 tokens: 36 -> 24 us; 1 x 777 25 -> 9)."""
+    B, T, D = x.shape
+    w, H, dev = f.w, f.H, x.device
+    wb = w["wb"] if f.delta else None
+    a = _FrontArgs()
+    a.B, a.T, a.D, a.NA, a.NB, a.neg_eigval, a.param_dtype = B, T, D, H, H if f.delta else 0, f.neg, f.gate_dtype
+    g = torch.empty(B, T, H, dtype=torch.float32, device=dev)
+    beta = torch.empty(B, T, H, dtype=torch.bfloat16, device=dev) if f.delta else None
+    dt = None if f.delta else torch.empty_like(g)
+    logits = pooled = saved = None
+    if want_selector:
+        nb = -(-T // 64)
+        logits = torch.empty(B, nb, f.wn.shape[0], dtype=torch.bfloat16, device=dev)
+        a.wn, a.logits, a.NL = f.wn.data_ptr(), logits.data_ptr(), f.wn.shape[0]
+        if keep:
+            pooled = torch.empty(B, nb, D, dtype=torch.bfloat16, device=dev)
+            a.pooled = pooled.data_ptr()
+    if keep:
+        a.ld = a.wab_rows = _ab_rows(a.NA + a.NB)
+        ab, wab = torch.empty(B, T, a.ld, dtype=torch.bfloat16, device=dev), torch.empty(a.ld, D, dtype=torch.bfloat16, device=dev)
+        a.ab, a.wab = ab.data_ptr(), wab.data_ptr()
+        saved = ab, wab, pooled
+    a.x, a.wa, a.wb, a.a_log, a.dt_bias = x.data_ptr(), w["wa"].data_ptr(), _p(wb), w["a_log"].data_ptr(), w["dt_bias"].data_ptr()
+    a.g, a.beta, a.dt = g.data_ptr(), _p(beta), _p(dt)
+    _capi.check(_capi.lib().natsl_layer_front(ctypes.byref(a), _capi.stream_ptr(dev)), "natsl_layer_front")
+    return g, beta, dt, logits, saved
+
+
 def _project(x, wq, wk, wv, wg, wa, wb, pool_block, whole=16):
     """-> ((q, k, v, gate, ab, block means or None), the joint weight of a and b).  The narrow projections share one product: their
     rows and, where these are no multiple of `whole`, enough others to make whole stages of 32 (the columns behind a and b are never read)."""
@@ -137,9 +175,48 @@ def _project(x, wq, wk, wv, wg, wa, wb, pool_block, whole=16):
     return (*_wide(x, (wq, wk, wv, wg)), F.linear(x, wab), pooled), wab
 
 
+def _project_bwd(x, wide, wab, n_a, n_b, dys, dpool, block, needs):
+    """dx and the weights' gradients (wq, wk, wv, wg, wa, wb) of the projections of one input: dx is one launch (natsl_project_bwd), or starts as what
+    is no wide product (natsl_dx_init) and the wide ones accumulate onto it; all weight gradients are one launch.  dys: gradients of the four wide
+    outputs and of the joint narrow one, dpool: of the block means; each may be None.  needs: x, then the six weights."""
+    B, T, D = x.shape
+    rows = B * T
+    wq, wk, wv, wg = wide
+    dys = [None if t is None else t.reshape(rows, t.shape[-1]).contiguous() for t in dys]
+    dx = None
+    if needs[0]:
+        dx = torch.empty_like(x)
+        dp = None if dpool is None else dpool.contiguous()
+        some = [(dy, w) for dy, w in zip(dys, (wq, wk, wv, wg, wab)) if dy is not None]
+        joint = sum(w.shape[0] for _, w in some) >= 128 and all(w.shape[0] % 32 == 0 for _, w in some) and \
+            _on_16(dx, *([] if dp is None else [dp]), *[t for pair in some for t in pair])
+    if needs[0] and joint:
+        # one pass over dx where four accumulating products and dx_init made five (340M geometry, 8 x 4096 tokens: 342 -> 237 us, 1 x 777
+        # 56 -> 49).  Below some 500 tokens the one launch takes longer than the five (760M, 128 tokens: 54 / 68), but a step is the host's
+        # there, which issues one for five: the layer at 760M, 300 tokens 1.45 -> 1.2 ms
+        rc = _capi.lib().natsl_project_bwd(_project_segs(*zip(*some)), len(some), _p(dp), dx.data_ptr(), B, T, D, block or T,
+                                           _capi.stream_ptr(x.device))
+        _capi.check(rc, "natsl_project_bwd")
+    elif needs[0]:
+        n = 0 if dys[4] is None else wab.shape[0]
+        rc = _capi.lib().natsl_dx_init(_p(dys[4]), wab.data_ptr(), _p(dp), dx.data_ptr(), B, T, D, n, max(n, 16), block or T,
+                                       _capi.stream_ptr(x.device))
+        _capi.check(rc, "natsl_dx_init")
+        dx2 = dx.view(rows, D)
+        for dy, w in zip(dys, wide):
+            if dy is not None:
+                dx2.addmm_(dy, w)
+    wants = [needs[1], needs[2], needs[3], needs[4], needs[5] or needs[6]]
+    dws = weight_grads(x.view(rows, D), [dy if want else None for dy, want in zip(dys, wants)])
+    da = db = None
+    if dws[4] is not None:
+        da = dws[4][:n_a]
+        db = dws[4][n_a:n_a + n_b] if n_b else None
+    return dx, dws[0], dws[1], dws[2], dws[3], da, db
+
+
 class _Project(torch.autograd.Function):
-    """dx is one launch (natsl_project_bwd), or starts as what is no wide product (natsl_dx_init) and the wide ones accumulate onto it;
-    all weight gradients are one launch."""
+    """The projections with the block means (selector blocks of other than 64 tokens, and widths that natsl_layer_front does not take)."""
 
     @staticmethod
     def forward(ctx, x, wq, wk, wv, wg, wa, wb, pool_block):
@@ -154,41 +231,35 @@ class _Project(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dq, dk, dv, dg, dab, dpool):
         x, wq, wk, wv, wg, wab = ctx.saved_tensors
-        B, T, D = x.shape
-        rows = B * T
-        flat = lambda t: None if t is None else t.reshape(rows, t.shape[-1]).contiguous()
-        dys = [flat(t) for t in (dq, dk, dv, dg, dab)]
-        need = ctx.needs_input_grad
-        dx = None
-        if need[0]:
-            dx = torch.empty_like(x)
-            dp = None if dpool is None else dpool.contiguous()
-            some = [(dy, w) for dy, w in zip(dys, (wq, wk, wv, wg, wab)) if dy is not None]
-            joint = sum(w.shape[0] for _, w in some) >= 128 and all(w.shape[0] % 32 == 0 for _, w in some) and \
-                _on_16(dx, *([] if dp is None else [dp]), *[t for pair in some for t in pair])
-        if need[0] and joint:
-            # one pass over dx where four accumulating products and dx_init made five (340M geometry, 8 x 4096 tokens: 342 -> 237 us, 1 x 777
-            # 56 -> 49).  Below some 500 tokens the one launch takes longer than the five (760M, 128 tokens: 54 / 68), but a step is the host's
-            # there, which issues one for five: the layer at 760M, 300 tokens 1.45 -> 1.2 ms
-            rc = _capi.lib().natsl_project_bwd(_project_segs(*zip(*some)), len(some), _p(dp), dx.data_ptr(), B, T, D, ctx.block or T,
-                                               _capi.stream_ptr(x.device))
-            _capi.check(rc, "natsl_project_bwd")
-        elif need[0]:
-            n = 0 if dys[4] is None else wab.shape[0]
-            rc = _capi.lib().natsl_dx_init(_p(dys[4]), wab.data_ptr(), _p(dp), dx.data_ptr(), B, T, D, n, max(n, 16), ctx.block or T,
-                                           _capi.stream_ptr(x.device))
-            _capi.check(rc, "natsl_dx_init")
-            dx2 = dx.view(rows, D)
-            for dy, w in zip(dys, (wq, wk, wv, wg)):
-                if dy is not None:
-                    dx2.addmm_(dy, w)
-        wants = [need[1], need[2], need[3], need[4], need[5] or need[6]]
-        dws = weight_grads(x.view(rows, D), [dy if want else None for dy, want in zip(dys, wants)])
-        da = db = None
-        if dws[4] is not None:
-            da = dws[4][:ctx.n_a]
-            db = dws[4][ctx.n_a:ctx.n_a + ctx.n_b] if ctx.n_b else None
-        return dx, dws[0], dws[1], dws[2], dws[3], da, db, None
+        return (*_project_bwd(x, (wq, wk, wv, wg), wab, ctx.n_a, ctx.n_b, (dq, dk, dv, dg, dab), dpool, ctx.block, ctx.needs_input_grad), None)
+
+
+class _ProjectAll(torch.autograd.Function):
+    """The projections, the gates behind the narrow ones and the selector's logits (f.wn: the selector's weight, or None without them)."""
+
+    @staticmethod
+    def forward(ctx, f, x, wq, wk, wv, wg, wa, wb, wn, a_log, dt_bias):
+        g, beta, dt, logits, (ab, wab, pooled) = _narrow(f, x, wn is not None, True)
+        ctx.f = f
+        ctx.save_for_backward(x, wq, wk, wv, wg, wab, ab, pooled, wn, a_log, dt_bias)
+        ctx.set_materialize_grads(False)
+        return (*_wide(x, (wq, wk, wv, wg)), g, beta, dt, logits)
+
+    @staticmethod
+    def backward(ctx, dq, dk, dv, dgate, dg, dbeta, ddt, dlogits):
+        f, need = ctx.f, ctx.needs_input_grad
+        x, wq, wk, wv, wg, wab, ab, pooled, wn, a_log, dt_bias = ctx.saved_tensors
+        dab = da_log = ddt_bias = dpool = dwn = None
+        if dg is not None or dbeta is not None or ddt is not None:
+            dab, da_log, ddt_bias = _gates_bwd(f, ab, dg, dbeta, ddt)
+        if dlogits is not None:
+            dl = dlogits.reshape(-1, wn.shape[0]).contiguous()
+            if need[1]:
+                dpool = _narrow_bwd(dl, wn, few=True).view(pooled.shape)
+            if need[8]:
+                dwn = _narrow_wgrad(dl, pooled.view(-1, pooled.shape[-1]))
+        dx, *dws = _project_bwd(x, (wq, wk, wv, wg), wab, f.H, f.H if f.delta else 0, (dq, dk, dv, dgate, dab), dpool, 64, need[1:8])
+        return (None, dx, *dws, dwn, da_log, ddt_bias)
 
 
 # ---- a narrow weight: the mixing logits' layer ------------------------------------------------------------------------------------
@@ -200,15 +271,28 @@ def _narrow_pays(rows, N, D):
     return N % 32 != 0 and N <= 48 and rows * D >= (4 << 20 if N < 32 else 6 << 20)
 
 
-def _narrow_bwd(dy, w):
-    """dy [rows, N] w"""
+def _narrow_bwd(dy, w, few=False):
+    """dy [rows, N] w.  few: the selector's, over the block means: a library product of this size is 4 to 8 us against 3 to 7, and 40 us of the host's
+    time against 5."""
     N, D = w.shape
-    if N % 4 or D % 128 or not _narrow_pays(dy.shape[0], N, D) or not _on_16(dy, w):
+    if N % 4 or N > 48 or D % 128 or not (few or _narrow_pays(dy.shape[0], N, D)) or not _on_16(dy, w):
         return torch.mm(dy, w)
     dx = torch.empty(dy.shape[0], D, dtype=dy.dtype, device=dy.device)
     _capi.check(_capi.lib().natsl_narrow_linear_bwd(dy.data_ptr(), w.data_ptr(), dx.data_ptr(), dy.shape[0], D, N, _capi.stream_ptr(dy.device)),
                 "natsl_narrow_linear_bwd")
     return dx
+
+
+def _narrow_wgrad(dy, x):
+    """dy [rows, N]^T x [rows, D]: natsl_narrow_wgrad up to some thousand rows (library / it, us: 12 x 1536 over 94 6.7 / 2.4, 512 8.1 / 3.2, 2048
+    7.0 / 6.7, 4096 9.7 / 11.2; 32 x 1024 over 512 7.4 / 5.1, 2048 8.6 / 13.9)."""
+    rows, N = dy.shape
+    D = x.shape[1]
+    if N > 64 or D % 2 or rows > (2048 if N <= 16 else 1024):
+        return torch.mm(dy.t(), x)
+    dw = torch.empty(N, D, dtype=dy.dtype, device=dy.device)
+    _capi.check(_capi.lib().natsl_narrow_wgrad(dy.data_ptr(), x.data_ptr(), dw.data_ptr(), rows, D, N, _capi.stream_ptr(dy.device)), "natsl_narrow_wgrad")
+    return dw
 
 
 # ---- convolutions, norms, mixing logits --------------------------------------------------------------------------------------------
@@ -313,6 +397,23 @@ def _gates(f, ab):
     return g, beta, dt
 
 
+def _gates_bwd(f, ab, dg, dbeta, ddt):
+    """-> gradients of ab, A_log, dt_bias; each of the three may be None."""
+    B, T, ld = ab.shape
+    c = lambda t, dt: None if t is None else t.to(dt).contiguous()
+    dg, dbeta, ddt = c(dg, torch.float32), c(dbeta, torch.bfloat16), c(ddt, torch.float32)
+    dab = torch.empty_like(ab)
+    da_log, ddt_bias = torch.empty_like(f.w["a_log"]), torch.empty_like(f.w["dt_bias"])
+    L = _capi.lib()
+    n = L.natsl_gates_bwd_workspace_bytes(B * T, f.H)
+    ws = torch.empty(n, dtype=torch.uint8, device=ab.device)
+    rc = L.natsl_gates_bwd(ab.data_ptr(), f.w["a_log"].data_ptr(), f.w["dt_bias"].data_ptr(), _p(dg), _p(dbeta), _p(ddt), int(f.delta), dab.data_ptr(),
+                           da_log.data_ptr(), ddt_bias.data_ptr(), ws.data_ptr(), n, B * T, f.H, ld, f.neg, f.gate_dtype,
+                           _capi.stream_ptr(ab.device))
+    _capi.check(rc, "natsl_gates_bwd")
+    return dab, da_log, ddt_bias
+
+
 class _Gates(torch.autograd.Function):
     @staticmethod
     def forward(ctx, f, ab, a_log, dt_bias):
@@ -323,20 +424,7 @@ class _Gates(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dg, dbeta, ddt):
-        f, ab = ctx.f, ctx.saved_tensors[0]
-        B, T, ld = ab.shape
-        c = lambda t, dt: None if t is None else t.to(dt).contiguous()
-        dg, dbeta, ddt = c(dg, torch.float32), c(dbeta, torch.bfloat16), c(ddt, torch.float32)
-        dab = torch.empty_like(ab)
-        da_log, ddt_bias = torch.empty_like(f.w["a_log"]), torch.empty_like(f.w["dt_bias"])
-        L = _capi.lib()
-        n = L.natsl_gates_bwd_workspace_bytes(B * T, f.H)
-        ws = torch.empty(n, dtype=torch.uint8, device=ab.device)
-        rc = L.natsl_gates_bwd(ab.data_ptr(), f.w["a_log"].data_ptr(), f.w["dt_bias"].data_ptr(), _p(dg), _p(dbeta), _p(ddt), int(f.delta), dab.data_ptr(),
-                               da_log.data_ptr(), ddt_bias.data_ptr(), ws.data_ptr(), n, B * T, f.H, ld, f.neg, f.gate_dtype,
-                               _capi.stream_ptr(ab.device))
-        _capi.check(rc, "natsl_gates_bwd")
-        return None, dab, da_log, ddt_bias
+        return (None, *_gates_bwd(ctx.f, ctx.saved_tensors[0], dg, dbeta, ddt))
 
 
 # ---- output norm-gate with the mixing logits -------------------------------------------------------------------------------------------
@@ -420,19 +508,30 @@ class _Select(torch.autograd.Function):
 class FastFront:
     """A layer's parameters at one forward, with the constants of its plan.  (The plan, which outlives the forward, holds no tensor.)"""
 
-    def __init__(self, constants, w):
+    def __init__(self, constants, w, wn):
         self.__dict__.update(constants)
-        self.w = w
+        self.w, self.wn = w, wn
 
     def grad(self, *tensors):
         return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
 
-    def project(self, x, pool_block):
+    def project(self, x, pool_block, selector):
+        """-> (q, k, v, gate, (g, beta, dt), selector logits or None without pool_block); selector: the layer's own product behind the means."""
         w = self.w
-        args = (x, w["wq"], w["wk"], w["wv"], w["wg"], w["wa"], w["wb"] if self.delta else None, pool_block)
-        if self.grad(*args[:7]):
-            return _Project.apply(*args)
-        return _project(*args)[0]
+        wb = w["wb"] if self.delta else None
+        narrow = (1 + self.delta) * self.H
+        if x.shape[-1] % 32 == 0 and narrow <= (32 if pool_block else 64) and (not pool_block or pool_block == 64 and self.wn is not None) and \
+                _on_16(x, w["wa"], *([] if wb is None else [wb]), *([self.wn] if pool_block else [])):
+            wide, wn = (w["wq"], w["wk"], w["wv"], w["wg"]), self.wn if pool_block else None
+            if self.grad(x, *wide, w["wa"], wb, wn, w["a_log"], w["dt_bias"]):
+                q, k, v, gate, g, beta, dt, logits = _ProjectAll.apply(self, x, *wide, w["wa"], wb, wn, w["a_log"], w["dt_bias"])
+            else:
+                g, beta, dt, logits, _ = _narrow(self, x, wn is not None, False)
+                q, k, v, gate = _wide(x, wide)
+            return q, k, v, gate, (g, beta, dt), logits
+        args = (x, w["wq"], w["wk"], w["wv"], w["wg"], w["wa"], wb, pool_block)
+        q, k, v, gate, ab, pooled = _Project.apply(*args) if self.grad(*args[:7]) else _project(*args)[0]
+        return q, k, v, gate, self.gates(ab), selector(pooled) if pool_block else None
 
     def conv_norm(self, q, k, v, states, want_states):
         """-> (conv(q), conv(k) or None, conv(v), normed q, normed k, mixing logits, raw q, k, v
@@ -495,6 +594,18 @@ def _front_plan(layer, kind, w):
                 gate_dtype=code("a_log"), out_dtype=code("out_norm1"), neg=int(delta and layer.allow_neg_eigval), out_eps=layer.o_norm.eps)
 
 
+def _selector_weight(layer, like):
+    """The weight of the selector's product where it is a plain one over few rows, else None (the layer's own product runs)."""
+    m = layer._modules.get("nats_layer")
+    if type(m) is not torch.nn.Linear or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__:
+        return None
+    w = m._parameters.get("weight")
+    if m._parameters.get("bias") is not None or type(w) is not torch.nn.Parameter or w.dtype != torch.bfloat16 or not w.is_contiguous() or \
+            w.device != like.device or w.dim() != 2 or w.shape[1] != like.shape[1] or w.shape[0] != layer.num_nats_head * layer.n_ops or w.shape[0] > 64:
+        return None
+    return w
+
+
 def fast_front(layer, kind, x, cache, cu_seqlens):
     """The layer's FastFront for this forward, or None where the general path has to run."""
     if not x.is_cuda or x.dtype != torch.bfloat16 or cu_seqlens is not None or not x.is_contiguous() or x.numel() == 0 or \
@@ -509,7 +620,7 @@ def fast_front(layer, kind, x, cache, cu_seqlens):
     constants = seen.front_plan[0]
     if constants is None or w["wq"].device != x.device:
         return None
-    f = FastFront(constants, w)
+    f = FastFront(constants, w, _selector_weight(layer, w["wa"]))
     if cache is not None:
         if torch.is_grad_enabled() and (x.requires_grad or any(t is not None and t.requires_grad for t in w.values())):
             return None

@@ -1,12 +1,202 @@
-// The gradient behind a narrow weight (the mixing logits' layer: a few dozen rows), bound by the wide tensor's bytes:
-//   X'[t][d] = sum_n Y'[t][n] W[n][d]   writes X' once
+// The layers' narrow products (weights of a few dozen rows), bound by the wide tensor's bytes:
+//   forward   Y[t][n] = sum_d X[t][d] W[n][d], in the same pass over X the means of its 64-token blocks, their selector logits and the
+//             gates behind Y
+//   backward  X'[t][d] = sum_n Y'[t][n] W[n][d]   writes X' once
 // bf16 operands, fp32 sums, one rounding.  Where the contraction is no multiple of 32 a library product takes two to three times as long as for
 // one that is (36 rows of 1152 over 32768 tokens 36 us, 32 rows of 1024 19).
+#include <type_traits>
+
 #include "natsl_device.h"
 #include "natsl_host.h"
 
 namespace natsl {
 
+// ---- forward -------------------------------------------------------------------------------------------------------------------------
+// A workgroup takes 64 tokens (a selector block); its waves share the contraction, 64 columns at a time in turn, and add up through LDS in
+// a fixed order.  A lane's operands are 16-byte pieces of rows as they lie in memory, requested a step ahead: nothing is staged.  The block's
+// mean is formed from the same registers (four rows a lane, then across the 16 lanes of a row group) and is the operand of the logits.
+// Against four launches (block means, two library products, gates), us: 32768 tokens of 1024, 12 rows and 12 logits 36 -> 24 (13 at the rate of a
+// copy: a workgroup has its 64 columns' share requested at once and little to overlap it with; two workgroups a CU spill, 28 - 40), 16 rows and 32
+// logits 39 -> 27; 6000 of 1536 26 -> 13; 777 of 1024 25 -> 9.
+struct FrontParams {
+  natsl_front f;
+  int nb;
+};
+
+template <int NT, int NL>
+struct FrontLds {
+  static constexpr int TILES = 4 * NT + NL, NW = 8, RED = NW * TILES * 1024, TOTAL = RED + 64 * 16 * NT * 2;
+};
+
+// the sum over the 16 lanes that share lane / 16, in all of them
+NATSL_DEVICE float row_sum16(float x) {
+  auto ror = [](const float v, auto c) __attribute__((always_inline)) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x120 + decltype(c)::value, 0xf, 0xf, true));
+  };
+  x += ror(x, std::integral_constant<int, 8>{});
+  x += ror(x, std::integral_constant<int, 4>{});
+  x += ror(x, std::integral_constant<int, 2>{});
+  return x + ror(x, std::integral_constant<int, 1>{});
+}
+
+template <int NT, int NL>
+__global__ __launch_bounds__((64 * FrontLds<NT, NL>::NW)) void narrow_front_kernel(const FrontParams p) {
+  using L = FrontLds<NT, NL>;
+  constexpr int NW = L::NW, TILES = L::TILES, NLA = NL > 0 ? NL : 1;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const natsl_front& f = p.f;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i16 = lane & 15, g4 = lane >> 4;
+  const int b = (int)blockIdx.x / p.nb, t0 = ((int)blockIdx.x - b * p.nb) * 64, len = min(64, f.T - t0), D = f.D, N = f.NA + f.NB;
+  const size_t row0 = (size_t)b * f.T + t0;
+  const bf16_t* x = reinterpret_cast<const bf16_t*>(f.x) + row0 * D + 8 * g4;
+  const bf16_t *xr[4], *wr[NT], *nr[NLA];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) xr[t] = x + (size_t)min(16 * t + i16, len - 1) * D;
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    const int r = min(16 * n + i16, N - 1);
+    wr[n] = reinterpret_cast<const bf16_t*>(r < f.NA ? f.wa : f.wb) + (size_t)(r < f.NA ? r : r - f.NA) * D + 8 * g4;
+  }
+#pragma unroll
+  for (int n = 0; n < NL; ++n) nr[n] = reinterpret_cast<const bf16_t*>(f.wn) + (size_t)min(16 * n + i16, f.NL - 1) * D + 8 * g4;
+
+  f32x4 acc[4][NT], lacc[NLA];
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[t][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int n = 0; n < NLA; ++n) lacc[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  const float inv = 1.f / (float)len;
+  struct Step { u32x4 x[2][4], w[2][NT], n[2][NLA]; };
+  const int pairs = (D + 63) >> 6;
+  auto load = [&](Step& s, const int pr) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int k = min(64 * pr + 32 * h, D - 32);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) s.x[h][t] = *reinterpret_cast<const u32x4*>(xr[t] + k);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) s.w[h][n] = *reinterpret_cast<const u32x4*>(wr[n] + k);
+#pragma unroll
+      for (int n = 0; n < NL; ++n) s.n[h][n] = *reinterpret_cast<const u32x4*>(nr[n] + k);
+    }
+  };
+  auto use = [&](Step& s, const int pr) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int k = 64 * pr + 32 * h;
+      if (h == 1 && k >= D) break;                  // (the width's odd 32 columns)
+      if (len < 64) {                               // rows past the end count for nothing
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          if (16 * t + i16 >= len) s.x[h][t] = (u32x4){0u, 0u, 0u, 0u};
+      }
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[t][n] = mfma16(__builtin_bit_cast(bf16x8, s.x[h][t]), __builtin_bit_cast(bf16x8, s.w[h][n]), acc[t][n]);
+      if constexpr (NL > 0) {
+        float m[8];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          float lo = 0.f, hi = 0.f;
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            lo += __uint_as_float(s.x[h][t][j] << 16);
+            hi += __uint_as_float(s.x[h][t][j] & 0xffff0000u);
+          }
+          m[2 * j] = row_sum16(lo) * inv;
+          m[2 * j + 1] = row_sum16(hi) * inv;
+        }
+        u32x4 a;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a[j] = pack_bf16x2(m[2 * j], m[2 * j + 1]);
+        if (f.pooled && i16 == 0) *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(f.pooled) + (size_t)blockIdx.x * D + k + 8 * g4) = a;
+#pragma unroll
+        for (int n = 0; n < NL; ++n) lacc[n] = mfma16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, s.n[h][n]), lacc[n]);
+      }
+    }
+  };
+  Step s0, s1;
+  int pr = wave;
+  if (pr < pairs) load(s0, pr);
+  for (; pr < pairs; pr += 2 * NW) {
+    if (pr + NW < pairs) load(s1, pr + NW);
+    use(s0, pr);
+    if (pr + NW >= pairs) break;
+    if (pr + 2 * NW < pairs) load(s0, pr + 2 * NW);
+    use(s1, pr + NW);
+  }
+  // ---- the waves' shares are added in order; rounded rows wait in LDS for the stores and the gates
+  f32x4* red = reinterpret_cast<f32x4*>(smem);
+  bf16_t* rows = reinterpret_cast<bf16_t*>(smem + L::RED);
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) red[(wave * TILES + 4 * n + t) * 64 + lane] = acc[t][n];
+#pragma unroll
+  for (int n = 0; n < NL; ++n) red[(wave * TILES + 4 * NT + n) * 64 + lane] = lacc[n];
+  __syncthreads();
+  for (int j = wave; j < TILES; j += NW) {
+    f32x4 sum = red[j * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) sum += red[(w * TILES + j) * 64 + lane];
+    if (j < 4 * NT) {
+      const int n = j >> 2, t = j & 3;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) rows[(16 * t + 4 * g4 + r) * (16 * NT) + 16 * n + i16] = f32_to_bf16(sum[r]);
+    } else {
+      const int col = 16 * (j - 4 * NT) + i16;      // (all rows of a logits tile are the block's)
+      if (g4 == 0 && col < f.NL) reinterpret_cast<bf16_t*>(f.logits)[(size_t)blockIdx.x * f.NL + col] = f32_to_bf16(sum[0]);
+    }
+  }
+  __syncthreads();
+  if (f.ab) {
+    unsigned* out = reinterpret_cast<unsigned*>(reinterpret_cast<bf16_t*>(f.ab) + row0 * f.ld);
+    const int half = f.ld >> 1;
+    for (int e = threadIdx.x; e < len * half; e += 64 * NW) {
+      const int r = e / half, c = 2 * (e - r * half);
+      const unsigned lo = c < N ? rows[r * (16 * NT) + c] : 0u, hi = c + 1 < N ? rows[r * (16 * NT) + c + 1] : 0u;
+      out[e] = lo | (hi << 16);
+    }
+  }
+  if (f.g) {
+    auto param = [&](const void* q, const int h) __attribute__((always_inline)) {
+      return f.param_dtype == NATSL_F32 ? reinterpret_cast<const float*>(q)[h] : bf16_to_f32(reinterpret_cast<const bf16_t*>(q)[h]);
+    };
+    for (int e = threadIdx.x; e < len * f.NA; e += 64 * NW) {
+      const int r = e / f.NA, h = e - r * f.NA;
+      const float dt = softplus_gate(bf16_to_f32(rows[r * (16 * NT) + h]) + param(f.dt_bias, h));
+      f.g[row0 * f.NA + e] = -expf(param(f.a_log, h)) * dt;
+      if (f.dt) f.dt[row0 * f.NA + e] = dt;
+      if (f.beta) {
+        const float s = bf16_to_f32(f32_to_bf16(sigmoid_gate(bf16_to_f32(rows[r * (16 * NT) + f.NA + h]))));
+        reinterpret_cast<bf16_t*>(f.beta)[row0 * f.NA + e] = f32_to_bf16(f.neg_eigval ? 2.f * s : s);
+      }
+    }
+  }
+  if (f.wab) {   // both weights behind each other and zeros up to wab_rows, for the products of the backward
+    for (int r = blockIdx.x; r < f.wab_rows; r += gridDim.x) {
+      const bf16_t* src = r < f.NA ? reinterpret_cast<const bf16_t*>(f.wa) + (size_t)r * D : reinterpret_cast<const bf16_t*>(f.wb) + (size_t)(r - f.NA) * D;
+      for (int c = 8 * threadIdx.x; c < D; c += 8 * 64 * NW)
+        *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(f.wab) + (size_t)r * D + c) =
+            r < N ? *reinterpret_cast<const u32x4*>(src + c) : (u32x4){0u, 0u, 0u, 0u};
+    }
+  }
+}
+
+template <int NT, int NL>
+static int launch_front(const FrontParams& p, hipStream_t s, const char* what) {
+  using L = FrontLds<NT, NL>;
+  auto kern = narrow_front_kernel<NT, NL>;
+  static std::atomic<unsigned long long> reserved{0};
+  if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, L::TOTAL, what)) return rc;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(p.f.B * p.nb)), dim3(64 * L::NW), L::TOTAL, s, p);
+  return check_launch(what);
+}
+
+// ---- backward ------------------------------------------------------------------------------------------------------------------------
 constexpr int NARROW_MAX = 48;                 // rows of the weight
 
 struct NarrowParams {
@@ -83,9 +273,91 @@ __global__ __launch_bounds__(256) void narrow_bwd_kernel(const NarrowParams p) {
   }
 }
 
+// dW[n][d] = sum_t dY[t][n] X[t][d] for a narrow weight over few rows (the block means behind the selector's).  A workgroup takes 32 columns and
+// every row of the weight, its eight waves the tokens, 32 at a time in turn; both operands have the tokens along the contraction and are
+// gathered from the rows as they lie (X two columns a word: one product for the even, one for the odd ones).  Added up through LDS in order.
+constexpr int NWG_WAVES = 8;
+template <int NT>
+__global__ __launch_bounds__(64 * NWG_WAVES) void narrow_wgrad_kernel(const bf16_t* dy, const bf16_t* x, bf16_t* dw, const int rows, const int D, const int N) {
+  __shared__ f32x4 sums[NWG_WAVES][2 * NT][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i16 = lane & 15, g4 = lane >> 4;
+  const int d = 32 * (int)blockIdx.x + 2 * i16;
+  f32x4 acc[2][NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) acc[0][n] = acc[1][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  const bf16_t* xc = x + min(d, D - 2);
+#pragma unroll 2
+  for (int t0 = 32 * wave; t0 < rows; t0 += 32 * NWG_WAVES) {
+    unsigned xv[8];
+    bf16_t yv[NT][8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int t = t0 + 8 * g4 + j;
+      const size_t r = (size_t)min(t, rows - 1);
+      const unsigned v = *reinterpret_cast<const unsigned*>(xc + r * D);
+      xv[j] = t < rows ? v : 0u;
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        const bf16_t y = dy[r * N + min(16 * n + i16, N - 1)];
+        yv[n][j] = t < rows ? y : 0;               // (both sides: nothing that a row behind the end holds enters a product)
+      }
+    }
+    u32x4 be, bo;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      be[j] = (xv[2 * j] & 0xffffu) | (xv[2 * j + 1] << 16);
+      bo[j] = (xv[2 * j] >> 16) | (xv[2 * j + 1] & 0xffff0000u);
+    }
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      u32x4 a;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) a[j] = (unsigned)yv[n][2 * j] | ((unsigned)yv[n][2 * j + 1] << 16);
+      acc[0][n] = mfma16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, be), acc[0][n]);
+      acc[1][n] = mfma16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, bo), acc[1][n]);
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    sums[wave][2 * n][lane] = acc[0][n];
+    sums[wave][2 * n + 1][lane] = acc[1][n];
+  }
+  __syncthreads();
+  if (wave >= NT || d >= D) return;                // wave n ends 16 rows of the weight
+  f32x4 e = {0.f, 0.f, 0.f, 0.f}, o = e;
+#pragma unroll
+  for (int w = 0; w < NWG_WAVES; ++w) {
+    e += sums[w][2 * wave][lane];
+    o += sums[w][2 * wave + 1][lane];
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int n = 16 * wave + 4 * g4 + r;
+    if (n < N) *reinterpret_cast<unsigned*>(dw + (size_t)n * D + d) = pack_bf16x2(e[r], o[r]);
+  }
+}
+
 }  // namespace natsl
 
 using namespace natsl;
+
+extern "C" int natsl_narrow_wgrad(const void* dy, const void* x, void* dw, int64_t rows, int D, int N, natsl_stream_t stream) {
+  const char* what = "natsl_narrow_wgrad";
+  if (!dy || !x || !dw) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
+  if (rows <= 0 || D <= 0 || N <= 0) return fail(NATSL_ERR_INVALID, "%s: non-positive dimension", what);
+  if (N > 64 || D % 2 || rows > 0x7fffff00ll) return fail(NATSL_ERR_UNSUPPORTED, "%s: N=%d (up to 64), D=%d (even)", what, N, D);
+  if (((uintptr_t)x | (uintptr_t)dw) & 3) return fail(NATSL_ERR_INVALID, "%s: tensors must start on 4 bytes", what);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const dim3 grid((unsigned)cdiv(D, 32)), wg(64 * NWG_WAVES);
+  const bf16_t *y = (const bf16_t*)dy, *xx = (const bf16_t*)x;
+  switch (cdiv(N, 16)) {
+    case 1: hipLaunchKernelGGL(narrow_wgrad_kernel<1>, grid, wg, 0, s, y, xx, (bf16_t*)dw, (int)rows, D, N); break;
+    case 2: hipLaunchKernelGGL(narrow_wgrad_kernel<2>, grid, wg, 0, s, y, xx, (bf16_t*)dw, (int)rows, D, N); break;
+    case 3: hipLaunchKernelGGL(narrow_wgrad_kernel<3>, grid, wg, 0, s, y, xx, (bf16_t*)dw, (int)rows, D, N); break;
+    default: hipLaunchKernelGGL(narrow_wgrad_kernel<4>, grid, wg, 0, s, y, xx, (bf16_t*)dw, (int)rows, D, N); break;
+  }
+  return check_launch(what);
+}
 
 extern "C" int natsl_narrow_linear_bwd(const void* dy, const void* w, void* dx, int64_t rows, int D, int N, natsl_stream_t stream) {
   const char* what = "natsl_narrow_linear_bwd";
@@ -103,4 +375,27 @@ extern "C" int natsl_narrow_linear_bwd(const void* dy, const void* w, void* dx, 
     default: hipLaunchKernelGGL(narrow_bwd_kernel<3>, grid, dim3(256), 0, s, p); break;
   }
   return check_launch(what);
+}
+
+extern "C" int natsl_layer_front(const natsl_front* a, natsl_stream_t stream) {
+  const char* what = "natsl_layer_front";
+  if (!a || !a->x || !a->wa || (a->NB > 0 && !a->wb) || (a->NL > 0 && (!a->wn || !a->logits)) || (a->g && (!a->a_log || !a->dt_bias)) || (!a->ab && !a->g))
+    return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
+  if (a->B <= 0 || a->T <= 0 || a->D <= 0 || a->NA <= 0 || a->NB < 0 || a->NL < 0) return fail(NATSL_ERR_INVALID, "%s: non-positive dimension", what);
+  const int N = a->NA + a->NB;
+  if (a->D % 32 || N > 64 || a->NL > 64 || (a->NL > 0 && N > 32))
+    return fail(NATSL_ERR_UNSUPPORTED, "%s: D=%d (a multiple of 32), %d rows (up to 64, 32 next to logits), %d logits (up to 64)", what, a->D, N, a->NL);
+  if ((a->ab && (a->ld < N || a->ld % 2)) || (a->beta && (!a->g || a->NB < a->NA)) || (a->dt && !a->g))
+    return fail(NATSL_ERR_UNSUPPORTED, "%s: rows of %d for %d columns, or gates that do not belong together", what, a->ld, N);
+  if (a->param_dtype != NATSL_BF16 && a->param_dtype != NATSL_F32) return fail(NATSL_ERR_UNSUPPORTED, "%s: parameters must be f32 or bf16", what);
+  if (((uintptr_t)a->x | (uintptr_t)a->wa | (uintptr_t)a->wb | (uintptr_t)a->wn | (uintptr_t)a->pooled | (uintptr_t)a->wab) & 15 || (uintptr_t)a->ab & 3)
+    return fail(NATSL_ERR_INVALID, "%s: tensors must start on 16 bytes", what);
+  FrontParams p{*a, cdiv(a->T, 64)};
+  if ((long long)a->B * p.nb > 0x7fffffffll) return fail(NATSL_ERR_UNSUPPORTED, "%s: problem too large", what);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const int nt = cdiv(N, 16), nl = cdiv(a->NL, 16);
+  if (nt == 4) return launch_front<4, 0>(p, s, what);
+  if (nt == 3) return launch_front<3, 0>(p, s, what);
+  if (nt == 2) return nl == 0 ? launch_front<2, 0>(p, s, what) : nl == 1 ? launch_front<2, 1>(p, s, what) : nl == 2 ? launch_front<2, 2>(p, s, what) : launch_front<2, 4>(p, s, what);
+  return nl == 0 ? launch_front<1, 0>(p, s, what) : nl == 1 ? launch_front<1, 1>(p, s, what) : nl == 2 ? launch_front<1, 2>(p, s, what) : launch_front<1, 4>(p, s, what);
 }

@@ -223,16 +223,15 @@ class NeuralAttentionSearchLinearAttnGDN(nn.Module):
         conv_states = cache.conv_state if cache is not None and cache.conv_state is not None else (None, None, None)
         if fast is not None:
             whole = selector_input is hidden_states
-            q, k, v, gate, ab, pooled = fast.project(hidden_states, self.nats_block_size if whole else 0)
+            q, k, v, gate, (g, beta, _), logits = fast.project(hidden_states, self.nats_block_size if whole else 0, self.nats_layer)
             if not whole:
-                pooled = nats_util.mean_pooling(selector_input, self.nats_block_size)
-            logits = self.nats_layer(pooled).unflatten(-1, (self.num_nats_head, self.n_ops))
+                logits = self.nats_layer(nats_util.mean_pooling(selector_input, self.nats_block_size))
+            logits = logits.unflatten(-1, (self.num_nats_head, self.n_ops))
             # (the types before the last block is forced are only needed where states are handed on)
             types, n_nats_blocks, attn_fraction, raw_types = fast.select(logits, bool(use_cache) or cache is not None)
             if cache is not None:
                 cache.foresee(raw_types, q_len)
             q, k, v, q_attn, k_attn, o_mix, _, _, v_attn, new_conv_states = fast.conv_norm(q, k, v, conv_states, bool(use_cache))
-            g, beta, _ = fast.gates(ab)
             q, k = (x.unflatten(-1, (-1, self.head_k_dim)) for x in (q, k))
             v = v.unflatten(-1, (-1, self.head_v_dim))
             q_attn, k_attn = (x.unflatten(-1, (-1, self.head_attn_k_dim)) for x in (q_attn, k_attn))

@@ -334,3 +334,66 @@ def test_narrow_projections_of_any_count_join_the_backward(n_a, n_b):
     want = torch.autograd.grad(outs + [means], [x32] + w32, ups)
     for a, b in zip(got, want):
         assert a.shape == b.shape and rel_l2(a.float(), b) <= 2 ** -8
+
+
+@pytest.mark.parametrize("B,T,D,n_a,n_b,n_l,params", [
+    (1, 1, 32, 1, 0, 0, torch.float32), (2, 63, 96, 6, 6, 12, torch.bfloat16), (1, 64, 512, 16, 0, 32, torch.float32), (3, 65, 544, 8, 8, 2, torch.bfloat16),
+    (2, 129, 1536, 6, 6, 12, torch.float32), (1, 257, 1024, 16, 16, 64, torch.bfloat16), (1, 200, 160, 36, 0, 0, torch.float32), (1, 70, 1184, 31, 31, 0, torch.float32)])
+def test_narrow_front(B, T, D, n_a, n_b, n_l, params):
+    """natsl_layer_front at the edges of its 64-token tiles, of its 64-column steps and of 16 weight rows, with and without logits; what it refuses."""
+    import ctypes
+    from neuralattentionsearchlinear_amd import _capi
+    from neuralattentionsearchlinear_amd._front import _FrontArgs
+    torch.manual_seed(T + D)
+    L, nb, ld, N = _capi.lib(), -(-T // 64), -(-(n_a + n_b) // 32) * 32, n_a + n_b
+    bf = lambda *s: (torch.randn(*s, device=DEV) / D ** 0.25).bfloat16()
+    x, wa, wb, wn = bf(B, T, D), bf(n_a, D), bf(n_b, D), bf(n_l, D)
+    a_log, bias = torch.randn(n_a, device=DEV).to(params), torch.randn(n_a, device=DEV).to(params)
+    delta = n_b == n_a
+    full = lambda *s, dt=torch.bfloat16: torch.full(s, 7., device=DEV, dtype=dt)
+    ab, pooled, logits, wab = full(B * T + 1, ld), full(B * nb + 1, D), full(B * nb + 1, max(n_l, 1)), full(ld + 1, D)
+    g, beta, dt = full(B * T + 1, n_a, dt=torch.float32), full(B * T + 1, n_a), full(B * T + 1, n_a, dt=torch.float32)
+    a = _FrontArgs()
+    for n, t in dict(x=x, wa=wa, wb=wb if n_b else None, wn=wn if n_l else None, a_log=a_log, dt_bias=bias, ab=ab, pooled=pooled if n_l else None,
+                     logits=logits if n_l else None, beta=beta if delta else None, wab=wab, g=g, dt=dt).items():
+        setattr(a, n, None if t is None else t.data_ptr())
+    a.B, a.T, a.D, a.NA, a.NB, a.NL, a.ld, a.neg_eigval, a.param_dtype, a.wab_rows = B, T, D, n_a, n_b, n_l, ld, int(T % 2), _capi.dtype_code(params), ld
+    run = lambda: L.natsl_layer_front(ctypes.byref(a), _capi.stream_ptr(x.device))
+    _capi.check(run(), "natsl_layer_front")
+    # exact products, fp32 sums, one rounding to bf16
+    close = lambda got, ref, k: bool(((got.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * k ** 0.5).all())
+    x2 = x.view(B * T, D).double()
+    assert close(ab[:B * T, :N], x2 @ torch.cat([wa, wb]).double().t(), D) and not bool(ab[:B * T, N:].any())
+    assert torch.equal(wab[:N], torch.cat([wa, wb])) and not bool(wab[N:ld].any())
+    if n_l:
+        means = torch.stack([x[:, t:t + 64].double().mean(1) for t in range(0, T, 64)], 1).view(B * nb, D)
+        assert close(pooled[:B * nb], means, 64) and close(logits[:B * nb], pooled[:B * nb].double() @ wn.double().t(), D)
+    step = torch.nn.functional.softplus(ab[:B * T, :n_a].double() + bias.double())
+    assert torch.allclose(dt[:B * T].double(), step, rtol=1e-5, atol=1e-30) and torch.allclose(g[:B * T].double(), -a_log.double().exp() * step, rtol=1e-5, atol=1e-30)
+    if delta:
+        ref = torch.sigmoid(ab[:B * T, n_a:N].double()) * (2 if T % 2 else 1)
+        assert close(beta[:B * T], ref, 1)
+    for t in (ab, pooled, logits, wab, g, beta, dt):                        # nothing behind the ends
+        assert bool((t[-1] == 7).all())
+    a.D = D + 8
+    assert run() != 0
+    a.D, a.NL = D, 65 if n_l else 0
+    a.NA = n_a if n_l else 65
+    assert run() != 0
+
+
+@pytest.mark.parametrize("rows,D,N", [(1, 32, 2), (31, 96, 12), (33, 1024, 16), (256, 130, 17), (513, 1152, 36), (1024, 64, 64)])
+def test_narrow_weight_gradient(rows, D, N):
+    """natsl_narrow_wgrad at the edges of its 32-token steps, 32 columns and 16 weight rows; and the library where it is not chosen."""
+    from neuralattentionsearchlinear_amd import _capi, _front
+    torch.manual_seed(rows)
+    L, P = _capi.lib(), _capi.ptr
+    x, dy = torch.randn(rows, D, device=DEV).bfloat16(), torch.randn(rows, N, device=DEV).bfloat16()
+    dw = torch.full((N + 1, D), 7., device=DEV).bfloat16()
+    _capi.check(L.natsl_narrow_wgrad(P(dy), P(x), P(dw), rows, D, N, _capi.stream_ptr(x.device)), "natsl_narrow_wgrad")
+    ref = dy.double().t() @ x.double()
+    close = lambda got: bool(((got.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * rows ** 0.5).all())
+    assert close(dw[:N]) and bool((dw[N] == 7).all()) and close(_front._narrow_wgrad(dy, x))
+    assert L.natsl_narrow_wgrad(P(dy), P(x), P(dw), rows, D, 65, _capi.stream_ptr(x.device)) != 0
+    many = torch.randn(2049, N, device=DEV).bfloat16(), torch.randn(2049, D, device=DEV).bfloat16()
+    assert torch.equal(_front._narrow_wgrad(*many), torch.mm(many[0].t(), many[1]))

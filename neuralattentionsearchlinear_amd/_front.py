@@ -40,7 +40,8 @@ class _FrontArgs(ctypes.Structure):
 class _ConvSeg(ctypes.Structure):
     _fields_ = ([(n, ctypes.c_void_p) for n in ("x", "weight", "bias", "state", "norm_weight", "y", "y_norm", "state_out", "dy_a", "dy_b", "dy_norm",
                                                 "dx_add", "dx", "dweight", "dbias", "dnorm_weight")] +
-                [("D", ctypes.c_int32), ("norm_lanes", ctypes.c_int32), ("norm_l2", ctypes.c_int32), ("norm_eps", ctypes.c_float)])
+                [("D", ctypes.c_int32), ("norm_lanes", ctypes.c_int32), ("norm_l2", ctypes.c_int32), ("norm_eps", ctypes.c_float),
+                 ("scale", ctypes.c_void_p), ("dscale", ctypes.c_void_p)])
 
 
 def _p(t):
@@ -296,28 +297,33 @@ def _narrow_wgrad(dy, x):
 
 
 # ---- convolutions, norms, mixing logits --------------------------------------------------------------------------------------------
-def _conv_segs(f, raw):
-    """The segments of natsl_conv_norm_*: q, k, v with their weights; f: the layer's FastFront."""
+def _conv_segs(f, raw, dt=None):
+    """The segments of natsl_conv_norm_*: q, k, v with their weights; f: the layer's FastFront; dt: what conv(v)'s heads are multiplied by, or None."""
     segs = (_ConvSeg * 3)()
     for s, x, n in zip(segs, raw, "qkv"):
         s.x, s.D, s.weight, s.bias = x.data_ptr(), x.shape[-1], _p(f.w["conv_w" + n]), _p(f.w["conv_b" + n])
+        if n == "v" and dt is not None:
+            s.norm_lanes, s.scale = x.shape[-1] // f.H // 8, dt.data_ptr()
         if n != "v":
             s.norm_lanes, s.norm_l2, s.norm_eps = f.norm_width // 8, int(f.l2), f.front_eps
             s.norm_weight = None if f.l2 else f.w["norm_" + n].data_ptr()
     return segs
 
 
-def _conv_norm(f, raw, states, want_states):
-    """-> (conv(q) or None, conv(k) or None, conv(v), normed q, normed k, new states)."""
+def _conv_norm(f, raw, states, want_states, dt=None):
+    """-> (conv(q) or None, conv(k) or None, conv(v) (times dt), normed q, normed k, new states)."""
     B, T, _ = raw[0].shape
-    segs = _conv_segs(f, raw)
+    segs = _conv_segs(f, raw, dt)
     ys = [torch.empty_like(raw[0]), None if f.l2 else torch.empty_like(raw[1]), torch.empty_like(raw[2])]
     ns = [torch.empty_like(raw[0]), torch.empty_like(raw[1])]
     new = None
     if want_states:
         new = tuple([torch.empty(B, x.shape[-1], f.W, dtype=torch.bfloat16, device=x.device) for x in raw])
     for i, s in enumerate(segs):
-        s.y = _p(ys[i])
+        if i < 2 or dt is None:
+            s.y = _p(ys[i])
+        else:
+            s.y_norm = ys[i].data_ptr()
         if i < 2:
             s.y_norm = ns[i].data_ptr()
         if states is not None and states[i] is not None:
@@ -329,15 +335,15 @@ def _conv_norm(f, raw, states, want_states):
 
 
 class _ConvNorm(torch.autograd.Function):
-    """(q, k, v projections) -> (conv(q), conv(k), conv(v), normed q, normed k, mixing logits, and what attention takes:
+    """(q, k, v projections) -> (conv(q), conv(k), conv(v) (times dt where that is given), normed q, normed k, mixing logits, and what attention takes:
     the projections themselves, or only conv(v) once more); the last three only carry attention's gradient to where it is added (dx_add, dy_b)."""
 
     @staticmethod
-    def forward(ctx, f, q, k, v, wq, bq, wk, bk, wv, bv, nq, nk, w_mix):
-        ys, ns, _ = _conv_norm(f, (q, k, v), None, False)
+    def forward(ctx, f, q, k, v, wq, bq, wk, bk, wv, bv, nq, nk, w_mix, dt):
+        ys, ns, _ = _conv_norm(f, (q, k, v), None, False, dt)
         ctx.f = f
         # (the parameters are saved for the check that nobody changes them before the backward reads them through f)
-        ctx.save_for_backward(q, k, v, ys[0], w_mix, wq, bq, wk, bk, wv, bv, nq, nk)
+        ctx.save_for_backward(q, k, v, ys[0], w_mix, dt, wq, bq, wk, bk, wv, bv, nq, nk)
         ctx.set_materialize_grads(False)
         raw = tuple(t.view(t.shape) for t in (q, k, v)) if f.raw_attention else (None, None, ys[2].detach())
         return (ys[0], ys[1], ys[2], ns[0], ns[1], F.linear(ys[0], w_mix)) + raw
@@ -345,7 +351,7 @@ class _ConvNorm(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dq, dk, dv, dqn, dkn, dlogits, dq_raw, dk_raw, dv_raw):
         f = ctx.f
-        q, k, v, yq, w_mix = ctx.saved_tensors[:5]
+        q, k, v, yq, w_mix, dt = ctx.saved_tensors[:6]
         B, T, _ = q.shape
         dev = q.device
         dw_mix = dq_mix = None
@@ -361,12 +367,17 @@ class _ConvNorm(torch.autograd.Function):
             t = t.contiguous()
             hold.append(t)
             return t.data_ptr()
-        segs = _conv_segs(f, (q, k, v))
-        dv_conv = None
+        segs = _conv_segs(f, (q, k, v), dt)
+        dv_conv = dv_scaled = ddt = None
         if not f.raw_attention:
             dv_conv, dv_raw = dv_raw, None
+        if dt is not None:
+            dv, dv_scaled = None, dv
+            if dv_scaled is not None and ctx.needs_input_grad[13]:
+                ddt = torch.empty_like(dt)
+                segs[2].dscale = ddt.data_ptr()
         grads = []
-        for s, x, n, da, db, dn, add in zip(segs, (q, k, v), "qkv", (dq, dk, dv), (dq_mix, None, dv_conv), (dqn, dkn, None), (dq_raw, dk_raw, dv_raw)):
+        for s, x, n, da, db, dn, add in zip(segs, (q, k, v), "qkv", (dq, dk, dv), (dq_mix, None, dv_conv), (dqn, dkn, dv_scaled), (dq_raw, dk_raw, dv_raw)):
             w, b = f.w["conv_w" + n], f.w["conv_b" + n]
             dx, dw = torch.empty_like(x), torch.empty_like(w)
             dbias = None if b is None else torch.empty_like(b)
@@ -381,7 +392,7 @@ class _ConvNorm(torch.autograd.Function):
         ws = torch.empty(n, dtype=torch.uint8, device=dev)
         _capi.check(L.natsl_conv_norm_bwd(segs, 3, B, T, f.W, f.act, f.norm_dtype, ws.data_ptr(), n, _capi.stream_ptr(dev)), "natsl_conv_norm_bwd")
         (dxq, dwq, dbq, dnq), (dxk, dwk, dbk, dnk), (dxv, dwv, dbv, _) = grads
-        return None, dxq, dxk, dxv, dwq, dbq, dwk, dbk, dwv, dbv, dnq, dnk, dw_mix
+        return None, dxq, dxk, dxv, dwq, dbq, dwk, dbk, dwv, dbv, dnq, dnk, dw_mix, ddt
 
 
 # ---- gates ---------------------------------------------------------------------------------------------------------------------------
@@ -533,15 +544,16 @@ class FastFront:
         q, k, v, gate, ab, pooled = _Project.apply(*args) if self.grad(*args[:7]) else _project(*args)[0]
         return q, k, v, gate, self.gates(ab), selector(pooled) if pool_block else None
 
-    def conv_norm(self, q, k, v, states, want_states):
-        """-> (conv(q), conv(k) or None, conv(v), normed q, normed k, mixing logits, raw q, k, v
-        (or None, None, conv(v) again: attention's), new states)."""
+    def conv_norm(self, q, k, v, states, want_states, dt=None):
+        """-> (conv(q), conv(k) or None, conv(v) (times dt), normed q, normed k, mixing logits, raw q, k, v
+        (or None, None, conv(v) again: attention's), new states).  dt (`takes_dt` only): fp32 [B,T,H], a number for every head of conv(v); as
+        separate passes (a training step of the Mamba layer, 8 x 4096) it is seven launches and 0.4 ms."""
         w = self.w
         args = (q, k, v, w["conv_wq"], w["conv_bq"], w["conv_wk"], w["conv_bk"], w["conv_wv"], w["conv_bv"],
-                w["norm_q"] if self.delta else None, w["norm_k"] if self.delta else None, w["w_mix"])
+                w["norm_q"] if self.delta else None, w["norm_k"] if self.delta else None, w["w_mix"], dt)
         if self.grad(*args):
             return _ConvNorm.apply(self, *args) + (None,)
-        ys, ns, new = _conv_norm(self, (q, k, v), states, want_states)
+        ys, ns, new = _conv_norm(self, (q, k, v), states, want_states, dt)
         return ys[0], ys[1], ys[2], ns[0], ns[1], F.linear(ys[0], w["w_mix"]), *((q, k, v) if self.raw_attention else (None, None, ys[2])), new
 
     def gates(self, ab):
@@ -591,7 +603,7 @@ def _front_plan(layer, kind, w):
     code = lambda n: _capi.dtype_code(w[n].dtype)
     return dict(delta=delta, H=layer.num_heads, W=layer.conv_size, act=0 if layer.q_conv1d.activation is None else 1, l2=not delta,
                 raw_attention=not delta, norm_width=width, front_eps=norms[0].eps, norm_dtype=code("norm_q") if delta else _capi.BF16,
-                gate_dtype=code("a_log"), out_dtype=code("out_norm1"), neg=int(delta and layer.allow_neg_eigval), out_eps=layer.o_norm.eps)
+                takes_dt=layer.head_v_dim in (8, 16, 32, 64, 128, 256, 512), gate_dtype=code("a_log"), out_dtype=code("out_norm1"), neg=int(delta and layer.allow_neg_eigval), out_eps=layer.o_norm.eps)
 
 
 def _selector_weight(layer, like):

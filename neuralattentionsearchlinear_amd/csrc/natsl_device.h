@@ -91,6 +91,9 @@ NATSL_DEVICE float xhalf_sum(float x) {
 NATSL_DEVICE float softplus_gate(const float x) { return x > 20.f ? x : log1pf(expf(x)); }
 NATSL_DEVICE float sigmoid_gate(const float x) { return 1.f / (1.f + expf(-x)); }
 
+// The convolutions' backward: the hardware's reciprocal is within an ulp, __expf's own error is larger, and a division is ten instructions
+NATSL_DEVICE float sigmoid_fast(const float x) { return __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
+
 // The softmax of a head's two mixing logits, rounded to bf16: what the mixing layer's separate softmax returns
 NATSL_DEVICE void mix_softmax(float& a, float& b) {
   const float mx = fmaxf(a, b), e0 = expf(a - mx), e1 = expf(b - mx);

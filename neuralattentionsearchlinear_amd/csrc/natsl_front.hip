@@ -1,12 +1,14 @@
 // The front of the hybrid layers around their projections: short convolutions with the row norms that follow them, the gates, the
 // input gradient's first terms, and the selector's straight-through gradient.  All of it is bound by HBM traffic (and, for short
 // inputs, by launches), so what touches the same rows is one pass and q, k, v share a launch:
-//   conv_norm_kernel      y = act(conv(x)) and, per head, rms(y) w or l2(y): one read, two writes
-//   conv_norm_bwd_kernel  the gradients that meet at y (linear branch, mixing logits, through the norm) are added in registers, then
+//   conv_norm_kernel      y = act(conv(x)) and, per head, rms(y) w, l2(y) or y times a number: one read, two writes
+//   conv_norm_bwd_kernel  the gradients that meet at y (linear branch, mixing logits, through the norm or the number) are added in registers, then
 //                         the convolution's backward; weight sums per run of tokens, added up in a fixed order afterwards
 //   gates_kernel          g = -exp(A_log) softplus(a + dt_bias), beta = sigmoid(b) (GDN) / dt (Mamba), and its backward
 //   dx_init_kernel        block mean's gradient spread over its tokens + the narrow projections' share of dx: what the four wide
 //                         products then accumulate onto
+#include <type_traits>
+
 #include "natsl_device.h"
 #include "natsl_host.h"
 
@@ -34,18 +36,64 @@ NATSL_DEVICE u32x4 down8(const float* f) {
 }
 NATSL_DEVICE const u32x4* row8(const void* p, const size_t elem) { return reinterpret_cast<const u32x4*>(reinterpret_cast<const bf16_t*>(p) + elem); }
 
-// sums over the `lanes` adjacent lanes (a power of two) that share a head row
+// CH adjacent channels as they lie in memory, and as fp32
+template <int CH> struct Piece;
+template <> struct Piece<8> {
+  typedef u32x4 type;
+  static NATSL_DEVICE type at(const void* p, const size_t elem) { return *row8(p, elem); }
+  static NATSL_DEVICE void up(const type w, float* f) { up8(w, f); }
+  static NATSL_DEVICE type down(const float* f) { return down8(f); }
+};
+template <> struct Piece<4> {
+  typedef u32x2 type;
+  static NATSL_DEVICE type at(const void* p, const size_t elem) { return *reinterpret_cast<const u32x2*>(reinterpret_cast<const bf16_t*>(p) + elem); }
+  static NATSL_DEVICE void up(const type w, float* f) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      f[2 * j] = __uint_as_float(w[j] << 16);
+      f[2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
+    }
+  }
+  static NATSL_DEVICE type down(const float* f) { return (u32x2){pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3])}; }
+};
+
+// sums over the `lanes` adjacent lanes (a power of two, the same for the wave) that share a head row
 NATSL_DEVICE void group_sum2(float& a, float& b, const int lanes) {
-  for (int d = 1; d < lanes; d <<= 1) {
-    a += __shfl_xor(a, d);
-    b += __shfl_xor(b, d);
+  auto add = [&](auto c) __attribute__((always_inline)) {
+    a += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(a), decltype(c)::value, 0xf, 0xf, true));
+    b += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(b), decltype(c)::value, 0xf, 0xf, true));
+  };
+  auto first = [&]() __attribute__((always_inline)) {
+    add(std::integral_constant<int, 0xb1>{});    // lane ^ 1
+    add(std::integral_constant<int, 0x4e>{});    // lane ^ 2
+    add(std::integral_constant<int, 0x141>{});   // 7 - lane: the other four, which all hold their sum
+  };
+  if (lanes == 8) {
+    first();
+  } else if (lanes >= 16) {
+    first();
+    add(std::integral_constant<int, 0x140>{});   // 15 - lane
+    if (lanes >= 32) {
+      auto both = [](const u32x2 r) __attribute__((always_inline)) { return __uint_as_float(r[0]) + __uint_as_float(r[1]); };
+      a = both(__builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(a), false, false));
+      b = both(__builtin_amdgcn_permlane16_swap(__float_as_uint(b), __float_as_uint(b), false, false));
+      if (lanes == 64) {
+        a = xhalf_sum(a);
+        b = xhalf_sum(b);
+      }
+    }
+  } else {
+    for (int d = 1; d < lanes; d <<= 1) {
+      a += __shfl_xor(a, d);
+      b += __shfl_xor(b, d);
+    }
   }
 }
 
 struct ConvNormParams {
   natsl_conv_seg seg[NATSL_CONV_SEGS];
   int first[NATSL_CONV_SEGS + 1];     // the segments' first workgroups
-  int n_seg, B, T, run, silu, norm_dtype;
+  int n_seg, B, T, run, silu, norm_dtype, ch;   // ch: channels of a thread
   float* part[NATSL_CONV_SEGS];        // backward: [run id][W+2][D] sums (taps, bias, norm weight)
 };
 
@@ -104,7 +152,8 @@ __global__ __launch_bounds__(256) void conv_norm_kernel(const ConvNormParams p) 
       for (int c = 0; c < 8; ++c) so[((size_t)b * D + d0 + c) * W + j] = f32_to_bf16(e[c]);
     }
   }
-  auto one_row = [&](const u32x4 in, const int t) __attribute__((always_inline)) {
+  auto number = [&](const int t) __attribute__((always_inline)) { return s.scale ? s.scale[((size_t)b * T + t) * (groups / s.norm_lanes) + cg / s.norm_lanes] : 0.f; };
+  auto one_row = [&](const u32x4 in, const float num, const int t) __attribute__((always_inline)) {
     float y[8], ss = 0.f, none = 0.f;
     up8(in, win[W - 1]);
 #pragma unroll
@@ -119,10 +168,13 @@ __global__ __launch_bounds__(256) void conv_norm_kernel(const ConvNormParams p) 
     if (s.y) *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(s.y) + at) = packed;
     if (s.y_norm) {
       up8(packed, y);
+      float rs = num;
+      if (!s.scale) {                                   // (nw is one where it is)
 #pragma unroll
-      for (int c = 0; c < 8; ++c) ss += y[c] * y[c];
-      group_sum2(ss, none, s.norm_lanes);
-      const float rs = rsqrtf((s.norm_l2 ? ss : ss / (8 * s.norm_lanes)) + s.norm_eps);
+        for (int c = 0; c < 8; ++c) ss += y[c] * y[c];
+        group_sum2(ss, none, s.norm_lanes);
+        rs = rsqrtf((s.norm_l2 ? ss : ss / (8 * s.norm_lanes)) + s.norm_eps);
+      }
 #pragma unroll
       for (int c = 0; c < 8; ++c) y[c] *= rs * nw[c];
       *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(s.y_norm) + at) = down8(y);
@@ -136,31 +188,40 @@ __global__ __launch_bounds__(256) void conv_norm_kernel(const ConvNormParams p) 
   int tb = t0;
   for (; tb + AHEAD <= t1; tb += AHEAD) {   // (no way out between a batch's loads and their use: they all go out together)
     u32x4 rows[AHEAD];
+    float num[AHEAD];
 #pragma unroll
-    for (int a = 0; a < AHEAD; ++a) rows[a] = *row8(s.x, base + (size_t)(tb + a) * D);
+    for (int a = 0; a < AHEAD; ++a) {
+      rows[a] = *row8(s.x, base + (size_t)(tb + a) * D);
+      num[a] = number(tb + a);
+    }
 #pragma unroll
-    for (int a = 0; a < AHEAD; ++a) one_row(rows[a], tb + a);
+    for (int a = 0; a < AHEAD; ++a) one_row(rows[a], num[a], tb + a);
   }
-  for (; tb < t1; ++tb) one_row(*row8(s.x, base + (size_t)tb * D), tb);
+  for (; tb < t1; ++tb) one_row(*row8(s.x, base + (size_t)tb * D), number(tb), tb);
 }
 
-// Backward: dy = dy_a + dy_b + (norm's backward of dy_norm), then dpre = dy act'(pre), dx[s] = sum_i w[W-1-i] dpre[s+i] + dx_add[s],
-// dw[j] = sum dpre[t] x[t-(W-1)+j].  pre and y are recomputed from x; two rows of every input are requested at a time.  A thread
+// Backward: dy = dy_a + dy_b + (backward of the norm, or of the number, of dy_norm), then dpre = dy act'(pre), dx[s] = sum_i w[W-1-i] dpre[s+i] +
+// dx_add[s], dw[j] = sum dpre[t] x[t-(W-1)+j].  pre and y are recomputed from x; a few rows of every input are requested at a time.  A thread
 // reads W-1 rows past its run (for dx of the run's last tokens) without adding them to its sums.
-template <int W>
+// Bound by vector issue and the bytes alike (340M geometry 0.86 GB, a Mamba layer 1.48 GB at 8 x 4096): 215 -> 198 and 455 -> 329 us, 760M 2 x 3000
+// 76 -> 62, against a branch around every channel's activation, a division in it, the head sums through LDS, dx_add requested where it is used and
+// eight channels a thread.  Four channels with two rows ahead 206 and 346, with four 245 and 360 (175 registers: two waves a SIMD).
+// A thread has CH channels: four (eight hold 229 - 262 registers, two waves a SIMD or one), eight for heads of 512, which have to fit a wave.
+template <int W, bool SILU, int CH>
 __global__ __launch_bounds__(256) void conv_norm_bwd_kernel(const ConvNormParams p) {
+  typedef Piece<CH> Pc;
   const int si = conv_segment(p);
   const natsl_conv_seg& s = p.seg[si];
-  const int D = s.D, T = p.T, groups = D / 8, runs = (T + p.run - 1) / p.run;
+  const int D = s.D, T = p.T, groups = D / CH, runs = (T + p.run - 1) / p.run;
   const long long gid = (long long)((int)blockIdx.x - p.first[si]) * 256 + threadIdx.x;
   if (gid >= (long long)p.B * runs * groups) return;
   const int cg = (int)(gid % groups), r = (int)((gid / groups) % runs), b = (int)(gid / ((long long)groups * runs));
-  const int d0 = 8 * cg, t0 = r * p.run, t1 = min(T, t0 + p.run);
+  const int d0 = CH * cg, t0 = r * p.run, t1 = min(T, t0 + p.run);
   const bf16_t* w = reinterpret_cast<const bf16_t*>(s.weight);
   const bf16_t* st = reinterpret_cast<const bf16_t*>(s.state);
-  float wt[W][8], bs[8], win[W][8], dwin[W][8], dws[W + 2][8], nw[8];
+  float wt[W][CH], bs[CH], win[W][CH], dwin[W][CH], dws[W + 2][CH], nw[CH];
 #pragma unroll
-  for (int c = 0; c < 8; ++c) {
+  for (int c = 0; c < CH; ++c) {
 #pragma unroll
     for (int j = 0; j < W; ++j) { wt[j][c] = bf16_to_f32(w[(size_t)(d0 + c) * W + j]); dwin[j][c] = 0.f; }
 #pragma unroll
@@ -169,58 +230,81 @@ __global__ __launch_bounds__(256) void conv_norm_bwd_kernel(const ConvNormParams
     nw[c] = s.norm_weight ? ldf(s.norm_weight, p.norm_dtype, (d0 + c) % (8 * s.norm_lanes)) : 1.f;
   }
   const size_t base = (size_t)b * T * D + d0;
+  const int lanes = s.norm_lanes * (8 / CH), heads = groups / lanes, head = cg / lanes;
+  const float inv_n = s.norm_l2 ? 1.f : 1.f / (CH * lanes), eps = s.norm_eps;
 #pragma unroll
   for (int j = 0; j < W - 1; ++j) {
     const int q = t0 - (W - 1) + j;
     if (q >= 0) {
-      up8(*row8(s.x, base + (size_t)q * D), win[j]);
+      Pc::up(Pc::at(s.x, base + (size_t)q * D), win[j]);
     } else {
 #pragma unroll
-      for (int c = 0; c < 8; ++c) win[j][c] = st ? bf16_to_f32(st[((size_t)b * D + d0 + c) * W + (W + q)]) : 0.f;
+      for (int c = 0; c < CH; ++c) win[j][c] = st ? bf16_to_f32(st[((size_t)b * D + d0 + c) * W + (W + q)]) : 0.f;
     }
   }
+  struct Row { typename Pc::type x, a, b, n, add; float scale; };
+  const typename Pc::type zero = {};
+  // row t of every input (rows behind the end repeat the last one), and dx_add of the row that t completes
+  auto load = [&](const int t) __attribute__((always_inline)) -> Row {
+    const int tc = min(t, T - 1);
+    const size_t at = base + (size_t)tc * D;
+    Row q;
+    q.x = Pc::at(s.x, at);
+    q.a = s.dy_a ? Pc::at(s.dy_a, at) : zero;
+    q.b = s.dy_b ? Pc::at(s.dy_b, at) : zero;
+    q.n = s.dy_norm ? Pc::at(s.dy_norm, at) : zero;
+    q.add = s.dx_add ? Pc::at(s.dx_add, base + (size_t)max(t - (W - 1), t0) * D) : zero;
+    q.scale = s.scale ? s.scale[((size_t)b * T + tc) * heads + head] : 0.f;
+    return q;
+  };
   // row t: its gradient at y, its sums (rows of the next run, t >= t1, have none), and dx of row t - (W-1)
-  auto one_row = [&](const u32x4 rx, const u32x4 ra, const u32x4 rb, const u32x4 rn, const int t, const bool own) __attribute__((always_inline)) {
-    float dp[8], g[8], g2[8], y[8], da[8];
-    up8(rx, win[W - 1]);
-    up8(ra, g);
-    up8(rb, g2);
+  auto one_row = [&](const Row& q, const int t, const bool own) __attribute__((always_inline)) {
+    float dp[CH], g[CH], g2[CH], y[CH], da[CH];
+    Pc::up(q.x, win[W - 1]);
+    Pc::up(q.a, g);
+    Pc::up(q.b, g2);
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
+    for (int c = 0; c < CH; ++c) {
       float acc = bs[c];
 #pragma unroll
       for (int j = 0; j < W; ++j) acc += wt[j][c] * win[j][c];
-      y[c] = acc;
-      da[c] = 1.f;
-      if (p.silu) {
-        const float sg = 1.f / (1.f + __expf(-acc));
+      if constexpr (SILU) {
+        const float sg = sigmoid_fast(acc);
         y[c] = acc * sg;
         da[c] = sg * (1.f + acc * (1.f - sg));
+      } else {
+        y[c] = acc;
+        da[c] = 1.f;
       }
       g[c] += g2[c];
     }
     if (s.dy_norm) {
-      float dn[8], ss = 0.f, an = 0.f;
-      up8(down8(y), y);                                 // the rounded activation, as the forward normalised it
-      up8(rn, dn);
+      float dn[CH], ss = 0.f, an = 0.f;
+      Pc::up(Pc::down(y), y);                                 // the rounded activation, as the forward normalised it
+      Pc::up(q.n, dn);
 #pragma unroll
-      for (int c = 0; c < 8; ++c) {
+      for (int c = 0; c < CH; ++c) {
         ss += y[c] * y[c];
         an += dn[c] * nw[c] * y[c];
       }
-      group_sum2(ss, an, s.norm_lanes);
-      const float inv_n = s.norm_l2 ? 1.f : 1.f / (8 * s.norm_lanes);
-      const float rs = rsqrtf(ss * inv_n + s.norm_eps);
-      const float m = an * rs * inv_n;                  // mean (sum) of a n
+      group_sum2(ss, an, lanes);
+      if (s.scale) {                                    // y times its head's number: an is that number's gradient
+        if (s.dscale && own && cg == head * lanes) s.dscale[((size_t)b * T + t) * heads + head] = an;
 #pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        const float n = y[c] * rs;
-        g[c] += rs * (dn[c] * nw[c] - n * m);
-        if (own) dws[W + 1][c] += dn[c] * n;
+        for (int c = 0; c < CH; ++c) g[c] += q.scale * dn[c];
+      } else {
+        const float rs = rsqrtf(ss * inv_n + eps);
+        const float m = an * rs * inv_n;                // mean (sum) of a n
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+          const float n = y[c] * rs;
+          g[c] += rs * (dn[c] * nw[c] - n * m);
+          if (own) dws[W + 1][c] += dn[c] * n;
+        }
       }
     }
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
+    for (int c = 0; c < CH; ++c) {
       dp[c] = own || t < T ? g[c] * da[c] : 0.f;
       if (own) {
 #pragma unroll
@@ -231,51 +315,35 @@ __global__ __launch_bounds__(256) void conv_norm_bwd_kernel(const ConvNormParams
     }
     const int sx = t - (W - 1);
     if (sx >= t0) {
-      float o[8];
-      const size_t at = base + (size_t)sx * D;
-      if (s.dx_add) {
-        up8(*row8(s.dx_add, at), o);
-      } else {
+      float o[CH];
+      Pc::up(q.add, o);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) o[c] = 0.f;
-      }
-#pragma unroll
-      for (int c = 0; c < 8; ++c)
+      for (int c = 0; c < CH; ++c)
 #pragma unroll
         for (int i = 0; i < W; ++i) o[c] += wt[W - 1 - i][c] * dwin[i][c];
-      *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(s.dx) + at) = down8(o);
+      *reinterpret_cast<typename Pc::type*>(reinterpret_cast<bf16_t*>(s.dx) + base + (size_t)sx * D) = Pc::down(o);
     }
 #pragma unroll
     for (int j = 0; j < W - 1; ++j)
 #pragma unroll
-      for (int c = 0; c < 8; ++c) { win[j][c] = win[j + 1][c]; dwin[j][c] = dwin[j + 1][c]; }
+      for (int c = 0; c < CH; ++c) { win[j][c] = win[j + 1][c]; dwin[j][c] = dwin[j + 1][c]; }
   };
-  constexpr int AHEAD = 2;
-  const u32x4 zero = {0u, 0u, 0u, 0u};
+  constexpr int AHEAD = CH == 4 ? 3 : 1;   // (three replace the whole window: no moves; eight channels leave room for one)
   int tb = t0;
   for (; tb + AHEAD <= t1; tb += AHEAD) {
-    u32x4 rx[AHEAD], ra[AHEAD], rb[AHEAD], rn[AHEAD];
+    Row q[AHEAD];
 #pragma unroll
-    for (int a = 0; a < AHEAD; ++a) {
-      const size_t at = base + (size_t)(tb + a) * D;
-      rx[a] = *row8(s.x, at);
-      ra[a] = s.dy_a ? *row8(s.dy_a, at) : zero;
-      rb[a] = s.dy_b ? *row8(s.dy_b, at) : zero;
-      rn[a] = s.dy_norm ? *row8(s.dy_norm, at) : zero;
-    }
+    for (int a = 0; a < AHEAD; ++a) q[a] = load(tb + a);
 #pragma unroll
-    for (int a = 0; a < AHEAD; ++a) one_row(rx[a], ra[a], rb[a], rn[a], tb + a, true);
+    for (int a = 0; a < AHEAD; ++a) one_row(q[a], tb + a, true);
   }
 #pragma unroll 1
-  for (; tb < t1 + W - 1; ++tb) {                         // the run's odd row, and the W-1 rows behind it that its dx needs
-    const size_t at = base + (size_t)min(tb, T - 1) * D;
-    one_row(*row8(s.x, at), s.dy_a ? *row8(s.dy_a, at) : zero, s.dy_b ? *row8(s.dy_b, at) : zero, s.dy_norm ? *row8(s.dy_norm, at) : zero, tb, tb < t1);
-  }
+  for (; tb < t1 + W - 1; ++tb) one_row(load(tb), tb, tb < t1);   // the run's odd row, and the W-1 rows behind it that its dx needs
   float* pr = p.part[si] + ((size_t)(b * runs + r) * (W + 2)) * D + d0;
 #pragma unroll
   for (int j = 0; j < W + 2; ++j) {
-    *reinterpret_cast<f32x4*>(pr + (size_t)j * D) = (f32x4){dws[j][0], dws[j][1], dws[j][2], dws[j][3]};
-    *reinterpret_cast<f32x4*>(pr + (size_t)j * D + 4) = (f32x4){dws[j][4], dws[j][5], dws[j][6], dws[j][7]};
+#pragma unroll
+    for (int c = 0; c < CH; c += 4) *reinterpret_cast<f32x4*>(pr + (size_t)j * D + c) = (f32x4){dws[j][c], dws[j][c + 1], dws[j][c + 2], dws[j][c + 3]};
   }
 }
 
@@ -519,8 +587,8 @@ static int conv_cus() {
 // Tokens per thread: long runs read the fewest rows twice (and leave the fewest partial sums), but what counts first is that the
 // workgroups fill whole rounds of the chip -- registers admit three of them on a CU forward, two backward
 // (340M geometry, 8 x 4096: backward with runs of 64 in 1.5 rounds 233 us, of 98 in one 208; forward 32 -> 64 tokens 100 -> 94).
-static int conv_run(int B, int T, int W, int groups, bool bwd) {
-  const long long slots = (long long)conv_cus() * (bwd ? 2 : 3);
+static int conv_run(int B, int T, int W, int groups, bool bwd, int ch) {
+  const long long slots = (long long)conv_cus() * (bwd && ch == 8 ? 2 : 3);
   int best = 8;
   double best_cost = 1e300;
   for (int run = 8; run <= (bwd ? 128 : 64); run += bwd ? 2 : 8) {
@@ -536,6 +604,7 @@ static int conv_plan(ConvNormParams& p, const natsl_conv_seg* seg, int n_seg, in
   if (B <= 0 || T <= 0) return fail(NATSL_ERR_INVALID, "%s: non-positive dimension", what);
   if (W < 2 || W > 4) return fail(NATSL_ERR_UNSUPPORTED, "%s: kernel size %d not built (2, 3, 4)", what, W);
   long long all = 0;
+  bool wide = false;                           // (heads of 512 need eight channels a lane to fit a wave)
   for (int i = 0; i < n_seg; ++i) {
     const natsl_conv_seg& s = seg[i];
     if (s.D <= 0 || s.D % 8) return fail(NATSL_ERR_UNSUPPORTED, "%s: D=%d must be a positive multiple of 8", what, s.D);
@@ -543,12 +612,14 @@ static int conv_plan(ConvNormParams& p, const natsl_conv_seg* seg, int n_seg, in
     if (s.y_norm || s.dy_norm) {
       const int l = s.norm_lanes;
       if (l <= 0 || l > 64 || (l & (l - 1)) || (s.D / 8) % l) return fail(NATSL_ERR_UNSUPPORTED, "%s: norm width %d", what, 8 * l);
+      wide |= l == 64;
       if (bwd && s.norm_weight && !s.dnorm_weight) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
+      if (s.scale && s.norm_weight) return fail(NATSL_ERR_INVALID, "%s: a norm or a number", what);
     }
     all += s.D;
   }
-  const int run = conv_run(B, T, W, all / 8, bwd);
-  p.n_seg = n_seg; p.B = B; p.T = T; p.run = run; p.silu = silu; p.norm_dtype = norm_dtype;
+  const int ch = bwd && !wide ? 4 : 8, run = conv_run(B, T, W, all / ch, bwd, ch);
+  p.ch = ch; p.n_seg = n_seg; p.B = B; p.T = T; p.run = run; p.silu = silu; p.norm_dtype = norm_dtype;
   long long wgs = 0;
   for (int i = 0; i < NATSL_CONV_SEGS; ++i) {
     p.part[i] = nullptr;
@@ -556,7 +627,7 @@ static int conv_plan(ConvNormParams& p, const natsl_conv_seg* seg, int n_seg, in
     if (i >= n_seg) continue;
     p.seg[i] = seg[i];
     if (!p.seg[i].y_norm && !p.seg[i].dy_norm) p.seg[i].norm_lanes = 1;
-    wgs += ((long long)B * cdiv(T, run) * (seg[i].D / 8) + 255) / 256;
+    wgs += ((long long)B * cdiv(T, run) * (seg[i].D / ch) + 255) / 256;
     if (wgs > 0x7fffffffll) return fail(NATSL_ERR_UNSUPPORTED, "%s: problem too large", what);
   }
   p.first[NATSL_CONV_SEGS] = (int)wgs;
@@ -630,9 +701,19 @@ extern "C" int natsl_conv_norm_bwd(const natsl_conv_seg* seg, int n_seg, int B, 
   }
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)p.first[NATSL_CONV_SEGS]);
-  if (W == 4) hipLaunchKernelGGL((conv_norm_bwd_kernel<4>), grid, dim3(256), 0, s, p);
-  else if (W == 3) hipLaunchKernelGGL((conv_norm_bwd_kernel<3>), grid, dim3(256), 0, s, p);
-  else hipLaunchKernelGGL((conv_norm_bwd_kernel<2>), grid, dim3(256), 0, s, p);
+  auto launch = [&](auto w_c) {
+    constexpr int WC = decltype(w_c)::value;
+    if (p.ch == 4) {
+      if (activation) hipLaunchKernelGGL((conv_norm_bwd_kernel<WC, true, 4>), grid, dim3(256), 0, s, p);
+      else hipLaunchKernelGGL((conv_norm_bwd_kernel<WC, false, 4>), grid, dim3(256), 0, s, p);
+    } else {
+      if (activation) hipLaunchKernelGGL((conv_norm_bwd_kernel<WC, true, 8>), grid, dim3(256), 0, s, p);
+      else hipLaunchKernelGGL((conv_norm_bwd_kernel<WC, false, 8>), grid, dim3(256), 0, s, p);
+    }
+  };
+  if (W == 4) launch(std::integral_constant<int, 4>{});
+  else if (W == 3) launch(std::integral_constant<int, 3>{});
+  else launch(std::integral_constant<int, 2>{});
   if ((rc = check_launch(what)) != NATSL_OK) return rc;
   hipLaunchKernelGGL(conv_norm_reduce_kernel, dim3((unsigned)wgs), dim3(1024), 0, s, r);
   if ((rc = check_launch(what)) != NATSL_OK || !norms) return rc;

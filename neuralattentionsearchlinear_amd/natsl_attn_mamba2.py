@@ -198,14 +198,16 @@ class NeuralAttentionSearchLinearAttnMamba(nn.Module):
             types, n_nats_blocks, attn_fraction, raw_types = fast.select(logits, bool(use_cache) or cache is not None)
             if cache is not None:
                 cache.foresee(raw_types, q_len)
-            _, _, v, q, k, o_mix, q_attn, k_attn, v_attn, new_conv_states = fast.conv_norm(q, k, v, conv_states, bool(use_cache))
+            _, _, v, q, k, o_mix, q_attn, k_attn, v_attn, new_conv_states = fast.conv_norm(q, k, v, conv_states, bool(use_cache),
+                                                                                           dt if fast.takes_dt else None)
             q, k = (x.unflatten(-1, (-1, self.head_k_dim)) for x in (q, k))
             v = v.unflatten(-1, (-1, self.head_v_dim))
             q_attn, k_attn = (x.unflatten(-1, (-1, self.head_attn_k_dim)) for x in (q_attn, k_attn))
             v_attn = v_attn.unflatten(-1, (-1, self.head_attn_v_dim))
             if self.attn_qk_norm:
                 q_attn, k_attn = self.q_norm(q_attn), self.k_norm(k_attn)
-            v = (v * dt.unsqueeze(-1)).to(v.dtype)             # the attention view keeps the un-scaled v (:391-393, :473)
+            if not fast.takes_dt:
+                v = (v * dt.unsqueeze(-1)).to(v.dtype)         # the attention view keeps the un-scaled v (:391-393, :473)
         else:
             q, k, v, q_attn, k_attn, v_attn, o_mix, g, raw_types, new_conv_states = self._general_front(
                 hidden_states, selector_input, conv_states, use_cache, cu_seqlens)

@@ -397,3 +397,49 @@ def test_narrow_weight_gradient(rows, D, N):
     assert L.natsl_narrow_wgrad(P(dy), P(x), P(dw), rows, D, 65, _capi.stream_ptr(x.device)) != 0
     many = torch.randn(2049, N, device=DEV).bfloat16(), torch.randn(2049, D, device=DEV).bfloat16()
     assert torch.equal(_front._narrow_wgrad(*many), torch.mm(many[0].t(), many[1]))
+
+
+@pytest.mark.parametrize("width", [8, 16, 32, 64, 128, 256, 512])
+@pytest.mark.parametrize("what,silu,T", [('rms', 1, 37), ('l2', 0, 9), ('number', 1, 130)])
+def test_convolution_with_heads_of_any_width(width, what, silu, T):
+    """natsl_conv_norm_* for every head width (lanes of a head within a row of 16 lanes, across rows, a whole wave; four and eight channels a
+    thread) and for each of what follows the convolution, against float64 autograd."""
+    from neuralattentionsearchlinear_amd import _capi
+    from neuralattentionsearchlinear_amd._front import _ConvSeg
+    torch.manual_seed(width + T)
+    L, B, D, W = _capi.lib(), 2, 2 * max(width, 48) // width * width, 3
+    bf = lambda *s: torch.randn(*s, device=DEV).bfloat16()
+    x, w, bias, nw, dy, dn, add = bf(B, T, D), bf(D, 1, W), bf(D), bf(width), bf(B, T, D), bf(B, T, D), bf(B, T, D)
+    num = torch.rand(B, T, D // width, device=DEV)
+    y, yn, dx = (torch.empty_like(x) for _ in range(3))
+    dw, db, dnw, dnum = torch.empty_like(w), torch.empty_like(bias), torch.empty_like(nw), torch.empty_like(num)
+    seg = (_ConvSeg * 1)()
+    s = seg[0]
+    for n, t in dict(x=x, weight=w, bias=bias, y=y, y_norm=yn, dy_a=dy, dy_norm=dn, dx_add=add, dx=dx, dweight=dw, dbias=db).items():
+        setattr(s, n, t.data_ptr())
+    s.D, s.norm_lanes, s.norm_l2, s.norm_eps = D, width // 8, int(what == 'l2'), 1e-5
+    if what == 'rms':
+        s.norm_weight, s.dnorm_weight = nw.data_ptr(), dnw.data_ptr()
+    if what == 'number':
+        s.scale, s.dscale = num.data_ptr(), dnum.data_ptr()
+    st = _capi.stream_ptr(x.device)
+    _capi.check(L.natsl_conv_norm_fwd(seg, 1, B, T, W, silu, _capi.BF16, st), "natsl_conv_norm_fwd")
+    n = L.natsl_conv_norm_bwd_workspace_bytes(seg, 1, B, T, W)
+    ws = torch.empty(n, dtype=torch.uint8, device=DEV)
+    _capi.check(L.natsl_conv_norm_bwd(seg, 1, B, T, W, silu, _capi.BF16, ws.data_ptr(), n, st), "natsl_conv_norm_bwd")
+    x6, w6, b6, nw6, num6 = (t.detach().double().requires_grad_(True) for t in (x, w, bias, nw, num))
+    c = torch.nn.functional.conv1d(torch.nn.functional.pad(x6.transpose(1, 2), (W - 1, 0)), w6, b6, groups=D).transpose(1, 2)
+    c = torch.nn.functional.silu(c) if silu else c
+    r = c + (c.detach().bfloat16().double() - c.detach())                  # (what follows reads the rounded activation)
+    h = r.view(B, T, -1, width)
+    if what == 'rms':
+        o = h * torch.rsqrt((h * h).mean(-1, keepdim=True) + 1e-5) * nw6
+    elif what == 'l2':
+        o = h * torch.rsqrt((h * h).sum(-1, keepdim=True) + 1e-5)
+    else:
+        o = h * num6.unsqueeze(-1)
+    torch.autograd.backward([c, o.reshape(B, T, D)], [dy.double(), dn.double()])
+    # one rounding to bf16 of each result: 2^-9 relative, 2^-8 in the norm with the few activations that fp32 rounds the other way
+    for name, got, ref in [('y', y, c), ('follows', yn, o.reshape(B, T, D)), ('dx', dx, x6.grad + add.double()), ('dw', dw, w6.grad), ('db', db, b6.grad)] + \
+            ([('dnw', dnw, nw6.grad)] if what == 'rms' else [('dnum', dnum, num6.grad)] if what == 'number' else []):
+        assert rel_l2(got.double(), ref.detach()) <= 2 ** -8, (name, rel_l2(got.double(), ref.detach()))

@@ -560,6 +560,8 @@ typedef struct natsl_mixed {
   natsl_cast cast_in[NATSL_MIXED_CASTS], cast_out[NATSL_MIXED_CASTS];
 } natsl_mixed;
 size_t natsl_mixed_workspace_bytes(int64_t total_chunks, int H);
+/* `to` waits for what `from` holds so far (two streams of one device). */
+int natsl_order_streams(natsl_stream_t from, natsl_stream_t to);
 int natsl_mixed_softmax_variant(int B, int T, int HQ, int HKV, int block, int packed);   /* natsl_softmax_fwd_variant of its softmax branch */
 int natsl_mixed_fwd(const natsl_mixed* m, int phases, natsl_stream_t stream, natsl_stream_t attn_stream);
 

@@ -1,6 +1,6 @@
 """Builds csrc/*.hip into csrc/libnatsl.so for gfx950 with hipcc (cross-compiles without a GPU), and the benchmark's
 clock probe (csrc/bench/) into csrc/libnatsl_bench.so, which is not part of the C ABI; and the layers' native host side
-(csrc/host/step_core.cpp, a Python module that sees torch's tensors) into _step_core.so."""
+(csrc/host/, a Python module that sees torch's tensors) into _step_core.so."""
 from __future__ import annotations
 
 import os
@@ -33,13 +33,13 @@ def _hipcc() -> str:
 def _build_step_core():
     import torch
     from torch.utils.cpp_extension import include_paths
-    src = os.path.join(CSRC, "host", "step_core.cpp")
+    srcs = [os.path.join(CSRC, "host", f) for f in ("step_core.cpp", "layer_core.cpp")]
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-fPIC", "-shared", "-std=c++17", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           *(f"-I{d}" for d in (sysconfig.get_paths()["include"], *include_paths())), src, "-o", STEP_CORE,
+           *(f"-I{d}" for d in (sysconfig.get_paths()["include"], *include_paths())), *srcs, "-o", STEP_CORE,
            "-L" + os.path.join(os.path.dirname(torch.__file__), "lib"), "-lc10", "-ltorch_cpu", "-ltorch_python"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
-        raise RuntimeError(f"compiling {src} failed:\n{r.stderr}")
+        raise RuntimeError(f"compiling {srcs} failed:\n{r.stderr}")
 
 
 def build(verbose: bool = False) -> str:

@@ -107,6 +107,7 @@ _SIGNATURES = {
     "natsl_wgrad": (c_int, [c_void_p, c_int, c_void_p, c_int64, c_int, c_int, c_void_p, c_size_t, c_void_p]),
     "natsl_mixed_softmax_variant": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "natsl_mixed_workspace_bytes": (c_size_t, [c_int64, c_int]),
+    "natsl_order_streams": (c_int, [c_void_p, c_void_p]),
     "natsl_mixed_fwd": (c_int, [c_void_p, c_int, c_void_p, c_void_p]),
     "natsl_layer_step_workspace_bytes": (c_size_t, [c_void_p]),
     "natsl_layer_step_fwd": (c_int, [c_void_p, c_void_p, c_size_t, c_void_p]),

@@ -14,8 +14,8 @@ import functools
 import torch
 import torch.nn.functional as F
 
-from . import _capi
-from ._layer_step import _PARAMS, watch, weight_shapes
+from . import _capi, _mixed_common
+from ._layer_step import _PARAMS, _PLAIN_TENSORS, watch, weight_shapes
 from .modules import _NORM_GATE_WIDTHS
 
 _NAMES = [p[0] for p in _PARAMS]
@@ -516,12 +516,101 @@ class _Select(torch.autograd.Function):
         return out, None
 
 
+# ---- a layer as one call each way -------------------------------------------------------------------------------------------------------
+class _Layer(torch.autograd.Function):
+    """A layer's training forward and its backward, one native call each (csrc/host/layer_core.cpp): what FastFront's steps and the mixed operator's
+    autograd function launch, in that order, without an autograd node, a Python call and an allocation for each."""
+
+    @staticmethod
+    def forward(ctx, f, flags, x, *weights):
+        side, joint, states = flags
+        out, fraction, kept = _capi.step_core().layer_train(f.native, x, weights, _capi.stream_ptr(x.device), side, joint, True, states)
+        ctx.native, ctx.how = f.native, f.how
+        ctx.save_for_backward(x, *weights, *kept)
+        ctx.mark_non_differentiable(fraction)
+        ctx.set_materialize_grads(False)
+        return out, fraction
+
+    @staticmethod
+    def backward(ctx, dout, _):
+        if dout is None:
+            return (None,) * len(ctx.needs_input_grad)
+        saved, n = ctx.saved_tensors, 1 + len(_NAMES) + 1
+        x, weights, kept = saved[0], saved[1:n], saved[n:]
+        w_mix = weights[_NAMES.index("w_mix")]
+        stream = _capi.stream_ptr(x.device)
+        grads = _capi.step_core().layer_backward(
+            ctx.native, dout.to(x.dtype), x, weights, kept, ctx.needs_input_grad[2:], stream, _beside(x, ctx.how, stream), ctx.how["invalid_attn"],
+            ctx.how["invalid_linear"], _narrow_pays(x.shape[0] * x.shape[1], *w_mix.shape))
+        return (None, None, *grads)
+
+
+def _beside(x, how, stream):
+    """The stream of the softmax branch: the side stream, or the caller's."""
+    B, T = x.shape[:2]
+    if _mixed_common._run_side_by_side(x.device, False, B, B, T, how["H"], how["K"], how["V"]):
+        return _mixed_common._get_attn_stream(x.device).cuda_stream
+    return stream
+
+
+def _native_plan(layer, kind, constants, w, wn):
+    """(what csrc/host/layer_core.cpp keeps of a layer, the sizes used here), or None where it is not built for the layer."""
+    delta, dev = constants["delta"], w["wq"].device
+    H, K, V, HQ = layer.num_heads, layer.head_k_dim, layer.head_v_dim, layer.num_attn_heads
+    KA, VA, HN, D = layer.head_attn_k_dim, layer.head_attn_v_dim, layer.num_nats_head, layer.hidden_size
+    if layer.nats_block_size != 64 or D % 32 or (1 + delta) * H > 32 or K not in (64, 128, 192) or V % 64 or KA not in (64, 128) or VA not in (64, 128) or \
+            HQ * KA != H * K or HQ * VA != H * V or HQ % HN or H % HN or not (delta or constants["takes_dt"] and not layer.attn_qk_norm):
+        return None
+    if not _on_16(*[t for t in w.values() if t is not None]):
+        return None
+    ops = layer.ops_for_incomplete_chunks
+    decay = layer.decay_for_non_gdn_blocks if delta else layer.decay_for_non_mamba_blocks
+    if ops not in ('all', 'attn', 'gated_delta_net' if delta else 'mamba'):
+        return None
+    L, c = _capi.lib(), constants
+    core = _capi.step_core().make_layer(
+        L._handle, _capi.check,
+        (dev.index, int(delta), D, H, K, V, HQ, KA, VA, HN, wn.shape[0], c["W"], c["act"], c["norm_width"], c["norm_dtype"], c["gate_dtype"], c["out_dtype"],
+         c["neg"], int(decay), int(ops in ('all', 'attn')), int(ops != 'attn')),
+        (c["front_eps"], c["out_eps"], KA ** -0.5, K ** -0.5 if delta else 1.0))
+    return core, dict(H=H, K=K, V=V, widths=(w["wq"].shape[0], w["wk"].shape[0], w["wv"].shape[0], w["wg"].shape[0]), D=D,
+                      cus=torch.cuda.get_device_properties(dev).multi_processor_count)
+
+
 class FastFront:
     """A layer's parameters at one forward, with the constants of its plan.  (The plan, which outlives the forward, holds no tensor.)"""
 
     def __init__(self, constants, w, wn):
         self.__dict__.update(constants)
-        self.w, self.wn = w, wn
+        self.w, self.wn, self.native = w, wn, None
+
+    def _call(self, x):
+        """-> (stream, the softmax branch's stream, whether the wide projections are one launch)."""
+        how, rows = self.how, x.shape[0] * x.shape[1]
+        stream = _capi.stream_ptr(x.device)
+        return stream, _beside(x, how, stream), _joint_pays(rows, how["D"], how["widths"], how["cus"])
+
+    def train(self, x):
+        """The layer's training forward on whole sequences (`native` only) -> (output, attention's share per head)."""
+        weights = (*self.w.values(), self.wn)
+        stream, side, joint = self._call(x)
+        if self.grad(x, *weights):
+            how = self.how
+            states = _mixed_common._keep_states_of(x.shape[0], x.shape[0], x.shape[1], how["H"], how["K"], how["V"])
+            return _Layer.apply(self, (side, joint, states), x, *weights)
+        return _capi.step_core().layer_train(self.native, x, weights, stream, side, joint, False, False)[:2]
+
+    def prompt(self, x, seen):
+        """The layer's forward outside of training (`native` only, no gradients).  seen: None, or a call that gets the blocks' types as soon as they are
+        enqueued -> (output, attention's share per head, None or what a cache keeps: types before the last block was forced, (k, v) of attention,
+        (k, v, beta, g) of the linear branch, convolution states, final state, the state that entered the last block, sum of g over it)."""
+        weights, core = (*self.w.values(), self.wn), _capi.step_core()
+        stream, side, joint = self._call(x)
+        front = core.layer_front(self.native, x, weights, stream)
+        if seen is not None:
+            seen(front[5])
+        out, ka, va, kl, vl, cq, ck, cv, ht, hs, gs = core.layer_rest(self.native, x, weights, front, stream, side, joint, seen is not None)
+        return out, front[7], None if seen is None else (front[5], (ka, va), (kl, vl, front[1], front[0]), (cq, ck, cv), ht, hs, gs)
 
     def grad(self, *tensors):
         return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
@@ -612,7 +701,7 @@ def _selector_weight(layer, like):
     if type(m) is not torch.nn.Linear or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__:
         return None
     w = m._parameters.get("weight")
-    if m._parameters.get("bias") is not None or type(w) is not torch.nn.Parameter or w.dtype != torch.bfloat16 or not w.is_contiguous() or \
+    if m._parameters.get("bias") is not None or w is None or type(w) not in _PLAIN_TENSORS or w.dtype != torch.bfloat16 or not w.is_contiguous() or \
             w.device != like.device or w.dim() != 2 or w.shape[1] != like.shape[1] or w.shape[0] != layer.num_nats_head * layer.n_ops or w.shape[0] > 64:
         return None
     return w
@@ -633,6 +722,14 @@ def fast_front(layer, kind, x, cache, cu_seqlens):
     if constants is None or w["wq"].device != x.device:
         return None
     f = FastFront(constants, w, _selector_weight(layer, w["wa"]))
+    if f.wn is not None and seen.native_plan is None:
+        seen.native_plan = (_native_plan(layer, kind, constants, w, f.wn),)
+    if f.wn is not None and seen.native_plan[0] is not None and layer.incomplete_block_start_with_ht and _mixed_common.TIMING_HOOK is None and \
+            x.device.index == torch.cuda.current_device() and x.dim() == 3 and x.shape[2] == layer.hidden_size and _on_16(x, f.wn):
+        f.native, how = seen.native_plan[0]
+        # (the Mamba layer calls its operator with that operator's defaults)
+        f.how = dict(how, invalid_attn=kind == 'gdn' and bool(layer.compute_dnats_for_invalid_blocks_attn),
+                     invalid_linear=kind != 'gdn' or bool(layer.compute_dnats_for_invalid_blocks_linear_att))
     if cache is not None:
         if torch.is_grad_enabled() and (x.requires_grad or any(t is not None and t.requires_grad for t in w.values())):
             return None

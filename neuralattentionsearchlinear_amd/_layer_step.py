@@ -97,7 +97,7 @@ class _Watch:
         self.plain &= {*map(type, weights)} <= _PLAIN_TENSORS
         self.core = _capi.step_core().make_watch(parts, [*layer._parameters], absent, options, [layer.__dict__[o] for o in options],
                                                  weights) if self.plain else None
-        self.step_plan = self.front_plan = None
+        self.step_plan = self.front_plan = self.native_plan = None
 
     def weights(self, layer):
         """The weights by field, None where the layer has none."""

@@ -83,11 +83,13 @@ def _run_side_by_side(dev, packed: bool, n_seqs: int, B: int, T: int, H: int, K:
 
 def _keep_chunk_states(q, v, cu_seqlens) -> bool:
     """Whether the differentiable forward keeps the linear branch's chunk states (see SAVE_CHUNK_STATES)."""
+    B, T, H, K = q.shape
+    return _keep_states_of(B if cu_seqlens is None else len(cu_seqlens) - 1, B, T, H, K, v.shape[-1])                     # (a host list here)
+
+
+def _keep_states_of(n_seq, B, T, H, K, V) -> bool:
     if SAVE_CHUNK_STATES is not None:
         return bool(SAVE_CHUNK_STATES)
-    B, T, H, K = q.shape
-    V = v.shape[-1]
-    n_seq = B if cu_seqlens is None else len(cu_seqlens) - 1                     # (a host list here)
     chunks = -(-B * T // CHUNK_SIZE) + n_seq                       # upper bound on the chunks of all sequences
     return chunks * H * (2 * K * V + 2 * CHUNK_SIZE * V + _PREP_WORKSPACE_BYTES) <= SAVE_CHUNK_STATES_MAX_BYTES
 
@@ -154,6 +156,25 @@ def linear_chunk_fwd(kind: str, q, k, v, g, beta, h0, types, scale: float, block
     if chunk_states:
         return o, ht, sc, (vn if kind == 'gdn' else v), ws
     return o, ht
+
+
+def state_behind(ht, hs, gs, last):
+    """The state the next block starts from where the input ends on a block's end: the final state ht [N,H,K,V] where the last block's type (last [N,HN,2])
+    is linear, else the one that entered it, hs, decayed by gs [N,H], the sum of g over it (None: not decayed)."""
+    n, H, K, V = ht.shape
+    dev = ht.device
+    # (a launch goes to the current device, torch's operations to their tensors')
+    if last.is_cuda and last.device == dev and dev.index in (None, torch.cuda.current_device()) and \
+            last.dtype in (torch.bfloat16, torch.float32) and last.dim() == 3 and last.shape[0] == n and \
+            last.stride(2) == 1 and H % last.shape[1] == 0 and last.shape[2] > 1 and n * H <= 65535:
+        h_start = torch.empty_like(ht)
+        rc = _capi.lib().natsl_roll_state(ht.data_ptr(), hs.data_ptr(), _capi.ptr(gs), last.data_ptr(), _capi.dtype_code(last.dtype), last.stride(0),
+                                          last.stride(1), h_start.data_ptr(), n, H, last.shape[1], K * V, _capi.stream_ptr(dev))
+        _capi.check(rc, "natsl_roll_state")
+        return h_start
+    lin = (last[..., 1] > 0)
+    lin = lin.repeat_interleave(H // lin.shape[1], dim=1).view(n, H, 1, 1)
+    return torch.where(lin, ht, hs if gs is None else hs * torch.exp(gs).view(n, H, 1, 1))
 
 
 def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn, initial_state, g, beta, nats_block_types,
@@ -384,20 +405,7 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
         else:
             if op_type_last_chunk is None:
                 raise AssertionError("op_type_last_chunk is required when the input ends on a block boundary")
-            last, n = op_type_last_chunk, ht.shape[0]
-            # (a launch goes to the current device, torch's operations to their tensors')
-            if last.is_cuda and last.device == dev and dev.index in (None, torch.cuda.current_device()) and \
-                    last.dtype in (torch.bfloat16, torch.float32) and last.dim() == 3 and last.shape[0] == n and \
-                    last.stride(2) == 1 and H % last.shape[1] == 0 and last.shape[2] > 1 and n * H <= 65535:
-                h_start = torch.empty_like(ht)
-                rc = L.natsl_roll_state(ht.data_ptr(), hs.data_ptr(), gs.data_ptr() if decay_non_linear else None, last.data_ptr(),
-                                        _capi.dtype_code(last.dtype), last.stride(0), last.stride(1), h_start.data_ptr(), n, H, last.shape[1], K * V, cur)
-                _capi.check(rc, "natsl_roll_state")
-            else:
-                lin = (last[..., 1] > 0)
-                lin = lin.repeat_interleave(H // lin.shape[1], dim=1).view(n, H, 1, 1)
-                rolled = hs * torch.exp(gs).view(n, H, 1, 1) if decay_non_linear else hs
-                h_start = torch.where(lin, ht, rolled)
+            h_start = state_behind(ht, hs, gs if decay_non_linear else None, op_type_last_chunk)
     return o_lin, o_attn, ht, h_start
 
 

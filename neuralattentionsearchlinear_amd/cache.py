@@ -112,6 +112,11 @@ class NAtSLayerCache:
         self._pending_first = None                       # K/V of the first forward, kept until update() has the types
         self._foreseen = None                            # counts on their way to the host (foresee)
 
+    def is_empty(self) -> bool:
+        """Whether nothing of a forward has been kept (but the hidden states of the one that runs)."""
+        return self.n_observed_tokens == 0 and self._n_tokens_in_nats_block == 0 and self.attn_k is None and self.l_attn_k is None and \
+            self.conv_state is None and self.recurrent_state is None and self.recurrent_state_block_start is None and self.n_attn_blocks is None
+
     # ------------------------------------------------------------------------------------------------
     def update_attn_types(self, input_hidden_states: torch.Tensor) -> Optional[torch.Tensor]:
         """Collect the hidden states of the incomplete block; once the new tokens complete at least one block,

@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "../../../include/natsl.h"
+#include "layer_core.h"
 
 namespace {
 
@@ -378,12 +379,20 @@ PyObject* run(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+template <class F>
+PyCFunction fast(F f) { return reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)); }
+
 PyMethodDef methods[] = {
     {"make_watch", make_watch, METH_VARARGS, nullptr},
-    {"holds", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(holds)), METH_FASTCALL, nullptr},
+    {"holds", fast(holds), METH_FASTCALL, nullptr},
     {"make_step", make_step, METH_VARARGS, nullptr},
-    {"takes", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(takes)), METH_FASTCALL, nullptr},
-    {"run", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(run)), METH_FASTCALL, nullptr},
+    {"takes", fast(takes), METH_FASTCALL, nullptr},
+    {"run", fast(run), METH_FASTCALL, nullptr},
+    {"make_layer", natsl_make_layer, METH_VARARGS, nullptr},
+    {"layer_train", fast(natsl_layer_train), METH_FASTCALL, nullptr},
+    {"layer_backward", fast(natsl_layer_backward), METH_FASTCALL, nullptr},
+    {"layer_front", fast(natsl_layer_prompt_front), METH_FASTCALL, nullptr},
+    {"layer_rest", fast(natsl_layer_prompt_rest), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_step_core", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -183,6 +183,14 @@ extern "C" int natsl_linear_chunk_states(int is_delta, const void* q, const void
                     dtype, seqs, n_seqs, total_units, stream, other ? &side : nullptr);
 }
 
+extern "C" int natsl_order_streams(natsl_stream_t from, natsl_stream_t to) {
+  const char* what = "natsl_order_streams";
+  hipStream_t a = reinterpret_cast<hipStream_t>(from), b = reinterpret_cast<hipStream_t>(to);
+  OnDeviceOf device;
+  if (const int rc = device.enter(a, b, what)) return rc;
+  return order_streams(a, b, what);
+}
+
 extern "C" int natsl_seq_table(const natsl_seq_row* rows, int n, natsl_seq_row* table, natsl_stream_t stream) {
   const char* what = "natsl_seq_table";
   static_assert(sizeof(natsl_seq_row) == 32, "a row is two pieces of 16 bytes");

@@ -23,6 +23,7 @@ import torch.nn.functional as F
 from . import nats_util
 from ._front import fast_front
 from ._layer_step import layer_step
+from ._mixed_common import state_behind
 from .cache import NAtSCache, NAtSLayerCache
 from .mixed_attn_gdn import nats_mixed_attn_gdn, nats_mixed_attn_gdn_chunk_inference, nats_mixed_attn_gdn_recurrent
 from .modules import FusedMultiInputRMSNormGated, RMSNorm, ShortConvolution
@@ -176,6 +177,17 @@ class NeuralAttentionSearchLinearAttnGDN(nn.Module):
         g = -self.A_log.float().exp() * F.softplus(self.a_proj(hidden_states).float() + self.dt_bias)
         return q, k, v, q_attn, k_attn, v_attn, o_weights, g, beta, raw_types, tuple(new_conv_states) if self.use_short_conv else None
 
+    def _into_cache(self, cache, q_len, raw_types, attn_kv, lattn, conv_states, state, state_entering, g_sum):
+        """An empty cache after its first prompt (FastFront.prompt's outputs)."""
+        k, v, beta, g = lattn
+        cache.update_attn_cache(attn_kv, nats_block_types=raw_types)
+        cache.update_lattn_cache((k, v), beta, g, 'chunk', self.ops_for_incomplete_chunks)
+        if q_len % self.nats_block_size == 0:
+            state_entering = state_behind(state, state_entering, g_sum if self.decay_for_non_gdn_blocks else None, raw_types[:, -1])
+        self.last_recurrent_state, self.last_block_start_state = state, state_entering
+        cache.update(recurrent_state=state, recurrent_state_block_start=state_entering, attn_state=attn_kv, conv_state=conv_states,
+                     nats_block_types=raw_types, l_attn_state=(k, v), g=g, n_new_tokens=q_len)
+
     def forward(self, hidden_states: torch.Tensor, attention_mask: Optional[torch.Tensor] = None, past_key_values=None,
                 use_cache: Optional[bool] = False, output_attentions: Optional[bool] = False, **kwargs):
         if attention_mask is not None:
@@ -219,6 +231,18 @@ class NeuralAttentionSearchLinearAttnGDN(nn.Module):
         fast = None
         if mode == 'chunk' and selector_input is not None and getattr(self.select_ops, '__func__', None) is _SELECT_OPS:
             fast = fast_front(self, 'gdn', hidden_states, cache, cu_seqlens)
+        if fast is not None and fast.native is not None and (not use_cache if cache is None else use_cache and cache.is_empty()) and \
+                (nats_mixed_attn_gdn, nats_mixed_attn_gdn_chunk_inference) == _OPERATORS:
+            if self.training and cache is None:
+                o, self.attn_fraction = fast.train(hidden_states)
+                self.last_recurrent_state = self.last_block_start_state = None
+                return o, None, past_key_values
+            if not self.training and not fast.grad(hidden_states, *fast.w.values(), fast.wn):
+                o, self.attn_fraction, kept = fast.prompt(hidden_states, None if cache is None else lambda types: cache.foresee(types, q_len))
+                self.last_recurrent_state = self.last_block_start_state = None
+                if cache is not None:
+                    self._into_cache(cache, q_len, *kept)
+                return o, None, past_key_values
         types = n_nats_blocks = None
         conv_states = cache.conv_state if cache is not None and cache.conv_state is not None else (None, None, None)
         if fast is not None:
@@ -312,3 +336,5 @@ class NeuralAttentionSearchLinearAttnGDN(nn.Module):
 
 # the selector that the fused front contains; a layer whose select_ops is another one takes the general front, which calls it
 _SELECT_OPS = NeuralAttentionSearchLinearAttnGDN.select_ops
+# ... and the operators: where others stand in their places, those are called
+_OPERATORS = (nats_mixed_attn_gdn, nats_mixed_attn_gdn_chunk_inference)

@@ -16,6 +16,7 @@ import torch.nn.functional as F
 from . import nats_util
 from ._front import fast_front
 from ._layer_step import layer_step
+from ._mixed_common import state_behind
 from .cache import NAtSLayerCache
 from .mixed_attn_mamba import (nats_mixed_attn_mamba, nats_mixed_attn_mamba_chunk_inference,
                                nats_mixed_attn_mamba_recurrent)
@@ -149,6 +150,17 @@ class NeuralAttentionSearchLinearAttnMamba(nn.Module):
         g = -self.A_log.float().exp() * dt
         return q, k, v, q_attn, k_attn, v_attn, o_weights, g, raw_types, tuple(new_conv_states) if self.use_short_conv else None
 
+    def _into_cache(self, cache, q_len, raw_types, attn_kv, lattn, conv_states, state, state_entering, g_sum):
+        """An empty cache after its first prompt (FastFront.prompt's outputs)."""
+        k, v, beta, g = lattn
+        cache.update_attn_cache(attn_kv, nats_block_types=raw_types)
+        cache.update_lattn_cache((k, v), beta, g, 'chunk', self.ops_for_incomplete_chunks)
+        if q_len % self.nats_block_size == 0:
+            state_entering = state_behind(state, state_entering, g_sum if self.decay_for_non_mamba_blocks else None, raw_types[:, -1])
+        self.last_recurrent_state, self.last_block_start_state = state, state_entering
+        cache.update(recurrent_state=state, recurrent_state_block_start=state_entering, attn_state=attn_kv, conv_state=conv_states,
+                     nats_block_types=raw_types, l_attn_state=(k, v), g=g, n_new_tokens=q_len)
+
     def forward(self, hidden_states: torch.Tensor, attention_mask: Optional[torch.Tensor] = None, cache_params=None,
                 use_cache: Optional[bool] = False, output_attentions: Optional[bool] = False, **kwargs):
         if attention_mask is not None:
@@ -186,6 +198,18 @@ class NeuralAttentionSearchLinearAttnMamba(nn.Module):
         fast = None
         if mode == 'chunk' and selector_input is not None and getattr(self.select_ops, '__func__', None) is _SELECT_OPS:
             fast = fast_front(self, 'mamba', hidden_states, cache, cu_seqlens)
+        if fast is not None and fast.native is not None and (not use_cache if cache is None else use_cache and cache.is_empty()) and \
+                (nats_mixed_attn_mamba, nats_mixed_attn_mamba_chunk_inference) == _OPERATORS:
+            if self.training and cache is None:
+                o, self.attn_fraction = fast.train(hidden_states)
+                self.last_recurrent_state = self.last_block_start_state = None
+                return o
+            if not self.training and not fast.grad(hidden_states, *fast.w.values(), fast.wn):
+                o, self.attn_fraction, kept = fast.prompt(hidden_states, None if cache is None else lambda types: cache.foresee(types, q_len))
+                self.last_recurrent_state = self.last_block_start_state = None
+                if cache is not None:
+                    self._into_cache(cache, q_len, *kept)
+                return o
         types = n_nats_blocks = None
         conv_states = cache.conv_state if cache is not None and cache.conv_state is not None else (None, None, None)
         if fast is not None:
@@ -278,3 +302,5 @@ class NeuralAttentionSearchLinearAttnMamba(nn.Module):
 
 # the selector that the fused front contains; a layer whose select_ops is another one takes the general front, which calls it
 _SELECT_OPS = NeuralAttentionSearchLinearAttnMamba.select_ops
+# ... and the operators: where others stand in their places, those are called
+_OPERATORS = (nats_mixed_attn_mamba, nats_mixed_attn_mamba_chunk_inference)

@@ -443,3 +443,104 @@ def test_convolution_with_heads_of_any_width(width, what, silu, T):
     for name, got, ref in [('y', y, c), ('follows', yn, o.reshape(B, T, D)), ('dx', dx, x6.grad + add.double()), ('dw', dw, w6.grad), ('db', db, b6.grad)] + \
             ([('dnw', dnw, nw6.grad)] if what == 'rms' else [('dnum', dnum, num6.grad)] if what == 'number' else []):
         assert rel_l2(got.double(), ref.detach()) <= 2 ** -8, (name, rel_l2(got.double(), ref.detach()))
+
+
+def _stepwise(monkeypatch):
+    """The fused steps one by one instead of the native call."""
+    from neuralattentionsearchlinear_amd import _front
+    monkeypatch.setattr(_front, '_native_plan', lambda *a: None)
+
+
+def _train(layer, x0, do):
+    x = x0.clone().requires_grad_(True)
+    layer.zero_grad(set_to_none=True)
+    o = layer(x)
+    o = o[0] if isinstance(o, tuple) else o
+    o.backward(do)
+    return dict({n: p.grad for n, p in layer.named_parameters()}, x=x.grad, out=o.detach(), fraction=layer.attn_fraction)
+
+
+@pytest.mark.parametrize("kind,geometry,B,T,more", [
+    ('gdn', None, 1, 64, {}), ('gdn', '340M', 2, 2113, {}), ('gdn', '760M', 1, 200, dict(allow_neg_eigval=True, conv_bias=True)),
+    ('gdn', None, 3, 130, dict(conv_size=3, conv_activation=None, compute_dnats_for_invalid_blocks_attn=True, compute_dnats_for_invalid_blocks_linear_att=True)),
+    ('mamba', None, 2, 257, {}), ('mamba', None, 2, 4100, dict(conv_bias=True, conv_size=2))])
+@pytest.mark.parametrize("side,keep", [(False, False), (True, True), (True, False), (None, None)])
+def test_native_layer_is_its_steps(kind, geometry, B, T, more, side, keep, monkeypatch):
+    """A training step through the native call against the same launches one by one: the streams' and the kept states' switches, sequences that cut a block."""
+    from neuralattentionsearchlinear_amd import _front, _mixed_common
+    layer = _layer(kind, geometry, 'all', **more).train()
+    torch.manual_seed(T)
+    x, do = (torch.randn(B, T, layer.hidden_size, device=DEV).bfloat16() for _ in range(2))
+    calls, inner = [], _front._Layer.forward
+    monkeypatch.setattr(_front._Layer, 'forward', staticmethod(lambda *a: (calls.append(1), inner(*a))[1]))
+    monkeypatch.setattr(_mixed_common, 'CONCURRENT_BRANCHES', side)
+    monkeypatch.setattr(_mixed_common, 'SAVE_CHUNK_STATES', keep)
+    got = [_train(layer, x, do) for _ in range(2)]
+    assert calls == [1, 1]
+    other = _layer(kind, geometry, 'all', **more).train()
+    other.load_state_dict(layer.state_dict())
+    _stepwise(monkeypatch)
+    want = _train(other, x, do)
+    assert calls == [1, 1]
+    for g in got:
+        for n, b in want.items():
+            # the same kernels; the mixing logits' products may be others (a rounding of a bf16 value now and then), and the block types' gradient is
+            # summed by atomic additions
+            assert g[n].shape == b.shape and g[n].dtype == b.dtype and rel_l2(g[n].float(), b.float()) <= (2e-2 if n == 'nats_layer.weight' else 5e-3), n
+
+
+@pytest.mark.parametrize("kind", ['gdn', 'mamba'])
+def test_native_layer_under_autograd(kind):
+    """What autograd asks of the one node: gradients for what wants them only, saved tensors through hooks, a second backward, changed weights
+    refused, no graph where nothing wants a gradient."""
+    layer = _layer(kind, None, 'all').train()
+    torch.manual_seed(5)
+    x, do = (torch.randn(2, 150, layer.hidden_size, device=DEV).bfloat16() for _ in range(2))
+    out = lambda t: (lambda o: o[0] if isinstance(o, tuple) else o)(layer(t))
+    want = _train(layer, x, do)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.to(DEV)):
+        got = _train(layer, x, do)
+    for n, b in want.items():
+        assert rel_l2(got[n].float(), b.float()) <= (2e-2 if n == 'nats_layer.weight' else 1e-6), n
+    layer.zero_grad(set_to_none=True)
+    some = {'wo': layer.o_proj.weight, 'wa': layer.a_proj.weight, 'mix': layer.nats_out_weights_layer.weight}
+    for p in layer.parameters():
+        p.requires_grad_(any(p is s for s in some.values()))
+    o = out(x)
+    o.backward(do, retain_graph=True)
+    first = {n: p.grad.clone() for n, p in some.items()}
+    o.backward(do)
+    for n, p in layer.named_parameters():
+        assert (p.grad is not None) == p.requires_grad
+    for n, p in some.items():
+        assert rel_l2(p.grad.float(), 2 * first[n].float()) <= 1e-2
+    o = out(x)
+    with torch.no_grad():
+        layer.a_proj.weight.mul_(1.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        o.backward(do)
+    for p in layer.parameters():
+        p.requires_grad_(False)
+    assert not out(x).requires_grad
+    with torch.no_grad():
+        assert torch.equal(out(x), out(x))
+
+
+@pytest.mark.parametrize("kind,T0", [('gdn', 128), ('gdn', 777), ('mamba', 64), ('mamba', 2113)])
+@pytest.mark.parametrize("ops", ['all', 'attn'])
+def test_native_prompt_is_its_steps(kind, T0, ops, monkeypatch):
+    """A first prompt through the native calls against the same launches one by one: outputs, what the cache holds, and the tokens behind it."""
+    layer = _layer(kind, None, ops)
+    torch.manual_seed(T0)
+    x = torch.randn(2, T0 + 3, layer.hidden_size, device=DEV).bfloat16()
+    fast, cf = _generate(layer, kind, x, T0, (1, 2))
+    other = _layer(kind, None, ops)
+    other.load_state_dict(layer.state_dict())
+    _stepwise(monkeypatch)
+    slow, cs = _generate(other, kind, x, T0, (1, 2))
+    names = ['attn_k', 'attn_v', 'l_attn_k', 'l_attn_v', 'lattn_g', 'lattn_beta', 'recurrent_state', 'recurrent_state_block_start', 'g_cumsum', 'block_type_state']
+    for a, b in zip(fast + list(cf.conv_state) + [getattr(cf, n) for n in names], slow + list(cs.conv_state) + [getattr(cs, n) for n in names]):
+        assert (a is None) == (b is None) and (a is None or a.shape == b.shape and rel_l2(a.float(), b.float()) <= 2e-3)
+    for n in ('n_attn_blocks', 'valid_attn_tokens'):
+        assert torch.equal(getattr(cf, n), getattr(cs, n))
+    assert rel_l2(layer.last_recurrent_state, other.last_recurrent_state) <= 2e-3

@@ -408,8 +408,8 @@ NATSL_DEVICE void softmax_phase(f32x16& s0, f32x16& s1, f32x16 (&acc)[DV / 32], 
   }
 }
 
-// NWAVES waves of 32 queries: the workgroup owns QTILE = 32*NWAVES queries.
-template <int DK, int DV, int NWAVES>
+// NWAVES waves of 32 queries: the workgroup owns QTILE = 32*NWAVES queries.  OWN: see below (8 waves and selector blocks of 64 keys).
+template <int DK, int DV, int NWAVES, bool OWN>
 __global__ __launch_bounds__(64 * NWAVES, NWAVES == 4 ? 2 : 1) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
   constexpr int NTHREADS = 64 * NWAVES, QW = 32, QTILE = QW * NWAVES;  // QW = queries per wave
@@ -616,11 +616,19 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
       //  * V(c) lives in ring buffer c % 4, row-major as it comes.  The late waves request V(k+3) at the end of their body k,
       //    after sync(k): the buffer it overwrites, V(k-1), was last read before sync(k).  It must have landed when they arrive
       //    at sync(k+2): they too leave exactly the newest request in flight.
-      constexpr int RING = 4, KTILE = 64 * DK * 2, VTILE = 64 * DV * 2;   // bytes
+      // OWN, selector blocks of one chunk: the tile's own four chunks (n_diag of them) come before the loop, and the loop's chunks are the
+      // prior attention blocks'.  In the loop, one chunk at a time, up to six of the eight waves wait at the barrier while two work; here the
+      // four lie in LDS together, own chunk j in slot j of both rings, and every wave walks those its queries see by itself.  The one barrier
+      // among them, when everybody is done with chunk 0, is where chunks 1 to 3 must have landed, and slot 0 is free from there on: the loop's
+      // K(0) has a fifth slot (K's ring starts there), its K(1) and V(0) take slot 0.  The same chunks in the same order: the same bits.
+      // us, all in the loop / so, alone on the device: no attention blocks, 128/128, B4 T4096 H16 66 / 56, B32 T320 H16 56 / 43; half attention,
+      // B2 T3000 H18 64/128 81 / 76, B8 T2000 H16 128/64 120 / 118; one tile per CU, half attention, B2 T2048 H16 128/128 37.5 / 38.1.  Blocks of
+      // more than a chunk stay in the loop: their chunks from dstart on can be more than the slots.
+      constexpr int OWN_EARLY = 2, RING = 4, KTILE = 64 * DK * 2, VTILE = 64 * DV * 2;   // bytes
       constexpr int KI = DK / 32, VI = DV / 32;                           // DMA instructions per wave and chunk: early waves K, late waves V
       constexpr int KROWS_I = 512 / DK, VROWS_I = 512 / DV;               // tile rows one instruction covers
       // (the swizzled operand addresses are formed with XOR: the ring starts on a 1 KiB boundary)
-      const unsigned lds_k = ((unsigned)(size_t)smem + 1023u) & ~1023u, lds_v = lds_k + RING * KTILE;
+      const unsigned lds_k = ((unsigned)(size_t)smem + 1023u) & ~1023u, lds_v = lds_k + (RING + OWN) * KTILE;
       const bool late = wave >= 4;
       const int gw = wave & 3;  // wave within its group
       // --- lane l of instruction i fills LDS row rows_per_instr*i + l/segs, position l%segs, with the segment that belongs there
@@ -639,30 +647,39 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
           src[j] = (unsigned)((size_t)r * vrow * sizeof(bf16_t)) + 16u * ((unsigned)pos ^ v_swizzle<DV>(r));
         }
       }
-      auto dma_v = [&](const int ks, const int c) __attribute__((always_inline)) {
+      auto k_slot = [](const int c) __attribute__((always_inline)) -> int { return !OWN ? c & 3 : (c & 3) ? (c & 3) - 1 : RING; };
+      auto dma_v = [&](const int ks, const int sl) __attribute__((always_inline)) {
         const char* g = reinterpret_cast<const char*>(vp + (size_t)ks * vrow);
 #pragma unroll
-        for (int j = 0; j < VI; ++j) dma16(g, src[j], lds_v + (c & 3) * VTILE + (VI * gw + j) * 1024);
+        for (int j = 0; j < VI; ++j) dma16(g, src[j], __builtin_amdgcn_readfirstlane(lds_v + sl * VTILE + (VI * gw + j) * 1024));
       };
-      auto dma_k = [&](const int ks, const int c) __attribute__((always_inline)) {
+      auto dma_k = [&](const int ks, const int sl) __attribute__((always_inline)) {
         const char* g = reinterpret_cast<const char*>(kp + (size_t)ks * krow);
 #pragma unroll
-        for (int j = 0; j < KI; ++j) dma16(g, src[j], lds_k + (c & 3) * KTILE + (KI * gw + j) * 1024);
+        for (int j = 0; j < KI; ++j) dma16(g, src[j], __builtin_amdgcn_readfirstlane(lds_k + sl * KTILE + (KI * gw + j) * 1024));
       };
       // operand addresses of this lane inside a tile (see qk_phase / pv_phase)
       const unsigned k_lane = (unsigned)(l32 * DK * 2) + 16u * (hf ^ (DK == 128 ? (l32 & 15) : ((l32 >> 1) & 7)));
       const unsigned v_lane = v_lane_addr<DV>(lane);
 
       // The first two chunks are requested before anything else when their addresses need no block list (the usual
-      // case: four or more chunks from dstart on), the next ones behind the loads of the block list.
-      const bool early_request = n_diag >= 4;
-      if (early_request) {
+      // case: four or more chunks from dstart on), the next ones behind the loads of the block list.  OWN: chunk 0, and the others behind the list.
+      const bool early_request = !OWN && n_diag >= 4;
+      auto request_own = [&](const int from, const int to) __attribute__((always_inline)) {
+        for (int c = from; c < to; ++c) {
+          if (late) dma_v(dstart + 64 * c, c);
+          else dma_k(dstart + 64 * c, c);
+        }
+      };
+      if (OWN) {
+        request_own(0, min(n_diag, OWN_EARLY));
+      } else if (early_request) {
         if (late) {
           dma_v(dstart, 0);
           dma_v(dstart + 64, 1);
         } else {
-          dma_k(dstart, 0);
-          dma_k(dstart + 64, 1);
+          dma_k(dstart, k_slot(0));
+          dma_k(dstart + 64, k_slot(1));
         }
       }
       // types of the blocks the chunks from dstart on fall into, as a bit mask (bit i = block dstart/Bs + i)
@@ -687,12 +704,20 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
         }
         if (lane == 0) wave_count[wave] = cnt;
       }
+      if (OWN) {
+        request_own(OWN_EARLY, n_diag);
+        // chunk 0 must have landed
+        if (n_diag < 4) __builtin_amdgcn_s_waitcnt(0x0f70);
+        else if (late) __builtin_amdgcn_s_waitcnt(0x0f70 | (3 * VI));
+        else __builtin_amdgcn_s_waitcnt(0x0f70 | (3 * KI));
+      }
       __syncthreads();
       int n_prior = 0;
 #pragma unroll
       for (int w2 = 0; w2 < NWAVES; ++w2) n_prior += wave_count[w2];
       n_prior = __builtin_amdgcn_readfirstlane(n_prior);
-      const int n_iters = n_diag + n_prior * per_blk;
+      const int n_loop_diag = OWN ? 0 : n_diag;           // of the loop's chunks, those from dstart on
+      const int n_iters = n_loop_diag + n_prior * per_blk;
 
       // chunk iterator (wave-uniform): first key of chunk nx_it, then on to the next; past the last chunk it repeats it
       int nx_it = 0, nx_j = 0, nx_sub = 0, ks_cur = dstart;
@@ -701,7 +726,7 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
       auto list_ahead = [&]() -> int { return lds_list[min(nx_j, MAX_LDS_LIST - 1)]; };
       auto next_chunk = [&](const int ahead = 0, const bool have_ahead = false) __attribute__((always_inline)) -> int {
         if (nx_it < n_iters) {
-          if (nx_it < n_diag) {
+          if (nx_it < n_loop_diag) {
             ks_cur = dstart + nx_it * 64;
           } else {
             int e;
@@ -719,18 +744,30 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
       };
       // the early waves' iterator runs four chunks ahead of the loop, the late waves' three
       if (early_request) nx_it = 2;
-      for (int c = nx_it; c < (late ? 3 : 4); ++c) {
-        const int ks = next_chunk();
-        if (c < n_iters) {
-          if (late) dma_v(ks, c);
-          else dma_k(ks, c);
+      auto request_to = [&](const int last) __attribute__((always_inline)) {   // chunks nx_it .. last - 1
+        for (int c = nx_it; c < last; ++c) {
+          const int ks = next_chunk();
+          if (c < n_iters) {
+            if (late) dma_v(ks, c & 3);
+            else dma_k(ks, k_slot(c));
+          }
         }
+      };
+      const int first_set = late ? 3 : 4;
+      if (OWN) {
+        if (!late) request_to(1);
+        if (n_iters == 0) {
+          __builtin_amdgcn_s_waitcnt(0x0f70);
+          __syncthreads();
+        }
+      } else {
+        request_to(first_set);
+        // K(0), K(1) and V(0) must have landed: the newer requests of a full set may stay in flight
+        if (n_iters < 4) __builtin_amdgcn_s_waitcnt(0x0f70);
+        else if (late) __builtin_amdgcn_s_waitcnt(0x0f70 | (2 * VI));
+        else __builtin_amdgcn_s_waitcnt(0x0f70 | (2 * KI));
+        __syncthreads();                          // "sync(-1)"
       }
-      // K(0), K(1) and V(0) must have landed: the newer requests of a full set may stay in flight
-      if (n_iters < 4) __builtin_amdgcn_s_waitcnt(0x0f70);
-      else if (late) __builtin_amdgcn_s_waitcnt(0x0f70 | (2 * VI));
-      else __builtin_amdgcn_s_waitcnt(0x0f70 | (2 * KI));
-      __syncthreads();                            // "sync(-1)"
 
       // which of the chunks from dstart on this wave takes part in (bit it), and which one is its own, causal chunk:
       // lane i works it out for chunk i, once
@@ -753,12 +790,52 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
       }
       m_ref = 0.f;       // an arbitrary finite reference until the row's first visible key sets the real one
       float thr = -INFINITY;
-      f32x16 s0, s1;
-      bool cur_active = act_mask & 1ull;
-      if (cur_active) qk_phase<DK>(lds_k + k_lane, QB, m_ref, s0, s1);
-      auto is_active = [&](const int it) -> bool { return it < n_diag ? (act_mask >> it) & 1ull : it < n_iters; };
-
+      // (called in both branches below, and not once before them: there the compiler moves the accumulators to other registers on
+      // the way into the loops, and 128/128 spills 24)
+      auto own_chunks = [&]() __attribute__((always_inline)) {
+#pragma unroll 1
+        for (int it = 0; it < 4; ++it) {
+          if (it == 1 && n_iters > 0) {
+            // own chunks 1 to 3 must have landed; the request for K(0) may stay in flight
+            if (late) __builtin_amdgcn_s_waitcnt(0x0f70);
+            else __builtin_amdgcn_s_waitcnt(0x0f70 | KI);
+            __syncthreads();
+            request_to(late ? 1 : 2);
+          }
+          if (!((act_mask >> it) & 1ull)) continue;
+          // (own copies of what the addresses and masks are made of: shared with the loop they would be held across both, in registers there are not)
+          int ln = lane;
+          asm volatile("" : "+v"(ln));
+          const int r32 = ln & 31;
+          const unsigned ka = (unsigned)(r32 * DK * 2) + 16u * ((ln >> 5) ^ (DK == 128 ? (r32 & 15) : ((r32 >> 1) & 7)));
+          const unsigned va = v_lane_addr<DV>(ln);
+          bf16x8 PB[4];
+          f32x16 s0, s1;
+          __builtin_amdgcn_s_setprio(3);
+          qk_phase<DK>(lds_k + it * KTILE + ka, QB, m_ref, s0, s1);
+          __builtin_amdgcn_s_setprio(0);
+          __builtin_amdgcn_sched_barrier(0);      // (nor the values' operands ahead of the exponentials: they would not fit)
+          softmax_phase<DV>(s0, s1, acc, m_ref, l_run, thr, ln, it == causal_it, qloc0, PB);
+          __builtin_amdgcn_sched_barrier(0);
+          __builtin_amdgcn_s_setprio(3);
+          pv_phase<DV>(lds_v + it * VTILE + va, PB, acc, l_run);
+          __builtin_amdgcn_s_setprio(0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        act_mask = 0;
+        causal_it = -1;
+        if (n_iters > 0) {
+          __builtin_amdgcn_s_waitcnt(0x0f70);
+          __syncthreads();                        // "sync(-1)": K(0), K(1) and V(0) have landed, and nobody reads the own chunks any more
+          request_to(first_set);
+        }
+      };
+      auto is_active = [&](const int it) -> bool { return it < n_loop_diag ? (act_mask >> it) & 1ull : it < n_iters; };
       if (!late) {
+        if (OWN) own_chunks();
+        bool cur_active = is_active(0);
+        f32x16 s0, s1;
+        if (cur_active) qk_phase<DK>(lds_k + k_slot(0) * KTILE + k_lane, QB, m_ref, s0, s1);
         for (int it = 0; it < n_iters; ++it) {
           const bool nxt_active = is_active(it + 1);
           const int ahead = list_ahead();
@@ -769,17 +846,21 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
             pv_phase<DV>(lds_v + (it & 3) * VTILE + v_lane, PB, acc, l_run);
           }
           __builtin_amdgcn_s_setprio(3);
-          if (nxt_active) qk_phase<DK>(lds_k + ((it + 1) & 3) * KTILE + k_lane, QB, m_ref, s0, s1);
+          if (nxt_active) qk_phase<DK>(lds_k + k_slot(it + 1) * KTILE + k_lane, QB, m_ref, s0, s1);
           __builtin_amdgcn_s_setprio(0);
           // K(it+2) must have landed; the request for K(it+3), the newest, may stay in flight if there is one
           if (it + 3 < n_iters) __builtin_amdgcn_s_waitcnt(0x0f70 | KI);
           else __builtin_amdgcn_s_waitcnt(0x0f70);
           __syncthreads();                                  // sync(it)
           const int ks = next_chunk(ahead, true);
-          if (it + 4 < n_iters) dma_k(ks, it + 4);
+          if (it + 4 < n_iters) dma_k(ks, k_slot(it + 4));
           cur_active = nxt_active;
         }
       } else {
+        if (OWN) own_chunks();
+        bool cur_active = is_active(0);
+        f32x16 s0, s1;
+        if (cur_active) qk_phase<DK>(lds_k + k_slot(0) * KTILE + k_lane, QB, m_ref, s0, s1);
         for (int it = 0; it < n_iters; ++it) {
           const bool nxt_active = is_active(it + 1);
           const int ahead = list_ahead();
@@ -793,11 +874,11 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
           __syncthreads();                                  // sync(it)
           __builtin_amdgcn_s_setprio(3);
           if (cur_active) pv_phase<DV>(lds_v + (it & 3) * VTILE + v_lane, PB, acc, l_run);
-          if (nxt_active) qk_phase<DK>(lds_k + ((it + 1) & 3) * KTILE + k_lane, QB, m_ref, s0, s1);
+          if (nxt_active) qk_phase<DK>(lds_k + k_slot(it + 1) * KTILE + k_lane, QB, m_ref, s0, s1);
           __builtin_amdgcn_s_setprio(0);
           // the matrix phases come first, while the early waves are in their vector phase; the requests follow
           const int ks = next_chunk(ahead, true);
-          if (it + 3 < n_iters) dma_v(ks, it + 3);
+          if (it + 3 < n_iters) dma_v(ks, (it + 3) & 3);
           cur_active = nxt_active;
         }
       }
@@ -1520,15 +1601,15 @@ void softmax_stream_kernel(const SoftmaxParams p, unsigned* queue) {
 
 }
 
-template <int DK, int DV, int NWAVES>
+template <int DK, int DV, int NWAVES, bool OWN = false>
 static int launch_softmax(const SoftmaxParams& p, hipStream_t stream) {
   constexpr int KP = DK + 8, VP = DV + 8, QTILE = 32 * NWAVES;
   size_t lds = (size_t)2 * (64 * KP + DV * VT_PITCH) * sizeof(bf16_t);
   const size_t epi = (size_t)QTILE * VP * sizeof(bf16_t);
   if (epi > lds) lds = epi;
-  const size_t ring = (size_t)4 * 64 * (DK + DV) * sizeof(bf16_t) + 1024;  // 8 waves: four K and four V tiles, 1 KiB aligned
+  const size_t ring = (size_t)64 * (4 * (DK + DV) + (OWN ? DK : 0)) * sizeof(bf16_t) + 1024;  // 8 waves: the K and V slots, 1 KiB aligned
   if (NWAVES == 8 && ring > lds) lds = ring;
-  auto kern = softmax_sparse_fwd_kernel<DK, DV, NWAVES>;
+  auto kern = softmax_sparse_fwd_kernel<DK, DV, NWAVES, OWN>;
   static std::atomic<unsigned long long> reserved{0};
   if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, lds, "softmax")) return rc;
   const long long grid = p.seqs ? (long long)p.total_tiles * (QTILE_TABLE / QTILE) * p.HQ
@@ -1679,7 +1760,8 @@ int softmax_fwd(const void* q, const void* k, const void* v, void* o, float* lse
   if (K == KK && V == VV) {                                           \
     if (sd && !seqs && T % 256 == 0) return launch_softmax_stream<KK, VV, false, false>(p, sd, queue, s); \
     if (sd) return queue ? launch_softmax_stream<KK, VV, true, false>(p, sd, queue, s) : launch_softmax_stream<KK, VV, true, true>(p, sd, nullptr, s); \
-    return p.variant == 8 ? launch_softmax<KK, VV, 8>(p, s) : launch_softmax<KK, VV, 4>(p, s); \
+    if (p.variant != 8) return launch_softmax<KK, VV, 4>(p, s);       \
+    return block == 64 ? launch_softmax<KK, VV, 8, true>(p, s) : launch_softmax<KK, VV, 8>(p, s); \
   }
   NATSL_SM(128, 128)
   NATSL_SM(64, 64)

@@ -111,3 +111,25 @@ def test_softmax_wide_tiles_packed():
     torch.cuda.synchronize()
     assert_close(o.float(), o_ref, "o_attn")
     assert_close(lse, lse_ref, "lse")
+
+
+@pytest.mark.parametrize("K,V", [(128, 128), (64, 64), (64, 128), (128, 64)])
+@pytest.mark.parametrize("T,same_block", [(320, True), (704, False), (1024, True)])
+def test_softmax_wide_tiles_own_chunks_then_prior_ones(T, same_block, K, V):
+    """Selector blocks of one chunk on the 8-wave shape: the tile's own chunks go before the others.  Selector head h has its first h
+    blocks attention-typed, so the last tile of head h has h prior chunks, through all the fillings of the rings (none, fewer than
+    they hold, as many, more), and a last tile of one, three and four chunks.  The tolerance is that of every test against the oracle."""
+    from neuralattentionsearchlinear_amd import nats_util
+    from neuralattentionsearchlinear_amd.attns import parallel_attn_nats_fwd
+    B, HQ, H, HN, block, dev = 4, 32, 16, 8, 64, torch.device('cuda:0')
+    q, k, v = make_qkv(B, T, H, K, V, 60, HQ=HQ)
+    ty = make_types(B, T // block, HN, 0.0, 0, torch.bfloat16)
+    for h in range(HN):
+        ty[:, :h, h] = torch.tensor([1, 0], dtype=ty.dtype)
+    o_ref, lse_ref = sb.softmax_branch(q, k, v, ty, K ** -0.5, block, same_block)
+    r = nats_util.route(ty.to(dev), T, block)
+    o, lse, _ = parallel_attn_nats_fwd(q.to(dev), k.to(dev), v.to(dev), ty.to(dev), r['nats_block_indices'], None, K ** -0.5, block,
+                                       compute_incomplete_chunk_scores=same_block, n_nats_blocks=r['n_nats_blocks'])
+    torch.cuda.synchronize()
+    assert_close(o.float(), o_ref, "o_attn")
+    assert_close(lse, lse_ref, "lse")

@@ -86,6 +86,16 @@ NATSL_DEVICE float xhalf_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// The same for x[lane ^ 16].
+NATSL_DEVICE float xrow_max(float x) {
+  u32x2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+NATSL_DEVICE float xrow_sum(float x) {
+  u32x2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 // The layers' gates, shared by whole sequences and single steps: both write rows of the same cache, so both take the library's
 // exponential (the hardware's differs from it by up to its argument in ulps, and g is kept and summed up in fp32).
 NATSL_DEVICE float softplus_gate(const float x) { return x > 20.f ? x : log1pf(expf(x)); }

@@ -108,19 +108,6 @@ struct ConvWindow {
       w[j] = bf16_to_f32(weight[d * W + j]);
     }
   }
-  // W == 4, every pointer on 8 bytes
-  NATSL_DEVICE void init4(const void* state, const void* weight, const void* bias, const size_t d, const size_t sd) {
-    const u32x2 es = reinterpret_cast<const u32x2*>(state)[sd], ws = reinterpret_cast<const u32x2*>(weight)[d];
-    b = bias ? bf16_to_f32(reinterpret_cast<const bf16_t*>(bias)[d]) : 0.f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      e[j] = __uint_as_float(j & 1 ? es[j >> 1] & 0xffff0000u : es[j >> 1] << 16);
-      w[j] = __uint_as_float(j & 1 ? ws[j >> 1] & 0xffff0000u : ws[j >> 1] << 16);
-    }
-  }
-  NATSL_DEVICE void save4(void* state, const size_t sd) const {
-    reinterpret_cast<u32x2*>(state)[sd] = (u32x2){pack_bf16x2(e[0], e[1]), pack_bf16x2(e[2], e[3])};
-  }
   NATSL_DEVICE float next(const float x, const bool silu) {
 #pragma unroll
     for (int j = 0; j + 1 < W; ++j) e[j] = e[j + 1];
@@ -134,6 +121,44 @@ struct ConvWindow {
   NATSL_DEVICE void save(bf16_t* state, const size_t sd) {
 #pragma unroll
     for (int j = 0; j < W; ++j) state[sd * W + j] = f32_to_bf16(e[j]);
+  }
+};
+
+// What one token needs from memory, as it was loaded: a launch that does little else asks for all of it before it looks at any of it.  A
+// load behind a branch, or converted where it stands, is waited for on the spot, so nothing here depends on which form an input has: the
+// absent one is read from another tensor's place and dropped.  (An attending wave made four to seven round trips one behind another before
+// its first keys, three are left: arguments, windows and flags, keys.  step_one_kernel, 340M geometry, one sequence of 800 tokens: 10.9 -> 9.6 us;
+// 16 heads of 128/64, eight sequences of 2000: 17.3 -> 16.7.)
+struct AnyRaw {             // an element of either type
+  bf16_t lo, hi;
+  NATSL_DEVICE void load(const void* p, const int dtype, const size_t i) {
+    const int size = dtype == NATSL_F32 ? 4 : 2;
+    const char* at = reinterpret_cast<const char*>(p) + i * size;
+    lo = *reinterpret_cast<const bf16_t*>(at);
+    hi = *reinterpret_cast<const bf16_t*>(at + size - 2);
+  }
+  NATSL_DEVICE float get(const int dtype) const { return __uint_as_float((unsigned)hi << 16 | (dtype == NATSL_F32 ? (unsigned)lo : 0u)); }
+};
+struct StepWindow {         // a convolution of width 4 at one channel, every pointer on 8 bytes; x: the new input
+  u32x2 e, w;
+  bf16_t b, x;
+  NATSL_DEVICE void load(const bf16_t* proj, const void* state, const void* weight, const void* bias, const size_t d, const size_t sd) {
+    x = proj[d];
+    e = reinterpret_cast<const u32x2*>(state)[sd];
+    w = reinterpret_cast<const u32x2*>(weight)[d];
+    b = reinterpret_cast<const bf16_t*>(bias ? bias : weight)[d];
+  }
+  NATSL_DEVICE float next(const bool bias, const bool silu) const {
+    float a = bias ? bf16_to_f32(b) : 0.f;
+    a += __uint_as_float(w[0] << 16) * __uint_as_float(e[0] & 0xffff0000u);
+    a += __uint_as_float(w[0] & 0xffff0000u) * __uint_as_float(e[1] << 16);
+    a += __uint_as_float(w[1] << 16) * __uint_as_float(e[1] & 0xffff0000u);
+    a += __uint_as_float(w[1] & 0xffff0000u) * bf16_to_f32(x);
+    if (silu) a = a / (1.f + __expf(-a));
+    return bf16_to_f32(f32_to_bf16(a));
+  }
+  NATSL_DEVICE void save(void* state, const size_t sd) const {
+    reinterpret_cast<u32x2*>(state)[sd] = (u32x2){e[0] >> 16 | e[1] << 16, e[1] >> 16 | (unsigned)x << 16};
   }
 };
 
@@ -165,11 +190,8 @@ __global__ __launch_bounds__(256) void step_mix_kernel(const StepMix p) {
       float lin = y, at = from_conv ? y : x;
       if (l2 || norm) {
         float a2 = on ? at * at : 0.f, y2 = on ? y * y : 0.f;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-          a2 += __shfl_xor(a2, o);
-          y2 += __shfl_xor(y2, o);
-        }
+        a2 = wave_sum(a2);
+        y2 = wave_sum(y2);
         __syncthreads();                               // the previous token's sums have been read
         if ((tid & 63) == 0) { red[0][tid >> 6] = a2; red[1][tid >> 6] = y2; }
         __syncthreads();
@@ -253,14 +275,15 @@ struct StepTail {
 template <int VA>
 struct TailRow {
   static constexpr int CPL = VA / 64;
-  float g[CPL], w1[CPL], w2[CPL];
+  bf16_t gate[CPL];
+  AnyRaw w1[CPL], w2[CPL];
   NATSL_DEVICE void load(const StepTail& p, const int row, const int hq) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int j = 0; j < CPL; ++j) {
-      g[j] = bf16_to_f32(p.proj[(size_t)row * p.ldp + p.cg + hq * VA + CPL * lane + j]);
-      w1[j] = ld_any(p.w1, p.w_dtype, CPL * lane + j);
-      w2[j] = ld_any(p.w2, p.w_dtype, CPL * lane + j);
+      gate[j] = p.proj[(size_t)row * p.ldp + p.cg + hq * VA + CPL * lane + j];
+      w1[j].load(p.w1, p.w_dtype, CPL * lane + j);
+      w2[j].load(p.w2, p.w_dtype, CPL * lane + j);
     }
   }
   NATSL_DEVICE void finish(const StepTail& p, const int row, const int hq, float d0, float d1, const float* at, const float* x1) const;
@@ -276,22 +299,17 @@ NATSL_DEVICE void TailRow<VA>::finish(const StepTail& p, const int row, const in
     sa += x1[j] * x1[j];
     sb += x2[j] * x2[j];
   }
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    d0 += __shfl_xor(d0, o);
-    d1 += __shfl_xor(d1, o);
-    sa += __shfl_xor(sa, o);
-    sb += __shfl_xor(sb, o);
-  }
-  d0 = bf16_to_f32(f32_to_bf16(d0));                   // (as the projection's output is)
-  d1 = bf16_to_f32(f32_to_bf16(d1));
+  sa = wave_sum(sa);
+  sb = wave_sum(sb);
+  d0 = bf16_to_f32(f32_to_bf16(wave_sum(d0)));         // (as the projection's output is)
+  d1 = bf16_to_f32(f32_to_bf16(wave_sum(d1)));
   mix_softmax(d0, d1);
   const float ra = rsqrtf(sa / VA + p.eps) * d0, rb = rsqrtf(sb / VA + p.eps) * d1;
   const size_t base = ((size_t)row * p.HQ + hq) * VA + CPL * lane;
 #pragma unroll
   for (int j = 0; j < CPL; ++j) {
-    const float mix = x1[j] * ra * w1[j] + x2[j] * rb * w2[j];
-    p.y[base + j] = f32_to_bf16(mix * g[j] / (1.f + __expf(-g[j])));
+    const float mix = x1[j] * ra * w1[j].get(p.w_dtype) + x2[j] * rb * w2[j].get(p.w_dtype), g = bf16_to_f32(gate[j]);
+    p.y[base + j] = f32_to_bf16(mix * g / (1.f + __expf(-g)));
   }
 }
 
@@ -328,8 +346,10 @@ __global__ __launch_bounds__(256) void step_tail_kernel(const StepTail p) {
 // needs itself, and the tail of a (sequence, head) is done by whichever wave is the last to have written something for it: they
 // count themselves in on arrived[], which the projections' launch has cleared.  No wave waits for another.  Bound by round trips to
 // memory one behind another (arguments, windows and flags, keys, the count, the others' results); with many keys by their bytes.
-// Against the three launches: 340M geometry, one sequence of 800 tokens, 11.0 us for 4.3 + 5.4 + 4.8 and two gaps of 3.5; 16 heads of
-// 128/64 and eight sequences of 2000 tokens, 18 us for 5 + 13.6 + 5.3.  Workgroups:
+// Against the three launches: 340M geometry, one sequence of 800 tokens, 9.6 us for 4.3 + 5.4 + 4.8 and two gaps of 3.5; 16 heads of
+// 128/64 and eight sequences of 2000 tokens, 16.7 us for 5 + 13.6 + 5.3 (the three before the changes noted at AnyRaw and wave_sum).  Of the
+// 9.6 us: 2.6 until the first keys are asked for, 1.6 - 2.4 for a chunk and the join of the waves, 0.8 to hand a result over and count it,
+// 1.4 for the tail, 2 - 3 before and behind the waves.  Workgroups:
 //   mixing logits   (sequence, 256 channels of q): their convolution, and their share of all heads' two logits
 //   recurrence      (sequence, head, 64 state columns), as in attend_and_recur
 //   attention       (sequence, head, split), as in attend_and_recur; the wave with the last chunk makes the new key and value
@@ -346,12 +366,6 @@ struct StepOne {
   int n_chunks, n_logits, n_rec;
 };
 constexpr int LOGIT_CHUNK = 256;
-
-NATSL_DEVICE float wave_sum(float x) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) x += __shfl_xor(x, o);
-  return x;
-}
 
 // Everything that the wave handed over (stores that write through) has arrived before the lane with `on` counts it in.  What orders the two
 // is this machine, not the language: the atomics are relaxed, s_waitcnt vmcnt(0) holds the count back until every lane's
@@ -397,16 +411,13 @@ NATSL_DEVICE void step_logits(const StepOne& p, const int b, const int chunk, co
 #pragma unroll
     for (int u = 0; u < 2 * U; ++u) r[u] = *reinterpret_cast<const u32x2*>(w + (size_t)(2 * min(h0 + 4 * (u >> 1), s.HQ - 1) + (u & 1)) * KD);
   };
-  bf16_t y = 0;
-  if (d < KD) {
-    const size_t sd = (size_t)b * KD + d;
-    ConvWindow<4> win;
-    win.init4(s.conv_state_q, s.conv_wq, s.conv_bq, d, sd);
-    y = f32_to_bf16(win.next(bf16_to_f32(p.m.proj[(size_t)b * p.m.ldp + p.m.cq + d]), s.flags & NATSL_STEP_SILU));
-    win.save4(s.conv_out_q, sd);
-  }
+  const size_t sd = (size_t)b * KD;
+  StepWindow win;
+  win.load(p.m.proj + (size_t)b * p.m.ldp + p.m.cq, s.conv_state_q, s.conv_wq, s.conv_bq, min(d, KD - 1), sd + min(d, KD - 1));
   load(wave);
-  qs[tid] = y;
+  const bf16_t y = f32_to_bf16(win.next(s.conv_bq != nullptr, s.flags & NATSL_STEP_SILU));
+  if (d < KD) win.save(s.conv_out_q, sd + d);
+  qs[tid] = d < KD ? y : (bf16_t)0;
   if (s.block_hidden) {
     const bf16_t* x = (const bf16_t*)s.x + (size_t)b * s.D;
     bf16_t* to = (bf16_t*)s.block_hidden + ((size_t)b * s.block + s.n_in) * s.D;
@@ -453,25 +464,26 @@ struct StepToken {
     const bool silu = s.flags & NATSL_STEP_SILU;
     const bf16_t* proj = p.m.proj + (size_t)n * p.m.ldp;
     const size_t block_row = (size_t)n * s.block + s.n_in;
-    ConvWindow<4> wq[C], wk[C], wv;
+    StepWindow wq[C], wk[C], wv;
     float xq[C], xk[C];
 #pragma unroll
     for (int i = 0; i < C; ++i) {
       const int d = h * DK + 64 * i + lane;
-      wq[i].init4(s.conv_state_q, s.conv_wq, s.conv_bq, d, (size_t)n * KD + d);
-      wk[i].init4(s.conv_state_k, s.conv_wk, s.conv_bk, d, (size_t)n * KD + d);
-      xq[i] = bf16_to_f32(proj[p.m.cq + d]);
-      xk[i] = bf16_to_f32(proj[p.m.ck + d]);
+      wq[i].load(proj + p.m.cq, s.conv_state_q, s.conv_wq, s.conv_bq, d, (size_t)n * KD + d);
+      wk[i].load(proj + p.m.ck, s.conv_state_k, s.conv_wk, s.conv_bk, d, (size_t)n * KD + d);
     }
     const int dv = h * s.V + vc;
-    wv.init4(s.conv_state_v, s.conv_wv, s.conv_bv, dv, (size_t)n * VD + dv);
-    const float xv = bf16_to_f32(proj[p.m.cv + dv]);
-    const float A = expf(ld_any(s.a_log, s.gate_dtype, h));
-    const float dt = softplus_gate(bf16_to_f32(proj[p.m.ca + h]) + ld_any(s.dt_bias, s.gate_dtype, h));
+    wv.load(proj + p.m.cv, s.conv_state_v, s.conv_wv, s.conv_bv, dv, (size_t)n * VD + dv);
+    AnyRaw a_log, dt_bias;
+    a_log.load(s.a_log, s.gate_dtype, h);
+    dt_bias.load(s.dt_bias, s.gate_dtype, h);
+    const bf16_t xa = proj[p.m.ca + h], xb = DELTA ? proj[p.m.cb + h] : (bf16_t)0;
+    const float A = expf(a_log.get(s.gate_dtype));
+    const float dt = softplus_gate(bf16_to_f32(xa) + dt_bias.get(s.gate_dtype));
     gt = -A * dt;
     bt = 1.f;
     if (DELTA) {
-      float sg = bf16_to_f32(f32_to_bf16(sigmoid_gate(bf16_to_f32(proj[p.m.cb + h]))));
+      float sg = bf16_to_f32(f32_to_bf16(sigmoid_gate(bf16_to_f32(xb))));
       if (s.flags & NATSL_STEP_NEG_EIGVAL) sg *= 2.f;
       bt = bf16_to_f32(f32_to_bf16(sg));
     }
@@ -479,8 +491,8 @@ struct StepToken {
     const bool l2 = s.flags & NATSL_STEP_L2_ROWS;
 #pragma unroll
     for (int i = 0; i < C; ++i) {
-      xq[i] = wq[i].next(xq[i], silu);
-      xk[i] = wk[i].next(xk[i], silu);
+      xq[i] = wq[i].next(s.conv_bq != nullptr, silu);
+      xk[i] = wk[i].next(s.conv_bk != nullptr, silu);
       if (l2) {
         ssq += wave_sum(xq[i] * xq[i]);
         ssk += wave_sum(xk[i] * xk[i]);
@@ -495,19 +507,19 @@ struct StepToken {
       if (first) {
         const int d = h * DK + 64 * i + lane;
         ((bf16_t*)s.block_k)[block_row * KD + d] = kb;
-        wk[i].save4(s.conv_out_k, (size_t)n * KD + d);
+        wk[i].save(s.conv_out_k, (size_t)n * KD + d);
       }
     }
     if (first && lane == 0) {
       s.block_g[block_row * s.H + h] = gt;
       if (DELTA) ((bf16_t*)s.block_beta)[block_row * s.H + h] = f32_to_bf16(bt);
     }
-    float y = wv.next(xv, silu);
+    float y = wv.next(s.conv_bv != nullptr, silu);
     if (!DELTA) y = bf16_to_f32(f32_to_bf16(y * dt));
     vt = y;
     if (kq == 0) {
       ((bf16_t*)s.block_v)[block_row * VD + dv] = f32_to_bf16(y);
-      wv.save4(s.conv_out_v, (size_t)n * VD + dv);
+      wv.save(s.conv_out_v, (size_t)n * VD + dv);
     }
     __builtin_amdgcn_wave_barrier();
     ld_row<R>(rows, NATSL_BF16, true, kq * R, qq);
@@ -525,25 +537,31 @@ struct StepToken {
 template <int N>
 struct StepRow {
   static constexpr int C = N / 64;
-  float x[C], nw[C];
-  ConvWindow<4> win[C];
+  StepWindow win[C];
+  AnyRaw nw[C];
   NATSL_DEVICE void request(const natsl_layer_step& s, const bf16_t* proj, const void* state, const void* weight, const void* bias, const void* norm,
                             const size_t seq, const int d0) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int i = 0; i < C; ++i) {
       const int d = d0 + 64 * i + lane;
-      x[i] = bf16_to_f32(proj[d]);
-      nw[i] = norm ? ld_any(norm, s.norm_dtype, 64 * i + lane) : 1.f;
-      if (s.flags & NATSL_STEP_ATTN_FROM_CONV) win[i].init4(state, weight, bias, d, seq + d);
+      win[i].load(proj, state, weight, bias, d, seq + d);
+      nw[i].load(norm ? norm : weight, s.norm_dtype, 64 * i + lane);
     }
   }
-  NATSL_DEVICE void form(const natsl_layer_step& s, const bool norm, bf16_t* dst, bf16_t* also) {
+  NATSL_DEVICE void form(const natsl_layer_step& s, const bool bias, const bool norm, bf16_t* dst, bf16_t* also) const {
     const int lane = threadIdx.x & 63;
-    float ss = 0.f, r = 1.f;
+    float x[C], ss = 0.f, r = 1.f;
+    AnyRaw m[C];
 #pragma unroll
-    for (int i = 0; i < C; ++i)
-      if (s.flags & NATSL_STEP_ATTN_FROM_CONV) x[i] = win[i].next(x[i], s.flags & NATSL_STEP_SILU);
+    for (int i = 0; i < C; ++i) {
+      // (a row is formed once, but inside a loop: without this the conversions move in front of it, and their waits with them)
+      StepWindow c = win[i];
+      m[i].lo = nw[i].lo;
+      m[i].hi = nw[i].hi;
+      asm volatile("" : "+v"(c.x), "+v"(c.b), "+v"(c.e), "+v"(c.w), "+v"(m[i].lo), "+v"(m[i].hi));
+      x[i] = s.flags & NATSL_STEP_ATTN_FROM_CONV ? c.next(bias, s.flags & NATSL_STEP_SILU) : bf16_to_f32(c.x);
+    }
     if (norm) {
 #pragma unroll
       for (int i = 0; i < C; ++i) ss += wave_sum(x[i] * x[i]);
@@ -551,7 +569,7 @@ struct StepRow {
     }
 #pragma unroll
     for (int i = 0; i < C; ++i) {
-      const bf16_t y = f32_to_bf16(norm ? x[i] * r * nw[i] : x[i]);
+      const bf16_t y = f32_to_bf16(norm ? x[i] * r * m[i].get(s.norm_dtype) : x[i]);
       dst[64 * i + lane] = y;
       if (also) also[64 * i + lane] = y;
     }
@@ -587,11 +605,11 @@ struct StepKeys {
     done = true;
     const natsl_layer_step& s = p.m.s;
     const bool norm = s.flags & NATSL_STEP_ATTN_NORM;
-    rq.form(s, norm, q, nullptr);
+    rq.form(s, s.conv_bq != nullptr, norm, q, nullptr);
     if (mine) {
       const size_t at = ((size_t)b * s.cache_tokens + first) * s.HQ + hq;
-      rk.form(s, norm, k, (bf16_t*)s.cache_k + at * KA);
-      rv.form(s, false, v, (bf16_t*)s.cache_v + at * VA);
+      rk.form(s, s.conv_bk != nullptr, norm, k, (bf16_t*)s.cache_k + at * KA);
+      rv.form(s, s.conv_bv != nullptr, false, v, (bf16_t*)s.cache_v + at * VA);
     }
     __builtin_amdgcn_wave_barrier();
     row.query(q, 0, p.a.scale_log2);
@@ -664,7 +682,8 @@ struct StepLayout {
 };
 
 // Workgroups of step_one_kernel that fit on the chip at once, less those of the logits and the recurrence: what its registers allow a CU
-// (195 - 228 with 192-wide states or 128-wide keys and values: two; 118 with 64-wide everything: four; else 147 - 168: three).
+// (214 with 192-wide states: two; 106 with 64-wide everything: four; else 130 - 166: three.  128-wide keys and values are counted as two, which
+// the splits below were measured with).
 static int step_one_slots(const natsl_layer_step& s, const int n_chunks) {
   const int KA = s.H * s.K / s.HQ, VA = s.H * s.V / s.HQ;
   const int per_cu = s.K == 192 || KA + VA == 256 ? 2 : KA + VA + s.K == 192 ? 4 : 3;

@@ -103,6 +103,23 @@ def test_layer_step_of_one_token(kind, B, T0, n, more, monkeypatch):
     test_layer_step_matches_the_general_path(kind, None, 'all', B, T0, (1,) * n, more, monkeypatch)
 
 
+@pytest.mark.parametrize("kind,more", [('gdn', {}), ('gdn', dict(conv_bias=True)), ('mamba', dict(expand_v=1))])
+def test_layer_step_of_one_token_with_float_parameters(kind, more, monkeypatch):
+    """The small parameters in fp32, with values that bf16 does not hold: the one-token launch reads either type without a branch."""
+    layer_of = _layer
+
+    def with_floats(*a, **kw):
+        layer = layer_of(*a, **kw)
+        names = [n for n, q in layer.named_parameters() if n in ('A_log', 'dt_bias') or 'norm.weight' in n]
+        assert len(names) >= 4, names
+        for n, q in layer.named_parameters():
+            if n in names:
+                q.data = q.data.float() * 1.003
+        return layer
+    monkeypatch.setitem(globals(), '_layer', with_floats)
+    test_layer_step_matches_the_general_path(kind, None, 'all', 2, 130, (1,) * 3, more, monkeypatch)
+
+
 @pytest.mark.parametrize("kind", ['gdn', 'mamba'])
 @pytest.mark.parametrize("float_gates", [False, True])
 def test_layer_step_forms_the_general_paths_gates(kind, float_gates, monkeypatch):

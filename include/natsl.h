@@ -467,6 +467,9 @@ typedef struct natsl_front {
 int natsl_layer_front(const natsl_front* a, natsl_stream_t stream);
 /* dw [N, D] = dy [rows, N]^T x [rows, D] (bf16, N up to 64, D even) for a narrow weight over few rows: the selector's over the block means. */
 int natsl_narrow_wgrad(const void* dy, const void* x, void* dw, int64_t rows, int D, int N, natsl_stream_t stream);
+/* The same over many rows, through partial sums in a workspace: the mixing logits' weight. */
+size_t natsl_narrow_wgrad_workspace_bytes(int64_t rows, int D, int N);
+int natsl_narrow_wgrad_split(const void* dy, const void* x, void* dw, int64_t rows, int D, int N, void* workspace, size_t workspace_bytes, natsl_stream_t stream);
 
 /* The layers' gates from one projection ab [rows, ld] (bf16; a in columns 0..H-1, b in H..2H-1 for the delta rule):
  * g = -exp(a_log) softplus(a + dt_bias) fp32 [rows, H], beta = sigmoid(b) bf16 (doubled with neg_eigval; NULL for Mamba),

@@ -102,6 +102,8 @@ _SIGNATURES = {
     "natsl_project_bwd": (c_int, [c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 4 + [c_void_p]),
     "natsl_layer_front": (c_int, [c_void_p, c_void_p]),
     "natsl_narrow_wgrad": (c_int, [c_void_p] * 3 + [c_int64, c_int, c_int, c_void_p]),
+    "natsl_narrow_wgrad_workspace_bytes": (c_size_t, [c_int64, c_int, c_int]),
+    "natsl_narrow_wgrad_split": (c_int, [c_void_p] * 3 + [c_int64, c_int, c_int, c_void_p, c_size_t, c_void_p]),
     "natsl_narrow_linear_bwd": (c_int, [c_void_p] * 3 + [c_int64, c_int, c_int, c_void_p]),
     "natsl_wgrad_workspace_bytes": (c_size_t, [c_void_p, c_int, c_int64, c_int]),
     "natsl_wgrad": (c_int, [c_void_p, c_int, c_void_p, c_int64, c_int, c_int, c_void_p, c_size_t, c_void_p]),

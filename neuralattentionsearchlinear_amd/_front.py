@@ -48,15 +48,33 @@ def _p(t):
     return None if t is None else t.data_ptr()
 
 
+def _narrow_split_pays(rows, N, D, alone):
+    """Whether natsl_narrow_wgrad_split forms dy [rows, N]^T x [rows, D].  us, library or natsl_wgrad / it: widths that are no multiple of 8, the library,
+    36 x 1152 over 2000 19 / 8.5, 6000 42 / 12, 32768 112 / 36; natsl_wgrad 24 x 768 over 2000 14 / 5.7, 32768 28 / 14, 32 x 2048 over 2000 16 / 7.3,
+    16000 24 / 21, 32768 39 / 46, 48 x 1536 over 16000 25 / 20, 32768 37 / 49, 64 x 2048 over 6000 20 / 24."""
+    if N > 64 or D % 2 or not 0 < rows < 1 << 31:
+        return False
+    return N % 8 != 0 or (alone and N <= 48 and rows * D <= 1 << 25)
+
+
 def weight_grads(x2, dys):
-    """[dy_i^T x2 for dy_i [rows, n_i] in dys] (bf16; entries may be None): natsl_wgrad for widths that are multiples of 8, else torch."""
+    """[dy_i^T x2 for dy_i [rows, n_i] in dys] (bf16; entries may be None): natsl_wgrad for widths that are multiples of 8, natsl_narrow_wgrad_split
+    for narrow ones that are not, or that are alone, else torch."""
     rows, D = x2.shape
     out = [None] * len(dys)
     todo = []
+    alone = sum(dy is not None for dy in dys) == 1
     for i, dy in enumerate(dys):
         if dy is None:
             continue
-        if dy.shape[1] % 8 or D % 8 or x2.data_ptr() % 16 or dy.data_ptr() % 16 or dy.dtype != torch.bfloat16:
+        if _narrow_split_pays(rows, dy.shape[1], D, alone) and x2.data_ptr() % 4 == 0 and dy.dtype == x2.dtype == torch.bfloat16:
+            out[i] = torch.empty(dy.shape[1], D, dtype=torch.bfloat16, device=x2.device)
+            L = _capi.lib()
+            n = L.natsl_narrow_wgrad_workspace_bytes(rows, D, dy.shape[1])
+            ws = torch.empty(n, dtype=torch.uint8, device=x2.device)
+            _capi.check(L.natsl_narrow_wgrad_split(dy.data_ptr(), x2.data_ptr(), out[i].data_ptr(), rows, D, dy.shape[1], ws.data_ptr(), n,
+                                                   _capi.stream_ptr(x2.device)), "natsl_narrow_wgrad_split")
+        elif dy.shape[1] % 8 or D % 8 or x2.data_ptr() % 16 or dy.data_ptr() % 16 or dy.dtype != torch.bfloat16:
             out[i] = torch.mm(dy.t(), x2)
         else:
             out[i] = torch.empty(dy.shape[1], D, dtype=torch.bfloat16, device=x2.device)
@@ -285,11 +303,11 @@ def _narrow_bwd(dy, w, few=False):
 
 
 def _narrow_wgrad(dy, x):
-    """dy [rows, N]^T x [rows, D]: natsl_narrow_wgrad up to some thousand rows (library / it, us: 12 x 1536 over 94 6.7 / 2.4, 512 8.1 / 3.2, 2048
-    7.0 / 6.7, 4096 9.7 / 11.2; 32 x 1024 over 512 7.4 / 5.1, 2048 8.6 / 13.9)."""
+    """dy [rows, N]^T x [rows, D]: natsl_narrow_wgrad up to two thousand rows (library / it, us: 12 x 1536 over 94 6.7 / 2.7, 512 8.1 / 3.2, 2048
+    7.0 / 5.1, 4096 9.6 / 7.6; 32 x 1024 over 512 7.3 / 3.6, 2048 8.6 / 6.5; 64 x 2048 over 2048 15.5 / 9.0)."""
     rows, N = dy.shape
     D = x.shape[1]
-    if N > 64 or D % 2 or rows > (2048 if N <= 16 else 1024):
+    if N > 64 or D % 2 or rows > 2048:
         return torch.mm(dy.t(), x)
     dw = torch.empty(N, D, dtype=dy.dtype, device=dy.device)
     _capi.check(_capi.lib().natsl_narrow_wgrad(dy.data_ptr(), x.data_ptr(), dw.data_ptr(), rows, D, N, _capi.stream_ptr(dy.device)), "natsl_narrow_wgrad")

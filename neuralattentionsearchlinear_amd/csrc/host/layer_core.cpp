@@ -5,6 +5,7 @@
 // tokens 380 and 193, about its kernels' time.
 // What is launched, and in which order, is what _front.py and _mixed_common.py describe.  Nothing here outlives a call but what make_layer()
 // is given: names of entry points, options and sizes, never a tensor.
+#include <algorithm>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
@@ -24,7 +25,7 @@ namespace {
 #define NATSL_ENTRIES(X)                                                                                                                   \
   X(layer_front) X(project) X(project_bwd) X(layer_select) X(hard_select_bwd) X(conv_norm_fwd) X(conv_norm_bwd) X(conv_norm_bwd_workspace_bytes) \
   X(mixed_fwd) X(mixed_workspace_bytes) X(norm_gate_logits_fwd) X(norm_gate_logits_bwd) X(norm_gate_bwd_workspace_bytes) X(wgrad)           \
-  X(wgrad_workspace_bytes) X(narrow_linear_bwd) X(narrow_wgrad) X(gates_bwd) X(gates_bwd_workspace_bytes) X(dx_init) X(softmax_sparse_bwd)  \
+  X(wgrad_workspace_bytes) X(narrow_linear_bwd) X(narrow_wgrad) X(narrow_wgrad_workspace_bytes) X(narrow_wgrad_split) X(gates_bwd) X(gates_bwd_workspace_bytes) X(dx_init) X(softmax_sparse_bwd)  \
   X(softmax_bwd_workspace_bytes) X(linear_workspace_bytes) X(linear_chunk_states) X(linear_block_sums) X(linear_chunk_bwd_steps)            \
   X(block_grads) X(order_streams)
 
@@ -242,14 +243,24 @@ void rest(const Call& c, const Front& f, const bool joint, const bool keep, cons
 // what the forward keeps, in this order behind x and the weights
 enum Kept { AB, WAB, POOLED, LOGITS, TYPES, RAW_Q, RAW_K, RAW_V, GATE, Y_Q, Y_K, Y_V, N_Q, N_K, MIX, G, BETA, DT, O_LIN, O_ATTN, LSE, IDX, NBLK, TAIL, STATES, V_NEW, WS, KEPT };
 
-// dy_i [rows, n_i]^T x [rows, D], one launch for those whose widths are multiples of 8
+// dy_i [rows, n_i]^T x [rows, D], one launch for those whose widths are multiples of 8; a narrow one that is not, or that is alone, by itself
+// (where: weight_grads of _front.py)
 void wgrads(const Call& c, const T& x, const std::vector<T>& dys, std::vector<T>& out) {
   const int64_t rows = x.size(0), D = x.size(1);
   out.assign(dys.size(), T());
   std::vector<natsl_wgrad_seg> segs;
+  const bool alone = std::count_if(dys.begin(), dys.end(), [](const T& t) { return t.defined(); }) == 1;
   for (size_t i = 0; i < dys.size(); ++i) {
     const T& dy = dys[i];
     if (!dy.defined()) continue;
+    const int64_t N = dy.size(1);
+    if (N <= 64 && D % 2 == 0 && (N % 8 || (alone && N <= 48 && rows * D <= int64_t(1) << 25))) {
+      out[i] = at::empty({N, D}, c.bf16);
+      const size_t n = c.l.narrow_wgrad_workspace_bytes(rows, (int)D, (int)N);
+      const T ws = c.bytes(n);
+      must(c.l.narrow_wgrad_split(at_(dy), at_(x), at_(out[i]), rows, (int)D, (int)N, at_(ws), n, c.stream), "natsl_narrow_wgrad_split");
+      continue;
+    }
     if (dy.size(1) % 8 || D % 8 || !on16(x) || !on16(dy)) {
       out[i] = at::mm(dy.t(), x);
       continue;
@@ -437,7 +448,7 @@ void backward(const Call& c, const Ts& s, const T& dout, const std::vector<bool>
   }
   if (want(WN)) {
     const int64_t r = dl2.size(0), n = l.NL;
-    if (n > 64 || l.D % 2 || r > (n <= 16 ? 2048 : 1024)) {
+    if (n > 64 || l.D % 2 || r > 2048) {
       grads[1 + WN] = at::mm(dl2.t(), s[POOLED]);
     } else {
       grads[1 + WN] = at::empty({n, l.D}, c.bf16);

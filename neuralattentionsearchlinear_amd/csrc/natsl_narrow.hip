@@ -4,6 +4,7 @@
 //   backward  X'[t][d] = sum_n Y'[t][n] W[n][d]   writes X' once
 // bf16 operands, fp32 sums, one rounding.  Where the contraction is no multiple of 32 a library product takes two to three times as long as for
 // one that is (36 rows of 1152 over 32768 tokens 36 us, 32 rows of 1024 19).
+#include <algorithm>
 #include <type_traits>
 
 #include "natsl_device.h"
@@ -276,30 +277,49 @@ __global__ __launch_bounds__(256) void narrow_bwd_kernel(const NarrowParams p) {
 // dW[n][d] = sum_t dY[t][n] X[t][d] for a narrow weight over few rows (the block means behind the selector's).  A workgroup takes 32 columns and
 // every row of the weight, its eight waves the tokens, 32 at a time in turn; both operands have the tokens along the contraction and are
 // gathered from the rows as they lie (X two columns a word: one product for the even, one for the odd ones).  Added up through LDS in order.
+// SPLIT, for many rows (the mixing logits' weight): gridDim.x workgroups share a column group's tokens and leave partial sums for
+// narrow_wgrad_sum_kernel.  Their number is a multiple of eight and their index the faster one: an XCD then takes every column of its tokens, and
+// reads the lines of X, which two column groups share, and of dY, which all do, once.  Bound by that reading, for few rows by two launches: a library product over so many rows
+// for so few outputs leaves most of the chip idle.  us, library / this: 36 x 1152 over 6000 tokens 42 / 12, 32768 112 / 36; 24 x 768 over 6000 42 / 7.2,
+// 32768 108 / 14 (natsl_wgrad 21 and 28).  A step asks for all its pieces before it uses one: left to itself the compiler had half of them in flight
+// (32768 tokens, 36 x 1152: 69 us).
 constexpr int NWG_WAVES = 8;
-template <int NT>
-__global__ __launch_bounds__(64 * NWG_WAVES) void narrow_wgrad_kernel(const bf16_t* dy, const bf16_t* x, bf16_t* dw, const int rows, const int D, const int N) {
+template <int NT, bool SPLIT>
+__global__ __launch_bounds__(64 * NWG_WAVES) void narrow_wgrad_kernel(const bf16_t* dy, const bf16_t* x, bf16_t* dw, float* parts, const int rows, const int D,
+                                                                      const int N) {
   __shared__ f32x4 sums[NWG_WAVES][2 * NT][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i16 = lane & 15, g4 = lane >> 4;
-  const int d = 32 * (int)blockIdx.x + 2 * i16;
+  const int d = 32 * (int)(SPLIT ? blockIdx.y : blockIdx.x) + 2 * i16, part = SPLIT ? (int)blockIdx.x : 0, n_parts = SPLIT ? (int)gridDim.x : 1;
   f32x4 acc[2][NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n) acc[0][n] = acc[1][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  const bf16_t* xc = x + min(d, D - 2);
-#pragma unroll 2
-  for (int t0 = 32 * wave; t0 < rows; t0 += 32 * NWG_WAVES) {
+  const int dc = min(d, D - 2);
+  int nc[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) nc[n] = min(16 * n + i16, N - 1);
+  // 32 tokens, `left` of them there; everything is requested before any of it is looked at
+  auto step = [&](const int t0, auto whole_c, const int left) __attribute__((always_inline)) {
+    constexpr bool WHOLE = decltype(whole_c)::value;
+    const bf16_t *xr = x + (size_t)t0 * D, *yr = dy + (size_t)t0 * N;
     unsigned xv[8];
     bf16_t yv[NT][8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const int t = t0 + 8 * g4 + j;
-      const size_t r = (size_t)min(t, rows - 1);
-      const unsigned v = *reinterpret_cast<const unsigned*>(xc + r * D);
-      xv[j] = t < rows ? v : 0u;
+      // (whole steps: a row's distance from the lane's first is the same in every lane)
+      xv[j] = WHOLE ? *reinterpret_cast<const unsigned*>(xr + (size_t)j * D + (unsigned)(8 * g4 * D + dc))
+                    : *reinterpret_cast<const unsigned*>(xr + (unsigned)(min(8 * g4 + j, left - 1) * D + dc));
 #pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        const bf16_t y = dy[r * N + min(16 * n + i16, N - 1)];
-        yv[n][j] = t < rows ? y : 0;               // (both sides: nothing that a row behind the end holds enters a product)
+      for (int n = 0; n < NT; ++n)
+        yv[n][j] = WHOLE ? yr[(size_t)j * N + (unsigned)(8 * g4 * N + nc[n])] : yr[(unsigned)(min(8 * g4 + j, left - 1) * N + nc[n])];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (!WHOLE) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {                // (both sides: nothing that a row behind the end holds enters a product)
+        const bool on = 8 * g4 + j < left;
+        xv[j] = on ? xv[j] : 0u;
+#pragma unroll
+        for (int n = 0; n < NT; ++n) yv[n][j] = on ? yv[n][j] : (bf16_t)0;
       }
     }
     u32x4 be, bo;
@@ -316,6 +336,11 @@ __global__ __launch_bounds__(64 * NWG_WAVES) void narrow_wgrad_kernel(const bf16
       acc[0][n] = mfma16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, be), acc[0][n]);
       acc[1][n] = mfma16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, bo), acc[1][n]);
     }
+  };
+#pragma unroll 1
+  for (int t0 = 32 * (NWG_WAVES * part + wave); t0 < rows; t0 += 32 * NWG_WAVES * n_parts) {
+    if (t0 + 32 <= rows) step(t0, std::true_type{}, 32);
+    else step(t0, std::false_type{}, rows - t0);
   }
 #pragma unroll
   for (int n = 0; n < NT; ++n) {
@@ -333,30 +358,81 @@ __global__ __launch_bounds__(64 * NWG_WAVES) void narrow_wgrad_kernel(const bf16
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int n = 16 * wave + 4 * g4 + r;
-    if (n < N) *reinterpret_cast<unsigned*>(dw + (size_t)n * D + d) = pack_bf16x2(e[r], o[r]);
+    if (n >= N) continue;
+    if (SPLIT) *reinterpret_cast<f32x2*>(parts + ((size_t)part * N + n) * D + d) = (f32x2){e[r], o[r]};
+    else *reinterpret_cast<unsigned*>(dw + (size_t)n * D + d) = pack_bf16x2(e[r], o[r]);
   }
+}
+
+// 128 elements of dW a workgroup; its four waves take every fourth part each, added up through LDS in order.
+__global__ __launch_bounds__(256) void narrow_wgrad_sum_kernel(const float* parts, bf16_t* dw, const int n_parts, const int elements) {
+  __shared__ f32x2 sums[4][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int e = 128 * (int)blockIdx.x + 2 * lane;
+  const float* src = parts + min(e, elements - 2);
+  f32x2 a = {0.f, 0.f};
+#pragma unroll 8
+  for (int i = wave; i < n_parts; i += 4) a += *reinterpret_cast<const f32x2*>(src + (size_t)i * elements);
+  sums[wave][lane] = a;
+  __syncthreads();
+  if (wave != 0 || e >= elements) return;
+#pragma unroll
+  for (int w = 1; w < 4; ++w) a += sums[w][lane];
+  *reinterpret_cast<unsigned*>(dw + e) = pack_bf16x2(a[0], a[1]);
+}
+
+// Parts of the rows: eight (one an XCD) until the bytes of X count for more than the partial sums and the rounds of workgroups do.  us with 8 / 16 / 32:
+// 6000 tokens 36 x 1152 11.6 / 14.4 / 15.9, 24 x 768 7.2 / 8.4 / 9.8; 16000 19.1 / 18.5 / 20.8, 10.6 / 11.5 / 10.7; 32768 38.8 / 33.6 / 35.6,
+// 15.7 / 16.8 / 14.1; 65536 73 / 60 / 59, 39 / 42 / 33.
+static int narrow_wgrad_parts(const int64_t rows) {
+  const int64_t steps = (rows + 32 * NWG_WAVES - 1) / (32 * NWG_WAVES);
+  return (int)std::min<int64_t>(rows <= 16384 ? 8 : 32, (steps + 7) / 8 * 8);
 }
 
 }  // namespace natsl
 
 using namespace natsl;
 
-extern "C" int natsl_narrow_wgrad(const void* dy, const void* x, void* dw, int64_t rows, int D, int N, natsl_stream_t stream) {
-  const char* what = "natsl_narrow_wgrad";
+static int narrow_wgrad(const char* what, const void* dy, const void* x, void* dw, const int64_t rows, const int D, const int N, float* parts, hipStream_t s) {
   if (!dy || !x || !dw) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
   if (rows <= 0 || D <= 0 || N <= 0) return fail(NATSL_ERR_INVALID, "%s: non-positive dimension", what);
   if (N > 64 || D % 2 || rows > 0x7fffff00ll) return fail(NATSL_ERR_UNSUPPORTED, "%s: N=%d (up to 64), D=%d (even)", what, N, D);
   if (((uintptr_t)x | (uintptr_t)dw) & 3) return fail(NATSL_ERR_INVALID, "%s: tensors must start on 4 bytes", what);
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)cdiv(D, 32)), wg(64 * NWG_WAVES);
+  const int n_parts = narrow_wgrad_parts(rows);
+  const dim3 grid(parts ? (unsigned)n_parts : (unsigned)cdiv(D, 32), parts ? (unsigned)cdiv(D, 32) : 1u), wg(64 * NWG_WAVES);
   const bf16_t *y = (const bf16_t*)dy, *xx = (const bf16_t*)x;
+#define NATSL_NW(NT)                                                                                                                          \
+  if (parts) hipLaunchKernelGGL((narrow_wgrad_kernel<NT, true>), grid, wg, 0, s, y, xx, (bf16_t*)dw, parts, (int)rows, D, N);                 \
+  else hipLaunchKernelGGL((narrow_wgrad_kernel<NT, false>), grid, wg, 0, s, y, xx, (bf16_t*)dw, parts, (int)rows, D, N);                      \
+  break
   switch (cdiv(N, 16)) {
-    case 1: hipLaunchKernelGGL(narrow_wgrad_kernel<1>, grid, wg, 0, s, y, xx, (bf16_t*)dw, (int)rows, D, N); break;
-    case 2: hipLaunchKernelGGL(narrow_wgrad_kernel<2>, grid, wg, 0, s, y, xx, (bf16_t*)dw, (int)rows, D, N); break;
-    case 3: hipLaunchKernelGGL(narrow_wgrad_kernel<3>, grid, wg, 0, s, y, xx, (bf16_t*)dw, (int)rows, D, N); break;
-    default: hipLaunchKernelGGL(narrow_wgrad_kernel<4>, grid, wg, 0, s, y, xx, (bf16_t*)dw, (int)rows, D, N); break;
+    case 1: NATSL_NW(1);
+    case 2: NATSL_NW(2);
+    case 3: NATSL_NW(3);
+    default: NATSL_NW(4);
   }
+#undef NATSL_NW
+  const int rc = check_launch(what);
+  if (rc != NATSL_OK || !parts) return rc;
+  hipLaunchKernelGGL(narrow_wgrad_sum_kernel, dim3((unsigned)cdiv(N * D, 128)), dim3(256), 0, s, parts, (bf16_t*)dw, n_parts, N * D);
   return check_launch(what);
+}
+
+extern "C" int natsl_narrow_wgrad(const void* dy, const void* x, void* dw, int64_t rows, int D, int N, natsl_stream_t stream) {
+  return narrow_wgrad("natsl_narrow_wgrad", dy, x, dw, rows, D, N, nullptr, reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" size_t natsl_narrow_wgrad_workspace_bytes(int64_t rows, int D, int N) {
+  return rows > 0 && D > 0 && N > 0 ? (size_t)narrow_wgrad_parts(rows) * N * D * sizeof(float) : 0;
+}
+
+extern "C" int natsl_narrow_wgrad_split(const void* dy, const void* x, void* dw, int64_t rows, int D, int N, void* workspace, size_t workspace_bytes,
+                                        natsl_stream_t stream) {
+  const char* what = "natsl_narrow_wgrad_split";
+  const size_t need = natsl_narrow_wgrad_workspace_bytes(rows, D, N);
+  if (!workspace || (uintptr_t)workspace & 7) return fail(NATSL_ERR_INVALID, "%s: the workspace must start on 8 bytes", what);
+  if (workspace_bytes < need) return fail(NATSL_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", what, need, workspace_bytes);
+  return narrow_wgrad(what, dy, x, dw, rows, D, N, (float*)workspace, reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" int natsl_narrow_linear_bwd(const void* dy, const void* w, void* dx, int64_t rows, int D, int N, natsl_stream_t stream) {

@@ -399,6 +399,25 @@ def test_narrow_weight_gradient(rows, D, N):
     assert torch.equal(_front._narrow_wgrad(*many), torch.mm(many[0].t(), many[1]))
 
 
+@pytest.mark.parametrize("rows,D,N", [(1, 32, 2), (31, 96, 12), (257, 130, 17), (2049, 1024, 16), (6000, 1152, 36), (6001, 66, 63), (16385, 64, 44), (20000, 96, 24)])
+def test_narrow_weight_gradient_over_many_rows(rows, D, N):
+    """natsl_narrow_wgrad_split with fewer steps of 256 tokens than parts, with cut ones, with 8 and 32 parts; and weight_grads, which takes it."""
+    from neuralattentionsearchlinear_amd import _capi, _front
+    torch.manual_seed(rows)
+    L, P = _capi.lib(), _capi.ptr
+    x, dy = torch.randn(rows, D, device=DEV).bfloat16(), torch.randn(rows, N, device=DEV).bfloat16()
+    dw = torch.full((N + 1, D), 7., device=DEV).bfloat16()
+    n = L.natsl_narrow_wgrad_workspace_bytes(rows, D, N)
+    ws = torch.empty(n, dtype=torch.uint8, device=DEV)
+    call = lambda size, cols: L.natsl_narrow_wgrad_split(P(dy), P(x), P(dw), rows, D, cols, P(ws), size, _capi.stream_ptr(x.device))
+    _capi.check(call(n, N), "natsl_narrow_wgrad_split")
+    ref = dy.double().t() @ x.double()
+    # (one rounding to bf16; fp32 sums of `rows` products of two normal values in any order)
+    close = lambda got: bool(((got.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * rows ** 0.5).all())
+    assert close(dw[:N]) and bool((dw[N] == 7).all()) and close(_front.weight_grads(x, [None, dy])[1])
+    assert call(n - 1, N) != 0 and call(n, 65) != 0
+
+
 @pytest.mark.parametrize("width", [8, 16, 32, 64, 128, 256, 512])
 @pytest.mark.parametrize("what,silu,T", [('rms', 1, 37), ('l2', 0, 9), ('number', 1, 130)])
 def test_convolution_with_heads_of_any_width(width, what, silu, T):

@@ -142,11 +142,13 @@ struct AnyRaw {             // an element of either type
 struct StepWindow {         // a convolution of width 4 at one channel, every pointer on 8 bytes; x: the new input
   u32x2 e, w;
   bf16_t b, x;
-  NATSL_DEVICE void load(const bf16_t* proj, const void* state, const void* weight, const void* bias, const size_t d, const size_t sd) {
-    x = proj[d];
-    e = reinterpret_cast<const u32x2*>(state)[sd];
-    w = reinterpret_cast<const u32x2*>(weight)[d];
-    b = reinterpret_cast<const bf16_t*>(bias ? bias : weight)[d];
+  // (channel d of sequence row `seq`, the same in every lane: offsets of 32 bits a lane on scalar bases)
+  NATSL_DEVICE void load(const bf16_t* proj, const void* state, const void* weight, const void* bias, const unsigned d, const size_t seq) {
+    auto at = [](const void* p, const unsigned bytes) __attribute__((always_inline)) -> const char* { return reinterpret_cast<const char*>(p) + bytes; };
+    x = *reinterpret_cast<const bf16_t*>(at(proj, 2u * d));
+    e = *reinterpret_cast<const u32x2*>(at(reinterpret_cast<const u32x2*>(state) + seq, 8u * d));
+    w = *reinterpret_cast<const u32x2*>(at(weight, 8u * d));
+    b = *reinterpret_cast<const bf16_t*>(at(bias ? bias : weight, 2u * d));
   }
   NATSL_DEVICE float next(const bool bias, const bool silu) const {
     float a = bias ? bf16_to_f32(b) : 0.f;
@@ -348,7 +350,7 @@ __global__ __launch_bounds__(256) void step_tail_kernel(const StepTail p) {
 // memory one behind another (arguments, windows and flags, keys, the count, the others' results); with many keys by their bytes.
 // Against the three launches: 340M geometry, one sequence of 800 tokens, 9.6 us for 4.3 + 5.4 + 4.8 and two gaps of 3.5; 16 heads of
 // 128/64 and eight sequences of 2000 tokens, 16.7 us for 5 + 13.6 + 5.3 (the three before the changes noted at AnyRaw and wave_sum).  Of the
-// 9.6 us: 2.6 until the first keys are asked for, 1.6 - 2.4 for a chunk and the join of the waves, 0.8 to hand a result over and count it,
+// 9.6 us: 2.2 until the first keys are asked for, 1.6 - 2.4 for a chunk and the join of the waves, 0.8 to hand a result over and count it,
 // 1.4 for the tail, 2 - 3 before and behind the waves.  Workgroups:
 //   mixing logits   (sequence, 256 channels of q): their convolution, and their share of all heads' two logits
 //   recurrence      (sequence, head, 64 state columns), as in attend_and_recur
@@ -413,7 +415,7 @@ NATSL_DEVICE void step_logits(const StepOne& p, const int b, const int chunk, co
   };
   const size_t sd = (size_t)b * KD;
   StepWindow win;
-  win.load(p.m.proj + (size_t)b * p.m.ldp + p.m.cq, s.conv_state_q, s.conv_wq, s.conv_bq, min(d, KD - 1), sd + min(d, KD - 1));
+  win.load(p.m.proj + (size_t)b * p.m.ldp + p.m.cq, s.conv_state_q, s.conv_wq, s.conv_bq, min(d, KD - 1), sd);
   load(wave);
   const bf16_t y = f32_to_bf16(win.next(s.conv_bq != nullptr, s.flags & NATSL_STEP_SILU));
   if (d < KD) win.save(s.conv_out_q, sd + d);
@@ -469,11 +471,11 @@ struct StepToken {
 #pragma unroll
     for (int i = 0; i < C; ++i) {
       const int d = h * DK + 64 * i + lane;
-      wq[i].load(proj + p.m.cq, s.conv_state_q, s.conv_wq, s.conv_bq, d, (size_t)n * KD + d);
-      wk[i].load(proj + p.m.ck, s.conv_state_k, s.conv_wk, s.conv_bk, d, (size_t)n * KD + d);
+      wq[i].load(proj + p.m.cq, s.conv_state_q, s.conv_wq, s.conv_bq, d, (size_t)n * KD);
+      wk[i].load(proj + p.m.ck, s.conv_state_k, s.conv_wk, s.conv_bk, d, (size_t)n * KD);
     }
     const int dv = h * s.V + vc;
-    wv.load(proj + p.m.cv, s.conv_state_v, s.conv_wv, s.conv_bv, dv, (size_t)n * VD + dv);
+    wv.load(proj + p.m.cv, s.conv_state_v, s.conv_wv, s.conv_bv, dv, (size_t)n * VD);
     AnyRaw a_log, dt_bias;
     a_log.load(s.a_log, s.gate_dtype, h);
     dt_bias.load(s.dt_bias, s.gate_dtype, h);
@@ -545,7 +547,7 @@ struct StepRow {
 #pragma unroll
     for (int i = 0; i < C; ++i) {
       const int d = d0 + 64 * i + lane;
-      win[i].load(proj, state, weight, bias, d, seq + d);
+      win[i].load(proj, state, weight, bias, d, seq);
       nw[i].load(norm ? norm : weight, s.norm_dtype, 64 * i + lane);
     }
   }
@@ -577,7 +579,7 @@ struct StepRow {
 };
 
 // What an attending wave of the step makes itself: its query, and in the wave with the last chunk (`mine`) the new key and value.  All
-// inputs are requested before the first chunk is, and used when that is on its way.
+// inputs are requested (request()) before the first chunk is, and used when that is on its way.
 template <int KA, int VA>
 struct StepKeys {
   static constexpr bool STEP = true;
@@ -589,7 +591,8 @@ struct StepKeys {
   StepRow<KA> rq, rk;
   StepRow<VA> rv;
   NATSL_DEVICE StepKeys(const StepOne& p, bf16_t* q, bf16_t* k, bf16_t* v, const int b, const int hq, const bool mine)
-      : p(p), q(q), k(k), v(v), b(b), hq(hq), first(p.a.TK - 1), mine(mine) {
+      : p(p), q(q), k(k), v(v), b(b), hq(hq), first(p.a.TK - 1), mine(mine) {}
+  NATSL_DEVICE void request() {
     const natsl_layer_step& s = p.m.s;
     const size_t KD = (size_t)s.H * s.K, VD = (size_t)s.H * s.V;
     const bf16_t* proj = p.m.proj + (size_t)b * p.m.ldp;
@@ -682,7 +685,7 @@ struct StepLayout {
 };
 
 // Workgroups of step_one_kernel that fit on the chip at once, less those of the logits and the recurrence: what its registers allow a CU
-// (214 with 192-wide states: two; 106 with 64-wide everything: four; else 130 - 166: three.  128-wide keys and values are counted as two, which
+// (236 with 192-wide states: two; 104 with 64-wide everything: four; else 129 - 168: three.  128-wide keys and values are counted as two, which
 // the splits below were measured with).
 static int step_one_slots(const natsl_layer_step& s, const int n_chunks) {
   const int KA = s.H * s.K / s.HQ, VA = s.H * s.V / s.HQ;

@@ -99,7 +99,9 @@ NATSL_DEVICE float sum_squares(const unsigned w, const float acc) {
 // Bound by the instructions of its phases and by the barriers between them (63 % of the wave cycles wait; 2.2 TB/s), so what counts is
 // their number and how many workgroups share a CU: six with PF (26 KB of LDS, 78 registers).  B8 T8192 H16 d128: 124 us; with row
 // norms by separate conversions, branches around the exponentials, the substitution in 16 lanes of every wave and five workgroups a
-// CU 137.  A loop over units with the next rows requested ahead takes registers from it: 150 us at four workgroups.
+// CU 137.  A loop over units with the next rows requested ahead takes registers from it: 150 us at four workgroups.  The gates' and the type's
+// round trips behind the tiles' instead of beside them, and gamma formed by one wave before the first barrier instead of by the idle one
+// behind it: 46.5 us for 42.4 (B4 T4096 H16, without PF), 122 for 117 (B8 T8192 H16, with).
 template <int DK, bool DELTA, bool PF>
 __global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams p) {
   static_assert(DELTA || !PF, "the Mamba form has its own prep");
@@ -145,6 +147,14 @@ __global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams 
   const int t0 = c * C;
   const bool l2 = (p.flags & NATSL_QK_L2NORM) != 0;
 
+  // ---- the per-token inputs and the chunk's type, which one wave each uses further down: asked for here, in every wave and as they lie, so that
+  // their round trips to memory are the tiles' own
+  const bool tok_ok = t0 + lane < len;
+  const size_t gi = (size_t)(bos + min(t0 + lane, len - 1)) * p.H + h;
+  const float g_tok = p.g[gi];
+  const bf16_t b_tok = DELTA ? p.beta[gi] : (bf16_t)0;
+  bf16_t type_lo, type_hi;
+
   // ---- load q, k tiles; row sums of squares from the registers just loaded -----------------
   {
     const int row = tid >> 2, seg = tid & 3;
@@ -160,6 +170,10 @@ __global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams 
       qa[i] = (ok && !PF) ? qr[seg + 4 * i] : z;
       kb[i] = ok ? kr[seg + 4 * i] : z;
     }
+    const int type_size = p.types_dtype == NATSL_F32 ? 4 : 2;
+    const char* type_at = reinterpret_cast<const char*>(p.types) + (((size_t)(bos_nats + t0 / p.block) * p.HN + h / (p.H / p.HN)) * 2 + 1) * type_size;
+    type_lo = *reinterpret_cast<const bf16_t*>(type_at);
+    type_hi = *reinterpret_cast<const bf16_t*>(type_at + type_size - 2);
 #pragma unroll
     for (int i = 0; i < KL; ++i) {
       const u32x4 a = qa[i], b = kb[i];
@@ -171,25 +185,17 @@ __global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams 
         sk = sum_squares(b[j], sk);
       }
     }
-    sq += __shfl_xor(sq, 1); sq += __shfl_xor(sq, 2);
-    sk += __shfl_xor(sk, 1); sk += __shfl_xor(sk, 2);
+    // (lanes 1 and 2 apart, by the quad's permutations)
+    auto quad_sum = [](float x) __attribute__((always_inline)) -> float {
+      x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0xb1, 0xf, 0xf, false));
+      return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x4e, 0xf, 0xf, false));
+    };
+    sq = quad_sum(sq);
+    sk = quad_sum(sk);
     if (seg == 0) {
       rq[row] = (l2 && !PF) ? rsqrtf(sq + 1e-6f) : 1.f;
       rk[row] = l2 ? rsqrtf(sk + 1e-6f) : 1.f;
     }
-  }
-  // ---- gamma = inclusive cumsum of g over the chunk (wave 0), beta -------------------------
-  if (wave == 0) {
-    const bool ok = t0 + lane < len;
-    const size_t gi = (size_t)(bos + t0 + lane) * p.H + h;
-    float x = ok ? p.g[gi] : 0.f;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const float y = __shfl_up(x, d);
-      if (lane >= d) x += y;
-    }
-    gam[lane] = x;
-    if (DELTA) bet[lane] = ok ? bf16_to_f32(p.beta[gi]) : 0.f;
   }
   __syncthreads();
 
@@ -208,9 +214,8 @@ __global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams 
     const int ti = wave >> 1, tj = wave & 1, l32 = lane & 31, hf = lane >> 5;
     const int i = 32 * ti + l32;  // P row owned by this lane
     bf16_t* prow = Pout + ((size_t)((2 * (i >> 4) + tj) * 64 + (i & 15))) * 8;
-    f32x16 gk;
+    f32x16 gk, gq;
     if (ti >= tj) {
-      f32x16 gq;
 #pragma unroll
       for (int r = 0; r < 16; ++r) gk[r] = gq[r] = 0.f;
 #pragma unroll
@@ -225,6 +230,20 @@ __global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams 
           gk = mfma32(ka, kb, gk);  // lane = column j, registers = rows i
         }
       }
+    } else {
+      // meanwhile, the wave above the diagonal: gamma = inclusive cumsum of g over the chunk; beta
+      float x = tok_ok ? g_tok : 0.f;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const float y = __shfl_up(x, d);
+        if (lane >= d) x += y;
+      }
+      gam[lane] = x;
+      if (DELTA) bet[lane] = tok_ok ? bf16_to_f32(b_tok) : 0.f;
+    }
+    // all waves are done reading the q, k tiles before the A blocks overwrite them
+    __syncthreads();
+    if (ti >= tj) {
       if (!PF) {
         // this lane's 16 key tokens are four runs of four: 16-byte reads of their gamma and 1/|k|
         const float gi = gam[i], fi = p.scale * rq[i];
@@ -237,7 +256,11 @@ __global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams 
           const f32x4 gj = *reinterpret_cast<const f32x4*>(gam + j0), rj = *reinterpret_cast<const f32x4*>(rk + j0);
           float pv[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) pv[e] = i >= j0 + e ? fi * rj[e] * gq[4 * q4 + e] * __expf(gi - gj[e]) : 0.f;
+          for (int e = 0; e < 4; ++e) {
+            float a = fi * rj[e] * gq[4 * q4 + e] * __expf(gi - gj[e]);
+            asm volatile("" : "+v"(a));                  // (a select, no branch around the exponential)
+            pv[e] = i >= j0 + e ? a : 0.f;
+          }
           w[q4 & 1][2 * (q4 >> 1)] = pack_bf16x2(pv[0], pv[1]);
           w[q4 & 1][2 * (q4 >> 1) + 1] = pack_bf16x2(pv[2], pv[3]);
         }
@@ -246,8 +269,6 @@ __global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams 
       }
     }
     if (DELTA) {
-      // all waves are done reading the q, k tiles before the A blocks overwrite them
-      __syncthreads();
       if (ti >= tj) {
         const int j = 32 * tj + l32;
         const float gj = gam[j], rkj = rk[j];
@@ -287,8 +308,7 @@ __global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams 
     if (lane == 2) {
       // is this chunk's selector block typed linear?  (kept next to the decay so the scan finds it
       // in the cache line it prefetches anyway)
-      const int hn = h / (p.H / p.HN);
-      Sout[3 * C + 2] = lin_type(p.types, p.types_dtype, ((size_t)(bos_nats + (c * C) / p.block) * p.HN + hn) * 2 + 1) ? 1.f : 0.f;
+      Sout[3 * C + 2] = rintf(__uint_as_float((unsigned)type_hi << 16 | (p.types_dtype == NATSL_F32 ? (unsigned)type_lo : 0u))) == 1.0f ? 1.f : 0.f;
     }
   }
   if (!DELTA) return;

@@ -111,6 +111,12 @@ def test_gdn_key_dim_192_other_shapes():
     _gdn(1, 512, 2, 2, 192, 48, 64, 0.3, True, seed=22, l2=False)    # narrow value dim
 
 
+@pytest.mark.parametrize("H,HN", [(1, 1), (3, 1), (5, 5), (17, 1), (18, 6), (32, 4)])
+def test_mamba_with_any_number_of_heads(H, HN):
+    """The scale vectors are formed for four heads a wave, sixteen a workgroup, with a cut chunk."""
+    _mamba(1, 165, H, HN, 64, 32, 64, 0.4, True, seed=40 + H, h0=True)
+
+
 def test_mamba_key_dim_192():
     _mamba(2, 512, 4, 2, 192, 384, 64, 0.3, True, seed=23, h0=True)
 

@@ -147,7 +147,7 @@ int natsl_softmax_fwd_variant(int B, int T, int HQ, int HKV, int block, int pack
 
 
 /* Backward of the softmax branch: dq [B,T,HQ,K], dk [B,T,HKV,K], dv [B,T,HKV,V] (bf16, summed over the query heads of
- * a kv head) and dnats fp32 [B,TN,HQ], which must be ZERO on entry: per block typed "attention" and query head, the sum
+ * a kv head) and dnats fp32 [B,TN,HQ] (written whole): per block typed "attention" and query head, the sum
  * of the score gradients dS = P (dP - delta) over (keys of the block) x (queries of later blocks), i.e. the gradient
  * with respect to a bias on that block's scores as later blocks see them; blocks not typed attention keep 0 unless
  * flags bit 1 is set (the reference's compute_dnats_for_invalid_blocks_attn, attns.py:1318-1325): then they get
@@ -213,7 +213,8 @@ int natsl_mamba_chunk_fwd(const void* q, const void* k, const void* v, const flo
  * keep its workspace (both forms: the reverse scan reads the scale vectors from it and, for the delta rule, the triangular solves
  * and the intra-chunk matrices).  Inputs as for the forward, plus
  *   v_new [B*T][H][V] (Mamba: v itself), d_o [B*T][H][V] bf16, dht [B][H][K][V] f32 or NULL,
- *   g_block_sums [B][TN][H] f32 = sum of g over every selector block (packed: flat over the sequences' blocks).
+ *   g_block_sums [B][TN][H] f32 = sum of g over every selector block (packed: flat over the sequences' blocks); NULL where these are the
+ *   chunks' (block 64, not packed): then the workspace's.
  * Outputs: dq, dk [B*T][H][K], dv [B*T][H][V] bf16; dg, dbeta (delta rule) [B*T][H] f32; dh0 [B][H][K][V] f32 or NULL;
  *   d_gate [chunks][H] f32 = derivative with respect to a gate on every chunk's state update (the selector's
  *   straight-through gradient for the linear operator, src/nats/ops/common/chunk_o.py:438-443, :487-492, before the sum over
@@ -254,6 +255,9 @@ int natsl_linear_block_sums(const void* workspace, float* g_block_sums, int B, i
 int natsl_block_grads(const void* types, int types_dtype, const float* d_gate, const float* d_rollback, const float* dnats, int HQ, float* dg,
                       void* d_types, int d_types_dtype, int invalid, int B, int T, int H, int HN, int TN, int block, const natsl_seq_row* seqs,
                       int n_seqs, natsl_stream_t stream);
+/* natsl_block_grads and natsl_hard_select_bwd (last_forced) of its d_types in one launch: dlogits [B,TN,HN,2]; logits, types and dlogits in `dtype`. */
+int natsl_block_grads_logits(const void* types, const void* logits, int dtype, const float* d_gate, const float* d_rollback, const float* dnats, int HQ,
+                             float* dg, void* dlogits, int invalid, int B, int T, int H, int HN, int TN, int block, natsl_stream_t stream);
 
 /* Layer tail: y = (rms(x1)*w1*xw[...,0] + rms(x2)*w2*xw[...,1]) * gate*sigmoid(gate) with
  * rms(x) = x*rsqrt(mean(x^2)+eps); x1, x2, gate, y [rows, D] and x_weights [rows, 2] in `dtype`,

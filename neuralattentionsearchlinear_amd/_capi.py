@@ -84,6 +84,7 @@ _SIGNATURES = {
                                      [c_float, c_int, c_int, c_void_p, c_int, c_int, c_void_p]),
     "natsl_linear_block_sums": (c_int, [c_void_p] * 2 + [c_int] * 5 + [c_void_p, c_int, c_int, c_void_p]),
     "natsl_block_grads": (c_int, [c_void_p, c_int] + [c_void_p] * 3 + [c_int, c_void_p, c_void_p] + [c_int] * 8 + [c_void_p, c_int, c_void_p]),
+    "natsl_block_grads_logits": (c_int, [c_void_p] * 2 + [c_int] + [c_void_p] * 3 + [c_int] + [c_void_p] * 2 + [c_int] * 7 + [c_void_p]),
     "natsl_kv_collect": (c_int, [c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_longlong, c_void_p] + [c_int] * 12 + [c_void_p]),
     "natsl_kv_counts": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p] + [c_int] * 4 + [c_void_p]),
     "natsl_kv_flags": (c_int, [c_void_p, c_void_p] + [c_int] * 4 + [c_void_p]),

@@ -205,8 +205,10 @@ def linear_chunk_backward_hip(kind, q, k, v, g, beta, h0, types, scale, block, d
                                                        chunk_states=True, outputs=False, beside=release)
         sp, ns, tot = _seq_args(seqs, NTtot)
         P, L, stream = _capi.ptr, _capi.lib(), _capi.stream_ptr(dev)
-        gsum = torch.empty(B * NB, H, dtype=f32, device=dev)
-        _capi.check(L.natsl_linear_block_sums(P(ws), P(gsum), B, T, H, NB, block, sp, ns, tot, stream), "natsl_linear_block_sums")
+        gsum = None                                        # (blocks of one chunk: the kernels take the workspace's)
+        if block != C or seqs is not None:
+            gsum = torch.empty(B * NB, H, dtype=f32, device=dev)
+            _capi.check(L.natsl_linear_block_sums(P(ws), P(gsum), B, T, H, NB, block, sp, ns, tot, stream), "natsl_linear_block_sums")
         d_states = torch.empty_like(states)
         dq, dk = (torch.empty_like(t) if have is None else have for t, have in zip((qb, kb), onto))
         dv, dv_sum = torch.empty_like(vb), onto[2]

@@ -95,7 +95,7 @@ def prepare_attn_nats_bwd(q, k, v, o, nats_block_types, nats_block_indices, n_na
     H, V = k.shape[2], v.shape[-1]
     TN, HN = ty.shape[1], ty.shape[2]
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    dnats = torch.zeros(B, TN, HQ, dtype=torch.float32, device=q.device)
+    dnats = torch.empty(B, TN, HQ, dtype=torch.float32, device=q.device)
     L = _capi.lib()
     sp, ns, tot = _seq_args(seqs, seqs.total_qtiles if seqs is not None else 0)
     ws_bytes = L.natsl_softmax_bwd_workspace_bytes(B, T, HQ)

@@ -23,11 +23,11 @@
 namespace {
 
 #define NATSL_ENTRIES(X)                                                                                                                   \
-  X(layer_front) X(project) X(project_bwd) X(layer_select) X(hard_select_bwd) X(conv_norm_fwd) X(conv_norm_bwd) X(conv_norm_bwd_workspace_bytes) \
+  X(layer_front) X(project) X(project_bwd) X(layer_select) X(conv_norm_fwd) X(conv_norm_bwd) X(conv_norm_bwd_workspace_bytes) \
   X(mixed_fwd) X(mixed_workspace_bytes) X(norm_gate_logits_fwd) X(norm_gate_logits_bwd) X(norm_gate_bwd_workspace_bytes) X(wgrad)           \
   X(wgrad_workspace_bytes) X(narrow_linear_bwd) X(narrow_wgrad) X(narrow_wgrad_workspace_bytes) X(narrow_wgrad_split) X(gates_bwd) X(gates_bwd_workspace_bytes) X(dx_init) X(softmax_sparse_bwd)  \
-  X(softmax_bwd_workspace_bytes) X(linear_workspace_bytes) X(linear_chunk_states) X(linear_block_sums) X(linear_chunk_bwd_steps)            \
-  X(block_grads) X(order_streams)
+  X(softmax_bwd_workspace_bytes) X(linear_workspace_bytes) X(linear_chunk_states) X(linear_chunk_bwd_steps)            \
+  X(block_grads_logits) X(order_streams)
 
 struct Layer {
 #define X(n) decltype(&natsl_##n) n;
@@ -303,7 +303,7 @@ struct Fork {
 };
 
 struct MixedGrads {
-  T q_a, k_a, v_a, q_l, k_l, v_l, g, beta, types;
+  T q_a, k_a, v_a, q_l, k_l, v_l, g, beta, logits;                // logits: the selector's
 };
 
 MixedGrads mixed_bwd(const Call& c, const Ts& s, const T& do_lin, const T& do_attn, const int invalid_attn, const int invalid_linear) {
@@ -317,7 +317,7 @@ MixedGrads mixed_bwd(const Call& c, const Ts& s, const T& do_lin, const T& do_at
   MixedGrads r;
   // The softmax branch's tensors are made first, on this stream, and live until this stream has its kernels behind it.
   r.q_a = like(q_a); r.k_a = like(k_a); r.v_a = like(v_a);
-  const T dnats = at::zeros({c.B, nb, l.HQ}, c.f32);
+  const T dnats = at::empty({c.B, nb, l.HQ}, c.f32);
   const size_t sb = l.softmax_bwd_workspace_bytes(B, Tn, l.HQ);
   const T sws = c.bytes(sb);
   auto softmax = [&](natsl_stream_t on) {
@@ -344,8 +344,6 @@ MixedGrads mixed_bwd(const Call& c, const Ts& s, const T& do_lin, const T& do_at
                                NATSL_BF16, B, Tn, l.H, l.HN, l.K, l.V, TN, 64, l.scale_linear, flags, at_(ws), n, NATSL_BF16, nullptr, 0, (int)chunks, c.stream,
                                beside ? c.side : nullptr), "natsl_linear_chunk_states");
   }
-  const T gsum = at::empty({c.B * nb, l.H}, c.f32);
-  must(l.linear_block_sums(at_(ws), f_(gsum), B, Tn, l.H, TN, 64, nullptr, 0, (int)chunks, c.stream), "natsl_linear_block_sums");
   const T d_states = like(states);
   r.q_l = like(q_l); r.k_l = like(k_l); r.v_l = like(v_l);
   r.g = at::empty({c.B, c.T_, l.H}, c.f32);
@@ -356,16 +354,16 @@ MixedGrads mixed_bwd(const Call& c, const Ts& s, const T& do_lin, const T& do_at
   }
   const T gate = at::empty({chunks, l.H}, c.f32), rb = like(gate);
   must(l.linear_chunk_bwd_steps(3 + (beside ? 4 : 0) + (delta ? 8 : 0), 0, nullptr, delta, at_(q_l), at_(k_l), at_(v_new), f_(s[G]), at_(s[BETA]), at_(do_lin), nullptr,
-                                at_(states), at_(s[TYPES]), NATSL_BF16, f_(gsum), at_(ws), at_(d_states), f_(parts), at_(r.q_l), at_(r.k_l), at_(r.v_l), f_(r.g),
+                                at_(states), at_(s[TYPES]), NATSL_BF16, nullptr, at_(ws), at_(d_states), f_(parts), at_(r.q_l), at_(r.k_l), at_(r.v_l), f_(r.g),
                                 at_(r.beta), nullptr, f_(gate), f_(rb), B, Tn, l.H, l.HN, l.K, l.V, TN, 64, l.scale_linear, flags, NATSL_BF16, nullptr, 0, (int)chunks,
                                 c.stream), "natsl_linear_chunk_bwd_steps");
   if (beside) {
     softmax(c.side);
     fork.join();
   }
-  r.types = like(s[TYPES]);
-  must(l.block_grads(at_(s[TYPES]), NATSL_BF16, f_(gate), l.decay ? f_(rb) : nullptr, f_(dnats), l.HQ, f_(r.g), at_(r.types), NATSL_BF16, invalid_linear, B, Tn, l.H,
-                     l.HN, TN, 64, nullptr, 0, c.stream), "natsl_block_grads");
+  r.logits = like(s[LOGITS]);
+  must(l.block_grads_logits(at_(s[TYPES]), at_(s[LOGITS]), NATSL_BF16, f_(gate), l.decay ? f_(rb) : nullptr, f_(dnats), l.HQ, f_(r.g), at_(r.logits), invalid_linear,
+                            B, Tn, l.H, l.HN, TN, 64, c.stream), "natsl_block_grads_logits");
   return r;
 }
 
@@ -395,9 +393,7 @@ void backward(const Call& c, const Ts& s, const T& dout, const std::vector<bool>
   }
   const MixedGrads m = mixed_bwd(c, s, do_lin, do_attn, invalid_attn, invalid_linear);
   // selector
-  const T dl = like(s[LOGITS]);
-  must(l.hard_select_bwd(at_(s[LOGITS]), at_(m.types), at_(dl), (int)c.B, (int)blocks_of(c.T_), l.HN, NATSL_BF16, 1, c.stream), "natsl_hard_select_bwd");
-  const T dl2 = dl.view({-1, l.NL});
+  const T dl2 = m.logits.view({-1, l.NL});
   // mixing logits, convolutions
   const T dmix2 = dmix.view({rows, -1}), yq2 = s[Y_Q].view({rows, -1}), dq_mix = narrow_bwd(c, dmix2, w[W_MIX], mix_pays);
   if (want(W_MIX)) grads[1 + W_MIX] = wgrad(c, yq2, dmix2);

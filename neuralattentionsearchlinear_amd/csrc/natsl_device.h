@@ -100,6 +100,15 @@ NATSL_DEVICE float xrow_sum(float x) {
 // exponential (the hardware's differs from it by up to its argument in ulps, and g is kept and summed up in fp32).
 NATSL_DEVICE float softplus_gate(const float x) { return x > 20.f ? x : log1pf(expf(x)); }
 NATSL_DEVICE float sigmoid_gate(const float x) { return 1.f / (1.f + expf(-x)); }
+// the selector's straight-through gradient: d0, d1 of the two types -> of their logits, through the softmax (rounded: as bf16 tensors hold it)
+NATSL_DEVICE void select_grad(const float x0, const float x1, const bool rounded, float& d0, float& d1) {
+  const float mx = fmaxf(x0, x1), e0 = expf(x0 - mx), e1 = expf(x1 - mx);
+  float y0 = e0 / (e0 + e1), y1 = e1 / (e0 + e1);
+  if (rounded) { y0 = bf16_to_f32(f32_to_bf16(y0)); y1 = bf16_to_f32(f32_to_bf16(y1)); }
+  const float m = d0 * y0 + d1 * y1;
+  d0 = y0 * (d0 - m);
+  d1 = y1 * (d1 - m);
+}
 
 // The convolutions' backward: the hardware's reciprocal is within an ulp, __expf's own error is larger, and a division is ten instructions
 NATSL_DEVICE float sigmoid_fast(const float x) { return __builtin_amdgcn_rcpf(1.f + __expf(-x)); }

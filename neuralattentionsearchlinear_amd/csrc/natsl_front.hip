@@ -563,14 +563,11 @@ __global__ __launch_bounds__(256) void select_bwd_kernel(const void* logits, con
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
   const float x0 = ldf(logits, dtype, 2 * i), x1 = ldf(logits, dtype, 2 * i + 1);
-  const float mx = fmaxf(x0, x1), e0 = expf(x0 - mx), e1 = expf(x1 - mx);
-  float y0 = e0 / (e0 + e1), y1 = e1 / (e0 + e1);
-  if (dtype == NATSL_BF16) { y0 = bf16_to_f32(f32_to_bf16(y0)); y1 = bf16_to_f32(f32_to_bf16(y1)); }
   float d0 = ldf(dtypes, dtype, 2 * i), d1 = ldf(dtypes, dtype, 2 * i + 1);
   if (last_forced && (i / HN) % TN == TN - 1) d0 = d1 = 0.f;   // the last block's type is a constant there
-  const float m = d0 * y0 + d1 * y1;
-  stf(dlogits, dtype, 2 * i, y0 * (d0 - m));
-  stf(dlogits, dtype, 2 * i + 1, y1 * (d1 - m));
+  select_grad(x0, x1, dtype == NATSL_BF16, d0, d1);
+  stf(dlogits, dtype, 2 * i, d0);
+  stf(dlogits, dtype, 2 * i + 1, d1);
 }
 
 static int conv_cus() {

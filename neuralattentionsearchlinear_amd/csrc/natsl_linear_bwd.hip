@@ -52,7 +52,8 @@ struct LinBwdParams {
   bf16_t* dv;             // dX [tokens][H][V] (written by the scan)
   const float* dht;       // [B][H][K][V] or null
   float* dh0;             // [B][H][K][V] or null
-  const float* gsum_blk;  // sum of g over every selector block, [B][TN][H]
+  const float* gsum_blk;  // sum of g over every selector block, [B][TN][H], gsum_stride floats apart
+  int gsum_stride;
   const bf16_t* ws_tm;    // the forward's workspace: TmB of every chunk-head in the forward scan's operand order,
   const bf16_t* ws_p;     // P likewise,
   const float* ws_sc;     // and the four scale vectors
@@ -510,7 +511,7 @@ __global__ __launch_bounds__((BwdScanLds<DK, NW>::THREADS)) void linear_bwd_scan
       if (nlast < CB) set_offsets(CB);
     }
   }
-  float gs_next = p.gsum_blk[((size_t)blk0 + ((NT - 1) * CB) / p.block) * p.H + h];
+  float gs_next = p.gsum_blk[(((size_t)blk0 + ((NT - 1) * CB) / p.block) * p.H + h) * p.gsum_stride];
   bool have_pend = false;
 
   for (int c = NT - 1; c >= 0; --c) {
@@ -798,7 +799,7 @@ __global__ __launch_bounds__((BwdScanLds<DK, NW>::THREADS)) void linear_bwd_scan
         const int tk = 16 * (x16 >> 2) + 4 * g4 + (x16 & 3);
         if (tk < nvalid) p.dbeta_parts[((row0 + tk) * p.H + h) * (p.V / 16) + NW * split + wave] = dbeta_part;
       }
-      if (c > 0) gs_next = p.gsum_blk[((size_t)blk0 + ((c - 1) * CB) / p.block) * p.H + h];
+      if (c > 0) gs_next = p.gsum_blk[(((size_t)blk0 + ((c - 1) * CB) / p.block) * p.H + h) * p.gsum_stride];
     }
     if (c % per == 0 && have_pend) {
 #pragma unroll
@@ -1157,7 +1158,7 @@ __global__ __launch_bounds__(256, DK <= 128 ? 2 : 1) void linear_bwd_chunk_kerne
     if (lane < nvalid) p.dg[(row0 + lane) * p.H + h] = x + dG;
     if (lane == 0) {
       p.gate[unit] = gate_sum;
-      p.rb[unit] = want_rb ? __expf(p.gsum_blk[((size_t)blk0 + blk) * p.H + h]) * (red[4] + red[5] + red[6] + red[7]) : 0.f;
+      p.rb[unit] = want_rb ? __expf(p.gsum_blk[(((size_t)blk0 + blk) * p.H + h) * p.gsum_stride]) * (red[4] + red[5] + red[6] + red[7]) : 0.f;
     }
   }
   // dX joins another gradient of the same tensor; what dq, dk are added to, where they are, is fetched before the barrier
@@ -1205,8 +1206,9 @@ struct BlockParams {
   const float* rb;        // [chunk][H] or null (no decay)
   const float* dnats;     // [blocks][HQ] or null: the softmax branch's share
   float* dg;              // [tokens][H]
-  void* d_types;          // [blocks][HN][2]
+  void* d_types;          // [blocks][HN][2], or with logits:
   int d_types_dtype;
+  const void* logits;     // null, or the selector's; d_types is then the gradient of these (the last block's types are constants)
   const SeqRow* seqs;
   int n_seqs, blocks, T, TN, nt, H, HN, HQ, per, invalid, pair_wgs;
   long long tokens;
@@ -1278,14 +1280,23 @@ __global__ __launch_bounds__(256) void block_grads_kernel(const BlockParams p) {
     soft += __shfl_xor(soft, d);
   }
   if (lane == 0) {
-    if (p.d_types_dtype == NATSL_F32) {
-      float* o = reinterpret_cast<float*>(p.d_types) + (size_t)pair * 2;
-      o[0] = (float)soft;
-      o[1] = (float)sum;
-    } else {
+    const bool half = p.d_types_dtype != NATSL_F32;
+    float d0 = (float)soft, d1 = (float)sum;
+    if (p.logits) {
+      if (half) { d0 = bf16_to_f32(f32_to_bf16(d0)); d1 = bf16_to_f32(f32_to_bf16(d1)); }
+      if (j % p.TN == p.TN - 1) d0 = d1 = 0.f;
+      const float x0 = half ? bf16_to_f32(reinterpret_cast<const bf16_t*>(p.logits)[(size_t)pair * 2]) : reinterpret_cast<const float*>(p.logits)[(size_t)pair * 2];
+      const float x1 = half ? bf16_to_f32(reinterpret_cast<const bf16_t*>(p.logits)[(size_t)pair * 2 + 1]) : reinterpret_cast<const float*>(p.logits)[(size_t)pair * 2 + 1];
+      select_grad(x0, x1, half, d0, d1);
+    }
+    if (half) {
       bf16_t* o = reinterpret_cast<bf16_t*>(p.d_types) + (size_t)pair * 2;
-      o[0] = f32_to_bf16((float)soft);
-      o[1] = f32_to_bf16((float)sum);
+      o[0] = f32_to_bf16(d0);
+      o[1] = f32_to_bf16(d1);
+    } else {
+      float* o = reinterpret_cast<float*>(p.d_types) + (size_t)pair * 2;
+      o[0] = d0;
+      o[1] = d1;
     }
   }
 }
@@ -1350,7 +1361,7 @@ extern "C" int natsl_linear_chunk_bwd_steps(int steps, int add, void* dv_sum, in
                                       int H, int HN, int K, int V, int TN, int block, float scale, int flags, int dtype,
                                       const natsl_seq_row* seqs, int n_seqs, int total_chunks, natsl_stream_t stream) {
   const char* what = "natsl_linear_chunk_bwd";
-  if (!q || !k || !v_new || !g || !d_o || !chunk_states || !types || !g_block_sums || !d_chunk_states || !dq || !dk || !dv || !dg ||
+  if (!q || !k || !v_new || !g || !d_o || !chunk_states || !types || (!g_block_sums && (seqs || block != CB)) || !d_chunk_states || !dq || !dk || !dv || !dg ||
       !d_gate || !d_rollback || !workspace || (delta_rule && (!beta || !dbeta || !dbeta_parts)))
     return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
   if (dtype != NATSL_BF16) return fail(NATSL_ERR_UNSUPPORTED, "%s: only bf16 tensors are supported (got dtype %d)", what, dtype);
@@ -1370,7 +1381,11 @@ extern "C" int natsl_linear_chunk_bwd_steps(int steps, int add, void* dv_sum, in
     const size_t units = (size_t)(seqs ? total_chunks : B * cdiv(T, CB)) * (size_t)H;
     p.ws_p = p.ws_tm + units * (CB * CB);
     p.ws_sc = reinterpret_cast<const float*>(p.ws_p + units * (CB * CB));
-  } p.types_dtype = types_dtype;
+    // a block that is a chunk: its sum of g lies with the chunk's scale vectors, and a launch that copies it is 5 to 10 us on the reverse scan's path
+    p.gsum_stride = g_block_sums ? 1 : 4 * CB;
+    if (!g_block_sums) p.gsum_blk = p.ws_sc + 3 * CB + 1;
+  }
+  p.types_dtype = types_dtype;
   p.dq = (bf16_t*)dq; p.dk = (bf16_t*)dk; p.dg = dg; p.dbeta = dbeta; p.dbeta_bf16 = steps >> 3 & 1; p.dbeta_parts = dbeta_parts; p.gate = d_gate; p.rb = d_rollback;
   p.B = B; p.T = T; p.H = H; p.HN = HN; p.V = V; p.TN = TN; p.block = block; p.nt = cdiv(T, CB);
   p.seqs = reinterpret_cast<const SeqRow*>(seqs); p.n_seqs = seqs ? n_seqs : 0; p.total_chunks = seqs ? total_chunks : B * p.nt;
@@ -1425,10 +1440,9 @@ extern "C" int natsl_linear_block_sums(const void* workspace, float* g_block_sum
   return check_launch(what);
 }
 
-extern "C" int natsl_block_grads(const void* types, int types_dtype, const float* d_gate, const float* d_rollback, const float* dnats, int HQ, float* dg,
-                                 void* d_types, int d_types_dtype, int invalid, int B, int T, int H, int HN, int TN, int block,
-                                 const natsl_seq_row* seqs, int n_seqs, natsl_stream_t stream) {
-  const char* what = "natsl_block_grads";
+static int block_grads(const void* types, int types_dtype, const float* d_gate, const float* d_rollback, const float* dnats, int HQ, float* dg,
+                       void* d_types, int d_types_dtype, const void* logits, int invalid, int B, int T, int H, int HN, int TN, int block,
+                       const natsl_seq_row* seqs, int n_seqs, natsl_stream_t stream, const char* what) {
   if (!types || !d_gate || !d_types || (d_rollback && !dg)) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
   if ((types_dtype != NATSL_BF16 && types_dtype != NATSL_F32) || (d_types_dtype != NATSL_BF16 && d_types_dtype != NATSL_F32))
     return fail(NATSL_ERR_UNSUPPORTED, "%s: block types must be f32 or bf16", what);
@@ -1436,10 +1450,23 @@ extern "C" int natsl_block_grads(const void* types, int types_dtype, const float
   if (const int rc = block_params(p, B, T, H, HN, TN, block, seqs, n_seqs, what)) return rc;
   if (dnats && (HQ <= 0 || HQ % HN)) return fail(NATSL_ERR_INVALID, "%s: HQ=%d must be a multiple of HN=%d", what, HQ, HN);
   p.types = types; p.types_dtype = types_dtype; p.gate = d_gate; p.rb = d_rollback; p.dnats = dnats; p.HQ = HQ; p.dg = dg;
-  p.d_types = d_types; p.d_types_dtype = d_types_dtype; p.invalid = invalid;
+  p.d_types = d_types; p.d_types_dtype = d_types_dtype; p.logits = logits; p.invalid = invalid;
   p.pair_wgs = (int)(((long long)p.blocks * HN + 3) / 4);
   const long long grid = p.pair_wgs + (d_rollback ? (p.tokens * H + 255) / 256 : 0);
   if (grid > 0x7fffffffll) return fail(NATSL_ERR_UNSUPPORTED, "%s: problem too large", what);
   hipLaunchKernelGGL(block_grads_kernel, dim3((unsigned)grid), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), p);
   return check_launch(what);
+}
+extern "C" int natsl_block_grads(const void* types, int types_dtype, const float* d_gate, const float* d_rollback, const float* dnats, int HQ, float* dg,
+                                 void* d_types, int d_types_dtype, int invalid, int B, int T, int H, int HN, int TN, int block,
+                                 const natsl_seq_row* seqs, int n_seqs, natsl_stream_t stream) {
+  return block_grads(types, types_dtype, d_gate, d_rollback, dnats, HQ, dg, d_types, d_types_dtype, nullptr, invalid, B, T, H, HN, TN, block, seqs, n_seqs,
+                     stream, "natsl_block_grads");
+}
+extern "C" int natsl_block_grads_logits(const void* types, const void* logits, int dtype, const float* d_gate, const float* d_rollback, const float* dnats,
+                                        int HQ, float* dg, void* dlogits, int invalid, int B, int T, int H, int HN, int TN, int block,
+                                        natsl_stream_t stream) {
+  const char* what = "natsl_block_grads_logits";
+  if (!logits) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
+  return block_grads(types, dtype, d_gate, d_rollback, dnats, HQ, dg, dlogits, dtype, logits, invalid, B, T, H, HN, TN, block, nullptr, 0, stream, what);
 }

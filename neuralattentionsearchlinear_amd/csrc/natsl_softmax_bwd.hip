@@ -27,7 +27,7 @@ struct SoftmaxBwdParams {
   const bf16_t *q, *k, *v, *o, *dout;
   const float* lse;
   bf16_t *dq, *dk, *dv;
-  float* dnats;   // [B, TN, HQ], zero on entry
+  float* dnats;   // [B, TN, HQ], zeroed by the dQ kernel, added to by the dk/dv kernel
   float* ndelta;  // [B, T, HQ] workspace: -delta (written by the dQ kernel, read by the dk/dv kernel)
   int* queue;     // [8] workspace: next unit of each XCD's list for the dk/dv kernel, zeroed by the dQ kernel
   const void* types;
@@ -109,6 +109,8 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const SoftmaxBwdParams p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hf = lane >> 5;
   if (blockIdx.x == 0 && tid < 8) p.queue[tid] = 0;   // the dk/dv kernel's work queues (it runs after this kernel)
+  // ... and what it adds to (a fill kernel in front of this one is 5 us of a backward)
+  for (size_t i = (size_t)blockIdx.x * 256 + tid; i < (size_t)p.B * p.TN * p.HQ; i += (size_t)gridDim.x * 256) p.dnats[i] = 0.f;
   int n, hq, tile, len, bos, bos_nats;
   if (p.seqs == nullptr) {
     const int nq_tiles = (p.T + QTILE - 1) / QTILE;

@@ -153,6 +153,38 @@ def test_softmax_bwd_repeatable_and_workspace_reuse():
         assert float((outs[0][3] - outs[rep][3]).abs().max()) <= 1e-3 * float(outs[0][3].abs().max() + 1.0)
 
 
+@pytest.mark.parametrize("B,T,HQ,HN,block,K,V", [(1, 1, 1, 1, 64, 64, 64), (1, 130, 3, 1, 64, 128, 128), (2, 640, 4, 2, 128, 64, 128), (3, 4097, 2, 2, 64, 128, 64)])
+def test_softmax_bwd_writes_dnats_whole(B, T, HQ, HN, block, K, V):
+    """What lies in dnats before the call does not matter: blocks that nothing adds to are 0, the others what they are on cleared memory (up to
+    the order of their float sums)."""
+    from neuralattentionsearchlinear_amd import _capi, nats_util
+    from neuralattentionsearchlinear_amd.attns import parallel_attn_nats_fwd
+    q, k, v = (t.to(DEV) for t in make_qkv(B, T, HQ, K, V, 41, HQ=HQ))
+    do = torch.randn(B, T, HQ, V, generator=torch.Generator().manual_seed(42)).bfloat16().to(DEV)
+    TN, scale = -(-T // block), K ** -0.5
+    ty = make_types(B, TN, HN, 0.4, 43, torch.bfloat16).to(DEV)
+    r = nats_util.route(ty, T, block)
+    o, lse, _ = parallel_attn_nats_fwd(q, k, v, ty, r['nats_block_indices'], None, scale, block,
+                                       compute_incomplete_chunk_scores=True, n_nats_blocks=r['n_nats_blocks'])
+    L = _capi.lib()
+    n = L.natsl_softmax_bwd_workspace_bytes(B, T, HQ)
+    ws = torch.empty(n, dtype=torch.uint8, device=DEV)
+    got = []
+    for before in (0.0, float('nan')):
+        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+        dn = torch.full((B, TN, HQ), before, dtype=torch.float32, device=DEV)
+        _capi.check(L.natsl_softmax_sparse_bwd(
+            _capi.ptr(q), _capi.ptr(k), _capi.ptr(v), _capi.ptr(o), _capi.ptr(lse), _capi.ptr(do), _capi.ptr(dq), _capi.ptr(dk), _capi.ptr(dv),
+            _capi.ptr(dn), _capi.ptr(ty), _capi.dtype_code(ty.dtype), _capi.ptr(r['nats_block_indices']), _capi.ptr(r['n_nats_blocks']), B, T, HQ,
+            HQ, HN, K, V, TN, block, float(scale), 1, _capi.dtype_code(q.dtype), _capi.ptr(ws), n, None, 0, 0, 0, _capi.stream_ptr(q.device)),
+            "natsl_softmax_sparse_bwd")
+        torch.cuda.synchronize()
+        got.append(dn)
+    not_attention = (ty[..., 0] == 0).repeat_interleave(HQ // HN, 2)
+    assert float(got[1][not_attention].abs().sum()) == 0.0
+    assert float((got[0] - got[1]).abs().max()) <= 1e-3 * float(got[0].abs().max() + 1.0)
+
+
 @pytest.mark.parametrize("same_block", [True, False])
 @pytest.mark.parametrize("K,V", [(128, 128), (64, 128)])
 def test_softmax_bwd_dnats_of_blocks_that_are_not_attention(K, V, same_block):

@@ -96,6 +96,39 @@ NATSL_DEVICE float xrow_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// sums over the `lanes` adjacent lanes (a power of two, the same for the wave) that share a head row
+NATSL_DEVICE void group_sum2(float& a, float& b, const int lanes) {
+  auto add = [&](auto c) __attribute__((always_inline)) {
+    a += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(a), decltype(c)::value, 0xf, 0xf, true));
+    b += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(b), decltype(c)::value, 0xf, 0xf, true));
+  };
+  auto first = [&]() __attribute__((always_inline)) {
+    add(std::integral_constant<int, 0xb1>{});    // lane ^ 1
+    add(std::integral_constant<int, 0x4e>{});    // lane ^ 2
+    add(std::integral_constant<int, 0x141>{});   // 7 - lane: the other four, which all hold their sum
+  };
+  if (lanes == 8) {
+    first();
+  } else if (lanes >= 16) {
+    first();
+    add(std::integral_constant<int, 0x140>{});   // 15 - lane
+    if (lanes >= 32) {
+      auto both = [](const u32x2 r) __attribute__((always_inline)) { return __uint_as_float(r[0]) + __uint_as_float(r[1]); };
+      a = both(__builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(a), false, false));
+      b = both(__builtin_amdgcn_permlane16_swap(__float_as_uint(b), __float_as_uint(b), false, false));
+      if (lanes == 64) {
+        a = xhalf_sum(a);
+        b = xhalf_sum(b);
+      }
+    }
+  } else {
+    for (int d = 1; d < lanes; d <<= 1) {
+      a += __shfl_xor(a, d);
+      b += __shfl_xor(b, d);
+    }
+  }
+}
+
 // The layers' gates, shared by whole sequences and single steps: both write rows of the same cache, so both take the library's
 // exponential (the hardware's differs from it by up to its argument in ulps, and g is kept and summed up in fp32).
 NATSL_DEVICE float softplus_gate(const float x) { return x > 20.f ? x : log1pf(expf(x)); }

@@ -117,33 +117,58 @@ __global__ __launch_bounds__(256) void norm_gate_bwd_kernel(const bf16_t* x1, co
     for (int j = 0; j < 8; ++j) { dwa[u][j] = 0.f; dwb[u][j] = 0.f; }
   }
   const long long first = (long long)blockIdx.x * rows_per_wg;
+  // A row is requested while the one before it is worked on, with the mixing weights, which were a second round trip behind the sums (rows of
+  // several pieces a lane have no registers for that).  us, before / after, with the sums across lanes through LDS before: 9324 rows of 128
+  // 17.6 / 13.9, 108000 51.5 / 47.0, 393216 138.4 / 137.7 (5.1 TB/s: bytes); 54001 of 192 44.6 / 44.0, 20001 of 384 39.7 / 37.8.  More
+  // rows a workgroup, for fewer partial sums, is slower there (146.6).
+  constexpr bool AHEAD = PER == 1;
+  u32x4 in[PER][4];
+  unsigned in_w = 0;
+  auto request = [&](const int it) __attribute__((always_inline)) {
+    const long long row = first + it * G + grp, r = row < rows ? row : rows - 1;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const size_t off = (size_t)r * D + (u * LANES + seg) * 8;
+      in[u][0] = *reinterpret_cast<const u32x4*>(x1 + off);
+      in[u][1] = *reinterpret_cast<const u32x4*>(x2 + off);
+      in[u][2] = *reinterpret_cast<const u32x4*>(gate + off);
+      in[u][3] = *reinterpret_cast<const u32x4*>(dy + off);
+    }
+    if (AHEAD) in_w = (unsigned)xw[r * 2] | (unsigned)xw[r * 2 + 1] << 16;
+  };
+  if (AHEAD) request(0);
   for (int it = 0; it * G < rows_per_wg; ++it) {
     const long long row = first + it * G + grp;
-    // (a lane group leaves the loop as a whole: the shuffles below stay inside a group)
-    if (it * G + grp >= rows_per_wg || row >= rows) continue;
+    // (a lane group leaves the loop as a whole: the sums below stay inside a group)
+    if (row >= rows) continue;
+    if (!AHEAD) request(it);
     float a[PER][8], b[PER][8], g[PER][8], d[PER][8];
     float sa = 0.f, sb = 0.f;
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
-      const size_t off = (size_t)row * D + (u * LANES + seg) * 8;
-      unpack8(*reinterpret_cast<const u32x4*>(x1 + off), a[u]);
-      unpack8(*reinterpret_cast<const u32x4*>(x2 + off), b[u]);
-      unpack8(*reinterpret_cast<const u32x4*>(gate + off), g[u]);
-      unpack8(*reinterpret_cast<const u32x4*>(dy + off), d[u]);
+      unpack8(in[u][0], a[u]);
+      unpack8(in[u][1], b[u]);
+      unpack8(in[u][2], g[u]);
+      unpack8(in[u][3], d[u]);
+    }
+    float xa, xb;
+    if constexpr (AHEAD) {
+      xa = bf16_to_f32((bf16_t)(in_w & 0xffffu));
+      xb = bf16_to_f32((bf16_t)(in_w >> 16));
+      if (dlogits) mix_softmax(xa, xb);
+    }
+    if (AHEAD && (it + 1) * G < rows_per_wg) request(it + 1);
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         sa += a[u][j] * a[u][j];
         sb += b[u][j] * b[u][j];
       }
     }
-#pragma unroll
-    for (int dd = 1; dd < LANES; dd <<= 1) {
-      sa += __shfl_xor(sa, dd);
-      sb += __shfl_xor(sb, dd);
-    }
+    group_sum2(sa, sb, LANES);
     const float ra = rsqrtf(sa / D + eps), rb = rsqrtf(sb / D + eps);
-    float xa, xb;
-    mix_weights(xw, row, dlogits != nullptr, xa, xb);
+    if constexpr (!AHEAD) mix_weights(xw, row, dlogits != nullptr, xa, xb);
     // pass 2: a, b become the normalised inputs, d becomes dmix, g becomes dgate / mix's factor
     float pa = 0.f, pb = 0.f;
 #pragma unroll
@@ -162,11 +187,7 @@ __global__ __launch_bounds__(256) void norm_gate_bwd_kernel(const bf16_t* x1, co
         b[u][j] = n2;
         d[u][j] = dmix;
       }
-#pragma unroll
-    for (int dd = 1; dd < LANES; dd <<= 1) {
-      pa += __shfl_xor(pa, dd);
-      pb += __shfl_xor(pb, dd);
-    }
+    group_sum2(pa, pb, LANES);
     if (seg == 0) {
       if (dlogits) {
         const float m = pa * xa + pb * xb;

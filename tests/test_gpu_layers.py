@@ -56,6 +56,26 @@ def test_norm_gate_backward(D, wdtype):
         assert rel_l2(got, r) <= 5e-3, f"{name}: rel-L2 {rel_l2(got, r):.3e}"
 
 
+@pytest.mark.parametrize("D", [32, 64, 96, 128, 192, 256, 384, 512])
+@pytest.mark.parametrize("rows", [1, 15, 17, 127, 129, 257])
+def test_norm_gate_backward_of_any_number_of_rows(D, rows):
+    """A row's gradients do not depend on the rows behind it: the first rows of a larger call, bit for bit (what is requested ahead past the last
+    row is not used)."""
+    from neuralattentionsearchlinear_amd.modules import two_inputs_rms_norm_gated
+    g = torch.Generator().manual_seed(D + rows)
+    x1, x2, gate, dy = (torch.randn(300, D, generator=g).bfloat16() for _ in range(4))
+    xw = torch.softmax(torch.randn(300, 2, generator=g), -1).bfloat16()
+    w1, w2 = (1 + 0.1 * torch.randn(D, generator=g)).bfloat16(), (1 + 0.1 * torch.randn(D, generator=g)).bfloat16()
+    grads = []
+    for n in (rows, 300):
+        dev = [t[:n].clone().to(DEV).view(1, n, 1, -1).requires_grad_(True) for t in (x1, x2, gate, xw)]
+        two_inputs_rms_norm_gated(*dev, w1.to(DEV), w2.to(DEV), 1e-5).backward(dy[:n].clone().to(DEV).view(1, n, 1, D))
+        grads.append([t.grad for t in dev])
+    torch.cuda.synchronize()
+    for name, a, b in zip(['dx1', 'dx2', 'dgate', 'dx_weights'], *grads):
+        assert torch.equal(a, b[:, :rows]), name
+
+
 # head geometry of the two published model configurations (experiments/configs/natsl_340M.json, natsl_760M.json):
 # linear heads K 128 / V 256 resp. K 192 / V 384, attention view K 64 / V 128 in both
 PUBLISHED = {'340M': dict(hidden_size=1024, head_dim=128, num_heads=6, num_attn_heads=12, norm_eps=1e-6),

@@ -443,6 +443,7 @@ class _MixedFunction(torch.autograd.Function):
             saved += list(aux['linear_saved'])
             ctx.n_linear_saved = len(aux['linear_saved'])
         ctx.save_for_backward(*saved)
+        ctx.set_materialize_grads(False)        # (a final state that nothing follows is neither filled with zeros nor read)
         if ht is None:
             return o_lin, o_attn, None
         return o_lin, o_attn, ht

@@ -357,3 +357,44 @@ def test_recomputed_chunk_states_side_by_side(kind, T, K, V, block, shared, pack
         for i, (a, b) in enumerate(zip(got[:-1], want[:-1])):
             assert torch.equal(a, b), (i, side, keep)
         assert rel_l2(got[-1], want[-1]) < 1e-2              # (block types: one atomic addition per unit, in any order)
+
+
+@pytest.mark.parametrize("kind", ['gdn', 'mamba'])
+@pytest.mark.parametrize("used", ['linear', 'attention', 'state', 'linear and attention'])
+@pytest.mark.parametrize("shared", [False, True])
+def test_outputs_without_a_gradient(kind, used, shared):
+    """An output that nothing follows gives the gradients that zeros for it give."""
+    from neuralattentionsearchlinear_amd.mixed_attn_gdn import nats_mixed_attn_gdn
+    from neuralattentionsearchlinear_amd.mixed_attn_mamba import nats_mixed_attn_mamba
+    B, T, H, K, V = 1, 320, 2, 64, 64
+    q, k, v = make_qkv(B, T, H, K, V, 51)
+    if kind == 'mamba':
+        q, k = F.normalize(q.float(), dim=-1).bfloat16(), F.normalize(k.float(), dim=-1).bfloat16()
+    g, beta = make_gates(B, T, H, 52)
+    ty = make_types(B, T // 64, H, 0.4, 53, torch.bfloat16)
+    gen = torch.Generator().manual_seed(54)
+    cot = {'linear': torch.randn(B, T, H, V, generator=gen), 'attention': torch.randn(B, T, H, V, generator=gen), 'state': torch.randn(B, H, K, V, generator=gen)}
+    got = []
+    for whole in (False, True):
+        leaf = lambda t: t.clone().to(DEV).requires_grad_(True)
+        leaves = [leaf(t) for t in (q, k, v)]
+        lin = leaves if shared else [leaf(t) for t in (q, k, v)]
+        gd, bd, tyd = leaf(g), leaf(beta), leaf(ty)
+        nb = ty.to(torch.int32).sum(1).to(DEV)
+        if kind == 'gdn':
+            outs = nats_mixed_attn_gdn(*leaves, *lin, None, gd, bd, tyd, nb, ops_for_incomplete_chunks='all', output_final_state_gated_delta=True,
+                                       decay_for_non_gdn_blocks=True)
+        else:
+            outs = nats_mixed_attn_mamba(*leaves, *lin, None, gd, tyd, nb, scale_lattn=1.0, ops_for_incomplete_chunks='all', output_final_state_mamba=True,
+                                         decay_for_non_mamba_blocks=True)
+        pairs = [(o, (c if n in used else torch.zeros_like(c)).to(DEV).to(o.dtype)) for o, (n, c) in zip(outs, cot.items()) if whole or n in used]
+        torch.autograd.backward([o for o, _ in pairs], [c for _, c in pairs])
+        torch.cuda.synchronize()
+        # (the selector's gradient is last: its sums over the keys' units are in no fixed order)
+        got.append([t.grad for t in (leaves if shared else leaves + lin)] + [gd.grad] + ([bd.grad] if kind == 'gdn' else []) + [tyd.grad])
+    for i, (a, b) in enumerate(zip(*got)):
+        a, b = (torch.zeros_like(gd) if t is None else t for t in (a, b))
+        if i == len(got[0]) - 1:
+            assert float((a.float() - b.float()).abs().max()) <= 1e-2 * float(b.float().abs().max()) + 1e-6
+        else:
+            assert torch.equal(a, b), i

@@ -51,18 +51,13 @@ int linear_fwd(bool delta, const void* q, const void* k, const void* v, const fl
                int n_seqs, int total_units, natsl_stream_t stream, const BesideScan* beside);
 
 // The softmax branch behind its C entries (natsl_softmax.hip); queue: SOFTMAX_QUEUE_BYTES of this call's own for the persistent kernel's
-// work queues, or null (see launch_softmax_stream); cleared: they have been zeroed on `stream` by route().
+// work queues, or null (see launch_softmax_stream).
 constexpr size_t SOFTMAX_QUEUE_BYTES = 64;
 enum SoftmaxUse { SOFTMAX_PER_TILE, SOFTMAX_ENTRY, SOFTMAX_OPERATOR };   // who calls: which kernel runs depends on it (see softmax_variant)
 int softmax_fwd(const void* q, const void* k, const void* v, void* o, float* lse, const void* types, int types_dtype,
                 const int32_t* nats_block_indices, const int32_t* n_nats_blocks, int B, int T, int HQ, int HKV, int HN, int K, int V, int TN,
                 int block, float scale, int same_block_visible, int dtype, const natsl_seq_row* seqs, int n_seqs, int total_units,
-                natsl_stream_t stream, SoftmaxUse use, unsigned* queue, bool cleared);
-// natsl_route (natsl_route.hip); queue: SOFTMAX_QUEUE_BYTES that the same launch zeroes, or null.  As a fill kernel of its own in front of the
-// softmax kernel that costs 5 us of an operator.
-int route(const void* types, int types_dtype, int B, int TN, int HN, int T, int block, int32_t* nats_block_indices, int32_t* n_nats_blocks,
-          int64_t* linear_chunk_offsets, int32_t* chunk_indices_linear, int64_t* starting_h_idx, int64_t* attn_n_iters,
-          const natsl_seq_row* seqs, int n_seqs, natsl_stream_t stream, unsigned* queue);
+                natsl_stream_t stream, SoftmaxUse use, unsigned* queue);
 
 inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 

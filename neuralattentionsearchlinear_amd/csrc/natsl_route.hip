@@ -186,9 +186,8 @@ constexpr int ROUTE_MAX_TN = 16384;
 
 __global__ __launch_bounds__(256) void route_kernel(const void* types, int dtype, int TN, int HN, int T, int block, int32_t* idx,
                                                     int32_t* nblk, int64_t* starting_h_idx, int64_t* attn_n_iters,
-                                                    const SeqRow* seqs, int n_seqs, unsigned* queue) {
+                                                    const SeqRow* seqs, int n_seqs) {
   extern __shared__ int dyn[];  // [2][tn+1] exclusive prefix counts
-  if (queue && blockIdx.x == 0 && threadIdx.x < SOFTMAX_QUEUE_BYTES / sizeof(unsigned)) queue[threadIdx.x] = 0u;
   const int n = blockIdx.x / HN, hn = blockIdx.x % HN;
   int bos_nats, tn, len;
   if (seqs == nullptr) {
@@ -346,10 +345,11 @@ extern "C" int natsl_layer_select(const void* logits, void* types, void* raw_typ
   return check_launch(what);
 }
 
-namespace natsl {
-int route(const void* types, int types_dtype, int B, int TN, int HN, int T, int block, int32_t* nats_block_indices, int32_t* n_nats_blocks,
-          int64_t* linear_chunk_offsets, int32_t* chunk_indices_linear, int64_t* starting_h_idx, int64_t* attn_n_iters,
-          const natsl_seq_row* seqs, int n_seqs, natsl_stream_t stream, unsigned* queue) {
+extern "C" int natsl_route(const void* types, int types_dtype, int B, int TN, int HN, int T, int block,
+                           int32_t* nats_block_indices, int32_t* n_nats_blocks, int64_t* linear_chunk_offsets,
+                           int32_t* chunk_indices_linear, int64_t* starting_h_idx, int64_t* attn_n_iters,
+                           const natsl_seq_row* seqs, int n_seqs, int total_units, natsl_stream_t stream) {
+  (void)total_units;
   if (!types) return fail(NATSL_ERR_INVALID, "route: null types pointer");
   if (B <= 0 || TN <= 0 || HN <= 0 || T <= 0) return fail(NATSL_ERR_INVALID, "route: non-positive dimension");
   if (types_dtype != NATSL_BF16 && types_dtype != NATSL_F32) return fail(NATSL_ERR_UNSUPPORTED, "route: dtype %d", types_dtype);
@@ -363,7 +363,7 @@ int route(const void* types, int types_dtype, int B, int TN, int HN, int T, int 
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const size_t lds = (size_t)2 * (TN + 1) * sizeof(int);
   hipLaunchKernelGGL(route_kernel, dim3(n * HN), dim3(256), lds, s, types, types_dtype, TN, HN, T, block, nats_block_indices,
-                     n_nats_blocks, starting_h_idx, attn_n_iters, reinterpret_cast<const SeqRow*>(seqs), n_seqs, queue);
+                     n_nats_blocks, starting_h_idx, attn_n_iters, reinterpret_cast<const SeqRow*>(seqs), n_seqs);
   int rc = check_launch("natsl_route");
   if (rc != NATSL_OK) return rc;
   if (linear_chunk_offsets || chunk_indices_linear) {
@@ -371,14 +371,4 @@ int route(const void* types, int types_dtype, int B, int TN, int HN, int T, int 
     rc = check_launch("natsl_route(offsets)");
   }
   return rc;
-}
-}  // namespace natsl
-
-extern "C" int natsl_route(const void* types, int types_dtype, int B, int TN, int HN, int T, int block,
-                           int32_t* nats_block_indices, int32_t* n_nats_blocks, int64_t* linear_chunk_offsets,
-                           int32_t* chunk_indices_linear, int64_t* starting_h_idx, int64_t* attn_n_iters,
-                           const natsl_seq_row* seqs, int n_seqs, int total_units, natsl_stream_t stream) {
-  (void)total_units;
-  return route(types, types_dtype, B, TN, HN, T, block, nats_block_indices, n_nats_blocks, linear_chunk_offsets, chunk_indices_linear, starting_h_idx,
-               attn_n_iters, seqs, n_seqs, stream, nullptr);
 }

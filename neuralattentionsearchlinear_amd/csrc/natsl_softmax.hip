@@ -1619,8 +1619,8 @@ static int launch_softmax(const SoftmaxParams& p, hipStream_t stream) {
   return check_launch("natsl_softmax_sparse_fwd");
 }
 
-// Ticket counters of the persistent kernel.  They are zeroed on the launch's stream, by the mixed operator's routing launch or by a fill kernel right
-// before it (a kernel, not hipMemsetAsync, so that both can be captured into a HIP graph and replayed); nothing is left to set back afterwards, so a launch
+// Ticket counters of the persistent kernel.  They are zeroed on the launch's stream by a fill kernel right before it (a kernel, not
+// hipMemsetAsync, so that both can be captured into a HIP graph and replayed); nothing is left to set back afterwards, so a launch
 // that was cut short cannot poison a later one.  Three homes:
 //  * the mixed operator's launches have theirs in the call's own workspace;
 //  * natsl_softmax_sparse_fwd has no workspace.  Its whole-tile launches rotate through STREAM_SLOTS slots of library-owned memory.
@@ -1670,14 +1670,13 @@ static const StreamDevice* stream_device(int* rc) {
 }
 
 template <int DK, int DV, bool RAGGED, bool DEALT>
-static int launch_softmax_stream(const SoftmaxParams& p, const StreamDevice* d, unsigned* queue, bool cleared, hipStream_t stream) {
+static int launch_softmax_stream(const SoftmaxParams& p, const StreamDevice* d, unsigned* queue, hipStream_t stream) {
   static std::atomic<unsigned long long> reserved{0};
   const size_t lds = (size_t)(4 * 64 * (DK + DV) + 64 * DV) * sizeof(bf16_t) + 1024;  // four K and four V tiles, the output's staging area; 1 KiB aligned
   auto kern = softmax_stream_kernel<DK, DV, RAGGED, DEALT>;
   if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, lds, "softmax")) return rc;
-  cleared = cleared && queue;
   if (!RAGGED && !queue) queue = d->queues + (size_t)(stream_launches.fetch_add(1) % STREAM_SLOTS) * STREAM_SLOT_WORDS;
-  if (queue && !cleared) hipLaunchKernelGGL(stream_queue_clear_kernel, dim3(1), dim3(64), 0, stream, queue);
+  if (queue) hipLaunchKernelGGL(stream_queue_clear_kernel, dim3(1), dim3(64), 0, stream, queue);
   hipLaunchKernelGGL(kern, dim3((unsigned)d->cus), dim3(512), lds, stream, p, queue);
   return check_launch("natsl_softmax_sparse_fwd");
 }
@@ -1727,7 +1726,7 @@ static_assert(SOFTMAX_QUEUE_BYTES == STREAM_SLOT_WORDS * sizeof(unsigned), "the 
 int softmax_fwd(const void* q, const void* k, const void* v, void* o, float* lse, const void* types, int types_dtype,
                 const int32_t* nats_block_indices, const int32_t* n_nats_blocks, int B, int T, int HQ, int HKV, int HN, int K,
                 int V, int TN, int block, float scale, int same_block_visible, int dtype, const natsl_seq_row* seqs,
-                int n_seqs, int total_units, natsl_stream_t stream, SoftmaxUse use, unsigned* queue, bool cleared) {
+                int n_seqs, int total_units, natsl_stream_t stream, SoftmaxUse use, unsigned* queue) {
   if (!q || !k || !v || !o || !lse || !types || !nats_block_indices || !n_nats_blocks)
     return fail(NATSL_ERR_INVALID, "softmax: null pointer argument");
   if (dtype != NATSL_BF16) return fail(NATSL_ERR_UNSUPPORTED, "softmax: only bf16 tensors are supported (got dtype %d)", dtype);
@@ -1759,8 +1758,8 @@ int softmax_fwd(const void* q, const void* k, const void* v, void* o, float* lse
   p.variant = variant == NATSL_SOFTMAX_TILE_128 ? 4 : 8;
 #define NATSL_SM(KK, VV)                                              \
   if (K == KK && V == VV) {                                           \
-    if (sd && !seqs && T % 256 == 0) return launch_softmax_stream<KK, VV, false, false>(p, sd, queue, cleared, s); \
-    if (sd) return queue ? launch_softmax_stream<KK, VV, true, false>(p, sd, queue, cleared, s) : launch_softmax_stream<KK, VV, true, true>(p, sd, nullptr, false, s); \
+    if (sd && !seqs && T % 256 == 0) return launch_softmax_stream<KK, VV, false, false>(p, sd, queue, s); \
+    if (sd) return queue ? launch_softmax_stream<KK, VV, true, false>(p, sd, queue, s) : launch_softmax_stream<KK, VV, true, true>(p, sd, nullptr, s); \
     if (p.variant != 8) return launch_softmax<KK, VV, 4>(p, s);       \
     return block == 64 ? launch_softmax<KK, VV, 8, true>(p, s) : launch_softmax<KK, VV, 8>(p, s); \
   }
@@ -1783,7 +1782,7 @@ extern "C" int natsl_softmax_sparse_fwd(const void* q, const void* k, const void
                                         const natsl_seq_row* seqs, int n_seqs, int total_units,
                                         natsl_stream_t stream) {
   return softmax_fwd(q, k, v, o, lse, types, types_dtype, nats_block_indices, n_nats_blocks, B, T, HQ, HKV, HN, K, V, TN, block,
-                     scale, same_block_visible, dtype, seqs, n_seqs, total_units, stream, SOFTMAX_ENTRY, nullptr, false);
+                     scale, same_block_visible, dtype, seqs, n_seqs, total_units, stream, SOFTMAX_ENTRY, nullptr);
 }
 
 extern "C" int natsl_softmax_sparse_fwd_per_tile(const void* q, const void* k, const void* v, void* o, float* lse,
@@ -1793,7 +1792,7 @@ extern "C" int natsl_softmax_sparse_fwd_per_tile(const void* q, const void* k, c
                                                  const natsl_seq_row* seqs, int n_seqs, int total_units,
                                                  natsl_stream_t stream) {
   return softmax_fwd(q, k, v, o, lse, types, types_dtype, nats_block_indices, n_nats_blocks, B, T, HQ, HKV, HN, K, V, TN, block,
-                     scale, same_block_visible, dtype, seqs, n_seqs, total_units, stream, SOFTMAX_PER_TILE, nullptr, false);
+                     scale, same_block_visible, dtype, seqs, n_seqs, total_units, stream, SOFTMAX_PER_TILE, nullptr);
 }
 
 static int variant_of(int B, int T, int HQ, int HKV, int block, int packed, SoftmaxUse use) {

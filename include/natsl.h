@@ -438,7 +438,7 @@ int natsl_roll_state(const float* ht, const float* hs, const float* gs, const vo
 /* The layers' short convolutions with what follows them, for up to NATSL_CONV_SEGS bf16 tensors [B, T, D_i] in one launch:
  *   y = act(conv(x)) (as natsl_short_conv_fwd; bf16 weights [D, W]), and, when y_norm is given, its rows of 8 * norm_lanes
  *   channels (a power of two of lanes) normalised: y rsqrt(mean y^2 + eps) norm_weight, or y rsqrt(sum y^2 + eps) (norm_l2); or,
- *   where scale [B, T, D / (8 norm_lanes)] is given, multiplied by its number (then without norm_weight; dscale: its gradient, may be NULL).
+ *   where scale [B, T, D / (8 norm_lanes)] is given, multiplied by its number (then without norm_weight; dscale: its gradient, zeros without dy_norm; may be NULL).
  * The backward takes the gradients that meet at y (dy_a, dy_b, and dy_norm through the norm; each may be NULL) and one that
  * meets at x (dx_add), and gives dx, dweight, dbias (bf16) and dnorm_weight (norm_dtype); sums in a fixed order.
  * Takes the place of natsl_short_conv_* and natsl_row_norm_* inside the layers (src/nats/layers/natsl_attn_gdn.py:425-505). */

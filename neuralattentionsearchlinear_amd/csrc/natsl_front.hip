@@ -269,6 +269,8 @@ __global__ __launch_bounds__(256) void conv_norm_bwd_kernel(const ConvNormParams
           if (own) dws[W + 1][c] += dn[c] * n;
         }
       }
+    } else if (s.dscale && own && cg == head * lanes) {
+      s.dscale[((size_t)b * T + t) * heads + head] = 0.f;
     }
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
@@ -573,7 +575,7 @@ static int conv_plan(ConvNormParams& p, const natsl_conv_seg* seg, int n_seg, in
     const natsl_conv_seg& s = seg[i];
     if (s.D <= 0 || s.D % 8) return fail(NATSL_ERR_UNSUPPORTED, "%s: D=%d must be a positive multiple of 8", what, s.D);
     if (!s.x || !s.weight || (bwd ? !s.dx || !s.dweight : !s.y && !s.y_norm)) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
-    if (s.y_norm || s.dy_norm) {
+    if (s.y_norm || s.dy_norm || (bwd && s.scale && s.dscale)) {
       const int l = s.norm_lanes;
       if (l <= 0 || l > 64 || (l & (l - 1)) || (s.D / 8) % l) return fail(NATSL_ERR_UNSUPPORTED, "%s: norm width %d", what, 8 * l);
       wide |= l == 64;
@@ -589,8 +591,11 @@ static int conv_plan(ConvNormParams& p, const natsl_conv_seg* seg, int n_seg, in
     p.part[i] = nullptr;
     p.first[i] = (int)wgs;
     if (i >= n_seg) continue;
-    p.seg[i] = seg[i];
-    if (!p.seg[i].y_norm && !p.seg[i].dy_norm) p.seg[i].norm_lanes = 1;
+    natsl_conv_seg& s = p.seg[i] = seg[i];
+    // (numbers that nothing is multiplied by are not read: without a tensor that follows them norm_lanes says nothing about their rows)
+    if (!bwd || !s.scale) s.dscale = nullptr;
+    if (bwd ? !s.dy_norm && !s.dscale : !s.y_norm) s.scale = nullptr;
+    if (!s.y_norm && !s.dy_norm && !s.dscale) s.norm_lanes = 1;
     wgs += ((long long)B * cdiv(T, run) * (seg[i].D / ch) + 255) / 256;
     if (wgs > 0x7fffffffll) return fail(NATSL_ERR_UNSUPPORTED, "%s: problem too large", what);
   }

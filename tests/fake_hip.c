@@ -10,6 +10,7 @@ static int current, next_event;
 static int event_device[256];
 static char launches[1 << 16];   /* a line per launch: kernel, stream, grid, and for kernels of the softmax queues their address */
 static size_t launched;
+static unsigned char segments[512];   /* the first bytes of the last convolution kernel's argument: its segments */
 static struct { const void* f; const char* name; } kernels[512];
 static int n_kernels;
 
@@ -23,6 +24,7 @@ static int device_of(const void* s) { return s ? (int)((size_t)s >> 12) : curren
 
 const char* fake_notes(void) { return notes; }
 const char* fake_launches(void) { return launches; }
+const void* fake_segments(void) { return segments; }
 void fake_reset(int device) { used = 0; notes[0] = 0; launched = 0; launches[0] = 0; current = device; }
 int fake_current(void) { return current; }
 
@@ -66,6 +68,7 @@ int hipLaunchKernel(const void* f, dim3_t grid, dim3_t block, void** args, size_
     if (kernels[i].f == f) name = kernels[i].name;
   if (strstr(name, "stream_queue_clear_kernel")) queue = *(void**)args[0];
   if (strstr(name, "softmax_stream_kernel")) queue = *(void**)args[1];
+  if (strstr(name, "conv_norm_kernel") || strstr(name, "conv_norm_bwd_kernel")) memcpy(segments, args[0], sizeof(segments));
   note("launch %lx:%d ", (unsigned long)(size_t)s, current);
   if (launched < sizeof(launches) - 256)
     launched += snprintf(launches + launched, 256, "%s %lx %u %lx\n", name, (unsigned long)(size_t)s, grid.x, (unsigned long)(size_t)queue);

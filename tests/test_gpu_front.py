@@ -464,6 +464,31 @@ def test_convolution_with_heads_of_any_width(width, what, silu, T):
         assert rel_l2(got.double(), ref.detach()) <= 2 ** -8, (name, rel_l2(got.double(), ref.detach()))
 
 
+def test_convolution_with_numbers_that_nothing_follows():
+    """natsl_conv_norm_bwd with a head's numbers and no gradient of the product: the numbers' is zero, the others are those without numbers."""
+    from neuralattentionsearchlinear_amd import _capi
+    from neuralattentionsearchlinear_amd._front import _ConvSeg
+    torch.manual_seed(3)
+    L, B, T, D, W, width = _capi.lib(), 2, 33, 128, 4, 64
+    x, w, dy = torch.randn(B, T, D, device=DEV).bfloat16(), torch.randn(D, 1, W, device=DEV).bfloat16(), torch.randn(B, T, D, device=DEV).bfloat16()
+    num, dnum = torch.rand(B, T, D // width, device=DEV), torch.full((B, T, D // width), 7., device=DEV)
+    got = []
+    for scale in (None, num):
+        dx, dw = torch.empty_like(x), torch.empty_like(w)
+        seg = (_ConvSeg * 1)()
+        s = seg[0]
+        for n, t in dict(x=x, weight=w, dy_a=dy, dx=dx, dweight=dw).items():
+            setattr(s, n, t.data_ptr())
+        s.D = D
+        if scale is not None:
+            s.norm_lanes, s.scale, s.dscale = width // 8, num.data_ptr(), dnum.data_ptr()
+        n = L.natsl_conv_norm_bwd_workspace_bytes(seg, 1, B, T, W)
+        ws = torch.empty(n, dtype=torch.uint8, device=DEV)
+        _capi.check(L.natsl_conv_norm_bwd(seg, 1, B, T, W, 1, _capi.BF16, ws.data_ptr(), n, _capi.stream_ptr(x.device)), "natsl_conv_norm_bwd")
+        got.append((dx, dw))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and not dnum.any()
+
+
 def _stepwise(monkeypatch):
     """The fused steps one by one instead of the native call."""
     from neuralattentionsearchlinear_amd import _front

@@ -542,9 +542,9 @@ class _Layer(torch.autograd.Function):
     @staticmethod
     def forward(ctx, f, flags, x, *weights):
         side, joint, states = flags
-        out, fraction, kept = _capi.step_core().layer_train(f.native, x, weights, _capi.stream_ptr(x.device), side, joint, True, states)
-        ctx.native, ctx.how = f.native, f.how
-        ctx.save_for_backward(x, *weights, *kept)
+        out, fraction, kept = _capi.step_core().layer_train(f.native, x, weights, _capi.stream_ptr(x.device), side, joint, ctx.needs_input_grad[2:], states)
+        ctx.native, ctx.how, ctx.mix = f.native, f.how, f.w["w_mix"].shape
+        ctx.save_for_backward(*kept)
         ctx.mark_non_differentiable(fraction)
         ctx.set_materialize_grads(False)
         return out, fraction
@@ -553,13 +553,10 @@ class _Layer(torch.autograd.Function):
     def backward(ctx, dout, _):
         if dout is None:
             return (None,) * len(ctx.needs_input_grad)
-        saved, n = ctx.saved_tensors, 1 + len(_NAMES) + 1
-        x, weights, kept = saved[0], saved[1:n], saved[n:]
-        w_mix = weights[_NAMES.index("w_mix")]
-        stream = _capi.stream_ptr(x.device)
+        stream = _capi.stream_ptr(dout.device)
         grads = _capi.step_core().layer_backward(
-            ctx.native, dout.to(x.dtype), x, weights, kept, ctx.needs_input_grad[2:], stream, _beside(x, ctx.how, stream), ctx.how["invalid_attn"],
-            ctx.how["invalid_linear"], _narrow_pays(x.shape[0] * x.shape[1], *w_mix.shape))
+            ctx.native, dout.to(torch.bfloat16), ctx.saved_tensors, ctx.needs_input_grad[2:], stream, _beside(dout, ctx.how, stream), ctx.how["invalid_attn"],
+            ctx.how["invalid_linear"], _narrow_pays(dout.shape[0] * dout.shape[1], *ctx.mix))
         return (None, None, *grads)
 
 
@@ -616,7 +613,7 @@ class FastFront:
             how = self.how
             states = _mixed_common._keep_states_of(x.shape[0], x.shape[0], x.shape[1], how["H"], how["K"], how["V"])
             return _Layer.apply(self, (side, joint, states), x, *weights)
-        return _capi.step_core().layer_train(self.native, x, weights, stream, side, joint, False, False)[:2]
+        return _capi.step_core().layer_train(self.native, x, weights, stream, side, joint, None, False)[:2]
 
     def prompt(self, x, seen):
         """The layer's forward outside of training (`native` only, no gradients).  seen: None, or a call that gets the blocks' types as soon as they are

@@ -45,6 +45,22 @@ enum Weight { WQ, WK, WV, WG, WA, WB, W_MIX, WO, CONV_WQ, CONV_WK, CONV_WV, CONV
 typedef at::Tensor T;
 typedef std::vector<T> Ts;
 
+// Which parts of the backward run for gradients of x and of the weights (in that order): what nobody wants is neither computed nor kept for, as in
+// a graph of one node for each (340M geometry, 8 x 4096 tokens, only o_proj trains: 2711 -> 1164 us a step).
+struct Needs {
+  std::vector<bool> of;
+  bool conv, gates, op, tail;  // convolutions, gates, operator (conv and gates are in front of it), norm-gate (the operator is in front of it)
+  Needs(const std::vector<bool>& need, const bool delta) : of(need) {
+    auto any = [&](std::initializer_list<Weight> ws) { return std::any_of(ws.begin(), ws.end(), [&](const Weight w) { return want(w); }); };
+    gates = x() || any({WA, WB, A_LOG, DT_BIAS});
+    conv = x() || any({WQ, WK, WV, CONV_WQ, CONV_WK, CONV_WV, CONV_BQ, CONV_BK, CONV_BV, NORM_Q, NORM_K}) || (!delta && any({WA, DT_BIAS}));
+    op = conv || gates || want(WN);
+    tail = op || any({W_MIX, WG, OUT_NORM1, OUT_NORM2});
+  }
+  bool x() const { return of[0]; }
+  bool want(const Weight w) const { return of[1 + w]; }
+};
+
 struct Failed {                // an entry point's code
   int rc;
   const char* what;
@@ -74,6 +90,7 @@ struct Call {
   Call(const Layer& layer, const T& input, const Ts& weights, natsl_stream_t s, natsl_stream_t beside)
       : l(layer), x(input), w(weights), stream(s), side(beside), B(input.size(0)), T_(input.size(1)), rows(B * T_), bf16(input.options()),
         f32(bf16.dtype(at::kFloat)), i32(bf16.dtype(at::kInt)), u8(bf16.dtype(at::kByte)) {}
+  T sized(const int64_t columns) const { return at::empty({B, T_, columns}, bf16); }
   T bytes(const size_t n) const { return at::empty({(int64_t)n}, u8); }
 };
 
@@ -82,7 +99,8 @@ struct Front {
   T g, beta, dt, logits, ab, wab, pooled, types, raw, counts, fraction;
 };
 
-Front front(const Call& c, const bool keep, const bool want_raw) {
+// needs: null outside of training
+Front front(const Call& c, const Needs* needs, const bool want_raw) {
   const Layer& l = c.l;
   Front o;
   natsl_front a{};
@@ -92,11 +110,11 @@ Front front(const Call& c, const bool keep, const bool want_raw) {
   else o.dt = like(o.g);
   o.logits = at::empty({c.B, nb, l.HN, 2}, c.bf16);
   a.NA = l.H; a.NB = l.delta ? l.H : 0; a.NL = l.NL;
-  if (keep) {
-    a.ld = a.wab_rows = (int32_t)up(a.NA + a.NB, 32);
-    o.pooled = at::empty({c.B * nb, l.D}, c.bf16);
-    o.ab = at::empty({c.B, c.T_, a.ld}, c.bf16);
-    o.wab = at::empty({a.ld, l.D}, c.bf16);
+  if (needs) {
+    const int32_t ld = (int32_t)up(a.NA + a.NB, 32);
+    if (needs->want(WN)) o.pooled = at::empty({c.B * nb, l.D}, c.bf16);
+    if (needs->gates) o.ab = c.sized(a.ld = ld);
+    if (needs->x()) o.wab = at::empty({a.wab_rows = ld, l.D}, c.bf16);
   }
   a.x = at_(c.x); a.wa = at_(c.w[WA]); a.wb = l.delta ? at_(c.w[WB]) : nullptr; a.wn = at_(c.w[WN]); a.a_log = at_(c.w[A_LOG]); a.dt_bias = at_(c.w[DT_BIAS]);
   a.ab = at_(o.ab); a.pooled = at_(o.pooled); a.logits = at_(o.logits); a.beta = at_(o.beta); a.wab = at_(o.wab); a.g = f_(o.g); a.dt = f_(o.dt);
@@ -240,7 +258,7 @@ void rest(const Call& c, const Front& f, const bool joint, const bool keep, cons
 }
 
 // ---- backward ----------------------------------------------------------------------------------------------------------------
-// what the forward keeps, in this order behind x and the weights
+// what the forward keeps, in this order behind x and the weights: each only where a part that runs reads it
 enum Kept { AB, WAB, POOLED, LOGITS, TYPES, RAW_Q, RAW_K, RAW_V, GATE, Y_Q, Y_K, Y_V, N_Q, N_K, MIX, G, BETA, DT, O_LIN, O_ATTN, LSE, IDX, NBLK, TAIL, STATES, V_NEW, WS, KEPT };
 
 // dy_i [rows, n_i]^T x [rows, D], one launch for those whose widths are multiples of 8; a narrow one that is not, or that is alone, by itself
@@ -367,16 +385,17 @@ MixedGrads mixed_bwd(const Call& c, const Ts& s, const T& do_lin, const T& do_at
   return r;
 }
 
-// grads: x, then the weights
-void backward(const Call& c, const Ts& s, const T& dout, const std::vector<bool>& need, const int invalid_attn, const int invalid_linear, const bool mix_pays, Ts& grads) {
+// dout: c.x; grads: x, then the weights
+void backward(const Call& c, const T& x, const Ts& s, const Needs& need, const int invalid_attn, const int invalid_linear, const bool mix_pays, Ts& grads) {
   const Layer& l = c.l;
   const Ts& w = c.w;
   grads.assign(1 + WEIGHTS, T());
-  auto want = [&](const int i) { return need[1 + i]; };
+  auto want = [&](const Weight i) { return need.want(i); };
   const int64_t rows = c.rows, vd = l.H * l.V;
-  const T d2 = dout.reshape({rows, l.D}).contiguous();
-  const T dy = at::mm(d2, w[WO]);
+  const T d2 = c.x.reshape({rows, l.D}).contiguous();
   if (want(WO)) grads[1 + WO] = wgrad(c, s[TAIL].view({rows, vd}), d2);
+  if (!need.tail) return;
+  const T dy = at::mm(d2, w[WO]);
   // norm-gate
   const T do_lin = like(s[O_LIN]), do_attn = like(s[O_ATTN]), dgate = like(s[GATE]), dmix = like(s[MIX]), dwn = at::empty({2, l.VA}, c.f32);
   {
@@ -391,15 +410,15 @@ void backward(const Call& c, const Ts& s, const T& dout, const std::vector<bool>
       grads[1 + OUT_NORM2] = d.select(0, 1);
     }
   }
-  const MixedGrads m = mixed_bwd(c, s, do_lin, do_attn, invalid_attn, invalid_linear);
-  // selector
-  const T dl2 = m.logits.view({-1, l.NL});
+  MixedGrads m;
+  if (need.op) m = mixed_bwd(c, s, do_lin, do_attn, invalid_attn, invalid_linear);
   // mixing logits, convolutions
-  const T dmix2 = dmix.view({rows, -1}), yq2 = s[Y_Q].view({rows, -1}), dq_mix = narrow_bwd(c, dmix2, w[W_MIX], mix_pays);
-  if (want(W_MIX)) grads[1 + W_MIX] = wgrad(c, yq2, dmix2);
+  const T dmix2 = dmix.view({rows, -1});
+  if (want(W_MIX)) grads[1 + W_MIX] = wgrad(c, s[Y_Q].view({rows, -1}), dmix2);
   T dx[4], ddt;
   dx[3] = dgate;
-  {
+  if (need.conv) {
+    const T dq_mix = narrow_bwd(c, dmix2, w[W_MIX], mix_pays);
     natsl_conv_seg g[3];
     conv_segs(c, &s[RAW_Q], s[DT], g);
     for (int i = 0; i < 3; ++i) {
@@ -433,8 +452,9 @@ void backward(const Call& c, const Ts& s, const T& dout, const std::vector<bool>
     must(l.conv_norm_bwd(g, 3, (int)c.B, (int)c.T_, l.W, l.act, l.norm_dtype, at_(ws), n, c.stream), "natsl_conv_norm_bwd");
   }
   // gates
-  const T dab = like(s[AB]);
-  {
+  T dab;
+  if (need.gates) {
+    dab = like(s[AB]);
     grads[1 + A_LOG] = like(w[A_LOG]);
     grads[1 + DT_BIAS] = like(w[DT_BIAS]);
     const size_t n = l.gates_bwd_workspace_bytes(rows, l.H);
@@ -442,6 +462,9 @@ void backward(const Call& c, const Ts& s, const T& dout, const std::vector<bool>
     must(l.gates_bwd(at_(s[AB]), at_(w[A_LOG]), at_(w[DT_BIAS]), f_(m.g), at_(m.beta), f_(ddt), l.delta, at_(dab), at_(grads[1 + A_LOG]), at_(grads[1 + DT_BIAS]), at_(ws), n,
                      rows, l.H, (int)s[AB].size(2), l.neg, l.gate_dtype, c.stream), "natsl_gates_bwd");
   }
+  // selector
+  T dl2;
+  if (need.op) dl2 = m.logits.view({-1, l.NL});
   if (want(WN)) {
     const int64_t r = dl2.size(0), n = l.NL;
     if (n > 64 || l.D % 2 || r > 2048) {
@@ -451,12 +474,13 @@ void backward(const Call& c, const Ts& s, const T& dout, const std::vector<bool>
       must(l.narrow_wgrad(at_(dl2), at_(s[POOLED]), at_(grads[1 + WN]), r, l.D, (int)n, c.stream), "natsl_narrow_wgrad");
     }
   }
-  const int64_t ld = dab.size(2);
-  std::vector<T> dys;
-  for (int i = 0; i < 4; ++i) dys.push_back(dx[i].view({rows, -1}));
-  dys.push_back(dab.view({rows, ld}));
-  if (need[0]) {
-    const T dpool = narrow_bwd(c, dl2, w[WN], true), dX = like(c.x);
+  std::vector<T> dys(5);
+  for (int i = 0; i < 4; ++i)
+    if (dx[i].defined()) dys[i] = dx[i].view({rows, -1});
+  if (dab.defined()) dys[4] = dab.view({rows, -1});
+  if (need.x()) {
+    const int64_t ld = dab.size(2);
+    const T dpool = narrow_bwd(c, dl2, w[WN], true), dX = c.sized(l.D);
     bool whole = true;
     natsl_project_seg segs[5];
     for (int i = 0; i < 5; ++i) {
@@ -474,10 +498,11 @@ void backward(const Call& c, const Ts& s, const T& dout, const std::vector<bool>
     grads[0] = dX;
   }
   for (int i = 0; i < 4; ++i)
-    if (!want(WQ + i)) dys[i] = T();
+    if (!want(Weight(WQ + i))) dys[i] = T();
   if (!want(WA) && !want(WB)) dys[4] = T();
+  if (std::none_of(dys.begin(), dys.end(), [](const T& t) { return t.defined(); })) return;
   std::vector<T> dws;
-  wgrads(c, c.x.view({rows, l.D}), dys, dws);
+  wgrads(c, x.view({rows, l.D}), dys, dws);
   for (int i = 0; i < 4; ++i) grads[1 + WQ + i] = dws[i];
   if (dws[4].defined()) {
     grads[1 + WA] = dws[4].slice(0, 0, l.H);
@@ -579,36 +604,81 @@ PyObject* natsl_make_layer(PyObject*, PyObject* args) {
   END_HANDLE_TH_ERRORS
 }
 
-// layer_train(layer, x, weights, stream, side, joint, keep, keep states) -> (out, attention's share per head, what the backward needs: a tuple of KEPT
-// tensors, or None without keep)
+bool needs_of(PyObject* seq, std::vector<bool>& need) {
+  THPObjectPtr fast(PySequence_Fast(seq, "what wants a gradient"));
+  if (!fast) return false;
+  if (PySequence_Fast_GET_SIZE(fast.get()) != 1 + WEIGHTS) {
+    PyErr_SetString(PyExc_ValueError, "what wants a gradient: x, then the weights");
+    return false;
+  }
+  need.resize(1 + WEIGHTS);
+  for (int i = 0; i <= WEIGHTS; ++i) need[(size_t)i] = PyObject_IsTrue(PySequence_Fast_GET_ITEM(fast.get(), i)) > 0;
+  return true;
+}
+
+// layer_train(layer, x, weights, stream, side, joint, what wants a gradient (x, then the weights) or None, keep states) -> (out, attention's share per
+// head, what the backward needs: x, the weights and KEPT tensors, None for those that it does not read; or None)
 PyObject* natsl_layer_train(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Ts w;
+  std::vector<bool> of;
   if (n != 8 || !THPVariable_Check(a[1])) {
-    PyErr_SetString(PyExc_TypeError, "layer_train(layer, x, weights, stream, side, joint, keep, keep states)");
+    PyErr_SetString(PyExc_TypeError, "layer_train(layer, x, weights, stream, side, joint, needs, keep states)");
     return nullptr;
   }
   Layer* l = layer_of(a[0]);
-  if (!l || !tensors_of(a[2], w)) return nullptr;
+  if (!l || !tensors_of(a[2], w) || (a[6] != Py_None && !needs_of(a[6], of))) return nullptr;
+  const bool keep = !of.empty();
+  if (!keep) of.resize(1 + WEIGHTS);
+  const Needs need(of, l->delta);
   const Call c(*l, THPVariable_Unpack(a[1]), w, stream_of(a[3]), stream_of(a[4]));
-  const bool joint = PyObject_IsTrue(a[5]) > 0, keep = PyObject_IsTrue(a[6]) > 0, states = PyObject_IsTrue(a[7]) > 0;
+  const bool joint = PyObject_IsTrue(a[5]) > 0, states = need.op && PyObject_IsTrue(a[7]) > 0;
   Front f;
   Rest r;
   if (!run_free(*l, [&] {
-        f = front(c, keep, false);
-        rest(c, f, joint, keep, keep && states, false, r);
+        f = front(c, keep ? &need : nullptr, false);
+        rest(c, f, joint, need.op, states, false, r);
       }))
     return nullptr;
   const Mixed& m = r.m;
   THPObjectPtr kept;
   if (keep) {
-    Ts s(KEPT);
-    s[AB] = f.ab; s[WAB] = f.wab; s[POOLED] = f.pooled; s[LOGITS] = f.logits; s[TYPES] = f.types; s[G] = f.g; s[BETA] = f.beta; s[DT] = f.dt;
-    for (int i = 0; i < 3; ++i) { s[RAW_Q + i] = r.raw[i]; s[Y_Q + i] = r.y[i]; }
-    s[GATE] = r.raw[3]; s[N_Q] = r.n[0]; s[N_K] = r.n[1]; s[MIX] = r.mix; s[TAIL] = r.tail;
-    s[O_LIN] = m.o_lin; s[O_ATTN] = m.o_attn; s[LSE] = m.lse; s[IDX] = m.idx; s[NBLK] = m.nblk;
+    Ts all(1 + WEIGHTS + KEPT);
+    T* const s = all.data() + 1 + WEIGHTS;
+    auto weights = [&](std::initializer_list<Weight> ws) {
+      for (const Weight i : ws) all[1 + i] = w[i];
+    };
+    if (need.want(WO)) s[TAIL] = r.tail;
+    if (need.tail) {
+      weights({WO, OUT_NORM1, OUT_NORM2});
+      s[GATE] = r.raw[3]; s[MIX] = r.mix; s[O_LIN] = m.o_lin; s[O_ATTN] = m.o_attn;
+    }
+    if (need.want(W_MIX)) s[Y_Q] = r.y[0];
+    if (need.op) {
+      for (int i = 0; i < 3; ++i) {
+        if (i > 0 || l->delta) s[Y_Q + i] = r.y[i];
+        if (need.conv || !l->delta) s[RAW_Q + i] = r.raw[i];
+      }
+      s[LOGITS] = f.logits; s[TYPES] = f.types; s[G] = f.g; s[BETA] = f.beta; s[N_Q] = r.n[0]; s[N_K] = r.n[1]; s[LSE] = m.lse; s[IDX] = m.idx; s[NBLK] = m.nblk;
+    }
     if (states) { s[STATES] = m.states; s[V_NEW] = m.v_new; s[WS] = m.ws; }
-    kept = tuple_of(s);
+    if (need.conv) {
+      weights({W_MIX, CONV_WQ, CONV_WK, CONV_WV, CONV_BQ, CONV_BK, CONV_BV, NORM_Q, NORM_K});
+      s[DT] = f.dt;
+    }
+    if (need.gates) {
+      weights({A_LOG, DT_BIAS});
+      s[AB] = f.ab;
+    }
+    if (need.x()) {
+      weights({WQ, WK, WV, WG, WN});
+      s[WAB] = f.wab;
+    }
+    if (need.x() || need.want(WA) || need.want(WB)) weights({WA, WB});          // (read as WAB, which was made of them)
+    s[POOLED] = f.pooled;
+    for (const Weight i : {WQ, WK, WV, WG, WA, WB})
+      if (need.want(i)) all[0] = c.x;
+    kept = tuple_of(all);
   } else {
     Py_INCREF(Py_None);
     kept = Py_None;
@@ -619,35 +689,31 @@ PyObject* natsl_layer_train(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// layer_backward(layer, dout, x, weights, kept, needs (x, then the weights), stream, side, invalid attention, invalid linear, whether the one-pass kernel has the
-// mixing logits' input gradient) -> gradients of x, then of the weights
+// layer_backward(layer, dout, what the forward kept, what wants a gradient (x, then the weights), stream, side, invalid attention, invalid linear, whether the
+// one-pass kernel has the mixing logits' input gradient) -> gradients of x, then of the weights
 PyObject* natsl_layer_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  Ts w, s, grads;
-  if (n != 11 || !THPVariable_Check(a[1]) || !THPVariable_Check(a[2])) {
-    PyErr_SetString(PyExc_TypeError, "layer_backward(layer, dout, x, weights, kept, needs, stream, side, invalid attention, invalid linear, mix)");
+  Ts kept, grads;
+  std::vector<bool> of;
+  if (n != 9 || !THPVariable_Check(a[1])) {
+    PyErr_SetString(PyExc_TypeError, "layer_backward(layer, dout, kept, needs, stream, side, invalid attention, invalid linear, mix)");
     return nullptr;
   }
   Layer* l = layer_of(a[0]);
-  if (!l || !tensors_of(a[3], w) || !tensors_of(a[4], s)) return nullptr;
-  std::vector<bool> need(1 + WEIGHTS);
-  for (int i = 0; i <= WEIGHTS; ++i) {
-    PyObject* o = PySequence_GetItem(a[5], i);
-    if (!o) return nullptr;
-    need[(size_t)i] = PyObject_IsTrue(o) > 0;
-    Py_DECREF(o);
-  }
-  if ((int)w.size() != WEIGHTS || (int)s.size() != KEPT) {
-    PyErr_SetString(PyExc_ValueError, "layer_backward: other numbers of tensors than the forward gave");
+  if (!l || !tensors_of(a[2], kept) || !needs_of(a[3], of)) return nullptr;
+  if ((int)kept.size() != 1 + WEIGHTS + KEPT) {
+    PyErr_SetString(PyExc_ValueError, "layer_backward: another number of tensors than the forward gave");
     return nullptr;
   }
-  const Call c(*l, THPVariable_Unpack(a[2]), w, stream_of(a[6]), stream_of(a[7]));
-  const T dout = THPVariable_Unpack(a[1]);
-  const int ia = PyObject_IsTrue(a[8]) > 0, il = PyObject_IsTrue(a[9]) > 0;
-  const bool mix = PyObject_IsTrue(a[10]) > 0;
-  if (!run_free(*l, [&] { backward(c, s, dout, need, ia, il, mix, grads); })) return nullptr;
+  const Needs need(of, l->delta);
+  const T x = kept[0];
+  const Ts w(kept.begin() + 1, kept.begin() + 1 + WEIGHTS), s(kept.begin() + 1 + WEIGHTS, kept.end());
+  const Call c(*l, THPVariable_Unpack(a[1]), w, stream_of(a[4]), stream_of(a[5]));
+  const int ia = PyObject_IsTrue(a[6]) > 0, il = PyObject_IsTrue(a[7]) > 0;
+  const bool mix = PyObject_IsTrue(a[8]) > 0;
+  if (!run_free(*l, [&] { backward(c, x, s, need, ia, il, mix, grads); })) return nullptr;
   for (int i = 0; i <= WEIGHTS; ++i)
-    if (!need[(size_t)i]) grads[(size_t)i] = T();
+    if (!of[(size_t)i]) grads[(size_t)i] = T();
   return tuple_of(grads);
   END_HANDLE_TH_ERRORS
 }
@@ -664,7 +730,7 @@ PyObject* natsl_layer_prompt_front(PyObject*, PyObject* const* a, Py_ssize_t n) 
   if (!l || !tensors_of(a[2], w)) return nullptr;
   const Call c(*l, THPVariable_Unpack(a[1]), w, stream_of(a[3]), nullptr);
   Front f;
-  if (!run_free(*l, [&] { f = front(c, false, true); })) return nullptr;
+  if (!run_free(*l, [&] { f = front(c, nullptr, true); })) return nullptr;
   return tuple_of({f.g, f.beta, f.dt, f.logits, f.types, f.raw, f.counts, f.fraction});
   END_HANDLE_TH_ERRORS
 }

@@ -151,8 +151,8 @@ def _wide(x, ws):
 
 def _narrow(f, x, want_selector, keep):
     """The narrow products of one input, the gates behind them and the selector's logits over the means of 64 tokens, one pass over x:
-    -> (g fp32, beta bf16 or None, dt fp32 or None [B,T,H], logits [B,TN,NL] or None, what the backward needs if `keep`: (a and b of every token,
-    their joint weight in whole stages of 32 rows, the block means or None)).  As separate products and passes it is four launches, two of them the
+    -> (g fp32, beta bf16 or None, dt fp32 or None [B,T,H], logits [B,TN,NL] or None, what the backward needs, each where `keep` says so: (a and b of
+    every token, their joint weight in whole stages of 32 rows, the block means)).  As separate products and passes it is four launches, two of them the
     library's (340M geometry, 8 x 4096 tokens: 36 -> 24 us; 1 x 777 25 -> 9)."""
     B, T, D = x.shape
     w, H, dev = f.w, f.H, x.device
@@ -162,23 +162,31 @@ def _narrow(f, x, want_selector, keep):
     g = torch.empty(B, T, H, dtype=torch.float32, device=dev)
     beta = torch.empty(B, T, H, dtype=torch.bfloat16, device=dev) if f.delta else None
     dt = None if f.delta else torch.empty_like(g)
-    logits = pooled = saved = None
+    logits = pooled = ab = wab = None
     if want_selector:
         nb = -(-T // 64)
         logits = torch.empty(B, nb, f.wn.shape[0], dtype=torch.bfloat16, device=dev)
         a.wn, a.logits, a.NL = f.wn.data_ptr(), logits.data_ptr(), f.wn.shape[0]
-        if keep:
+        if keep[2]:
             pooled = torch.empty(B, nb, D, dtype=torch.bfloat16, device=dev)
             a.pooled = pooled.data_ptr()
-    if keep:
-        a.ld = a.wab_rows = _ab_rows(a.NA + a.NB)
-        ab, wab = torch.empty(B, T, a.ld, dtype=torch.bfloat16, device=dev), torch.empty(a.ld, D, dtype=torch.bfloat16, device=dev)
-        a.ab, a.wab = ab.data_ptr(), wab.data_ptr()
-        saved = ab, wab, pooled
+    if keep[0]:
+        a.ld = _ab_rows(a.NA + a.NB)
+        ab = torch.empty(B, T, a.ld, dtype=torch.bfloat16, device=dev)
+        a.ab = ab.data_ptr()
+    if keep[1]:
+        a.wab_rows = _ab_rows(a.NA + a.NB)
+        wab = torch.empty(a.wab_rows, D, dtype=torch.bfloat16, device=dev)
+        a.wab = wab.data_ptr()
     a.x, a.wa, a.wb, a.a_log, a.dt_bias = x.data_ptr(), w["wa"].data_ptr(), _p(wb), w["a_log"].data_ptr(), w["dt_bias"].data_ptr()
     a.g, a.beta, a.dt = g.data_ptr(), _p(beta), _p(dt)
     _capi.check(_capi.lib().natsl_layer_front(ctypes.byref(a), _capi.stream_ptr(dev)), "natsl_layer_front")
-    return g, beta, dt, logits, saved
+    return g, beta, dt, logits, (ab, wab, pooled)
+
+
+def _only_for(ctx, *outputs):
+    """Marks the outputs (tensor or None, whether an input that it is made from wants a gradient) for which nothing behind them has to run backwards."""
+    ctx.mark_non_differentiable(*[t for t, wanted in outputs if t is not None and not wanted])
 
 
 def _project(x, wq, wk, wv, wg, wa, wb, pool_block, whole=16):
@@ -258,11 +266,17 @@ class _ProjectAll(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, f, x, wq, wk, wv, wg, wa, wb, wn, a_log, dt_bias):
-        g, beta, dt, logits, (ab, wab, pooled) = _narrow(f, x, wn is not None, True)
+        _, nx, nq, nk, nv, ng, na, nb, nn, nal, ndt = ctx.needs_input_grad
+        gates = nx or na or nb or nal or ndt
+        g, beta, dt, logits, (ab, wab, pooled) = _narrow(f, x, wn is not None, (gates, nx, nn))
+        q, k, v, gate = _wide(x, (wq, wk, wv, wg))
         ctx.f = f
-        ctx.save_for_backward(x, wq, wk, wv, wg, wab, ab, pooled, wn, a_log, dt_bias)
+        only = lambda on, *ts: ts if on else (None,) * len(ts)
+        ctx.save_for_backward(*only(any(ctx.needs_input_grad[1:8]), x), *only(nx, wq, wk, wv, wg, wab), ab, pooled, *only(nx, wn), *only(gates, a_log, dt_bias))
         ctx.set_materialize_grads(False)
-        return (*_wide(x, (wq, wk, wv, wg)), g, beta, dt, logits)
+        _only_for(ctx, (q, nx or nq), (k, nx or nk), (v, nx or nv), (gate, nx or ng), (g, nx or na or nal or ndt), (beta, nx or nb), (dt, nx or na or ndt),
+                  (logits, nx or nn))
+        return q, k, v, gate, g, beta, dt, logits
 
     @staticmethod
     def backward(ctx, dq, dk, dv, dgate, dg, dbeta, ddt, dlogits):
@@ -272,12 +286,14 @@ class _ProjectAll(torch.autograd.Function):
         if dg is not None or dbeta is not None or ddt is not None:
             dab, da_log, ddt_bias = _gates_bwd(f, ab, dg, dbeta, ddt)
         if dlogits is not None:
-            dl = dlogits.reshape(-1, wn.shape[0]).contiguous()
+            dl = dlogits.reshape(-1, dlogits.shape[-1]).contiguous()
             if need[1]:
-                dpool = _narrow_bwd(dl, wn, few=True).view(pooled.shape)
+                dpool = _narrow_bwd(dl, wn, few=True).view(*dlogits.shape[:2], -1)
             if need[8]:
                 dwn = _narrow_wgrad(dl, pooled.view(-1, pooled.shape[-1]))
-        dx, *dws = _project_bwd(x, (wq, wk, wv, wg), wab, f.H, f.H if f.delta else 0, (dq, dk, dv, dgate, dab), dpool, 64, need[1:8])
+        dx, dws = None, (None,) * 6
+        if x is not None:
+            dx, *dws = _project_bwd(x, (wq, wk, wv, wg), wab, f.H, f.H if f.delta else 0, (dq, dk, dv, dgate, dab), dpool, 64, need[1:8])
         return (None, dx, *dws, dwn, da_log, ddt_bias)
 
 
@@ -364,7 +380,12 @@ class _ConvNorm(torch.autograd.Function):
         ctx.save_for_backward(q, k, v, ys[0], w_mix, dt, wq, bq, wk, bk, wv, bv, nq, nk)
         ctx.set_materialize_grads(False)
         raw = tuple(t.view(t.shape) for t in (q, k, v)) if f.raw_attention else (None, None, ys[2].detach())
-        return (ys[0], ys[1], ys[2], ns[0], ns[1], F.linear(ys[0], w_mix)) + raw
+        _, nq_, nk_, nv_, *nw, nnq, nnk, nmix, ndt = ctx.needs_input_grad
+        cq, ck, cv = nq_ or nw[0] or nw[1], nk_ or nw[2] or nw[3], nv_ or nw[4] or nw[5]
+        mix = F.linear(ys[0], w_mix)
+        _only_for(ctx, (ys[0], cq), (ys[1], ck), (ys[2], cv or ndt), (ns[0], cq or nnq), (ns[1], ck or nnk), (mix, cq or nmix),
+                  *zip(raw, (nq_, nk_, nv_ if f.raw_attention else cv)))
+        return (ys[0], ys[1], ys[2], ns[0], ns[1], mix) + raw
 
     @staticmethod
     def backward(ctx, dq, dk, dv, dqn, dkn, dlogits, dq_raw, dk_raw, dv_raw):
@@ -641,7 +662,7 @@ class FastFront:
             if self.grad(x, *wide, w["wa"], wb, wn, w["a_log"], w["dt_bias"]):
                 q, k, v, gate, g, beta, dt, logits = _ProjectAll.apply(self, x, *wide, w["wa"], wb, wn, w["a_log"], w["dt_bias"])
             else:
-                g, beta, dt, logits, _ = _narrow(self, x, wn is not None, False)
+                g, beta, dt, logits, _ = _narrow(self, x, wn is not None, (False, False, False))
                 q, k, v, gate = _wide(x, wide)
             return q, k, v, gate, (g, beta, dt), logits
         args = (x, w["wq"], w["wk"], w["wv"], w["wg"], w["wa"], wb, pool_block)

@@ -616,6 +616,37 @@ def test_native_layer_of_which_a_part_trains(kind, train, monkeypatch):
     assert calls == [1] and held <= most + (64 << 10), (held, most)
 
 
+@pytest.mark.parametrize("kind", ['gdn', 'mamba'])
+@pytest.mark.parametrize("train,follow", [
+    (('nats_layer',), {'logits'}), (('A_log',), {'g'}), (('dt_bias',), {'g', 'dt', 'v'}), (('g_proj',), {'gate'}), (('k_proj',), {'k', 'ky', 'kn', 'kr'}),
+    (('a_proj',), {'g', 'dt', 'v'}), (('q_conv1d',), {'qy', 'qn', 'mix'}), (('nats_out_weights_layer',), {'mix'}), (('v_conv1d',), {'v', 'vr'})])
+def test_steps_of_which_a_part_trains(kind, train, follow):
+    """Of the fused steps' outputs only those follow a gradient that are made from what trains (qy: the convolution, qn: its norm, qr: attention's view
+    where that is the projection, or for v in the delta rule's layer the convolution; v: with dt)."""
+    from neuralattentionsearchlinear_amd import _front
+    layer = _layer(kind, None, 'all').train()
+    for n, p in layer.named_parameters():
+        p.requires_grad_(n.startswith(train))
+    delta = kind == 'gdn'
+    x = torch.randn(2, 130, layer.hidden_size, device=DEV).bfloat16()
+    f = _front.fast_front(layer, kind, x, None, None)
+    q, k, v, gate, (g, beta, dt), logits = f.project(x, 64, layer.nats_layer)
+    qy, ky, vy, qn, kn, mix, qr, kr, vr, _ = f.conv_norm(q, k, v, None, False, None if delta else dt)
+    got = dict(gate=gate, g=g, beta=beta, dt=dt, logits=logits, k=k, qy=qy, ky=ky, v=vy, qn=qn, kn=kn, mix=mix, qr=qr, kr=kr, vr=vr)
+    if delta:
+        follow = follow - {'kr'} - ({'dt', 'v'} if 'dt' in follow else set())
+    else:
+        follow = follow - {'ky'} - ({'vr'} if train == ('v_conv1d',) else set())
+    assert {n for n, t in got.items() if t is not None and t.requires_grad} == follow
+    with torch.no_grad():
+        if not any(n.endswith('_proj') for n in train):
+            x.add_(1.0)                                    # (nothing of the input is read by these gradients)
+    outs = [t for n, t in got.items() if n in follow]
+    torch.autograd.backward(outs, [torch.randn_like(t) for t in outs])
+    for n, p in layer.named_parameters():
+        assert (p.grad is not None and bool(p.grad.any())) == n.startswith(train), n
+
+
 @pytest.mark.parametrize("kind,T0", [('gdn', 128), ('gdn', 777), ('mamba', 64), ('mamba', 2113)])
 @pytest.mark.parametrize("ops", ['all', 'attn'])
 def test_native_prompt_is_its_steps(kind, T0, ops, monkeypatch):

@@ -575,8 +575,10 @@ class _Layer(torch.autograd.Function):
         if dout is None:
             return (None,) * len(ctx.needs_input_grad)
         stream = _capi.stream_ptr(dout.device)
+        kept = list(ctx.saved_tensors)
+        ctx.maybe_clear_saved_tensors()                    # (not where the graph is retained; nodes of their own are freed one by one, too)
         grads = _capi.step_core().layer_backward(
-            ctx.native, dout.to(torch.bfloat16), ctx.saved_tensors, ctx.needs_input_grad[2:], stream, _beside(dout, ctx.how, stream), ctx.how["invalid_attn"],
+            ctx.native, dout.to(torch.bfloat16), kept, ctx.needs_input_grad[2:], stream, _beside(dout, ctx.how, stream), ctx.how["invalid_attn"],
             ctx.how["invalid_linear"], _narrow_pays(dout.shape[0] * dout.shape[1], *ctx.mix))
         return (None, None, *grads)
 

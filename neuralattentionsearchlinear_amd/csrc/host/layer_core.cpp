@@ -48,7 +48,7 @@ typedef std::vector<T> Ts;
 // Which parts of the backward run for gradients of x and of the weights (in that order): what nobody wants is neither computed nor kept for, as in
 // a graph of one node for each (340M geometry, 8 x 4096 tokens, only o_proj trains: 2711 -> 1164 us a step).
 struct Needs {
-  std::vector<bool> of;
+  std::vector<bool> of;        // empty: nothing
   bool conv, gates, op, tail;  // convolutions, gates, operator (conv and gates are in front of it), norm-gate (the operator is in front of it)
   Needs(const std::vector<bool>& need, const bool delta) : of(need) {
     auto any = [&](std::initializer_list<Weight> ws) { return std::any_of(ws.begin(), ws.end(), [&](const Weight w) { return want(w); }); };
@@ -57,8 +57,8 @@ struct Needs {
     op = conv || gates || want(WN);
     tail = op || any({W_MIX, WG, OUT_NORM1, OUT_NORM2});
   }
-  bool x() const { return of[0]; }
-  bool want(const Weight w) const { return of[1 + w]; }
+  bool x() const { return !of.empty() && of[0]; }
+  bool want(const Weight w) const { return !of.empty() && of[1 + w]; }
 };
 
 struct Failed {                // an entry point's code
@@ -72,6 +72,10 @@ void must(const int rc, const char* what) {
 void* at_(const T& t) { return t.defined() ? t.data_ptr() : nullptr; }
 float* f_(const T& t) { return t.defined() ? static_cast<float*>(t.data_ptr()) : nullptr; }
 int32_t* i_(const T& t) { return t.defined() ? static_cast<int32_t*>(t.data_ptr()) : nullptr; }
+// Tensors that nothing reads any more: what a call allocates next may take their memory (a step at the 340M geometry, 8 x 4096 tokens, has a peak
+// of 1.8 GB so, and of 2.2 GB where all live to its end).  What the side stream works on is dropped behind its join.
+template <class... Dropped>
+void drop(Dropped&... t) { (t.reset(), ...); }
 T like(const T& t) { return at::empty(t.sizes(), t.options()); }
 int64_t up(const int64_t n, const int64_t m) { return (n + m - 1) / m * m; }
 int64_t blocks_of(const int64_t t) { return (t + 63) / 64; }
@@ -99,8 +103,7 @@ struct Front {
   T g, beta, dt, logits, ab, wab, pooled, types, raw, counts, fraction;
 };
 
-// needs: null outside of training
-Front front(const Call& c, const Needs* needs, const bool want_raw) {
+Front front(const Call& c, const Needs& needs, const bool want_raw) {
   const Layer& l = c.l;
   Front o;
   natsl_front a{};
@@ -110,12 +113,10 @@ Front front(const Call& c, const Needs* needs, const bool want_raw) {
   else o.dt = like(o.g);
   o.logits = at::empty({c.B, nb, l.HN, 2}, c.bf16);
   a.NA = l.H; a.NB = l.delta ? l.H : 0; a.NL = l.NL;
-  if (needs) {
-    const int32_t ld = (int32_t)up(a.NA + a.NB, 32);
-    if (needs->want(WN)) o.pooled = at::empty({c.B * nb, l.D}, c.bf16);
-    if (needs->gates) o.ab = c.sized(a.ld = ld);
-    if (needs->x()) o.wab = at::empty({a.wab_rows = ld, l.D}, c.bf16);
-  }
+  const int32_t ld = (int32_t)up(a.NA + a.NB, 32);
+  if (needs.want(WN)) o.pooled = at::empty({c.B * nb, l.D}, c.bf16);
+  if (needs.gates) o.ab = c.sized(a.ld = ld);
+  if (needs.x()) o.wab = at::empty({a.wab_rows = ld, l.D}, c.bf16);
   a.x = at_(c.x); a.wa = at_(c.w[WA]); a.wb = l.delta ? at_(c.w[WB]) : nullptr; a.wn = at_(c.w[WN]); a.a_log = at_(c.w[A_LOG]); a.dt_bias = at_(c.w[DT_BIAS]);
   a.ab = at_(o.ab); a.pooled = at_(o.pooled); a.logits = at_(o.logits); a.beta = at_(o.beta); a.wab = at_(o.wab); a.g = f_(o.g); a.dt = f_(o.dt);
   a.B = (int32_t)c.B; a.T = (int32_t)c.T_; a.D = l.D; a.neg_eigval = l.neg; a.param_dtype = l.gate_dtype;
@@ -221,7 +222,7 @@ struct Rest {
   Mixed m;
 };
 
-void rest(const Call& c, const Front& f, const bool joint, const bool keep, const bool keep_states, const bool cache, Rest& r) {
+void rest(const Call& c, const Front& f, const bool joint, const Needs& needs, const bool keep_states, const bool cache, Rest& r) {
   const Layer& l = c.l;
   project(c, joint, r.raw);
   natsl_conv_seg s[3];
@@ -242,6 +243,8 @@ void rest(const Call& c, const Front& f, const bool joint, const bool keep, cons
   }
   must(l.conv_norm_fwd(s, 3, (int)c.B, (int)c.T_, l.W, l.act, l.norm_dtype, c.stream), "natsl_conv_norm_fwd");
   r.mix = mix_logits(c, r.y[0]);
+  if (l.delta && !needs.conv) drop(r.raw[0], r.raw[1], r.raw[2]);
+  if (!l.delta && !needs.want(W_MIX)) drop(r.y[0]);
   Mixed& m = r.m;
   if (l.delta) {
     m.q_a = r.n[0]; m.k_a = r.n[1]; m.v_a = r.y[2];
@@ -250,10 +253,18 @@ void rest(const Call& c, const Front& f, const bool joint, const bool keep, cons
     m.q_a = r.raw[0]; m.k_a = r.raw[1]; m.v_a = r.raw[2];
     m.q_l = r.n[0]; m.k_l = r.n[1]; m.v_l = r.y[2];
   }
-  mixed(c, f, keep, keep_states, cache, m);
+  mixed(c, f, needs.op, keep_states, cache, m);
+  drop(m.q_a, m.q_l);
+  if (!keep_states) drop(m.ws);
+  if (!cache) drop(m.k_a, m.v_a, m.k_l, m.v_l);
+  if (!needs.op) {
+    if (!needs.want(W_MIX)) drop(r.y[0]);
+    drop(r.raw[0], r.raw[1], r.raw[2], r.y[1], r.y[2], r.n[0], r.n[1]);
+  }
   r.tail = like(m.o_attn);
   must(l.norm_gate_logits_fwd(at_(m.o_lin), at_(m.o_attn), at_(r.raw[3]), at_(r.mix), at_(c.w[OUT_NORM1]), at_(c.w[OUT_NORM2]), at_(r.tail), c.rows * l.HQ, l.VA,
                               NATSL_BF16, l.out_eps, l.out_dtype, c.stream), "natsl_norm_gate_logits_fwd");
+  if (!needs.tail) drop(m.o_lin, m.o_attn, r.raw[3], r.mix);
   r.out = at::linear(r.tail.view({c.B, c.T_, l.H * l.V}), c.w[WO]);
 }
 
@@ -385,8 +396,8 @@ MixedGrads mixed_bwd(const Call& c, const Ts& s, const T& do_lin, const T& do_at
   return r;
 }
 
-// dout: c.x; grads: x, then the weights
-void backward(const Call& c, const T& x, const Ts& s, const Needs& need, const int invalid_attn, const int invalid_linear, const bool mix_pays, Ts& grads) {
+// dout: c.x; s: what the forward kept, dropped on the way; grads: x, then the weights
+void backward(const Call& c, const T& x, Ts& s, const Needs& need, const int invalid_attn, const int invalid_linear, const bool mix_pays, Ts& grads) {
   const Layer& l = c.l;
   const Ts& w = c.w;
   grads.assign(1 + WEIGHTS, T());
@@ -394,10 +405,11 @@ void backward(const Call& c, const T& x, const Ts& s, const Needs& need, const i
   const int64_t rows = c.rows, vd = l.H * l.V;
   const T d2 = c.x.reshape({rows, l.D}).contiguous();
   if (want(WO)) grads[1 + WO] = wgrad(c, s[TAIL].view({rows, vd}), d2);
+  drop(s[TAIL]);
   if (!need.tail) return;
-  const T dy = at::mm(d2, w[WO]);
+  T dy = at::mm(d2, w[WO]);
   // norm-gate
-  const T do_lin = like(s[O_LIN]), do_attn = like(s[O_ATTN]), dgate = like(s[GATE]), dmix = like(s[MIX]), dwn = at::empty({2, l.VA}, c.f32);
+  T do_lin = like(s[O_LIN]), do_attn = like(s[O_ATTN]), dgate = like(s[GATE]), dmix = like(s[MIX]), dwn = at::empty({2, l.VA}, c.f32);
   {
     const size_t n = l.norm_gate_bwd_workspace_bytes(rows * l.HQ, l.VA);
     const T ws = c.bytes(n);
@@ -410,15 +422,20 @@ void backward(const Call& c, const T& x, const Ts& s, const Needs& need, const i
       grads[1 + OUT_NORM2] = d.select(0, 1);
     }
   }
+  drop(dy, s[O_LIN], s[GATE], s[MIX]);
   MixedGrads m;
   if (need.op) m = mixed_bwd(c, s, do_lin, do_attn, invalid_attn, invalid_linear);
+  drop(do_lin, do_attn);
+  for (const Kept i : {O_ATTN, LSE, IDX, NBLK, TYPES, LOGITS, G, BETA, N_Q, N_K, Y_K, Y_V, STATES, V_NEW, WS}) drop(s[i]);
   // mixing logits, convolutions
-  const T dmix2 = dmix.view({rows, -1});
-  if (want(W_MIX)) grads[1 + W_MIX] = wgrad(c, s[Y_Q].view({rows, -1}), dmix2);
+  dmix = dmix.view({rows, -1});
+  if (want(W_MIX)) grads[1 + W_MIX] = wgrad(c, s[Y_Q].view({rows, -1}), dmix);
+  drop(s[Y_Q]);
   T dx[4], ddt;
-  dx[3] = dgate;
+  dx[3] = std::move(dgate);
   if (need.conv) {
-    const T dq_mix = narrow_bwd(c, dmix2, w[W_MIX], mix_pays);
+    const T dq_mix = narrow_bwd(c, dmix, w[W_MIX], mix_pays);
+    drop(dmix);
     natsl_conv_seg g[3];
     conv_segs(c, &s[RAW_Q], s[DT], g);
     for (int i = 0; i < 3; ++i) {
@@ -451,6 +468,7 @@ void backward(const Call& c, const T& x, const Ts& s, const Needs& need, const i
     const T ws = c.bytes(n);
     must(l.conv_norm_bwd(g, 3, (int)c.B, (int)c.T_, l.W, l.act, l.norm_dtype, at_(ws), n, c.stream), "natsl_conv_norm_bwd");
   }
+  drop(dmix, m.q_a, m.k_a, m.v_a, m.q_l, m.k_l, m.v_l, s[RAW_Q], s[RAW_K], s[RAW_V], s[DT]);
   // gates
   T dab;
   if (need.gates) {
@@ -462,6 +480,7 @@ void backward(const Call& c, const T& x, const Ts& s, const Needs& need, const i
     must(l.gates_bwd(at_(s[AB]), at_(w[A_LOG]), at_(w[DT_BIAS]), f_(m.g), at_(m.beta), f_(ddt), l.delta, at_(dab), at_(grads[1 + A_LOG]), at_(grads[1 + DT_BIAS]), at_(ws), n,
                      rows, l.H, (int)s[AB].size(2), l.neg, l.gate_dtype, c.stream), "natsl_gates_bwd");
   }
+  drop(m.g, m.beta, ddt, s[AB]);
   // selector
   T dl2;
   if (need.op) dl2 = m.logits.view({-1, l.NL});
@@ -477,6 +496,7 @@ void backward(const Call& c, const T& x, const Ts& s, const Needs& need, const i
   std::vector<T> dys(5);
   for (int i = 0; i < 4; ++i)
     if (dx[i].defined()) dys[i] = dx[i].view({rows, -1});
+  drop(dx[0], dx[1], dx[2], dx[3]);
   if (dab.defined()) dys[4] = dab.view({rows, -1});
   if (need.x()) {
     const int64_t ld = dab.size(2);
@@ -628,21 +648,19 @@ PyObject* natsl_layer_train(PyObject*, PyObject* const* a, Py_ssize_t n) {
   }
   Layer* l = layer_of(a[0]);
   if (!l || !tensors_of(a[2], w) || (a[6] != Py_None && !needs_of(a[6], of))) return nullptr;
-  const bool keep = !of.empty();
-  if (!keep) of.resize(1 + WEIGHTS);
   const Needs need(of, l->delta);
   const Call c(*l, THPVariable_Unpack(a[1]), w, stream_of(a[3]), stream_of(a[4]));
   const bool joint = PyObject_IsTrue(a[5]) > 0, states = need.op && PyObject_IsTrue(a[7]) > 0;
   Front f;
   Rest r;
   if (!run_free(*l, [&] {
-        f = front(c, keep ? &need : nullptr, false);
-        rest(c, f, joint, need.op, states, false, r);
+        f = front(c, need, false);
+        rest(c, f, joint, need, states, false, r);
       }))
     return nullptr;
   const Mixed& m = r.m;
   THPObjectPtr kept;
-  if (keep) {
+  if (!of.empty()) {
     Ts all(1 + WEIGHTS + KEPT);
     T* const s = all.data() + 1 + WEIGHTS;
     auto weights = [&](std::initializer_list<Weight> ws) {
@@ -689,13 +707,13 @@ PyObject* natsl_layer_train(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// layer_backward(layer, dout, what the forward kept, what wants a gradient (x, then the weights), stream, side, invalid attention, invalid linear, whether the
+// layer_backward(layer, dout, what the forward kept (a list, emptied: its tensors are dropped after their last use), what wants a gradient (x, then the weights), stream, side, invalid attention, invalid linear, whether the
 // one-pass kernel has the mixing logits' input gradient) -> gradients of x, then of the weights
 PyObject* natsl_layer_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Ts kept, grads;
   std::vector<bool> of;
-  if (n != 9 || !THPVariable_Check(a[1])) {
+  if (n != 9 || !THPVariable_Check(a[1]) || !PyList_Check(a[2])) {
     PyErr_SetString(PyExc_TypeError, "layer_backward(layer, dout, kept, needs, stream, side, invalid attention, invalid linear, mix)");
     return nullptr;
   }
@@ -705,9 +723,12 @@ PyObject* natsl_layer_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     PyErr_SetString(PyExc_ValueError, "layer_backward: another number of tensors than the forward gave");
     return nullptr;
   }
+  if (PyList_SetSlice(a[2], 0, PyList_GET_SIZE(a[2]), nullptr) < 0) return nullptr;
   const Needs need(of, l->delta);
   const T x = kept[0];
-  const Ts w(kept.begin() + 1, kept.begin() + 1 + WEIGHTS), s(kept.begin() + 1 + WEIGHTS, kept.end());
+  const Ts w(kept.begin() + 1, kept.begin() + 1 + WEIGHTS);
+  Ts s(kept.begin() + 1 + WEIGHTS, kept.end());
+  kept.clear();
   const Call c(*l, THPVariable_Unpack(a[1]), w, stream_of(a[4]), stream_of(a[5]));
   const int ia = PyObject_IsTrue(a[6]) > 0, il = PyObject_IsTrue(a[7]) > 0;
   const bool mix = PyObject_IsTrue(a[8]) > 0;
@@ -730,7 +751,7 @@ PyObject* natsl_layer_prompt_front(PyObject*, PyObject* const* a, Py_ssize_t n) 
   if (!l || !tensors_of(a[2], w)) return nullptr;
   const Call c(*l, THPVariable_Unpack(a[1]), w, stream_of(a[3]), nullptr);
   Front f;
-  if (!run_free(*l, [&] { f = front(c, nullptr, true); })) return nullptr;
+  if (!run_free(*l, [&] { f = front(c, Needs({}, l->delta), true); })) return nullptr;
   return tuple_of({f.g, f.beta, f.dt, f.logits, f.types, f.raw, f.counts, f.fraction});
   END_HANDLE_TH_ERRORS
 }
@@ -757,7 +778,7 @@ PyObject* natsl_layer_prompt_rest(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Rest r;
   Ts out(11);
   if (!run_free(*l, [&] {
-        rest(c, f, joint, false, false, cache, r);
+        rest(c, f, joint, Needs({}, l->delta), false, cache, r);
         out[0] = r.out;
         if (cache) {
           const Mixed& m = r.m;

@@ -647,6 +647,48 @@ def test_steps_of_which_a_part_trains(kind, train, follow):
         assert (p.grad is not None and bool(p.grad.any())) == n.startswith(train), n
 
 
+@pytest.mark.parametrize("kind,geometry,heads", [('gdn', '340M', {}), ('mamba', None, dict(hidden_size=512, head_dim=128, expand_v=0.5, num_heads=16, num_attn_heads=16))])
+@pytest.mark.parametrize("what", ['train', 'retain', 'eval', 'prompt'])
+def test_native_layer_needs_no_more_memory_than_its_steps(kind, geometry, heads, what, monkeypatch):
+    """The most that is allocated during a call: the native one drops a tensor behind its last use, as a graph of a node for each step does.  Sizes of
+    6 to 12 MB, so that what the allocator rounds up stays below two per cent."""
+    torch.manual_seed(1)
+    layer = _layer(kind, geometry, 'all', **heads)
+    layer.train(what in ('train', 'retain'))
+    x = torch.randn(4, 2048, layer.hidden_size, device=DEV).bfloat16().requires_grad_(layer.training)
+    do = torch.randn(x.shape, device=DEV).bfloat16()
+
+    def most():
+        out = []
+        for _ in range(2):                                 # (the first one allocates what is kept for good)
+            layer.zero_grad(set_to_none=True)
+            x.grad = None
+            torch.cuda.synchronize()
+            torch.cuda.reset_peak_memory_stats()
+            before = torch.cuda.memory_allocated()
+            if what == 'prompt':
+                with torch.no_grad():
+                    o = _generate(layer, kind, x, x.shape[1], ())
+            else:
+                with torch.set_grad_enabled(layer.training):
+                    o = layer(x)
+                o = o[0] if isinstance(o, tuple) else o
+                if layer.training:
+                    o.backward(do, retain_graph=what == 'retain')
+            torch.cuda.synchronize()
+            out.append(torch.cuda.max_memory_allocated() - before)
+            del o
+        return out[1]
+    native = most()
+    _stepwise(monkeypatch)
+    torch.cuda.empty_cache()
+    from neuralattentionsearchlinear_amd import _layer_step
+    _layer_step._watches.pop(layer)                        # (its plan has the native form)
+    steps = most()
+    print(kind, what, native >> 20, steps >> 20)
+    assert native <= 1.02 * steps
+
+
 @pytest.mark.parametrize("kind,T0", [('gdn', 128), ('gdn', 777), ('mamba', 64), ('mamba', 2113)])
 @pytest.mark.parametrize("ops", ['all', 'attn'])
 def test_native_prompt_is_its_steps(kind, T0, ops, monkeypatch):

@@ -185,7 +185,7 @@ __global__ __launch_bounds__(256) void short_conv_bwd_kernel(const void* x, cons
         for (int j = 0; j < W; ++j) acc += wt[j][c] * win[j][c];
         float da = 1.f;
         if (silu) {
-          const float sg = sigmoid_fast(acc);
+          const float sg = 1.f / (1.f + __expf(-acc));
           da = sg * (1.f + acc * (1.f - sg));
         }
         dp[c] = g[c] * da;

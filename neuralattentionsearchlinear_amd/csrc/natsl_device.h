@@ -143,9 +143,6 @@ NATSL_DEVICE void select_grad(const float x0, const float x1, const bool rounded
   d1 = y1 * (d1 - m);
 }
 
-// The convolutions' backward: the hardware's reciprocal is within an ulp, __expf's own error is larger, and a division is ten instructions
-NATSL_DEVICE float sigmoid_fast(const float x) { return __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
-
 // The softmax of a head's two mixing logits, rounded to bf16: what the mixing layer's separate softmax returns
 NATSL_DEVICE void mix_softmax(float& a, float& b) {
   const float mx = fmaxf(a, b), e0 = expf(a - mx), e1 = expf(b - mx);

@@ -170,9 +170,10 @@ __global__ __launch_bounds__(256) void conv_norm_kernel(const ConvNormParams p) 
 // Backward: dy = dy_a + dy_b + (backward of the norm, or of the number, of dy_norm), then dpre = dy act'(pre), dx[s] = sum_i w[W-1-i] dpre[s+i] +
 // dx_add[s], dw[j] = sum dpre[t] x[t-(W-1)+j].  pre and y are recomputed from x; a few rows of every input are requested at a time.  A thread
 // reads W-1 rows past its run (for dx of the run's last tokens) without adding them to its sums.
-// Bound by vector issue and the bytes alike (340M geometry 0.86 GB, a Mamba layer 1.48 GB at 8 x 4096): 215 -> 198 and 455 -> 329 us, 760M 2 x 3000
-// 76 -> 62, against a branch around every channel's activation, a division in it, the head sums through LDS, dx_add requested where it is used and
-// eight channels a thread.  Four channels with two rows ahead 206 and 346, with four 245 and 360 (175 registers: two waves a SIMD).
+// Bound by vector issue and the bytes alike (340M geometry 0.86 GB, a Mamba layer 1.48 GB at 8 x 4096): 215 -> 199 and 475 -> 385 us, 760M 2 x 3000
+// 76 -> 63, against a branch around every channel's activation, the head sums through LDS, dx_add requested where it is used and eight channels a
+// thread.  The activation's division is eight per cent of that (189, 357 and 58 with the hardware's reciprocal, which is off by an ulp).  Four
+// channels with two rows ahead 4 - 5 % slower, with four 10 - 24 % (175 registers: two waves a SIMD).
 // A thread has CH channels: four (eight hold 229 - 262 registers, two waves a SIMD or one), eight for heads of 512, which have to fit a wave.
 template <int W, bool SILU, int CH>
 __global__ __launch_bounds__(256) void conv_norm_bwd_kernel(const ConvNormParams p) {
@@ -236,7 +237,7 @@ __global__ __launch_bounds__(256) void conv_norm_bwd_kernel(const ConvNormParams
 #pragma unroll
       for (int j = 0; j < W; ++j) acc += wt[j][c] * win[j][c];
       if constexpr (SILU) {
-        const float sg = sigmoid_fast(acc);
+        const float sg = 1.f / (1.f + __expf(-acc));
         y[c] = acc * sg;
         da[c] = sg * (1.f + acc * (1.f - sg));
       } else {

@@ -224,6 +224,33 @@ def test_layer_rejects_unbuilt_paths():
         layer(x[:, :32].to(DEV).bfloat16())                       # decoding needs a cache
 
 
+def test_short_convolution_backward_divides():
+    """silu' in the backward of the fp32 convolution is formed with a correctly rounded division.  At x where x log2(e) rounds to a whole number k the
+    exponential is exactly 2^k, so sigmoid = 1 / (1 + 2^k) rounded once, and silu' = sigmoid (x (1 - sigmoid) + 1) with one rounding in the
+    parentheses: known bit by bit.  (A reciprocal that is good to an ulp differs at two of these points.)"""
+    import numpy as np
+    from neuralattentionsearchlinear_amd.modules import ShortConvolution
+    f32, xs, want = np.float32, [], []
+    for k in range(-22, 23):
+        x = f32(-k / 1.4426950408889634)
+        near = [x, *(np.nextafter(x, f32(d)) for d in (-100, 100))]
+        x = next((c for c in near if f32(-c * f32(1.4426950408889634)) == f32(k)), None)
+        if x is not None:
+            sg = f32(1) / (f32(1) + f32(2.0 ** k))
+            xs.append(float(x))
+            want.append(float(sg * f32(float(x) * float(f32(1) - sg) + 1.0)))
+    assert len(xs) >= 30
+    conv = ShortConvolution(8, 2, bias=False, activation='silu').to(DEV).float()
+    with torch.no_grad():
+        conv.weight.zero_()
+        conv.weight[:, 0, 1] = 1.0                          # y = silu(x)
+    x = torch.tensor(xs, device=DEV).view(1, -1, 1).repeat(1, 1, 8).requires_grad_(True)
+    y = conv(x)
+    y = y[0] if isinstance(y, tuple) else y
+    y.backward(torch.ones_like(y))
+    assert torch.equal(x.grad, torch.tensor(want, device=DEV).view(1, -1, 1).expand_as(x))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("W,D,act,bias", [(4, 768, 'silu', False), (4, 1536, 'silu', True), (3, 64, None, True), (2, 8, 'silu', False)])
 def test_short_convolution(W, D, act, bias, dtype):

@@ -521,6 +521,16 @@ int natsl_project_bwd(const natsl_project_seg* segs, int n_seg, const void* dpoo
  * bytes.  (The mixing logits' layer, src/nats/layers/natsl_attn_gdn.py:425-491.) */
 int natsl_narrow_linear_bwd(const void* dy, const void* w, void* dx, int64_t rows, int D, int N, natsl_stream_t stream);
 
+/* Which of several ways to the same product the layers take: rules on sizes, on the host, for every caller the same.  Alignments are the caller's.
+ * natsl_narrow_fwd_pays: the mixing logits [rows, N] = x [rows, D] w^T by natsl_layer_front.  natsl_narrow_linear_bwd_pays: dx by
+ * natsl_narrow_linear_bwd; few != 0: the selector's, over the block means.  natsl_narrow_wgrad_pays: dw [N, D] = dy [rows, N]^T x by natsl_narrow_wgrad
+ * (1; few only) or natsl_narrow_wgrad_split (2); alone: no other weight's gradient shares its launch of natsl_wgrad.  0: the other way (natsl_wgrad, the library). */
+int natsl_narrow_fwd_pays(int64_t rows, int D, int N);
+int natsl_narrow_linear_bwd_pays(int64_t rows, int D, int N, int few);
+int natsl_narrow_wgrad_pays(int64_t rows, int D, int N, int few, int alone);
+/* Whether natsl_project_bwd takes the projections' widths and the tensors' alignment; else dx is natsl_dx_init's and the wide products accumulate onto it. */
+int natsl_project_bwd_takes(const natsl_project_seg* segs, int n_seg, const void* dpool, const void* dx);
+
 /* natsl_gdn_chunk_fwd (is_delta) or natsl_mamba_chunk_fwd with NATSL_STATES_ONLY and no state of the last block.  beside: NULL, or
  * another stream of the same device that is made to wait for `stream` up to the kernel in front of the scan, for work that shares the
  * GPU with the scan. */

@@ -102,6 +102,10 @@ _SIGNATURES = {
     "natsl_project": (c_int, [c_void_p, c_int, c_void_p, c_int64, c_int, c_int, c_void_p]),
     "natsl_project_bwd": (c_int, [c_void_p, c_int, c_void_p, c_void_p] + [c_int] * 4 + [c_void_p]),
     "natsl_layer_front": (c_int, [c_void_p, c_void_p]),
+    "natsl_narrow_fwd_pays": (c_int, [c_int64, c_int, c_int]),
+    "natsl_narrow_linear_bwd_pays": (c_int, [c_int64, c_int, c_int, c_int]),
+    "natsl_narrow_wgrad_pays": (c_int, [c_int64, c_int, c_int, c_int, c_int]),
+    "natsl_project_bwd_takes": (c_int, [c_void_p, c_int, c_void_p, c_void_p]),
     "natsl_narrow_wgrad": (c_int, [c_void_p] * 3 + [c_int64, c_int, c_int, c_void_p]),
     "natsl_narrow_wgrad_workspace_bytes": (c_size_t, [c_int64, c_int, c_int]),
     "natsl_narrow_wgrad_split": (c_int, [c_void_p] * 3 + [c_int64, c_int, c_int, c_void_p, c_size_t, c_void_p]),

@@ -48,28 +48,18 @@ def _p(t):
     return None if t is None else t.data_ptr()
 
 
-def _narrow_split_pays(rows, N, D, alone):
-    """Whether natsl_narrow_wgrad_split forms dy [rows, N]^T x [rows, D].  us, library or natsl_wgrad / it: widths that are no multiple of 8, the library,
-    36 x 1152 over 2000 19 / 8.5, 6000 42 / 12, 32768 112 / 36; natsl_wgrad 24 x 768 over 2000 14 / 5.7, 32768 28 / 14, 32 x 2048 over 2000 16 / 7.3,
-    16000 24 / 21, 32768 39 / 46, 48 x 1536 over 16000 25 / 20, 32768 37 / 49, 64 x 2048 over 6000 20 / 24."""
-    if N > 64 or D % 2 or not 0 < rows < 1 << 31:
-        return False
-    return N % 8 != 0 or (alone and N <= 48 and rows * D <= 1 << 25)
-
-
 def weight_grads(x2, dys):
     """[dy_i^T x2 for dy_i [rows, n_i] in dys] (bf16; entries may be None): natsl_wgrad for widths that are multiples of 8, natsl_narrow_wgrad_split
     for narrow ones that are not, or that are alone, else torch."""
     rows, D = x2.shape
     out = [None] * len(dys)
-    todo = []
+    todo, L = [], _capi.lib()
     alone = sum(dy is not None for dy in dys) == 1
     for i, dy in enumerate(dys):
         if dy is None:
             continue
-        if _narrow_split_pays(rows, dy.shape[1], D, alone) and x2.data_ptr() % 4 == 0 and dy.dtype == x2.dtype == torch.bfloat16:
+        if L.natsl_narrow_wgrad_pays(rows, D, dy.shape[1], 0, alone) and x2.data_ptr() % 4 == 0 and dy.dtype == x2.dtype == torch.bfloat16:
             out[i] = torch.empty(dy.shape[1], D, dtype=torch.bfloat16, device=x2.device)
-            L = _capi.lib()
             n = L.natsl_narrow_wgrad_workspace_bytes(rows, D, dy.shape[1])
             ws = torch.empty(n, dtype=torch.uint8, device=x2.device)
             _capi.check(L.natsl_narrow_wgrad_split(dy.data_ptr(), x2.data_ptr(), out[i].data_ptr(), rows, D, dy.shape[1], ws.data_ptr(), n,
@@ -83,7 +73,6 @@ def weight_grads(x2, dys):
         segs = (_WgradSeg * len(todo))()
         for s, i in zip(segs, todo):
             s.dy, s.out, s.n, s.ld = dys[i].data_ptr(), out[i].data_ptr(), dys[i].shape[1], dys[i].shape[1]
-        L = _capi.lib()
         n = L.natsl_wgrad_workspace_bytes(segs, len(todo), rows, D)
         ws = torch.empty(n, dtype=torch.uint8, device=x2.device)
         _capi.check(L.natsl_wgrad(segs, len(todo), x2.data_ptr(), rows, D, D, ws.data_ptr(), n, _capi.stream_ptr(x2.device)), "natsl_wgrad")
@@ -215,13 +204,13 @@ def _project_bwd(x, wide, wab, n_a, n_b, dys, dpool, block, needs):
         dx = torch.empty_like(x)
         dp = None if dpool is None else dpool.contiguous()
         some = [(dy, w) for dy, w in zip(dys, (wq, wk, wv, wg, wab)) if dy is not None]
-        joint = sum(w.shape[0] for _, w in some) >= 128 and all(w.shape[0] % 32 == 0 for _, w in some) and \
-            _on_16(dx, *([] if dp is None else [dp]), *[t for pair in some for t in pair])
+        segs = _project_segs(*zip(*some)) if some else None
+        joint = _capi.lib().natsl_project_bwd_takes(segs, len(some), _p(dp), dx.data_ptr())
     if needs[0] and joint:
         # one pass over dx where four accumulating products and dx_init made five (340M geometry, 8 x 4096 tokens: 342 -> 237 us, 1 x 777
         # 56 -> 49).  Below some 500 tokens the one launch takes longer than the five (760M, 128 tokens: 54 / 68), but a step is the host's
         # there, which issues one for five: the layer at 760M, 300 tokens 1.45 -> 1.2 ms
-        rc = _capi.lib().natsl_project_bwd(_project_segs(*zip(*some)), len(some), _p(dp), dx.data_ptr(), B, T, D, block or T,
+        rc = _capi.lib().natsl_project_bwd(segs, len(some), _p(dp), dx.data_ptr(), B, T, D, block or T,
                                            _capi.stream_ptr(x.device))
         _capi.check(rc, "natsl_project_bwd")
     elif needs[0]:
@@ -299,18 +288,14 @@ class _ProjectAll(torch.autograd.Function):
 
 # ---- a narrow weight: the mixing logits' layer ------------------------------------------------------------------------------------
 def _narrow_pays(rows, N, D):
-    """Whether natsl_narrow_linear_bwd beats the library's product.  Measured (library / it, us, tensors in the cache): 8 x 512 over 16000
-    10.3 / 7.2, 24 x 768 over 2048 6.5 / 6.8, 6000 12.5 / 7.7, 32768 26.1 / 14.2, 36 x 1152 over 2048 7.3 / 7.9, 6000 11.1 / 9.2, 40 x 1024 over
-    6000 9.9 / 9.4 (from memory 10.2 / 10.7), 48 x 768 over 65536 39 / 29.  The library's kernels for 32 and 64 rows are as good or better
-    (32 x 512 over 6000 5.5 / 7.5, 64 x 1024 over 32768 20 / 27), 52 to 60 rows lose below 2^24 elements."""
-    return N % 32 != 0 and N <= 48 and rows * D >= (4 << 20 if N < 32 else 6 << 20)
+    """Whether natsl_narrow_linear_bwd forms dy [rows, N] w [N, D]."""
+    return bool(_capi.lib().natsl_narrow_linear_bwd_pays(rows, D, N, 0))
 
 
 def _narrow_bwd(dy, w, few=False):
-    """dy [rows, N] w.  few: the selector's, over the block means: a library product of this size is 4 to 8 us against 3 to 7, and 40 us of the host's
-    time against 5."""
+    """dy [rows, N] w.  few: the selector's, over the block means."""
     N, D = w.shape
-    if N % 4 or N > 48 or D % 128 or not (few or _narrow_pays(dy.shape[0], N, D)) or not _on_16(dy, w):
+    if not _capi.lib().natsl_narrow_linear_bwd_pays(dy.shape[0], D, N, few) or not _on_16(dy, w):
         return torch.mm(dy, w)
     dx = torch.empty(dy.shape[0], D, dtype=dy.dtype, device=dy.device)
     _capi.check(_capi.lib().natsl_narrow_linear_bwd(dy.data_ptr(), w.data_ptr(), dx.data_ptr(), dy.shape[0], D, N, _capi.stream_ptr(dy.device)),
@@ -319,15 +304,27 @@ def _narrow_bwd(dy, w, few=False):
 
 
 def _narrow_wgrad(dy, x):
-    """dy [rows, N]^T x [rows, D]: natsl_narrow_wgrad up to two thousand rows (library / it, us: 12 x 1536 over 94 6.7 / 2.7, 512 8.1 / 3.2, 2048
-    7.0 / 5.1, 4096 9.6 / 7.6; 32 x 1024 over 512 7.3 / 3.6, 2048 8.6 / 6.5; 64 x 2048 over 2048 15.5 / 9.0)."""
+    """dy [rows, N]^T x [rows, D] over the block means"""
     rows, N = dy.shape
     D = x.shape[1]
-    if N > 64 or D % 2 or rows > 2048:
+    if not _capi.lib().natsl_narrow_wgrad_pays(rows, D, N, 1, 0) or x.data_ptr() % 4:
         return torch.mm(dy.t(), x)
     dw = torch.empty(N, D, dtype=dy.dtype, device=dy.device)
     _capi.check(_capi.lib().natsl_narrow_wgrad(dy.data_ptr(), x.data_ptr(), dw.data_ptr(), rows, D, N, _capi.stream_ptr(dy.device)), "natsl_narrow_wgrad")
     return dw
+
+
+def _mix_logits(yq, w):
+    """yq [B, T, D] w^T [B, T, N]"""
+    B, T, D = yq.shape
+    if not _capi.lib().natsl_narrow_fwd_pays(B * T, D, w.shape[0]) or not _on_16(yq, w):
+        return F.linear(yq, w)
+    y = torch.empty(B, T, w.shape[0], dtype=torch.bfloat16, device=yq.device)
+    a = _FrontArgs()
+    a.x, a.wa, a.ab = yq.data_ptr(), w.data_ptr(), y.data_ptr()
+    a.B, a.T, a.D, a.NA, a.ld, a.param_dtype = 1, B * T, D, w.shape[0], w.shape[0], _capi.BF16
+    _capi.check(_capi.lib().natsl_layer_front(ctypes.byref(a), _capi.stream_ptr(yq.device)), "natsl_layer_front")
+    return y
 
 
 # ---- convolutions, norms, mixing logits --------------------------------------------------------------------------------------------
@@ -382,7 +379,7 @@ class _ConvNorm(torch.autograd.Function):
         raw = tuple(t.view(t.shape) for t in (q, k, v)) if f.raw_attention else (None, None, ys[2].detach())
         _, nq_, nk_, nv_, *nw, nnq, nnk, nmix, ndt = ctx.needs_input_grad
         cq, ck, cv = nq_ or nw[0] or nw[1], nk_ or nw[2] or nw[3], nv_ or nw[4] or nw[5]
-        mix = F.linear(ys[0], w_mix)
+        mix = _mix_logits(ys[0], w_mix)
         _only_for(ctx, (ys[0], cq), (ys[1], ck), (ys[2], cv or ndt), (ns[0], cq or nnq), (ns[1], ck or nnk), (mix, cq or nmix),
                   *zip(raw, (nq_, nk_, nv_ if f.raw_attention else cv)))
         return (ys[0], ys[1], ys[2], ns[0], ns[1], mix) + raw
@@ -564,7 +561,7 @@ class _Layer(torch.autograd.Function):
     def forward(ctx, f, flags, x, *weights):
         side, joint, states = flags
         out, fraction, kept = _capi.step_core().layer_train(f.native, x, weights, _capi.stream_ptr(x.device), side, joint, ctx.needs_input_grad[2:], states)
-        ctx.native, ctx.how, ctx.mix = f.native, f.how, f.w["w_mix"].shape
+        ctx.native, ctx.how = f.native, f.how
         ctx.save_for_backward(*kept)
         ctx.mark_non_differentiable(fraction)
         ctx.set_materialize_grads(False)
@@ -579,7 +576,7 @@ class _Layer(torch.autograd.Function):
         ctx.maybe_clear_saved_tensors()                    # (not where the graph is retained; nodes of their own are freed one by one, too)
         grads = _capi.step_core().layer_backward(
             ctx.native, dout.to(torch.bfloat16), kept, ctx.needs_input_grad[2:], stream, _beside(dout, ctx.how, stream), ctx.how["invalid_attn"],
-            ctx.how["invalid_linear"], _narrow_pays(dout.shape[0] * dout.shape[1], *ctx.mix))
+            ctx.how["invalid_linear"])
         return (None, None, *grads)
 
 
@@ -681,7 +678,7 @@ class FastFront:
         if self.grad(*args):
             return _ConvNorm.apply(self, *args) + (None,)
         ys, ns, new = _conv_norm(self, (q, k, v), states, want_states, dt)
-        return ys[0], ys[1], ys[2], ns[0], ns[1], F.linear(ys[0], w["w_mix"]), *((q, k, v) if self.raw_attention else (None, None, ys[2])), new
+        return ys[0], ys[1], ys[2], ns[0], ns[1], _mix_logits(ys[0], w["w_mix"]), *((q, k, v) if self.raw_attention else (None, None, ys[2])), new
 
     def gates(self, ab):
         if self.grad(ab, self.w["a_log"], self.w["dt_bias"]):

@@ -27,7 +27,7 @@ namespace {
   X(mixed_fwd) X(mixed_workspace_bytes) X(norm_gate_logits_fwd) X(norm_gate_logits_bwd) X(norm_gate_bwd_workspace_bytes) X(wgrad)           \
   X(wgrad_workspace_bytes) X(narrow_linear_bwd) X(narrow_wgrad) X(narrow_wgrad_workspace_bytes) X(narrow_wgrad_split) X(gates_bwd) X(gates_bwd_workspace_bytes) X(dx_init) X(softmax_sparse_bwd)  \
   X(softmax_bwd_workspace_bytes) X(linear_workspace_bytes) X(linear_chunk_states) X(linear_chunk_bwd_steps)            \
-  X(block_grads_logits) X(order_streams)
+  X(block_grads_logits) X(order_streams) X(narrow_fwd_pays) X(narrow_linear_bwd_pays) X(narrow_wgrad_pays) X(project_bwd_takes)
 
 struct Layer {
 #define X(n) decltype(&natsl_##n) n;
@@ -157,12 +157,10 @@ void conv_segs(const Call& c, const T* raw, const T& dt, natsl_conv_seg (&s)[3])
   }
 }
 
-// The mixing logits: the one-pass kernel up to 32 rows of the weight (24 x 768 over 32768 tokens 20 -> 16 us, 32 x 2048 over 16000 24 -> 21), and for a
-// few thousand tokens of more, where it takes 3 us more than the library's kernel but 30 less of the host's time.
 T mix_logits(const Call& c, const T& yq) {
   const T& w = c.w[W_MIX];
   const int64_t n = w.size(0), d = w.size(1);
-  if (n > 64 || d % 32 || n % 2 || (n > 32 && c.rows > 4096) || !on16(w)) return at::linear(yq, w);
+  if (!c.l.narrow_fwd_pays(c.rows, (int)d, (int)n) || !on16(w)) return at::linear(yq, w);
   T y = at::empty({c.B, c.T_, n}, c.bf16);
   natsl_front a{};
   a.x = at_(yq); a.wa = at_(w); a.ab = at_(y);
@@ -273,7 +271,6 @@ void rest(const Call& c, const Front& f, const bool joint, const Needs& needs, c
 enum Kept { AB, WAB, POOLED, LOGITS, TYPES, RAW_Q, RAW_K, RAW_V, GATE, Y_Q, Y_K, Y_V, N_Q, N_K, MIX, G, BETA, DT, O_LIN, O_ATTN, LSE, IDX, NBLK, TAIL, STATES, V_NEW, WS, KEPT };
 
 // dy_i [rows, n_i]^T x [rows, D], one launch for those whose widths are multiples of 8; a narrow one that is not, or that is alone, by itself
-// (where: weight_grads of _front.py)
 void wgrads(const Call& c, const T& x, const std::vector<T>& dys, std::vector<T>& out) {
   const int64_t rows = x.size(0), D = x.size(1);
   out.assign(dys.size(), T());
@@ -283,7 +280,7 @@ void wgrads(const Call& c, const T& x, const std::vector<T>& dys, std::vector<T>
     const T& dy = dys[i];
     if (!dy.defined()) continue;
     const int64_t N = dy.size(1);
-    if (N <= 64 && D % 2 == 0 && (N % 8 || (alone && N <= 48 && rows * D <= int64_t(1) << 25))) {
+    if (c.l.narrow_wgrad_pays(rows, (int)D, (int)N, 0, alone) && !(reinterpret_cast<uintptr_t>(x.data_ptr()) & 3)) {
       out[i] = at::empty({N, D}, c.bf16);
       const size_t n = c.l.narrow_wgrad_workspace_bytes(rows, (int)D, (int)N);
       const T ws = c.bytes(n);
@@ -308,9 +305,9 @@ T wgrad(const Call& c, const T& x, const T& dy) {
   return out[0];
 }
 
-T narrow_bwd(const Call& c, const T& dy, const T& w, const bool pays) {
+T narrow_bwd(const Call& c, const T& dy, const T& w, const bool few) {
   const int64_t N = w.size(0), D = w.size(1);
-  if (N % 4 || N > 48 || D % 128 || !pays || !on16(dy) || !on16(w)) return at::mm(dy, w);
+  if (!c.l.narrow_linear_bwd_pays(dy.size(0), (int)D, (int)N, few) || !on16(dy) || !on16(w)) return at::mm(dy, w);
   T dx = at::empty({dy.size(0), D}, c.bf16);
   must(c.l.narrow_linear_bwd(at_(dy), at_(w), at_(dx), dy.size(0), (int)D, (int)N, c.stream), "natsl_narrow_linear_bwd");
   return dx;
@@ -397,7 +394,7 @@ MixedGrads mixed_bwd(const Call& c, const Ts& s, const T& do_lin, const T& do_at
 }
 
 // dout: c.x; s: what the forward kept, dropped on the way; grads: x, then the weights
-void backward(const Call& c, const T& x, Ts& s, const Needs& need, const int invalid_attn, const int invalid_linear, const bool mix_pays, Ts& grads) {
+void backward(const Call& c, const T& x, Ts& s, const Needs& need, const int invalid_attn, const int invalid_linear, Ts& grads) {
   const Layer& l = c.l;
   const Ts& w = c.w;
   grads.assign(1 + WEIGHTS, T());
@@ -434,7 +431,7 @@ void backward(const Call& c, const T& x, Ts& s, const Needs& need, const int inv
   T dx[4], ddt;
   dx[3] = std::move(dgate);
   if (need.conv) {
-    const T dq_mix = narrow_bwd(c, dmix, w[W_MIX], mix_pays);
+    const T dq_mix = narrow_bwd(c, dmix, w[W_MIX], false);
     drop(dmix);
     natsl_conv_seg g[3];
     conv_segs(c, &s[RAW_Q], s[DT], g);
@@ -486,7 +483,7 @@ void backward(const Call& c, const T& x, Ts& s, const Needs& need, const int inv
   if (need.op) dl2 = m.logits.view({-1, l.NL});
   if (want(WN)) {
     const int64_t r = dl2.size(0), n = l.NL;
-    if (n > 64 || l.D % 2 || r > 2048) {
+    if (!l.narrow_wgrad_pays(r, l.D, (int)n, 1, 0)) {
       grads[1 + WN] = at::mm(dl2.t(), s[POOLED]);
     } else {
       grads[1 + WN] = at::empty({n, l.D}, c.bf16);
@@ -501,14 +498,12 @@ void backward(const Call& c, const T& x, Ts& s, const Needs& need, const int inv
   if (need.x()) {
     const int64_t ld = dab.size(2);
     const T dpool = narrow_bwd(c, dl2, w[WN], true), dX = c.sized(l.D);
-    bool whole = true;
     natsl_project_seg segs[5];
     for (int i = 0; i < 5; ++i) {
       const T& ww = i < 4 ? w[WQ + i] : s[WAB];
-      whole = whole && ww.size(0) % 32 == 0 && on16(ww) && on16(dys[i]);
       segs[i] = {at_(dys[i]), at_(ww), (int32_t)ww.size(0), (int32_t)ww.size(0)};
     }
-    if (whole && on16(dpool)) {
+    if (l.project_bwd_takes(segs, 5, at_(dpool), at_(dX))) {
       must(l.project_bwd(segs, 5, at_(dpool), at_(dX), (int)c.B, (int)c.T_, l.D, 64, c.stream), "natsl_project_bwd");
     } else {
       must(l.dx_init(at_(dys[4]), at_(s[WAB]), at_(dpool), at_(dX), (int)c.B, (int)c.T_, l.D, (int)ld, (int)ld, 64, c.stream), "natsl_dx_init");
@@ -707,14 +702,14 @@ PyObject* natsl_layer_train(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// layer_backward(layer, dout, what the forward kept (a list, emptied: its tensors are dropped after their last use), what wants a gradient (x, then the weights), stream, side, invalid attention, invalid linear, whether the
-// one-pass kernel has the mixing logits' input gradient) -> gradients of x, then of the weights
+// layer_backward(layer, dout, what the forward kept (a list, emptied: its tensors are dropped after their last use), what wants a gradient (x, then the weights), stream, side, invalid attention, invalid linear)
+// -> gradients of x, then of the weights
 PyObject* natsl_layer_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Ts kept, grads;
   std::vector<bool> of;
-  if (n != 9 || !THPVariable_Check(a[1]) || !PyList_Check(a[2])) {
-    PyErr_SetString(PyExc_TypeError, "layer_backward(layer, dout, kept, needs, stream, side, invalid attention, invalid linear, mix)");
+  if (n != 8 || !THPVariable_Check(a[1]) || !PyList_Check(a[2])) {
+    PyErr_SetString(PyExc_TypeError, "layer_backward(layer, dout, kept, needs, stream, side, invalid attention, invalid linear)");
     return nullptr;
   }
   Layer* l = layer_of(a[0]);
@@ -731,8 +726,7 @@ PyObject* natsl_layer_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   kept.clear();
   const Call c(*l, THPVariable_Unpack(a[1]), w, stream_of(a[4]), stream_of(a[5]));
   const int ia = PyObject_IsTrue(a[6]) > 0, il = PyObject_IsTrue(a[7]) > 0;
-  const bool mix = PyObject_IsTrue(a[8]) > 0;
-  if (!run_free(*l, [&] { backward(c, x, s, need, ia, il, mix, grads); })) return nullptr;
+  if (!run_free(*l, [&] { backward(c, x, s, need, ia, il, grads); })) return nullptr;
   for (int i = 0; i <= WEIGHTS; ++i)
     if (!of[(size_t)i]) grads[(size_t)i] = T();
   return tuple_of(grads);

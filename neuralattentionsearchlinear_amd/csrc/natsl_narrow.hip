@@ -393,6 +393,32 @@ static int narrow_wgrad_parts(const int64_t rows) {
 
 using namespace natsl;
 
+// The one-pass kernel up to 32 rows of the weight (24 x 768 over 32768 tokens 20 -> 16 us, 32 x 2048 over 16000 24 -> 21), and for a few thousand
+// tokens of more, where it takes 3 us more than the library's kernel but 30 less of the host's time.
+extern "C" int natsl_narrow_fwd_pays(const int64_t rows, const int D, const int N) {
+  return N > 0 && N <= 64 && N % 2 == 0 && D > 0 && D % 32 == 0 && rows > 0 && rows < 1ll << 30 && (N <= 32 || rows <= 4096);
+}
+
+// Measured (library / natsl_narrow_linear_bwd, us, tensors in the cache): 8 x 512 over 16000 10.3 / 7.2, 24 x 768 over 2048 6.5 / 6.8, 6000 12.5 / 7.7,
+// 32768 26.1 / 14.2, 36 x 1152 over 2048 7.3 / 7.9, 6000 11.1 / 9.2, 40 x 1024 over 6000 9.9 / 9.4 (from memory 10.2 / 10.7), 48 x 768 over 65536
+// 39 / 29.  The library's kernels for 32 and 64 rows are as good or better (32 x 512 over 6000 5.5 / 7.5, 64 x 1024 over 32768 20 / 27), 52 to 60
+// rows lose below 2^24 elements.  few: a library product of the selector's size is 4 to 8 us against 3 to 7, and 40 us of the host's time against 5.
+extern "C" int natsl_narrow_linear_bwd_pays(const int64_t rows, const int D, const int N, const int few) {
+  if (N <= 0 || N % 4 || N > NARROW_MAX || D <= 0 || D % 128 || rows <= 0) return 0;
+  return few || (N % 32 != 0 && rows * D >= (N < 32 ? 4 << 20 : 6 << 20));
+}
+
+// few, over the block means (library / natsl_narrow_wgrad, us): 12 x 1536 over 94 6.7 / 2.7, 512 8.1 / 3.2, 2048 7.0 / 5.1, 4096 9.6 / 7.6;
+// 32 x 1024 over 512 7.3 / 3.6, 2048 8.6 / 6.5; 64 x 2048 over 2048 15.5 / 9.0.
+// Else the split product (the other way / it, us): widths that are no multiple of 8, which leaves the library, 36 x 1152 over 2000 19 / 8.5, 6000 42 / 12,
+// 32768 112 / 36; natsl_wgrad 24 x 768 over 2000 14 / 5.7, 32768 28 / 14, 32 x 2048 over 2000 16 / 7.3, 16000 24 / 21, 32768 39 / 46, 48 x 1536 over
+// 16000 25 / 20, 32768 37 / 49, 64 x 2048 over 6000 20 / 24.
+extern "C" int natsl_narrow_wgrad_pays(const int64_t rows, const int D, const int N, const int few, const int alone) {
+  if (N <= 0 || N > 64 || D <= 0 || D % 2 || rows <= 0 || rows > 0x7fffff00ll) return 0;
+  if (few) return rows <= 2048;
+  return N % 8 != 0 || (alone && N <= 48 && rows * D <= 1ll << 25) ? 2 : 0;
+}
+
 static int narrow_wgrad(const char* what, const void* dy, const void* x, void* dw, const int64_t rows, const int D, const int N, float* parts, hipStream_t s) {
   if (!dy || !x || !dw) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
   if (rows <= 0 || D <= 0 || N <= 0) return fail(NATSL_ERR_INVALID, "%s: non-positive dimension", what);

@@ -385,6 +385,20 @@ extern "C" int natsl_project(const natsl_project_seg* segs, int n_seg, const voi
   return launch_project_any<false, false>(p, reinterpret_cast<hipStream_t>(stream), what);
 }
 
+// (as the whole of natsl_project_bwd's conditions on these: it refuses what this does not take)
+extern "C" int natsl_project_bwd_takes(const natsl_project_seg* segs, const int n_seg, const void* dpool, const void* dx) {
+  if (!segs || n_seg <= 0 || n_seg > NATSL_PROJECT_SEGS) return 0;
+  uintptr_t low = (uintptr_t)dpool | (uintptr_t)dx;
+  long long columns = 0;
+  for (int i = 0; i < n_seg; ++i) {
+    const natsl_project_seg& s = segs[i];
+    if (s.n <= 0 || s.n % PJ_K || s.ld < s.n || s.ld % 8) return 0;
+    columns += s.n;
+    low |= (uintptr_t)s.y | (uintptr_t)s.w;
+  }
+  return columns >= 4 * PJ_K && low % 16 == 0;
+}
+
 extern "C" int natsl_project_bwd(const natsl_project_seg* segs, int n_seg, const void* dpool, void* dx, int B, int T, int D, int block, natsl_stream_t stream) {
   const char* what = "natsl_project_bwd";
   if (B <= 0 || T <= 0 || block <= 0) return fail(NATSL_ERR_INVALID, "%s: non-positive dimension", what);

@@ -191,3 +191,21 @@ def test_layer_plans_keep_nothing_alive():
     assert not any(r() is not None for r in old)
     again = watch(layer)
     assert again is not seen and again is not None and watch(layer) is again
+
+
+def test_which_way_a_narrow_product_goes():
+    """The rules that every caller takes (natsl_narrow_*_pays, natsl_project_bwd_takes) at their edges, and that none takes what its kernel refuses."""
+    from neuralattentionsearchlinear_amd._front import _ProjectSeg
+    L = _lib()
+    fwd, bwd, wgrad = L.natsl_narrow_fwd_pays, L.natsl_narrow_linear_bwd_pays, L.natsl_narrow_wgrad_pays
+    assert fwd(1 << 20, 768, 32) and not fwd(4097, 768, 34) and fwd(4096, 768, 64) and not fwd(64, 768, 66) and not fwd(64, 760, 24) and not fwd(64, 768, 23)
+    assert not fwd(0, 768, 24) and not fwd(1 << 31, 768, 24)
+    assert bwd(6000, 768, 24, 0) and not bwd(2048, 768, 24, 0) and bwd(1, 768, 24, 1) and bwd(1, 128, 32, 1) and not bwd(1, 128, 52, 1) and not bwd(1, 96, 24, 1)
+    assert not bwd(0, 768, 24, 1) and not bwd(6000, 768, 22, 1)
+    assert wgrad(2048, 1536, 12, 1, 0) == 1 and wgrad(2049, 1536, 12, 1, 0) == 0 and wgrad(64, 1535, 12, 1, 0) == 0 and wgrad(64, 1536, 65, 1, 1) == 0
+    assert wgrad(32768, 1152, 36, 0, 0) == 2 and wgrad(32768, 768, 24, 0, 0) == 0 and wgrad(32768, 768, 24, 0, 1) == 2 and wgrad(6000, 2048, 64, 0, 1) == 0
+    assert wgrad(1 << 15, 1024, 24, 0, 1) == 2 and wgrad((1 << 15) + 1, 1024, 24, 0, 1) == 0 and wgrad(1 << 31, 64, 12, 0, 1) == 0
+    segs = lambda *ns, y=1 << 20: (_ProjectSeg * len(ns))(*[_ProjectSeg(y, 1 << 20, n, n) for n in ns])
+    takes = lambda s, dpool=1 << 20, dx=1 << 20: L.natsl_project_bwd_takes(s, len(s), dpool, dx)
+    assert takes(segs(768, 32)) and takes(segs(64, 64), None) and not takes(segs(64, 32)) and not takes(segs(768, 16)) and not takes(segs(768, y=(1 << 20) + 8))
+    assert not takes(segs(768), (1 << 20) + 2) and not takes(segs(768), None, 8) and not takes(segs(*[768] * 9)) and not L.natsl_project_bwd_takes(None, 0, None, None)

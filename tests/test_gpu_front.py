@@ -533,6 +533,35 @@ def test_native_layer_is_its_steps(kind, geometry, B, T, more, side, keep, monke
             assert g[n].shape == b.shape and g[n].dtype == b.dtype and rel_l2(g[n].float(), b.float()) <= (2e-2 if n == 'nats_layer.weight' else 5e-3), n
 
 
+@pytest.mark.parametrize("kind,geometry,B,T", [('gdn', '340M', 2, 1999), ('gdn', '760M', 1, 1100), ('gdn', '760M', 4, 1100), ('mamba', None, 3, 700)])
+def test_native_layer_takes_the_steps_products(kind, geometry, B, T, monkeypatch):
+    """One rule chooses each product, whichever way the layer runs: the same bits in training, as native call and as steps, and in evaluation with
+    gradients (always the steps) and without.  (What the selector's gradient, summed by atomic additions, enters is left to
+    test_native_layer_is_its_steps.)"""
+    from neuralattentionsearchlinear_amd import _front
+    torch.manual_seed(T)
+    layer, other = _layer(kind, geometry, 'all'), _layer(kind, geometry, 'all')
+    other.load_state_dict(layer.state_dict())
+    x, do = (torch.randn(B, T, layer.hidden_size, device=DEV).bfloat16() for _ in range(2))
+    calls, inner = [], _front._Layer.forward
+    monkeypatch.setattr(_front._Layer, 'forward', staticmethod(lambda *a: (calls.append(1), inner(*a))[1]))
+    native = _train(layer.train(), x, do)
+    first = lambda o: o[0] if isinstance(o, tuple) else o
+    evaluated = [first(layer.eval()(x))]
+    with torch.no_grad():
+        evaluated.append(first(layer(x)))
+    _stepwise(monkeypatch)
+    library, linear = [], _front.F.linear
+    monkeypatch.setattr(_front.F, 'linear', lambda a, w, *more: (library.append(w.data_ptr()), linear(a, w, *more))[1])
+    steps = _train(other.train(), x, do)
+    w = other.nats_out_weights_layer.weight
+    assert (w.data_ptr() in library) != bool(_front._capi.lib().natsl_narrow_fwd_pays(B * T, w.shape[1], w.shape[0]))
+    assert calls == [1] and evaluated[0].requires_grad and all(torch.equal(native['out'], o) for o in evaluated)
+    for n, want in steps.items():
+        if n not in ('x', 'nats_layer.weight'):
+            assert torch.equal(native[n], want), n
+
+
 @pytest.mark.parametrize("kind", ['gdn', 'mamba'])
 def test_native_layer_under_autograd(kind):
     """What autograd asks of the one node: gradients for what wants them only, saved tensors through hooks, a second backward, changed weights
@@ -613,7 +642,8 @@ def test_native_layer_of_which_a_part_trains(kind, train, monkeypatch):
     other.load_state_dict(layer.state_dict())
     _stepwise(monkeypatch)
     _, most = forward(other)
-    assert calls == [1] and held <= most + (64 << 10), (held, most)
+    # (the allocator gives a tensor a block with up to 1 MiB more than it asks for; up to 27 tensors are kept, of 2 MB and more)
+    assert calls == [1] and held <= most + most // 2, (held, most)
 
 
 @pytest.mark.parametrize("kind", ['gdn', 'mamba'])

@@ -564,6 +564,12 @@ bool tensors_of(PyObject* seq, Ts& out) {
   }
   return true;
 }
+bool weights_of(PyObject* seq, Ts& out) {
+  if (!tensors_of(seq, out)) return false;
+  if ((int)out.size() == WEIGHTS) return true;
+  PyErr_Format(PyExc_ValueError, "%d weights, got %d", (int)WEIGHTS, (int)out.size());
+  return false;
+}
 // body() without the interpreter's lock; an entry point's failure becomes the exception that `check` raises
 template <class F>
 bool run_free(const Layer& l, F body) {
@@ -642,7 +648,7 @@ PyObject* natsl_layer_train(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return nullptr;
   }
   Layer* l = layer_of(a[0]);
-  if (!l || !tensors_of(a[2], w) || (a[6] != Py_None && !needs_of(a[6], of))) return nullptr;
+  if (!l || !weights_of(a[2], w) || (a[6] != Py_None && !needs_of(a[6], of))) return nullptr;
   const Needs need(of, l->delta);
   const Call c(*l, THPVariable_Unpack(a[1]), w, stream_of(a[3]), stream_of(a[4]));
   const bool joint = PyObject_IsTrue(a[5]) > 0, states = need.op && PyObject_IsTrue(a[7]) > 0;
@@ -742,7 +748,7 @@ PyObject* natsl_layer_prompt_front(PyObject*, PyObject* const* a, Py_ssize_t n) 
     return nullptr;
   }
   Layer* l = layer_of(a[0]);
-  if (!l || !tensors_of(a[2], w)) return nullptr;
+  if (!l || !weights_of(a[2], w)) return nullptr;
   const Call c(*l, THPVariable_Unpack(a[1]), w, stream_of(a[3]), nullptr);
   Front f;
   if (!run_free(*l, [&] { f = front(c, Needs({}, l->delta), true); })) return nullptr;
@@ -760,7 +766,7 @@ PyObject* natsl_layer_prompt_rest(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return nullptr;
   }
   Layer* l = layer_of(a[0]);
-  if (!l || !tensors_of(a[2], w) || !tensors_of(a[3], fr)) return nullptr;
+  if (!l || !weights_of(a[2], w) || !tensors_of(a[3], fr)) return nullptr;
   if (fr.size() != 8) {
     PyErr_SetString(PyExc_ValueError, "layer_rest: what layer_front gave");
     return nullptr;

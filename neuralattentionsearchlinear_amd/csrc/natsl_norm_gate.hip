@@ -91,12 +91,14 @@ __global__ __launch_bounds__(256) void norm_gate_kernel(const bf16_t* x1, const 
 // A workgroup takes ROWS consecutive rows; a lane group keeps its columns' share of dw1, dw2 in registers over the rows it
 // handles, the groups' shares are added in a fixed order through LDS, and one row of partial sums per workgroup goes to
 // part[workgroup][2][D]; colsum_reduce_kernel adds those up (no atomics: the same bits on every run).
+constexpr int NG_BWD_ROWS = 128;   // rows per workgroup
 template <int LANES, int PER>
 __global__ __launch_bounds__(256) void norm_gate_bwd_kernel(const bf16_t* x1, const bf16_t* x2, const bf16_t* gate, const bf16_t* xw,
                                                             const void* w1, const void* w2, const bf16_t* dy, bf16_t* dx1, bf16_t* dx2,
                                                             bf16_t* dgate, float* dxw, bf16_t* dlogits, float* part, long long rows, int rows_per_wg,
                                                             float eps, int w_dtype) {
   constexpr int D = LANES * PER * 8, G = 256 / LANES;
+  static_assert(NG_BWD_ROWS % G == 0, "a workgroup's last pass would take the next one's rows, too");
   __shared__ float acc_s[G][2][D];
   const int grp = threadIdx.x / LANES, seg = threadIdx.x % LANES;
   float wa[PER][8], wb[PER][8], dwa[PER][8], dwb[PER][8];
@@ -258,8 +260,6 @@ __global__ __launch_bounds__(1024) void colsum_reduce_kernel(const float* part, 
     out[i] = t;
   }
 }
-
-constexpr int NG_BWD_ROWS = 128;   // rows per workgroup of the backward
 
 }  // namespace natsl
 

@@ -76,6 +76,40 @@ def test_norm_gate_backward_of_any_number_of_rows(D, rows):
         assert torch.equal(a, b[:, :rows]), name
 
 
+@pytest.mark.parametrize("D", [32, 64, 96, 128, 192, 256, 384, 512])
+@pytest.mark.parametrize("rows", [1, 127, 129, 257])
+@pytest.mark.parametrize("logits", [False, True])
+def test_norm_gate_backward_sums_every_row_once(D, rows, logits):
+    """The weights' gradients are sums over the rows: around the 128 rows of a workgroup, with mixing weights and with the layers' mixing logits, against
+    float64 autograd; with the rows' own gradients."""
+    from neuralattentionsearchlinear_amd import _capi
+    g = torch.Generator().manual_seed(D + rows)
+    x1, x2, gate, dy = (torch.randn(rows, D, generator=g).bfloat16() for _ in range(4))
+    mix = torch.randn(rows, 2, generator=g).bfloat16()
+    if not logits:
+        mix = torch.softmax(mix.float(), -1).bfloat16()
+    w = 1 + 0.1 * torch.randn(2, D, generator=g)
+    weights = torch.softmax(mix.float(), -1).bfloat16() if logits else mix                   # (rounded, as the mixing layer's softmax is)
+    a, b, gt, xw, w6 = (t.double().requires_grad_(True) for t in (x1, x2, gate, weights, w))
+    n1, n2 = (t * torch.rsqrt((t * t).mean(-1, keepdim=True) + 1e-5) for t in (a, b))
+    ((n1 * w6[0] * xw[:, :1] + n2 * w6[1] * xw[:, 1:]) * gt * torch.sigmoid(gt)).backward(dy.double())
+    t = [v.to(DEV) for v in (x1, x2, gate, mix, w[0].contiguous(), w[1].contiguous(), dy)]
+    dx1, dx2, dgate = (torch.empty_like(t[0]) for _ in range(3))
+    dmix = torch.empty(rows, 2, device=DEV, dtype=torch.bfloat16 if logits else torch.float32)
+    dw = torch.empty(2, D, device=DEV)
+    L, P = _capi.lib(), _capi.ptr
+    n = L.natsl_norm_gate_bwd_workspace_bytes(rows, D)
+    ws = torch.empty(n, dtype=torch.uint8, device=DEV)
+    call = L.natsl_norm_gate_logits_bwd if logits else L.natsl_norm_gate_bwd
+    _capi.check(call(*map(P, t), P(dx1), P(dx2), P(dgate), P(dmix), P(dw), P(dw[1]), P(ws), n, rows, D, _capi.BF16, 1e-5, _capi.F32,
+                     _capi.stream_ptr(torch.device(DEV))), "natsl_norm_gate_bwd")
+    m, of = xw.detach(), xw.grad
+    # sums of at most 257 products in fp32: far below 1e-5 of the norm; the other gradients are rounded to bf16, 2^-9 relative
+    for name, got, ref, bound in (('dw', dw, w6.grad, 1e-5), ('dx1', dx1, a.grad, 2 ** -8), ('dx2', dx2, b.grad, 2 ** -8), ('dgate', dgate, gt.grad, 2 ** -8),
+                                  ('dmix', dmix, m * (of - (m * of).sum(-1, keepdim=True)) if logits else of, 2 ** -8 if logits else 1e-5)):
+        assert rel_l2(got.double().cpu(), ref) <= bound, (name, rel_l2(got.double().cpu(), ref))
+
+
 # head geometry of the two published model configurations (experiments/configs/natsl_340M.json, natsl_760M.json):
 # linear heads K 128 / V 256 resp. K 192 / V 384, attention view K 64 / V 128 in both
 PUBLISHED = {'340M': dict(hidden_size=1024, head_dim=128, num_heads=6, num_attn_heads=12, norm_eps=1e-6),

@@ -4,10 +4,21 @@ import pytest
 import torch
 
 from tests._util import rel_l2
-from tests.test_gpu_layer_step import _generate, _layer
+from tests.test_gpu_layer_step import _generate as _generate_views, _layer
 
 pytestmark = pytest.mark.gpu
 DEV = 'cuda:0'
+
+
+def _generate(layer, kind, x, T0, sizes):
+    """_generate of the steps' tests on hidden states of their own, as a model's layers hand them on (the fused front and the native calls take contiguous
+    ones; a view of several sequences' first tokens is not)."""
+    whole = layer.forward
+    try:
+        layer.forward = lambda t, **kw: whole(t.contiguous(), **kw)
+        return _generate_views(layer, kind, x, T0, sizes)
+    finally:
+        del layer.forward
 
 
 def _general(monkeypatch):
@@ -53,7 +64,14 @@ def test_front_on_a_cache(kind, T0, sizes, monkeypatch):
     layer = _layer(kind, None, 'all')
     torch.manual_seed(T0)
     x = torch.randn(2, T0 + sum(sizes), layer.hidden_size, device=DEV).bfloat16()
+    from neuralattentionsearchlinear_amd import _front
+    calls, tail = [], _front.FastFront.tail
+    monkeypatch.setattr(_front.FastFront, 'tail', lambda *a: (calls.append(1), tail(*a))[1])
+    native = _front.FastFront.prompt
+    monkeypatch.setattr(_front.FastFront, 'prompt', lambda *a: (calls.append(1), native(*a))[1])
     fast, cf = _generate(layer, kind, x, T0, sizes)
+    # (pieces of fewer than 64 tokens are steps)
+    assert len(calls) == 1 + sum(n >= 64 for n in sizes)
     _general(monkeypatch)
     slow, cs = _generate(layer, kind, x, T0, sizes)
     for a, b in zip(fast + list(cf.conv_state), slow + list(cs.conv_state)):
@@ -507,12 +525,16 @@ def _train(layer, x0, do):
 @pytest.mark.parametrize("kind,geometry,B,T,more", [
     ('gdn', None, 1, 64, {}), ('gdn', '340M', 2, 2113, {}), ('gdn', '760M', 1, 200, dict(allow_neg_eigval=True, conv_bias=True)),
     ('gdn', None, 3, 130, dict(conv_size=3, conv_activation=None, compute_dnats_for_invalid_blocks_attn=True, compute_dnats_for_invalid_blocks_linear_att=True)),
-    ('mamba', None, 2, 257, {}), ('mamba', None, 2, 4100, dict(conv_bias=True, conv_size=2))])
+    ('mamba', None, 2, 257, {}), ('mamba', None, 2, 4100, dict(conv_bias=True, conv_size=2)),
+    ('gdn', None, 2, 200, dict(ops_for_incomplete_chunks='gated_delta_net')), ('mamba', None, 2, 300, dict(ops_for_incomplete_chunks='mamba'))])
 @pytest.mark.parametrize("side,keep", [(False, False), (True, True), (True, False), (None, None)])
 def test_native_layer_is_its_steps(kind, geometry, B, T, more, side, keep, monkeypatch):
-    """A training step through the native call against the same launches one by one: the streams' and the kept states' switches, sequences that cut a block."""
+    """A training step through the native call against the same launches one by one: the streams' and the kept states' switches, sequences that cut a block,
+    incomplete blocks for both operators and for the linear one alone."""
     from neuralattentionsearchlinear_amd import _front, _mixed_common
-    layer = _layer(kind, geometry, 'all', **more).train()
+    more = dict(more)
+    ops = more.pop('ops_for_incomplete_chunks', 'all')
+    layer = _layer(kind, geometry, ops, **more).train()
     torch.manual_seed(T)
     x, do = (torch.randn(B, T, layer.hidden_size, device=DEV).bfloat16() for _ in range(2))
     calls, inner = [], _front._Layer.forward
@@ -521,7 +543,7 @@ def test_native_layer_is_its_steps(kind, geometry, B, T, more, side, keep, monke
     monkeypatch.setattr(_mixed_common, 'SAVE_CHUNK_STATES', keep)
     got = [_train(layer, x, do) for _ in range(2)]
     assert calls == [1, 1]
-    other = _layer(kind, geometry, 'all', **more).train()
+    other = _layer(kind, geometry, ops, **more).train()
     other.load_state_dict(layer.state_dict())
     _stepwise(monkeypatch)
     want = _train(other, x, do)
@@ -563,9 +585,12 @@ def test_native_layer_takes_the_steps_products(kind, geometry, B, T, monkeypatch
 
 
 @pytest.mark.parametrize("kind", ['gdn', 'mamba'])
-def test_native_layer_under_autograd(kind):
+def test_native_layer_under_autograd(kind, monkeypatch):
     """What autograd asks of the one node: gradients for what wants them only, saved tensors through hooks, a second backward, changed weights
     refused, no graph where nothing wants a gradient."""
+    from neuralattentionsearchlinear_amd import _front
+    calls, inner = [], _front._Layer.forward
+    monkeypatch.setattr(_front._Layer, 'forward', staticmethod(lambda *a: (calls.append(1), inner(*a))[1]))
     layer = _layer(kind, None, 'all').train()
     torch.manual_seed(5)
     x, do = (torch.randn(2, 150, layer.hidden_size, device=DEV).bfloat16() for _ in range(2))
@@ -575,6 +600,7 @@ def test_native_layer_under_autograd(kind):
         got = _train(layer, x, do)
     for n, b in want.items():
         assert rel_l2(got[n].float(), b.float()) <= (2e-2 if n == 'nats_layer.weight' else 1e-6), n
+    assert len(calls) == 2
     layer.zero_grad(set_to_none=True)
     some = {'wo': layer.o_proj.weight, 'wa': layer.a_proj.weight, 'mix': layer.nats_out_weights_layer.weight}
     for p in layer.parameters():
@@ -592,6 +618,7 @@ def test_native_layer_under_autograd(kind):
         layer.a_proj.weight.mul_(1.0)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         o.backward(do)
+    assert len(calls) == 4
     for p in layer.parameters():
         p.requires_grad_(False)
     assert not out(x).requires_grad
@@ -720,9 +747,14 @@ def test_native_layer_needs_no_more_memory_than_its_steps(kind, geometry, heads,
 
 
 @pytest.mark.parametrize("kind,T0", [('gdn', 128), ('gdn', 777), ('mamba', 64), ('mamba', 2113)])
-@pytest.mark.parametrize("ops", ['all', 'attn'])
+@pytest.mark.parametrize("ops", ['all', 'attn', 'linear'])
 def test_native_prompt_is_its_steps(kind, T0, ops, monkeypatch):
     """A first prompt through the native calls against the same launches one by one: outputs, what the cache holds, and the tokens behind it."""
+    from neuralattentionsearchlinear_amd import _front
+    if ops == 'linear':
+        ops = 'gated_delta_net' if kind == 'gdn' else 'mamba'
+    calls, inner = [], _front.FastFront.prompt
+    monkeypatch.setattr(_front.FastFront, 'prompt', lambda *a: (calls.append(1), inner(*a))[1])
     layer = _layer(kind, None, ops)
     torch.manual_seed(T0)
     x = torch.randn(2, T0 + 3, layer.hidden_size, device=DEV).bfloat16()
@@ -730,7 +762,9 @@ def test_native_prompt_is_its_steps(kind, T0, ops, monkeypatch):
     other = _layer(kind, None, ops)
     other.load_state_dict(layer.state_dict())
     _stepwise(monkeypatch)
+    assert calls == [1]
     slow, cs = _generate(other, kind, x, T0, (1, 2))
+    assert calls == [1]
     names = ['attn_k', 'attn_v', 'l_attn_k', 'l_attn_v', 'lattn_g', 'lattn_beta', 'recurrent_state', 'recurrent_state_block_start', 'g_cumsum', 'block_type_state']
     for a, b in zip(fast + list(cf.conv_state) + [getattr(cf, n) for n in names], slow + list(cs.conv_state) + [getattr(cs, n) for n in names]):
         assert (a is None) == (b is None) and (a is None or a.shape == b.shape and rel_l2(a.float(), b.float()) <= 2e-3)

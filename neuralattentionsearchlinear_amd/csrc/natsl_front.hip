@@ -552,8 +552,9 @@ static int conv_cus() {
 }
 
 // Tokens per thread: long runs read the fewest rows twice (and leave the fewest partial sums), but what counts first is that the
-// workgroups fill whole rounds of the chip -- registers admit three of them on a CU forward, two backward
-// (340M geometry, 8 x 4096: backward with runs of 64 in 1.5 rounds 233 us, of 98 in one 208; forward 32 -> 64 tokens 100 -> 94).
+// workgroups fill whole rounds of the chip -- registers admit three of them on a CU forward (150) and backward with four channels a thread
+// (165), two with eight (247).  340M geometry, 8 x 4096: forward 32 -> 64 tokens 100 -> 94 us; backward, with eight channels, runs of 64 in 1.5
+// rounds 233 us, of 98 in one 208.
 static int conv_run(int B, int T, int W, int groups, bool bwd, int ch) {
   const long long slots = (long long)conv_cus() * (bwd && ch == 8 ? 2 : 3);
   int best = 8;

@@ -622,8 +622,9 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
       // among them, when everybody is done with chunk 0, is where chunks 1 to 3 must have landed, and slot 0 is free from there on: the loop's
       // K(0) has a fifth slot (K's ring starts there), its K(1) and V(0) take slot 0.  The same chunks in the same order: the same bits.
       // us, all in the loop / so, alone on the device: no attention blocks, 128/128, B4 T4096 H16 66 / 56, B32 T320 H16 56 / 43; half attention,
-      // B2 T3000 H18 64/128 81 / 76, B8 T2000 H16 128/64 120 / 118; one tile per CU, half attention, B2 T2048 H16 128/128 37.5 / 38.1.  Blocks of
-      // more than a chunk stay in the loop: their chunks from dstart on can be more than the slots.
+      // B2 T3000 H18 64/128 81 / 76, B8 T2000 H16 128/64 120 / 118; one tile per CU, half attention, B2 T2048 H16 128/128 37.5 / 38.1.  Measured
+      // and chosen for blocks of one chunk.  (Blocks of 128 and 256 have no more own chunks, as tiles start on multiples of 256 in their sequence; of
+      // other blocks the chunks from dstart on can be more than the slots.)
       constexpr int OWN_EARLY = 2, RING = 4, KTILE = 64 * DK * 2, VTILE = 64 * DV * 2;   // bytes
       constexpr int KI = DK / 32, VI = DV / 32;                           // DMA instructions per wave and chunk: early waves K, late waves V
       constexpr int KROWS_I = 512 / DK, VROWS_I = 512 / DV;               // tile rows one instruction covers

@@ -7,7 +7,7 @@ from __future__ import annotations
 
 import ctypes
 import os
-from ctypes import c_char_p, c_float, c_int, c_int64, c_longlong, c_size_t, c_void_p
+from ctypes import c_char_p, c_float, c_int, c_int64, c_longlong, c_size_t, c_uint64, c_void_p
 
 import torch
 
@@ -118,6 +118,8 @@ _SIGNATURES = {
     "natsl_mixed_fwd": (c_int, [c_void_p, c_int, c_void_p, c_void_p]),
     "natsl_layer_step_workspace_bytes": (c_size_t, [c_void_p]),
     "natsl_layer_step_fwd": (c_int, [c_void_p, c_void_p, c_size_t, c_void_p]),
+    "natsl_layer_step_sync_bytes": (c_size_t, [c_void_p]),
+    "natsl_layer_step_sync_fwd": (c_int, [c_void_p, c_void_p, c_size_t, c_void_p, c_size_t, c_uint64, c_void_p]),
     "natsl_kv_compact": (c_int, [c_void_p, c_void_p, c_longlong, c_int, c_void_p, c_void_p, c_longlong, c_void_p, c_int, c_void_p,
                                  c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
 }

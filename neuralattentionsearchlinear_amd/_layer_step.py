@@ -21,6 +21,7 @@ from . import _capi
 from .modules import FusedMultiInputRMSNormGated, L2Norm, RMSNorm, ShortConvolution
 
 MAX_ROWS = 64
+MAX_WAIT_US = 10_000_000                                 # what a part of a step's launch waits for another before it gives up
 
 _INTS = ("B", "T", "D", "H", "K", "V", "HQ", "HN", "block", "conv_width", "is_delta", "flags", "n_in", "n_kept", "cache_tokens", "types_dtype",
          "norm_dtype", "gate_dtype", "out_norm_dtype", "reserved")
@@ -183,8 +184,9 @@ class _Plan:
         self.device = params[0].device
         L = _capi.lib()
         address = lambda f: ctypes.cast(f, ctypes.c_void_p).value
-        self.core = _capi.step_core().make_step(ctypes.addressof(s), ctypes.sizeof(s), address(L.natsl_layer_step_fwd),
-                                                address(L.natsl_layer_step_workspace_bytes), self.device.index)
+        self.core = _capi.step_core().make_step(ctypes.addressof(s), ctypes.sizeof(s), address(L.natsl_layer_step_sync_fwd),
+                                                address(L.natsl_layer_step_workspace_bytes), address(L.natsl_layer_step_sync_bytes), MAX_WAIT_US,
+                                                self.device.index)
         self.built = True
 
 
@@ -223,12 +225,12 @@ def layer_step(layer, kind, x, cache):
         if full:
             cache._grow(cache.n_attn_tokens_max + T)
     done = core.run(plan.core, x, n_in, cache.n_attn_blocks_max, _capi.stream_ptr(x.device), types,
-                    0 if types is None else _capi.dtype_code(types.dtype), *tensors())
+                    0 if types is None else _capi.dtype_code(types.dtype), *tensors(), getattr(cache, 'step_shared', None))
     if type(done) is not tuple:
         if done is None:                                   # (the cache's tensors are not what the kernels address)
             return None
-        _capi.check(done, "natsl_layer_step_fwd")
-    out, state_out, start, new_conv, g_out = done
+        _capi.check(done, "natsl_layer_step_sync_fwd")
+    out, state_out, start, new_conv, g_out, cache.step_shared = done
     if types is None:
         cache.note_step(state_out, start, new_conv, g_out, T)
     else:

@@ -111,6 +111,7 @@ class NAtSLayerCache:
         self.n_observed_tokens = 0
         self._pending_first = None                       # K/V of the first forward, kept until update() has the types
         self._foreseen = None                            # counts on their way to the host (foresee)
+        self.step_shared = None                        # what the parts of a generation step in one launch meet on
 
     def is_empty(self) -> bool:
         """Whether nothing of a forward has been kept (but the hidden states of the one that runs)."""

@@ -8,6 +8,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
 #include <ATen/ops/empty.h>
+#include <ATen/ops/zeros.h>
 
 #include <vector>
 
@@ -208,18 +209,20 @@ PyObject* holds(PyObject*, PyObject* const* args, Py_ssize_t n) {
 // ---- the step ----------------------------------------------------------------------------------------------------------
 struct Step {
   natsl_layer_step fixed;
-  decltype(&natsl_layer_step_fwd) fwd;
+  decltype(&natsl_layer_step_sync_fwd) fwd;
+  decltype(&natsl_layer_step_sync_bytes) sync_bytes;
+  unsigned long long max_wait_us;
   decltype(&natsl_layer_step_workspace_bytes) workspace_bytes;
   int device;
 };
 
 void free_step(PyObject* capsule) { delete static_cast<Step*>(PyCapsule_GetPointer(capsule, STEP)); }
 
-// make_step(address of the structure with everything that stays the same, its size, addresses of the two entry points, device index)
+// make_step(address of the structure with everything that stays the same, its size, addresses of the three entry points, the longest wait, device index)
 PyObject* make_step(PyObject*, PyObject* args) {
-  unsigned long long fixed, size, fwd, bytes;
+  unsigned long long fixed, size, fwd, bytes, sync_bytes, max_wait_us;
   int device;
-  if (!PyArg_ParseTuple(args, "KKKKi", &fixed, &size, &fwd, &bytes, &device)) return nullptr;
+  if (!PyArg_ParseTuple(args, "KKKKKKi", &fixed, &size, &fwd, &bytes, &sync_bytes, &max_wait_us, &device)) return nullptr;
   if (size != sizeof(natsl_layer_step)) {
     PyErr_SetString(PyExc_ValueError, "the step's structure has another size than the library's");
     return nullptr;
@@ -228,6 +231,8 @@ PyObject* make_step(PyObject*, PyObject* args) {
   s->fixed = *reinterpret_cast<const natsl_layer_step*>(fixed);
   s->fwd = reinterpret_cast<decltype(s->fwd)>(fwd);
   s->workspace_bytes = reinterpret_cast<decltype(s->workspace_bytes)>(bytes);
+  s->sync_bytes = reinterpret_cast<decltype(s->sync_bytes)>(sync_bytes);
+  s->max_wait_us = max_wait_us;
   s->device = device;
   PyObject* capsule = PyCapsule_New(s, STEP, free_step);
   if (!capsule) delete s;
@@ -295,12 +300,12 @@ PyObject* takes(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// run(step, x, n_in, n_kept, stream, types or None, their code, the cache's tensors ...)
-// -> None: the cache's tensors do not fit; a number: the entry point's error; else (out, state, block start, conv states, g sum)
+// run(step, x, n_in, n_kept, stream, types or None, their code, the cache's tensors ..., what its steps in one launch share or None)
+// -> None: the cache's tensors do not fit; a number: the entry point's error; else (out, state, block start, conv states, g sum, what they share)
 PyObject* run(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 7 + CACHE_ARGS || !THPVariable_Check(args[1])) {
-    PyErr_SetString(PyExc_TypeError, "run(step, x, n_in, n_kept, stream, types, types' code, the cache's tensors ...)");
+  if (n != 8 + CACHE_ARGS || !THPVariable_Check(args[1])) {
+    PyErr_SetString(PyExc_TypeError, "run(step, x, n_in, n_kept, stream, types, types' code, the cache's tensors ..., shared)");
     return nullptr;
   }
   auto* step = static_cast<Step*>(PyCapsule_GetPointer(args[0], STEP));
@@ -361,9 +366,17 @@ PyObject* run(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const size_t bytes = step->workspace_bytes(&s);
   at::Tensor ws = at::empty({(int64_t)bytes}, f32.dtype(at::kByte));
   void* const ws_ptr = ws.data_ptr();
+  // What the parts of a step in one launch meet on belongs to the cache, whose steps follow one another; it holds something from step to step and
+  // is made anew for another number of sequences.
+  const size_t shared_bytes = step->sync_bytes(&s);
+  at::Tensor shared;
+  if (args[7 + CACHE_ARGS] != Py_None && THPVariable_Check(args[7 + CACHE_ARGS])) shared = THPVariable_Unpack(args[7 + CACHE_ARGS]);
+  if (shared_bytes && (!shared.defined() || shared.nbytes() != shared_bytes || shared.get_device() != step->device || !shared.is_contiguous()))
+    shared = at::zeros({(int64_t)(shared_bytes / 4)}, f32.dtype(at::kInt));
+  void* const shared_ptr = shared_bytes ? shared.data_ptr() : nullptr;
   int rc;
   Py_BEGIN_ALLOW_THREADS
-  rc = step->fwd(&s, ws_ptr, bytes, stream);
+  rc = step->fwd(&s, ws_ptr, bytes, shared_ptr, shared_bytes, step->max_wait_us, stream);
   Py_END_ALLOW_THREADS
   if (rc) return PyLong_FromLong(rc);
   THPObjectPtr conv(PyTuple_New(3));
@@ -373,9 +386,9 @@ PyObject* run(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (!t) return nullptr;
     PyTuple_SET_ITEM(conv.get(), i, t);
   }
-  THPObjectPtr o(THPVariable_Wrap(out)), so(THPVariable_Wrap(state_out)), st(THPVariable_Wrap(c.start)), g(THPVariable_Wrap(g_out));
-  if (!o || !so || !st || !g) return nullptr;
-  return PyTuple_Pack(5, o.get(), so.get(), st.get(), conv.get(), g.get());
+  THPObjectPtr o(THPVariable_Wrap(out)), so(THPVariable_Wrap(state_out)), st(THPVariable_Wrap(c.start)), g(THPVariable_Wrap(g_out)), kept(shared.defined() ? THPVariable_Wrap(shared) : Py_NewRef(Py_None));
+  if (!o || !so || !st || !g || !kept) return nullptr;
+  return PyTuple_Pack(6, o.get(), so.get(), st.get(), conv.get(), g.get(), kept.get());
   END_HANDLE_TH_ERRORS
 }
 

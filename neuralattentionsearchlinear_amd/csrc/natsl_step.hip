@@ -1,9 +1,10 @@
 // A generation step of a whole hybrid layer: a few new tokens of each cached sequence, from the hidden states to the layer's
-// output, in three launches for one token a sequence and five for several.  At this size a step is bound by launches and by the
+// output, in one launch for one token of few sequences, three for one token a sequence and five for several.  At this size a step is bound by launches and by the
 // host that issues them (the same step as separate operations was 40 launches, 0.2 ms of kernels and 0.57 ms of host time for one
 // 340M-geometry layer), so each kernel takes as much of the step as its data dependences allow:
 //   rows_gemm_kernel     q, k, v, gate, a (and beta) projections as one pass over all their weights; the output projection
 //   step_one_kernel      one token a sequence: all that the other three do
+//   step_all_kernel      ... and both products
 //   step_mix_kernel      short convolutions, activations, row norms, gates; the new rows of every cache, written in place
 //   attend_and_recur     attention over the cached keys next to the token recurrence (natsl_decode.hip)
 //   step_tail_kernel     join of the attention's splits, mixing weights, two-input norm and gate
@@ -139,16 +140,25 @@ struct AnyRaw {             // an element of either type
   }
   NATSL_DEVICE float get(const int dtype) const { return __uint_as_float((unsigned)hi << 16 | (dtype == NATSL_F32 ? (unsigned)lo : 0u)); }
 };
+// A number that crosses from one workgroup to another inside a launch (StepAll): a bf16 and, in the word's lower half, the launch's tag, so that
+// it is its own flag.  Written through and read past the reader's L2.
+NATSL_DEVICE unsigned tagged(const bf16_t x, const unsigned tag) { return (unsigned)x << 16 | tag; }
+NATSL_DEVICE unsigned ld_word(const unsigned* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 struct StepWindow {         // a convolution of width 4 at one channel, every pointer on 8 bytes; x: the new input
   u32x2 e, w;
   bf16_t b, x;
   // (channel d of sequence row `seq`, the same in every lane: offsets of 32 bits a lane on scalar bases)
-  NATSL_DEVICE void load(const bf16_t* proj, const void* state, const void* weight, const void* bias, const unsigned d, const size_t seq) {
+  // fixed(): what was there before the launch; input(): from the projections, word(): from those of this launch, `late` where it is not there yet.
+  NATSL_DEVICE void fixed(const void* state, const void* weight, const void* bias, const unsigned d, const size_t seq) {
     auto at = [](const void* p, const unsigned bytes) __attribute__((always_inline)) -> const char* { return reinterpret_cast<const char*>(p) + bytes; };
-    x = *reinterpret_cast<const bf16_t*>(at(proj, 2u * d));
     e = *reinterpret_cast<const u32x2*>(at(reinterpret_cast<const u32x2*>(state) + seq, 8u * d));
     w = *reinterpret_cast<const u32x2*>(at(weight, 8u * d));
     b = *reinterpret_cast<const bf16_t*>(at(bias ? bias : weight, 2u * d));
+  }
+  NATSL_DEVICE void input(const bf16_t* proj, const unsigned d) { x = proj[d]; }
+  NATSL_DEVICE void word(const unsigned w, const unsigned tag, unsigned& late) {
+    x = (bf16_t)(w >> 16);
+    late |= (w & 0xffffu) ^ tag;
   }
   NATSL_DEVICE float next(const bool bias, const bool silu) const {
     float a = bias ? bf16_to_f32(b) : 0.f;
@@ -279,20 +289,22 @@ struct TailRow {
   static constexpr int CPL = VA / 64;
   bf16_t gate[CPL];
   AnyRaw w1[CPL], w2[CPL];
-  NATSL_DEVICE void load(const StepTail& p, const int row, const int hq) {
+  NATSL_DEVICE void load(const StepTail& p, const int row, const int hq, const bool gates = true) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int j = 0; j < CPL; ++j) {
-      gate[j] = p.proj[(size_t)row * p.ldp + p.cg + hq * VA + CPL * lane + j];
+      if (gates) gate[j] = p.proj[(size_t)row * p.ldp + p.cg + hq * VA + CPL * lane + j];
       w1[j].load(p.w1, p.w_dtype, CPL * lane + j);
       w2[j].load(p.w2, p.w_dtype, CPL * lane + j);
     }
   }
-  NATSL_DEVICE void finish(const StepTail& p, const int row, const int hq, float d0, float d1, const float* at, const float* x1) const;
+  NATSL_DEVICE void finish(const StepTail& p, const int row, const int hq, float d0, float d1, const float* at, const float* x1, unsigned* words = nullptr,
+                           unsigned tag = 0) const;
 };
 
 template <int VA>
-NATSL_DEVICE void TailRow<VA>::finish(const StepTail& p, const int row, const int hq, float d0, float d1, const float* at, const float* x1) const {
+NATSL_DEVICE void TailRow<VA>::finish(const StepTail& p, const int row, const int hq, float d0, float d1, const float* at, const float* x1, unsigned* words,
+                               const unsigned tag) const {
   const int lane = threadIdx.x & 63;
   float x2[CPL], sa = 0.f, sb = 0.f;
 #pragma unroll
@@ -311,7 +323,9 @@ NATSL_DEVICE void TailRow<VA>::finish(const StepTail& p, const int row, const in
 #pragma unroll
   for (int j = 0; j < CPL; ++j) {
     const float mix = x1[j] * ra * w1[j].get(p.w_dtype) + x2[j] * rb * w2[j].get(p.w_dtype), g = bf16_to_f32(gate[j]);
-    p.y[base + j] = f32_to_bf16(mix * g / (1.f + __expf(-g)));
+    const bf16_t y = f32_to_bf16(mix * g / (1.f + __expf(-g)));
+    if (words) __hip_atomic_store(words + base + j, tagged(y, tag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else p.y[base + j] = y;
   }
 }
 
@@ -366,6 +380,9 @@ struct StepOne {
   float *o_lin, *logits;      // [B][H*V] rounded to bf16; [B][n_chunks][HQ][2]
   unsigned* arrived;          // [B][HQ]
   int n_chunks, n_logits, n_rec;
+  // with HERE (StepAll): what the launch's parts meet on (StepSync), the projections and the tail's rows as tagged words, like proj and y
+  unsigned *sync, *proj_words, *y_words;
+  unsigned long long max_wait;
 };
 constexpr int LOGIT_CHUNK = 256;
 
@@ -383,23 +400,63 @@ NATSL_DEVICE unsigned long long arrive(const StepOne& p, const int b, const int 
   return last;
 }
 
-template <int VA>
+// What the parts of a launch with the products in it (HERE) meet on, in lines of their own.  Zeros at first; a launch leaves the epoch, which its
+// words' tags come from, one higher, and everything else as it was, but FAILED when it did.
+struct StepSync {
+  static constexpr int LINE = 32, LEFT = 0, FAILED = LINE, EPOCH = 2 * LINE, ARRIVED = 3 * LINE;
+};
+NATSL_DEVICE unsigned step_tag(const StepOne& p) { return (ld_word(p.sync + StepSync::EPOCH) + 1u) & 0xffffu; }
+
+// Until ask(), which requests words, finds that none of any lane's is late, or the time is over: then the step has failed, its outputs become
+// NaN, and every wave still ends.  Waves that wait are fewer than the chip holds (step_may_wait), and the workgroups that they wait for
+// come first in the grid and wait for nothing or for others before them, so those always run.
+template <class Ask>
+NATSL_DEVICE void wait_for(const StepOne& p, Ask ask) {
+  if (!__ballot(ask() != 0u)) return;
+  const unsigned long long since = __builtin_amdgcn_s_memrealtime();
+  for (unsigned n = 1;; ++n) {
+    __builtin_amdgcn_s_sleep(2);
+    if (!__ballot(ask() != 0u)) return;
+    if (n % 64u == 0u && ld_word(p.sync + StepSync::FAILED)) return;
+    if (__builtin_amdgcn_s_memrealtime() - since > p.max_wait) {
+      if ((threadIdx.x & 63) == 0) __hip_atomic_store(p.sync + StepSync::FAILED, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return;
+    }
+  }
+}
+
+template <int VA, bool HERE>
 NATSL_DEVICE void step_tail(const StepOne& p, const int b, const int hq) {
   constexpr int CPL = VA / 64;
   const int lane = threadIdx.x & 63;
   const size_t rh = (size_t)b * p.a.HQ + hq;
   TailRow<VA> out;
-  out.load(p.t, b, hq);
+  out.load(p.t, b, hq, !HERE);
+  unsigned tag = 0;
+  if constexpr (HERE) tag = step_tag(p);
   float at[CPL], x1[CPL];
 #pragma unroll
   for (int j = 0; j < CPL; ++j) x1[j] = ld_agent(p.o_lin + rh * VA + CPL * lane + j);
   const float* lg = p.logits + (((size_t)b * p.n_chunks + min(lane, p.n_chunks - 1)) * p.a.HQ + hq) * 2;
   const float d0 = ld_agent(lg), d1 = ld_agent(lg + 1);
   join_splits<VA, true>(p.a.partials + rh * p.a.nsplit * (2 + VA), p.a.nsplit, at);
-  out.finish(p.t, b, hq, lane < p.n_chunks ? d0 : 0.f, lane < p.n_chunks ? d1 : 0.f, at, x1);
+  if constexpr (HERE) {
+    const unsigned* gates = p.proj_words + (size_t)b * p.t.ldp + p.t.cg + hq * VA + CPL * lane;
+    wait_for(p, [&]() __attribute__((always_inline)) {
+      unsigned late = 0;
+#pragma unroll
+      for (int j = 0; j < CPL; ++j) {
+        const unsigned w = ld_word(gates + j);
+        out.gate[j] = (bf16_t)(w >> 16);
+        late |= (w & 0xffffu) ^ tag;
+      }
+      return late;
+    });
+  }
+  out.finish(p.t, b, hq, lane < p.n_chunks ? d0 : 0.f, lane < p.n_chunks ? d1 : 0.f, at, x1, HERE ? p.y_words : nullptr, tag);
 }
 
-template <int VA>
+template <int VA, bool HERE>
 NATSL_DEVICE void step_logits(const StepOne& p, const int b, const int chunk, const int expected) {
   __shared__ __align__(16) bf16_t qs[LOGIT_CHUNK];
   const natsl_layer_step& s = p.m.s;
@@ -415,8 +472,19 @@ NATSL_DEVICE void step_logits(const StepOne& p, const int b, const int chunk, co
   };
   const size_t sd = (size_t)b * KD;
   StepWindow win;
-  win.load(p.m.proj + (size_t)b * p.m.ldp + p.m.cq, s.conv_state_q, s.conv_wq, s.conv_bq, min(d, KD - 1), sd);
+  win.fixed(s.conv_state_q, s.conv_wq, s.conv_bq, min(d, KD - 1), sd);
   load(wave);
+  if constexpr (HERE) {
+    const unsigned tag = step_tag(p);
+    const unsigned* w = p.proj_words + (size_t)b * p.m.ldp + p.m.cq + min(d, KD - 1);
+    wait_for(p, [&]() __attribute__((always_inline)) {
+      unsigned late = 0;
+      win.word(ld_word(w), tag, late);
+      return late;
+    });
+  } else {
+    win.input(p.m.proj + (size_t)b * p.m.ldp + p.m.cq, min(d, KD - 1));
+  }
   const bf16_t y = f32_to_bf16(win.next(s.conv_bq != nullptr, s.flags & NATSL_STEP_SILU));
   if (d < KD) win.save(s.conv_out_q, sd + d);
   qs[tid] = d < KD ? y : (bf16_t)0;
@@ -445,12 +513,12 @@ NATSL_DEVICE void step_logits(const StepOne& p, const int b, const int chunk, co
   }
   for (int h0 = wave; h0 < s.HQ; h0 += 256) {           // lane i counts in for the wave's i-th head
     const int h = h0 + 4 * lane;
-    for (unsigned long long last = arrive(p, b, h, h < s.HQ, expected); last; last &= last - 1) step_tail<VA>(p, b, h0 + 4 * __builtin_ctzll(last));
+    for (unsigned long long last = arrive(p, b, h, h < s.HQ, expected); last; last &= last - 1) step_tail<VA, HERE>(p, b, h0 + 4 * __builtin_ctzll(last));
   }
 }
 
 // The recurrence's token: q and k of the head go through the wave's own piece of LDS, the rest stays in registers.
-template <int DK>
+template <int DK, bool HERE>
 struct StepToken {
   const StepOne& p;
   bf16_t* rows;               // [2][DK], this wave's
@@ -471,15 +539,48 @@ struct StepToken {
 #pragma unroll
     for (int i = 0; i < C; ++i) {
       const int d = h * DK + 64 * i + lane;
-      wq[i].load(proj + p.m.cq, s.conv_state_q, s.conv_wq, s.conv_bq, d, (size_t)n * KD);
-      wk[i].load(proj + p.m.ck, s.conv_state_k, s.conv_wk, s.conv_bk, d, (size_t)n * KD);
+      wq[i].fixed(s.conv_state_q, s.conv_wq, s.conv_bq, d, (size_t)n * KD);
+      wk[i].fixed(s.conv_state_k, s.conv_wk, s.conv_bk, d, (size_t)n * KD);
     }
     const int dv = h * s.V + vc;
-    wv.load(proj + p.m.cv, s.conv_state_v, s.conv_wv, s.conv_bv, dv, (size_t)n * VD);
+    wv.fixed(s.conv_state_v, s.conv_wv, s.conv_bv, dv, (size_t)n * VD);
     AnyRaw a_log, dt_bias;
     a_log.load(s.a_log, s.gate_dtype, h);
     dt_bias.load(s.dt_bias, s.gate_dtype, h);
-    const bf16_t xa = proj[p.m.ca + h], xb = DELTA ? proj[p.m.cb + h] : (bf16_t)0;
+    bf16_t xa, xb = 0;
+    if constexpr (HERE) {
+      const unsigned tag = step_tag(p);
+      const unsigned* w = p.proj_words + (size_t)n * p.m.ldp;
+      wait_for(p, [&]() __attribute__((always_inline)) {
+        unsigned late = 0, words[2 * C + 3];
+#pragma unroll
+        for (int i = 0; i < C; ++i) {
+          words[2 * i] = ld_word(w + p.m.cq + h * DK + 64 * i + lane);
+          words[2 * i + 1] = ld_word(w + p.m.ck + h * DK + 64 * i + lane);
+        }
+        words[2 * C] = ld_word(w + p.m.cv + dv);
+        words[2 * C + 1] = ld_word(w + p.m.ca + h);
+        words[2 * C + 2] = ld_word(w + (DELTA ? p.m.cb : p.m.ca) + h);
+#pragma unroll
+        for (int i = 0; i < C; ++i) {
+          wq[i].word(words[2 * i], tag, late);
+          wk[i].word(words[2 * i + 1], tag, late);
+        }
+        wv.word(words[2 * C], tag, late);
+        xa = (bf16_t)(words[2 * C + 1] >> 16);
+        if (DELTA) xb = (bf16_t)(words[2 * C + 2] >> 16);
+        return late | ((words[2 * C + 1] & 0xffffu) ^ tag) | ((words[2 * C + 2] & 0xffffu) ^ tag);
+      });
+    } else {
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        wq[i].input(proj + p.m.cq, h * DK + 64 * i + lane);
+        wk[i].input(proj + p.m.ck, h * DK + 64 * i + lane);
+      }
+      wv.input(proj + p.m.cv, dv);
+      xa = proj[p.m.ca + h];
+      if (DELTA) xb = proj[p.m.cb + h];
+    }
     const float A = expf(a_log.get(s.gate_dtype));
     const float dt = softplus_gate(bf16_to_f32(xa) + dt_bias.get(s.gate_dtype));
     gt = -A * dt;
@@ -541,15 +642,27 @@ struct StepRow {
   static constexpr int C = N / 64;
   StepWindow win[C];
   AnyRaw nw[C];
-  NATSL_DEVICE void request(const natsl_layer_step& s, const bf16_t* proj, const void* state, const void* weight, const void* bias, const void* norm,
-                            const size_t seq, const int d0) {
+  NATSL_DEVICE void request(const natsl_layer_step& s, const void* state, const void* weight, const void* bias, const void* norm, const size_t seq,
+                            const int d0) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int i = 0; i < C; ++i) {
-      const int d = d0 + 64 * i + lane;
-      win[i].load(proj, state, weight, bias, d, seq);
+      win[i].fixed(state, weight, bias, d0 + 64 * i + lane, seq);
       nw[i].load(norm ? norm : weight, s.norm_dtype, 64 * i + lane);
     }
+  }
+  NATSL_DEVICE void input(const bf16_t* proj, const int d0) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < C; ++i) win[i].input(proj, d0 + 64 * i + lane);
+  }
+  NATSL_DEVICE void words(const unsigned* proj, const int d0, const unsigned tag, unsigned& late) {
+    const int lane = threadIdx.x & 63;
+    unsigned w[C];
+#pragma unroll
+    for (int i = 0; i < C; ++i) w[i] = ld_word(proj + d0 + 64 * i + lane);
+#pragma unroll
+    for (int i = 0; i < C; ++i) win[i].word(w[i], tag, late);
   }
   NATSL_DEVICE void form(const natsl_layer_step& s, const bool bias, const bool norm, bf16_t* dst, bf16_t* also) const {
     const int lane = threadIdx.x & 63;
@@ -580,7 +693,7 @@ struct StepRow {
 
 // What an attending wave of the step makes itself: its query, and in the wave with the last chunk (`mine`) the new key and value.  All
 // inputs are requested (request()) before the first chunk is, and used when that is on its way.
-template <int KA, int VA>
+template <int KA, int VA, bool HERE>
 struct StepKeys {
   static constexpr bool STEP = true;
   const StepOne& p;
@@ -595,17 +708,37 @@ struct StepKeys {
   NATSL_DEVICE void request() {
     const natsl_layer_step& s = p.m.s;
     const size_t KD = (size_t)s.H * s.K, VD = (size_t)s.H * s.V;
-    const bf16_t* proj = p.m.proj + (size_t)b * p.m.ldp;
     const bool norm = s.flags & NATSL_STEP_ATTN_NORM;
-    rq.request(s, proj + p.m.cq, s.conv_state_q, s.conv_wq, s.conv_bq, norm ? s.norm_q : nullptr, b * KD, hq * KA);
+    rq.request(s, s.conv_state_q, s.conv_wq, s.conv_bq, norm ? s.norm_q : nullptr, b * KD, hq * KA);
     if (mine) {
-      rk.request(s, proj + p.m.ck, s.conv_state_k, s.conv_wk, s.conv_bk, norm ? s.norm_k : nullptr, b * KD, hq * KA);
-      rv.request(s, proj + p.m.cv, s.conv_state_v, s.conv_wv, s.conv_bv, nullptr, b * VD, hq * VA);
+      rk.request(s, s.conv_state_k, s.conv_wk, s.conv_bk, norm ? s.norm_k : nullptr, b * KD, hq * KA);
+      rv.request(s, s.conv_state_v, s.conv_wv, s.conv_bv, nullptr, b * VD, hq * VA);
+    }
+    if constexpr (!HERE) {
+      const bf16_t* proj = p.m.proj + (size_t)b * p.m.ldp;
+      rq.input(proj + p.m.cq, hq * KA);
+      if (mine) {
+        rk.input(proj + p.m.ck, hq * KA);
+        rv.input(proj + p.m.cv, hq * VA);
+      }
     }
   }
   NATSL_DEVICE void ready(AttnRow<KA, VA, false>& row) {
     if (done) return;
     done = true;
+    if constexpr (HERE) {        // (the first chunk's keys are on their way by now)
+      const unsigned tag = step_tag(p);
+      const unsigned* w = p.proj_words + (size_t)b * p.m.ldp;
+      wait_for(p, [&]() __attribute__((always_inline)) {
+        unsigned late = 0;
+        rq.words(w + p.m.cq, hq * KA, tag, late);
+        if (mine) {
+          rk.words(w + p.m.ck, hq * KA, tag, late);
+          rv.words(w + p.m.cv, hq * VA, tag, late);
+        }
+        return late;
+      });
+    }
     const natsl_layer_step& s = p.m.s;
     const bool norm = s.flags & NATSL_STEP_ATTN_NORM;
     rq.form(s, s.conv_bq != nullptr, norm, q, nullptr);
@@ -628,23 +761,23 @@ NATSL_DEVICE const StepOne& step_one_args() {
   return *(const StepOne*)(arg_ptr)at;
 }
 
-template <int KA, int VA, int K, bool DELTA>
-__global__ __launch_bounds__(256) void step_one_kernel(const StepOne) {
-  const StepOne& p = step_one_args();
+// The roles of the workgroups between the products; id: which of them
+template <int KA, int VA, int K, bool DELTA, bool HERE>
+NATSL_DEVICE void step_roles(const StepOne& p, int id) {
   __shared__ __align__(16) bf16_t rows[4][2 * K > KA ? 2 * K : KA], own_k[KA], own_v[VA];
   const natsl_layer_step& s = p.m.s;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int expected = p.a.nsplit + VA / 16 + p.n_chunks;
-  int id = blockIdx.x, b, hq;
+  int b, hq;
   if (id < p.n_logits) {
-    step_logits<VA>(p, id / p.n_chunks, id % p.n_chunks, expected);
+    step_logits<VA, HERE>(p, id / p.n_chunks, id % p.n_chunks, expected);
     return;
   }
   id -= p.n_logits;
   if (id < p.n_rec) {
     const int per = (s.V + 63) / 64, col16 = (id % per) * 4 + wave, nh = id / per;
     if (col16 * 16 >= s.V) return;
-    StepToken<K> token{p, rows[wave], col16 == 0, expected, VA};
+    StepToken<K, HERE> token{p, rows[wave], col16 == 0, expected, VA};
     recurrent_columns<K, DELTA>(p.r, nh, col16, token);
     if (!token.last) return;
     b = nh / s.H;
@@ -655,19 +788,161 @@ __global__ __launch_bounds__(256) void step_one_kernel(const StepOne) {
     hq = id / p.a.nsplit % s.HQ;
     b = id / p.a.nsplit / s.HQ;
     const bool mine = (p.a.TK - 1) / KEYS_PER_CHUNK % (4 * p.a.nsplit) == 4 * split + wave;
-    attend<KA, VA, false, 4>(p.a, b, 0, hq, split, StepKeys<KA, VA>(p, rows[wave], own_k, own_v, b, hq, mine));
+    attend<KA, VA, false, 4>(p.a, b, 0, hq, split, StepKeys<KA, VA, HERE>(p, rows[wave], own_k, own_v, b, hq, mine));
     if (wave != 0 || !arrive(p, b, hq, lane == 0, expected)) return;
   }
-  step_tail<VA>(p, b, hq);
+  step_tail<VA, HERE>(p, b, hq);
 }
 
-static int launch_step_one(const char* what, const StepOne& p, const int K, const int KA, const int VA, hipStream_t st) {
+template <int KA, int VA, int K, bool DELTA>
+__global__ __launch_bounds__(256) void step_one_kernel(const StepOne) {
+  step_roles<KA, VA, K, DELTA, false>(step_one_args(), blockIdx.x);
+}
+
+// ---- ... and the products in the same launch ----------------------------------------------------------------------------
+// One sequence's step is bound by the host, which takes 22 us for a token and its three launches (18 of kernels, each of which begins with a trip
+// to memory for its arguments and one for its first operands).  Here the workgroups of the projections come first, those between the products
+// ask for windows, states and keys before they wait for them, and those of the output projection hold their weights when the rows come.
+// What crosses is words that are their own flags: counters behind the stores cost two trips more at each crossing, and with a few hundred
+// waves looking at the same ones far more (340M geometry 20.5 us, 760M 30).  A token with its host work, one sequence of 777: 340M geometry 22.1 ->
+// 15.9 us, 760M 22.4 -> 17.3, 16 heads of 128/64 21.9 -> 15.5; four of 500 (340M) 27.4 -> 23.1.
+// The sums are those of rows_gemm_kernel, in its order: a wave is two of its eight (accumulators 0 and 1).
+struct StepAll {
+  StepOne one;
+  RowsGemm in, out;
+  int in_tiles, out_tiles;
+};
+constexpr int STEP_ROWS = 8192;       // numbers of the rows that a workgroup of the output projection keeps: 16 KiB
+
+NATSL_DEVICE const StepAll& step_all_args() {
+  typedef __attribute__((address_space(4))) const StepAll* arg_ptr;
+  unsigned long long at = (unsigned long long)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(at));
+  return *(const StepAll*)(arg_ptr)at;
+}
+
+// One tile of 16 weight rows; OUT: of the output projection, behind everything else, else of the projections in front.  U: steps of 32 that a
+// wave has on their way at once.
+template <bool OUT, int U>
+NATSL_DEVICE void step_product(const StepAll& all, const int tile) {
+  extern __shared__ __align__(16) bf16_t step_rows[];   // OUT: [M][D]
+  __shared__ f32x4 red[8][64];
+  const RowsGemm& p = OUT ? all.out : all.in;
+  const StepOne& one = all.one;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int si = 0;
+  if constexpr (!OUT) {
+#pragma unroll
+    for (int i = 1; i < GEMM_SEGS; ++i) si = i < p.n_seg && tile >= p.seg[i].tile0 ? i : si;
+  }
+  const GemmSeg sg = p.seg[si];
+  const int n0 = 16 * (tile - sg.tile0), r16 = lane & 15, kg = lane >> 4, steps = p.D / 32;
+  const bf16_t* wp = sg.w + (size_t)min(n0 + r16, sg.rows - 1) * p.D + 8 * kg;
+  const size_t x_at = (size_t)min(r16, p.M - 1) * p.D + 8 * kg;
+  f32x4 acc[2] = {(f32x4){0.f, 0.f, 0.f, 0.f}, (f32x4){0.f, 0.f, 0.f, 0.f}};
+  unsigned tag = 0;
+  for (int s0 = wave; s0 < steps; s0 += 4 * U) {
+    bf16x8 a[U], b[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) a[u] = ld8(wp + 32 * min(s0 + 4 * u, steps - 1));
+    if constexpr (OUT) {
+      // the rows go through LDS: a thread brings its share of their words, two at a time
+      if (s0 == wave) {
+        constexpr int N = 8;
+        const auto* y = reinterpret_cast<const unsigned long long*>(one.y_words);
+        unsigned* to = reinterpret_cast<unsigned*>(step_rows);
+        const int pairs = p.M * p.D / 2;
+        tag = step_tag(one);
+        for (int i0 = threadIdx.x; i0 < pairs; i0 += 256 * N) {
+          unsigned long long w[N];
+          wait_for(one, [&]() __attribute__((always_inline)) {
+            unsigned late = 0;
+#pragma unroll
+            for (int j = 0; j < N; ++j) w[j] = __hip_atomic_load(y + min(i0 + 256 * j, pairs - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int j = 0; j < N; ++j) late |= (((unsigned)w[j] & 0xffffu) ^ tag) | (((unsigned)(w[j] >> 32) & 0xffffu) ^ tag);
+            return late;
+          });
+#pragma unroll
+          for (int j = 0; j < N; ++j)
+            if (i0 + 256 * j < pairs) to[i0 + 256 * j] = __builtin_amdgcn_perm((unsigned)(w[j] >> 32), (unsigned)w[j], 0x07060302);
+        }
+        __syncthreads();
+      }
+    } else {
+      if (s0 == wave) tag = step_tag(one);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) b[u] = OUT ? *reinterpret_cast<const bf16x8*>(step_rows + x_at + 32 * min(s0 + 4 * u, steps - 1)) : ld8(p.x + x_at + 32 * min(s0 + 4 * u, steps - 1));
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (s0 + 4 * u < steps) acc[u & 1] = mfma16(a[u], b[u], acc[u & 1]);
+  }
+  red[wave][lane] = acc[0];
+  red[wave + 4][lane] = acc[1];
+  __syncthreads();
+  if (wave != 0) return;
+  f32x4 sum = red[0][lane];
+#pragma unroll
+  for (int w = 1; w < 8; ++w) sum += red[w][lane];
+  const int n = n0 + 4 * kg;
+  if constexpr (!OUT) {
+    if (r16 < p.M) {
+      unsigned* dst = one.proj_words + (size_t)r16 * p.ldo + sg.col0 + n;    // (a row's tiles are whole in the words)
+#pragma unroll
+      for (int j = 0; j < 4; j += 2) {
+        const unsigned long long lo = tagged(f32_to_bf16(sum[j]), tag), hi = tagged(f32_to_bf16(sum[j + 1]), tag);
+        __hip_atomic_store(reinterpret_cast<unsigned long long*>(dst + j), lo | hi << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    return;
+  }
+  unsigned left = 0u;
+  if (lane == 0) left = __hip_atomic_fetch_add(one.sync + StepSync::LEFT, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // (a step that has failed leaves no numbers)
+  if (ld_word(one.sync + StepSync::FAILED)) sum = (f32x4){NAN, NAN, NAN, NAN};
+  if (r16 < p.M) {
+    bf16_t* dst = p.out + (size_t)r16 * p.ldo + n;
+    if (n + 4 <= sg.rows) {
+      *reinterpret_cast<u32x2*>(dst) = (u32x2){pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3])};
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (n + j < sg.rows) dst[j] = f32_to_bf16(sum[j]);
+    }
+  }
+  if (__builtin_amdgcn_readfirstlane(left) + 1u == (unsigned)all.out_tiles) {       // all tails are written: nobody counts or looks any more
+    for (int i = lane; i < one.m.s.B * one.a.HQ; i += 64) __hip_atomic_store(one.arrived + i, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (lane == 0) {
+      __hip_atomic_store(one.sync + StepSync::LEFT, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(one.sync + StepSync::EPOCH, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+}
+
+// (as many workgroups a CU as step_one_kernel's registers allow: the splits count on them)
+template <int KA, int VA, int K, bool DELTA>
+__global__ __launch_bounds__(256, K == 192 || KA + VA == 256 ? 2 : KA + VA + K == 192 ? 4 : 3) void step_all_kernel(const StepAll) {
+  const StepAll& all = step_all_args();
+  constexpr int U = K == 192 ? 18 : KA + VA + K == 192 ? 8 : 12;
+  int id = blockIdx.x;
+  if (id < all.in_tiles) return step_product<false, 12>(all, id);
+  id -= all.in_tiles;
+  const int roles = (int)gridDim.x - all.in_tiles - all.out_tiles;
+  if (id < roles) step_roles<KA, VA, K, DELTA, true>(all.one, id);
+  else step_product<true, U>(all, id - roles);
+}
+
+// all: the products of the launch, or null where they are launches of their own
+static int launch_step_one(const char* what, const StepOne& p, const StepAll* all, const int K, const int KA, const int VA, hipStream_t st) {
   const natsl_layer_step& s = p.m.s;
-  const dim3 grid((unsigned)(p.n_logits + p.n_rec + s.B * s.HQ * p.a.nsplit));
-#define NATSL_S1(KK, VV, KL, DD)                                                              \
-  if (KA == KK && VA == VV && K == KL && (s.is_delta != 0) == DD) {                           \
-    hipLaunchKernelGGL((step_one_kernel<KK, VV, KL, DD>), grid, dim3(256), 0, st, p);         \
-    return check_launch(what);                                                                \
+  const unsigned roles = (unsigned)(p.n_logits + p.n_rec + s.B * s.HQ * p.a.nsplit), grid = all ? all->in_tiles + roles + all->out_tiles : roles;
+  const size_t rows = all ? (size_t)s.B * s.H * s.V * sizeof(bf16_t) : 0;
+#define NATSL_S1(KK, VV, KL, DD)                                                                            \
+  if (KA == KK && VA == VV && K == KL && (s.is_delta != 0) == DD) {                                         \
+    if (all) hipLaunchKernelGGL((step_all_kernel<KK, VV, KL, DD>), dim3(grid), dim3(256), rows, st, *all);  \
+    else hipLaunchKernelGGL((step_one_kernel<KK, VV, KL, DD>), dim3(grid), dim3(256), 0, st, p);            \
+    return check_launch(what);                                                                              \
   }
 #define NATSL_S3(KK, VV)                                                                                                     \
   NATSL_S1(KK, VV, 64, true) NATSL_S1(KK, VV, 128, true) NATSL_S1(KK, VV, 192, true) NATSL_S1(KK, VV, 64, false)             \
@@ -681,16 +956,30 @@ static int launch_step_one(const char* what, const StepOne& p, const int K, cons
 struct StepLayout {
   int ldp, cq, ck, cv, cg, ca, cb, tiles, nsplit, n_chunks;
   bool one;
+  bool all;                   // ... and the products can be in it
   size_t proj, q_conv, q_lin, q_attn, o_lin, y, partials, logits, arrived, bytes;
+  size_t proj_words, y_words, sync_bytes;   // in the caller's memory behind StepSync
 };
 
 // Workgroups of step_one_kernel that fit on the chip at once, less those of the logits and the recurrence: what its registers allow a CU
 // (236 with 192-wide states: two; 104 with 64-wide everything: four; else 129 - 168: three.  128-wide keys and values are counted as two, which
 // the splits below were measured with).
-static int step_one_slots(const natsl_layer_step& s, const int n_chunks) {
+static int step_one_per_cu(const natsl_layer_step& s) {
   const int KA = s.H * s.K / s.HQ, VA = s.H * s.V / s.HQ;
-  const int per_cu = s.K == 192 || KA + VA == 256 ? 2 : KA + VA + s.K == 192 ? 4 : 3;
-  return per_cu * 256 - s.B * (n_chunks + s.H * cdiv(s.V, 64));
+  return s.K == 192 || KA + VA == 256 ? 2 : KA + VA + s.K == 192 ? 4 : 3;
+}
+static int step_one_slots(const natsl_layer_step& s, const int n_chunks) {
+  return step_one_per_cu(s) * 256 - s.B * (n_chunks + s.H * cdiv(s.V, 64));
+}
+
+// Workgroups that wait when the products are in the launch too: those between the products and those behind them.  At most half of what fits on
+// the chip, so that one that is waited for always finds room, and no more than this: with 268 of the 340M geometry (four sequences of 500 tokens) a
+// token is 0.87 of the three launches' time, with 304 and 352 of 16 heads of 128/64 (six of 300, four of 1200) 1.02, where the
+// host is no longer what a step waits for.
+constexpr int STEP_WAITERS = 280;
+static bool step_may_wait(const natsl_layer_step& s, const int n_chunks, const int nsplit) {
+  const int n = s.B * (n_chunks + s.H * cdiv(s.V, 64) + s.HQ * nsplit) + cdiv(s.D, 16);
+  return n <= STEP_WAITERS && 2 * n <= step_one_per_cu(s) * 256;
 }
 
 // One token a sequence: one launch between the two products.  That kernel is built for the layers' own convolution width and reads windows
@@ -741,6 +1030,15 @@ static StepLayout step_layout(const natsl_layer_step& s) {
   l.logits = take((size_t)M * l.n_chunks * s.HQ * 2 * 4);
   l.arrived = take((size_t)M * s.HQ * 4);
   l.bytes = at;
+  // The products in the launch: a row tile of tokens, whose rows fit the output projection's workgroups (each of its waves has a part of a row), and
+  // no more workgroups that wait than may; whether they do at this step's number of
+  // keys is step_fwd's to see, so that a cache's steps all want the same memory.
+  l.all = l.one && M <= 16 && M * VD <= STEP_ROWS && VD >= 128 && step_may_wait(s, l.n_chunks, 1);
+  at = 0;
+  take((StepSync::ARRIVED + (size_t)M * s.HQ) * 4);
+  l.proj_words = take((size_t)M * l.ldp * 4);
+  l.y_words = take((size_t)M * VD * 4);
+  l.sync_bytes = l.all ? at : 0;
   return l;
 }
 
@@ -768,8 +1066,8 @@ extern "C" size_t natsl_layer_step_workspace_bytes(const natsl_layer_step* step)
   return step && step_check(*step, "natsl_layer_step") == NATSL_OK ? step_layout(*step).bytes : 0;
 }
 
-extern "C" int natsl_layer_step_fwd(const natsl_layer_step* step, void* workspace, size_t workspace_bytes, natsl_stream_t stream) {
-  const char* what = "natsl_layer_step_fwd";
+static int step_fwd(const char* what, const natsl_layer_step* step, void* workspace, size_t workspace_bytes, unsigned* sync, size_t sync_bytes,
+                    unsigned long long max_wait_us, natsl_stream_t stream) {
   if (!step || !workspace) return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
   const natsl_layer_step& s = *step;
   int rc = step_check(s, what);
@@ -782,7 +1080,11 @@ extern "C" int natsl_layer_step_fwd(const natsl_layer_step* step, void* workspac
     return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
   const StepLayout l = step_layout(s);
   if (workspace_bytes < l.bytes) return fail(NATSL_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", what, l.bytes, workspace_bytes);
+  if (sync && ((uintptr_t)sync % 8 || sync_bytes < l.sync_bytes))
+    return fail(NATSL_ERR_INVALID, "%s: %zu bytes of the step's own memory needed, %zu given", what, l.sync_bytes, sync_bytes);
   const int KD = s.H * s.K, VD = s.H * s.V, KA = KD / s.HQ, VA = VD / s.HQ, M = s.B * s.T;
+  const int out_tiles = cdiv(s.D, 16);
+  const bool in_one = sync && l.all && step_may_wait(s, l.n_chunks, l.nsplit);
   char* ws = reinterpret_cast<char*>(workspace);
   bf16_t *proj = (bf16_t*)(ws + l.proj), *q_conv = (bf16_t*)(ws + l.q_conv), *q_lin = (bf16_t*)(ws + l.q_lin), *q_attn = (bf16_t*)(ws + l.q_attn),
          *o_lin = (bf16_t*)(ws + l.o_lin), *y = (bf16_t*)(ws + l.y);
@@ -800,13 +1102,13 @@ extern "C" int natsl_layer_step_fwd(const natsl_layer_step* step, void* workspac
   const GemmSeg segs[GEMM_SEGS] = {{(const bf16_t*)s.wq, KD, 0, l.cq}, {(const bf16_t*)s.wk, KD, 0, l.ck}, {(const bf16_t*)s.wv, VD, 0, l.cv},
                                    {(const bf16_t*)s.wg, VD, 0, l.cg}, {(const bf16_t*)s.wa, s.H, 0, l.ca}, {(const bf16_t*)s.wb, s.H, 0, l.cb}};
   g.n_seg = s.is_delta ? 6 : 5;
-  unsigned* arrived = (unsigned*)(ws + l.arrived);
-  g.zero = arrived; g.n_zero = l.one ? M * s.HQ : 0;
+  unsigned* arrived = in_one ? sync + StepSync::ARRIVED : (unsigned*)(ws + l.arrived);
+  g.zero = arrived; g.n_zero = l.one && !in_one ? M * s.HQ : 0;
   for (int i = 0; i < GEMM_SEGS; ++i) {
     g.seg[i] = segs[i];
     g.seg[i].tile0 = segs[i].col0 / 16;
   }
-  if ((rc = gemm(g, l.tiles)) != NATSL_OK) return rc;
+  if (!in_one && (rc = gemm(g, l.tiles)) != NATSL_OK) return rc;
 
   StepMix m;
   m.s = s; m.proj = proj; m.ldp = l.ldp; m.cq = l.cq; m.ck = l.ck; m.cv = l.cv; m.ca = l.ca; m.cb = l.cb;
@@ -839,8 +1141,15 @@ extern "C" int natsl_layer_step_fwd(const natsl_layer_step* step, void* workspac
     f.m = m; f.a = a; f.r = r; f.t = t;
     f.o_lin = (float*)(ws + l.o_lin); f.logits = (float*)(ws + l.logits); f.arrived = arrived;
     f.n_chunks = l.n_chunks; f.n_logits = s.B * l.n_chunks; f.n_rec = s.B * s.H * cdiv(s.V, 64);
-    if ((rc = launch_step_one(what, f, s.K, KA, VA, st)) != NATSL_OK) return rc;
-    return gemm(o, cdiv(s.D, 16));
+    if (in_one) {
+      char* mem = reinterpret_cast<char*>(sync);
+      f.sync = sync; f.proj_words = reinterpret_cast<unsigned*>(mem + l.proj_words); f.y_words = reinterpret_cast<unsigned*>(mem + l.y_words);
+      f.max_wait = 100 * max_wait_us;                     // (the counter behind s_memrealtime runs at 100 MHz)
+      const StepAll all = {f, g, o, l.tiles, out_tiles};
+      return launch_step_one(what, f, &all, s.K, KA, VA, st);
+    }
+    if ((rc = launch_step_one(what, f, nullptr, s.K, KA, VA, st)) != NATSL_OK) return rc;
+    return gemm(o, out_tiles);
   }
 
   const dim3 mgrid(3 * s.H + (s.block_hidden ? cdiv(s.D, 256) : 0), s.B);
@@ -855,4 +1164,17 @@ extern "C" int natsl_layer_step_fwd(const natsl_layer_step* step, void* workspac
   else hipLaunchKernelGGL((step_tail_kernel<64>), tgrid, dim3(256), 0, st, t);
   if ((rc = check_launch(what)) != NATSL_OK) return rc;
   return gemm(o, cdiv(s.D, 16));
+}
+
+extern "C" int natsl_layer_step_fwd(const natsl_layer_step* step, void* workspace, size_t workspace_bytes, natsl_stream_t stream) {
+  return step_fwd("natsl_layer_step_fwd", step, workspace, workspace_bytes, nullptr, 0, 0, stream);
+}
+
+extern "C" size_t natsl_layer_step_sync_bytes(const natsl_layer_step* step) {
+  return step && step_check(*step, "natsl_layer_step") == NATSL_OK ? step_layout(*step).sync_bytes : 0;
+}
+
+extern "C" int natsl_layer_step_sync_fwd(const natsl_layer_step* step, void* workspace, size_t workspace_bytes, void* shared, size_t shared_bytes,
+                                         uint64_t max_wait_us, natsl_stream_t stream) {
+  return step_fwd("natsl_layer_step_sync_fwd", step, workspace, workspace_bytes, reinterpret_cast<unsigned*>(shared), shared_bytes, max_wait_us, stream);
 }

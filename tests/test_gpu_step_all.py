@@ -1,0 +1,69 @@
+"""The one-token generation step as one launch, products included, against the same step as three launches, bit for bit; and what becomes of a
+part of it that waits too long."""
+import ctypes
+
+import pytest
+import torch
+
+from tests.test_gpu_layer_step import _generate, _layer
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda:0'
+
+
+def _three_launches(monkeypatch):
+    from neuralattentionsearchlinear_amd import _capi
+    none = ctypes.CFUNCTYPE(ctypes.c_size_t, ctypes.c_void_p)(lambda step: 0)
+    monkeypatch.setattr(_capi.lib(), 'natsl_layer_step_sync_bytes', none)
+    return none                                            # (held by the caller while a plan has its address)
+
+
+@pytest.mark.parametrize("kind,geometry,B,T0,n,more", [
+    ('gdn', '340M', 1, 777, 5, {}),
+    ('gdn', '340M', 3, 100, 30, {}),                                       # over the end of a block: the cache and the splits change
+    ('gdn', '760M', 1, 300, 3, dict(allow_neg_eigval=True, conv_bias=True)),
+    ('gdn', None, 1, 64, 2, dict(head_dim=64, num_heads=2, num_attn_heads=2, expand_v=1)),   # rows of 128: one step of the products a wave
+    ('gdn', None, 5, 127, 3, dict(hidden_size=288, head_dim=64, num_heads=5, num_attn_heads=5)),  # 9 steps, 5-row weights, products' waves of 2 and 3
+    ('mamba', None, 2, 95, 3, dict(expand_v=1)),
+    ('mamba', None, 16, 64, 2, dict(head_dim=64, num_heads=2, num_attn_heads=2, expand_v=1)),   # a whole row tile
+    ('mamba', None, 1, 257, 2, dict(attn_with_short_conv=False, conv_bias=True)),
+])
+def test_one_launch_is_the_three(kind, geometry, B, T0, n, more, monkeypatch):
+    layer = _layer(kind, geometry, 'all', **more)
+    torch.manual_seed(T0)
+    x = torch.randn(B, T0 + n, layer.hidden_size, device=DEV).bfloat16()
+    one, c1 = _generate(layer, kind, x, T0, (1,) * n)
+    again, _ = _generate(layer, kind, x, T0, (1,) * n)
+    assert c1.step_shared is not None and int(c1.step_shared[64]) == n, "the steps were not one launch each"
+    held = _three_launches(monkeypatch)
+    layer2 = _layer(kind, geometry, 'all', **more)
+    three, c3 = _generate(layer2, kind, x, T0, (1,) * n)
+    assert c3.step_shared is None and held is not None
+    for i, (a, b, c) in enumerate(zip(one, again, three)):
+        assert torch.equal(a, b) and torch.equal(a, c), f"step {i}"
+    for name in ('attn_k', 'attn_v', 'recurrent_state', 'g_cumsum', 'lattn_g', 'l_attn_k', 'l_attn_v'):
+        a, b = getattr(c1, name), getattr(c3, name)
+        n_in = c1._n_tokens_in_nats_block
+        if name.startswith('l'):
+            a, b = a[:, :n_in], b[:, :n_in]
+        elif name.startswith('attn'):
+            a, b = a[:, :c1.n_attn_tokens_max], b[:, :c1.n_attn_tokens_max]
+        assert torch.equal(a, b), name
+
+
+def test_a_step_that_waits_too_long_gives_no_numbers(monkeypatch):
+    """With no time to wait every part of the launch gives up at once: it ends, its output is NaN, and so are those of later steps on that cache;
+    another cache is not touched by it."""
+    import neuralattentionsearchlinear_amd._layer_step as LS
+    torch.manual_seed(0)
+    x = torch.randn(1, 103, 256, device=DEV).bfloat16()
+    good, _ = _generate(_layer('gdn', None, 'all'), 'gdn', x, 100, (1,) * 3)
+    monkeypatch.setattr(LS, 'MAX_WAIT_US', 0)
+    layer = _layer('gdn', None, 'all')
+    bad, cache = _generate(layer, 'gdn', x, 100, (1,) * 3)
+    torch.cuda.synchronize()
+    assert int(cache.step_shared[32]) == 1
+    assert all(bool(o.isnan().all()) for o in bad[1:])
+    monkeypatch.undo()
+    after, _ = _generate(_layer('gdn', None, 'all'), 'gdn', x, 100, (1,) * 3)
+    assert all(torch.equal(a, b) for a, b in zip(good, after))

@@ -270,8 +270,9 @@ void rest(const Call& c, const Front& f, const bool joint, const Needs& needs, c
 // what the forward keeps, in this order behind x and the weights: each only where a part that runs reads it
 enum Kept { AB, WAB, POOLED, LOGITS, TYPES, RAW_Q, RAW_K, RAW_V, GATE, Y_Q, Y_K, Y_V, N_Q, N_K, MIX, G, BETA, DT, O_LIN, O_ATTN, LSE, IDX, NBLK, TAIL, STATES, V_NEW, WS, KEPT };
 
-// dy_i [rows, n_i]^T x [rows, D], one launch for those whose widths are multiples of 8; a narrow one that is not, or that is alone, by itself
-void wgrads(const Call& c, const T& x, const std::vector<T>& dys, std::vector<T>& out) {
+// dy_i [rows, n_i]^T x [rows, D], one launch for those whose widths are multiples of 8; a narrow one that is not, or that is alone, by itself.  On
+// the stream `on`; what is only used there is kept in `hold`.
+void wgrads(const Call& c, const T& x, const std::vector<T>& dys, std::vector<T>& out, natsl_stream_t on, Ts& hold) {
   const int64_t rows = x.size(0), D = x.size(1);
   out.assign(dys.size(), T());
   std::vector<natsl_wgrad_seg> segs;
@@ -284,7 +285,8 @@ void wgrads(const Call& c, const T& x, const std::vector<T>& dys, std::vector<T>
       out[i] = at::empty({N, D}, c.bf16);
       const size_t n = c.l.narrow_wgrad_workspace_bytes(rows, (int)D, (int)N);
       const T ws = c.bytes(n);
-      must(c.l.narrow_wgrad_split(at_(dy), at_(x), at_(out[i]), rows, (int)D, (int)N, at_(ws), n, c.stream), "natsl_narrow_wgrad_split");
+      hold.push_back(ws);
+      must(c.l.narrow_wgrad_split(at_(dy), at_(x), at_(out[i]), rows, (int)D, (int)N, at_(ws), n, on), "natsl_narrow_wgrad_split");
       continue;
     }
     if (dy.size(1) % 8 || D % 8 || !on16(x) || !on16(dy)) {
@@ -297,19 +299,27 @@ void wgrads(const Call& c, const T& x, const std::vector<T>& dys, std::vector<T>
   if (segs.empty()) return;
   const size_t n = c.l.wgrad_workspace_bytes(segs.data(), (int)segs.size(), rows, (int)D);
   const T ws = c.bytes(n);
-  must(c.l.wgrad(segs.data(), (int)segs.size(), at_(x), rows, (int)D, (int)D, at_(ws), n, c.stream), "natsl_wgrad");
+  hold.push_back(ws);
+  must(c.l.wgrad(segs.data(), (int)segs.size(), at_(x), rows, (int)D, (int)D, at_(ws), n, on), "natsl_wgrad");
 }
-T wgrad(const Call& c, const T& x, const T& dy) {
+T wgrad(const Call& c, const T& x, const T& dy, natsl_stream_t on, Ts& hold) {
   std::vector<T> out;
-  wgrads(c, x, {dy}, out);
+  wgrads(c, x, {dy}, out, on, hold);
   return out[0];
 }
+T wgrad(const Call& c, const T& x, const T& dy) {
+  Ts hold;
+  return wgrad(c, x, dy, c.stream, hold);
+}
 
-T narrow_bwd(const Call& c, const T& dy, const T& w, const bool few) {
+bool narrow_bwd_takes(const Call& c, const T& dy, const T& w, const bool few) {
+  return c.l.narrow_linear_bwd_pays(dy.size(0), (int)w.size(1), (int)w.size(0), few) && on16(dy) && on16(w);
+}
+T narrow_bwd(const Call& c, const T& dy, const T& w, const bool few, natsl_stream_t on, T dx = T()) {
   const int64_t N = w.size(0), D = w.size(1);
-  if (!c.l.narrow_linear_bwd_pays(dy.size(0), (int)D, (int)N, few) || !on16(dy) || !on16(w)) return at::mm(dy, w);
-  T dx = at::empty({dy.size(0), D}, c.bf16);
-  must(c.l.narrow_linear_bwd(at_(dy), at_(w), at_(dx), dy.size(0), (int)D, (int)N, c.stream), "natsl_narrow_linear_bwd");
+  if (!narrow_bwd_takes(c, dy, w, few)) return at::mm(dy, w);
+  if (!dx.defined()) dx = at::empty({dy.size(0), D}, c.bf16);
+  must(c.l.narrow_linear_bwd(at_(dy), at_(w), at_(dx), dy.size(0), (int)D, (int)N, on), "natsl_narrow_linear_bwd");
   return dx;
 }
 
@@ -332,7 +342,9 @@ struct MixedGrads {
   T q_a, k_a, v_a, q_l, k_l, v_l, g, beta, logits;                // logits: the selector's
 };
 
-MixedGrads mixed_bwd(const Call& c, const Ts& s, const T& do_lin, const T& do_attn, const int invalid_attn, const int invalid_linear) {
+// behind: what else may run behind the softmax branch, on the stream that it is given: beside the linear branch's last kernel, where there are two.
+template <class Behind>
+MixedGrads mixed_bwd(const Call& c, const Ts& s, const T& do_lin, const T& do_attn, const int invalid_attn, const int invalid_linear, Behind behind) {
   const Layer& l = c.l;
   const int64_t nb = blocks_of(c.T_), chunks = c.B * nb;
   const bool delta = l.delta, beside = c.side != c.stream, saved = s[STATES].defined();
@@ -385,7 +397,10 @@ MixedGrads mixed_bwd(const Call& c, const Ts& s, const T& do_lin, const T& do_at
                                 c.stream), "natsl_linear_chunk_bwd_steps");
   if (beside) {
     softmax(c.side);
+    behind(c.side);
     fork.join();
+  } else {
+    behind(c.stream);
   }
   r.logits = like(s[LOGITS]);
   must(l.block_grads_logits(at_(s[TYPES]), at_(s[LOGITS]), NATSL_BF16, f_(gate), l.decay ? f_(rb) : nullptr, f_(dnats), l.HQ, f_(r.g), at_(r.logits), invalid_linear,
@@ -420,18 +435,30 @@ void backward(const Call& c, const T& x, Ts& s, const Needs& need, const int inv
     }
   }
   drop(dy, s[O_LIN], s[GATE], s[MIX]);
-  MixedGrads m;
-  if (need.op) m = mixed_bwd(c, s, do_lin, do_attn, invalid_attn, invalid_linear);
-  drop(do_lin, do_attn);
-  for (const Kept i : {O_ATTN, LSE, IDX, NBLK, TYPES, LOGITS, G, BETA, N_Q, N_K, Y_K, Y_V, STATES, V_NEW, WS}) drop(s[i]);
-  // mixing logits, convolutions
+  // mixing logits: they need the norm-gate only, and the softmax branch's stream is done 75 to 160 us before the linear branch's (a layer's training
+  // step at 340M 8 x 4096 3 202 -> 3 184 us, 760M 2 x 3000 1 468 -> 1 446; o_proj's weight gradient there as well: 3 223 and 1 485 for 3 266 and 1 503)
+  Ts hold;                                               // (what that stream uses lives until it is joined)
+  T dq_mix;
   dmix = dmix.view({rows, -1});
-  if (want(W_MIX)) grads[1 + W_MIX] = wgrad(c, s[Y_Q].view({rows, -1}), dmix);
-  drop(s[Y_Q]);
+  auto mixing = [&](natsl_stream_t on) {
+    if (want(W_MIX)) grads[1 + W_MIX] = wgrad(c, s[Y_Q].view({rows, -1}), dmix, on, hold);
+    // (its place is the softmax branch's output gradient, which only that branch reads; where that is too small it waits)
+    if (!need.op || !need.conv) return;
+    const int64_t n = rows * w[W_MIX].size(1);
+    if (n <= do_attn.numel() && narrow_bwd_takes(c, dmix, w[W_MIX], false))
+      dq_mix = narrow_bwd(c, dmix, w[W_MIX], false, on, do_attn.view({-1}).narrow(0, 0, n).view({rows, -1}));
+  };
+  MixedGrads m;
+  if (need.op) m = mixed_bwd(c, s, do_lin, do_attn, invalid_attn, invalid_linear, mixing);
+  else mixing(c.stream);
+  drop(do_lin, do_attn, s[Y_Q]);
+  hold.clear();
+  for (const Kept i : {O_ATTN, LSE, IDX, NBLK, TYPES, LOGITS, G, BETA, N_Q, N_K, Y_K, Y_V, STATES, V_NEW, WS}) drop(s[i]);
+  // convolutions
   T dx[4], ddt;
   dx[3] = std::move(dgate);
   if (need.conv) {
-    const T dq_mix = narrow_bwd(c, dmix, w[W_MIX], false);
+    if (!dq_mix.defined()) dq_mix = narrow_bwd(c, dmix, w[W_MIX], false, c.stream);
     drop(dmix);
     natsl_conv_seg g[3];
     conv_segs(c, &s[RAW_Q], s[DT], g);
@@ -465,7 +492,7 @@ void backward(const Call& c, const T& x, Ts& s, const Needs& need, const int inv
     const T ws = c.bytes(n);
     must(l.conv_norm_bwd(g, 3, (int)c.B, (int)c.T_, l.W, l.act, l.norm_dtype, at_(ws), n, c.stream), "natsl_conv_norm_bwd");
   }
-  drop(dmix, m.q_a, m.k_a, m.v_a, m.q_l, m.k_l, m.v_l, s[RAW_Q], s[RAW_K], s[RAW_V], s[DT]);
+  drop(dmix, dq_mix, m.q_a, m.k_a, m.v_a, m.q_l, m.k_l, m.v_l, s[RAW_Q], s[RAW_K], s[RAW_V], s[DT]);
   // gates
   T dab;
   if (need.gates) {
@@ -497,7 +524,7 @@ void backward(const Call& c, const T& x, Ts& s, const Needs& need, const int inv
   if (dab.defined()) dys[4] = dab.view({rows, -1});
   if (need.x()) {
     const int64_t ld = dab.size(2);
-    const T dpool = narrow_bwd(c, dl2, w[WN], true), dX = c.sized(l.D);
+    const T dpool = narrow_bwd(c, dl2, w[WN], true, c.stream), dX = c.sized(l.D);
     natsl_project_seg segs[5];
     for (int i = 0; i < 5; ++i) {
       const T& ww = i < 4 ? w[WQ + i] : s[WAB];
@@ -517,7 +544,7 @@ void backward(const Call& c, const T& x, Ts& s, const Needs& need, const int inv
   if (!want(WA) && !want(WB)) dys[4] = T();
   if (std::none_of(dys.begin(), dys.end(), [](const T& t) { return t.defined(); })) return;
   std::vector<T> dws;
-  wgrads(c, x.view({rows, l.D}), dys, dws);
+  wgrads(c, x.view({rows, l.D}), dys, dws, c.stream, hold);
   for (int i = 0; i < 4; ++i) grads[1 + WQ + i] = dws[i];
   if (dws[4].defined()) {
     grads[1 + WA] = dws[4].slice(0, 0, l.H);

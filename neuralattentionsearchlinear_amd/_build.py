@@ -33,7 +33,7 @@ def _hipcc() -> str:
 def _build_step_core():
     import torch
     from torch.utils.cpp_extension import include_paths
-    srcs = [os.path.join(CSRC, "host", f) for f in ("step_core.cpp", "layer_core.cpp")]
+    srcs = [os.path.join(CSRC, "host", f) for f in ("step_core.cpp", "layer_core.cpp", "mixed_core.cpp")]
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-fPIC", "-shared", "-std=c++17", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            *(f"-I{d}" for d in (sysconfig.get_paths()["include"], *include_paths())), *srcs, "-o", STEP_CORE,
            "-L" + os.path.join(os.path.dirname(torch.__file__), "lib"), "-lc10", "-ltorch_cpu", "-ltorch_python"]

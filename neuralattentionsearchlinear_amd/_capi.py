@@ -19,6 +19,7 @@ F32, BF16 = 0, 1
 DECAY_NON_LINEAR, QK_L2NORM, INTRA_CHUNK, QUERY_ONLY, FRESH_BLOCK_START, STATES_ONLY = 1, 2, 4, 8, 16, 32
 
 _lib = _step_core = None
+_entries = None
 
 _SIGNATURES = {
     "natsl_version": (c_int, []),
@@ -154,6 +155,14 @@ def step_core():
         from . import _step_core as core
         _step_core = core
     return _step_core
+
+
+def entries():
+    """What the native host side of the operators calls (csrc/host/mixed_core.cpp)."""
+    global _entries
+    if _entries is None:
+        _entries = step_core().make_entries(lib()._handle)
+    return _entries
 
 
 def exported_symbols():

@@ -406,6 +406,9 @@ PyMethodDef methods[] = {
     {"layer_backward", fast(natsl_layer_backward), METH_FASTCALL, nullptr},
     {"layer_front", fast(natsl_layer_prompt_front), METH_FASTCALL, nullptr},
     {"layer_rest", fast(natsl_layer_prompt_rest), METH_FASTCALL, nullptr},
+    {"make_entries", natsl_make_entries, METH_VARARGS, nullptr},
+    {"mixed_plain", fast(natsl_mixed_plain), METH_FASTCALL, nullptr},
+    {"hard_select", fast(natsl_hard_select_plain), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_step_core", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -137,6 +137,12 @@ def hard_select(logits: torch.Tensor, force_last_block: bool = False, seqs: Opti
     force_last_block it also applies `types[:, -1] = 1` and counts the blocks (:553-554)."""
     if logits.shape[-1] != 2:
         raise NotImplementedError("the selector is built for n_ops == 2")
+    if seqs is None and logits.is_cuda and not (torch.is_grad_enabled() and logits.requires_grad):
+        done = _capi.step_core().hard_select(_capi.entries(), logits, force_last_block, _capi.stream_ptr(logits.device))
+        if type(done) is tuple:
+            return done
+        if done is not None:
+            _capi.check(done, "natsl_hard_select")
     logits = logits.contiguous()
     B, TN, HN, _ = logits.shape
     types = torch.empty_like(logits)

@@ -575,15 +575,14 @@ class _Layer(torch.autograd.Function):
         kept = list(ctx.saved_tensors)
         ctx.maybe_clear_saved_tensors()                    # (not where the graph is retained; nodes of their own are freed one by one, too)
         grads = _capi.step_core().layer_backward(
-            ctx.native, dout.to(torch.bfloat16), kept, ctx.needs_input_grad[2:], stream, _beside(dout, ctx.how, stream), ctx.how["invalid_attn"],
+            ctx.native, dout.to(torch.bfloat16), kept, ctx.needs_input_grad[2:], stream, _beside(dout, ctx.how, stream, True), ctx.how["invalid_attn"],
             ctx.how["invalid_linear"])
         return (None, None, *grads)
 
 
-def _beside(x, how, stream):
+def _beside(x, how, stream, gradients):
     """The stream of the softmax branch: the side stream, or the caller's."""
-    B, T = x.shape[:2]
-    if _mixed_common._run_side_by_side(x.device, False, B, B, T, how["H"], how["K"], how["V"]):
+    if _mixed_common._layer_runs_side_by_side(x.device, x.shape[0], x.shape[1], how, gradients):
         return _mixed_common._get_attn_stream(x.device).cuda_stream
     return stream
 
@@ -619,17 +618,18 @@ class FastFront:
         self.__dict__.update(constants)
         self.w, self.wn, self.native = w, wn, None
 
-    def _call(self, x):
+    def _call(self, x, gradients=False):
         """-> (stream, the softmax branch's stream, whether the wide projections are one launch)."""
         how, rows = self.how, x.shape[0] * x.shape[1]
         stream = _capi.stream_ptr(x.device)
-        return stream, _beside(x, how, stream), _joint_pays(rows, how["D"], how["widths"], how["cus"])
+        return stream, _beside(x, how, stream, gradients), _joint_pays(rows, how["D"], how["widths"], how["cus"])
 
     def train(self, x):
         """The layer's training forward on whole sequences (`native` only) -> (output, attention's share per head)."""
         weights = (*self.w.values(), self.wn)
-        stream, side, joint = self._call(x)
-        if self.grad(x, *weights):
+        gradients = self.grad(x, *weights)
+        stream, side, joint = self._call(x, gradients)
+        if gradients:
             how = self.how
             states = _mixed_common._keep_states_of(x.shape[0], x.shape[0], x.shape[1], how["H"], how["K"], how["V"])
             return _Layer.apply(self, (side, joint, states), x, *weights)

@@ -6,6 +6,7 @@
 // products reach).  Here the tokens are split as well: a unit is (slice of the tokens, 256 x 256 output tile), partial tiles go to
 // a workspace in fp32 and wgrad_reduce_kernel adds them in a fixed order.
 //
+// (WG_N rows of dY by 64 NB columns of X, NB 3 or 4: 256 or 192.)
 // Both operands have the contraction index as their slow dimension in memory and the matrix instruction wants it inside a lane:
 // tiles of 32 tokens x 256 columns go to LDS row by row (LDS-DMA, no staging registers) and operands are fetched with the
 // transposing read ds_read_b64_tr_b16.  What fixes the tile is the LDS: a wave that owns 128 x 128 of the output reads 8 operands
@@ -25,12 +26,13 @@ constexpr int WG_ROW = WG_N * 2;               // bytes of a tile row
 constexpr int WG_TILE = WG_T * WG_ROW;         // 16 KiB per operand
 constexpr int WG_STAGE = 2 * WG_TILE;
 constexpr int WG_STAGES = 4;
+constexpr double WG_TOKEN_US = 0.0213, WG_TOKEN_US_3 = 0.0187;   // a unit's time a token, by tile width (at the power limit)
 
 struct WgradSeg { const bf16_t* dy; bf16_t* out; int n, ld, tile0, block0; };   // tile0, block0: first row of tiles, of 32-row blocks
 struct WgradParams {
   const bf16_t* x;
   float* part;
-  int ldx, D, n_seg, tiles_d, tiles, blocks, splits, units;   // blocks: 32-row blocks of all weights
+  int ldx, D, n_seg, tiles_d, tiles, blocks, splits, units, nb;   // blocks: 32-row blocks of all weights; nb: the kernel's NB
   long long T, slice;                          // tokens; tokens per slice (a multiple of WG_T)
   WgradSeg seg[NATSL_WGRAD_SEGS];
 };
@@ -39,13 +41,16 @@ NATSL_DEVICE void wg_dma(const void* base, const unsigned voff, const unsigned l
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(lds) : "memory", "m0");
 }
 
-// Partial sums lie as strips of 32 rows x 256 columns (wg_strip), those that the weights have and no others: whole tiles of a 24-row weight
+// Partial sums lie as strips of 32 rows x a tile's columns (wg_strip), those that the weights have and no others: whole tiles of a 24-row weight
 // would be eight times as much (24 x 768 over 32768 tokens: 59 MiB, 7.4 as strips).
-constexpr int WG_STRIP = 32 * WG_N;
+// A tile has 64 NB columns of x: 256, or 192 where that leaves fewer CUs without work.
+constexpr int wg_strip_size(const int nb) { return 32 * 64 * nb; }
+template <int NB>
 NATSL_DEVICE size_t wg_strip(const WgradParams& p, const int split, const int td, const int block) {
-  return (((size_t)split * p.tiles_d + td) * p.blocks + block) * WG_STRIP;
+  return (((size_t)split * p.tiles_d + td) * p.blocks + block) * wg_strip_size(NB);
 }
 
+template <int NB>
 __global__ __launch_bounds__(256, 1) void wgrad_kernel(const WgradParams p) {
   extern __shared__ __align__(256) unsigned char wg_smem[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -58,7 +63,7 @@ __global__ __launch_bounds__(256, 1) void wgrad_kernel(const WgradParams p) {
 #pragma unroll
   for (int i = 1; i < NATSL_WGRAD_SEGS; ++i) si = i < p.n_seg && tn >= p.seg[i].tile0 ? i : si;
   const WgradSeg sg = p.seg[si];
-  const int n0 = (tn - sg.tile0) * WG_N, d0 = td * WG_N;
+  const int n0 = (tn - sg.tile0) * WG_N, d0 = td * 64 * NB;
   const long long t_first = (long long)split * p.slice;
   const int n_tok = (int)(p.T - t_first < p.slice ? p.T - t_first : p.slice);
   const int n_st = (n_tok + WG_T - 1) / WG_T;
@@ -74,7 +79,7 @@ __global__ __launch_bounds__(256, 1) void wgrad_kernel(const WgradParams p) {
   for (int i = 0; i < 4; ++i) {
     const int row = 8 * wave + 2 * i + r2, seg = slot ^ (4 * (row & 3));
     va[i] = (unsigned)(row * sg.ld * 2 + min(n0 / 8 + seg, sg.n / 8 - 1) * 16);
-    vb[i] = (unsigned)(row * p.ldx * 2 + min(d0 / 8 + seg, p.D / 8 - 1) * 16);
+    vb[i] = (unsigned)(row * p.ldx * 2 + min(d0 / 8 + min(seg, 8 * NB - 1), p.D / 8 - 1) * 16);   // (rows are 256 columns apart in LDS)
   }
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)wg_smem;
   auto request = [&](const int st) __attribute__((always_inline)) {
@@ -112,23 +117,22 @@ __global__ __launch_bounds__(256, 1) void wgrad_kernel(const WgradParams p) {
   // operand addresses: 16-lane group g, supplier (j, c) of the transposing read; column block cb of 32 columns
   const int g = lane >> 4, j = (lane & 15) >> 2, c = lane & 3;
   const int wn = wave >> 1, wd = wave & 1;
-  unsigned oa[4], ob[4];
+  unsigned oa[4], ob[NB];
+  const unsigned row = (8 * (g >> 1) + j) * WG_ROW + (2 * (g & 1) + (c >> 1)) * 16 + (c & 1) * 8;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const unsigned row = (8 * (g >> 1) + j) * WG_ROW + (2 * (g & 1) + (c >> 1)) * 16 + (c & 1) * 8;
-    oa[i] = lds0 + row + (4 * wn + (i ^ j)) * 64;
-    ob[i] = lds0 + WG_TILE + row + (4 * wd + (i ^ j)) * 64;
-  }
+  for (int i = 0; i < 4; ++i) oa[i] = lds0 + row + (4 * wn + (i ^ j)) * 64;
+#pragma unroll
+  for (int i = 0; i < NB; ++i) ob[i] = lds0 + WG_TILE + row + ((NB * wd + i) ^ j) * 64;
   typedef s16x4 __attribute__((address_space(3))) * lds_s4_t;
   auto operand = [&](const unsigned at) __attribute__((always_inline)) {
     return join4(__builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4_t)(uintptr_t)at), __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4_t)(uintptr_t)(at + 4 * WG_ROW)));
   };
 
-  f32x16 acc[4][4];
+  f32x16 acc[4][NB];
 #pragma unroll
   for (int a = 0; a < 4; ++a)
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
 
@@ -143,11 +147,11 @@ __global__ __launch_bounds__(256, 1) void wgrad_kernel(const WgradParams p) {
   __syncthreads();
   finish_partial(0);
   finish_partial(1);
-  bf16x8 A[2][4], B[2][4];
+  bf16x8 A[2][4], B[2][NB];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     A[0][i] = operand(oa[i]);
-    B[0][i] = operand(ob[i]);
+    if (i < NB) B[0][i] = operand(ob[i]);
   }
   // One stage's products.  AHEAD: stage st + 3 is a whole one, and its eight requests go out one behind every four products (issued
   // together they took 290 cycles in which the matrix cores had nothing: 4608 + 2 x 6 rows x 1024 columns over 32768 tokens 321 -> 264 us,
@@ -167,14 +171,15 @@ __global__ __launch_bounds__(256, 1) void wgrad_kernel(const WgradParams p) {
 #pragma unroll
       for (int a = 0; a < 4; ++a) {
         A[kk ^ 1][a] = operand(oa[a] + at);
-        B[kk ^ 1][a] = operand(ob[a] + at);
+        if (a < NB) B[kk ^ 1][a] = operand(ob[a] + at);
         if (WHOLE || a < blocks) {
 #pragma unroll
-          for (int b = 0; b < 4; ++b) acc[a][b] = mfma32(A[kk][a], B[kk][b], acc[a][b]);
+          for (int b = 0; b < NB; ++b) acc[a][b] = mfma32(A[kk][a], B[kk][b], acc[a][b]);
         }
         // one read next to each product: the scheduler otherwise saves registers by reading an operand right before its use
+        if constexpr (NB == 3) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < NB; ++i) {
           __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         }
@@ -199,33 +204,34 @@ __global__ __launch_bounds__(256, 1) void wgrad_kernel(const WgradParams p) {
   for (; st < n_st; ++st) stage(std::false_type{}, std::false_type{}, st);
 
   // lane: column d = lane%32 of each 32x32 tile, rows 8*(r/4) + 4*(lane/32) + r%4: four rows of a column per 16-byte store
-  float* dst = p.part + wg_strip(p, split, td, sg.block0 + (tn - sg.tile0) * 8 + 4 * (wave >> 1)) + (wave & 1) * 4096 + lane * 4;
+  float* dst = p.part + wg_strip<NB>(p, split, td, sg.block0 + (tn - sg.tile0) * 8 + 4 * (wave >> 1)) + (wave & 1) * (1024 * NB) + lane * 4;
 #pragma unroll
   for (int a = 0; a < 4; ++a)
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        if (a < blocks) *reinterpret_cast<f32x4*>(dst + a * WG_STRIP + (b * 4 + q) * 256) = (f32x4){acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]};
+        if (a < blocks) *reinterpret_cast<f32x4*>(dst + a * wg_strip_size(NB) + (b * 4 + q) * 256) = (f32x4){acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]};
 }
 
 // Adds the slices' partial tiles in order and writes the gradient: a workgroup takes one 32 x 32 block of a tile per wave.
+template <int NB>
 __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const WgradParams p) {
   const int lane = threadIdx.x & 63;
   const int id = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int tile = id >> 6, wave = (id >> 4) & 3, ab = id & 15;          // tile, wave of the tile, 32x32 block of the wave
+  const int tile = id / (16 * NB), wave = id / (4 * NB) & 3, ab = id % (4 * NB);   // tile, wave of the tile, 32x32 block of the wave
   const int tn = tile / p.tiles_d, td = tile - tn * p.tiles_d;
   int si = 0;
 #pragma unroll
   for (int i = 1; i < NATSL_WGRAD_SEGS; ++i) si = i < p.n_seg && tn >= p.seg[i].tile0 ? i : si;
   const WgradSeg sg = p.seg[si];
-  const int n = (tn - sg.tile0) * WG_N + 128 * (wave >> 1) + 32 * (ab >> 2), d = td * WG_N + 128 * (wave & 1) + 32 * (ab & 3) + (lane & 31);
+  const int n = (tn - sg.tile0) * WG_N + 128 * (wave >> 1) + 32 * (ab / NB), d = td * 64 * NB + 32 * NB * (wave & 1) + 32 * (ab % NB) + (lane & 31);
   if (n >= sg.n || d - (lane & 31) >= p.D) return;
   f32x4 sum[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) sum[q] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  const float* src = p.part + wg_strip(p, 0, td, sg.block0 + (tn - sg.tile0) * 8 + 4 * (wave >> 1) + (ab >> 2)) + (wave & 1) * 4096 + (ab & 3) * 1024 + lane * 4;
-  const size_t step = (size_t)p.tiles_d * p.blocks * WG_STRIP;
+  const float* src = p.part + wg_strip<NB>(p, 0, td, sg.block0 + (tn - sg.tile0) * 8 + 4 * (wave >> 1) + ab / NB) + (wave & 1) * (1024 * NB) + (ab % NB) * 1024 + lane * 4;
+  const size_t step = (size_t)p.tiles_d * p.blocks * wg_strip_size(NB);
   int s = 0;
   for (; s + 6 <= p.splits; s += 6) {          // (six slices on their way at a time; one by one a slice takes a round trip, 0.4 us)
     f32x4 v[6][4];
@@ -263,18 +269,24 @@ static int wgrad_cus() {
   return n;
 }
 
-// Slices of the tokens: a CU holds one unit at a time, so the launch takes ceil(tiles * slices / CUs) rounds of T / slices tokens
-// (measured: 17 ns a token), and every slice writes and reads its partial sums once more (0.1 us a whole tile; full: whole tiles'
-// worth of rows.  24 rows x 768 columns over 32768 tokens: 37 us with 32 slices of whole tiles, 27 with 85 of the strips that there are).
-static int wgrad_splits(long long T, int tiles, double full) {
+// Slices of the tokens and width of the tiles: a CU holds one unit at a time, so the launch takes ceil(tiles * slices / CUs) rounds of T / slices tokens,
+// and every slice writes and reads its partial sums once more (0.1 us a whole tile; full_rows: whole tiles' worth of rows.  24 rows x 768 columns over
+// 32768 tokens: 37 us with 32 slices of whole tiles, 27 with 85 of the strips that there are).  A tile of 192 columns takes 0.88 of the time of
+// one of 256 for 0.75 of its work and is taken where such tiles fill the CUs better: 6944 rows x 1536 columns over 6000 tokens, 232 units for 174, 155 -> 139
+// us; 1536 x 2304 over 6000 56 -> 53, 1024 x 1536 over 8192 41 -> 39; over 24000 tokens four slices of the first in tiles of 256 stay (461, 493 in 192).
+struct WgradSplit { int nb, splits; };
+static WgradSplit wgrad_splits(long long T, int tile_rows, int D, double full_rows) {
   const int cus = wgrad_cus();
-  int best = 1;
+  WgradSplit best{4, 1};
   double best_cost = 1e300;
-  for (int s = 1; s <= 128; ++s) {
-    if (s > 1 && T < 64ll * s) break;
-    const double rounds = (double)(((long long)tiles * s + cus - 1) / cus);
-    const double cost = rounds * (4.0 + 0.017 * (double)T / s) + 0.1 * full * s;
-    if (cost < best_cost) { best_cost = cost; best = s; }
+  for (int nb = 4; nb >= 3; --nb) {
+    const int tiles = tile_rows * cdiv(D, 64 * nb);
+    for (int s = 1; s <= 128; ++s) {
+      if (s > 1 && T < 64ll * s) break;
+      const double rounds = (double)(((long long)tiles * s + cus - 1) / cus);
+      const double cost = rounds * (4.0 + (nb == 4 ? WG_TOKEN_US : WG_TOKEN_US_3) * (double)T / s) + 0.1 * full_rows * (cdiv(D, 64 * nb) * nb / 4.) * s;
+      if (cost < best_cost) { best_cost = cost; best = {nb, s}; }
+    }
   }
   return best;
 }
@@ -284,7 +296,6 @@ static int wgrad_plan(WgradParams& p, const natsl_wgrad_seg* segs, int n_seg, co
   if (T <= 0 || D <= 0) return fail(NATSL_ERR_INVALID, "%s: non-positive dimension", what);
   if (D % 8 || ldx % 8 || ldx < D) return fail(NATSL_ERR_UNSUPPORTED, "%s: the input's width and row stride must be multiples of 8", what);
   p.x = (const bf16_t*)x; p.ldx = ldx; p.D = D; p.n_seg = n_seg; p.T = T;
-  p.tiles_d = cdiv(D, WG_N);
   int rows = 0;
   long long blocks = 0;
   for (int i = 0; i < NATSL_WGRAD_SEGS; ++i) {
@@ -296,9 +307,12 @@ static int wgrad_plan(WgradParams& p, const natsl_wgrad_seg* segs, int n_seg, co
     rows += cdiv(s.n, WG_N);
     blocks += cdiv(s.n, 32);
   }
-  p.tiles = rows * p.tiles_d;
   p.blocks = (int)blocks;
-  const int splits = wgrad_splits(T, p.tiles, blocks / 8. * p.tiles_d);
+  const WgradSplit how = wgrad_splits(T, rows, D, blocks / 8.);
+  const int splits = how.splits;
+  p.nb = how.nb;
+  p.tiles_d = cdiv(D, 64 * p.nb);
+  p.tiles = rows * p.tiles_d;
   p.slice = (T + splits - 1) / splits;
   p.slice = (p.slice + WG_T - 1) / WG_T * WG_T;
   p.splits = (int)((T + p.slice - 1) / p.slice);
@@ -307,7 +321,7 @@ static int wgrad_plan(WgradParams& p, const natsl_wgrad_seg* segs, int n_seg, co
   return NATSL_OK;
 }
 
-static size_t wgrad_bytes(const WgradParams& p) { return (size_t)p.splits * p.tiles_d * p.blocks * WG_STRIP * sizeof(float); }
+static size_t wgrad_bytes(const WgradParams& p) { return (size_t)p.splits * p.tiles_d * p.blocks * wg_strip_size(p.nb) * sizeof(float); }
 
 }  // namespace natsl
 
@@ -335,10 +349,14 @@ extern "C" int natsl_wgrad(const natsl_wgrad_seg* segs, int n_seg, const void* x
   if (workspace_bytes < wgrad_bytes(p)) return fail(NATSL_ERR_WORKSPACE, "%s: workspace too small", what);
   p.part = reinterpret_cast<float*>(workspace);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  static std::atomic<unsigned long long> reserved{0};
-  if ((rc = reserve_lds(reinterpret_cast<const void*>(wgrad_kernel), reserved, WG_STAGES * WG_STAGE, what)) != NATSL_OK) return rc;
-  hipLaunchKernelGGL(wgrad_kernel, dim3((unsigned)(cdiv(p.units, 8) * 8)), dim3(256), WG_STAGES * WG_STAGE, s, p);
-  if ((rc = check_launch(what)) != NATSL_OK) return rc;
-  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((unsigned)(p.tiles * 16)), dim3(256), 0, s, p);
-  return check_launch(what);
+  auto launch = [&](auto nb) -> int {
+    constexpr int NB = decltype(nb)::value;
+    static std::atomic<unsigned long long> reserved{0};
+    if (const int r = reserve_lds(reinterpret_cast<const void*>(wgrad_kernel<NB>), reserved, WG_STAGES * WG_STAGE, what)) return r;
+    hipLaunchKernelGGL(wgrad_kernel<NB>, dim3((unsigned)(cdiv(p.units, 8) * 8)), dim3(256), WG_STAGES * WG_STAGE, s, p);
+    if (const int r = check_launch(what)) return r;
+    hipLaunchKernelGGL(wgrad_reduce_kernel<NB>, dim3((unsigned)(p.tiles * 4 * NB)), dim3(256), 0, s, p);
+    return check_launch(what);
+  };
+  return p.nb == 4 ? launch(std::integral_constant<int, 4>{}) : launch(std::integral_constant<int, 3>{});
 }

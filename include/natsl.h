@@ -557,7 +557,8 @@ typedef struct natsl_cast { const void* src; void* dst; int64_t n; } natsl_cast;
 typedef struct natsl_mixed {
   int32_t is_delta, B, T, H, HN, K, V, TN, block, flags;
   int32_t T_attn, TN_attn, HQ, HKV, KA, VA, same_block_visible, types_dtype;
-  int32_t n_seqs, total_chunks, total_qtiles, n_cast_in, n_cast_out, reserved;
+  int32_t n_seqs, total_chunks, total_qtiles, n_cast_in, n_cast_out;
+  int32_t private_tables;   /* block_indices and n_blocks are room for this call only: nobody reads them afterwards, they need not be written */
   float scale_attn, scale_linear;
   const void *q_attn, *k_attn, *v_attn, *types_attn;
   void* o_attn;

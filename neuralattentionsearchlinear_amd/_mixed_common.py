@@ -19,7 +19,7 @@ class _Cast(ctypes.Structure):
 
 _MAX_CASTS = 8
 _INTS = ("is_delta", "B", "T", "H", "HN", "K", "V", "TN", "block", "flags", "T_attn", "TN_attn", "HQ", "HKV", "KA", "VA", "same_block_visible",
-         "types_dtype", "n_seqs", "total_chunks", "total_qtiles", "n_cast_in", "n_cast_out", "reserved")
+         "types_dtype", "n_seqs", "total_chunks", "total_qtiles", "n_cast_in", "n_cast_out", "private_tables")
 _POINTERS = ("q_attn", "k_attn", "v_attn", "types_attn", "o_attn", "lse", "block_indices", "n_blocks", "q", "k", "v", "g", "beta", "h0", "o", "ht",
              "h_block_start", "g_block_sum", "chunk_states", "chunk_v_new", "types", "workspace")
 
@@ -374,7 +374,7 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
     m.is_delta, m.B, m.T, m.H, m.HN, m.K, m.V, m.TN, m.block = int(kind == 'gdn'), B, T, H, HN, K, V, TN, nats_block_size
     m.flags = (_capi.DECAY_NON_LINEAR if decay_non_linear else 0) | (_capi.QK_L2NORM if qk_l2norm else 0) | (_capi.INTRA_CHUNK if lin_intra else 0)
     m.T_attn, m.TN_attn, m.HQ, m.HKV, m.KA, m.VA = T_attn, types_attn.shape[1], HQ, HKV, KA, VA
-    m.same_block_visible, m.types_dtype = int(attn_same_block), _capi.dtype_code(types.dtype)
+    m.same_block_visible, m.types_dtype, m.private_tables = int(attn_same_block), _capi.dtype_code(types.dtype), int(not return_aux)
     m.scale_attn, m.scale_linear = scale_attn, scale_lattn
     m.g, m.types, m.types_attn, m.workspace_bytes = g.data_ptr(), types.data_ptr(), types_attn.data_ptr(), ws_bytes
     for name, t in (("h0", h0), ("ht", ht), ("h_block_start", hs), ("g_block_sum", gs), ("chunk_states", sc), ("chunk_v_new", vn)):

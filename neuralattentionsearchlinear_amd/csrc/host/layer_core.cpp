@@ -192,6 +192,7 @@ void mixed(const Call& c, const Front& f, const bool keep, const bool keep_state
     const int64_t idx = up(c.B * nb * l.HN * 8, 256), nblk = up(c.B * l.HN * 8, 256), lse = up(c.rows * l.HQ * 4, 256);
     scratch = c.bytes((size_t)(idx + nblk + lse) + ws);
     char* p = static_cast<char*>(scratch.data_ptr());
+    a.private_tables = 1;
     a.block_indices = reinterpret_cast<int32_t*>(p); a.n_blocks = reinterpret_cast<int32_t*>(p + idx); a.lse = reinterpret_cast<float*>(p + idx + nblk);
     a.workspace = p + idx + nblk + lse;
   }

@@ -163,6 +163,7 @@ PyObject* natsl_mixed_plain(PyObject*, PyObject* const* a, Py_ssize_t n) {
     m.n_cast_out = 2;
   }
   m.is_delta = delta;
+  m.private_tables = 1;
   m.B = (int32_t)B; m.T = m.T_attn = (int32_t)Tn; m.H = (int32_t)H; m.HN = (int32_t)HN; m.K = (int32_t)K; m.V = (int32_t)V; m.TN = m.TN_attn = (int32_t)TN;
   m.block = (int32_t)block; m.HQ = (int32_t)HQ; m.HKV = (int32_t)HKV; m.KA = (int32_t)KA; m.VA = (int32_t)VA;
   m.flags = (options & 2 ? NATSL_DECAY_NON_LINEAR : 0) | (options & 4 ? NATSL_QK_L2NORM : 0) | (options & 8 ? NATSL_INTRA_CHUNK : 0);

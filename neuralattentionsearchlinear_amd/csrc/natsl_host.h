@@ -59,6 +59,10 @@ int softmax_fwd(const void* q, const void* k, const void* v, void* o, float* lse
                 int block, float scale, int same_block_visible, int dtype, const natsl_seq_row* seqs, int n_seqs, int total_units,
                 natsl_stream_t stream, SoftmaxUse use, unsigned* queue);
 
+// Whether the kernel that such a call takes finds a tile's blocks in the types as well as in a routing table, which may be null then: the kernels of
+// one workgroup a tile, unpacked, up to 256 selector blocks.
+bool softmax_reads_types(int B, int T, int HQ, int HKV, int TN, int block, const natsl_seq_row* seqs, SoftmaxUse use);
+
 inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 }  // namespace natsl

@@ -121,12 +121,14 @@ using namespace natsl;
 static int mixed_phases(const natsl_mixed* m, const int phases, natsl_stream_t stream, natsl_stream_t attn_stream, bool& forked, const char* what) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream), side = reinterpret_cast<hipStream_t>(attn_stream);
   const bool fork = side != s;
+  // (a table that nobody reads afterwards is not made where the softmax kernel does not need it)
+  const bool no_tables = m->private_tables && softmax_reads_types(m->B, m->T_attn, m->HQ, m->HKV, m->TN_attn, m->block, m->seqs, SOFTMAX_OPERATOR);
   int rc = NATSL_OK;
   if ((phases & NATSL_MIXED_CONVERT) && (rc = cast_all<true>(m->cast_in, m->n_cast_in, s, what)) != NATSL_OK) return rc;
   if (phases & NATSL_MIXED_ROUTE) {
     if (fork && (rc = order_streams(s, side, what)) != NATSL_OK) return rc;
     forked = fork;
-    rc = natsl_route(m->types_attn, m->types_dtype, m->B, m->TN_attn, m->HN, m->T_attn, m->block, m->block_indices, m->n_blocks, nullptr, nullptr,
+    rc = no_tables ? NATSL_OK : natsl_route(m->types_attn, m->types_dtype, m->B, m->TN_attn, m->HN, m->T_attn, m->block, m->block_indices, m->n_blocks, nullptr, nullptr,
                      nullptr, nullptr, m->seqs, m->n_seqs, 0, attn_stream);
     if (rc != NATSL_OK) return rc;
   }
@@ -136,8 +138,8 @@ static int mixed_phases(const natsl_mixed* m, const int phases, natsl_stream_t s
     const size_t at = natsl_linear_workspace_bytes(chunks, m->H);
     unsigned* queue = nullptr;
     if (m->workspace && m->workspace_bytes >= at + SOFTMAX_QUEUE_BYTES) queue = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(m->workspace) + at);
-    return softmax_fwd(m->q_attn, m->k_attn, m->v_attn, m->o_attn, m->lse, m->types_attn, m->types_dtype, m->block_indices, m->n_blocks, m->B,
-                       m->T_attn, m->HQ, m->HKV, m->HN, m->KA, m->VA, m->TN_attn, m->block, m->scale_attn, m->same_block_visible, NATSL_BF16,
+    return softmax_fwd(m->q_attn, m->k_attn, m->v_attn, m->o_attn, m->lse, m->types_attn, m->types_dtype, no_tables ? nullptr : m->block_indices,
+                       no_tables ? nullptr : m->n_blocks, m->B, m->T_attn, m->HQ, m->HKV, m->HN, m->KA, m->VA, m->TN_attn, m->block, m->scale_attn, m->same_block_visible, NATSL_BF16,
                        m->seqs, m->n_seqs, m->total_qtiles, attn_stream, SOFTMAX_OPERATOR, queue);
   };
   // Side by side, the scan comes first and the softmax kernel right behind the prep kernel: its workgroups take a CU each for as long

@@ -408,6 +408,27 @@ NATSL_DEVICE void softmax_phase(f32x16& s0, f32x16& s1, f32x16 (&acc)[DV / 32], 
   }
 }
 
+// The attention blocks among the first n (at most TYPES_AHEAD), in order, into `list`, by one wave; -> how many.  What the routing launch would
+// have written is 2.6 - 3.5 us of a small call; the types are as many loads as its table.
+constexpr int TYPES_AHEAD = 256;
+NATSL_DEVICE int list_from_types(const SoftmaxParams& p, const size_t first, const int hn, const int n, int* list) {
+  const int lane = threadIdx.x & 63;
+  bool is[TYPES_AHEAD / 64];
+#pragma unroll
+  for (int i = 0; i < TYPES_AHEAD / 64; ++i) {
+    const int j = 64 * i + lane;
+    is[i] = type_is_one(p.types, p.types_dtype, ((first + (size_t)min(j, max(n - 1, 0))) * p.HN + hn) * 2) && j < n;
+  }
+  int count = 0;
+#pragma unroll
+  for (int i = 0; i < TYPES_AHEAD / 64; ++i) {
+    const unsigned long long those = __ballot(is[i]);
+    if (is[i]) list[count + __popcll(those & ((1ull << lane) - 1ull))] = 64 * i + lane;
+    count += __popcll(those);
+  }
+  return count;
+}
+
 // NWAVES waves of 32 queries: the workgroup owns QTILE = 32*NWAVES queries.  OWN: see below (8 waves and selector blocks of 64 keys).
 template <int DK, int DV, int NWAVES, bool OWN>
 __global__ __launch_bounds__(64 * NWAVES, NWAVES == 4 ? 2 : 1) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -695,13 +716,17 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
       __shared__ int wave_count[NWAVES];
       {
         const int jmax = min(dblk, p.TN);
-        const int n_attn = *n_attn_p;
         int cnt = 0;
-        for (int j = tid; j < jmax; j += NTHREADS) {
-          const int e = list[j * list_stride];
-          const bool ok = j < n_attn && (e + 1) * Bs <= dstart;
-          cnt += __popcll(__ballot(ok));
-          if (ok && j < MAX_LDS_LIST) lds_list[j] = e;
+        if (p.idx == nullptr) {
+          if (wave == 0) cnt = list_from_types(p, (size_t)bos_nats, hn, jmax, lds_list);
+        } else {
+          const int n_attn = *n_attn_p;
+          for (int j = tid; j < jmax; j += NTHREADS) {
+            const int e = list[j * list_stride];
+            const bool ok = j < n_attn && (e + 1) * Bs <= dstart;
+            cnt += __popcll(__ballot(ok));
+            if (ok && j < MAX_LDS_LIST) lds_list[j] = e;
+          }
         }
         if (lane == 0) wave_count[wave] = cnt;
       }
@@ -904,16 +929,23 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
       // attention blocks that end at or before dstart: ids into LDS, count.  The list is sorted and
       // holds distinct block ids, so entry j >= j: only the first dstart/Bs entries can qualify.
       const int jmax = min(dblk, p.TN);
-      const int n_attn = *n_attn_p;
-      int cnt = 0;
-      for (int j = tid; j < jmax; j += NTHREADS) {
-        const int e = list[j * list_stride];
-        if (j < n_attn && (e + 1) * Bs <= dstart) {
-          ++cnt;
-          if (j < MAX_LDS_LIST) lds_list[j] = e;
+      if (p.idx == nullptr) {
+        if (wave == 0) {
+          const int cnt = list_from_types(p, (size_t)bos_nats, hn, jmax, lds_list);
+          if (lane == 0) lds_count = cnt;
         }
+      } else {
+        const int n_attn = *n_attn_p;
+        int cnt = 0;
+        for (int j = tid; j < jmax; j += NTHREADS) {
+          const int e = list[j * list_stride];
+          if (j < n_attn && (e + 1) * Bs <= dstart) {
+            ++cnt;
+            if (j < MAX_LDS_LIST) lds_list[j] = e;
+          }
+        }
+        if (cnt) atomicAdd(&lds_count, cnt);
       }
-      if (cnt) atomicAdd(&lds_count, cnt);
     }
     // types of the blocks the chunks from dstart on fall into, as a bit mask (bit i = block dstart/Bs + i)
     unsigned long long diag_attn;
@@ -1724,11 +1756,18 @@ static int softmax_variant(int B, int T, int HQ, int HKV, int block, bool packed
 
 static_assert(SOFTMAX_QUEUE_BYTES == STREAM_SLOT_WORDS * sizeof(unsigned), "the counters of one launch");
 
+bool softmax_reads_types(int B, int T, int HQ, int HKV, int TN, int block, const natsl_seq_row* seqs, SoftmaxUse use) {
+  if (use != SOFTMAX_OPERATOR || seqs || TN > TYPES_AHEAD || B <= 0 || T <= 0 || HQ <= 0 || HKV <= 0 || block <= 0) return false;
+  const StreamDevice* sd = nullptr;
+  int rc;
+  return softmax_variant(B, T, HQ, HKV, block, false, use, 0, &sd, &rc) >= 0 && !sd;
+}
+
 int softmax_fwd(const void* q, const void* k, const void* v, void* o, float* lse, const void* types, int types_dtype,
                 const int32_t* nats_block_indices, const int32_t* n_nats_blocks, int B, int T, int HQ, int HKV, int HN, int K,
                 int V, int TN, int block, float scale, int same_block_visible, int dtype, const natsl_seq_row* seqs,
                 int n_seqs, int total_units, natsl_stream_t stream, SoftmaxUse use, unsigned* queue) {
-  if (!q || !k || !v || !o || !lse || !types || !nats_block_indices || !n_nats_blocks)
+  if (!q || !k || !v || !o || !lse || !types || !nats_block_indices != !n_nats_blocks || (!nats_block_indices && !softmax_reads_types(B, T, HQ, HKV, TN, block, seqs, use)))
     return fail(NATSL_ERR_INVALID, "softmax: null pointer argument");
   if (dtype != NATSL_BF16) return fail(NATSL_ERR_UNSUPPORTED, "softmax: only bf16 tensors are supported (got dtype %d)", dtype);
   if (types_dtype != NATSL_BF16 && types_dtype != NATSL_F32) return fail(NATSL_ERR_UNSUPPORTED, "softmax: block types must be f32 or bf16");

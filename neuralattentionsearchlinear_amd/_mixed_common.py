@@ -45,8 +45,9 @@ TIMING_HOOK = None
 # walks the chunks one by one with a few large workgroups, so the softmax kernel fills the CUs it leaves; both take most of a CU's
 # LDS (127 KiB / 159 KiB) and never share one, so a scan that fills the chip by itself gains nothing (B8 T8192 H16: 1042
 # and 1045 us); B4 T8192 H8 400 -> 326, Mamba B4 T8192 H32 764 -> 699, four packed documents of 65536 tokens 2274 -> 2162 us.  Ordering two
-# streams costs a call about 40 us (36 us one after the other, 78 us side by side at T 256), which the overlap repays from a chain of
-# 2048 tokens at K = 128 on (4096 at K = 64): 87 -> 78 us at B1 T2048 H6, 154 -> 111 us at T 4096, but 56 -> 81 us at T 1024.
+# streams costs a call about 50 us (22 us one after the other, where the softmax tiles share a launch with the prep kernel, 72 us side by side at T 256),
+# which the overlap repays from a chain of 2048 tokens at K = 128 on (4096 at K = 64): at B1 H4 T2000 84 -> 74 us with half attention and 66 -> 72 with
+# a tenth, 154 -> 111 us at H6 T 4096, but 48 -> 72 us at T 1024.
 CONCURRENT_BRANCHES = None
 _SIDE_BY_SIDE_TOKENS_X_K = 2048 * 128
 _SCAN_COLUMNS_PER_WG = 64           # state columns of the scans' widest workgroup (csrc/natsl_linear.hip, natsl_linear_bwd.hip)

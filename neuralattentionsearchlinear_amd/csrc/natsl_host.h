@@ -44,11 +44,19 @@ struct BesideScan {
   int (*ready)(hipStream_t, hipStream_t, const char*);
   hipStream_t other;
 };
-// The two chunked linear branches behind their C entries (natsl_linear.hip); beside: null, or what the scan shares the chip with.
+// The softmax branch in the launch of the prep kernel, or before it: softmax(call, p, wgs) enqueues it, together with the prep's `wgs` workgroups
+// unless p is null.
+struct LinearParams;
+struct PrepWith {
+  int (*softmax)(void* call, const LinearParams* p, unsigned wgs);
+  void* call;
+};
+// The two chunked linear branches behind their C entries (natsl_linear.hip); beside: null, or what the scan shares the chip with; with: null, or
+// what goes with the prep kernel.
 int linear_fwd(bool delta, const void* q, const void* k, const void* v, const float* g, const void* beta, const float* h0, void* o, float* ht,
                float* hs, float* gs, void* chunk_states, void* chunk_v_new, const void* types, int types_dtype, int B, int T, int H, int HN, int K,
                int V, int TN, int block, float scale, int flags, void* workspace, size_t workspace_bytes, int dtype, const natsl_seq_row* seqs,
-               int n_seqs, int total_units, natsl_stream_t stream, const BesideScan* beside);
+               int n_seqs, int total_units, natsl_stream_t stream, const BesideScan* beside, const PrepWith* with = nullptr);
 
 // The softmax branch behind its C entries (natsl_softmax.hip); queue: SOFTMAX_QUEUE_BYTES of this call's own for the persistent kernel's
 // work queues, or null (see launch_softmax_stream).
@@ -57,7 +65,10 @@ enum SoftmaxUse { SOFTMAX_PER_TILE, SOFTMAX_ENTRY, SOFTMAX_OPERATOR };   // who 
 int softmax_fwd(const void* q, const void* k, const void* v, void* o, float* lse, const void* types, int types_dtype,
                 const int32_t* nats_block_indices, const int32_t* n_nats_blocks, int B, int T, int HQ, int HKV, int HN, int K, int V, int TN,
                 int block, float scale, int same_block_visible, int dtype, const natsl_seq_row* seqs, int n_seqs, int total_units,
-                natsl_stream_t stream, SoftmaxUse use, unsigned* queue);
+                natsl_stream_t stream, SoftmaxUse use, unsigned* queue, const LinearParams* prep = nullptr, unsigned prep_wgs = 0);
+
+// Whether softmax_fwd can take the linear branch's prep into its launch (`prep`, `prep_wgs`: see PrepWith): see softmax_prep_kernel.
+bool softmax_takes_prep(int B, int T, int HQ, int HKV, int KA, int VA, int block, const natsl_seq_row* seqs, bool delta, int K, long long prep_wgs);
 
 // Whether the kernel that such a call takes finds a tile's blocks in the types as well as in a routing table, which may be null then: the kernels of
 // one workgroup a tile, unpacked, up to 256 selector blocks.

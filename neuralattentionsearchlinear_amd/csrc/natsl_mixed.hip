@@ -5,8 +5,8 @@
 #include <cstring>
 #include <mutex>
 
-#include "natsl_device.h"
 #include "natsl_host.h"
+#include "natsl_linear_prep.h"
 
 namespace natsl {
 
@@ -132,7 +132,7 @@ static int mixed_phases(const natsl_mixed* m, const int phases, natsl_stream_t s
                      nullptr, nullptr, m->seqs, m->n_seqs, 0, attn_stream);
     if (rc != NATSL_OK) return rc;
   }
-  auto softmax = [&]() {
+  auto softmax = [&](const LinearParams* prep, unsigned prep_wgs) {
     // the work queues lie behind the linear branch's part of the workspace
     const long long chunks = m->seqs ? m->total_chunks : (long long)m->B * cdiv(m->T, 64);
     const size_t at = natsl_linear_workspace_bytes(chunks, m->H);
@@ -140,22 +140,27 @@ static int mixed_phases(const natsl_mixed* m, const int phases, natsl_stream_t s
     if (m->workspace && m->workspace_bytes >= at + SOFTMAX_QUEUE_BYTES) queue = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(m->workspace) + at);
     return softmax_fwd(m->q_attn, m->k_attn, m->v_attn, m->o_attn, m->lse, m->types_attn, m->types_dtype, no_tables ? nullptr : m->block_indices,
                        no_tables ? nullptr : m->n_blocks, m->B, m->T_attn, m->HQ, m->HKV, m->HN, m->KA, m->VA, m->TN_attn, m->block, m->scale_attn, m->same_block_visible, NATSL_BF16,
-                       m->seqs, m->n_seqs, m->total_qtiles, attn_stream, SOFTMAX_OPERATOR, queue);
+                       m->seqs, m->n_seqs, m->total_qtiles, attn_stream, SOFTMAX_OPERATOR, queue, prep, prep_wgs);
   };
   // Side by side, the scan comes first and the softmax kernel right behind the prep kernel: its workgroups take a CU each for as long
   // as there are tiles, so it has to find the scan's in place and fill the CUs they leave (the other way round the scan waits
   // for it).
   const bool both = fork && (phases & NATSL_MIXED_SOFTMAX) && (phases & NATSL_MIXED_LINEAR);
-  if ((phases & NATSL_MIXED_SOFTMAX) && !both && (rc = softmax()) != NATSL_OK) return rc;
+  // One after the other: the softmax tiles and the prep in one launch where the tiles are the small ones.
+  const bool joined = !fork && (phases & NATSL_MIXED_SOFTMAX) && (phases & NATSL_MIXED_LINEAR) && !(m->flags & NATSL_STATES_ONLY) && m->B > 0 && m->T > 0 && m->H > 0 &&
+                      softmax_takes_prep(m->B, m->T_attn, m->HQ, m->HKV, m->KA, m->VA, m->block, m->seqs, m->is_delta != 0, m->K,
+                                         linear_prep_wgs(m->is_delta != 0, (long long)m->B * cdiv(m->T, 64), m->H));
+  if ((phases & NATSL_MIXED_SOFTMAX) && !both && !joined && (rc = softmax(nullptr, 0)) != NATSL_OK) return rc;
   if (phases & NATSL_MIXED_LINEAR) {
     const BesideScan beside{order_streams, side};
+    const PrepWith with{[](void* call, const LinearParams* p, unsigned wgs) { return (*static_cast<decltype(softmax)*>(call))(p, wgs); }, &softmax};
     rc = linear_fwd(m->is_delta != 0, m->q, m->k, m->v, m->g, m->is_delta ? m->beta : nullptr, m->h0, m->o, m->ht, m->h_block_start, m->g_block_sum,
                     m->chunk_states, m->is_delta ? m->chunk_v_new : nullptr, m->types, m->types_dtype, m->B, m->T, m->H, m->HN, m->K, m->V, m->TN,
                     m->block, m->scale_linear, m->is_delta ? m->flags : m->flags & ~NATSL_QK_L2NORM, m->workspace, m->workspace_bytes, NATSL_BF16,
-                    m->seqs, m->n_seqs, m->total_chunks, stream, both ? &beside : nullptr);
+                    m->seqs, m->n_seqs, m->total_chunks, stream, both ? &beside : nullptr, joined ? &with : nullptr);
     if (rc != NATSL_OK) return rc;
   }
-  if (both && (rc = softmax()) != NATSL_OK) return rc;
+  if (both && (rc = softmax(nullptr, 0)) != NATSL_OK) return rc;
   if (phases & NATSL_MIXED_JOIN) {
     if (fork && (rc = order_streams(side, s, what)) != NATSL_OK) return rc;
     forked = false;

@@ -10,8 +10,8 @@
 // staged through registers, V transposed on the way, double buffered, one chunk as one pipelined instruction stream per
 // wave) and, for full tiles on 8 waves, the three-phase schedule further down (K and V by LDS-DMA as they lie in memory, V
 // transposed by the operand reads, the two waves of a SIMD half a chunk apart).
-#include "natsl_device.h"
 #include "natsl_host.h"
+#include "natsl_linear_prep.h"
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -431,8 +431,7 @@ NATSL_DEVICE int list_from_types(const SoftmaxParams& p, const size_t first, con
 
 // NWAVES waves of 32 queries: the workgroup owns QTILE = 32*NWAVES queries.  OWN: see below (8 waves and selector blocks of 64 keys).
 template <int DK, int DV, int NWAVES, bool OWN>
-__global__ __launch_bounds__(64 * NWAVES, NWAVES == 4 ? 2 : 1) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
+__device__ __attribute__((always_inline)) inline void softmax_tile(const SoftmaxParams& p, const unsigned wg) {
   constexpr int NTHREADS = 64 * NWAVES, QW = 32, QTILE = QW * NWAVES;  // QW = queries per wave
   constexpr int KP = DK + 8, VP = DV + 8;  // row pitch (elements) of the K tile and of the epilogue tile
   constexpr int TP = VT_PITCH;
@@ -455,7 +454,7 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
     // (unsigned arithmetic throughout: a signed division by a run-time value costs a third more scalar instructions,
     // and this preamble is what every tile starts with)
     const unsigned n_pairs = (unsigned)(p.B * p.HQ);
-    const unsigned xcd = blockIdx.x & 7u, j = blockIdx.x >> 3;
+    const unsigned xcd = wg & 7u, j = wg >> 3;
     const unsigned nq_tiles = ((unsigned)p.T + QTILE - 1) / QTILE;
     const unsigned jq = j / nq_tiles;
     const unsigned pair = jq * 8 + xcd;
@@ -468,8 +467,8 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
     bos_nats = n * p.TN;
   } else {
     const int tiles_per_256 = QTILE_TABLE / QTILE;
-    const int gt = p.total_tiles * tiles_per_256 - 1 - (int)blockIdx.x / p.HQ;
-    hq = (int)blockIdx.x % p.HQ;
+    const int gt = p.total_tiles * tiles_per_256 - 1 - (int)wg / p.HQ;
+    hq = (int)wg % p.HQ;
     n = 0;
     for (int i = 1; i < p.n_seqs; ++i)
       if (p.seqs[i].qtile_off * tiles_per_256 <= gt) n = i;
@@ -1057,6 +1056,33 @@ void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
       const u32x4 w = *reinterpret_cast<const u32x4*>(Os + row * VP + seg * 8);
       *reinterpret_cast<u32x4*>(p.o + ((size_t)(bos + qi) * p.HQ + hq) * DV + seg * 8) = w;
     }
+  }
+}
+
+template <int DK, int DV, int NWAVES, bool OWN>
+__global__ __launch_bounds__(64 * NWAVES, NWAVES == 4 ? 2 : 1) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void softmax_sparse_fwd_kernel(const SoftmaxParams p) {
+  softmax_tile<DK, DV, NWAVES, OWN>(p, blockIdx.x);
+}
+
+// A small call's tiles of 128 queries and, in the workgroups behind them, the linear branch's prep: neither reads what the other writes, and each by itself
+// leaves most of the chip idle for as long as its one or two rounds take (fp32 B1 T256 H2 64/64: 9.5 us of 16 workgroups, then 5.7 us of 8).  Bound by the
+// chain of a tile's chunks, which the prep hides behind.  A workgroup is one or the other, so both lie in the same LDS and two share a CU; with the
+// prep's arrays behind a tile's, 128/128 and 64/128 had one: B8 T512 H15 49.0 us as two launches, 57.8 so, 45.2 in the same.
+// LK: the prep's key width, 0 for the Mamba form's scale vectors.
+// Operators' forward, two launches / one, us: GDN B1 T256 H2 64/64 21.4 / 15.6, B1 T1024 H8 128/128 48.5 / 42.4, B4 T1000 H15 64/128 67.3 / 56.1;
+// Mamba B1 T256 H2 18.1 / 15.8, B4 T1000 H15 128/128 49.2 / 46.3.
+template <int DK, int DV, int LK>
+__global__ __launch_bounds__(256, 2) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void softmax_prep_kernel(const SoftmaxParams p, const LinearParams l, const unsigned tiles) {
+  if (blockIdx.x < tiles) {
+    softmax_tile<DK, DV, 4, false>(p, blockIdx.x);
+  } else if constexpr (LK != 0) {
+    extern __shared__ __align__(16) unsigned char smem[];   // (a workgroup is one or the other: the prep's arrays lie where a tile's would)
+    float* rows = reinterpret_cast<float*>(smem + PREP_REGION<LK, true, false>);
+    linear_prep<LK, true, false>(l, blockIdx.x - tiles, smem, rows, rows + C, rows + 2 * C, rows + 3 * C);
+  } else {
+    mamba_scale(l, blockIdx.x - tiles);
   }
 }
 
@@ -1652,6 +1678,29 @@ static int launch_softmax(const SoftmaxParams& p, hipStream_t stream) {
   return check_launch("natsl_softmax_sparse_fwd");
 }
 
+// What a prep may come with: the key widths that operators and the published geometries join to these heads.  (64 with value heads of 64 or 128, 128 with
+// either, 192 with 64/128: the others keep two launches, each would be a kernel of its own.)
+constexpr bool takes_prep(const int dk, const int dv, const int lk) { return lk == 0 || lk == dk || (lk == 192 && dk == 64 && dv == 128); }
+template <int DK, int DV, int LK>
+static int launch_softmax_prep(const SoftmaxParams& p, const LinearParams& l, const unsigned prep_wgs, hipStream_t stream) {
+  constexpr int KP = DK + 8, VP = DV + 8, QTILE = 128;
+  constexpr size_t stages = (size_t)2 * (64 * KP + DV * VT_PITCH) * sizeof(bf16_t), epi = (size_t)QTILE * VP * sizeof(bf16_t), tile = epi > stages ? epi : stages;
+  constexpr size_t prep = LK == 0 ? 0 : PREP_REGION<LK == 0 ? 64 : LK, true, false> + 4 * C * sizeof(float), lds = prep > tile ? prep : tile;
+  auto kern = softmax_prep_kernel<DK, DV, LK>;
+  static std::atomic<unsigned long long> reserved{0};
+  if (const int rc = reserve_lds(reinterpret_cast<const void*>(kern), reserved, lds, "softmax")) return rc;
+  const unsigned tiles = 8u * (((unsigned)(p.B * p.HQ) + 7u) / 8u) * (((unsigned)p.T + QTILE - 1) / QTILE);
+  hipLaunchKernelGGL(kern, dim3(tiles + prep_wgs), dim3(256), lds, stream, p, l, tiles);
+  return check_launch("natsl_softmax_sparse_fwd");
+}
+template <int DK, int DV>
+static int launch_softmax_with(const SoftmaxParams& p, const LinearParams& l, const unsigned prep_wgs, hipStream_t stream) {
+  if (!l.beta) return launch_softmax_prep<DK, DV, 0>(p, l, prep_wgs, stream);
+  if (l.K == DK) return launch_softmax_prep<DK, DV, DK>(p, l, prep_wgs, stream);
+  if constexpr (takes_prep(DK, DV, 192)) if (l.K == 192) return launch_softmax_prep<DK, DV, 192>(p, l, prep_wgs, stream);
+  return fail(NATSL_ERR_UNSUPPORTED, "softmax: no launch with a prep of K=%d", l.K);
+}
+
 // Ticket counters of the persistent kernel.  They are zeroed on the launch's stream by a fill kernel right before it (a kernel, not
 // hipMemsetAsync, so that both can be captured into a HIP graph and replayed); nothing is left to set back afterwards, so a launch
 // that was cut short cannot poison a later one.  Three homes:
@@ -1763,10 +1812,21 @@ bool softmax_reads_types(int B, int T, int HQ, int HKV, int TN, int block, const
   return softmax_variant(B, T, HQ, HKV, block, false, use, 0, &sd, &rc) >= 0 && !sd;
 }
 
+// Wherever tiles of 128 queries are taken and the branches follow each other: 86 sizes of one to 1472 workgroups in all, 10 to 80 % attention, gain 2 to 37 %.
+// Those have two prep workgroups a tile at most, which equal heads come to; with more (many linear heads on few attention heads) the prep, here two
+// workgroups a CU for its own kernel's four to six, would be the longer part.
+bool softmax_takes_prep(int B, int T, int HQ, int HKV, int KA, int VA, int block, const natsl_seq_row* seqs, bool delta, int K, long long prep_wgs) {
+  if (seqs || B <= 0 || T <= 0 || HQ <= 0 || HKV <= 0 || block <= 0 || prep_wgs <= 0 || !takes_prep(KA, VA, delta ? K : 0)) return false;
+  if (prep_wgs > 2 * 8 * (((long long)B * HQ + 7) / 8) * (((long long)T + 127) / 128)) return false;
+  const StreamDevice* sd = nullptr;
+  int rc;
+  return softmax_variant(B, T, HQ, HKV, block, false, SOFTMAX_OPERATOR, 0, &sd, &rc) == NATSL_SOFTMAX_TILE_128;
+}
+
 int softmax_fwd(const void* q, const void* k, const void* v, void* o, float* lse, const void* types, int types_dtype,
                 const int32_t* nats_block_indices, const int32_t* n_nats_blocks, int B, int T, int HQ, int HKV, int HN, int K,
                 int V, int TN, int block, float scale, int same_block_visible, int dtype, const natsl_seq_row* seqs,
-                int n_seqs, int total_units, natsl_stream_t stream, SoftmaxUse use, unsigned* queue) {
+                int n_seqs, int total_units, natsl_stream_t stream, SoftmaxUse use, unsigned* queue, const LinearParams* prep, unsigned prep_wgs) {
   if (!q || !k || !v || !o || !lse || !types || !nats_block_indices != !n_nats_blocks || (!nats_block_indices && !softmax_reads_types(B, T, HQ, HKV, TN, block, seqs, use)))
     return fail(NATSL_ERR_INVALID, "softmax: null pointer argument");
   if (dtype != NATSL_BF16) return fail(NATSL_ERR_UNSUPPORTED, "softmax: only bf16 tensors are supported (got dtype %d)", dtype);
@@ -1800,6 +1860,7 @@ int softmax_fwd(const void* q, const void* k, const void* v, void* o, float* lse
   if (K == KK && V == VV) {                                           \
     if (sd && !seqs && T % 256 == 0) return launch_softmax_stream<KK, VV, false, false>(p, sd, queue, s); \
     if (sd) return queue ? launch_softmax_stream<KK, VV, true, false>(p, sd, queue, s) : launch_softmax_stream<KK, VV, true, true>(p, sd, nullptr, s); \
+    if (prep && !seqs && p.variant != 8) return launch_softmax_with<KK, VV>(p, *prep, prep_wgs, s); \
     if (p.variant != 8) return launch_softmax<KK, VV, 4>(p, s);       \
     return block == 64 ? launch_softmax<KK, VV, 8, true>(p, s) : launch_softmax<KK, VV, 8>(p, s); \
   }

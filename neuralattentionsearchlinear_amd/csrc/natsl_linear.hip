@@ -46,8 +46,11 @@
 
 namespace natsl {
 
+// K = 192: 52 KB of LDS let three workgroups on a CU.  The compiler, asked for four of them only, took 172 registers a lane (32 of them to move
+// others out of the way), which leave two; asked for three, 138.  1536 chunk-heads 28.0 -> 23.9 us, 3072 52 -> 44, 6240 112 -> 85.
 template <int DK, bool DELTA, bool PF>
-__global__ __launch_bounds__(256, 4) void linear_prep_kernel(const LinearParams p) {
+__global__ __launch_bounds__(256, DK == 192 ? 3 : 4) __attribute__((amdgpu_waves_per_eu(DK == 192 ? 3 : 4)))
+void linear_prep_kernel(const LinearParams p) {
   __shared__ __align__(16) unsigned char region0[PREP_REGION<DK, DELTA, PF>];
   __shared__ __align__(16) float gam[C], rq[C], rk[C], bet[C];
   linear_prep<DK, DELTA, PF>(p, blockIdx.x, region0, gam, rq, rk, bet);

@@ -87,17 +87,17 @@ def _scan_leaves_cus(dev, n_seqs: int, H: int, V: int) -> bool:
 
 
 def _layer_runs_side_by_side(dev, B: int, T: int, how, gradients: bool) -> bool:
-    """_run_side_by_side for a layer's native calls.  Ordering the streams costs the host 90 us of a forward and 150 us of a training step, which then are
-    330 and 740 us of host time: two streams pay where one would take longer than that.  What one takes follows the products' work (tokens
-    times weights) and the length of the chains: 240 us + 12.3 ns a million + 0.122 us a token of a sequence for a training step.  One stream's
-    time over two streams', us: training 340M 4 x 1024 672 / 760, 6 x 1024 863 / 805, 1 x 2048 602 / 712, 1 x 3000 765 / 742, 1 x 4096 990 / 781; 760M 1 x 1536
-    681 / 762, 2 x 1536 948 / 899; 16 heads of 128/64 2 x 1536 702 / 738, 3 x 1536 866 / 804.  A forward from chains of 2048 tokens at K = 128 on, as the
-    operators: 340M 3 x 2048 311 / 339, 4 x 2048 363 / 360, 1 x 3000 265 / 307, 2 x 3000 336 / 322; 760M 1 x 2048 296 / 329, 1 x 3000 379 / 350; shorter
-    ones are 0.95 to 1.06 either way."""
+    """_run_side_by_side for a layer's native calls.  Ordering the streams costs the host 90 us of a forward and 100 to 150 us of a training step: two streams
+    pay where one would take longer than the host then does.  What one takes follows the products' work (tokens times weights) and the length of the chains.
+    The host's share of a training step is one of two figures, which a process keeps: 400 and 590 us with one stream (340M 1 x 832), 505 to 600 and 700 to
+    720 with two; two processes of three have the smaller one.  One stream's time over two streams', us, mean of six processes: 340M 1 x 1500 561 / 590,
+    1 x 2048 576 / 552, 4 x 1024 637 / 633, 1 x 3000 755 / 626; 760M 1 x 1200 588 / 626, 1 x 1536 645 / 618; 16 heads of 128/64 1 x 1536 535 / 586,
+    2 x 1536 649 / 616.  A forward from chains of 2048 tokens at K = 128 on, as the operators, and with more work: 340M 1 x 2048 242 / 346, 3 x 2048 303 / 356,
+    4 x 2048 363 / 360, 1 x 3000 258 / 318, 2 x 3000 336 / 322; 760M 1 x 2048 282 / 342, 1 x 3000 379 / 350; shorter ones are 0.95 to 1.06 either way."""
     if CONCURRENT_BRANCHES is not None:
         return bool(CONCURRENT_BRANCHES)
     work = B * T * how["D"] * (sum(how["widths"]) + how["widths"][-1])       # (the output projection is as wide as the gate's)
-    if work + 10_000_000 * T < 42_000_000_000 if gradients else work + 12_000_000 * T < 72_000_000_000 or T * how["K"] < _SIDE_BY_SIDE_TOKENS_X_K:
+    if work + 15_000_000 * T < 42_000_000_000 if gradients else work + 12_000_000 * T < 72_000_000_000 or T * how["K"] < _SIDE_BY_SIDE_TOKENS_X_K:
         return False
     return _scan_leaves_cus(dev, B, how["H"], how["V"])
 

@@ -1812,7 +1812,7 @@ bool softmax_reads_types(int B, int T, int HQ, int HKV, int TN, int block, const
   return softmax_variant(B, T, HQ, HKV, block, false, use, 0, &sd, &rc) >= 0 && !sd;
 }
 
-// Wherever tiles of 128 queries are taken and the branches follow each other: 86 sizes of one to 1472 workgroups in all, 10 to 80 % attention, gain 2 to 37 %.
+// Wherever tiles of 128 queries are taken and the branches follow each other: 120 sizes of 9 to 1472 workgroups in all, 10 to 80 % attention, gain 2 to 37 %.
 // Those have two prep workgroups a tile at most, which equal heads come to; with more (many linear heads on few attention heads) the prep, here two
 // workgroups a CU for its own kernel's four to six, would be the longer part.
 bool softmax_takes_prep(int B, int T, int HQ, int HKV, int KA, int VA, int block, const natsl_seq_row* seqs, bool delta, int K, long long prep_wgs) {

@@ -274,21 +274,25 @@ static int wgrad_cus() {
 // 32768 tokens: 37 us with 32 slices of whole tiles, 27 with 85 of the strips that there are).  A tile of 192 columns takes 0.88 of the time of
 // one of 256 for 0.75 of its work and is taken where such tiles fill the CUs better: 6944 rows x 1536 columns over 6000 tokens, 232 units for 174, 155 -> 139
 // us; 1536 x 2304 over 6000 56 -> 53, 1024 x 1536 over 8192 41 -> 39; over 24000 tokens four slices of the first in tiles of 256 stay (461, 493 in 192).
+// The slices for tiles of 256 go by 17 ns a token, what a unit takes on a chip that is not full, the choice of the width by what units take at the power limit: with
+// that for the slices too, 6176 rows x 1024 columns over 18688 tokens went from two slices, 200 units in one round, to five in two (88 -> 109 us a launch and 11 -> 17 of sums).
 struct WgradSplit { int nb, splits; };
 static WgradSplit wgrad_splits(long long T, int tile_rows, int D, double full_rows) {
   const int cus = wgrad_cus();
-  WgradSplit best{4, 1};
-  double best_cost = 1e300;
-  for (int nb = 4; nb >= 3; --nb) {
-    const int tiles = tile_rows * cdiv(D, 64 * nb);
-    for (int s = 1; s <= 128; ++s) {
-      if (s > 1 && T < 64ll * s) break;
-      const double rounds = (double)(((long long)tiles * s + cus - 1) / cus);
-      const double cost = rounds * (4.0 + (nb == 4 ? WG_TOKEN_US : WG_TOKEN_US_3) * (double)T / s) + 0.1 * full_rows * (cdiv(D, 64 * nb) * nb / 4.) * s;
-      if (cost < best_cost) { best_cost = cost; best = {nb, s}; }
-    }
-  }
-  return best;
+  auto cost = [&](const int nb, const int s, const double token_us) {
+    const double rounds = (double)(((long long)tile_rows * cdiv(D, 64 * nb) * s + cus - 1) / cus);
+    return rounds * (4.0 + token_us * (double)T / s) + 0.1 * full_rows * (cdiv(D, 64 * nb) * nb / 4.) * s;
+  };
+  auto slices = [&](const int nb, const double token_us) {
+    int best = 1;
+    double best_cost = 1e300;
+    for (int s = 1; s <= 128 && (s == 1 || T >= 64ll * s); ++s)
+      if (const double c = cost(nb, s, token_us); c < best_cost) { best_cost = c; best = s; }
+    return best;
+  };
+  const int s4 = slices(4, 0.017), s3 = slices(3, WG_TOKEN_US_3);
+  // (two per cent nearer than they look: 6944 rows x 1536 columns over 18688 tokens 385 us in tiles of 192, 368 in four slices of 256)
+  return 1.02 * cost(3, s3, WG_TOKEN_US_3) < cost(4, s4, WG_TOKEN_US) ? WgradSplit{3, s3} : WgradSplit{4, s4};
 }
 
 static int wgrad_plan(WgradParams& p, const natsl_wgrad_seg* segs, int n_seg, const void* x, int64_t T, int D, int ldx, const char* what) {

@@ -13,7 +13,7 @@ DEV = 'cuda:0'
 @pytest.mark.parametrize("gradients", [False, True])
 @pytest.mark.parametrize("kind,B,T,H,KA,VA,K,V,block", [
     ('gdn', 1, 1, 1, 64, 64, 64, 64, 64), ('gdn', 3, 65, 3, 64, 64, 64, 64, 64), ('gdn', 1, 256, 2, 64, 128, 64, 128, 64), ('gdn', 2, 333, 4, 128, 64, 128, 64, 128),
-    ('gdn', 1, 1000, 4, 128, 128, 128, 128, 256), ('gdn', 2, 300, 6, 64, 128, 192, 128, 64), ('gdn', 1, 200, 2, 128, 128, 64, 64, 64),
+    ('gdn', 1, 1000, 4, 128, 128, 128, 128, 256), ('gdn', 2, 300, 6, 64, 128, 192, 128, 64), ('gdn', 1, 777, 6, 64, 128, 128, 256, 64), ('gdn', 1, 200, 2, 128, 128, 64, 64, 64),
     ('gdn', 1, 1344, 8, 64, 64, 64, 64, 64), ('gdn', 1, 1345, 8, 64, 64, 64, 64, 64), ('gdn', 120, 64, 1, 128, 128, 128, 128, 64),
     ('mamba', 1, 1, 1, 64, 64, 64, 64, 64), ('mamba', 2, 333, 17, 128, 64, 128, 64, 256), ('mamba', 1, 700, 5, 64, 128, 192, 128, 64),
     ('mamba', 1, 1500, 16, 128, 128, 128, 128, 64)])

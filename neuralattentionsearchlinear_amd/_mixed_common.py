@@ -198,6 +198,38 @@ def state_behind(ht, hs, gs, last):
     return torch.where(lin, ht, hs if gs is None else hs * torch.exp(gs).view(n, H, 1, 1))
 
 
+def _same_rows(t, shape) -> bool:
+    """Whether t holds the rows of `shape` in its order (sizes of one more or less do not move a number)."""
+    return t.shape == shape or [n for n in t.shape if n != 1] == [n for n in shape if n != 1]
+
+
+def _check_operands(q_attn, k_attn, v_attn, q, k, v, g, beta, types, n_prefix: int = 0):
+    """ValueError unless the tensors go together: the kernels take every size from q_attn, q and the widths of the others, so a tensor of another size would be
+    read past its end or at strides that are not its own.  (The branches may have other numbers of tokens than each other while these make as many blocks,
+    which the native entry compares.)"""
+    B, T, H, K = q.shape
+    _, T_attn, HQ, KA = q_attn.shape
+    keys = (B, T_attn + n_prefix, *k_attn.shape[2:3])
+    for name, t, shape in (("q_attn", q_attn, (B, T_attn, HQ, KA)), ("k_attn", k_attn, (*keys, KA)), ("v_attn", v_attn, (*keys, *v_attn.shape[3:4])),
+                           ("k_lattn", k, (B, T, H, K)), ("v_lattn", v, (B, T, H, *v.shape[3:4])), ("nats_block_types", types, (B, *types.shape[1:3], 2))):
+        if len(shape) != 4 or t.shape != shape:
+            raise ValueError(f"{name} must have shape {list(shape)} beside q_lattn {list(q.shape)} and q_attn {list(q_attn.shape)}, got {list(t.shape)}")
+    for name, t in (("g", g), ("beta", beta)):
+        if t is not None and not _same_rows(t, (B, T, H)):
+            raise ValueError(f"{name} must have shape {[B, T, H]} beside q_lattn {list(q.shape)}, got {list(t.shape)}")
+    for name, t in (("q_attn", q_attn), ("k_attn", k_attn), ("v_attn", v_attn), ("k_lattn", k), ("v_lattn", v), ("g", g), ("beta", beta),
+                    ("nats_block_types", types)):
+        if t is not None and t.device != q.device:
+            raise ValueError(f"{name} is on {t.device}, q_lattn on {q.device}")
+
+
+def _check_packed(seqs, T: int, T_attn: int, TN: int):
+    """ValueError unless the packed sequences lie in rows of T (and T_attn) tokens and TN selector blocks."""
+    if seqs is not None and seqs.n_seqs and (seqs.cu_seqlens[0] < 0 or seqs.cu_seqlens[-1] > min(T, T_attn) or seqs.cu_seqlens_nats[0] < 0 or seqs.cu_seqlens_nats[-1] > TN):
+        raise ValueError(f"cu_seqlens runs from {seqs.cu_seqlens[0]} to {seqs.cu_seqlens[-1]} in {min(T, T_attn)} tokens, cu_seqlens_nats from "
+                         f"{seqs.cu_seqlens_nats[0]} to {seqs.cu_seqlens_nats[-1]} in {TN} selector blocks")
+
+
 def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn, initial_state, g, beta, nats_block_types,
                   scale_attn, scale_lattn, cu_seqlens, cu_seqlens_nats, nats_block_size, attn_sw_size,
                   attn_same_block: bool, lin_intra: bool, output_final_state: bool, decay_non_linear: bool,
@@ -229,6 +261,10 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
         raise NotImplementedError("packed sequences are not supported by the prefill hand-off")
     if not q_lattn.is_cuda:
         raise _capi.NatslError("the NAtS-L mixed operator runs on the GPU only (no CPU fallback)")
+    if nats_block_types.shape[-1] != 2:
+        raise NotImplementedError("routing is built for n_ops == 2")
+    _check_operands(q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn, g, beta, nats_block_types,
+                    0 if attn_prefix_valid is None else attn_prefix_valid.shape[1] * nats_block_size)
     io_dtype = q_lattn.dtype
     if io_dtype not in (torch.bfloat16, torch.float32):
         raise NotImplementedError(f"dtype {io_dtype} is not supported (bf16, or fp32 which is computed in bf16)")
@@ -296,8 +332,6 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
     types = types.contiguous()
     B, T, H, K = q_lattn.shape
     V = v_lattn.shape[-1]
-    if types.shape[-1] != 2:
-        raise NotImplementedError("routing is built for n_ops == 2")
     TN, HN = types.shape[1], types.shape[2]
     # Boundaries that lie on the GPU are read behind everything that can be made without them: the host waits there for the work before this
     # call, and what it does afterwards the GPU waits for.
@@ -369,8 +403,8 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
             set_pointer(base + at)
     h0 = None
     if initial_state is not None:
-        if tuple(initial_state.shape) != (n_seqs, H, K, V):
-            raise ValueError(f"initial state must have shape {(n_seqs, H, K, V)}, got {tuple(initial_state.shape)}")
+        if tuple(initial_state.shape) != (n_seqs, H, K, V) or initial_state.device != dev:
+            raise ValueError(f"initial state must have shape {(n_seqs, H, K, V)} on {dev}, got {tuple(initial_state.shape)} on {initial_state.device}")
         h0 = initial_state.detach().to(f32).contiguous()
     m.is_delta, m.B, m.T, m.H, m.HN, m.K, m.V, m.TN, m.block = int(kind == 'gdn'), B, T, H, HN, K, V, TN, nats_block_size
     m.flags = (_capi.DECAY_NON_LINEAR if decay_non_linear else 0) | (_capi.QK_L2NORM if qk_l2norm else 0) | (_capi.INTRA_CHUNK if lin_intra else 0)
@@ -383,6 +417,7 @@ def _mixed_forward_impl(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn,
             setattr(m, name, t.data_ptr())
     if late:
         seqs = pack_sequences_here(cu_seqlens, cu_seqlens_nats, nats_block_size, dev)
+    _check_packed(seqs, T, T_attn, TN)
     if seqs is not None:
         m.seqs, m.n_seqs, m.total_chunks, m.total_qtiles = seqs.table.data_ptr(), seqs.n_seqs, seqs.total_chunks, seqs.total_qtiles
     ref = ctypes.byref(m)

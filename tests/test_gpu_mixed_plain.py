@@ -92,8 +92,6 @@ def test_plain_call_is_the_general_one(kind, name, sizes, change, monkeypatch):
 def _others():
     yield 'half', lambda a: a.update({n: a[n].half() for n in ('qa', 'q')})
     yield 'integer types', lambda a: a.update(types=a['types'].int())
-    yield 'a longer key tensor', lambda a: a.update(ka=torch.cat([a['ka'], a['ka']], 1))
-    yield 'a shorter gate', lambda a: a.update(g=a['g'][:, :-1])
     yield 'blocks of 96', lambda a: a.update(block=96)
     yield 'types of three', lambda a: a.update(types=torch.cat([a['types'], a['types'][..., :1]], -1))
     yield 'a state of another shape', lambda a: a.update(h0=torch.zeros(1, 2, 64, 64, device=DEV))
@@ -122,6 +120,30 @@ def test_other_calls_end_as_they_did(name, change, monkeypatch):
         assert isinstance(with_it, list) and all(torch.equal(x, y) for x, y in zip(with_it, without))
     else:
         assert with_it == without
+
+
+def _misfits():
+    yield 'a longer key tensor', lambda a: a.update(ka=torch.cat([a['ka'], a['ka']], 1))
+    yield 'a shorter gate', lambda a: a.update(g=a['g'][:, :-1])
+    yield 'a shorter beta in fp32', lambda a: a.update(beta=a['beta'][:, :-1].float())
+    yield 'a value tensor of one sequence', lambda a: a.update(v=a['v'][:1])
+    yield 'types of one sequence', lambda a: a.update(types=a['types'][:1])
+    yield 'a gate on the CPU', lambda a: a.update(g=a['g'].cpu())
+
+
+@pytest.mark.parametrize("gradients", [False, True])
+@pytest.mark.parametrize("name,change", list(_misfits()), ids=[f[0] for f in _misfits()])
+def test_tensors_that_do_not_go_together_are_refused(name, change, gradients, monkeypatch):
+    """... before anything is launched."""
+    from neuralattentionsearchlinear_amd import _capi
+    a = _args('gdn')
+    change(a)
+    if gradients:
+        a['q'] = a['q'].clone().requires_grad_(True)
+    for entry in ('natsl_mixed_fwd', 'natsl_route'):
+        monkeypatch.setattr(_capi.lib(), entry, lambda *x: pytest.fail("launched"))
+    with pytest.raises(ValueError, match=r"must have shape|is on cpu"):
+        _call('gdn', a)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])

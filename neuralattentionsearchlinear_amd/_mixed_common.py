@@ -578,7 +578,7 @@ def _plain_forward(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn, init
     side = _get_attn_stream(dev).cuda_stream if B > 0 and _run_side_by_side(dev, False, B, B, T, H, K, v_lattn.shape[-1]) else cur
     options = (kind == 'gdn') | bool(decay_non_linear) << 1 | bool(qk_l2norm) << 2 | bool(lin_intra) << 3 | bool(attn_same_block) << 4 | \
         bool(output_final_state) << 5
-    done = _capi.step_core().mixed_plain(_capi.entries(), options, int(block), scale_attn, scale_lattn, cur, side, q_attn, k_attn, v_attn, q_lattn, k_lattn,
+    done = _capi.step_core().mixed_plain(_capi.entries(), options, block, scale_attn, scale_lattn, cur, side, q_attn, k_attn, v_attn, q_lattn, k_lattn,
                                          v_lattn, initial_state, g, beta, types)
     if done is not None and type(done) is not tuple:
         _capi.check(done, "natsl_mixed_fwd")
@@ -600,7 +600,8 @@ def mixed_forward(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn, initi
     # (the prefill operators are plain functions in the reference too: their outputs carry no gradient)
     if inference or not _wants_grad(*tensors):
         if not inference and cu_seqlens is None and attn_prefix_valid is None and attn_sw_size is None and n_tokens_in_current_block == 0 and \
-                not use_g_for_attn and incomplete_block_start_with_ht and TIMING_HOOK is None and q_lattn.is_cuda and q_lattn.dim() == 4:
+                not use_g_for_attn and incomplete_block_start_with_ht and TIMING_HOOK is None and q_lattn.is_cuda and q_lattn.dim() == 4 and \
+                type(nats_block_size) is int:
             done = _plain_forward(kind, q_attn, k_attn, v_attn, q_lattn, k_lattn, v_lattn, initial_state, g, beta, nats_block_types, scale_attn,
                                   scale_lattn, nats_block_size, attn_same_block, lin_intra, output_final_state, decay_non_linear, qk_l2norm)
             if done is not None:

@@ -92,6 +92,8 @@ def test_plain_call_is_the_general_one(kind, name, sizes, change, monkeypatch):
 def _others():
     yield 'half', lambda a: a.update({n: a[n].half() for n in ('qa', 'q')})
     yield 'integer types', lambda a: a.update(types=a['types'].int())
+    yield 'blocks of 64.9', lambda a: a.update(block=64.9)
+    yield 'blocks of 64.0', lambda a: a.update(block=64.0)
     yield 'blocks of 96', lambda a: a.update(block=96)
     yield 'types of three', lambda a: a.update(types=torch.cat([a['types'], a['types'][..., :1]], -1))
     yield 'a state of another shape', lambda a: a.update(h0=torch.zeros(1, 2, 64, 64, device=DEV))

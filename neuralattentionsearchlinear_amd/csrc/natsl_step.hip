@@ -420,6 +420,7 @@ NATSL_DEVICE void wait_for(const StepOne& p, Ask ask) {
     if (n % 64u == 0u && ld_word(p.sync + StepSync::FAILED)) return;
     if (__builtin_amdgcn_s_memrealtime() - since > p.max_wait) {
       if ((threadIdx.x & 63) == 0) __hip_atomic_store(p.sync + StepSync::FAILED, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // (seen before whatever the wave makes of what it has: see arrive())
       return;
     }
   }

@@ -637,9 +637,12 @@ typedef struct natsl_layer_step {
 size_t natsl_layer_step_workspace_bytes(const natsl_layer_step* step);
 int natsl_layer_step_fwd(const natsl_layer_step* step, void* workspace, size_t workspace_bytes, natsl_stream_t stream);
 /* The same with memory that the caller keeps from step to step, natsl_layer_step_sync_bytes of it on the device, zeros before the first step and
- * not touched between steps (0 bytes: such a step has no use for it): a step of one token of few sequences is one launch then instead of three.
+ * not touched between steps: a step of one token of few sequences is one launch then instead of three.  0 bytes: such a step meets nowhere, but it is given
+ * the memory of the cache's other steps, where there is any, to know whether one of them failed.
  * Steps that may run at the same time, or of other numbers of sequences, have memory of their own.  A part of the launch that waits
- * longer than max_wait_us for another gives up: the step's output, and that of every later step with this memory, is NaN. */
+ * longer than max_wait_us for another gives up: the step's output, and that of every later step with this memory, in one launch or in several, is NaN.
+ * Word NATSL_STEP_SYNC_FAILED of the memory is not 0 from then on. */
+enum { NATSL_STEP_SYNC_FAILED = 32 };
 size_t natsl_layer_step_sync_bytes(const natsl_layer_step* step);
 int natsl_layer_step_sync_fwd(const natsl_layer_step* step, void* workspace, size_t workspace_bytes, void* shared, size_t shared_bytes,
                               uint64_t max_wait_us, natsl_stream_t stream);

@@ -367,16 +367,21 @@ PyObject* run(PyObject*, PyObject* const* args, Py_ssize_t n) {
   at::Tensor ws = at::empty({(int64_t)bytes}, f32.dtype(at::kByte));
   void* const ws_ptr = ws.data_ptr();
   // What the parts of a step in one launch meet on belongs to the cache, whose steps follow one another; it holds something from step to step and
-  // is made anew for another number of sequences.
+  // is made anew for another number of sequences, but for the word that says that a step has failed.  Steps of several launches look at that, too.
   const size_t shared_bytes = step->sync_bytes(&s);
   at::Tensor shared;
   if (args[7 + CACHE_ARGS] != Py_None && THPVariable_Check(args[7 + CACHE_ARGS])) shared = THPVariable_Unpack(args[7 + CACHE_ARGS]);
-  if (shared_bytes && (!shared.defined() || shared.nbytes() != shared_bytes || shared.get_device() != step->device || !shared.is_contiguous()))
+  if (shared.defined() && (shared.get_device() != step->device || !shared.is_contiguous() || shared.scalar_type() != at::kInt)) shared = at::Tensor();
+  if (shared_bytes && (!shared.defined() || shared.nbytes() != shared_bytes)) {
+    const at::Tensor before = shared;
     shared = at::zeros({(int64_t)(shared_bytes / 4)}, f32.dtype(at::kInt));
-  void* const shared_ptr = shared_bytes ? shared.data_ptr() : nullptr;
+    if (before.defined()) shared.narrow(0, NATSL_STEP_SYNC_FAILED, 1).copy_(before.narrow(0, NATSL_STEP_SYNC_FAILED, 1));
+  }
+  const size_t given = shared.defined() ? shared.nbytes() : 0;
+  void* const shared_ptr = given ? shared.data_ptr() : nullptr;
   int rc;
   Py_BEGIN_ALLOW_THREADS
-  rc = step->fwd(&s, ws_ptr, bytes, shared_ptr, shared_bytes, step->max_wait_us, stream);
+  rc = step->fwd(&s, ws_ptr, bytes, shared_ptr, given, step->max_wait_us, stream);
   Py_END_ALLOW_THREADS
   if (rc) return PyLong_FromLong(rc);
   THPObjectPtr conv(PyTuple_New(3));

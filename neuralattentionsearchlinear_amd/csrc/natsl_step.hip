@@ -29,6 +29,7 @@ struct RowsGemm {
   int M, D, ldo, n_seg;
   GemmSeg seg[GEMM_SEGS];
   unsigned* zero; int n_zero;   // cleared for a later launch of the step
+  const unsigned* failed;       // null, or where a step says that it has failed: then the rows are NaN
 };
 
 template <int MT>
@@ -38,6 +39,7 @@ __global__ __launch_bounds__(512) void rows_gemm_kernel(const RowsGemm p) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (blockIdx.x == 0)
     for (int i = threadIdx.x; i < p.n_zero; i += 512) p.zero[i] = 0u;
+  const bool failed = p.failed && *p.failed != 0u;        // (of steps before this one: their launches are over)
   int si = 0;
 #pragma unroll
   for (int i = 1; i < GEMM_SEGS; ++i) si = i < p.n_seg && (int)blockIdx.x >= p.seg[i].tile0 ? i : si;
@@ -78,6 +80,7 @@ __global__ __launch_bounds__(512) void rows_gemm_kernel(const RowsGemm p) {
   f32x4 sum = red[0][wave][lane];
 #pragma unroll
   for (int w = 1; w < NW; ++w) sum += red[w][wave][lane];
+  if (failed) sum = (f32x4){NAN, NAN, NAN, NAN};
   // lane: row m = lane%16 of the tile, columns 4*(lane/16)..
   const int m = 16 * wave + r16, n = n0 + 4 * kg;
   if (m >= p.M) return;
@@ -405,6 +408,7 @@ NATSL_DEVICE unsigned long long arrive(const StepOne& p, const int b, const int 
 struct StepSync {
   static constexpr int LINE = 32, LEFT = 0, FAILED = LINE, EPOCH = 2 * LINE, ARRIVED = 3 * LINE;
 };
+static_assert(StepSync::FAILED == NATSL_STEP_SYNC_FAILED, "what the header says");
 NATSL_DEVICE unsigned step_tag(const StepOne& p) { return (ld_word(p.sync + StepSync::EPOCH) + 1u) & 0xffffu; }
 
 // Until ask(), which requests words, finds that none of any lane's is late, or the time is over: then the step has failed, its outputs become
@@ -1081,8 +1085,9 @@ static int step_fwd(const char* what, const natsl_layer_step* step, void* worksp
     return fail(NATSL_ERR_INVALID, "%s: null pointer argument", what);
   const StepLayout l = step_layout(s);
   if (workspace_bytes < l.bytes) return fail(NATSL_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", what, l.bytes, workspace_bytes);
-  if (sync && ((uintptr_t)sync % 8 || sync_bytes < l.sync_bytes))
-    return fail(NATSL_ERR_INVALID, "%s: %zu bytes of the step's own memory needed, %zu given", what, l.sync_bytes, sync_bytes);
+  const size_t sync_needed = std::max(l.sync_bytes, (size_t)StepSync::ARRIVED * 4);
+  if (sync && ((uintptr_t)sync % 8 || sync_bytes < sync_needed))
+    return fail(NATSL_ERR_INVALID, "%s: %zu bytes of the step's own memory needed, %zu given", what, sync_needed, sync_bytes);
   const int KD = s.H * s.K, VD = s.H * s.V, KA = KD / s.HQ, VA = VD / s.HQ, M = s.B * s.T;
   const int out_tiles = cdiv(s.D, 16);
   const bool in_one = sync && l.all && step_may_wait(s, l.n_chunks, l.nsplit);
@@ -1102,7 +1107,7 @@ static int step_fwd(const char* what, const natsl_layer_step* step, void* worksp
   g.x = (const bf16_t*)s.x; g.out = proj; g.M = M; g.D = s.D; g.ldo = l.ldp;
   const GemmSeg segs[GEMM_SEGS] = {{(const bf16_t*)s.wq, KD, 0, l.cq}, {(const bf16_t*)s.wk, KD, 0, l.ck}, {(const bf16_t*)s.wv, VD, 0, l.cv},
                                    {(const bf16_t*)s.wg, VD, 0, l.cg}, {(const bf16_t*)s.wa, s.H, 0, l.ca}, {(const bf16_t*)s.wb, s.H, 0, l.cb}};
-  g.n_seg = s.is_delta ? 6 : 5;
+  g.n_seg = s.is_delta ? 6 : 5; g.failed = nullptr;
   unsigned* arrived = in_one ? sync + StepSync::ARRIVED : (unsigned*)(ws + l.arrived);
   g.zero = arrived; g.n_zero = l.one && !in_one ? M * s.HQ : 0;
   for (int i = 0; i < GEMM_SEGS; ++i) {
@@ -1136,6 +1141,7 @@ static int step_fwd(const char* what, const natsl_layer_step* step, void* worksp
   t.eps = s.out_norm_eps;
   RowsGemm o;
   o.x = y; o.out = (bf16_t*)s.out; o.M = M; o.D = VD; o.ldo = s.D; o.n_seg = 1; o.zero = nullptr; o.n_zero = 0;
+  o.failed = sync ? sync + StepSync::FAILED : nullptr;    // (what a failed step left in the cache is nothing to go on from, in however many launches)
   for (int i = 0; i < GEMM_SEGS; ++i) o.seg[i] = {(const bf16_t*)s.wo, s.D, 0, 0};
   if (l.one) {
     StepOne f;

@@ -67,3 +67,35 @@ def test_a_step_that_waits_too_long_gives_no_numbers(monkeypatch):
     monkeypatch.undo()
     after, _ = _generate(_layer('gdn', None, 'all'), 'gdn', x, 100, (1,) * 3)
     assert all(torch.equal(a, b) for a, b in zip(good, after))
+
+
+@pytest.mark.parametrize("T,launches", [(2, 'five'), (1, 'three')])
+def test_a_failed_step_is_not_gone_on_from_in_several_launches(T, launches, monkeypatch):
+    """A step that failed leaves stale numbers in the cache's rows: later steps on it give none, in however many launches they are, and for another number
+    of sequences, whose steps meet in other memory, too."""
+    import neuralattentionsearchlinear_amd._layer_step as LS
+    from neuralattentionsearchlinear_amd.cache import NAtSCache
+    torch.manual_seed(0)
+    x = torch.randn(1, 110, 256, device=DEV).bfloat16()
+    layer = _layer('gdn', None, 'all')
+    monkeypatch.setattr(LS, 'MAX_WAIT_US', 0)
+    holder = NAtSCache()
+    with torch.no_grad():
+        for piece in (x[:, :100], x[:, 100:101]):
+            layer(piece, past_key_values=holder, use_cache=True)
+        assert int(holder[0].step_shared[32]) == 1
+        monkeypatch.undo()
+        held = _three_launches(monkeypatch) if launches == 'three' else None
+        later = _layer('gdn', None, 'all')                 # (the same weights; a plan of its own)
+        out = later(x[:, 101:101 + T], past_key_values=holder, use_cache=True)[0]
+        assert bool(out.isnan().all()), "numbers from a cache that a failed step has written"
+        del held                                           # (the plan has its address until here)
+        if launches == 'five':
+            cache = holder[0]
+            for name, t in list(vars(cache).items()):      # the same sequence twice
+                if torch.is_tensor(t) and name != 'step_shared':
+                    setattr(cache, name, t.repeat_interleave(2, 0))
+            cache.conv_state = tuple(t.repeat_interleave(2, 0) for t in cache.conv_state)
+            before = cache.step_shared.numel()
+            out = later(x[:, 103:104].repeat_interleave(2, 0), past_key_values=holder, use_cache=True)[0]
+            assert cache.step_shared.numel() != before and bool(out.isnan().all())

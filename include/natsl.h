@@ -639,7 +639,9 @@ int natsl_layer_step_fwd(const natsl_layer_step* step, void* workspace, size_t w
 /* The same with memory that the caller keeps from step to step, natsl_layer_step_sync_bytes of it on the device, zeros before the first step and
  * not touched between steps: a step of one token of few sequences is one launch then instead of three.  0 bytes: such a step meets nowhere, but it is given
  * the memory of the cache's other steps, where there is any, to know whether one of them failed.
- * Steps that may run at the same time, or of other numbers of sequences, have memory of their own.  A part of the launch that waits
+ * Steps that may run at the same time, or of other numbers of sequences, have memory of their own.  A process has one launch at a time on a device whose
+ * parts wait for each other and have not all started, or several on one stream: steps on another stream meanwhile, and captured ones, are several
+ * launches.  Those of two processes fit on a device side by side; where more processes step on one, they can keep each other waiting.  A part of the launch that waits
  * longer than max_wait_us for another gives up: the step's output, and that of every later step with this memory, in one launch or in several, is NaN.
  * Word NATSL_STEP_SYNC_FAILED of the memory is not 0 from then on. */
 enum { NATSL_STEP_SYNC_FAILED = 32 };

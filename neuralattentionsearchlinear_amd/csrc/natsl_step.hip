@@ -10,6 +10,8 @@
 //   step_tail_kernel     join of the attention's splits, mixing weights, two-input norm and gate
 // Roundings to bf16 are where the layer's separate operations round (projections, convolutions, norms, gates, branch outputs).
 #include <algorithm>
+#include <atomic>
+#include <mutex>
 
 #include "natsl_decode_device.h"
 #include "natsl_host.h"
@@ -32,14 +34,17 @@ struct RowsGemm {
   const unsigned* failed;       // null, or where a step says that it has failed: then the rows are NaN
 };
 
-template <int MT>
+// FAILED: p.failed is looked at.  (For all launches, and through an argument that may be null, it was 0.5 us of eight sequences' step on 16 heads of 128/64.)
+template <int MT, bool FAILED>
 __global__ __launch_bounds__(512) void rows_gemm_kernel(const RowsGemm p) {
   constexpr int NW = 8, U = 4;
   __shared__ f32x4 red[NW][MT][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (blockIdx.x == 0)
     for (int i = threadIdx.x; i < p.n_zero; i += 512) p.zero[i] = 0u;
-  const bool failed = p.failed && *p.failed != 0u;        // (of steps before this one: their launches are over)
+  // (by steps before this one, whose launches are over.  The lanes' load, waited for with the weights': a scalar one holds up the first use of an argument)
+  unsigned failed = 0u;
+  if constexpr (FAILED) failed = __hip_atomic_load(p.failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   int si = 0;
 #pragma unroll
   for (int i = 1; i < GEMM_SEGS; ++i) si = i < p.n_seg && (int)blockIdx.x >= p.seg[i].tile0 ? i : si;
@@ -80,7 +85,7 @@ __global__ __launch_bounds__(512) void rows_gemm_kernel(const RowsGemm p) {
   f32x4 sum = red[0][wave][lane];
 #pragma unroll
   for (int w = 1; w < NW; ++w) sum += red[w][wave][lane];
-  if (failed) sum = (f32x4){NAN, NAN, NAN, NAN};
+  if (FAILED && failed != 0u) sum = (f32x4){NAN, NAN, NAN, NAN};
   // lane: row m = lane%16 of the tile, columns 4*(lane/16)..
   const int m = 16 * wave + r16, n = n0 + 4 * kg;
   if (m >= p.M) return;
@@ -386,6 +391,7 @@ struct StepOne {
   // with HERE (StepAll): what the launch's parts meet on (StepSync), the projections and the tail's rows as tagged words, like proj and y
   unsigned *sync, *proj_words, *y_words;
   unsigned long long max_wait;
+  unsigned long long *started, ticket;   // what the host reads (StepsUnderWay), and what the launch leaves there
 };
 constexpr int LOGIT_CHUNK = 256;
 
@@ -406,14 +412,16 @@ NATSL_DEVICE unsigned long long arrive(const StepOne& p, const int b, const int 
 // What the parts of a launch with the products in it (HERE) meet on, in lines of their own.  Zeros at first; a launch leaves the epoch, which its
 // words' tags come from, one higher, and everything else as it was, but FAILED when it did.
 struct StepSync {
-  static constexpr int LINE = 32, LEFT = 0, FAILED = LINE, EPOCH = 2 * LINE, ARRIVED = 3 * LINE;
+  static constexpr int LINE = 32, LEFT = 0, FAILED = LINE, EPOCH = 2 * LINE, STARTED = 3 * LINE, ARRIVED = 4 * LINE;
 };
 static_assert(StepSync::FAILED == NATSL_STEP_SYNC_FAILED, "what the header says");
 NATSL_DEVICE unsigned step_tag(const StepOne& p) { return (ld_word(p.sync + StepSync::EPOCH) + 1u) & 0xffffu; }
 
 // Until ask(), which requests words, finds that none of any lane's is late, or the time is over: then the step has failed, its outputs become
-// NaN, and every wave still ends.  Waves that wait are fewer than the chip holds (step_may_wait), and the workgroups that they wait for
-// come first in the grid and wait for nothing or for others before them, so those always run.
+// NaN, and every wave still ends.  The workgroups that a wave waits for come before its own in the grid, and wait for nothing or for others before
+// them; each XCD starts its share of the grid in order.  So a launch always ends next to others that do: of what an XCD has not started, the first
+// is waited for by none that would have to end before it.  Two launches that have not started all of their workgroups can keep each other's
+// out, one on this XCD and the other on that, unless both fit: see step_may_wait and StepsUnderWay.
 template <class Ask>
 NATSL_DEVICE void wait_for(const StepOne& p, Ask ask) {
   if (!__ballot(ask() != 0u)) return;
@@ -851,6 +859,11 @@ NATSL_DEVICE void step_product(const StepAll& all, const int tile) {
 #pragma unroll
     for (int u = 0; u < U; ++u) a[u] = ld8(wp + 32 * min(s0 + 4 * u, steps - 1));
     if constexpr (OUT) {
+      // (these workgroups are the grid's last on every XCD, and have time until the rows come: told at the launch's end, a token took 1.7 us more)
+      if (s0 == 0 && lane == 0 && __hip_atomic_fetch_add(one.sync + StepSync::STARTED, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == (unsigned)all.out_tiles) {
+        __hip_atomic_store(one.sync + StepSync::STARTED, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(one.started, one.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
       // the rows go through LDS: a thread brings its share of their words, two at a time
       if (s0 == wave) {
         constexpr int N = 8;
@@ -978,13 +991,58 @@ static int step_one_slots(const natsl_layer_step& s, const int n_chunks) {
 }
 
 // Workgroups that wait when the products are in the launch too: those between the products and those behind them.  At most half of what fits on
-// the chip, so that one that is waited for always finds room, and no more than this: with 268 of the 340M geometry (four sequences of 500 tokens) a
-// token is 0.87 of the three launches' time, with 304 and 352 of 16 heads of 128/64 (six of 300, four of 1200) 1.02, where the
-// host is no longer what a step waits for.
+// the chip, so that those of two launches (of two processes: StepsUnderWay) leave room for one that is waited for, and no more than this: with 268 of the
+// 340M geometry (four sequences of 500 tokens) a token is 0.87 of the three launches' time, with 304 and 352 of 16 heads of 128/64 (six of 300, four of
+// 1200) 1.02, where the host is no longer what a step waits for.
 constexpr int STEP_WAITERS = 280;
-static bool step_may_wait(const natsl_layer_step& s, const int n_chunks, const int nsplit) {
+static bool step_may_wait(const natsl_layer_step& s, const int n_chunks, const int nsplit, const int cus) {
   const int n = s.B * (n_chunks + s.H * cdiv(s.V, 64) + s.HQ * nsplit) + cdiv(s.D, 16);
-  return n <= STEP_WAITERS && 2 * n <= step_one_per_cu(s) * 256;
+  return n <= STEP_WAITERS && 2 * n <= step_one_per_cu(s) * cus;
+}
+
+// The launches whose workgroups wait for each other, by device: of a process's, one at a time has workgroups that have not started, or several of one
+// stream, which follow one another.  Steps on another stream (of another cache: another thread's, another request's) are several launches, which wait for
+// nothing, until the last has started all of its workgroups, which it writes into pinned memory that the host looks at; so are those that are
+// captured, whose replays nobody counts.  Held from the look to the launch, so that tickets are in the order of their launches.
+struct StepsUnderWay {
+  std::mutex mu;
+  unsigned long long issued = 0, *started = nullptr;
+  hipStream_t on = nullptr;
+  std::atomic<int> cus{0};
+};
+static StepsUnderWay* steps_under_way() {
+  static StepsUnderWay devs[64];
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
+  if (devs[dev].cus.load(std::memory_order_relaxed) == 0 && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
+    devs[dev].cus.store(n, std::memory_order_relaxed);
+  return &devs[dev];
+}
+// The next launch's ticket, or 0: not now.
+static unsigned long long step_ticket(StepsUnderWay& u, hipStream_t st) {
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &capturing) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  if (capturing != hipStreamCaptureStatusNone) return 0;
+  if (!u.started) {
+    void* p = nullptr;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;                // (another thread may be capturing: this is none of its graph's)
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    const hipError_t e = hipHostMalloc(&p, 64, hipHostMallocMapped | hipHostMallocCoherent);    // one line a device, for as long as the process lives
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      return 0;
+    }
+    u.started = static_cast<unsigned long long*>(p);
+    __atomic_store_n(u.started, 0ull, __ATOMIC_RELAXED);
+  }
+  // (every thread's own default stream has the same name)
+  if ((st != u.on || st == hipStreamPerThread) && __atomic_load_n(u.started, __ATOMIC_ACQUIRE) < u.issued) return 0;
+  u.on = st;
+  return ++u.issued;
 }
 
 // One token a sequence: one launch between the two products.  That kernel is built for the layers' own convolution width and reads windows
@@ -1036,9 +1094,9 @@ static StepLayout step_layout(const natsl_layer_step& s) {
   l.arrived = take((size_t)M * s.HQ * 4);
   l.bytes = at;
   // The products in the launch: a row tile of tokens, whose rows fit the output projection's workgroups (each of its waves has a part of a row), and
-  // no more workgroups that wait than may; whether they do at this step's number of
-  // keys is step_fwd's to see, so that a cache's steps all want the same memory.
-  l.all = l.one && M <= 16 && M * VD <= STEP_ROWS && VD >= 128 && step_may_wait(s, l.n_chunks, 1);
+  // no more workgroups that wait than may, and some of the last ones on each of eight XCDs (StepSync::STARTED); whether they do at this step's number of
+  // keys, and on this device, is step_fwd's to see, so that a cache's steps all want the same memory.
+  l.all = l.one && M <= 16 && M * VD <= STEP_ROWS && VD >= 128 && s.D >= 128 && step_may_wait(s, l.n_chunks, 1, 256);
   at = 0;
   take((StepSync::ARRIVED + (size_t)M * s.HQ) * 4);
   l.proj_words = take((size_t)M * l.ldp * 4);
@@ -1090,7 +1148,14 @@ static int step_fwd(const char* what, const natsl_layer_step* step, void* worksp
     return fail(NATSL_ERR_INVALID, "%s: %zu bytes of the step's own memory needed, %zu given", what, sync_needed, sync_bytes);
   const int KD = s.H * s.K, VD = s.H * s.V, KA = KD / s.HQ, VA = VD / s.HQ, M = s.B * s.T;
   const int out_tiles = cdiv(s.D, 16);
-  const bool in_one = sync && l.all && step_may_wait(s, l.n_chunks, l.nsplit);
+  StepsUnderWay* const under_way = sync && l.all ? steps_under_way() : nullptr;
+  std::unique_lock<std::mutex> turn;
+  unsigned long long ticket = 0;
+  if (under_way && step_may_wait(s, l.n_chunks, l.nsplit, under_way->cus.load(std::memory_order_relaxed))) {
+    turn = std::unique_lock<std::mutex>(under_way->mu);
+    if ((ticket = step_ticket(*under_way, reinterpret_cast<hipStream_t>(stream))) == 0) turn.unlock();
+  }
+  const bool in_one = ticket != 0;
   char* ws = reinterpret_cast<char*>(workspace);
   bf16_t *proj = (bf16_t*)(ws + l.proj), *q_conv = (bf16_t*)(ws + l.q_conv), *q_lin = (bf16_t*)(ws + l.q_lin), *q_attn = (bf16_t*)(ws + l.q_attn),
          *o_lin = (bf16_t*)(ws + l.o_lin), *y = (bf16_t*)(ws + l.y);
@@ -1098,9 +1163,9 @@ static int step_fwd(const char* what, const natsl_layer_step* step, void* worksp
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
 
   auto gemm = [&](const RowsGemm& g, int tiles) {
-    if (M <= 16) hipLaunchKernelGGL((rows_gemm_kernel<1>), dim3(tiles), dim3(512), 0, st, g);
-    else if (M <= 32) hipLaunchKernelGGL((rows_gemm_kernel<2>), dim3(tiles), dim3(512), 0, st, g);
-    else hipLaunchKernelGGL((rows_gemm_kernel<4>), dim3(tiles), dim3(512), 0, st, g);
+    auto kernel = g.failed ? (M <= 16 ? rows_gemm_kernel<1, true> : M <= 32 ? rows_gemm_kernel<2, true> : rows_gemm_kernel<4, true>)
+                           : (M <= 16 ? rows_gemm_kernel<1, false> : M <= 32 ? rows_gemm_kernel<2, false> : rows_gemm_kernel<4, false>);
+    hipLaunchKernelGGL(kernel, dim3(tiles), dim3(512), 0, st, g);
     return check_launch(what);
   };
   RowsGemm g;
@@ -1151,6 +1216,7 @@ static int step_fwd(const char* what, const natsl_layer_step* step, void* worksp
     if (in_one) {
       char* mem = reinterpret_cast<char*>(sync);
       f.sync = sync; f.proj_words = reinterpret_cast<unsigned*>(mem + l.proj_words); f.y_words = reinterpret_cast<unsigned*>(mem + l.y_words);
+      f.started = under_way->started; f.ticket = ticket;
       f.max_wait = 100 * max_wait_us;                     // (the counter behind s_memrealtime runs at 100 MHz)
       const StepAll all = {f, g, o, l.tiles, out_tiles};
       return launch_step_one(what, f, &all, s.K, KA, VA, st);

@@ -75,7 +75,17 @@ int hipLaunchKernel(const void* f, dim3_t grid, dim3_t block, void** args, size_
   return 0;
 }
 int hipFuncSetAttribute(const void* f, int attr, int value) { (void)f; (void)attr; (void)value; return 0; }
-int hipDeviceGetAttribute(int* v, int attr, int d) { (void)attr; (void)d; *v = 256; return 0; }
+int fake_cus = 256, fake_capturing, fake_no_host_memory;
+unsigned long long fake_host_words[8];   /* the first pinned memory that is asked for */
+int hipDeviceGetAttribute(int* v, int attr, int d) { (void)attr; (void)d; *v = fake_cus; return 0; }
+int hipStreamIsCapturing(void* s, int* status) { (void)s; *status = fake_capturing; return 0; }
+int hipThreadExchangeStreamCaptureMode(int* mode) { (void)mode; return 0; }
+int hipHostMalloc(void** p, size_t n, unsigned flags) {
+  (void)flags;
+  if (fake_no_host_memory || n > sizeof(fake_host_words)) return 2;   /* hipErrorOutOfMemory */
+  *p = fake_host_words;
+  return 0;
+}
 int hipGetDevicePropertiesR0600(void* p, int d) { (void)p; (void)d; return 1; }
 int hipGetSymbolAddress(void** p, const void* symbol) { (void)symbol; *p = (void*)4096; return 0; }
 int hipGetLastError(void) { return 0; }

@@ -99,3 +99,25 @@ def test_a_failed_step_is_not_gone_on_from_in_several_launches(T, launches, monk
             before = cache.step_shared.numel()
             out = later(x[:, 103:104].repeat_interleave(2, 0), past_key_values=holder, use_cache=True)[0]
             assert cache.step_shared.numel() != before and bool(out.isnan().all())
+
+
+def test_caches_on_streams_of_their_own():
+    """Steps of three caches, each on its own stream, in turn and without a wait between: those that find another's under way are three launches, and
+    all give what they give alone."""
+    from neuralattentionsearchlinear_amd.cache import NAtSCache
+    layer, n = _layer('gdn', '340M', 'all'), 20
+    torch.manual_seed(1)
+    xs = [torch.randn(1, 150 + n, layer.hidden_size, device=DEV).bfloat16() for _ in range(3)]
+    alone = [_generate(layer, 'gdn', x, 150, (1,) * n)[0] for x in xs]
+    torch.cuda.synchronize()
+    streams, holders, outs = [torch.cuda.Stream() for _ in xs], [NAtSCache() for _ in xs], [[] for _ in xs]
+    with torch.no_grad():
+        for t in range(n + 1):
+            for x, s, h, o in zip(xs, streams, holders, outs):
+                with torch.cuda.stream(s):
+                    piece = x[:, :150] if t == 0 else x[:, 149 + t:150 + t]
+                    o.append(layer(piece, past_key_values=h, use_cache=True)[0])
+    torch.cuda.synchronize()
+    for a, o in zip(alone, outs):
+        assert all(torch.equal(p, q) for p, q in zip(a, o))
+    assert all(int(h[0].step_shared[32]) == 0 for h in holders)

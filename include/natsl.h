@@ -648,6 +648,9 @@ enum { NATSL_STEP_SYNC_FAILED = 32 };
 size_t natsl_layer_step_sync_bytes(const natsl_layer_step* step);
 int natsl_layer_step_sync_fwd(const natsl_layer_step* step, void* workspace, size_t workspace_bytes, void* shared, size_t shared_bytes,
                               uint64_t max_wait_us, natsl_stream_t stream);
+/* A number that changes with every such launch of this process on the device that gives up, 0 before the first: by when the host sees it, the launch's memory
+ * says so, too. */
+uint64_t natsl_layer_step_gave_up(int device);
 
 #ifdef __cplusplus
 }

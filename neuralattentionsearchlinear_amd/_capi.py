@@ -17,6 +17,7 @@ STEP_CORE_PATH = os.path.join(_HERE, "_step_core.so")
 
 F32, BF16 = 0, 1
 DECAY_NON_LINEAR, QK_L2NORM, INTRA_CHUNK, QUERY_ONLY, FRESH_BLOCK_START, STATES_ONLY = 1, 2, 4, 8, 16, 32
+STEP_SYNC_FAILED = 32                                    # the word of a step's shared memory that says that one has failed
 
 _lib = _step_core = None
 _entries = None
@@ -121,6 +122,7 @@ _SIGNATURES = {
     "natsl_layer_step_fwd": (c_int, [c_void_p, c_void_p, c_size_t, c_void_p]),
     "natsl_layer_step_sync_bytes": (c_size_t, [c_void_p]),
     "natsl_layer_step_sync_fwd": (c_int, [c_void_p, c_void_p, c_size_t, c_void_p, c_size_t, c_uint64, c_void_p]),
+    "natsl_layer_step_gave_up": (c_uint64, [c_int]),
     "natsl_kv_compact": (c_int, [c_void_p, c_void_p, c_longlong, c_int, c_void_p, c_void_p, c_longlong, c_void_p, c_int, c_void_p,
                                  c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
 }

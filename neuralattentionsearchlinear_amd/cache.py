@@ -111,7 +111,8 @@ class NAtSLayerCache:
         self.n_observed_tokens = 0
         self._pending_first = None                       # K/V of the first forward, kept until update() has the types
         self._foreseen = None                            # counts on their way to the host (foresee)
-        self.step_shared = None                        # what the parts of a generation step in one launch meet on
+        self.step_shared = None                          # what the parts of a generation step in one launch meet on
+        self._gave_up = 0                                # natsl_layer_step_gave_up when that was last looked into
 
     def is_empty(self) -> bool:
         """Whether nothing of a forward has been kept (but the hidden states of the one that runs)."""
@@ -287,6 +288,7 @@ class NAtSLayerCache:
             foreseen = self._count(nats_block_types, types, n_complete)
         _, _, after, host, ready = foreseen
         ready.synchronize()                                                     # the host needs the largest count to size the cache
+        self._check_steps()
         new_max = int(host)
         tail_dst = new_max if tail_tokens else -1
         L, P = _capi.lib(), _capi.ptr
@@ -347,6 +349,19 @@ class NAtSLayerCache:
         ready = torch.cuda.Event()
         ready.record(torch.cuda.current_stream(types.device))
         return key, n_complete, after, host, ready
+
+    def _check_steps(self):
+        """Where the host has waited for the cache's steps anyway: an error if one of them gave up, whose outputs, and those since, are NaN.  (Without a launch
+        that gave up on the device since the last look this is one read of host memory.)"""
+        shared = getattr(self, 'step_shared', None)
+        if shared is None:
+            return
+        gave_up = _capi.lib().natsl_layer_step_gave_up(shared.device.index)
+        if gave_up != getattr(self, '_gave_up', 0):
+            self._gave_up = gave_up
+            if int(shared[_capi.STEP_SYNC_FAILED]):
+                raise _capi.NatslError("a generation step on this cache waited too long for a part of its launch and gave up: the cache holds stale rows, and "
+                                       "every output since is NaN")
 
     def foresee(self, nats_block_types: torch.Tensor, n_new_tokens: int):
         """Called by a forward as soon as it knows the new blocks' types: the counts update() needs on the host are enqueued here, so

@@ -391,7 +391,7 @@ struct StepOne {
   // with HERE (StepAll): what the launch's parts meet on (StepSync), the projections and the tail's rows as tagged words, like proj and y
   unsigned *sync, *proj_words, *y_words;
   unsigned long long max_wait;
-  unsigned long long *started, ticket;   // what the host reads (StepsUnderWay), and what the launch leaves there
+  unsigned long long *started, ticket;   // what the host reads (StepsUnderWay; behind it the last one that failed), and what the launch leaves there
 };
 constexpr int LOGIT_CHUNK = 256;
 
@@ -433,6 +433,7 @@ NATSL_DEVICE void wait_for(const StepOne& p, Ask ask) {
     if (__builtin_amdgcn_s_memrealtime() - since > p.max_wait) {
       if ((threadIdx.x & 63) == 0) __hip_atomic_store(p.sync + StepSync::FAILED, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // (seen before whatever the wave makes of what it has: see arrive())
+      if ((threadIdx.x & 63) == 0) __hip_atomic_store(p.started + 1, p.ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       return;
     }
   }
@@ -1006,17 +1007,19 @@ static bool step_may_wait(const natsl_layer_step& s, const int n_chunks, const i
 // captured, whose replays nobody counts.  Held from the look to the launch, so that tickets are in the order of their launches.
 struct StepsUnderWay {
   std::mutex mu;
-  unsigned long long issued = 0, *started = nullptr;
+  unsigned long long issued = 0;
+  std::atomic<unsigned long long*> words{nullptr};   // the last launch that has started, the last that gave up
   hipStream_t on = nullptr;
   std::atomic<int> cus{0};
 };
+static StepsUnderWay steps_of[64];
 static StepsUnderWay* steps_under_way() {
-  static StepsUnderWay devs[64];
   int dev = 0, n = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
-  if (devs[dev].cus.load(std::memory_order_relaxed) == 0 && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
-    devs[dev].cus.store(n, std::memory_order_relaxed);
-  return &devs[dev];
+  StepsUnderWay& u = steps_of[dev];
+  if (u.cus.load(std::memory_order_relaxed) == 0 && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
+    u.cus.store(n, std::memory_order_relaxed);
+  return &u;
 }
 // The next launch's ticket, or 0: not now.
 static unsigned long long step_ticket(StepsUnderWay& u, hipStream_t st) {
@@ -1026,7 +1029,8 @@ static unsigned long long step_ticket(StepsUnderWay& u, hipStream_t st) {
     return 0;
   }
   if (capturing != hipStreamCaptureStatusNone) return 0;
-  if (!u.started) {
+  unsigned long long* words = u.words.load(std::memory_order_relaxed);
+  if (!words) {
     void* p = nullptr;
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;                // (another thread may be capturing: this is none of its graph's)
     (void)hipThreadExchangeStreamCaptureMode(&mode);
@@ -1036,11 +1040,13 @@ static unsigned long long step_ticket(StepsUnderWay& u, hipStream_t st) {
       (void)hipGetLastError();
       return 0;
     }
-    u.started = static_cast<unsigned long long*>(p);
-    __atomic_store_n(u.started, 0ull, __ATOMIC_RELAXED);
+    words = static_cast<unsigned long long*>(p);
+    __atomic_store_n(words, 0ull, __ATOMIC_RELAXED);
+    __atomic_store_n(words + 1, 0ull, __ATOMIC_RELAXED);
+    u.words.store(words, std::memory_order_release);
   }
   // (every thread's own default stream has the same name)
-  if ((st != u.on || st == hipStreamPerThread) && __atomic_load_n(u.started, __ATOMIC_ACQUIRE) < u.issued) return 0;
+  if ((st != u.on || st == hipStreamPerThread) && __atomic_load_n(words, __ATOMIC_ACQUIRE) < u.issued) return 0;
   u.on = st;
   return ++u.issued;
 }
@@ -1216,7 +1222,7 @@ static int step_fwd(const char* what, const natsl_layer_step* step, void* worksp
     if (in_one) {
       char* mem = reinterpret_cast<char*>(sync);
       f.sync = sync; f.proj_words = reinterpret_cast<unsigned*>(mem + l.proj_words); f.y_words = reinterpret_cast<unsigned*>(mem + l.y_words);
-      f.started = under_way->started; f.ticket = ticket;
+      f.started = under_way->words.load(std::memory_order_relaxed); f.ticket = ticket;
       f.max_wait = 100 * max_wait_us;                     // (the counter behind s_memrealtime runs at 100 MHz)
       const StepAll all = {f, g, o, l.tiles, out_tiles};
       return launch_step_one(what, f, &all, s.K, KA, VA, st);
@@ -1250,4 +1256,9 @@ extern "C" size_t natsl_layer_step_sync_bytes(const natsl_layer_step* step) {
 extern "C" int natsl_layer_step_sync_fwd(const natsl_layer_step* step, void* workspace, size_t workspace_bytes, void* shared, size_t shared_bytes,
                                          uint64_t max_wait_us, natsl_stream_t stream) {
   return step_fwd("natsl_layer_step_sync_fwd", step, workspace, workspace_bytes, reinterpret_cast<unsigned*>(shared), shared_bytes, max_wait_us, stream);
+}
+
+extern "C" uint64_t natsl_layer_step_gave_up(int device) {
+  const unsigned long long* words = device >= 0 && device < 64 ? steps_of[device].words.load(std::memory_order_acquire) : nullptr;
+  return words ? __atomic_load_n(words + 1, __ATOMIC_ACQUIRE) : 0;
 }

@@ -121,3 +121,19 @@ def test_caches_on_streams_of_their_own():
     for a, o in zip(alone, outs):
         assert all(torch.equal(p, q) for p, q in zip(a, o))
     assert all(int(h[0].step_shared[32]) == 0 for h in holders)
+
+
+def test_a_failed_step_is_reported_where_the_host_waits(monkeypatch):
+    """The host waits for a cache's steps at a block's end: there a step that gave up is an error, and no other cache's."""
+    import neuralattentionsearchlinear_amd._layer_step as LS
+    from neuralattentionsearchlinear_amd import _capi
+    torch.manual_seed(0)
+    x = torch.randn(1, 130, 256, device=DEV).bfloat16()
+    good, _ = _generate(_layer('gdn', None, 'all'), 'gdn', x, 120, (1,) * 10)
+    with monkeypatch.context() as mp:
+        mp.setattr(LS, 'MAX_WAIT_US', 0)
+        with pytest.raises(_capi.NatslError, match="gave up"):
+            _generate(_layer('gdn', None, 'all'), 'gdn', x, 120, (1,) * 10)
+    assert _capi.lib().natsl_layer_step_gave_up(0) > 0
+    after, cache = _generate(_layer('gdn', None, 'all'), 'gdn', x, 120, (1,) * 10)
+    assert all(torch.equal(a, b) for a, b in zip(good, after)) and cache._gave_up == _capi.lib().natsl_layer_step_gave_up(0)

@@ -83,6 +83,10 @@ for stream, done, capturing, no_memory, device in json.loads(sys.argv[4]):
     shared = lib.natsl_layer_step_sync_bytes(s)
     rc = lib.natsl_layer_step_sync_fwd(s, P(1 << 20), Z(lib.natsl_layer_step_workspace_bytes(s)), P(1 << 21), Z(shared), ctypes.c_uint64(1000), P(stream))
     out.append((rc, len(fake.fake_launches().decode().splitlines())))
+lib.natsl_layer_step_gave_up.restype = ctypes.c_ulonglong
+before = lib.natsl_layer_step_gave_up(0)
+(ctypes.c_ulonglong * 8).in_dll(fake, "fake_host_words")[1] = 4
+out.append([before, *(lib.natsl_layer_step_gave_up(d) for d in (0, 1, -1, 64))])
 print(json.dumps(out))
 """
 
@@ -99,7 +103,7 @@ def test_one_launch_at_a_time_waits_to_start(fake_hip):  # noqa: F811
     r = subprocess.run([sys.executable, "-c", TURNS, fake_hip, _capi.LIB_PATH, bytes(_step("gdn_340M", 1, 1, 473, 1024)).hex(),
                         json.dumps([c for c, _ in calls])], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
-    assert json.loads(r.stdout) == [[0, n] for _, n in calls]
+    assert json.loads(r.stdout) == [[0, n] for _, n in calls] + [[0, 4, 0, 0, 0]]       # (and what a launch that gives up leaves there)
 
 
 @pytest.mark.parametrize("cus,one", [(256, True), (128, False), (32, False)])

@@ -10,13 +10,18 @@ pytestmark = pytest.mark.gpu
 DEV = 'cuda:0'
 
 
+# kind, B, T, H, head widths of the softmax branch, of the linear branch, block, whether one launch takes both (test_kernel_choices.py)
+CASES = [
+    ('gdn', 1, 1, 1, 64, 64, 64, 64, 64, True), ('gdn', 3, 65, 3, 64, 64, 64, 64, 64, True), ('gdn', 1, 256, 2, 64, 128, 64, 128, 64, True),
+    ('gdn', 2, 333, 4, 128, 64, 128, 64, 128, True), ('gdn', 1, 1000, 4, 128, 128, 128, 128, 256, True), ('gdn', 2, 300, 6, 64, 128, 192, 128, 64, True),
+    ('gdn', 1, 777, 6, 64, 128, 128, 256, 64, True), ('gdn', 1, 200, 2, 128, 128, 64, 64, 64, False), ('gdn', 1, 1344, 8, 64, 64, 64, 64, 64, True),
+    ('gdn', 1, 1345, 8, 64, 64, 64, 64, 64, True), ('gdn', 120, 64, 1, 128, 128, 128, 128, 64, True), ('mamba', 1, 1, 1, 64, 64, 64, 64, 64, True),
+    ('mamba', 2, 333, 17, 128, 64, 128, 64, 256, True), ('mamba', 1, 700, 5, 64, 128, 192, 128, 64, True), ('mamba', 1, 1500, 16, 128, 128, 128, 128, 64, True),
+    ('gdn', 1, 3839, 16, 64, 64, 64, 64, 64, True), ('gdn', 1, 3841, 16, 64, 64, 64, 64, 64, False)]    # (of 16 heads: one tile of 256 queries a CU)
+
+
 @pytest.mark.parametrize("gradients", [False, True])
-@pytest.mark.parametrize("kind,B,T,H,KA,VA,K,V,block", [
-    ('gdn', 1, 1, 1, 64, 64, 64, 64, 64), ('gdn', 3, 65, 3, 64, 64, 64, 64, 64), ('gdn', 1, 256, 2, 64, 128, 64, 128, 64), ('gdn', 2, 333, 4, 128, 64, 128, 64, 128),
-    ('gdn', 1, 1000, 4, 128, 128, 128, 128, 256), ('gdn', 2, 300, 6, 64, 128, 192, 128, 64), ('gdn', 1, 777, 6, 64, 128, 128, 256, 64), ('gdn', 1, 200, 2, 128, 128, 64, 64, 64),
-    ('gdn', 1, 1344, 8, 64, 64, 64, 64, 64), ('gdn', 1, 1345, 8, 64, 64, 64, 64, 64), ('gdn', 120, 64, 1, 128, 128, 128, 128, 64),
-    ('mamba', 1, 1, 1, 64, 64, 64, 64, 64), ('mamba', 2, 333, 17, 128, 64, 128, 64, 256), ('mamba', 1, 700, 5, 64, 128, 192, 128, 64),
-    ('mamba', 1, 1500, 16, 128, 128, 128, 128, 64)])
+@pytest.mark.parametrize("kind,B,T,H,KA,VA,K,V,block", [c[:-1] for c in CASES])
 def test_one_launch_gives_what_two_give(kind, B, T, H, KA, VA, K, V, block, gradients, monkeypatch):
     import neuralattentionsearchlinear_amd._mixed_common as MC
     from neuralattentionsearchlinear_amd.mixed_attn_gdn import nats_mixed_attn_gdn

@@ -9,10 +9,13 @@ pytestmark = pytest.mark.gpu
 DEV = 'cuda:0'
 
 
-@pytest.mark.parametrize("blocks,B,H,HN,block,share,wide", [
+CASES = [
     (1, 1, 2, 2, 64, 0.5, False), (2, 3, 2, 1, 64, 1.0, True), (5, 40, 16, 16, 64, 0.4, False), (5, 40, 16, 4, 128, 0.4, False), (63, 1, 4, 2, 64, 0.3, True),
     (64, 2, 2, 2, 64, 0.0, False), (65, 1, 4, 4, 64, 0.5, False), (129, 1, 2, 1, 128, 0.2, False), (193, 2, 1, 1, 64, 1.0, True), (255, 1, 1, 1, 64, 0.7, False),
-    (256, 1, 2, 2, 64, 0.1, False), (257, 1, 1, 1, 64, 0.3, False)])
+    (256, 1, 2, 2, 64, 0.1, False), (257, 1, 1, 1, 64, 0.3, False)]
+
+
+@pytest.mark.parametrize("blocks,B,H,HN,block,share,wide", CASES)
 def test_tiles_find_their_blocks_in_the_types(blocks, B, H, HN, block, share, wide, monkeypatch):
     import neuralattentionsearchlinear_amd._mixed_common as MC
     from neuralattentionsearchlinear_amd import _capi

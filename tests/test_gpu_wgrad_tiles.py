@@ -6,10 +6,15 @@ pytestmark = pytest.mark.gpu
 DEV = 'cuda:0'
 
 
-# (rows of dY, columns of x): one tile of either width and eight columns more or less; several tiles; token slices that end inside a stage
-@pytest.mark.parametrize("T,D,widths", [(40, 184, (264,)), (65, 192, (256, 8)), (97, 200, (248,)), (130, 248, (136,)), (70, 256, (512, 24)), (1999, 384, (1152, 16)),
-                                        (700, 392, (40,)), (2011, 512, (768, 768)), (3001, 576, (2304, 32)), (2500, 1536, (1152, 1152, 2304, 2304, 16)),
-                                        (4097, 1024, (768, 768, 1536, 1536, 16))])
+# (tokens, columns of x, rows of dY) -> the tiles' columns and the slices of the tokens on 256 compute units (test_kernel_choices.py; None: another kernel
+# takes it).  One tile of either width and eight columns more or less; several tiles, last ones partly filled; token slices that end inside a stage
+CASES = [(40, 184, (264,), 192, 1), (65, 192, (256, 8), 192, 1), (97, 200, (248,), 192, 1), (130, 248, (136,), 256, 2), (70, 256, (512, 24), 256, 1),
+         (1999, 384, (1152, 16), 192, 7), (700, 392, (40,), None, 0), (2011, 512, (768, 768), 256, 5), (3001, 576, (2304, 32), 192, 5),
+         (2500, 1536, (1152, 1152, 2304, 2304, 16), 192, 1), (4097, 1024, (768, 768, 1536, 1536, 16), 256, 3),
+         (900, 360, (520, 24), 192, 6), (997, 1360, (648,), 192, 3), (700, 392, (264,), 256, 6)]
+
+
+@pytest.mark.parametrize("T,D,widths", [c[:3] for c in CASES])
 def test_weight_grads_by_tile_width(T, D, widths):
     from neuralattentionsearchlinear_amd._front import weight_grads
     torch.manual_seed(T)

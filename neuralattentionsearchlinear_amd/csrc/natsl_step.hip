@@ -939,7 +939,8 @@ NATSL_DEVICE void step_product(const StepAll& all, const int tile) {
   }
 }
 
-// (as many workgroups a CU as step_one_kernel's registers allow: the splits count on them)
+// (as many workgroups a CU as step_one_kernel's registers allow: the splits count on them.  For that the delta rule with 128-wide linear keys, other than on
+// 128/128 heads, keeps 4 vector registers of a lane (20 bytes) in scratch; the other forms none.)
 template <int KA, int VA, int K, bool DELTA>
 __global__ __launch_bounds__(256, K == 192 || KA + VA == 256 ? 2 : KA + VA + K == 192 ? 4 : 3) void step_all_kernel(const StepAll) {
   const StepAll& all = step_all_args();
@@ -1034,7 +1035,7 @@ static unsigned long long step_ticket(StepsUnderWay& u, hipStream_t st) {
     void* p = nullptr;
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;                // (another thread may be capturing: this is none of its graph's)
     (void)hipThreadExchangeStreamCaptureMode(&mode);
-    const hipError_t e = hipHostMalloc(&p, 64, hipHostMallocMapped | hipHostMallocCoherent);    // one line a device, for as long as the process lives
+    const hipError_t e = hipHostMalloc(&p, 64, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent);    // one line a device, for as long as the process lives
     (void)hipThreadExchangeStreamCaptureMode(&mode);
     if (e != hipSuccess) {
       (void)hipGetLastError();

@@ -1,10 +1,10 @@
-"""The layers' generation step as one native call (natsl_layer_step_fwd): a few new tokens of cached sequences, from the hidden
+"""The layers' generation step as one native call (natsl_layer_step_sync_fwd): a few new tokens of cached sequences, from the hidden
 states to the layer's output, with the cache's new rows written in place.
 
 A step of a layer is a few microseconds of memory traffic per kernel, so what it costs is launches and host time: the same step
-as separate torch operations and operator calls is forty launches and ~0.57 ms of host time (340M geometry), this is three
-launches (five for several tokens a sequence) and 20 us behind one call of csrc/host/step_core.cpp, which also compares the layer with its plan, checks the cache's tensors and
-allocates the step's.  `layer_step` declines (returns None) whatever the call is not built for -- other dtypes,
+as separate torch operations and operator calls is forty launches and ~0.57 ms of host time (340M geometry), this is one
+launch for one token of few sequences, three for more, five for several tokens a sequence, and at most 20 us behind one call of
+csrc/host/step_core.cpp, which also compares the layer with its plan, checks the cache's tensors and allocates the step's.  `layer_step` declines (returns None) whatever the call is not built for -- other dtypes,
 tensors that want gradients, replaced or hooked submodules, the 'attn' mode, more than 64 new tokens in all -- and the layers'
 general path runs.
 """

@@ -1,7 +1,8 @@
 // Host side of the mixed operators' forward and of the selector's hard choice (_mixed_common.py, nats_util.py) for calls that need nothing out of the
 // ordinary: no gradient, no packed sequences, tensors of the types and shapes that go together.  What a call does besides launching took twice as
 // long as its launches when it was Python: the host has 42 us with B1 T256 H4 128/128 and 57 with fp32 B1 T256 H2 64/64, 25 and 30 with this, and the call then
-// takes what its kernels take, 32 and 33.  Everything else is declined (None) and runs, or is refused, there.  Nothing outlives a call.
+// takes what its kernels take: 32 and 33 (the second 27 since the routing launch is gone and the branches' first kernels are one).  Everything else is
+// declined (None) and runs, or is refused, there.  Nothing outlives a call.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
